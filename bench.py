@@ -489,20 +489,20 @@ def main() -> int:
                     return st_odd(s7, zw7, None, inplace_safe=True)
             odd = {}
             for pad_to in (8, 0):
-                keep_pad = pf.pad_tokens_to
-                pf.pad_tokens_to = pad_to
+                keep_pad = pf.pad_tokens_to, pf.pad_tokens_end_n
+                pf.pad_tokens_to, pf.pad_tokens_end_n = pad_to, 1 << 30
                 try:
                     _, per_odd, out_odd = timed(step_odd, 2, 5)
                 finally:
-                    pf.pad_tokens_to = keep_pad
+                    pf.pad_tokens_to, pf.pad_tokens_end_n = keep_pad
                 odd[pad_to] = (statistics.median(per_odd) / 4, out_odd[1].clone())
             shapes["odd_size_n700_4_blocks"] = {
                 "ms_per_block": round(odd[8][0], 3), "ms_per_block_unpadded": round(odd[0][0], 3),
                 "same_bits": bool(torch.equal(odd[8][1], odd[0][1])),
                 "workload": "PairformerStack 4 blocks, N_token=700, no pair mask, fp32 tensors under "
-                            "torch.autocast(bfloat16): as 704 tokens with 4 masked (the default from 320 "
-                            "tokens on; the two copies of the pair tensor weigh 12 times what they weigh "
-                            "in a trunk) against the rows as they are"}
+                            "torch.autocast(bfloat16): as 704 tokens with 4 masked (the "
+                            "two copies of the pair tensor weigh 12 times what they weigh "
+                            "in a trunk) against the rows as they are (the default)"}
             del st_odd, s7, z7, zw7, step_odd, odd
             torch.cuda.empty_cache()
             stack = None

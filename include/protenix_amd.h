@@ -104,6 +104,42 @@ PTX_API int ptx_layernorm_fwd(const void* x, const void* gamma, const void* beta
                       int dtype, void* stream);
 
 /*
+ * The row-local stages of the triangle updates on packed weights: the same operations as
+ * ptx_trimul_project / _output and ptx_triattn_project / _gate_output / _output, on weights
+ * laid out once per weight set by ptx_trimul_pack / ptx_triattn_pack (matrices [out][in] as in
+ * those calls, in the arithmetic type; packed: ptx_*_packed_elems elements).  The faster way at
+ * every size for callers that keep their weights.  c_z, c_hidden, heads, dtype as there.
+ *   ptx_trimul_contract_ld: ptx_trimul_contract with rows of x at a pitch of ldx elements
+ *     (x [c][n][ldx]); ptx_trimul_output_packed takes ldx = n rounded up to a multiple of 8.
+ *   ptx_triattn_late_gate: 1 where the output stage forms the gate itself; ptx_triattn_project_packed
+ *     then takes g = NULL and ptx_triattn_output_packed an ungated o.
+ */
+PTX_API int64_t ptx_trimul_packed_elems(int c_z, int c_hidden);
+PTX_API int ptx_trimul_pack(const void* w_ap, const void* w_ag, const void* w_bp, const void* w_bg,
+                      const void* w_z, const void* w_g, void* packed, int c_z, int c_hidden, int dtype,
+                      void* stream);
+PTX_API int ptx_trimul_project_packed(const void* z, const void* mask, const void* ln_w, const void* ln_b,
+                      const void* packed, void* a, void* b, int n, int c_z, int c_hidden,
+                      int k_pitch, int incoming, float eps, int dtype, void* stream);
+PTX_API int ptx_trimul_contract_ld(const void* a, const void* b, void* x, int n, int ldx, int c, int k_pitch,
+                      int dtype, void* stream);
+PTX_API int ptx_trimul_output_packed(const void* x, int ldx, const void* z, const void* ln_in_w,
+                      const void* ln_in_b, const void* ln_out_w, const void* ln_out_b,
+                      const void* packed, void* out, int n, int c_z, int c_hidden, int add_residual,
+                      float eps, int dtype, void* stream);
+PTX_API int64_t ptx_triattn_packed_elems(int c_in, int heads);
+PTX_API int ptx_triattn_late_gate(int c_in, int heads, int dtype);
+PTX_API int ptx_triattn_pack(const void* w_q, const void* w_k, const void* w_v, const void* w_g,
+                      const void* w_b, const void* w_o, void* packed, int c_in, int heads, int dtype,
+                      void* stream);
+PTX_API int ptx_triattn_project_packed(const void* z, const void* ln_w, const void* ln_b, const void* packed,
+                      void* q, void* k, void* vt, void* g, void* tri_bias, int n, int c_in, int heads,
+                      int key_pitch, int transposed, float eps, int dtype, void* stream);
+PTX_API int ptx_triattn_output_packed(const void* o, const void* z, const void* ln_w, const void* ln_b,
+                      const void* packed, void* out, int n, int c_in, int heads, int transposed,
+                      int add_residual, float eps, int dtype, void* stream);
+
+/*
  * LayerNorm backward.  Replaces fast_layer_norm_cuda_v2.backward_{none,with_bias,with_weight,
  * with_both}_affine (layer_norm_cuda.cpp:159-178; kernels layer_norm_cuda_kernel.cu:395-760,
  * host :860-990), fp32 arithmetic, with xc = x - mean and gd = gamma * dout:

@@ -35,6 +35,16 @@ SIGNATURES = {
     "ptx_layernorm_bwd_static": (_i, [_p] * 8 + [_l, _i, _i, _p]),
     "ptx_trimul_project": (_i, [_p] * 10 + [_i, _i, _i, _i, _i, _f, _i, _p]),
     "ptx_trimul_contract": (_i, [_p, _p, _p, _i, _i, _i, _i, _p]),
+    "ptx_trimul_packed_elems": (_l, [_i, _i]),
+    "ptx_trimul_pack": (_i, [_p] * 7 + [_i, _i, _i, _p]),
+    "ptx_trimul_project_packed": (_i, [_p] * 7 + [_i, _i, _i, _i, _i, _f, _i, _p]),
+    "ptx_trimul_contract_ld": (_i, [_p, _p, _p, _i, _i, _i, _i, _i, _p]),
+    "ptx_trimul_output_packed": (_i, [_p, _i] + [_p] * 7 + [_i, _i, _i, _i, _f, _i, _p]),
+    "ptx_triattn_packed_elems": (_l, [_i, _i]),
+    "ptx_triattn_late_gate": (_i, [_i, _i, _i]),
+    "ptx_triattn_pack": (_i, [_p] * 7 + [_i, _i, _i, _p]),
+    "ptx_triattn_project_packed": (_i, [_p] * 9 + [_i, _i, _i, _i, _i, _f, _i, _p]),
+    "ptx_triattn_output_packed": (_i, [_p] * 6 + [_i, _i, _i, _i, _i, _f, _i, _p]),
     "ptx_trimul_output": (_i, [_p] * 9 + [_i, _i, _i, _i, _f, _i, _p]),
     "ptx_triangle_multiplicative_update_workspace_elems": (_l, [_i, _i]),
     "ptx_triangle_multiplicative_update": (_i, [_p, _i] + [_p] * 11 + [_i, _i, _i, _i, _f, _i, _p]),

@@ -232,17 +232,24 @@ PTX_API int ptx_trimul_project(const void* z, const void* mask, const void* ln_w
 
 PTX_API int ptx_trimul_contract(const void* a, const void* b, void* x, int n, int c, int k_pitch, int dtype,
                         void* stream) {
+  return ptx_trimul_contract_ld(a, b, x, n, n, c, k_pitch, dtype, stream);
+}
+
+PTX_API int ptx_trimul_contract_ld(const void* a, const void* b, void* x, int n, int ldx, int c, int k_pitch,
+                                   int dtype, void* stream) {
   if (dtype == PTX_MIXED) dtype = PTX_BF16;   // no residual-stream tensor here
   PTX_REQUIRE(dtype_ok(dtype), PTX_ERR_BAD_ARG, "trimul_contract: unknown dtype %d", dtype);
   PTX_REQUIRE(n >= 0 && c >= 0, PTX_ERR_BAD_ARG, "trimul_contract: n=%d c=%d", n, c);
   PTX_REQUIRE(k_pitch == ptx_key_pitch(n), PTX_ERR_BAD_ARG,
               "trimul_contract: k_pitch=%d, expected %d", k_pitch, ptx_key_pitch(n));
   PTX_REQUIRE(n < 32768, PTX_ERR_UNSUPPORTED, "trimul_contract: n=%d too large", n);
+  PTX_REQUIRE(ldx >= n && (ldx == n || ldx % 8 == 0), PTX_ERR_BAD_ARG,
+              "trimul_contract: ldx=%d (n=%d, or a multiple of 8 above it)", ldx, n);
   if (n == 0 || c == 0) return PTX_OK;
   PTX_REQUIRE(a && b && x, PTX_ERR_BAD_ARG, "trimul_contract: null pointer");
   PTX_REQUIRE(aligned16(a) && aligned16(b), PTX_ERR_BAD_ARG,
               "trimul_contract: a and b must be 16-byte aligned");
-  PTX_DISPATCH(dtype, ptx::nt_gemm_batched<T>((const T*)a, (const T*)b, (T*)x, n, k_pitch, c,
+  PTX_DISPATCH(dtype, ptx::nt_gemm_batched<T>((const T*)a, (const T*)b, (T*)x, n, ldx, k_pitch, c,
                                               (hipStream_t)stream));
   return after_launch("trimul_contract");
 }
@@ -381,6 +388,124 @@ PTX_API int ptx_triattn_fwd_rows(const void* q, const void* k, const void* vt, c
   return triattn_fwd_checked("triattn_fwd_rows", q, k, vt, g, tri_bias, mask, o, n, heads, d,
                              key_pitch, mask_transposed, inf, row_begin, row_count, n_keys, dtype,
                              stream);
+}
+
+// ---- the row-local stages on packed weights (pairproj.hip) ----
+PTX_API int64_t ptx_trimul_packed_elems(int c_z, int c_hidden) {
+  return c_z > 0 && c_hidden > 0 ? ptx::pp_trimul_packed_elems(c_z, c_hidden) : 0;
+}
+
+PTX_API int ptx_trimul_pack(const void* w_ap, const void* w_ag, const void* w_bp, const void* w_bg,
+                            const void* w_z, const void* w_g, void* packed, int c_z, int c_hidden, int dtype,
+                            void* stream) {
+  PTX_REQUIRE(dtype_ok_z(dtype), PTX_ERR_BAD_ARG, "trimul_pack: unknown dtype %d", dtype);
+  PTX_REQUIRE(pair_width_ok(c_z, c_hidden, dtype), PTX_ERR_UNSUPPORTED, "trimul_pack: %s (got c_z=%d c_hidden=%d)",
+              kWidthMsg, c_z, c_hidden);
+  PTX_REQUIRE(w_ap && w_ag && w_bp && w_bg && w_z && w_g && packed, PTX_ERR_BAD_ARG, "trimul_pack: null pointer");
+  PTX_REQUIRE(aligned16(packed), PTX_ERR_BAD_ARG, "trimul_pack: packed must be 16-byte aligned");
+  if (dtype == PTX_MIXED) dtype = PTX_BF16;
+  PTX_DISPATCH(dtype, ptx::pp_trimul_pack<T>(w_ap, w_ag, w_bp, w_bg, w_z, w_g, packed, c_z, c_hidden,
+                                             (hipStream_t)stream));
+  return after_launch("trimul_pack");
+}
+
+PTX_API int ptx_trimul_project_packed(const void* z, const void* mask, const void* ln_w, const void* ln_b,
+                                      const void* packed, void* a, void* b, int n, int c_z, int c_hidden,
+                                      int k_pitch, int incoming, float eps, int dtype, void* stream) {
+  PTX_REQUIRE(dtype_ok_z(dtype), PTX_ERR_BAD_ARG, "trimul_project_packed: unknown dtype %d", dtype);
+  PTX_REQUIRE(n >= 0, PTX_ERR_BAD_ARG, "trimul_project_packed: n=%d", n);
+  PTX_REQUIRE(pair_width_ok(c_z, c_hidden, dtype), PTX_ERR_UNSUPPORTED,
+              "trimul_project_packed: %s (got c_z=%d c_hidden=%d)", kWidthMsg, c_z, c_hidden);
+  PTX_REQUIRE(k_pitch == ptx_key_pitch(n), PTX_ERR_BAD_ARG, "trimul_project_packed: k_pitch=%d, expected %d", k_pitch,
+              ptx_key_pitch(n));
+  PTX_REQUIRE(n <= 8192, PTX_ERR_UNSUPPORTED, "trimul_project_packed: n=%d too large (8192 at most)", n);
+  if (n == 0) return PTX_OK;
+  PTX_REQUIRE(z && packed && a && b, PTX_ERR_BAD_ARG, "trimul_project_packed: null pointer");
+  PTX_REQUIRE(aligned16(z) && aligned16(packed) && aligned16(a) && aligned16(b) && (!ln_w || aligned16(ln_w)) &&
+                  (!ln_b || aligned16(ln_b)),
+              PTX_ERR_BAD_ARG, "trimul_project_packed: pointers must be 16-byte aligned");
+  PTX_DISPATCH_Z(dtype, (ptx::pp_trimul_in<T, TZ>)(z, mask, ln_w, ln_b, packed, a, b, n, c_z, k_pitch, incoming, eps,
+                                                   (hipStream_t)stream));
+  return after_launch("trimul_project_packed");
+}
+
+PTX_API int ptx_trimul_output_packed(const void* x, int ldx, const void* z, const void* ln_in_w, const void* ln_in_b,
+                                     const void* ln_out_w, const void* ln_out_b, const void* packed, void* out, int n,
+                                     int c_z, int c_hidden, int add_residual, float eps, int dtype, void* stream) {
+  PTX_REQUIRE(dtype_ok_z(dtype), PTX_ERR_BAD_ARG, "trimul_output_packed: unknown dtype %d", dtype);
+  PTX_REQUIRE(n >= 0, PTX_ERR_BAD_ARG, "trimul_output_packed: n=%d", n);
+  PTX_REQUIRE(pair_width_ok(c_z, c_hidden, dtype), PTX_ERR_UNSUPPORTED,
+              "trimul_output_packed: %s (got c_z=%d c_hidden=%d)", kWidthMsg, c_z, c_hidden);
+  PTX_REQUIRE(n < 32768, PTX_ERR_UNSUPPORTED, "trimul_output_packed: n=%d too large", n);
+  PTX_REQUIRE(ldx >= n && ldx % 8 == 0, PTX_ERR_BAD_ARG, "trimul_output_packed: ldx=%d (a multiple of 8, >= n=%d)", ldx, n);
+  if (n == 0) return PTX_OK;
+  PTX_REQUIRE(x && z && packed && out, PTX_ERR_BAD_ARG, "trimul_output_packed: null pointer");
+  PTX_REQUIRE(aligned16(x) && aligned16(out) && aligned16(z) && aligned16(packed) && (!ln_out_w || aligned16(ln_out_w)) &&
+                  (!ln_out_b || aligned16(ln_out_b)) && (!ln_in_w || aligned16(ln_in_w)) && (!ln_in_b || aligned16(ln_in_b)),
+              PTX_ERR_BAD_ARG, "trimul_output_packed: pointers must be 16-byte aligned");
+  PTX_DISPATCH_Z(dtype, (ptx::pp_trimul_out<T, TZ>)(x, ldx, z, ln_in_w, ln_in_b, ln_out_w, ln_out_b, packed, out, n, c_z,
+                                                    c_hidden, add_residual, eps, (hipStream_t)stream));
+  return after_launch("trimul_output_packed");
+}
+
+PTX_API int64_t ptx_triattn_packed_elems(int c_in, int heads) {
+  return c_in > 0 && heads > 0 ? ptx::pp_triattn_packed_elems(c_in, heads) : 0;
+}
+
+PTX_API int ptx_triattn_late_gate(int c_in, int heads, int dtype) {
+  return ptx::pp_late_gate(c_in, heads, dtype != PTX_F32);
+}
+
+PTX_API int ptx_triattn_pack(const void* w_q, const void* w_k, const void* w_v, const void* w_g, const void* w_b,
+                             const void* w_o, void* packed, int c_in, int heads, int dtype, void* stream) {
+  PTX_REQUIRE(dtype_ok_z(dtype), PTX_ERR_BAD_ARG, "triattn_pack: unknown dtype %d", dtype);
+  PTX_REQUIRE(heads > 0 && heads <= 8 && pair_width_ok(c_in, heads * 32, dtype), PTX_ERR_UNSUPPORTED,
+              "triattn_pack: %s (got c_in=%d heads=%d)", kWidthMsg, c_in, heads);
+  PTX_REQUIRE(w_q && w_k && w_v && w_g && w_b && w_o && packed, PTX_ERR_BAD_ARG, "triattn_pack: null pointer");
+  PTX_REQUIRE(aligned16(packed), PTX_ERR_BAD_ARG, "triattn_pack: packed must be 16-byte aligned");
+  if (dtype == PTX_MIXED) dtype = PTX_BF16;
+  PTX_DISPATCH(dtype, ptx::pp_triattn_pack<T>(w_q, w_k, w_v, w_g, w_b, w_o, packed, c_in, heads, (hipStream_t)stream));
+  return after_launch("triattn_pack");
+}
+
+PTX_API int ptx_triattn_project_packed(const void* z, const void* ln_w, const void* ln_b, const void* packed, void* q,
+                                       void* k, void* vt, void* g, void* tri_bias, int n, int c_in, int heads,
+                                       int key_pitch, int transposed, float eps, int dtype, void* stream) {
+  PTX_REQUIRE(dtype_ok_z(dtype), PTX_ERR_BAD_ARG, "triattn_project_packed: unknown dtype %d", dtype);
+  PTX_REQUIRE(n >= 0, PTX_ERR_BAD_ARG, "triattn_project_packed: n=%d", n);
+  PTX_REQUIRE(heads > 0 && heads <= 8 && pair_width_ok(c_in, heads * 32, dtype), PTX_ERR_UNSUPPORTED,
+              "triattn_project_packed: %s (got c_in=%d heads=%d)", kWidthMsg, c_in, heads);
+  PTX_REQUIRE(key_pitch == ptx_key_pitch(n), PTX_ERR_BAD_ARG, "triattn_project_packed: key_pitch=%d, expected %d",
+              key_pitch, ptx_key_pitch(n));
+  PTX_REQUIRE(n <= 8192, PTX_ERR_UNSUPPORTED, "triattn_project_packed: n=%d too large (8192 at most)", n);
+  if (n == 0) return PTX_OK;
+  const bool late = ptx::pp_late_gate(c_in, heads, dtype != PTX_F32);
+  PTX_REQUIRE(z && packed && q && k && vt && tri_bias && (g || late), PTX_ERR_BAD_ARG,
+              "triattn_project_packed: null pointer");
+  PTX_REQUIRE(aligned16(z) && aligned16(packed) && aligned16(q) && aligned16(k) && aligned16(vt) && (!g || aligned16(g)) &&
+                  aligned16(tri_bias) && (!ln_w || aligned16(ln_w)) && (!ln_b || aligned16(ln_b)),
+              PTX_ERR_BAD_ARG, "triattn_project_packed: pointers must be 16-byte aligned");
+  PTX_DISPATCH_Z(dtype, (ptx::pp_triattn_in<T, TZ>)(z, ln_w, ln_b, packed, q, k, vt, g, tri_bias, n, c_in, heads,
+                                                    key_pitch, transposed, eps, (hipStream_t)stream));
+  return after_launch("triattn_project_packed");
+}
+
+PTX_API int ptx_triattn_output_packed(const void* o, const void* z, const void* ln_w, const void* ln_b,
+                                      const void* packed, void* out, int n, int c_in, int heads, int transposed,
+                                      int add_residual, float eps, int dtype, void* stream) {
+  PTX_REQUIRE(dtype_ok_z(dtype), PTX_ERR_BAD_ARG, "triattn_output_packed: unknown dtype %d", dtype);
+  PTX_REQUIRE(n >= 0, PTX_ERR_BAD_ARG, "triattn_output_packed: n=%d", n);
+  PTX_REQUIRE(heads > 0 && heads <= 8 && pair_width_ok(c_in, heads * 32, dtype), PTX_ERR_UNSUPPORTED,
+              "triattn_output_packed: %s (got c_in=%d heads=%d)", kWidthMsg, c_in, heads);
+  PTX_REQUIRE(n < 32768, PTX_ERR_UNSUPPORTED, "triattn_output_packed: n=%d too large", n);
+  if (n == 0) return PTX_OK;
+  PTX_REQUIRE(o && z && packed && out, PTX_ERR_BAD_ARG, "triattn_output_packed: null pointer");
+  PTX_REQUIRE(aligned16(o) && aligned16(z) && aligned16(packed) && aligned16(out) && (!ln_w || aligned16(ln_w)) &&
+                  (!ln_b || aligned16(ln_b)),
+              PTX_ERR_BAD_ARG, "triattn_output_packed: pointers must be 16-byte aligned");
+  PTX_DISPATCH_Z(dtype, (ptx::pp_triattn_out<T, TZ>)(o, z, ln_w, ln_b, packed, out, n, c_in, heads, transposed,
+                                                     add_residual, eps, (hipStream_t)stream));
+  return after_launch("triattn_output_packed");
 }
 
 PTX_API int64_t ptx_triattn_core_workspace_elems(int n_rows, int s, int heads) {

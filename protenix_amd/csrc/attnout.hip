@@ -93,7 +93,7 @@ __global__ __launch_bounds__((kGoWaves * 64), 1) void triattn_gate_out_kernel(Ga
       f32x8 v[kKSteps];
 #pragma unroll
       for (int kk = 0; kk < kKSteps; ++kk) v[kk] = to_f32(zraw[kk]);
-      normalize_row<T, kKSteps, float, false>(v, lds_affine[0], lds_affine[1], p.eps, g, xf);
+      normalize_row<T, TZ, kKSteps, float, false>(v, lds_affine[0], lds_affine[1], p.eps, g, xf);
     }
     // gate per head, applied to the attention output in place (both rounded to T like the
     // reference's sigmoid(linear_g(x)) and o * g)

@@ -81,6 +81,33 @@ template <typename T, typename TZ = T>
 int pair_bias_fwd(const void* z, const void* ln_w, const void* ln_b, const void* w, void* bias,
                   int n, int c_z, int heads, int out_f32, float eps, hipStream_t stream);
 
+// The row-local stages of the triangle updates on packed weights (pairproj.hip).
+// Whether the attention's gate is formed by the output stage (no gate tensor exists then).
+inline bool pp_late_gate(int c_z, int heads, bool bits16) { return c_z == 128 && heads == 4 && bits16; }
+int64_t pp_trimul_packed_elems(int c_z, int hidden);
+template <typename T>
+int pp_trimul_pack(const void* w_ap, const void* w_ag, const void* w_bp, const void* w_bg, const void* w_z,
+                   const void* w_g, void* packed, int c_z, int hidden, hipStream_t stream);
+int64_t pp_triattn_packed_elems(int c_z, int heads);
+template <typename T>
+int pp_triattn_pack(const void* w_q, const void* w_k, const void* w_v, const void* w_g, const void* w_b,
+                    const void* w_o, void* packed, int c_z, int heads, hipStream_t stream);
+template <typename T, typename TZ = T>
+int pp_trimul_in(const void* z, const void* mask, const void* ln_w, const void* ln_b, const void* packed, void* a,
+                 void* b, int n, int c_z, int k_pitch, int incoming, float eps, hipStream_t stream);
+template <typename T, typename TZ = T>
+int pp_triattn_in(const void* z, const void* ln_w, const void* ln_b, const void* packed, void* q, void* k, void* vt,
+                  void* g, void* tri_bias, int n, int c_z, int heads, int key_pitch, int transposed, float eps,
+                  hipStream_t stream);
+// x [hidden][n][ldx]: ldx = n, or n rounded up to a multiple of 8 (rows of any n then start aligned)
+template <typename T, typename TZ = T>
+int pp_trimul_out(const void* x, int ldx, const void* z, const void* ln_in_w, const void* ln_in_b,
+                  const void* ln_out_w, const void* ln_out_b, const void* packed, void* out, int n, int c_z,
+                  int hidden, int add_residual, float eps, hipStream_t stream);
+template <typename T, typename TZ = T>
+int pp_triattn_out(const void* o, const void* z, const void* ln_w, const void* ln_b, const void* packed, void* out,
+                   int n, int c_z, int heads, int transposed, int add_residual, float eps, hipStream_t stream);
+
 // Small linear layers of the single-representation track (single.hip):
 //   out[rows][n_out] = [res +] x[rows][k] w[n_out][k]^T [+ bias on columns < bias_cols];
 //   output columns >= split_col go, transposed, to out_t[n_out - split_col][ldt] instead
@@ -101,9 +128,9 @@ int single_attention_fwd(const void* q, const void* k, const void* vt, const voi
                          int64_t ld, int64_t ldt, int64_t ldo, float scale, hipStream_t stream);
 
 // x[c][i][j] = sum_k a[c][i][k] * b[c][j][k] for `batch` independent products;
-// a, b rows have pitch k_pitch (a multiple of 64, >= n), x is dense [batch][n][n].
+// a, b rows have pitch k_pitch (a multiple of 64, >= n), x is [batch][n][ldx].
 template <typename T>
-int nt_gemm_batched(const T* a, const T* b, T* x, int n, int k_pitch, int batch,
+int nt_gemm_batched(const T* a, const T* b, T* x, int n, int ldx, int k_pitch, int batch,
                     hipStream_t stream);
 
 // Flash-style triangle attention core (see triattn.hip).

@@ -60,7 +60,7 @@ template <typename T> struct GemmCfg {
 template <typename T, int JB>
 __global__ __launch_bounds__(256) void nt_gemm_batched_kernel(const T* __restrict__ a,
                                                               const T* __restrict__ b,
-                                                              T* __restrict__ x, int n, int k_pitch,
+                                                              T* __restrict__ x, int n, int ldx, int k_pitch,
                                                               int batch, int tiles_i, int tiles_j) {
   typedef typename Vec8<T>::type V8;
   typedef typename Vec4<T>::type V4;
@@ -223,16 +223,16 @@ __global__ __launch_bounds__(256) void nt_gemm_batched_kernel(const T* __restric
   // 8 rows per store instruction instead of 32-byte pieces of 32 lines: 150 against 145 us per
   // launch at N = 768, 1780 against 1745 at 2048 - with one wave per SIMD the extra LDS round
   // trips cost more than the lines save.)
-  const bool vec_ok = (n % G::VE) == 0;
+  const bool vec_ok = (ldx % G::VE) == 0;   // (a vector that starts inside n ends inside the pitch)
   auto store_tile = [&](int m) {
     int c, ti, tj;
     entry_coords(m, c, ti, tj);
-    T* x_c = x + (int64_t)c * n * n;
+    T* x_c = x + (int64_t)c * n * ldx;
     const int i0 = ti * 256 + wi * 128, j0 = tj * (64 * JB) + wj * (32 * JB);
 #pragma unroll
     for (int rb = 0; rb < 4; ++rb) {
       const int i = i0 + rb * 32 + ln;
-      T* x_row = x_c + (int64_t)i * n;
+      T* x_row = x_c + (int64_t)i * ldx;
 #pragma unroll
       for (int jb = 0; jb < JB; ++jb) {
         const int jt = j0 + jb * 32;
@@ -263,7 +263,7 @@ __global__ __launch_bounds__(256) void nt_gemm_batched_kernel(const T* __restric
             const int j = jt + 16 * p + 8 * g;
             if (i < n) {
               if (vec_ok) {
-                if (j < n) *reinterpret_cast<u32x4*>(x_row + j) = out;   // n % 8 == 0: all in range
+                if (j < n) *reinterpret_cast<u32x4*>(x_row + j) = out;
               } else {
                 const T* e8 = reinterpret_cast<const T*>(&out);
 #pragma unroll
@@ -338,7 +338,7 @@ static int contraction_grid() {
 }
 
 template <typename T>
-int nt_gemm_batched(const T* a, const T* b, T* x, int n, int k_pitch, int batch,
+int nt_gemm_batched(const T* a, const T* b, T* x, int n, int ldx, int k_pitch, int batch,
                     hipStream_t stream) {
   if (n == 0 || batch == 0) return 0;
   const int grid = contraction_grid();
@@ -347,12 +347,12 @@ int nt_gemm_batched(const T* a, const T* b, T* x, int n, int k_pitch, int batch,
   const int tiles_j = (n + 255) / 256;
   const int64_t blocks = std::min<int64_t>(grid, groups * tiles_i * tiles_j * 8);
   nt_gemm_batched_kernel<T, 4><<<dim3((unsigned)((blocks + 7) & ~7)), dim3(256), 0, stream>>>(
-      a, b, x, n, k_pitch, batch, tiles_i, tiles_j);
+      a, b, x, n, ldx, k_pitch, batch, tiles_i, tiles_j);
   return 0;
 }
 
-template int nt_gemm_batched<float>(const float*, const float*, float*, int, int, int, hipStream_t);
-template int nt_gemm_batched<bf16_t>(const bf16_t*, const bf16_t*, bf16_t*, int, int, int,
+template int nt_gemm_batched<float>(const float*, const float*, float*, int, int, int, int, hipStream_t);
+template int nt_gemm_batched<bf16_t>(const bf16_t*, const bf16_t*, bf16_t*, int, int, int, int,
                                      hipStream_t);
 
 }  // namespace ptx

@@ -1,0 +1,1035 @@
+// The row-local stages of the triangle updates on packed weights: LayerNorm + projections
+// (trimul_in, triattn_in), and the output stages (trimul_out, triattn_out).
+//
+// A workgroup of four waves takes a tile of 32 * RBW pair-tensor rows.  Its rows are read once, in
+// whole cache lines (8 lanes per row), normalised in fp32 and parked in LDS as MFMA operand
+// fragments; after one barrier every wave multiplies them by its own share of the output columns.
+// The weights were packed into fragment order beforehand (pair_pack), so a fragment is one
+// contiguous 1 KB load from the L2 into registers, used for all of the tile's row blocks: no LDS
+// traffic for them, and no barrier in the loop.  (The L2s deliver a buffer that all compute units
+// read at 28 - 31 TB/s: 128 KB of weights per 64 rows are 42 us per launch at N = 768, under
+// the 120 us that the pair tensor's own bytes take.  Read from row-major weights, a fragment touches 32
+// cache lines per load instruction and costs the first-level cache four times as much.)
+// Short workgroups, three or four of them per compute unit at different points of their lives,
+// take the place of the resident kernels of rowgemm.hip (which still serve callers that hand in
+// row-major weights): those hold 128 KB of weights per compute unit and two waves per SIMD, need eight row
+// tiles per compute unit to have something for every wave, and end in a partial round of tiles.
+#include "common.h"
+#include "kernels.h"
+#include "rowtile.h"
+#include <algorithm>
+#include <type_traits>
+
+namespace ptx {
+
+namespace {
+
+constexpr int kPpWaves = 4;
+
+// Hidden widths (see Widths in rowgemm.hip): 128 for rows of at most 128 channels, else the row width.
+template <int KS> struct PpWidths {
+  static constexpr int SL = KS > 8 ? KS : 8;
+  static constexpr int HIDDEN = 16 * SL;
+  static constexpr int HEADS = HIDDEN / 32;
+};
+
+// ---- normalised rows in LDS -------------------------------------------------------------
+// Row block rb, 8-channel group c8, 16-byte piece: one plane of 32 rows x 16 bytes.  A fragment
+// read (K step kk: groups 2 kk + lane / 32, lane % 32 = row) is two contiguous halves of planes;
+// the plane pitch spreads the writes (8 neighbouring lanes hold 8 groups of one row).
+constexpr int kPlanePitch = 32 * 16 + 32;
+template <typename T, int KS> struct FragLds {
+  static constexpr int PIECES = (int)sizeof(T) / 2;
+  static constexpr int ROWBLOCK = 2 * KS * PIECES * kPlanePitch;   // bytes per 32 rows
+  static __device__ __forceinline__ void put(char* base, int rb, int row, int c8, typename Vec8<T>::type v) {
+    const u32x4_t* s = reinterpret_cast<const u32x4_t*>(&v);
+    char* d = base + rb * ROWBLOCK + c8 * PIECES * kPlanePitch + row * 16;
+#pragma unroll
+    for (int pc = 0; pc < PIECES; ++pc) *reinterpret_cast<u32x4_t*>(d + pc * kPlanePitch) = s[pc];
+  }
+  static __device__ __forceinline__ typename Vec8<T>::type get(const char* base, int rb, int kk, int lane) {
+    typename Vec8<T>::type v;
+    u32x4_t* d = reinterpret_cast<u32x4_t*>(&v);
+    const char* s = base + rb * ROWBLOCK + (2 * kk + (lane >> 5)) * PIECES * kPlanePitch + (lane & 31) * 16;
+#pragma unroll
+    for (int pc = 0; pc < PIECES; ++pc) d[pc] = *reinterpret_cast<const u32x4_t*>(s + pc * kPlanePitch);
+    return v;
+  }
+};
+
+// Fragment `f` of a packed weight set: [fragment][16-byte piece][lane].
+template <typename T>
+__device__ __forceinline__ typename Vec8<T>::type packed_frag(const T* packed, int f, int lane) {
+  constexpr int PIECES = (int)sizeof(T) / 2;
+  typename Vec8<T>::type v;
+  u32x4_t* d = reinterpret_cast<u32x4_t*>(&v);
+  const u32x4_t* s = reinterpret_cast<const u32x4_t*>(packed + (int64_t)f * kFragElems) + lane;
+#pragma unroll
+  for (int pc = 0; pc < PIECES; ++pc) d[pc] = s[pc * kWave];
+  return v;
+}
+
+// A row in 8 neighbouring lanes: lane j holds the 16-byte pieces j, j + 8, .. of the stored row (PE
+// channels each), so that every access covers whole 128-byte lines.
+template <typename TZ, int KS> struct RowPieces {
+  static constexpr int PE = 16 / (int)sizeof(TZ);
+  static constexpr int NP = 16 * KS / (8 * PE);   // pieces per lane
+  typedef typename VecE<TZ>::type V;
+};
+
+// LayerNorm of such a row (statistics in fp32, two passes) with this lane's gamma / beta.
+template <int PE, int NP>
+__device__ __forceinline__ void normalize_pieces(float (&v)[NP][PE], const float (&gm)[NP][PE], const float (&bt)[NP][PE], float eps) {
+  float s = 0.0f;
+#pragma unroll
+  for (int q = 0; q < NP; ++q)
+#pragma unroll
+    for (int t = 0; t < PE; ++t) s += v[q][t];
+  const float mean = lane_group_sum<8>(s) * (1.0f / (8 * NP * PE));
+  float d2 = 0.0f;
+#pragma unroll
+  for (int q = 0; q < NP; ++q)
+#pragma unroll
+    for (int t = 0; t < PE; ++t) {
+      const float d = v[q][t] - mean;
+      d2 += d * d;
+    }
+  const float rstd = rsqrtf(lane_group_sum<8>(d2) * (1.0f / (8 * NP * PE)) + eps);
+#pragma unroll
+  for (int q = 0; q < NP; ++q)
+#pragma unroll
+    for (int t = 0; t < PE; ++t) v[q][t] = (v[q][t] - mean) * rstd * gm[q][t] + bt[q][t];
+}
+
+template <typename T, int PE, int NP>
+__device__ __forceinline__ void load_affine_pieces(const T* gamma, const T* beta, int j, float (&gm)[NP][PE], float (&bt)[NP][PE]) {
+  const T* gp = (gamma ? gamma : default_gamma<T>()) + PE * j;
+  const T* bp = (beta ? beta : default_beta<T>()) + PE * j;
+#pragma unroll
+  for (int q = 0; q < NP; ++q)
+#pragma unroll
+    for (int e = 0; e < PE; e += 4) {
+      const f32x4 g4 = to_f32(*reinterpret_cast<const typename Vec4<T>::type*>(gp + 8 * PE * q + e));
+      const f32x4 b4 = to_f32(*reinterpret_cast<const typename Vec4<T>::type*>(bp + 8 * PE * q + e));
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        gm[q][e + t] = g4[t];
+        bt[q][e + t] = b4[t];
+      }
+    }
+}
+
+// Piece (PE values) number c / PE of a row into the fragment tile, rounded to T.
+template <typename T, int KS, int PE>
+__device__ __forceinline__ void put_piece(char* frag, int rb, int row, int piece, const float (&v)[PE]) {
+  if constexpr (PE == 8) {
+    f32x8 f;
+#pragma unroll
+    for (int t = 0; t < 8; ++t) f[t] = v[t];
+    FragLds<T, KS>::put(frag, rb, row, piece, from_f32<T>(f));
+  } else {
+    const typename Vec4<T>::type h = from_f32<T>(f32x4{v[0], v[1], v[2], v[3]});
+    char* d = frag + rb * FragLds<T, KS>::ROWBLOCK;
+    if constexpr (sizeof(T) == 2)   // half of a group's 16 bytes
+      *reinterpret_cast<typename Vec4<T>::type*>(d + (piece >> 1) * kPlanePitch + row * 16 + 8 * (piece & 1)) = h;
+    else
+      *reinterpret_cast<typename Vec4<T>::type*>(d + piece * kPlanePitch + row * 16) = h;
+  }
+}
+
+// The tile's rows, normalised, into LDS; the raw pieces stay in `raw` (row rb * 32 + 8 * wave + lane / 8).
+// off(r): element offset of row r of the tile.
+template <typename T, typename TZ, int KS, int RBW, typename Off>
+__device__ __forceinline__ void norm_rows(char* frag, const TZ* x, Off off, const T* gamma, const T* beta, float eps,
+                                          int wave, int lane,
+                                          typename RowPieces<TZ, KS>::V (&raw)[RBW][RowPieces<TZ, KS>::NP]) {
+  typedef RowPieces<TZ, KS> RP;
+  constexpr int PE = RP::PE, NP = RP::NP;
+  const int j = lane & 7, r8 = wave * 8 + (lane >> 3);
+#pragma unroll
+  for (int rb = 0; rb < RBW; ++rb) {
+    const TZ* rp = x + off(rb * 32 + r8) + PE * j;
+#pragma unroll
+    for (int q = 0; q < NP; ++q) raw[rb][q] = *reinterpret_cast<const typename RP::V*>(rp + 8 * PE * q);
+  }
+  float gm[NP][PE], bt[NP][PE];
+  load_affine_pieces<T, PE, NP>(gamma, beta, j, gm, bt);
+#pragma unroll
+  for (int rb = 0; rb < RBW; ++rb) {
+    float v[NP][PE];
+#pragma unroll
+    for (int q = 0; q < NP; ++q)
+#pragma unroll
+      for (int t = 0; t < PE; ++t) v[q][t] = to_f32(raw[rb][q][t]);
+    normalize_pieces<PE, NP>(v, gm, bt, eps);
+#pragma unroll
+    for (int q = 0; q < NP; ++q) put_piece<T, KS, PE>(frag, rb, r8, j + 8 * q, v[q]);
+  }
+}
+
+// The update of the tile's rows (T, [32 RBW][16 KS] at a pitch of kUpdPitch<KS>) added to the raw rows norm_rows() left
+// in registers (or stored as it is) and written in the same layout: whole lines.
+template <int KS> constexpr int kUpdPitch = 16 * KS + 8;
+template <typename T, typename TZ, int KS, int RBW, typename Off>
+__device__ __forceinline__ void store_rows(TZ* out, Off off, const T* upd, int wave, int lane, int add,
+                                           const typename RowPieces<TZ, KS>::V (&raw)[RBW][RowPieces<TZ, KS>::NP]) {
+  typedef RowPieces<TZ, KS> RP;
+  constexpr int PE = RP::PE, NP = RP::NP;
+  const int j = lane & 7, r8 = wave * 8 + (lane >> 3);
+#pragma unroll
+  for (int rb = 0; rb < RBW; ++rb) {
+    const int64_t o = off(rb * 32 + r8);
+    const T* up = upd + (rb * 32 + r8) * kUpdPitch<KS> + PE * j;
+    if (o >= 0) {
+#pragma unroll
+      for (int q = 0; q < NP; ++q) {
+        typename RP::V v;
+#pragma unroll
+        for (int e = 0; e < PE; e += 4) {
+          const f32x4 u = to_f32(*reinterpret_cast<const typename Vec4<T>::type*>(up + 8 * PE * q + e));
+#pragma unroll
+          for (int t = 0; t < 4; ++t) v[e + t] = from_f32<TZ>(add ? to_f32(raw[rb][q][e + t]) + u[t] : u[t]);
+        }
+        *reinterpret_cast<typename RP::V*>(out + o + PE * j + 8 * PE * q) = v;
+      }
+    }
+  }
+}
+
+// One 32 x 32 result tile (lane <-> row, register <-> column) into the update's tile.
+template <typename T, int KS>
+__device__ __forceinline__ void put_update(T* upd, int rb, int ob, const float (&vals)[16], int lane) {
+  T* d = upd + (rb * 32 + (lane & 31)) * kUpdPitch<KS> + ob * 32 + 4 * (lane >> 5);
+#pragma unroll
+  for (int qd = 0; qd < 4; ++qd)
+    *reinterpret_cast<typename Vec4<T>::type*>(d + 8 * qd) =
+        from_f32<T>(f32x4{vals[4 * qd], vals[4 * qd + 1], vals[4 * qd + 2], vals[4 * qd + 3]});
+}
+
+// Workgroups are dealt round-robin to the 8 XCDs: runs of four neighbouring tiles go to one XCD, whose L2
+// then sees both halves of the 128-byte lines that two tiles of 32 16-bit values share.
+__device__ __forceinline__ uint32_t xcd_run(uint32_t b, uint32_t n) {
+  constexpr uint32_t RUN = 4;
+  const uint32_t base = b / (8 * RUN) * (8 * RUN), o = b - base;
+  return base + 8 * RUN <= n ? base + (o & 7) * RUN + (o >> 3) : b;
+}
+
+// Which logical rows a tile of ROWS rows stands for.  linear: ROWS consecutive rows p = i * n + j (n is a multiple
+// of the 16-byte vector length, so that vectors of consecutive rows stay inside one i); otherwise ROWS
+// positions j of one i, the last tile of an i partial.
+struct TileRows {
+  int64_t p0;
+  int i0, j0, n;
+  int64_t n_rows;
+  bool linear;
+  __device__ __forceinline__ bool at(int r, int& i, int& j) const {
+    if (linear) {
+      const int64_t p = p0 + r;
+      const bool ok = p < n_rows;
+      const uint32_t pc = (uint32_t)(ok ? p : n_rows - 1);
+      i = pc / (uint32_t)n;
+      j = pc - i * (uint32_t)n;
+      return ok;
+    }
+    i = i0;
+    j = min(j0 + r, n - 1);
+    return j0 + r < n;
+  }
+};
+__device__ __forceinline__ TileRows tile_rows(int64_t tile, int rows, int n, int tiles_per_i) {
+  TileRows t;
+  t.n = n;
+  t.n_rows = (int64_t)n * n;
+  t.linear = tiles_per_i == 0;
+  t.p0 = tile * rows;
+  t.i0 = t.linear ? 0 : (int)((uint32_t)tile / (uint32_t)tiles_per_i);
+  t.j0 = t.linear ? 0 : ((int)tile - t.i0 * tiles_per_i) * rows;
+  return t;
+}
+
+struct ProjInParams {
+  const void* x;          // pair tensor; logical row (i, j) at i * si + j * sj
+  int64_t si, sj;
+  const void *gamma, *beta;
+  float eps;
+  const void* packed;     // weight fragments (pair_pack)
+  void* out[5];           // trimul_in: a, b; triattn_in: q, k, v^T, gate (or null), bias
+  const void* mask;       // trimul_in: value of (i, k) at i * mi + k * mk, or null
+  int64_t mi, mk;
+  int n, pitch, backward;
+  int tiles_per_i;        // triattn_in: 0 = linear tiles
+  int heads;
+  float q_scale;
+};
+
+}  // namespace
+
+// a, b[c][i][k] = mask * sigmoid(gate) * projection in the contraction's fragment order.  Tile: a patch of 4 * RBW
+// outer indices i x 8 inner indices k, which makes a row block's 32 values of one channel 64 contiguous bytes.
+template <typename T, typename TZ, int KS, int RBW>
+__global__ __launch_bounds__(kPpWaves * 64, (sizeof(T) == 2 && KS <= 8 ? 3 : 1)) void pp_trimul_in_kernel(ProjInParams p) {
+  typedef typename Vec8<T>::type V8;
+  typedef typename VecE<T>::type VE_t;
+  typedef Cfg<T> C;
+  constexpr int CPM = PpWidths<KS>::HIDDEN / 32;    // chunks (of 32 channels) per operand
+  constexpr int CHW = 2 * CPM / kPpWaves;           // chunks per wave
+  __shared__ __attribute__((aligned(16))) char frag[RBW * FragLds<T, KS>::ROWBLOCK];
+  __shared__ __attribute__((aligned(16))) T stage[kPpWaves][32 * C::PITCH];
+  __shared__ __attribute__((aligned(16))) float lmask[32 * RBW];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int g = lane >> 5;
+  const int n = p.n;
+  const uint32_t n_kb = (uint32_t)p.pitch >> 3, n_ip = (uint32_t)(n + 4 * RBW - 1) / (4 * RBW);
+  // Patches in the order of the memory rows they read, back to front behind a kernel that wrote the pair tensor
+  // front to back (the tail is what the memory-side cache still holds).
+  const uint32_t bx = xcd_run(blockIdx.x, gridDim.x), tile = p.backward ? gridDim.x - 1 - bx : bx;
+  int pi0, pk0;
+  if (p.backward) {   // incoming: the inner index is the slow one of z
+    const uint32_t kb = tile / n_ip;
+    pk0 = kb * 8;
+    pi0 = (tile - kb * n_ip) * (4 * RBW);
+  } else {
+    const uint32_t ip = tile / n_kb;
+    pi0 = ip * (4 * RBW);
+    pk0 = (tile - ip * n_kb) * 8;
+  }
+  const T* packed = (const T*)p.packed;
+  V8 w[2][KS];
+  auto load_w = [&](int ch) {
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int kk = 0; kk < KS; ++kk) w[t][kk] = packed_frag<T>(packed, (ch * 2 + t) * KS + kk, lane);
+  };
+  typename RowPieces<TZ, KS>::V raw[RBW][RowPieces<TZ, KS>::NP];
+  norm_rows<T, TZ, KS, RBW>(
+      frag, (const TZ*)p.x,
+      [&](int r) {
+        const int i = min(pi0 + (r >> 3), n - 1), k = min(pk0 + (r & 7), n - 1);
+        return i * p.si + k * p.sj;
+      },
+      (const T*)p.gamma, (const T*)p.beta, p.eps, wave, lane, raw);
+  load_w(wave * CHW);
+  if (threadIdx.x < 32 * RBW) {
+    const int i = min(pi0 + (int)(threadIdx.x >> 3), n - 1), k = pk0 + (int)(threadIdx.x & 7);
+    float mv = 1.0f;
+    if (p.mask) mv = to_f32(((const T*)p.mask)[i * p.mi + min(k, n - 1) * p.mk]);
+    lmask[threadIdx.x] = k < n ? mv : 0.0f;   // (the contraction relies on zeros between n and the pitch)
+  }
+  __syncthreads();
+
+  T* st = stage[wave];
+  const int n_rb = (n + 31) >> 5, n_ks = p.pitch >> 4;
+  // this lane's vector of row block 0 inside a channel block's planes
+  uint32_t rel[C::NPASS];
+#pragma unroll
+  for (int ps = 0; ps < C::NPASS; ++ps) {
+    int chn, r0;
+    stage_coord<T>(ps, lane, chn, r0);
+    const int i = pi0 + (r0 >> 3);
+    rel[ps] = (uint32_t)(trimul_frag_offset(chn, i >> 5, pk0 >> 4, n_rb, n_ks) + ((pk0 >> 3) & 1) * 256 + (i & 31) * 8 + (r0 & 7));
+  }
+#pragma unroll
+  for (int c = 0; c < CHW; ++c) {
+    const int ch = wave * CHW + c;
+    T* outp = (T*)p.out[ch / CPM] + trimul_frag_offset((ch % CPM) * 32, 0, 0, n_rb, n_ks);
+#pragma unroll
+    for (int rb = 0; rb < RBW; ++rb) {
+      f32x16 acc[2];
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[0][r] = acc[1][r] = 0.0f;
+#pragma unroll
+      for (int kk = 0; kk < KS; ++kk) {
+        const V8 xv = FragLds<T, KS>::get(frag, rb, kk, lane);
+        mma32(acc[0], xv, w[0][kk]);   // lane <-> channel, register <-> row
+        mma32(acc[1], xv, w[1][kk]);
+      }
+      if (rb == RBW - 1 && c + 1 < CHW) load_w(ch + 1);
+      float vals[16];
+#pragma unroll
+      for (int qd = 0; qd < 4; ++qd) {
+        const f32x4 m4 = *reinterpret_cast<const f32x4*>(&lmask[rb * 32 + 8 * qd + 4 * g]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int r = 4 * qd + e;
+          vals[r] = m4[e] * sigmoidf_fast(acc[1][r]) * acc[0][r];
+        }
+      }
+      wave_lds_sync();
+      stage_put<T>(st, vals, lane);
+      wave_lds_sync();
+      // row block rb: outer indices 4 rb .. 4 rb + 3 further on; a patch of 4 RBW outer indices lies in one block of 32
+#pragma unroll
+      for (int ps = 0; ps < C::NPASS; ++ps) {
+        int chn, r0;
+        stage_coord<T>(ps, lane, chn, r0);
+        *reinterpret_cast<VE_t*>(outp + rel[ps] + rb * 32) = stage_get_vec<T>(st, chn, r0);
+      }
+    }
+  }
+}
+
+// q (scaled), K, V^T, triangle bias and (GATE) sigmoid(gate) in the attention core's layouts.
+template <typename T, typename TZ, int KS, int RBW, bool GATE>
+__global__ __launch_bounds__(kPpWaves * 64, (sizeof(T) == 2 && KS <= 8 ? 3 : 1)) void pp_triattn_in_kernel(ProjInParams p) {
+  typedef typename Vec8<T>::type V8;
+  typedef typename VecE<T>::type VE_t;
+  typedef Cfg<T> C;
+  constexpr int HP = PpWidths<KS>::HEADS / 2;            // pairs of heads
+  constexpr int NPAIR = (GATE ? 4 : 3) * HP + 1;         // q, k, v (, gate): HP pairs of tiles each; the bias: one tile
+  __shared__ __attribute__((aligned(16))) char frag[RBW * FragLds<T, KS>::ROWBLOCK];
+  __shared__ __attribute__((aligned(16))) T stage[kPpWaves][2][32 * C::PITCH];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int n = p.n;
+  const int64_t n_rows = (int64_t)n * n;
+  const uint32_t bx = xcd_run(blockIdx.x, gridDim.x);
+  const int64_t tile = p.backward ? gridDim.x - 1 - bx : bx;
+  const TileRows tr = tile_rows(tile, 32 * RBW, n, p.tiles_per_i);
+  const T* packed = (const T*)p.packed;
+  V8 w[2][KS];
+  auto load_w = [&](int pair) {   // pair -> tiles 2 pair, 2 pair + 1 (the bias' tile twice)
+    const int t0 = pair < NPAIR - 1 ? 2 * pair : 8 * HP, t1 = pair < NPAIR - 1 ? t0 + 1 : t0;
+#pragma unroll
+    for (int kk = 0; kk < KS; ++kk) {
+      w[0][kk] = packed_frag<T>(packed, t0 * KS + kk, lane);
+      w[1][kk] = packed_frag<T>(packed, t1 * KS + kk, lane);
+    }
+  };
+  typename RowPieces<TZ, KS>::V raw[RBW][RowPieces<TZ, KS>::NP];
+  norm_rows<T, TZ, KS, RBW>(
+      frag, (const TZ*)p.x,
+      [&](int r) {
+        int i, j;
+        tr.at(r, i, j);
+        return i * p.si + j * p.sj;
+      },
+      (const T*)p.gamma, (const T*)p.beta, p.eps, wave, lane, raw);
+  load_w(wave);
+  __syncthreads();
+
+  const int key_tiles = p.pitch >> 6, q_blocks = (n + 31) >> 5;
+  const int64_t head_plane = (int64_t)n * key_tiles * kAttnTileElems;
+#pragma unroll 1
+  for (int pair = wave; pair < NPAIR; pair += kPpWaves) {
+    const int which = pair < NPAIR - 1 ? pair / HP : 4;   // 0 q, 1 k, 2 v, 3 gate, 4 bias
+    const int h0 = (pair % HP) * 2;
+#pragma unroll
+    for (int rb = 0; rb < RBW; ++rb) {
+      f32x16 acc[2];
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[0][r] = acc[1][r] = 0.0f;
+      if (which == 2 || which == 4) {
+#pragma unroll
+        for (int kk = 0; kk < KS; ++kk) {
+          const V8 xv = FragLds<T, KS>::get(frag, rb, kk, lane);
+          mma32(acc[0], xv, w[0][kk]);   // lane <-> channel, register <-> row
+          mma32(acc[1], xv, w[1][kk]);
+        }
+      } else {
+#pragma unroll
+        for (int kk = 0; kk < KS; ++kk) {
+          const V8 xv = FragLds<T, KS>::get(frag, rb, kk, lane);
+          mma32(acc[0], w[0][kk], xv);   // lane <-> row, register <-> channel
+          mma32(acc[1], w[1][kk], xv);
+        }
+      }
+      if (rb == RBW - 1 && pair + kPpWaves < NPAIR) load_w(pair + kPpWaves);
+      wave_lds_sync();
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        float vals[16];
+        if (which == 0) {
+#pragma unroll
+          for (int r = 0; r < 16; ++r) vals[r] = to_f32(from_f32<T>(acc[t][r])) * p.q_scale;
+        } else if (which == 4) {
+#pragma unroll
+          for (int r = 0; r < 16; ++r) vals[r] = acc[t][r] * 1.4426950408889634f;   // the core works in log2 units
+        } else if (GATE && which == 3) {
+#pragma unroll
+          for (int r = 0; r < 16; ++r) vals[r] = sigmoidf_fast(acc[t][r]);
+        } else {
+#pragma unroll
+          for (int r = 0; r < 16; ++r) vals[r] = acc[t][r];
+        }
+        stage_put<T>(stage[wave][t], vals, lane);
+      }
+      wave_lds_sync();
+      if (which == 2 || which == 4) {
+        // vectors of VE consecutive keys of one i
+        const int v0 = (lane % C::LPM) * C::VE;
+        int i, j;
+        const bool ok = tr.at(rb * 32 + v0, i, j);
+        if (which == 2) {
+          T* outp = (T*)p.out[2] + attn_v_offset(0, i, j, 0, n, key_tiles);
+#pragma unroll
+          for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int ps = 0; ps < C::NPASS; ++ps) {
+              int chn, r0;
+              stage_coord<T>(ps, lane, chn, r0);
+              if (ok) *reinterpret_cast<VE_t*>(outp + (h0 + t) * head_plane + chn * 8) = stage_get_vec<T>(stage[wave][t], chn, r0);
+            }
+        } else {
+          T* outp = (T*)p.out[4];
+#pragma unroll
+          for (int ps = 0; ps < C::NPASS; ++ps) {
+            int chn, r0;
+            stage_coord<T>(ps, lane, chn, r0);
+            if (ok && chn < p.heads)
+              *reinterpret_cast<VE_t*>(outp + attn_b_offset(chn, i, j, q_blocks, key_tiles)) = stage_get_vec<T>(stage[wave][0], chn, r0);
+          }
+        }
+      } else {
+#pragma unroll
+        for (int ps = 0; ps < C::NPASS; ++ps) {
+          int mj, m0;
+          stage_coord<T>(ps, lane, mj, m0);
+          int i, j;
+          const bool ok = tr.at(rb * 32 + mj, i, j);
+          if (which == 1) {
+            T* outp = (T*)p.out[1] + attn_k_offset(0, i, j, m0, n, key_tiles);
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+              if (ok) *reinterpret_cast<VE_t*>(outp + (h0 + t) * head_plane) = stage_get_vec<T>(stage[wave][t], mj, m0);
+          } else {
+            T* outp = (T*)(which == 0 ? p.out[0] : p.out[3]) + ((int64_t)i * n + j) * 32 + m0;
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+              if (ok) *reinterpret_cast<VE_t*>(outp + (int64_t)(h0 + t) * n_rows * 32) = stage_get_vec<T>(stage[wave][t], mj, m0);
+          }
+        }
+      }
+    }
+  }
+}
+
+namespace {
+struct ProjOutParams {
+  const void* z;          // pair tensor: LayerNorm input and residual; row (i, j) at i * si + j * sj (also of out)
+  int64_t si, sj;
+  const void *gamma, *beta;     // LayerNorm of z (trimul_out; triattn_out with the gate formed here)
+  const void *gamma2, *beta2;   // trimul_out: LayerNorm of the triangle product
+  float eps;
+  const void* packed;     // weight fragments of this stage
+  const void* packed_g;   // triattn_out: fragments of the gate's weights
+  const void* x;          // trimul_out: triangle product [hidden][n][ldx]; triattn_out: attention output [heads][n * n][32]
+  int ldx;
+  void* out;
+  int n, add_residual, tiles_per_i;
+};
+}  // namespace
+
+// out = [z +] (W_z LN_out(x)) * sigmoid(W_g LN_in(z)); out may be z.
+template <typename T, typename TZ, int KS, int RBW>
+__global__ __launch_bounds__(kPpWaves * 64, (sizeof(T) == 2 && KS <= 8 ? 3 : 1)) void pp_trimul_out_kernel(ProjOutParams p) {
+  typedef typename Vec8<T>::type V8;
+  typedef typename VecE<T>::type VE_t;
+  typedef Cfg<T> C;
+  constexpr int SL = PpWidths<KS>::SL, HIDDEN = PpWidths<KS>::HIDDEN, NOB = KS / 2;
+  constexpr int XP = 32 * RBW + 4;   // pitch of the triangle product's tile (elements)
+  constexpr size_t kXt = sizeof(T) * HIDDEN * XP, kUpd = sizeof(T) * 32 * RBW * kUpdPitch<KS>;
+  __shared__ __attribute__((aligned(16))) char frag[RBW * FragLds<T, KS>::ROWBLOCK];
+  __shared__ __attribute__((aligned(16))) char frag2[RBW * FragLds<T, SL>::ROWBLOCK];
+  __shared__ __attribute__((aligned(16))) char scratch[kXt > kUpd ? kXt : kUpd];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int n = p.n;
+  const TileRows tr = tile_rows(xcd_run(blockIdx.x, gridDim.x), 32 * RBW, n, p.tiles_per_i);
+  const T* packed = (const T*)p.packed;
+
+  // the triangle product's rows of every channel: vectors of VE rows
+  constexpr int VPC = 32 * RBW / C::VE, NV = HIDDEN * VPC / (kPpWaves * 64);
+  const int v0 = (threadIdx.x % VPC) * C::VE, c0 = threadIdx.x / VPC;
+  VE_t xv[NV];
+  {
+    int i, j;
+    tr.at(v0, i, j);
+    // (a tile past the end of a plane re-reads its last vector: those rows are not stored)
+    const int64_t off = min((int64_t)i * p.ldx + j, (int64_t)n * p.ldx - C::VE) & ~(int64_t)(C::VE - 1);
+    const T* src = (const T*)p.x + off;
+    const int64_t plane = (int64_t)n * p.ldx;
+#pragma unroll
+    for (int q = 0; q < NV; ++q) xv[q] = *reinterpret_cast<const VE_t*>(src + (c0 + q * (kPpWaves * 64 / VPC)) * plane);
+  }
+  auto z_row = [&](int r) {
+    int i, j;
+    const bool ok = tr.at(r, i, j);
+    const int64_t o = i * p.si + j * p.sj;
+    return ok ? o : -1;
+  };
+  typename RowPieces<TZ, KS>::V raw[RBW][RowPieces<TZ, KS>::NP];
+  norm_rows<T, TZ, KS, RBW>(
+      frag, (const TZ*)p.z, [&](int r) { return max(z_row(r), (int64_t)0); }, (const T*)p.gamma, (const T*)p.beta, p.eps,
+      wave, lane, raw);
+  T* xt = reinterpret_cast<T*>(scratch);
+#pragma unroll
+  for (int q = 0; q < NV; ++q) {
+    u32x2* d = reinterpret_cast<u32x2*>(xt + (c0 + q * (kPpWaves * 64 / VPC)) * XP + v0);
+    const u32x2* s = reinterpret_cast<const u32x2*>(&xv[q]);
+    d[0] = s[0];
+    d[1] = s[1];
+  }
+  __syncthreads();
+  {
+    typedef RowPieces<T, SL> RP;
+    constexpr int PE = RP::PE, NP = RP::NP;
+    const int j = lane & 7, r8 = wave * 8 + (lane >> 3);
+    float gm[NP][PE], bt[NP][PE];
+    load_affine_pieces<T, PE, NP>((const T*)p.gamma2, (const T*)p.beta2, j, gm, bt);
+#pragma unroll
+    for (int rb = 0; rb < RBW; ++rb) {
+      float v[NP][PE];
+#pragma unroll
+      for (int q = 0; q < NP; ++q)
+#pragma unroll
+        for (int t = 0; t < PE; ++t) v[q][t] = to_f32(xt[(PE * (j + 8 * q) + t) * XP + rb * 32 + r8]);
+      normalize_pieces<PE, NP>(v, gm, bt, p.eps);
+#pragma unroll
+      for (int q = 0; q < NP; ++q) put_piece<T, SL, PE>(frag2, rb, r8, j + 8 * q, v[q]);
+    }
+  }
+  V8 wz[SL], wg[KS];
+  auto load_w = [&](int ob) {
+#pragma unroll
+    for (int kk = 0; kk < SL; ++kk) wz[kk] = packed_frag<T>(packed, ob * (SL + KS) + kk, lane);
+#pragma unroll
+    for (int kk = 0; kk < KS; ++kk) wg[kk] = packed_frag<T>(packed, ob * (SL + KS) + SL + kk, lane);
+  };
+  if (wave < NOB) load_w(wave);
+  __syncthreads();   // both operand tiles are complete, and the product's tile has been read
+  T* upd = reinterpret_cast<T*>(scratch);
+#pragma unroll
+  for (int ob = wave; ob < NOB; ob += kPpWaves) {
+#pragma unroll
+    for (int rb = 0; rb < RBW; ++rb) {
+      f32x16 az, ag;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) az[r] = ag[r] = 0.0f;
+#pragma unroll
+      for (int kk = 0; kk < SL; ++kk) mma32(az, wz[kk], FragLds<T, SL>::get(frag2, rb, kk, lane));
+#pragma unroll
+      for (int kk = 0; kk < KS; ++kk) mma32(ag, wg[kk], FragLds<T, KS>::get(frag, rb, kk, lane));
+      if (rb == RBW - 1 && ob + kPpWaves < NOB) load_w(ob + kPpWaves);
+      float vals[16];
+#pragma unroll
+      for (int r = 0; r < 16; ++r)   // linear_z's output rounded to T, times the gate, rounded to T
+        vals[r] = to_f32(from_f32<T>(az[r])) * sigmoidf_fast(ag[r]);
+      put_update<T, KS>(upd, rb, ob, vals, lane);
+    }
+  }
+  __syncthreads();
+  store_rows<T, TZ, KS, RBW>((TZ*)p.out, z_row, upd, wave, lane, p.add_residual, raw);
+}
+
+// out = [z +] W_o (gate * o): GATE: gate = sigmoid(W_g LN(z)) formed here (16-bit arithmetic, rows of 128 channels,
+// 4 heads: wave = head), otherwise o arrives gated.  out may be z.
+template <typename T, typename TZ, int KS, bool GATE, int RBW>
+__global__ __launch_bounds__(kPpWaves * 64, (sizeof(T) == 2 && KS <= 8 ? 3 : 1)) void pp_triattn_out_kernel(ProjOutParams p) {
+  typedef typename Vec8<T>::type V8;
+  constexpr int SL = PpWidths<KS>::SL, NOB = KS / 2;
+  static_assert(!GATE || (KS == 8 && sizeof(T) == 2), "gate formed here: rows of 128 channels, 16-bit arithmetic");
+  constexpr size_t kFrag = GATE ? RBW * FragLds<T, KS>::ROWBLOCK : 16, kUpd = sizeof(T) * 32 * RBW * kUpdPitch<KS>;
+  __shared__ __attribute__((aligned(16))) char scratch[kFrag > kUpd ? kFrag : kUpd];   // the normalised rows, then the update
+  __shared__ __attribute__((aligned(16))) char fo[RBW * FragLds<T, SL>::ROWBLOCK];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int n = p.n, nl = lane & 31, g = lane >> 5;
+  const int64_t n_rows = (int64_t)n * n;
+  const TileRows tr = tile_rows(xcd_run(blockIdx.x, gridDim.x), 32 * RBW, n, 0);
+  const T* packed = (const T*)p.packed;
+  V8 w[SL];
+  auto load_w = [&](int ob) {
+#pragma unroll
+    for (int kk = 0; kk < SL; ++kk) w[kk] = packed_frag<T>(packed, ob * SL + kk, lane);
+  };
+  // this wave's share of the attention output: heads wave, wave + 4, .. as fragments
+  constexpr int HPW = PpWidths<KS>::HEADS / kPpWaves;
+  V8 of[RBW][HPW][2];
+#pragma unroll
+  for (int rb = 0; rb < RBW; ++rb) {
+    const int64_t pr = min(tr.p0 + rb * 32 + nl, n_rows - 1);
+#pragma unroll
+    for (int q = 0; q < HPW; ++q)
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+        of[rb][q][u] = load8<T>((const T*)p.x + ((int64_t)(wave + 4 * q) * n_rows + pr) * 32 + 16 * u + 8 * g);
+  }
+  auto z_row = [&](int r) {
+    int i, j;
+    const bool ok = tr.at(r, i, j);
+    const int64_t o = i * p.si + j * p.sj;
+    return ok ? o : -1;
+  };
+  auto z_row0 = [&](int r) { return max(z_row(r), (int64_t)0); };
+  typename RowPieces<TZ, KS>::V raw[RBW][RowPieces<TZ, KS>::NP];
+  if constexpr (GATE) {
+    V8 wg[KS];
+#pragma unroll
+    for (int kk = 0; kk < KS; ++kk) wg[kk] = packed_frag<T>((const T*)p.packed_g, wave * KS + kk, lane);
+    norm_rows<T, TZ, KS, RBW>(scratch, (const TZ*)p.z, z_row0, (const T*)p.gamma, (const T*)p.beta, p.eps, wave, lane, raw);
+    load_w(wave);
+    __syncthreads();
+#pragma unroll
+    for (int rb = 0; rb < RBW; ++rb) {
+      f32x16 ag;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) ag[r] = 0.0f;
+#pragma unroll
+      for (int kk = 0; kk < KS; ++kk) mma32(ag, wg[kk], FragLds<T, KS>::get(scratch, rb, kk, lane));
+      // (weight rows packed so that registers 8 u + t are the channels 16 u + 8 g + t of the lane's own fragments;
+      // gate and gated output rounded to T like the reference's sigmoid(linear_g(x)) and o * g)
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        const f32x8 ov = to_f32(of[rb][0][u]);
+        f32x8 gated;
+#pragma unroll
+        for (int t = 0; t < 8; ++t) gated[t] = ov[t] * to_f32(from_f32<T>(sigmoidf_fast(ag[8 * u + t])));
+        of[rb][0][u] = from_f32<T>(gated);
+      }
+    }
+  } else {
+    if (wave < NOB) load_w(wave);
+    if (p.add_residual) {
+      typedef RowPieces<TZ, KS> RP;
+#pragma unroll
+      for (int rb = 0; rb < RBW; ++rb) {
+        const TZ* rp = (const TZ*)p.z + z_row0(rb * 32 + wave * 8 + (lane >> 3)) + RP::PE * (lane & 7);
+#pragma unroll
+        for (int q = 0; q < RP::NP; ++q) raw[rb][q] = *reinterpret_cast<const typename RP::V*>(rp + 8 * RP::PE * q);
+      }
+    }
+  }
+#pragma unroll
+  for (int rb = 0; rb < RBW; ++rb)
+#pragma unroll
+    for (int q = 0; q < HPW; ++q)
+#pragma unroll
+      for (int u = 0; u < 2; ++u) FragLds<T, SL>::put(fo, rb, nl, 2 * (2 * (wave + 4 * q) + u) + g, of[rb][q][u]);
+  __syncthreads();   // (and the normalised rows have been read)
+  T* upd = reinterpret_cast<T*>(scratch);
+#pragma unroll
+  for (int ob = wave; ob < NOB; ob += kPpWaves) {
+#pragma unroll
+    for (int rb = 0; rb < RBW; ++rb) {
+      f32x16 acc;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
+#pragma unroll
+      for (int kk = 0; kk < SL; ++kk) mma32(acc, w[kk], FragLds<T, SL>::get(fo, rb, kk, lane));
+      if (rb == RBW - 1 && ob + kPpWaves < NOB) load_w(ob + kPpWaves);
+      float vals[16];
+#pragma unroll
+      for (int r = 0; r < 16; ++r) vals[r] = acc[r];
+      put_update<T, KS>(upd, rb, ob, vals, lane);   // (rounded to T, as the module's output is)
+    }
+  }
+  __syncthreads();
+  store_rows<T, TZ, KS, RBW>((TZ*)p.out, z_row, upd, wave, lane, p.add_residual, raw);
+}
+
+// ---------------------------------------------------------------------------
+// Weight packing: every 32-row tile of the matrices as KS (or more) fragments, one lane's 8
+// elements in 16-byte pieces [fragment][piece][lane].
+// ---------------------------------------------------------------------------
+namespace {
+struct PackTile {
+  const void* w;
+  int row0, n_out, ldw, ksteps, frag0, perm;
+};
+constexpr int kMaxPackTiles = 52;
+struct PackList {
+  PackTile t[kMaxPackTiles];
+};
+}  // namespace
+
+template <typename T>
+__global__ __launch_bounds__(256) void pair_pack_kernel(PackList list, T* __restrict__ packed) {
+  const PackTile t = list.t[blockIdx.x];
+  const int lane = threadIdx.x & 63;
+  int m = lane & 31;
+  if (t.perm) m = 16 * (m >> 4) + 8 * ((m >> 2) & 1) + 4 * ((m >> 3) & 1) + (m & 3);
+  const T* row = (const T*)t.w + (int64_t)min(t.row0 + m, t.n_out - 1) * t.ldw + 8 * (lane >> 5);
+  constexpr int PIECES = (int)sizeof(T) / 2;
+  for (int kk = threadIdx.x >> 6; kk < t.ksteps; kk += 4) {
+    typename Vec8<T>::type v;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = row[16 * kk + e];
+    const u32x4_t* s = reinterpret_cast<const u32x4_t*>(&v);
+    u32x4_t* d = reinterpret_cast<u32x4_t*>(packed + (int64_t)(t.frag0 + kk) * kFragElems) + lane;
+#pragma unroll
+    for (int pc = 0; pc < PIECES; ++pc) d[pc * kWave] = s[pc];
+  }
+}
+
+int64_t pp_trimul_packed_elems(int c_z, int hidden) {
+  return 5 * (int64_t)c_z * hidden + (int64_t)c_z * c_z;
+}
+
+template <typename T>
+int pp_trimul_pack(const void* w_ap, const void* w_ag, const void* w_bp, const void* w_bg, const void* w_z,
+                   const void* w_g, void* packed, int c_z, int hidden, hipStream_t stream) {
+  PackList l;
+  int nt = 0, f = 0;
+  const int ks = c_z / 16, sl = hidden / 16;
+  for (int op = 0; op < 2; ++op)
+    for (int cb = 0; cb < hidden / 32; ++cb)
+      for (int t = 0; t < 2; ++t) {
+        l.t[nt++] = PackTile{op ? (t ? w_bg : w_bp) : (t ? w_ag : w_ap), 32 * cb, hidden, c_z, ks, f, 0};
+        f += ks;
+      }
+  for (int ob = 0; ob < c_z / 32; ++ob) {
+    l.t[nt++] = PackTile{w_z, 32 * ob, c_z, hidden, sl, f, 0};
+    l.t[nt++] = PackTile{w_g, 32 * ob, c_z, c_z, ks, f + sl, 0};
+    f += sl + ks;
+  }
+  pair_pack_kernel<T><<<dim3(nt), dim3(256), 0, stream>>>(l, (T*)packed);
+  return 0;
+}
+
+int64_t pp_triattn_packed_elems(int c_z, int heads) {
+  return (int64_t)(4 * heads + 1) * 32 * c_z + (int64_t)c_z * heads * 32;
+}
+
+template <typename T>
+int pp_triattn_pack(const void* w_q, const void* w_k, const void* w_v, const void* w_g, const void* w_b,
+                    const void* w_o, void* packed, int c_z, int heads, hipStream_t stream) {
+  PackList l;
+  int nt = 0, f = 0;
+  const int ks = c_z / 16, sl = heads * 2;
+  // (the gate formed in the output kernel: its rows permuted, see pp_triattn_out_kernel)
+  const bool late = pp_late_gate(c_z, heads, sizeof(T) == 2);
+  const void* m[4] = {w_q, w_k, w_v, w_g};
+  for (int which = 0; which < 4; ++which)
+    for (int h = 0; h < heads; ++h) {
+      l.t[nt++] = PackTile{m[which], 32 * h, heads * 32, c_z, ks, f, which == 3 && late};
+      f += ks;
+    }
+  l.t[nt++] = PackTile{w_b, 0, heads, c_z, ks, f, 0};
+  f += ks;
+  for (int ob = 0; ob < c_z / 32; ++ob) {
+    l.t[nt++] = PackTile{w_o, 32 * ob, c_z, heads * 32, sl, f, 0};
+    f += sl;
+  }
+  pair_pack_kernel<T><<<dim3(nt), dim3(256), 0, stream>>>(l, (T*)packed);
+  return 0;
+}
+
+// ---------------------------------------------------------------------------
+// launchers
+// ---------------------------------------------------------------------------
+// Row blocks (of 32 rows) per workgroup, by the launch's number of rows.  More of them share the
+// weights a wave fetches; fewer leave more workgroups and more of them per compute unit.  Lines from
+// sweeps over n (us per launch, fp32 rows; c = channels):
+//   trimul_in   c = 128: 1 / 2 at n = 128: 8.0 / 8.5, at 192: 14.5 / 13.8; 2 / 4 at 387: 41 / 43, 512: 62 / 61,
+//               768: 184 / 157; c = 256: 1 / 2 at 128: 23 / 18, 2 / 4 at 256: 69 / 54, 600: 373 / 295
+//   triattn_in  c = 128: as trimul_in for 1 / 2; 2 / 4 at 768: 180 / 181; c = 64: 2 / 4 at 512: 98 / 88;
+//               c = 256: 1 / 2 at 128: 29 / 25, 2 / 4 at 600: 356 / 434 (registers)
+//   trimul_out  c = 128: 1 / 2 at 387: 41 / 43, 512: 68 / 65, 768: 186 / 162; c = 64 at 512: 39 / 43; c = 256 at 600: 292 / 352
+//   triattn_out c = 128: 1 / 2 at 256: 17.4 / 17.4, 387: 34.8 / 33.7, 768: 170 / 140; c = 64, 256: no gain
+// 32-bit arithmetic: one (twice the registers per fragment).
+static int in_row_blocks(int64_t rows, int ks, bool attention) {
+  if (rows < (ks > 8 ? 96 * 96 : 160 * 160)) return 1;
+  const int64_t four = attention ? (ks == 4 ? 400 * 400 : INT64_MAX) : (ks > 8 ? 200 * 200 : 448 * 448);
+  return rows >= four ? 4 : 2;
+}
+static int out_row_blocks(int64_t rows, int ks, bool attention) {
+  return ks == 8 && rows >= (attention ? 320 * 320 : 448 * 448) ? 2 : 1;
+}
+
+template <typename T, typename TZ, int KS>
+static int pp_trimul_in_ks(ProjInParams p, hipStream_t stream) {
+  const int rbw = sizeof(T) == 2 ? in_row_blocks((int64_t)p.n * p.n, KS, false) : 1;
+  const dim3 grid((unsigned)((p.n + 4 * rbw - 1) / (4 * rbw)) * (unsigned)(p.pitch / 8)), block(kPpWaves * 64);
+  if constexpr (sizeof(T) == 2) {
+    if (rbw == 4) {
+      pp_trimul_in_kernel<T, TZ, KS, 4><<<grid, block, 0, stream>>>(p);
+      return 0;
+    }
+    if (rbw == 2) {
+      pp_trimul_in_kernel<T, TZ, KS, 2><<<grid, block, 0, stream>>>(p);
+      return 0;
+    }
+  }
+  pp_trimul_in_kernel<T, TZ, KS, 1><<<grid, block, 0, stream>>>(p);
+  return 0;
+}
+
+template <typename T, typename TZ>
+int pp_trimul_in(const void* z, const void* mask, const void* ln_w, const void* ln_b, const void* packed, void* a,
+                 void* b, int n, int c_z, int k_pitch, int incoming, float eps, hipStream_t stream) {
+  ProjInParams p = {};
+  p.x = z;
+  p.si = incoming ? c_z : (int64_t)n * c_z;
+  p.sj = incoming ? (int64_t)n * c_z : c_z;
+  p.gamma = ln_w;
+  p.beta = ln_b;
+  p.eps = eps;
+  p.packed = packed;
+  p.out[0] = a;
+  p.out[1] = b;
+  p.mask = mask;
+  p.mi = incoming ? 1 : n;
+  p.mk = incoming ? n : 1;
+  p.n = n;
+  p.pitch = k_pitch;
+  p.backward = incoming != 0;
+  if (c_z == 64) return pp_trimul_in_ks<T, TZ, 4>(p, stream);
+  if (c_z == 256) {
+    if constexpr (sizeof(T) == 2) return pp_trimul_in_ks<T, TZ, 16>(p, stream);
+    else return -1;
+  }
+  return pp_trimul_in_ks<T, TZ, 8>(p, stream);
+}
+
+template <typename T, typename TZ, int KS, bool GATE>
+static int pp_triattn_in_ks(ProjInParams p, hipStream_t stream) {
+  const int rbw = sizeof(T) == 2 ? in_row_blocks((int64_t)p.n * p.n, KS, true) : 1;
+  const int rows = 32 * rbw;
+  p.tiles_per_i = p.n % Cfg<T>::VE == 0 ? 0 : (p.n + rows - 1) / rows;
+  const int64_t tiles = p.tiles_per_i ? (int64_t)p.n * p.tiles_per_i : ((int64_t)p.n * p.n + rows - 1) / rows;
+  const dim3 grid((unsigned)tiles), block(kPpWaves * 64);
+  if constexpr (sizeof(T) == 2) {
+    if constexpr (KS == 4) {
+      if (rbw == 4) {
+        pp_triattn_in_kernel<T, TZ, KS, 4, GATE><<<grid, block, 0, stream>>>(p);
+        return 0;
+      }
+    }
+    if (rbw == 2) {
+      pp_triattn_in_kernel<T, TZ, KS, 2, GATE><<<grid, block, 0, stream>>>(p);
+      return 0;
+    }
+  }
+  pp_triattn_in_kernel<T, TZ, KS, 1, GATE><<<grid, block, 0, stream>>>(p);
+  return 0;
+}
+
+template <typename T, typename TZ>
+int pp_triattn_in(const void* z, const void* ln_w, const void* ln_b, const void* packed, void* q, void* k, void* vt,
+                  void* g, void* tri_bias, int n, int c_z, int heads, int key_pitch, int transposed, float eps,
+                  hipStream_t stream) {
+  ProjInParams p = {};
+  p.x = z;
+  p.si = transposed ? c_z : (int64_t)n * c_z;
+  p.sj = transposed ? (int64_t)n * c_z : c_z;
+  p.gamma = ln_w;
+  p.beta = ln_b;
+  p.eps = eps;
+  p.packed = packed;
+  p.out[0] = q; p.out[1] = k; p.out[2] = vt; p.out[3] = g; p.out[4] = tri_bias;
+  p.n = n;
+  p.pitch = key_pitch;
+  p.backward = 1;
+  p.heads = heads;
+  p.q_scale = 1.4426950408889634f / sqrtf(32.0f);   // log2(e) / sqrt(d), see triattn.hip
+  if (c_z == 64) return pp_triattn_in_ks<T, TZ, 4, true>(p, stream);
+  if (c_z == 256) {
+    if constexpr (sizeof(T) == 2) return pp_triattn_in_ks<T, TZ, 16, true>(p, stream);
+    else return -1;
+  }
+  if constexpr (sizeof(T) == 2) return pp_triattn_in_ks<T, TZ, 8, false>(p, stream);
+  else return pp_triattn_in_ks<T, TZ, 8, true>(p, stream);
+}
+
+template <typename T, typename TZ, int KS>
+static int pp_trimul_out_ks(ProjOutParams p, hipStream_t stream) {
+  const int rbw = sizeof(T) == 2 ? out_row_blocks((int64_t)p.n * p.n, KS, false) : 1, rows = 32 * rbw;
+  p.tiles_per_i = p.ldx == p.n && p.n % Cfg<T>::VE == 0 ? 0 : (p.n + rows - 1) / rows;
+  const int64_t tiles = p.tiles_per_i ? (int64_t)p.n * p.tiles_per_i : ((int64_t)p.n * p.n + rows - 1) / rows;
+  const dim3 grid((unsigned)tiles), block(kPpWaves * 64);
+  if constexpr (sizeof(T) == 2 && KS == 8) {
+    if (rbw == 2) {
+      pp_trimul_out_kernel<T, TZ, KS, 2><<<grid, block, 0, stream>>>(p);
+      return 0;
+    }
+  }
+  pp_trimul_out_kernel<T, TZ, KS, 1><<<grid, block, 0, stream>>>(p);
+  return 0;
+}
+
+template <typename T, typename TZ, int KS, bool GATE>
+static int pp_triattn_out_ks(const ProjOutParams& p, hipStream_t stream) {
+  const int rbw = sizeof(T) == 2 ? out_row_blocks((int64_t)p.n * p.n, KS, true) : 1, rows = 32 * rbw;
+  const dim3 grid((unsigned)(((int64_t)p.n * p.n + rows - 1) / rows)), block(kPpWaves * 64);
+  if constexpr (sizeof(T) == 2 && KS == 8) {
+    if (rbw == 2) {
+      pp_triattn_out_kernel<T, TZ, KS, GATE, 2><<<grid, block, 0, stream>>>(p);
+      return 0;
+    }
+  }
+  pp_triattn_out_kernel<T, TZ, KS, GATE, 1><<<grid, block, 0, stream>>>(p);
+  return 0;
+}
+
+template <typename T, typename TZ>
+int pp_trimul_out(const void* x, int ldx, const void* z, const void* ln_in_w, const void* ln_in_b,
+                  const void* ln_out_w, const void* ln_out_b, const void* packed, void* out, int n, int c_z,
+                  int hidden, int add_residual, float eps, hipStream_t stream) {
+  ProjOutParams p = {};
+  p.z = z;
+  p.si = (int64_t)n * c_z;
+  p.sj = c_z;
+  p.gamma = ln_in_w;
+  p.beta = ln_in_b;
+  p.gamma2 = ln_out_w;
+  p.beta2 = ln_out_b;
+  p.eps = eps;
+  p.packed = (const T*)packed + (int64_t)4 * c_z * hidden;
+  p.x = x;
+  p.ldx = ldx;
+  p.out = out;
+  p.n = n;
+  p.add_residual = add_residual;
+  if (c_z == 64) return pp_trimul_out_ks<T, TZ, 4>(p, stream);
+  if (c_z == 256) {
+    if constexpr (sizeof(T) == 2) return pp_trimul_out_ks<T, TZ, 16>(p, stream);
+    else return -1;
+  }
+  return pp_trimul_out_ks<T, TZ, 8>(p, stream);
+}
+
+template <typename T, typename TZ>
+int pp_triattn_out(const void* o, const void* z, const void* ln_w, const void* ln_b, const void* packed, void* out,
+                   int n, int c_z, int heads, int transposed, int add_residual, float eps, hipStream_t stream) {
+  ProjOutParams p = {};
+  p.z = z;
+  p.si = transposed ? c_z : (int64_t)n * c_z;
+  p.sj = transposed ? (int64_t)n * c_z : c_z;
+  p.gamma = ln_w;
+  p.beta = ln_b;
+  p.eps = eps;
+  p.packed = (const T*)packed + (int64_t)(4 * heads + 1) * 32 * c_z;
+  p.packed_g = (const T*)packed + (int64_t)3 * heads * 32 * c_z;
+  p.x = o;
+  p.out = out;
+  p.n = n;
+  p.add_residual = add_residual;
+  if (c_z == 64) return pp_triattn_out_ks<T, TZ, 4, false>(p, stream);
+  if (c_z == 256) {
+    if constexpr (sizeof(T) == 2) return pp_triattn_out_ks<T, TZ, 16, false>(p, stream);
+    else return -1;
+  }
+  return pp_triattn_out_ks<T, TZ, 8, sizeof(T) == 2>(p, stream);
+}
+
+#define PTX_INSTANTIATE_PACK(T)                                                                                        \
+  template int pp_trimul_pack<T>(const void*, const void*, const void*, const void*, const void*, const void*, void*, \
+                                 int, int, hipStream_t);                                                              \
+  template int pp_triattn_pack<T>(const void*, const void*, const void*, const void*, const void*, const void*,       \
+                                  void*, int, int, hipStream_t);
+PTX_INSTANTIATE_PACK(float)
+PTX_INSTANTIATE_PACK(bf16_t)
+#undef PTX_INSTANTIATE_PACK
+#define PTX_INSTANTIATE(T, TZ)                                                                                        \
+  template int pp_trimul_in<T, TZ>(const void*, const void*, const void*, const void*, const void*, void*, void*,    \
+                                   int, int, int, int, float, hipStream_t);                                          \
+  template int pp_triattn_in<T, TZ>(const void*, const void*, const void*, const void*, void*, void*, void*, void*,  \
+                                    void*, int, int, int, int, int, float, hipStream_t);                             \
+  template int pp_trimul_out<T, TZ>(const void*, int, const void*, const void*, const void*, const void*,            \
+                                    const void*, const void*, void*, int, int, int, int, float, hipStream_t);        \
+  template int pp_triattn_out<T, TZ>(const void*, const void*, const void*, const void*, const void*, void*, int,    \
+                                     int, int, int, int, float, hipStream_t);
+PTX_INSTANTIATE(float, float)
+PTX_INSTANTIATE(bf16_t, bf16_t)
+PTX_INSTANTIATE(bf16_t, float)
+#undef PTX_INSTANTIATE
+
+}  // namespace ptx

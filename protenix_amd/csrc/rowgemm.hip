@@ -300,7 +300,7 @@ rowgemm_in_kernel(RowGemmInParams p) {
       f32x8 v[KS];
 #pragma unroll
       for (int kk = 0; kk < KS; ++kk) v[kk] = to_f32(raw[kk]);
-      normalize_row<T, KS, float, false>(v, lds_affine[0], lds_affine[1], p.eps, lane >> 5, xf.f[0]);
+      normalize_row<T, TZ, KS, float, false>(v, lds_affine[0], lds_affine[1], p.eps, lane >> 5, xf.f[0]);
     }
   };
   normalize_prefetched();
@@ -397,7 +397,8 @@ rowgemm_in_kernel(RowGemmInParams p) {
 #pragma unroll
       for (int kk = 0; kk < KS; ++kk)
         store8<T>(&lds_res[wave][rb * 32 + n][16 * kk + 8 * g], zraw.f[rb][kk]);
-      normalize_raw<T>(zraw.f[rb], gamma, beta, p.eps, g, xf.f[rb]);
+      if constexpr (sizeof(T) == 4) normalize_row<T, T, KS>(zraw.f[rb], gamma, beta, p.eps, g, xf.f[rb]);
+      else normalize_raw<T>(zraw.f[rb], gamma, beta, p.eps, g, xf.f[rb]);
     }
   } else {
     if constexpr (kPrefetch) {
@@ -463,9 +464,9 @@ rowgemm_in_kernel(RowGemmInParams p) {
             v[2 * cg + k2][t] = to_f32(st[(16 * k2 + 8 * g + t) * C::PITCH + n]);
       }
       if constexpr (kRegRes)
-        normalize_row<T, SL, float, false>(v, lds_affine2[2], lds_affine2[3], p.eps, g, xf2.f[rb]);
+        normalize_row<T, T, SL, float, false>(v, lds_affine2[2], lds_affine2[3], p.eps, g, xf2.f[rb]);
       else
-        normalize_row<T>(v, gamma2, beta2, p.eps, g, xf2.f[rb]);
+        normalize_row<T, T, SL>(v, gamma2, beta2, p.eps, g, xf2.f[rb]);
       if constexpr (kRegRes) {
         // The raw fp32 rows stay in registers for the residual add: lane (row n, half g)
         // holds channels 16*kk + 8*g .. +7, which the permuted weight columns make the very
@@ -481,7 +482,7 @@ rowgemm_in_kernel(RowGemmInParams p) {
 #pragma unroll
         for (int kk = 0; kk < KS; ++kk) zres[rb][kk] = load8<TZ>(rp + 16 * kk);
         if constexpr (MIXED)
-          normalize_row<T, KS, float, false>(zres[rb], lds_affine2[0], lds_affine2[1], p.eps, g, xf.f[rb]);
+          normalize_row<T, TZ, KS, float, false>(zres[rb], lds_affine2[0], lds_affine2[1], p.eps, g, xf.f[rb]);
         else
           normalize_raw<T, KS, float, false>(zres[rb], lds_affine2[0], lds_affine2[1], p.eps, g, xf.f[rb]);
       }

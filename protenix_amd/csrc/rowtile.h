@@ -52,34 +52,53 @@ template <typename T> __device__ __forceinline__ const T* default_beta() {
   return reinterpret_cast<const T*>(kZerosAny);
 }
 
+// Sums over a row in fragment layout (lane g of a row's two holds the groups 2 kk + g of 8 channels),
+// associated as in the kernels that hold a row in 8 neighbouring lanes, whose lane j has every
+// eighth 16-byte piece of the stored row (TZ: 4 channels of fp32 rows, 8 of 16-bit rows) and whose sums
+// meet in lane_group_sum<8>(): every kernel then forms the same bits from the same row.  Four
+// chains per lane instead of one of 8 KS dependent adds, met on the vector ALU instead of through LDS.
+template <typename TZ> __device__ __forceinline__ int row_sum_chain(int kk, int t) {
+  return sizeof(TZ) == 4 ? (kk & 1) * 2 + (t >> 2) : kk & 3;
+}
+template <typename TZ> __device__ __forceinline__ float row_sum4(const float (&s)[4]) {
+  auto halves = [](float a, float b) {   // lower half-wave: a.lower + a.upper; upper: b.lower + b.upper
+    const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b),
+                                                    false, false);
+    return __builtin_bit_cast(float, (uint32_t)r[0]) + __builtin_bit_cast(float, (uint32_t)r[1]);
+  };
+  float p;
+  if constexpr (sizeof(TZ) == 4) p = halves(s[0] + s[1], s[2] + s[3]);   // pieces 0 - 3 | 4 - 7 (mod 8)
+  else p = halves(halves(s[0], s[1]), halves(s[2], s[3]));               // groups 0 - 3 | 4 - 7 (mod 8)
+  return halves(p, p);
+}
+
 // Mean / rstd of a row of 16*KS channels spread over the two half-wave lanes that hold it,
 // then gamma/beta (either may be null); result rounded to T like the reference's
 // LayerNorm output.
 // gamma / beta are read as type P: T from global memory (null: the stand-ins above), or float
 // from a copy the caller keeps in LDS (P = float, DEFAULTS = false: never null).
-template <typename T, int KS, typename P = T, bool DEFAULTS = true>
+// TZ: the type the row is stored in (it decides how the sums associate).
+template <typename T, typename TZ, int KS, typename P = T, bool DEFAULTS = true>
 __device__ __forceinline__ void normalize_row(f32x8 (&v)[KS], const P* __restrict__ gamma,
                                               const P* __restrict__ beta, float eps, int g,
                                               typename Vec8<T>::type (&out)[KS]) {
   const P* gp = (DEFAULTS && !gamma ? default_gamma<P>() : gamma) + 8 * g;
   const P* bp = (DEFAULTS && !beta ? default_beta<P>() : beta) + 8 * g;
-  float s = 0.0f;
+  float s[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
   for (int kk = 0; kk < KS; ++kk)
 #pragma unroll
-    for (int t = 0; t < 8; ++t) s += v[kk][t];
-  s += swap32(s);
-  const float mean = s * (1.0f / (16 * KS));
-  float q = 0.0f;
+    for (int t = 0; t < 8; ++t) s[row_sum_chain<TZ>(kk, t)] += v[kk][t];
+  const float mean = row_sum4<TZ>(s) * (1.0f / (16 * KS));
+  float q[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
   for (int kk = 0; kk < KS; ++kk)
 #pragma unroll
     for (int t = 0; t < 8; ++t) {
       const float d = v[kk][t] - mean;
-      q += d * d;
+      q[row_sum_chain<TZ>(kk, t)] += d * d;
     }
-  q += swap32(q);
-  const float rstd = rsqrtf(q * (1.0f / (16 * KS)) + eps);
+  const float rstd = rsqrtf(row_sum4<TZ>(q) * (1.0f / (16 * KS)) + eps);
 #pragma unroll
   for (int kk = 0; kk < KS; ++kk) {
     // (no branch around these loads, so the compiler may issue them as early as registers allow)
@@ -100,27 +119,25 @@ __device__ __forceinline__ void normalize_raw(const typename Vec8<T>::type (&raw
                                               typename Vec8<T>::type (&out)[KS]) {
   const P* gp = (DEFAULTS && !gamma ? default_gamma<P>() : gamma) + 8 * g;
   const P* bp = (DEFAULTS && !beta ? default_beta<P>() : beta) + 8 * g;
-  float s = 0.0f;
+  float s[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
   for (int kk = 0; kk < KS; ++kk) {
     const f32x8 v = to_f32(raw[kk]);
 #pragma unroll
-    for (int t = 0; t < 8; ++t) s += v[t];
+    for (int t = 0; t < 8; ++t) s[row_sum_chain<T>(kk, t)] += v[t];
   }
-  s += swap32(s);
-  const float mean = s * (1.0f / (16 * KS));
-  float q = 0.0f;
+  const float mean = row_sum4<T>(s) * (1.0f / (16 * KS));
+  float q[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
   for (int kk = 0; kk < KS; ++kk) {
     const f32x8 v = to_f32(raw[kk]);
 #pragma unroll
     for (int t = 0; t < 8; ++t) {
       const float d = v[t] - mean;
-      q += d * d;
+      q[row_sum_chain<T>(kk, t)] += d * d;
     }
   }
-  q += swap32(q);
-  const float rstd = rsqrtf(q * (1.0f / (16 * KS)) + eps);
+  const float rstd = rsqrtf(row_sum4<T>(q) * (1.0f / (16 * KS)) + eps);
 #pragma unroll
   for (int kk = 0; kk < KS; ++kk) {
     const f32x8 v = to_f32(raw[kk]);
@@ -152,7 +169,7 @@ __device__ __forceinline__ void load_rows_at(RowFrags<T, RB, KS>& out, const TZ*
       f32x8 v[KS];
 #pragma unroll
       for (int kk = 0; kk < KS; ++kk) v[kk] = to_f32(load8<TZ>(rp + 16 * kk));
-      normalize_row<T, KS, P, DEFAULTS>(v, gamma, beta, eps, g, out.f[rb]);
+      normalize_row<T, TZ, KS, P, DEFAULTS>(v, gamma, beta, eps, g, out.f[rb]);
     }
   }
 }
@@ -242,6 +259,17 @@ __device__ __forceinline__ typename VecE<T>::type add_vec(typename VecE<T>::type
 #pragma unroll
   for (int e = 0; e < Cfg<T>::VE; ++e) o[e] = from_f32<T>(to_f32(v[e]) + to_f32(r[e]));
   return o;
+}
+
+// Sum over groups of LPM (4 or 8) neighbouring lanes on the vector ALU's lane-permute path
+// (quad swaps, then the mirror of each half row): every lane of a group ends up with the sum.
+template <int LPM> __device__ __forceinline__ float lane_group_sum(float v) {
+  static_assert(LPM == 4 || LPM == 8, "groups of 4 or 8 lanes");
+  v += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0xB1, 0xf, 0xf, true));   // quad_perm [1,0,3,2]
+  v += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0x4E, 0xf, 0xf, true));   // quad_perm [2,3,0,1]
+  if (LPM == 8)
+    v += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0x141, 0xf, 0xf, true));  // row_half_mirror
+  return v;
 }
 
 // LDS traffic inside one wave: make the stores visible before the loads.

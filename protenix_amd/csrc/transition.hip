@@ -91,17 +91,6 @@ __global__ void transition_pack_kernel(const T* __restrict__ w_a, const T* __res
 // a Pairformer block, bias[h][row] = (W LN_pb(out[row]))[h], formed from the finished rows
 // while they pass through the epilogue (a kernel of its own would read the pair tensor once
 // more for it).
-// Sum over groups of LPM (4 or 8) neighbouring lanes on the vector ALU's lane-permute path
-// (quad swaps, then the mirror of each half row): every lane of a group ends up with the sum.
-template <int LPM> __device__ __forceinline__ float group_sum(float v) {
-  static_assert(LPM == 4 || LPM == 8, "groups of 4 or 8 lanes");
-  v += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0xB1, 0xf, 0xf, true));   // quad_perm [1,0,3,2]
-  v += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0x4E, 0xf, 0xf, true));   // quad_perm [2,3,0,1]
-  if (LPM == 8)
-    v += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0x141, 0xf, 0xf, true));  // row_half_mirror
-  return v;
-}
-
 struct PairBiasArgs {
   const void *gamma, *beta, *w;   // LayerNorm of the bias (either may be null), W [heads][c]
   void* out;                      // [heads][n_rows], fp32 or T
@@ -246,7 +235,7 @@ __global__ __launch_bounds__((TrCfg<T, KS>::NW * 64), 2) void transition_fused_k
       f32x8 v[KS];
 #pragma unroll
       for (int kk = 0; kk < KS; ++kk) v[kk] = zr[kk];
-      normalize_row<T, KS>(v, (const T*)ao.gamma, (const T*)ao.beta, ao.eps, g, xg);
+      normalize_row<T, TZ, KS>(v, (const T*)ao.gamma, (const T*)ao.beta, ao.eps, g, xg);
     }
     // gate of head c from the fragments at `f0` of a chunk buffer, applied to the attention
     // output in place (both rounded to T like the reference's sigmoid(linear_g(x)) and o * g)
@@ -310,7 +299,7 @@ __global__ __launch_bounds__((TrCfg<T, KS>::NW * 64), 2) void transition_fused_k
       out_block(b, 0, 2);
       out_block(b, 8, 3);
     }
-    normalize_row<T, KS>(zr, gamma, beta, eps, g, xf.f[0]);
+    normalize_row<T, TZ, KS>(zr, gamma, beta, eps, g, xf.f[0]);
   }
 
   f32x16 acc_o[RB][NOB];   // [row block][output column block]: lane <-> row, register <-> column
@@ -536,7 +525,7 @@ __global__ __launch_bounds__((TrCfg<T, KS>::NW * 64), 2) void transition_fused_k
       for (int ob = 0; ob < NOB; ++ob)
 #pragma unroll
         for (int e = 0; e < C::VE; ++e) sum += to_f32(done[0][ob][ps][e]);
-      sum = group_sum<C::LPM>(sum);
+      sum = lane_group_sum<C::LPM>(sum);
       mean[ps] = sum * (1.0f / kCx);
       float q = 0.0f;
 #pragma unroll
@@ -546,7 +535,7 @@ __global__ __launch_bounds__((TrCfg<T, KS>::NW * 64), 2) void transition_fused_k
           const float d = to_f32(done[0][ob][ps][e]) - mean[ps];
           q += d * d;
         }
-      q = group_sum<C::LPM>(q);
+      q = lane_group_sum<C::LPM>(q);
       rstd[ps] = rsqrtf(q * (1.0f / kCx) + pb.eps);
     }
     // per wave: 32 rows x 64 normalised columns in T, behind all waves' staging tiles (other

@@ -326,6 +326,30 @@ def _mask_for(mask: Optional[torch.Tensor], z: torch.Tensor, dtype: Optional[tor
     return out
 
 
+def trimul_pack(w: dict) -> torch.Tensor:
+    """The six weight matrices of a triangle multiplication in the row-local kernels' fragment order."""
+    _dev(w["w_ap"], "w_ap")
+    lib = _lib.load()
+    c_h, c_z = w["w_ap"].shape
+    packed = torch.empty((lib.ptx_trimul_packed_elems(c_z, c_h),), dtype=w["w_ap"].dtype, device=w["w_ap"].device)
+    with torch.cuda.device(packed.device):
+        _call("trimul_pack", lib.ptx_trimul_pack, *(_ptr(w[k]) for k in ("w_ap", "w_ag", "w_bp", "w_bg", "w_z", "w_g")),
+              _ptr(packed), c_z, c_h, _dt(packed), _stream())
+    return packed
+
+
+def triattn_pack(w: dict) -> torch.Tensor:
+    """The six weight matrices of a triangle attention in the row-local kernels' fragment order."""
+    _dev(w["w_q"], "w_q")
+    lib = _lib.load()
+    heads, c_in = w["w_b"].shape
+    packed = torch.empty((lib.ptx_triattn_packed_elems(c_in, heads),), dtype=w["w_q"].dtype, device=w["w_q"].device)
+    with torch.cuda.device(packed.device):
+        _call("triattn_pack", lib.ptx_triattn_pack, *(_ptr(w[k]) for k in ("w_q", "w_k", "w_v", "w_g", "w_b", "w_o")),
+              _ptr(packed), c_in, heads, _dt(packed), _stream())
+    return packed
+
+
 def triangle_multiplication(z: torch.Tensor, mask: Optional[torch.Tensor], w: dict, incoming: bool,
                             add_residual: bool, out: Optional[torch.Tensor] = None,
                             eps: float = 1e-5) -> torch.Tensor:
@@ -339,19 +363,30 @@ def triangle_multiplication(z: torch.Tensor, mask: Optional[torch.Tensor], w: di
     dt, st = _dt_stream(z, cd), _stream()
     pitch = key_pitch(n)
     mask = _mask_for(mask, z, cd)
+    packed = w.get("packed")        # the weights in fragment order (trimul_pack), or row-major only
+    ldx = (n + 7) // 8 * 8 if packed is not None else n
     # contraction operands in the library's fragment order (see include/protenix_amd.h)
     n_op = lib.ptx_trimul_operand_elems(n, c_h)
     a = _workspace((n_op,), cd, z.device)
     b = _workspace((n_op,), cd, z.device)
     with torch.cuda.device(z.device):
-        _call("trimul_project", lib.ptx_trimul_project, _ptr(z), _ptr(mask), _ptr(w["ln_in_w"]), _ptr(w["ln_in_b"]), _ptr(w["w_ap"]),
-            _ptr(w["w_ag"]), _ptr(w["w_bp"]), _ptr(w["w_bg"]), _ptr(a), _ptr(b), n, c_z, c_h, pitch,
-            int(incoming), eps, dt, st)
-        x = _workspace((c_h, n, n), cd, z.device)
-        _call("trimul_contract", lib.ptx_trimul_contract, _ptr(a), _ptr(b), _ptr(x), n, c_h, pitch, dt, st)
+        if packed is not None:
+            _call("trimul_project", lib.ptx_trimul_project_packed, _ptr(z), _ptr(mask), _ptr(w["ln_in_w"]),
+                  _ptr(w["ln_in_b"]), _ptr(packed), _ptr(a), _ptr(b), n, c_z, c_h, pitch, int(incoming), eps, dt, st)
+        else:
+            _call("trimul_project", lib.ptx_trimul_project, _ptr(z), _ptr(mask), _ptr(w["ln_in_w"]), _ptr(w["ln_in_b"]), _ptr(w["w_ap"]),
+                _ptr(w["w_ag"]), _ptr(w["w_bp"]), _ptr(w["w_bg"]), _ptr(a), _ptr(b), n, c_z, c_h, pitch,
+                int(incoming), eps, dt, st)
+        x = _workspace((c_h, n, ldx), cd, z.device)
+        _call("trimul_contract", lib.ptx_trimul_contract_ld, _ptr(a), _ptr(b), _ptr(x), n, ldx, c_h, pitch, dt, st)
         del a, b
         if out is None:
             out = torch.empty_like(z)
+        if packed is not None:
+            _call("trimul_output", lib.ptx_trimul_output_packed, _ptr(x), ldx, _ptr(z), _ptr(w["ln_in_w"]),
+                  _ptr(w["ln_in_b"]), _ptr(w["ln_out_w"]), _ptr(w["ln_out_b"]), _ptr(packed), _ptr(out), n, c_z, c_h,
+                  int(add_residual), eps, dt, st)
+            return out
         _call("trimul_output", lib.ptx_trimul_output, _ptr(x), _ptr(z), _ptr(w["ln_in_w"]), _ptr(w["ln_in_b"]), _ptr(w["ln_out_w"]),
             _ptr(w["ln_out_b"]), _ptr(w["w_z"]), _ptr(w["w_g"]), _ptr(out), n, c_z, c_h,
             int(add_residual), eps, dt, st)
@@ -445,16 +480,23 @@ def triangle_attention(z: torch.Tensor, mask: Optional[torch.Tensor], w: dict, h
     n_kv, n_tb = lib.ptx_triattn_kv_elems(n, heads), lib.ptx_triattn_bias_elems(n, heads)
     # rows of 128 channels in bf16 arithmetic: no gate tensor, the output kernel forms the gate
     late_gate = late_gate_enabled and c == 128 and heads == 4 and d == 32 and cd == torch.bfloat16
+    # (the packed weights are laid out for the gate's place: not with the switch thrown)
+    packed = w.get("packed") if late_gate_enabled else None
     q = _workspace((heads, n, n, d), cd, dev)
     g = _workspace((heads, n, n, d), cd, dev)     # the gate, then (or only) the attention output
     k = _workspace((n_kv,), cd, dev)
     vt = _workspace((n_kv,), cd, dev)
     tb = _workspace((n_tb,), cd, dev)
     with torch.cuda.device(dev):
-        _call("triattn_project", lib.ptx_triattn_project, _ptr(z), _ptr(w["ln_w"]),
-              _ptr(w["ln_b"]), _ptr(w["w_q"]), _ptr(w["w_k"]), _ptr(w["w_v"]), _ptr(w["w_g"]),
-              _ptr(w["w_b"]), _ptr(q), _ptr(k), _ptr(vt), None if late_gate else _ptr(g), _ptr(tb),
-              n, c, heads, d, pitch, int(transposed), eps, dt, st)
+        if packed is not None:
+            _call("triattn_project", lib.ptx_triattn_project_packed, _ptr(z), _ptr(w["ln_w"]), _ptr(w["ln_b"]),
+                  _ptr(packed), _ptr(q), _ptr(k), _ptr(vt), None if late_gate else _ptr(g), _ptr(tb),
+                  n, c, heads, pitch, int(transposed), eps, dt, st)
+        else:
+            _call("triattn_project", lib.ptx_triattn_project, _ptr(z), _ptr(w["ln_w"]),
+                  _ptr(w["ln_b"]), _ptr(w["w_q"]), _ptr(w["w_k"]), _ptr(w["w_v"]), _ptr(w["w_g"]),
+                  _ptr(w["w_b"]), _ptr(q), _ptr(k), _ptr(vt), None if late_gate else _ptr(g), _ptr(tb),
+                  n, c, heads, d, pitch, int(transposed), eps, dt, st)
         # o overwrites g: each element of g is read once, by the thread that then writes o there
         if mask is not None and n_valid is not None:
             # mask = m (x) m, padding at the end: the valid rows attend the valid keys with no
@@ -486,7 +528,10 @@ def triangle_attention(z: torch.Tensor, mask: Optional[torch.Tensor], w: dict, h
                   _ptr(pbw[2].contiguous()) if pbw else None, _ptr(bias), 0 if pbw is None else pbw[2].shape[0],
                   1, eps, dt, st)
             return out, bias
-        if late_gate:
+        if packed is not None:
+            _call("triattn_output", lib.ptx_triattn_output_packed, _ptr(g), _ptr(z), _ptr(w["ln_w"]), _ptr(w["ln_b"]),
+                  _ptr(packed), _ptr(out), n, c, heads, int(transposed), int(add_residual), eps, dt, st)
+        elif late_gate:
             _call("triattn_output", lib.ptx_triattn_gate_output, _ptr(g), _ptr(z), _ptr(w["ln_w"]),
                   _ptr(w["ln_b"]), _ptr(w["w_g"]), _ptr(w["w_o"]), _ptr(out), n, c, heads,
                   int(transposed), int(add_residual), eps, dt, st)

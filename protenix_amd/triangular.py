@@ -59,6 +59,18 @@ def _per_batch(z: torch.Tensor, mask: Optional[torch.Tensor]):
     return zb, mb
 
 
+def _with_packed(w: dict, c_z: int, pack) -> dict:
+    """Adds the weights in fragment order where the packed kernels exist (what they refuse is left to
+    the kernels on row-major weights, which refuse it with their own message)."""
+    mat = w["w_ap"] if "w_ap" in w else w["w_q"]
+    wide = c_z == 256 and mat.shape[0] == 256 and mat.dtype == torch.bfloat16
+    if mat.is_cuda and mat.dtype in (torch.float32, torch.bfloat16) and (
+            wide or (c_z in (64, 128) and mat.shape[0] == 128)) and (
+            "w_b" not in w or w["w_b"].shape[0] * 32 == mat.shape[0]):
+        w["packed"] = pack(w)
+    return w
+
+
 def kernel_triangular_mult(x: torch.Tensor, direction: str, mask: Optional[torch.Tensor],
                            norm_in_weight: Optional[torch.Tensor], norm_in_bias: Optional[torch.Tensor],
                            p_in_weight: torch.Tensor, g_in_weight: torch.Tensor,
@@ -113,8 +125,8 @@ class TriangleMultiplicativeUpdate(nn.Module):
               self.linear_g.weight)
         names = ("ln_in_w", "ln_in_b", "ln_out_w", "ln_out_b", "w_ap", "w_ag", "w_bp", "w_bg",
                  "w_z", "w_g")
-        return self._cache.get(ps, dtype, device,
-                               lambda: dict(zip(names, (_cv(p, dtype, device) for p in ps))))
+        return self._cache.get(ps, dtype, device, lambda: _with_packed(
+            dict(zip(names, (_cv(p, dtype, device) for p in ps))), self.c_z, ops.trimul_pack))
 
     def forward(self, z: torch.Tensor, mask: Optional[torch.Tensor] = None,
                 inplace_safe: bool = False, _add_with_inplace: bool = False,
@@ -212,8 +224,8 @@ class TriangleAttention(nn.Module):
         ps = (self.layer_norm.weight, self.layer_norm.bias, m.linear_q.weight, m.linear_k.weight,
               m.linear_v.weight, m.linear_g.weight, self.linear.weight, m.linear_o.weight)
         names = ("ln_w", "ln_b", "w_q", "w_k", "w_v", "w_g", "w_b", "w_o")
-        return self._cache.get(ps, dtype, device,
-                               lambda: dict(zip(names, (_cv(p, dtype, device) for p in ps))))
+        return self._cache.get(ps, dtype, device, lambda: _with_packed(
+            dict(zip(names, (_cv(p, dtype, device) for p in ps))), self.c_in, ops.triattn_pack))
 
     def _run(self, x: torch.Tensor, mask: Optional[torch.Tensor], transposed: bool,
              residual_inplace: bool, then_transition=None):
