@@ -23,6 +23,7 @@
 #include "common.h"
 #include "kernels.h"
 #include "rowtile.h"
+#include "transition.h"
 #include <type_traits>
 
 namespace ptx {
@@ -91,13 +92,6 @@ __global__ void transition_pack_kernel(const T* __restrict__ w_a, const T* __res
 // a Pairformer block, bias[h][row] = (W LN_pb(out[row]))[h], formed from the finished rows
 // while they pass through the epilogue (a kernel of its own would read the pair tensor once
 // more for it).
-struct PairBiasArgs {
-  const void *gamma, *beta, *w;   // LayerNorm of the bias (either may be null), W [heads][c]
-  void* out;                      // [heads][n_rows], fp32 or T
-  int heads, out_f32;
-  float eps;
-};
-
 // AO: the last stage of a triangle attention in front of the transition,
 //   x' = x + W_o (sigmoid(W_g LN_att(x)) * o)                      (layers.py:380-396)
 //   out = x' + transition(x'),
@@ -116,13 +110,6 @@ struct PairBiasArgs {
 //   rows of a 32-row block permuted as in triattn_gate_out_kernel, so that accumulator
 //   registers 8 u .. 8 u + 7 of half-wave g are the channels 16 u + 8 g .. + 7 of the block:
 //   a lane's own fragment of K step 2 c + u.
-struct AttnOutArgs {
-  const void* o;             // attention output, head-major [4][n_rows][32], T, rows in the attention's order
-  const void *gamma, *beta;  // the attention's LayerNorm (either may be null)
-  RowMap omap;               // row of x -> element offset of its 32 channels inside a head's plane of o
-  float eps;
-};
-constexpr int kAoChunks = 3;   // chunks of 24 fragments that hold the 64 fragments of W_g and W_o
 
 template <typename T, int KS, typename TZ = T, bool PB = false, bool AO = false>
 __global__ __launch_bounds__((TrCfg<T, KS>::NW * 64), 2) void transition_fused_kernel(
@@ -616,6 +603,9 @@ template <typename T, int KS, typename TZ>
 static int transition_fwd_ks(const void* x, const void* ln_w, const void* ln_b, const void* packed,
                              void* out, int64_t rows, int n_factor, int add_residual, float eps,
                              hipStream_t stream) {
+  if (transition_small<T, KS, TZ, false, false>((const TZ*)x, (const T*)ln_w, (const T*)ln_b, (const T*)packed, (TZ*)out, rows,
+                                                16 * KS * n_factor / 32, add_residual, eps, PairBiasArgs{}, AttnOutArgs{}, stream))
+    return 0;
   const int64_t rows_per_block = TrCfg<T, KS>::NW * TrCfg<T, KS>::RB * 32;
   const int64_t blocks = (rows + rows_per_block - 1) / rows_per_block;
   transition_fused_kernel<T, KS, TZ, false><<<dim3((unsigned)blocks), dim3(TrCfg<T, KS>::NW * 64), 0, stream>>>(
@@ -637,6 +627,9 @@ int transition_pair_bias_fwd(const void* x, const void* ln_w, const void* ln_b, 
     const int64_t rows_per_block = TrCfg<T, KS>::NW * 32;
     const int64_t blocks = (rows + rows_per_block - 1) / rows_per_block;
     const PairBiasArgs pb = {pb_ln_w, pb_ln_b, pb_w, bias, heads, bias_f32, pb_eps};
+    if (transition_small<T, KS, TZ, true, false>((const TZ*)x, (const T*)ln_w, (const T*)ln_b, (const T*)packed, (TZ*)out, rows,
+                                                 16 * KS * n_factor / 32, add_residual, eps, pb, AttnOutArgs{}, stream))
+      return 0;
     transition_fused_kernel<T, KS, TZ, true><<<dim3((unsigned)blocks), dim3(TrCfg<T, KS>::NW * 64), 0, stream>>>(
         (const TZ*)x, (const T*)ln_w, (const T*)ln_b, (const T*)packed, (TZ*)out, rows,
         16 * KS * n_factor / 32, add_residual, eps, pb, AttnOutArgs{});
@@ -711,10 +704,16 @@ int triattn_output_transition_fwd(const void* o, const void* z, const void* att_
     const int n_chunks = 16 * KS * n_factor / 32;
     if (pb_w) {
       const PairBiasArgs pb = {pb_ln_w, pb_ln_b, pb_w, bias, heads, bias_f32, pb_eps};
+      if (transition_small<T, KS, TZ, true, true>((const TZ*)z, (const T*)ln_w, (const T*)ln_b, (const T*)packed, (TZ*)out, rows,
+                                                  n_chunks, 1, eps, pb, ao, stream))
+        return 0;
       transition_fused_kernel<T, KS, TZ, true, true><<<dim3((unsigned)blocks), dim3(TrCfg<T, KS>::NW * 64), 0, stream>>>(
           (const TZ*)z, (const T*)ln_w, (const T*)ln_b, (const T*)packed, (TZ*)out, rows, n_chunks, 1, eps,
           pb, ao);
     } else {
+      if (transition_small<T, KS, TZ, false, true>((const TZ*)z, (const T*)ln_w, (const T*)ln_b, (const T*)packed, (TZ*)out, rows,
+                                                   n_chunks, 1, eps, PairBiasArgs{}, ao, stream))
+        return 0;
       transition_fused_kernel<T, KS, TZ, false, true><<<dim3((unsigned)blocks), dim3(TrCfg<T, KS>::NW * 64), 0, stream>>>(
           (const TZ*)z, (const T*)ln_w, (const T*)ln_b, (const T*)packed, (TZ*)out, rows, n_chunks, 1, eps,
           PairBiasArgs{}, ao);
