@@ -1,4 +1,5 @@
-"""Builds protenix_amd/libprotenix_amd.so from csrc/*.hip with hipcc for gfx950.
+"""Builds protenix_amd/libprotenix_amd.so from csrc/*.hip with hipcc for gfx950, and the native host
+path protenix_amd/_host.so from csrc/host.cpp.
 
 Run as ``python -m protenix_amd.build``.  hipcc cross-compiles, so no GPU is
 needed; the library is left in-tree next to this file.
@@ -24,6 +25,24 @@ FLAGS = [
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-Wno-unused-command-line-argument",
 ]
+
+
+# The native host path (csrc/host.cpp): a torch extension module around the library, plain C++.
+HOST_LIB = os.path.join(HERE, "_host.so")
+
+
+def _host_command() -> list:
+    import sysconfig
+
+    import torch
+
+    t = os.path.dirname(torch.__file__)
+    abi = int(torch._C._GLIBCXX_USE_CXX11_ABI)
+    return ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+            f"-D_GLIBCXX_USE_CXX11_ABI={abi}", "-DTORCH_EXTENSION_NAME=_host", f"-I{t}/include",
+            f"-I{t}/include/torch/csrc/api/include", "-I/opt/rocm/include", f"-I{sysconfig.get_paths()['include']}",
+            os.path.join(CSRC, "host.cpp"), "-o", HOST_LIB, f"-L{HERE}", "-lprotenix_amd", f"-L{t}/lib", "-lc10", "-lc10_hip",
+            "-ltorch_cpu", "-ltorch_hip", "-ltorch_python", "-ltorch", "-L/opt/rocm/lib", "-lamdhip64", "-Wl,-rpath,$ORIGIN"]
 
 
 def _hipcc() -> str:
@@ -59,6 +78,7 @@ def build(verbose: bool = False) -> str:
             if verbose and msg:
                 print(msg, file=sys.stderr)
     _run([hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB, *objs])
+    _run(_host_command())
     return LIB
 
 

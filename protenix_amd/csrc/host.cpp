@@ -1,0 +1,577 @@
+// The native host path: what protenix_amd/*.py does between a module call and the C ABI of
+// libprotenix_amd.so (allocation, argument lists, streams, autograd bookkeeping), in C++.  One call
+// per stack, update or operator instead of some twenty Python-level calls per block: below a few
+// hundred tokens the GPU finishes a block's kernels faster than Python can enqueue them (93 tokens:
+// 390 us of Python per block against about 110 us of kernels).
+//
+// Weights are laid out by Python (the modules' caches) and handed over once as a Plan, with a record of
+// the parameters, sub-modules and hooks they came from: valid() compares identities and version
+// counters, so that a parameter that was replaced or changed in place is noticed on the next call.
+// The kernels, their order and their arguments are those of ops.py.
+#include <torch/extension.h>
+
+#include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
+#include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
+
+#include "../../include/protenix_amd.h"
+
+namespace {
+
+namespace py = pybind11;
+using at::Tensor;
+using c10::optional;
+
+void check(int rc, const char* what) {
+  if (rc == PTX_OK) return;
+  const char* kind = rc == 1 ? "bad argument" : rc == 2 ? "unsupported shape" : rc == 3 ? "launch failure" : "error";
+  throw std::runtime_error(std::string(what) + ": " + kind + " (" + std::to_string(rc) + "): " + ptx_last_error_string());
+}
+
+int code_of(at::ScalarType t) {
+  switch (t) {
+    case at::kFloat: return PTX_F32;
+    case at::kBFloat16: return PTX_BF16;
+    case at::kHalf: return PTX_F16;
+    default: throw std::runtime_error(std::string("protenix_amd kernels take float32 or bfloat16 tensors, got ") + toString(t));
+  }
+}
+// rows `z` with weights and workspaces in `compute`
+int code_of_rows(at::ScalarType z, at::ScalarType compute) {
+  return z == compute ? code_of(z) : PTX_MIXED;
+}
+
+void* ptr(const Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; }
+hipStream_t current_stream(const Tensor& t) {
+  return c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(t.device().index()).stream();
+}
+
+Tensor take(const py::dict& d, const char* key) {
+  if (!d.contains(key)) return Tensor();
+  py::object o = d[key];
+  return o.is_none() ? Tensor() : o.cast<Tensor>();
+}
+int take_int(const py::dict& d, const char* key) { return d.contains(key) ? d[key].cast<int>() : 0; }
+
+// ---- what a plan's weights were made from ---------------------------------------------------
+struct Guard {
+  struct Entry {
+    py::object dict, key, value;   // dict[key] is value
+    int64_t version = -1;          // of a parameter
+    const void* data = nullptr;
+  };
+  std::vector<Entry> entries;
+  std::vector<py::object> empty;   // dicts that must have no entries (hooks)
+
+  void add(const py::dict& d, const py::handle& key) {
+    Entry e;
+    e.dict = d;
+    e.key = py::reinterpret_borrow<py::object>(key);
+    e.value = d[key];
+    if (THPVariable_Check(e.value.ptr())) {
+      const Tensor& t = THPVariable_Unpack(e.value.ptr());
+      e.version = t.is_inference() ? -2 : (int64_t)t._version();
+      e.data = t.data_ptr();
+    }
+    entries.push_back(std::move(e));
+  }
+  // `m` and everything below it; the plain attributes named in `attrs` where they exist
+  void walk(const py::object& m, const py::list& attrs) {
+    py::dict d = m.attr("__dict__");
+    py::dict params = d["_parameters"], mods = d["_modules"];
+    for (auto item : params) add(params, item.first);
+    empty.push_back(d["_forward_hooks"]);
+    empty.push_back(d["_forward_pre_hooks"]);
+    for (auto a : attrs)
+      if (d.contains(a)) add(d, a);
+    for (auto item : mods) {
+      add(mods, item.first);
+      if (!item.second.is_none()) walk(py::reinterpret_borrow<py::object>(item.second), attrs);
+    }
+  }
+  bool valid() const {
+    for (const Entry& e : entries) {
+      PyObject* now = PyDict_GetItem(e.dict.ptr(), e.key.ptr());   // borrowed
+      if (now != e.value.ptr()) return false;
+      if (e.version != -1) {
+        const Tensor& t = THPVariable_Unpack(now);
+        if (e.version == -2 || t.is_inference() || (int64_t)t._version() != e.version || t.data_ptr() != e.data) return false;
+      }
+    }
+    for (const py::object& d : empty)
+      if (PyDict_Size(d.ptr()) != 0) return false;
+    return true;
+  }
+};
+
+struct TriMul {
+  Tensor ln_in_w, ln_in_b, ln_out_w, ln_out_b, packed;
+  int c_z = 0, c_h = 0;
+  bool incoming = false;
+  explicit TriMul(const py::dict& d)
+      : ln_in_w(take(d, "ln_in_w")), ln_in_b(take(d, "ln_in_b")), ln_out_w(take(d, "ln_out_w")), ln_out_b(take(d, "ln_out_b")),
+        packed(take(d, "packed")), c_z(take_int(d, "c_z")), c_h(take_int(d, "c_h")), incoming(take_int(d, "incoming") != 0) {}
+};
+struct TriAtt {
+  Tensor ln_w, ln_b, packed;
+  int c = 0, heads = 0;
+  float inf = 0;
+  bool transposed = false;
+  explicit TriAtt(const py::dict& d)
+      : ln_w(take(d, "ln_w")), ln_b(take(d, "ln_b")), packed(take(d, "packed")), c(take_int(d, "c")), heads(take_int(d, "heads")),
+        inf((float)d["inf"].cast<double>()), transposed(take_int(d, "transposed") != 0) {}
+};
+struct Mask {   // of one pair tensor: as the triangle multiplications / the starting node read it, transposed, valid tokens
+  Tensor m, mt;
+  int n_valid = -1;
+};
+std::vector<Mask> masks_of(const py::list& l) {
+  std::vector<Mask> v;
+  for (auto h : l) {
+    py::tuple t = py::reinterpret_borrow<py::tuple>(h);
+    Mask m;
+    if (!t[0].is_none()) m.m = t[0].cast<Tensor>();
+    if (!t[1].is_none()) m.mt = t[1].cast<Tensor>();
+    if (!t[2].is_none()) m.n_valid = t[2].cast<int>();
+    v.push_back(std::move(m));
+  }
+  return v;
+}
+
+// One workspace, cut into 256-byte aligned parts; a triangle update's intermediates of one pair tensor.
+struct Cut {
+  char* base;
+  int64_t used = 0;
+  void* part(int64_t bytes) {
+    void* p = base ? base + used : nullptr;
+    used += (bytes + 255) / 256 * 256;
+    return p;
+  }
+};
+struct TriMulWs {
+  void *a, *b, *x;
+  TriMulWs(Cut& c, int n, int c_h, int64_t es) {
+    a = c.part(ptx_trimul_operand_elems(n, c_h) * es);
+    b = c.part(ptx_trimul_operand_elems(n, c_h) * es);
+    x = c.part((int64_t)c_h * n * ((n + 7) / 8 * 8) * es);
+  }
+};
+struct TriAttWs {
+  void *q, *g, *k, *vt, *tb;
+  TriAttWs(Cut& c, int n, int heads, int64_t es) {
+    q = c.part((int64_t)heads * n * n * 32 * es);
+    g = c.part((int64_t)heads * n * n * 32 * es);
+    k = c.part(ptx_triattn_kv_elems(n, heads) * es);
+    vt = c.part(ptx_triattn_kv_elems(n, heads) * es);
+    tb = c.part(ptx_triattn_bias_elems(n, heads) * es);
+  }
+};
+int64_t workspace_bytes(int n, int c_h, int heads, int64_t es) {
+  Cut m{nullptr}, a{nullptr};
+  if (c_h) TriMulWs(m, n, c_h, es);
+  if (heads) TriAttWs(a, n, heads, es);
+  return std::max(m.used, a.used);
+}
+
+constexpr float kEps = 1e-5f;
+
+void run_trimul(const TriMul& w, const void* z, const Tensor& mask, void* out, int n, bool add, int dt, int64_t es, void* ws,
+                hipStream_t st) {
+  Cut c{(char*)ws};
+  TriMulWs s(c, n, w.c_h, es);
+  const int pitch = ptx_key_pitch(n), ldx = (n + 7) / 8 * 8;
+  check(ptx_trimul_project_packed(z, ptr(mask), ptr(w.ln_in_w), ptr(w.ln_in_b), ptr(w.packed), s.a, s.b, n, w.c_z, w.c_h, pitch,
+                                  w.incoming, kEps, dt, st), "trimul_project");
+  check(ptx_trimul_contract_ld(s.a, s.b, s.x, n, ldx, w.c_h, pitch, dt, st), "trimul_contract");
+  check(ptx_trimul_output_packed(s.x, ldx, z, ptr(w.ln_in_w), ptr(w.ln_in_b), ptr(w.ln_out_w), ptr(w.ln_out_b), ptr(w.packed), out, n,
+                                 w.c_z, w.c_h, add, kEps, dt, st), "trimul_output");
+}
+
+// projection and core; the attention output is left in ws.g
+TriAttWs run_triatt_core(const TriAtt& w, const void* z, const Mask& mask, int n, int dt, int64_t es, void* ws, hipStream_t st) {
+  Cut c{(char*)ws};
+  TriAttWs s(c, n, w.heads, es);
+  const int pitch = ptx_key_pitch(n);
+  void* gate = ptx_triattn_late_gate(w.c, w.heads, dt) ? nullptr : s.g;
+  check(ptx_triattn_project_packed(z, ptr(w.ln_w), ptr(w.ln_b), ptr(w.packed), s.q, s.k, s.vt, gate, s.tb, n, w.c, w.heads, pitch,
+                                   w.transposed, kEps, dt, st), "triattn_project");
+  const void* m = ptr(w.transposed ? mask.mt : mask.m);
+  if (m && mask.n_valid >= 0) {
+    // padding at the end: valid rows over valid keys without a mask, padded rows with it (ops.py)
+    check(ptx_triattn_fwd_rows(s.q, s.k, s.vt, gate, s.tb, nullptr, s.g, n, w.heads, 32, pitch, 0, w.inf, 0, mask.n_valid,
+                               mask.n_valid, dt, st), "triattn_fwd");
+    check(ptx_triattn_fwd_rows(s.q, s.k, s.vt, gate, s.tb, m, s.g, n, w.heads, 32, pitch, 0, w.inf, mask.n_valid,
+                               n - mask.n_valid, n, dt, st), "triattn_fwd_padded_rows");
+  } else {
+    check(ptx_triattn_fwd(s.q, s.k, s.vt, gate, s.tb, m, s.g, n, w.heads, 32, pitch, 0, w.inf, dt, st), "triattn_fwd");
+  }
+  return s;
+}
+
+void run_triatt(const TriAtt& w, const void* z, const Mask& mask, void* out, int n, bool add, int dt, int64_t es, void* ws,
+                hipStream_t st) {
+  const TriAttWs s = run_triatt_core(w, z, mask, n, dt, es, ws, st);
+  check(ptx_triattn_output_packed(s.g, z, ptr(w.ln_w), ptr(w.ln_b), ptr(w.packed), out, n, w.c, w.heads, w.transposed, add, kEps, dt,
+                                  st), "triattn_output");
+}
+
+// ---- one Pairformer block ----------------------------------------------------------------------
+struct Block {
+  TriMul out, in;
+  TriAtt start, end;
+  // pair transition (fused: with the ending node's output stage in front, one launch)
+  bool fused;
+  Tensor tr_ln_w, tr_ln_b, tr_packed;
+  int n_factor, c_z, c_s;
+  // single track
+  Tensor pb_ln_w, pb_ln_b, pb_w, a_ln_w, a_ln_b, w_in, b_q, w_o, s_ln_w, s_ln_b, s_wa, s_wb, s_wo;
+  int heads = 0, d = 0;
+  double a_eps = kEps, s_eps = kEps;
+  at::ScalarType compute;
+  Guard guard;
+
+  Block(const py::object& module, const py::dict& d_, const py::list& attrs)
+      : out(d_["tri_mul_out"].cast<py::dict>()), in(d_["tri_mul_in"].cast<py::dict>()), start(d_["tri_att_start"].cast<py::dict>()),
+        end(d_["tri_att_end"].cast<py::dict>()), fused(take_int(d_, "fused") != 0), tr_ln_w(take(d_, "tr_ln_w")),
+        tr_ln_b(take(d_, "tr_ln_b")), tr_packed(take(d_, "tr_packed")), n_factor(take_int(d_, "n_factor")), c_z(take_int(d_, "c_z")),
+        c_s(take_int(d_, "c_s")) {
+    compute = tr_packed.scalar_type();
+    if (c_s) {
+      pb_ln_w = take(d_, "pb_ln_w"); pb_ln_b = take(d_, "pb_ln_b"); pb_w = take(d_, "pb_w");
+      a_ln_w = take(d_, "a_ln_w"); a_ln_b = take(d_, "a_ln_b");
+      w_in = take(d_, "w_in"); b_q = take(d_, "b_q"); w_o = take(d_, "w_o");
+      s_ln_w = take(d_, "s_ln_w"); s_ln_b = take(d_, "s_ln_b");
+      s_wa = take(d_, "s_wa"); s_wb = take(d_, "s_wb"); s_wo = take(d_, "s_wo");
+      heads = take_int(d_, "heads");
+      d = take_int(d_, "d");
+      a_eps = d_["a_eps"].cast<double>();
+      s_eps = d_["s_eps"].cast<double>();
+    }
+    guard.walk(module, attrs);
+  }
+  bool valid() const { return guard.valid(); }
+
+  // The five pair updates of the pair tensors of z [batch][n][n][c_z] in place; the single attention's pair
+  // bias (fp32 [batch][heads][n][n]) of the finished z into `bias` (null: none wanted).
+  void pair_track(const Tensor& z, const std::vector<Mask>& masks, int64_t batch, int n, void* ws, float* bias, hipStream_t st) const {
+    const int dt = code_of_rows(z.scalar_type(), compute);
+    const int64_t es = at::elementSize(compute), plane = (int64_t)n * n * c_z * z.element_size();
+    char* zp = (char*)z.data_ptr();
+    static const Mask none;
+    auto mask = [&](int64_t b) -> const Mask& { return masks.empty() ? none : masks[b]; };
+    for (int64_t b = 0; b < batch; ++b) run_trimul(out, zp + b * plane, mask(b).m, zp + b * plane, n, true, dt, es, ws, st);
+    for (int64_t b = 0; b < batch; ++b) run_trimul(in, zp + b * plane, mask(b).m, zp + b * plane, n, true, dt, es, ws, st);
+    for (int64_t b = 0; b < batch; ++b) run_triatt(start, zp + b * plane, mask(b), zp + b * plane, n, true, dt, es, ws, st);
+    const int64_t bias_plane = (int64_t)heads * n * n;
+    if (fused) {
+      for (int64_t b = 0; b < batch; ++b) {
+        void* zb = zp + b * plane;
+        const TriAttWs s = run_triatt_core(end, zb, mask(b), n, dt, es, ws, st);
+        check(ptx_triattn_output_transition_fwd(s.g, zb, ptr(end.ln_w), ptr(end.ln_b), ptr(tr_packed), ptr(tr_ln_w), ptr(tr_ln_b), zb, n,
+                                                c_z, end.heads, end.transposed, n_factor, kEps, kEps, bias ? ptr(pb_ln_w) : nullptr,
+                                                bias ? ptr(pb_ln_b) : nullptr, bias ? ptr(pb_w) : nullptr,
+                                                bias ? bias + b * bias_plane : nullptr, bias ? heads : 0, 1, kEps, dt, st),
+              "triattn_output_transition");
+      }
+      return;
+    }
+    for (int64_t b = 0; b < batch; ++b) run_triatt(end, zp + b * plane, mask(b), zp + b * plane, n, true, dt, es, ws, st);
+    check(ptx_transition_fwd(zp, ptr(tr_ln_w), ptr(tr_ln_b), ptr(tr_packed), zp, batch * n * n, c_z, n_factor, 1, kEps, dt, st),
+          "transition");
+    if (bias)
+      for (int64_t b = 0; b < batch; ++b)
+        check(ptx_pair_bias_fwd(zp + b * plane, ptr(pb_ln_w), ptr(pb_ln_b), ptr(pb_w), bias + b * bias_plane, n, c_z, heads, 1, kEps, dt, st),
+              "pair_bias");
+  }
+
+  // elements of s' type that single_track() wants as scratch
+  int64_t single_elems(int64_t batch, int n) const {
+    const int64_t rows = batch * n, hd = (int64_t)heads * d, ldt = (n + 31) / 32 * 32;
+    auto up = [](int64_t e) { return (e + 63) / 64 * 64; };
+    return up(rows * c_s) + up((int64_t)n * 3 * hd) + up(hd * ldt) + up(rows * hd) + up(rows * s_wa.size(0));
+  }
+  // mid = s + attention(s; bias); s_out = mid + transition(mid)
+  void single_track(const void* s, void* mid, void* s_out, const float* bias, at::ScalarType type, int64_t batch, int n, void* ws,
+                    hipStream_t st) const {
+    const int dt = code_of(type), hd = heads * d, ldt = (n + 31) / 32 * 32, hidden = (int)s_wa.size(0);
+    const int64_t es = at::elementSize(type), rows = batch * n;
+    Cut c{(char*)ws};
+    void* y = c.part(rows * c_s * es);
+    void* qkg = c.part((int64_t)n * 3 * hd * es);
+    void* vt = c.part((int64_t)hd * ldt * es);
+    void* o = c.part(rows * hd * es);
+    void* h = c.part(rows * hidden * es);
+    check(ptx_layernorm_fwd(s, ptr(a_ln_w), ptr(a_ln_b), y, nullptr, nullptr, rows, c_s, (float)a_eps, dt, st), "layernorm");
+    for (int64_t b = 0; b < batch; ++b) {
+      check(ptx_linear_fwd((char*)y + b * n * c_s * es, ptr(w_in), ptr(b_q), hd, nullptr, qkg, vt, 3 * hd, ldt, n, c_s, 4 * hd, dt, st),
+            "linear");
+      check(ptx_single_attention_fwd(qkg, (char*)qkg + hd * es, vt, (char*)qkg + 2 * (int64_t)hd * es, bias + b * heads * (int64_t)n * n, 1,
+                                     (char*)o + b * n * hd * es, n, heads, d, 3 * hd, ldt, hd, (float)(1.0 / std::sqrt((double)d)), dt, st),
+            "single_attention");
+    }
+    check(ptx_linear_fwd(o, ptr(w_o), nullptr, 0, s, mid, nullptr, c_s, 0, (int)rows, hd, c_s, dt, st), "linear");
+    check(ptx_layernorm_fwd(mid, ptr(s_ln_w), ptr(s_ln_b), y, nullptr, nullptr, rows, c_s, (float)s_eps, dt, st), "layernorm");
+    check(ptx_swiglu_fwd(y, ptr(s_wa), ptr(s_wb), h, (int)rows, c_s, hidden, dt, st), "swiglu");
+    check(ptx_linear_fwd(h, ptr(s_wo), nullptr, 0, mid, s_out, nullptr, c_s, 0, (int)rows, hidden, c_s, dt, st), "linear");
+  }
+};
+
+// Events of one call, each recorded on one stream only; handed back to the runtime at its end.
+struct Event {
+  hipEvent_t e = nullptr;
+  Event() {
+    if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) throw std::runtime_error("hipEventCreate failed");
+  }
+  ~Event() { (void)hipEventDestroy(e); }
+  void record(hipStream_t s) { hip(hipEventRecord(e, s)); }
+  void wait(hipStream_t s) { hip(hipStreamWaitEvent(s, e, 0)); }
+  static void hip(hipError_t r) {
+    if (r != hipSuccess) throw std::runtime_error(std::string("hipEvent: ") + hipGetErrorString(r));
+  }
+};
+
+// The blocks in sequence on z (contiguous, updated in place).  `side` = (stream id, device index, device type) of a second
+// stream for the single track, which then runs underneath the next block's pair kernels, or None.  Returns the
+// new s (undefined for a stack without a single track).  Not for a stream that is being captured (native.py)
+optional<Tensor> run_blocks(const std::vector<const Block*>& blocks, const optional<Tensor>& s_opt, const Tensor& z, const py::list& mask_list,
+                            const py::object& side_obj) {
+  const std::vector<Mask> masks = masks_of(mask_list);
+  optional<c10::Stream> side_stream;
+  if (!side_obj.is_none()) {
+    py::tuple t = py::reinterpret_borrow<py::tuple>(side_obj);
+    side_stream = c10::Stream::unpack3(t[0].cast<int64_t>(), (c10::DeviceIndex)t[1].cast<int>(), (c10::DeviceType)t[2].cast<int>());
+  }
+  py::gil_scoped_release nogil;
+  const int n = (int)z.size(-2);
+  const int64_t batch = z.numel() / ((int64_t)n * n * z.size(-1));
+  at::DeviceGuard dev(z.device());
+  const hipStream_t main = current_stream(z);
+  int64_t ws_bytes = 0;
+  bool single = false;
+  int64_t s_elems = 0, bias_elems = 0;
+  for (const Block* b : blocks) {
+    ws_bytes = std::max(ws_bytes, workspace_bytes(n, std::max(b->out.c_h, b->in.c_h), std::max(b->start.heads, b->end.heads),
+                                                  at::elementSize(b->compute)));
+    if (b->c_s) {
+      single = true;
+      s_elems = std::max(s_elems, b->single_elems(batch, n));
+      bias_elems = std::max(bias_elems, batch * b->heads * (int64_t)n * n);
+    }
+  }
+  const auto bytes = z.options().dtype(at::kByte);
+  Tensor ws = at::empty({ws_bytes}, bytes);
+  if (!single) {
+    for (const Block* b : blocks) b->pair_track(z, masks, batch, n, ws.data_ptr(), nullptr, main);
+    return s_opt;
+  }
+  const Tensor& s0 = *s_opt;
+  const int64_t es = s0.element_size();
+  // The pair bias travels from the main stream to the side stream through a ring of two buffers.
+  const int ring = side_stream ? 2 : 1;
+  Tensor bias = at::empty({ring, bias_elems}, z.options().dtype(at::kFloat));
+  optional<c10::hip::HIPStreamMasqueradingAsCUDA> side;
+  hipStream_t ss = main;
+  Tensor sws, mid, s_out;
+  auto alloc_single = [&]() {
+    sws = at::empty({s_elems * es}, bytes);
+    mid = at::empty_like(s0);
+    s_out = at::empty_like(s0);
+  };
+  optional<Event> ready, done[2];
+  if (side_stream) {
+    side.emplace(c10::hip::HIPStreamMasqueradingAsCUDA::UNCHECKED, *side_stream);
+    ss = side->stream();
+    ready.emplace();
+    done[0].emplace();
+    done[1].emplace();
+    ready->record(main);   // everything the inputs depend on
+    ready->wait(ss);
+    c10::hip::HIPStreamGuardMasqueradingAsCUDA on_side(*side_stream);
+    alloc_single();        // (from the side stream's pool)
+  } else {
+    alloc_single();
+  }
+  const void* s = s0.data_ptr();
+  int k = 0;
+  for (const Block* b : blocks) {
+    float* bp = (float*)bias.data_ptr() + (int64_t)(k % ring) * bias_elems;
+    if (side_stream && k >= ring) done[k % ring]->wait(main);   // the buffer's last reader
+    b->pair_track(z, masks, batch, n, ws.data_ptr(), bp, main);
+    if (side_stream) {
+      ready->record(main);
+      ready->wait(ss);
+    }
+    b->single_track(s, mid.data_ptr(), s_out.data_ptr(), bp, s0.scalar_type(), batch, n, sws.data_ptr(), ss);
+    if (side_stream) done[k % ring]->record(ss);
+    s = s_out.data_ptr();
+    ++k;
+  }
+  if (side_stream) {
+    done[(k - 1) % ring]->wait(main);
+    c10::Stream m = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(z.device().index()).unwrap();
+    s_out.record_stream(m);   // (the other buffers are free for reuse once main is past this point)
+  }
+  return s_out;
+}
+
+// ---- single updates ----------------------------------------------------------------------------
+struct Update {
+  optional<TriMul> mul;
+  optional<TriAtt> att;
+  at::ScalarType compute;
+  Guard guard;
+  Update(const py::object& module, const py::dict& d, const py::list& attrs) {
+    if (d.contains("heads")) att.emplace(d);
+    else mul.emplace(d);
+    compute = (att ? att->packed : mul->packed).scalar_type();
+    guard.walk(module, attrs);
+  }
+  bool valid() const { return guard.valid(); }
+  // out = [z +] update for every pair tensor of z (contiguous); out may be z
+  void run(const Tensor& z, const Tensor& out, const py::list& mask_list, bool add) const {
+    const std::vector<Mask> masks = masks_of(mask_list);
+    py::gil_scoped_release nogil;
+    const int n = (int)z.size(-2), c = (int)z.size(-1);
+    const int64_t batch = n ? z.numel() / ((int64_t)n * n * c) : 0, plane = (int64_t)n * n * c * z.element_size();
+    at::DeviceGuard dev(z.device());
+    const hipStream_t st = current_stream(z);
+    const int dt = code_of_rows(z.scalar_type(), compute);
+    const int64_t es = at::elementSize(compute);
+    Tensor ws = at::empty({workspace_bytes(n, mul ? mul->c_h : 0, att ? att->heads : 0, es)}, z.options().dtype(at::kByte));
+    static const Mask none;
+    for (int64_t b = 0; b < batch; ++b) {
+      const Mask& m = masks.empty() ? none : masks[b];
+      const char* zb = (const char*)z.data_ptr() + b * plane;
+      char* ob = (char*)out.data_ptr() + b * plane;
+      if (mul) run_trimul(*mul, zb, m.m, ob, n, add, dt, es, ws.data_ptr(), st);
+      else run_triatt(*att, zb, m, ob, n, add, dt, es, ws.data_ptr(), st);
+    }
+  }
+};
+
+// ---- LayerNorm ---------------------------------------------------------------------------------
+Tensor same_as(const optional<Tensor>& t, const Tensor& x) {
+  return t && t->defined() ? t->to(x.options()).contiguous() : Tensor();
+}
+
+struct LayerNormFn : torch::autograd::Function<LayerNormFn> {
+  static Tensor forward(torch::autograd::AutogradContext* ctx, const Tensor& input, const optional<Tensor>& weight,
+                        const optional<Tensor>& bias, double eps) {
+    at::DeviceGuard dev(input.device());
+    const Tensor x = input.contiguous(), w = same_as(weight, x), b = same_as(bias, x);
+    const int64_t cols = x.size(-1), rows = cols ? x.numel() / cols : 0;
+    Tensor y = at::empty_like(x), stats = at::empty({2, rows}, x.options().dtype(at::kFloat));
+    float* st = stats.data_ptr<float>();
+    check(ptx_layernorm_fwd(ptr(x), ptr(w), ptr(b), ptr(y), st, st + rows, rows, (int)cols, (float)eps, code_of(x.scalar_type()),
+                            current_stream(x)), "layernorm");
+    ctx->save_for_backward({x, weight ? *weight : Tensor(), stats});
+    // (needs_input_grad counts the tensors that were given)
+    ctx->saved_data["w"] = weight ? (int64_t)1 : (int64_t)-1;
+    ctx->saved_data["b"] = bias ? (int64_t)(weight ? 2 : 1) : (int64_t)-1;
+    return y;
+  }
+  static torch::autograd::variable_list backward(torch::autograd::AutogradContext* ctx, torch::autograd::variable_list grads) {
+    const auto saved = ctx->get_saved_variables();
+    const Tensor &x = saved[0], &weight = saved[1], &stats = saved[2];
+    at::DeviceGuard dev(x.device());
+    const Tensor dout = grads[0].to(x.scalar_type()).contiguous();
+    const Tensor w = weight.defined() ? same_as(weight, x) : Tensor();
+    const int64_t cols = x.size(-1), rows = cols ? x.numel() / cols : 0;
+    auto needs = [&](const char* key) {
+      const int64_t i = ctx->saved_data[key].toInt();
+      return i >= 0 && ctx->needs_input_grad(i);
+    };
+    const bool need_w = needs("w"), need_b = needs("b");
+    Tensor dx = at::empty_like(x), dw, db, ws;
+    if (need_w) dw = at::empty({cols}, x.options());
+    if (need_b) db = at::empty({cols}, x.options());
+    if (need_w || need_b)
+      ws = at::empty({ptx_layernorm_bwd_workspace_elems(std::max<int64_t>(rows, 1), (int)cols)}, x.options().dtype(at::kFloat));
+    const float* st = stats.data_ptr<float>();
+    check(ptx_layernorm_bwd(ptr(dout), ptr(x), st, st + rows, ptr(w), ptr(dx), ptr(dw), ptr(db), (float*)ptr(ws), rows, (int)cols,
+                            code_of(x.scalar_type()), current_stream(x)), "layernorm_bwd");
+    return {ctx->needs_input_grad(0) ? dx : Tensor(), dw, db, Tensor()};
+  }
+};
+
+// LayerNorm over the last dimension of a GPU tensor, differentiable.
+Tensor layer_norm(const Tensor& x, const optional<Tensor>& weight, const optional<Tensor>& bias, double eps, bool grad) {
+  py::gil_scoped_release nogil;
+  if (grad) return LayerNormFn::apply(x, weight, bias, eps);
+  at::DeviceGuard dev(x.device());
+  const Tensor xc = x.contiguous(), w = same_as(weight, xc), b = same_as(bias, xc);
+  const int64_t cols = xc.size(-1), rows = cols ? xc.numel() / cols : 0;
+  Tensor y = at::empty_like(xc);
+  check(ptx_layernorm_fwd(ptr(xc), ptr(w), ptr(b), ptr(y), nullptr, nullptr, rows, (int)cols, (float)eps, code_of(xc.scalar_type()),
+                          current_stream(xc)), "layernorm");
+  return y;
+}
+
+// ---- the attention operator on standard-layout tensors ---------------------------------------------
+struct TriAttentionFn : torch::autograd::Function<TriAttentionFn> {
+  static Tensor forward(torch::autograd::AutogradContext* ctx, const Tensor& Q, const Tensor& K, const Tensor& V,
+                        const optional<Tensor>& bias1, const Tensor& bias2) {
+    at::DeviceGuard dev(Q.device());
+    const int64_t B = Q.size(0), N = Q.size(1), S = Q.size(2), H = Q.size(3), D = Q.size(4);
+    const auto type = Q.scalar_type();
+    const Tensor q = Q.contiguous(), k = K.to(type).contiguous(), v = V.to(type).contiguous();
+    const Tensor b2 = bias2.to(type).expand({B, 1, H, S, S}).contiguous();
+    const Tensor b1 = bias1 && bias1->defined() ? bias1->to(type).expand({B, N, 1, 1, S}).contiguous() : Tensor();
+    Tensor o = at::empty_like(q), m = at::empty({B, N, S, H}, q.options().dtype(at::kFloat));
+    Tensor ws = at::empty({ptx_triattn_core_workspace_elems((int)N, (int)S, (int)H)}, q.options());
+    check(ptx_triattn_core_fwd(ptr(q), ptr(k), ptr(v), ptr(b1), ptr(b2), ptr(o), (float*)ptr(m), ptr(ws), (int)B, (int)N, (int)S, (int)H,
+                               (int)D, code_of(type), current_stream(q)), "triattn_core_fwd");
+    ctx->save_for_backward({q, k, v, b1, b2, o, m});
+    ctx->saved_data["k"] = K.scalar_type();
+    ctx->saved_data["v"] = V.scalar_type();
+    ctx->saved_data["b2"] = bias2.scalar_type();
+    ctx->saved_data["b2s"] = bias2.sizes().vec();
+    ctx->saved_data["b2i"] = (int64_t)(bias1 ? 4 : 3);   // (needs_input_grad counts the tensors that were given)
+    return o;
+  }
+  static torch::autograd::variable_list backward(torch::autograd::AutogradContext* ctx, torch::autograd::variable_list grads) {
+    const auto t = ctx->get_saved_variables();
+    const Tensor &q = t[0], &k = t[1], &v = t[2], &b1 = t[3], &b2 = t[4], &o = t[5], &m = t[6];
+    at::DeviceGuard dev(q.device());
+    const int64_t B = q.size(0), N = q.size(1), S = q.size(2), H = q.size(3), D = q.size(4);
+    const Tensor dout = grads[0].to(q.scalar_type()).contiguous();
+    const bool want_b2 = ctx->needs_input_grad(ctx->saved_data["b2i"].toInt());
+    Tensor dq = at::empty_like(q), dk = at::empty_like(k), dv = at::empty_like(v), db2 = want_b2 ? at::empty_like(b2) : Tensor();
+    Tensor delta = at::empty({N * S * H}, q.options().dtype(at::kFloat));
+    check(ptx_triattn_core_bwd(ptr(q), ptr(k), ptr(v), ptr(b1), ptr(b2), ptr(o), (const float*)ptr(m), ptr(dout), ptr(dq), ptr(dk), ptr(dv),
+                               ptr(db2), (float*)ptr(delta), (int)B, (int)N, (int)S, (int)H, (int)D, code_of(q.scalar_type()),
+                               current_stream(q)), "triattn_core_bwd");
+    if (want_b2) {
+      const auto shape = ctx->saved_data["b2s"].toIntVector();
+      if (db2.sizes() != c10::IntArrayRef(shape)) db2 = at::sum_to(db2, shape);
+      db2 = db2.to(ctx->saved_data["b2"].toScalarType());
+    }
+    return {dq, dk.to(ctx->saved_data["k"].toScalarType()), dv.to(ctx->saved_data["v"].toScalarType()), Tensor(), db2};
+  }
+};
+
+Tensor tri_attention(const Tensor& q, const Tensor& k, const Tensor& v, const optional<Tensor>& b1, const Tensor& b2) {
+  py::gil_scoped_release nogil;
+  return TriAttentionFn::apply(q, k, v, b1, b2);
+}
+
+}  // namespace
+
+PYBIND11_MODULE(_host, m) {
+  m.doc() = "native host path of protenix_amd (see csrc/host.cpp)";
+  m.def("abi_version", []() { return ptx_version(); });
+  py::class_<Block>(m, "Block")
+      .def(py::init<const py::object&, const py::dict&, const py::list&>())
+      .def("valid", &Block::valid);
+  py::class_<Update>(m, "Update")
+      .def(py::init<const py::object&, const py::dict&, const py::list&>())
+      .def("valid", &Update::valid)
+      .def("run", &Update::run);
+  m.def("first_stale", [](const std::vector<const Block*>& blocks) {
+    for (size_t i = 0; i < blocks.size(); ++i)
+      if (!blocks[i]->valid()) return (int64_t)i;
+    return (int64_t)-1;
+  }, "index of the first block whose weights are no longer the module's, or -1");
+  m.def("run_blocks", &run_blocks);
+  m.def("layer_norm", &layer_norm);
+  m.def("tri_attention", &tri_attention);
+}

@@ -14,7 +14,7 @@ from typing import Optional, Union
 import torch
 import torch.nn as nn
 
-from . import ops
+from . import native, ops
 
 
 def _forward_only(*tensors: Optional[torch.Tensor], module: Optional[nn.Module] = None) -> None:
@@ -82,8 +82,11 @@ class FusedLayerNorm(nn.Module):
         if input.shape[-1] != self.normalized_shape[0]:
             raise RuntimeError(
                 f"expected last dimension {self.normalized_shape[0]}, got {tuple(input.shape)}")
-        if torch.is_grad_enabled() and any(
-                t is not None and t.requires_grad for t in (input, self.weight, self.bias)):
+        grad = torch.is_grad_enabled() and any(
+            t is not None and t.requires_grad for t in (input, self.weight, self.bias))
+        if ops.use_native() and input.is_cuda and input.numel() > 0:
+            return native.host().layer_norm(input, self.weight, self.bias, self.eps, grad)
+        if grad:
             return FusedLayerNormAffineFunction.apply(input, self.weight, self.bias,
                                                       self.normalized_shape, self.eps)
         return ops.layer_norm(input, self.weight, self.bias, self.eps)

@@ -1,0 +1,219 @@
+"""Python's side of the native host path (csrc/host.cpp): which calls it takes, and the plans - weights
+laid out for the kernels, with a record of the parameters they came from - it takes them with.
+
+Plans live here, keyed weakly by module: they are built on a module's first call, checked on every call
+(a replaced or modified parameter, a replaced sub-module or a registered hook makes a plan stale)
+and go away with the module.  What the native path does not cover returns None here and runs through
+the Python path, which has the same kernels in the same order and all the error messages.
+"""
+from __future__ import annotations
+
+import contextlib
+import threading
+import weakref
+from typing import Optional
+
+import torch
+import torch.nn.modules.module as _nn_module
+
+from . import ops
+
+_plans: "weakref.WeakKeyDictionary" = weakref.WeakKeyDictionary()
+_host = None
+_local = threading.local()
+
+
+@contextlib.contextmanager
+def off():
+    """This thread takes the Python path inside."""
+    keep = getattr(_local, "off", False)
+    _local.off = True
+    try:
+        yield
+    finally:
+        _local.off = keep
+
+# plain attributes of the modules that the plans depend on
+_ATTRS = ["inf", "no_heads", "c_hidden", "n", "n_heads", "num_heads", "c_in", "c_z", "c_s", "eps", "starting", "_outgoing",
+          "precision"]
+
+
+def host():
+    """The extension module, built together with the kernel library."""
+    global _host
+    if _host is None:
+        from . import _lib
+        lib = _lib.load()
+        try:
+            from . import _host as mod
+        except ImportError as e:
+            raise RuntimeError("protenix_amd: the native host path (_host.so) is missing or stale; rebuild with "
+                               "`python -m protenix_amd.build`") from e
+        if mod.abi_version() != lib.ptx_version():
+            raise RuntimeError("protenix_amd: _host.so and libprotenix_amd.so differ; rebuild with `python -m protenix_amd.build`")
+        _host = mod
+    return _host
+
+
+def _usable(z: torch.Tensor) -> bool:
+    return (ops.use_native() and not getattr(_local, "off", False) and z.is_cuda and not torch.is_grad_enabled() and z.dim() >= 3 and z.shape[-2] == z.shape[-3]
+            and z.numel() > 0 and z.dtype in (torch.float32, torch.bfloat16)
+            and not _nn_module._global_forward_hooks and not _nn_module._global_forward_pre_hooks)
+
+
+def _masks(z: torch.Tensor, mask: Optional[torch.Tensor], cd: torch.dtype) -> list:
+    """Per pair tensor: (mask, transposed mask, valid tokens or None) as ops.py hands them to the kernels."""
+    if mask is None:
+        return []
+    from .triangular import _per_batch
+    n = z.shape[-2]
+    out = []
+    for m in _per_batch(z, mask)[1]:
+        nv = ops.padded_tail(m, n)
+        mm = ops._mask_for(m, z, cd)
+        out.append((None, None, None) if mm is None else (mm, ops._mask_for(m, z, cd, transpose=True), nv))
+    return out
+
+
+def _mul_spec(m, cd, device) -> Optional[dict]:
+    w = m._weights(cd, device)
+    if "packed" not in w:
+        return None
+    return {**{k: w[k] for k in ("ln_in_w", "ln_in_b", "ln_out_w", "ln_out_b", "packed")}, "c_z": m.c_z, "c_h": m.c_hidden,
+            "incoming": int(not m._outgoing)}
+
+
+def _att_spec(a, cd, device, transposed: bool) -> Optional[dict]:
+    w = a._weights(cd, device)
+    if "packed" not in w:
+        return None
+    return {"ln_w": w["ln_w"], "ln_b": w["ln_b"], "packed": w["packed"], "c": a.c_in, "heads": a.no_heads, "inf": float(a.inf),
+            "transposed": int(transposed)}
+
+
+def _block_spec(blk, z: torch.Tensor, cd: torch.dtype, sd: Optional[torch.dtype]) -> Optional[dict]:
+    from .primitives import _cv
+    dev, c, tr, end = z.device, z.shape[-1], blk.pair_transition, blk.tri_att_end
+    if not (c in (64, 128) or (c == 256 and cd == torch.bfloat16)):
+        return None
+    if not (tr.c_in == c and (tr.n * c) % 64 == 0 and 0 < tr.n <= 64
+            and all(m.c_z == c for m in (blk.tri_mul_out, blk.tri_mul_in))
+            and all(a.c_in == c and a.c_hidden == 32 for a in (blk.tri_att_start, end))):
+        return None
+    spec = {"tri_mul_out": _mul_spec(blk.tri_mul_out, cd, dev), "tri_mul_in": _mul_spec(blk.tri_mul_in, cd, dev),
+            "tri_att_start": _att_spec(blk.tri_att_start, cd, dev, False), "tri_att_end": _att_spec(end, cd, dev, True),
+            "c_z": c, "c_s": blk.c_s, "n_factor": tr.n}
+    if any(v is None for v in spec.values()):
+        return None
+    spec["fused"] = int(ops.fuses_attention_transition(z, end.no_heads, end.c_hidden, tr.n))
+    if spec["fused"]:
+        t = blk._fused_weights(cd, dev)
+    else:
+        t = tr._weights(cd, dev)
+    spec.update(tr_ln_w=t["ln_w"], tr_ln_b=t["ln_b"], tr_packed=t["packed"])
+    if blk.c_s > 0:
+        apb, st = blk.attention_pair_bias, blk.single_transition
+        att, cs = apb.attention, blk.c_s
+        H, d = att.num_heads, att.c_hidden
+        lins = (att.linear_q, att.linear_k, att.linear_v, att.linear_g, att.linear_o, st.linear_no_bias_a, st.linear_no_bias_b,
+                st.linear_no_bias)
+        if not (sd in (torch.float32, torch.bfloat16) and c in (128, 256) and 1 <= apb.n_heads <= 32 and apb.n_heads == H
+                and all(l is not None and l.precision is None for l in lins)
+                and att.c_q == att.c_k == att.c_v == cs == st.c_in and cs % 16 == 0 and cs not in (64, 128, 256)
+                and d % 8 == 0 and d <= 32 and (3 * H * d) % 32 == 0 and (st.n * cs) % 16 == 0):
+            return None
+        pw = apb.pair_bias_weights(z)
+        w_in, b_q = att._fused_in(sd, dev)
+        st_ps = (st.linear_no_bias_a.weight, st.linear_no_bias_b.weight, st.linear_no_bias.weight)
+        s_wa, s_wb, s_wo = st._cache_ab.get(st_ps, sd, dev, lambda: tuple(_cv(p, sd, dev) for p in st_ps))
+        w_o = att._cache_out.get((att.linear_o.weight,), sd, dev, lambda: _cv(att.linear_o.weight, sd, dev))
+        spec.update(pb_ln_w=pw[0], pb_ln_b=pw[1], pb_w=pw[2], a_ln_w=_cv(apb.layernorm_a.weight, sd, dev),
+                    a_ln_b=_cv(apb.layernorm_a.bias, sd, dev), a_eps=float(apb.layernorm_a.eps), w_in=w_in, b_q=b_q, w_o=w_o,
+                    s_ln_w=_cv(st.layernorm1.weight, sd, dev), s_ln_b=_cv(st.layernorm1.bias, sd, dev),
+                    s_eps=float(st.layernorm1.eps), s_wa=s_wa, s_wb=s_wb, s_wo=s_wo, heads=H, d=d)
+    return spec
+
+
+def _block_plan(blk, z, cd, sd):
+    """A valid plan for this block, or None."""
+    key = (cd, sd if blk.c_s > 0 else None, z.device.index, z.dtype)
+    plans = _plans.setdefault(blk, {})
+    plan = plans.get(key)
+    if plan is None or not plan.valid():
+        spec = _block_spec(blk, z, cd, sd)
+        plan = None if spec is None else host().Block(blk, spec, _ATTRS)
+        if plan is not None and not plan.valid():      # hooks, or parameters without version counters
+            plan = None
+        plans[key] = plan
+    return plan
+
+
+def run_blocks(owner, blocks, s: Optional[torch.Tensor], z: torch.Tensor, pair_mask: Optional[torch.Tensor], side):
+    """The blocks on (s, z), z contiguous and updated in place: the new s (None without a single track), or NotImplemented
+    where the Python path is to be taken.  `owner`: the module the list of plans is kept with; `side`: None or a callable
+    that returns the second stream for the single track."""
+    # A recording is made by the Python path: its time does not count, and a recording in which the two
+    # streams wait for each other in both directions (the ring of bias buffers) is none this code relies on.
+    if not _usable(z) or not z.is_contiguous() or torch.cuda.is_current_stream_capturing():
+        return NotImplemented
+    ac = ops.autocast_compute_dtype(z)
+    cd = ops.compute_dtype(z)
+    if ac is not None and cd == z.dtype:
+        return NotImplemented
+    if pair_mask is not None and not (pair_mask.is_cuda and pair_mask.dim() >= 2):
+        return NotImplemented
+    single = any(b.c_s > 0 for b in blocks)
+    sd = None
+    if single:
+        n = z.shape[-2]
+        if s is None or not s.is_cuda or s.dim() < 2 or s.shape[-2] != n or s.numel() // (n * s.shape[-1]) != z.numel() // (
+                n * n * z.shape[-1]) or any(b.c_s != s.shape[-1] for b in blocks):
+            return NotImplemented
+        sd = s.dtype
+    key = (cd, sd, z.device.index, z.dtype)
+    kept = _plans.setdefault(owner, {}).get(("stack", key))
+    plans = None
+    if kept is not None and len(kept[0]) == len(blocks) and all(a() is b for a, b in zip(kept[0], blocks)):
+        plans = kept[1]
+        stale = host().first_stale(plans)
+        while stale >= 0:
+            plan = _block_plan(blocks[stale], z, cd, sd)
+            if plan is None:
+                return NotImplemented
+            plans[stale] = plan
+            stale = host().first_stale(plans)
+    else:
+        plans = []
+        for b in blocks:
+            plan = _block_plan(b, z, cd, sd)
+            if plan is None:
+                return NotImplemented
+            plans.append(plan)
+        _plans[owner][("stack", key)] = ([weakref.ref(b) for b in blocks], plans)
+    masks = _masks(z, pair_mask, cd)
+    stream = None
+    if side is not None and single:
+        st = side()
+        stream = (st.stream_id, st.device_index, st.device_type)
+    return host().run_blocks(plans, s.contiguous() if single else s, z, masks, stream)
+
+
+def run_update(module, z: torch.Tensor, cd: torch.dtype, mask: Optional[torch.Tensor], out: torch.Tensor, add: bool,
+               transposed: Optional[bool] = None) -> bool:
+    """One triangle update of every pair tensor of z (contiguous) into out; False: take the Python path.
+    `transposed`: None for a triangle multiplication."""
+    if not _usable(z) or (mask is not None and not mask.is_cuda):
+        return False
+    key = (cd, z.device.index, transposed)
+    plans = _plans.setdefault(module, {})
+    plan = plans.get(key)
+    if plan is None or not plan.valid():
+        spec = _mul_spec(module, cd, z.device) if transposed is None else _att_spec(module, cd, z.device, transposed)
+        if spec is None or z.shape[-1] != spec.get("c_z", spec.get("c")):
+            return False
+        plan = host().Update(module, spec, _ATTRS)
+        if not plan.valid():
+            return False
+        plans[key] = plan
+    plan.run(z, out, _masks(z, mask, cd), add)
+    return True

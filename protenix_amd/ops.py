@@ -50,6 +50,17 @@ def _stream() -> int:
 kernel_timer: Optional[dict] = None
 
 
+# The native host path (native.py): whole stacks, updates and the differentiable operators in one
+# call each.  Off while kernels are timed one by one or one of the switches below that tests throw
+# is thrown; False takes the Python path always (tests compare the two, bit for bit).
+native_enabled = True
+
+
+def use_native() -> bool:
+    return (native_enabled and kernel_timer is None and not poison_workspaces and late_gate_enabled
+            and fuse_attention_transition)
+
+
 def _call(name: str, fn, *args) -> None:
     if kernel_timer is None:
         _lib.check(fn(*args), name)

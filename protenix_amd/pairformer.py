@@ -15,7 +15,7 @@ from typing import Optional, Tuple
 import torch
 import torch.nn as nn
 
-from . import ops
+from . import native, ops
 from .primitives import Transition, _WeightCache, _cv
 from .transformer import AttentionPairBias
 from .triangular import (TriangleAttention, TriangleMultiplicationIncoming,
@@ -114,6 +114,9 @@ class PairformerBlock(nn.Module):
             return s, pad.result(z if inplace_safe else None)
         if not inplace_safe or not z.is_contiguous():
             z = z.clone(memory_format=torch.contiguous_format)
+        s_new = native.run_blocks(self, (self,), s, z, pair_mask, None)
+        if s_new is not NotImplemented:
+            return s_new, z
         return self._forward_unpadded(s, z, pair_mask, None)
 
     def _forward_unpadded(self, s, z, pair_mask, pad):
@@ -127,6 +130,19 @@ class PairformerBlock(nn.Module):
         if self.c_s > 0:
             s = self._single_track(s, bias if pad is None else pad.crop_bias(bias))
         return s, z
+
+    def _fused_weights(self, cd: torch.dtype, device: torch.device) -> dict:
+        """Weights of the launch that holds the ending node's last stage and the pair transition."""
+        att, tr = self.tri_att_end, self.pair_transition
+        ps = (att.mha.linear_g.weight, att.mha.linear_o.weight, tr.layernorm1.weight,
+              tr.layernorm1.bias, tr.linear_no_bias_a.weight, tr.linear_no_bias_b.weight,
+              tr.linear_no_bias.weight)
+
+        def make():
+            w_g, w_o, ln_w, ln_b, w_a, w_b, w_to = (_cv(p, cd, device) for p in ps)
+            return {"packed": ops.attention_transition_pack(w_g, w_o, w_a, w_b, w_to),
+                    "ln_w": ln_w, "ln_b": ln_b, "n_factor": tr.n}
+        return self._fused_cache.get(ps, cd, device, make)
 
     def _pair_track(self, z: torch.Tensor, pair_mask: Optional[torch.Tensor],
                     want_bias: bool = False) -> Optional[torch.Tensor]:
@@ -147,14 +163,7 @@ class PairformerBlock(nn.Module):
             # the ending node's last stage and the transition (and the pair bias) in one launch:
             # the tensor between the two never travels through memory
             def fused_weights(cd, device):
-                ps = (att.mha.linear_g.weight, att.mha.linear_o.weight, tr.layernorm1.weight,
-                      tr.layernorm1.bias, tr.linear_no_bias_a.weight, tr.linear_no_bias_b.weight,
-                      tr.linear_no_bias.weight)
-                def make():
-                    w_g, w_o, ln_w, ln_b, w_a, w_b, w_to = (_cv(p, cd, device) for p in ps)
-                    return {"packed": ops.attention_transition_pack(w_g, w_o, w_a, w_b, w_to),
-                            "ln_w": ln_w, "ln_b": ln_b, "n_factor": tr.n}
-                tt = dict(self._fused_cache.get(ps, cd, device, make))
+                tt = dict(self._fused_weights(cd, device))
                 tt["pair_bias_w"] = None if apb is None else apb.pair_bias_weights(z)
                 return tt
             _, biases = att._run(z, pair_mask, transposed=True, residual_inplace=True,
@@ -250,6 +259,10 @@ class PairformerStack(nn.Module):
                 "triangle_multiplicative must be 'cuequivariance' or 'torch', but got "
                 f"{triangle_multiplicative}")
         assert triangle_attention in ("torch", "deepspeed", "triattention", "cuequivariance")
+        if pad is None and len(self.blocks) > 0:
+            s_new = native.run_blocks(self, tuple(self.blocks), s, z, pair_mask, lambda: self._side_stream(z.device))
+            if s_new is not NotImplemented:
+                return s_new, z
         ac = ops.autocast_compute_dtype(z)
         if (not z.is_cuda or s is None or any(b.c_s == 0 for b in self.blocks)
                 or (ac is not None and ops.compute_dtype(z) == z.dtype)):

@@ -13,7 +13,7 @@ from typing import List, Optional, Tuple
 
 import torch
 
-from . import _lib, ops
+from . import _lib, native, ops
 from .layer_norm import _forward_only
 
 
@@ -53,6 +53,14 @@ class TriAttentionFunction(torch.autograd.Function):
     uninitialised tensor for it (op.py:120), its Bias1 being the mask bias, so a Bias1 that
     requires a gradient is refused here instead.  The kernels use no atomics: every call is
     deterministic whatever the flag says."""
+
+    @classmethod
+    def apply(cls, Q, K, V, Bias1, Bias2, deterministic=False):
+        # the same function as a C++ autograd node where nothing is to be refused
+        if (ops.use_native() and Q.is_cuda and Q.dim() == 5 and K.shape == Q.shape and V.shape == Q.shape and Q.numel() > 0
+                and Q.dtype in (torch.float32, torch.bfloat16) and not (Bias1 is not None and Bias1.requires_grad)):
+            return native.host().tri_attention(Q, K, V, Bias1, Bias2)
+        return super().apply(Q, K, V, Bias1, Bias2, deterministic)
 
     @staticmethod
     def forward(ctx, Q, K, V, Bias1, Bias2, deterministic=False):

@@ -17,7 +17,7 @@ from typing import List, Optional
 import torch
 import torch.nn as nn
 
-from . import ops
+from . import native, ops
 from .layer_norm import LayerNorm, _forward_only
 from .primitives import Linear, _cv, _WeightCache
 
@@ -146,15 +146,16 @@ class TriangleMultiplicativeUpdate(nn.Module):
         if z is not z_in and add_inplace:
             # rows rounded for the kernels: the update is added to the caller's own rows
             return z_in.add_(self.forward(z_in, mask=mask))
-        w = self._weights(cd, z.device)
         src = z if z.is_contiguous() else z.contiguous()
-        zb, mb = _per_batch(src, mask)
         out = src if add_inplace else torch.empty_like(src)
-        ob = out.view(zb.shape)
-        for bi in range(zb.shape[0]):
-            ops.triangle_multiplication(zb[bi], None if mb is None else mb[bi], w,
-                                        incoming=not self._outgoing, add_residual=add_inplace,
-                                        out=ob[bi])
+        if not native.run_update(self, src, cd, mask, out, add_inplace):
+            w = self._weights(cd, z.device)
+            zb, mb = _per_batch(src, mask)
+            ob = out.view(zb.shape)
+            for bi in range(zb.shape[0]):
+                ops.triangle_multiplication(zb[bi], None if mb is None else mb[bi], w,
+                                            incoming=not self._outgoing, add_residual=add_inplace,
+                                            out=ob[bi])
         if add_inplace and out is not z:
             z.copy_(out)
             return z
@@ -249,15 +250,16 @@ class TriangleAttention(nn.Module):
         if residual_inplace and x is not x_in:
             # rows rounded for the kernels: the update is added to the caller's own rows
             return x_in.add_(self._run(x_in, mask, transposed, residual_inplace=False))
-        w = self._weights(cd, x.device)
         src = x if x.is_contiguous() else x.contiguous()
-        xb, mb = _per_batch(src, mask)
         out = src if residual_inplace else torch.empty_like(src)
-        ob = out.view(xb.shape)
-        for bi in range(xb.shape[0]):
-            ops.triangle_attention(xb[bi], None if mb is None else mb[bi], w, self.no_heads,
-                                   self.c_hidden, self.inf, transposed=transposed,
-                                   add_residual=residual_inplace, out=ob[bi])
+        if not native.run_update(self, src, cd, mask, out, residual_inplace, transposed):
+            w = self._weights(cd, x.device)
+            xb, mb = _per_batch(src, mask)
+            ob = out.view(xb.shape)
+            for bi in range(xb.shape[0]):
+                ops.triangle_attention(xb[bi], None if mb is None else mb[bi], w, self.no_heads,
+                                       self.c_hidden, self.inf, transposed=transposed,
+                                       add_residual=residual_inplace, out=ob[bi])
         if residual_inplace and out is not x:
             x.copy_(out)
             return x
