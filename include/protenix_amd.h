@@ -34,7 +34,7 @@
 extern "C" {
 #endif
 
-#define PTX_ABI_VERSION 3
+#define PTX_ABI_VERSION 4
 #define PTX_API __attribute__((visibility("default")))
 
 /*
@@ -113,20 +113,28 @@ PTX_API int ptx_layernorm_fwd(const void* x, const void* gamma, const void* beta
  *     (x [c][n][ldx]); ptx_trimul_output_packed takes ldx = n rounded up to a multiple of 8.
  *   ptx_triattn_late_gate: 1 where the output stage forms the gate itself; ptx_triattn_project_packed
  *     then takes g = NULL and ptx_triattn_output_packed an ungated o.
+ *   carry: NULL, or a stage of the single-representation track (ptx_single_*_stage, operands of
+ *     the pair rows' storage type) that the launch runs along: on workgroups of its own, so it
+ *     must not depend on this launch nor this launch on it.
  */
+typedef struct ptx_single_stage {
+  int64_t opaque[32];
+} ptx_single_stage;
 PTX_API int64_t ptx_trimul_packed_elems(int c_z, int c_hidden);
 PTX_API int ptx_trimul_pack(const void* w_ap, const void* w_ag, const void* w_bp, const void* w_bg,
                       const void* w_z, const void* w_g, void* packed, int c_z, int c_hidden, int dtype,
                       void* stream);
 PTX_API int ptx_trimul_project_packed(const void* z, const void* mask, const void* ln_w, const void* ln_b,
                       const void* packed, void* a, void* b, int n, int c_z, int c_hidden,
-                      int k_pitch, int incoming, float eps, int dtype, void* stream);
+                      int k_pitch, int incoming, float eps, int dtype,
+                      const ptx_single_stage* carry, void* stream);
 PTX_API int ptx_trimul_contract_ld(const void* a, const void* b, void* x, int n, int ldx, int c, int k_pitch,
                       int dtype, void* stream);
 PTX_API int ptx_trimul_output_packed(const void* x, int ldx, const void* z, const void* ln_in_w,
                       const void* ln_in_b, const void* ln_out_w, const void* ln_out_b,
                       const void* packed, void* out, int n, int c_z, int c_hidden, int add_residual,
-                      float eps, int dtype, void* stream);
+                      float eps, int dtype,
+                      const ptx_single_stage* carry, void* stream);
 PTX_API int64_t ptx_triattn_packed_elems(int c_in, int heads);
 PTX_API int ptx_triattn_late_gate(int c_in, int heads, int dtype);
 PTX_API int ptx_triattn_pack(const void* w_q, const void* w_k, const void* w_v, const void* w_g,
@@ -134,10 +142,12 @@ PTX_API int ptx_triattn_pack(const void* w_q, const void* w_k, const void* w_v, 
                       void* stream);
 PTX_API int ptx_triattn_project_packed(const void* z, const void* ln_w, const void* ln_b, const void* packed,
                       void* q, void* k, void* vt, void* g, void* tri_bias, int n, int c_in, int heads,
-                      int key_pitch, int transposed, float eps, int dtype, void* stream);
+                      int key_pitch, int transposed, float eps, int dtype,
+                      const ptx_single_stage* carry, void* stream);
 PTX_API int ptx_triattn_output_packed(const void* o, const void* z, const void* ln_w, const void* ln_b,
                       const void* packed, void* out, int n, int c_in, int heads, int transposed,
-                      int add_residual, float eps, int dtype, void* stream);
+                      int add_residual, float eps, int dtype,
+                      const ptx_single_stage* carry, void* stream);
 
 /*
  * LayerNorm backward.  Replaces fast_layer_norm_cuda_v2.backward_{none,with_bias,with_weight,
@@ -455,6 +465,28 @@ PTX_API int ptx_swiglu_fwd(const void* x, const void* w_a, const void* w_b, void
 PTX_API int ptx_single_attention_fwd(const void* q, const void* k, const void* vt, const void* g,
                    const void* bias, int bias_f32, void* out, int n, int heads, int d, int64_t ld,
                    int64_t ldt, int64_t ldo, float scale, int dtype, void* stream);
+
+/*
+ * The same operations as descriptions (nothing is launched; the pointers are kept), to be run by
+ * ptx_single_stage_run or carried by a ptx_*_packed launch.
+ *   ptx_single_layernorm_stage: ptx_layernorm_fwd, the same bits (rows of up to 512 fp32 or 1024 bf16
+ *     values in whole 16-byte vectors, else PTX_ERR_UNSUPPORTED).
+ *   ptx_single_linear_stage: ptx_linear_fwd, with w2 != NULL ptx_swiglu_fwd.
+ *     packed = 1: w (w2) in the kernel's fragment order, which it reads several times as fast:
+ *     [n_out / 16][k / 32][piece][4][16][V] with V = 4 fp32 or 8 bf16 values in 16 bytes and element
+ *     (column block, step, piece, g, c, e) = w[16 block + c][32 step + 4 V piece + V g + e]; k a multiple
+ *     of 32, n_out of 16.
+ *   ptx_single_attention_stage: ptx_single_attention_fwd.
+ */
+PTX_API int ptx_single_layernorm_stage(ptx_single_stage* stage, const void* x, const void* gamma,
+                   const void* beta, void* y, int rows, int cols, float eps, int dtype);
+PTX_API int ptx_single_linear_stage(ptx_single_stage* stage, const void* x, const void* w, const void* w2,
+                   const void* bias, int bias_cols, const void* res, void* out, void* out_t, int split_col, int64_t ldt,
+                   int rows, int k, int n_out, int dtype, int packed);
+PTX_API int ptx_single_attention_stage(ptx_single_stage* stage, const void* q, const void* k, const void* vt,
+                   const void* g, const void* bias, int bias_f32, void* out, int n, int heads, int d,
+                   int64_t ld, int64_t ldt, int64_t ldo, float scale, int dtype);
+PTX_API int ptx_single_stage_run(const ptx_single_stage* stage, void* stream);
 
 /*
  * Measurement aid with no counterpart in the reference: streams `bytes` (a multiple of 16)

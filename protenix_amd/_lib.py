@@ -14,7 +14,7 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libprotenix_amd.so")
 
 PTX_F32, PTX_BF16, PTX_MIXED, PTX_F16 = 0, 1, 2, 3
-ABI_VERSION = 3
+ABI_VERSION = 4
 
 _p = ctypes.c_void_p
 _i = ctypes.c_int
@@ -37,14 +37,14 @@ SIGNATURES = {
     "ptx_trimul_contract": (_i, [_p, _p, _p, _i, _i, _i, _i, _p]),
     "ptx_trimul_packed_elems": (_l, [_i, _i]),
     "ptx_trimul_pack": (_i, [_p] * 7 + [_i, _i, _i, _p]),
-    "ptx_trimul_project_packed": (_i, [_p] * 7 + [_i, _i, _i, _i, _i, _f, _i, _p]),
+    "ptx_trimul_project_packed": (_i, [_p] * 7 + [_i, _i, _i, _i, _i, _f, _i, _p, _p]),
     "ptx_trimul_contract_ld": (_i, [_p, _p, _p, _i, _i, _i, _i, _i, _p]),
-    "ptx_trimul_output_packed": (_i, [_p, _i] + [_p] * 7 + [_i, _i, _i, _i, _f, _i, _p]),
+    "ptx_trimul_output_packed": (_i, [_p, _i] + [_p] * 7 + [_i, _i, _i, _i, _f, _i, _p, _p]),
     "ptx_triattn_packed_elems": (_l, [_i, _i]),
     "ptx_triattn_late_gate": (_i, [_i, _i, _i]),
     "ptx_triattn_pack": (_i, [_p] * 7 + [_i, _i, _i, _p]),
-    "ptx_triattn_project_packed": (_i, [_p] * 9 + [_i, _i, _i, _i, _i, _f, _i, _p]),
-    "ptx_triattn_output_packed": (_i, [_p] * 6 + [_i, _i, _i, _i, _i, _f, _i, _p]),
+    "ptx_triattn_project_packed": (_i, [_p] * 9 + [_i, _i, _i, _i, _i, _f, _i, _p, _p]),
+    "ptx_triattn_output_packed": (_i, [_p] * 6 + [_i, _i, _i, _i, _i, _f, _i, _p, _p]),
     "ptx_trimul_output": (_i, [_p] * 9 + [_i, _i, _i, _i, _f, _i, _p]),
     "ptx_triangle_multiplicative_update_workspace_elems": (_l, [_i, _i]),
     "ptx_triangle_multiplicative_update": (_i, [_p, _i] + [_p] * 11 + [_i, _i, _i, _i, _f, _i, _p]),
@@ -64,6 +64,10 @@ SIGNATURES = {
     "ptx_triattn_output_transition_fwd": (_i, [_p] * 8 + [_i, _i, _i, _i, _i, _f, _f, _p, _p, _p, _p, _i, _i,
                                                _f, _i, _p]),
     "ptx_transition_pair_bias_fwd": (_i, [_p] * 5 + [_l, _i, _i, _i, _f, _p, _p, _p, _p, _i, _i, _f, _i, _p]),
+    "ptx_single_layernorm_stage": (_i, [_p, _p, _p, _p, _p, _i, _i, _f, _i]),
+    "ptx_single_linear_stage": (_i, [_p, _p, _p, _p, _p, _i, _p, _p, _p, _i, _l, _i, _i, _i, _i, _i]),
+    "ptx_single_attention_stage": (_i, [_p, _p, _p, _p, _p, _p, _i, _p, _i, _i, _i, _l, _l, _l, _f, _i]),
+    "ptx_single_stage_run": (_i, [_p, _p]),
     "ptx_linear_fwd": (_i, [_p, _p, _p, _i, _p, _p, _p, _i, _l, _i, _i, _i, _i, _p]),
     "ptx_swiglu_fwd": (_i, [_p, _p, _p, _p, _i, _i, _i, _i, _p]),
     "ptx_single_attention_fwd": (_i, [_p, _p, _p, _p, _p, _i, _p, _i, _i, _i, _l, _l, _l, _f, _i, _p]),

@@ -409,9 +409,16 @@ PTX_API int ptx_trimul_pack(const void* w_ap, const void* w_ag, const void* w_bp
   return after_launch("trimul_pack");
 }
 
+// (a carried stage works on operands of the rows' type)
+static bool carry_ok(const ptx_single_stage* carry, int dtype) {
+  const ptx::SingleStage* st = (const ptx::SingleStage*)carry;
+  return !st || st->kind == ptx::kStageNone || (st->bits16 != 0) == (dtype == PTX_BF16);
+}
+
 PTX_API int ptx_trimul_project_packed(const void* z, const void* mask, const void* ln_w, const void* ln_b,
                                       const void* packed, void* a, void* b, int n, int c_z, int c_hidden,
-                                      int k_pitch, int incoming, float eps, int dtype, void* stream) {
+                                      int k_pitch, int incoming, float eps, int dtype,
+                                     const ptx_single_stage* carry, void* stream) {
   PTX_REQUIRE(dtype_ok_z(dtype), PTX_ERR_BAD_ARG, "trimul_project_packed: unknown dtype %d", dtype);
   PTX_REQUIRE(n >= 0, PTX_ERR_BAD_ARG, "trimul_project_packed: n=%d", n);
   PTX_REQUIRE(pair_width_ok(c_z, c_hidden, dtype), PTX_ERR_UNSUPPORTED,
@@ -424,14 +431,17 @@ PTX_API int ptx_trimul_project_packed(const void* z, const void* mask, const voi
   PTX_REQUIRE(aligned16(z) && aligned16(packed) && aligned16(a) && aligned16(b) && (!ln_w || aligned16(ln_w)) &&
                   (!ln_b || aligned16(ln_b)),
               PTX_ERR_BAD_ARG, "trimul_project_packed: pointers must be 16-byte aligned");
+  PTX_REQUIRE(carry_ok(carry, dtype), PTX_ERR_BAD_ARG, "trimul_project_packed: the carried stage must be of the pair tensor's type");
   PTX_DISPATCH_Z(dtype, (ptx::pp_trimul_in<T, TZ>)(z, mask, ln_w, ln_b, packed, a, b, n, c_z, k_pitch, incoming, eps,
+                                                   (const ptx::SingleStage*)carry,
                                                    (hipStream_t)stream));
   return after_launch("trimul_project_packed");
 }
 
 PTX_API int ptx_trimul_output_packed(const void* x, int ldx, const void* z, const void* ln_in_w, const void* ln_in_b,
                                      const void* ln_out_w, const void* ln_out_b, const void* packed, void* out, int n,
-                                     int c_z, int c_hidden, int add_residual, float eps, int dtype, void* stream) {
+                                     int c_z, int c_hidden, int add_residual, float eps, int dtype,
+                                     const ptx_single_stage* carry, void* stream) {
   PTX_REQUIRE(dtype_ok_z(dtype), PTX_ERR_BAD_ARG, "trimul_output_packed: unknown dtype %d", dtype);
   PTX_REQUIRE(n >= 0, PTX_ERR_BAD_ARG, "trimul_output_packed: n=%d", n);
   PTX_REQUIRE(pair_width_ok(c_z, c_hidden, dtype), PTX_ERR_UNSUPPORTED,
@@ -443,8 +453,10 @@ PTX_API int ptx_trimul_output_packed(const void* x, int ldx, const void* z, cons
   PTX_REQUIRE(aligned16(x) && aligned16(out) && aligned16(z) && aligned16(packed) && (!ln_out_w || aligned16(ln_out_w)) &&
                   (!ln_out_b || aligned16(ln_out_b)) && (!ln_in_w || aligned16(ln_in_w)) && (!ln_in_b || aligned16(ln_in_b)),
               PTX_ERR_BAD_ARG, "trimul_output_packed: pointers must be 16-byte aligned");
+  PTX_REQUIRE(carry_ok(carry, dtype), PTX_ERR_BAD_ARG, "trimul_output_packed: the carried stage must be of the pair tensor's type");
   PTX_DISPATCH_Z(dtype, (ptx::pp_trimul_out<T, TZ>)(x, ldx, z, ln_in_w, ln_in_b, ln_out_w, ln_out_b, packed, out, n, c_z,
-                                                    c_hidden, add_residual, eps, (hipStream_t)stream));
+                                                    c_hidden, add_residual, eps, (const ptx::SingleStage*)carry,
+                                                   (hipStream_t)stream));
   return after_launch("trimul_output_packed");
 }
 
@@ -470,7 +482,8 @@ PTX_API int ptx_triattn_pack(const void* w_q, const void* w_k, const void* w_v, 
 
 PTX_API int ptx_triattn_project_packed(const void* z, const void* ln_w, const void* ln_b, const void* packed, void* q,
                                        void* k, void* vt, void* g, void* tri_bias, int n, int c_in, int heads,
-                                       int key_pitch, int transposed, float eps, int dtype, void* stream) {
+                                       int key_pitch, int transposed, float eps, int dtype,
+                                     const ptx_single_stage* carry, void* stream) {
   PTX_REQUIRE(dtype_ok_z(dtype), PTX_ERR_BAD_ARG, "triattn_project_packed: unknown dtype %d", dtype);
   PTX_REQUIRE(n >= 0, PTX_ERR_BAD_ARG, "triattn_project_packed: n=%d", n);
   PTX_REQUIRE(heads > 0 && heads <= 8 && pair_width_ok(c_in, heads * 32, dtype), PTX_ERR_UNSUPPORTED,
@@ -485,14 +498,17 @@ PTX_API int ptx_triattn_project_packed(const void* z, const void* ln_w, const vo
   PTX_REQUIRE(aligned16(z) && aligned16(packed) && aligned16(q) && aligned16(k) && aligned16(vt) && (!g || aligned16(g)) &&
                   aligned16(tri_bias) && (!ln_w || aligned16(ln_w)) && (!ln_b || aligned16(ln_b)),
               PTX_ERR_BAD_ARG, "triattn_project_packed: pointers must be 16-byte aligned");
+  PTX_REQUIRE(carry_ok(carry, dtype), PTX_ERR_BAD_ARG, "triattn_project_packed: the carried stage must be of the pair tensor's type");
   PTX_DISPATCH_Z(dtype, (ptx::pp_triattn_in<T, TZ>)(z, ln_w, ln_b, packed, q, k, vt, g, tri_bias, n, c_in, heads,
-                                                    key_pitch, transposed, eps, (hipStream_t)stream));
+                                                    key_pitch, transposed, eps, (const ptx::SingleStage*)carry,
+                                                   (hipStream_t)stream));
   return after_launch("triattn_project_packed");
 }
 
 PTX_API int ptx_triattn_output_packed(const void* o, const void* z, const void* ln_w, const void* ln_b,
                                       const void* packed, void* out, int n, int c_in, int heads, int transposed,
-                                      int add_residual, float eps, int dtype, void* stream) {
+                                      int add_residual, float eps, int dtype,
+                                     const ptx_single_stage* carry, void* stream) {
   PTX_REQUIRE(dtype_ok_z(dtype), PTX_ERR_BAD_ARG, "triattn_output_packed: unknown dtype %d", dtype);
   PTX_REQUIRE(n >= 0, PTX_ERR_BAD_ARG, "triattn_output_packed: n=%d", n);
   PTX_REQUIRE(heads > 0 && heads <= 8 && pair_width_ok(c_in, heads * 32, dtype), PTX_ERR_UNSUPPORTED,
@@ -503,8 +519,10 @@ PTX_API int ptx_triattn_output_packed(const void* o, const void* z, const void* 
   PTX_REQUIRE(aligned16(o) && aligned16(z) && aligned16(packed) && aligned16(out) && (!ln_w || aligned16(ln_w)) &&
                   (!ln_b || aligned16(ln_b)),
               PTX_ERR_BAD_ARG, "triattn_output_packed: pointers must be 16-byte aligned");
+  PTX_REQUIRE(carry_ok(carry, dtype), PTX_ERR_BAD_ARG, "triattn_output_packed: the carried stage must be of the pair tensor's type");
   PTX_DISPATCH_Z(dtype, (ptx::pp_triattn_out<T, TZ>)(o, z, ln_w, ln_b, packed, out, n, c_in, heads, transposed,
-                                                     add_residual, eps, (hipStream_t)stream));
+                                                     add_residual, eps, (const ptx::SingleStage*)carry,
+                                                   (hipStream_t)stream));
   return after_launch("triattn_output_packed");
 }
 
@@ -783,57 +801,62 @@ PTX_API int ptx_triattn_output_transition_fwd(const void* o, const void* z, cons
   return after_launch("triattn_output_transition");
 }
 
-PTX_API int ptx_linear_fwd(const void* x, const void* w, const void* bias, int bias_cols,
-                           const void* res, void* out, void* out_t, int split_col, int64_t ldt,
-                           int rows, int k, int n_out, int dtype, void* stream) {
+static_assert(sizeof(ptx::SingleStage) <= sizeof(ptx_single_stage), "ptx_single_stage is too small");
+
+PTX_API int ptx_single_layernorm_stage(ptx_single_stage* stage, const void* x, const void* gamma, const void* beta, void* y,
+                                       int rows, int cols, float eps, int dtype) {
+  PTX_REQUIRE(dtype_ok(dtype), PTX_ERR_BAD_ARG, "layernorm_stage: unknown dtype %d", dtype);
+  PTX_REQUIRE(stage && rows >= 0 && cols > 0, PTX_ERR_BAD_ARG, "layernorm_stage: rows=%d cols=%d", rows, cols);
+  PTX_REQUIRE(rows == 0 || (x && y && aligned16(x) && aligned16(y) && (!gamma || aligned16(gamma)) && (!beta || aligned16(beta))),
+              PTX_ERR_BAD_ARG, "layernorm_stage: pointers must be given and 16-byte aligned");
+  const int rc = ptx::single_stage_layernorm((ptx::SingleStage*)stage, x, gamma, beta, y, rows, cols, eps, dtype == PTX_BF16);
+  PTX_REQUIRE(rc == 0, PTX_ERR_UNSUPPORTED, "layernorm_stage: rows of %d", cols);
+  return PTX_OK;
+}
+
+PTX_API int ptx_single_linear_stage(ptx_single_stage* stage, const void* x, const void* w, const void* w2, const void* bias,
+                                    int bias_cols, const void* res, void* out, void* out_t, int split_col, int64_t ldt, int rows, int k,
+                                    int n_out, int dtype, int packed) {
   PTX_REQUIRE(dtype_ok(dtype), PTX_ERR_BAD_ARG, "linear: unknown dtype %d", dtype);
+  PTX_REQUIRE(stage, PTX_ERR_BAD_ARG, "linear: null stage");
   PTX_REQUIRE(rows >= 0 && k > 0 && n_out >= 0, PTX_ERR_BAD_ARG, "linear: rows=%d k=%d n_out=%d",
               rows, k, n_out);
   PTX_REQUIRE(k % 16 == 0 && n_out % 8 == 0, PTX_ERR_UNSUPPORTED,
               "linear: k must be a multiple of 16 and n_out of 8 (got k=%d n_out=%d)", k, n_out);
+  PTX_REQUIRE(!packed || (k % 32 == 0 && n_out % 16 == 0), PTX_ERR_UNSUPPORTED,
+              "linear: packed weights need k %% 32 == 0 and n_out %% 16 == 0 (got k=%d n_out=%d)", k, n_out);
   if (split_col < 0 || split_col > n_out) split_col = n_out;
-  if (rows == 0 || n_out == 0) return PTX_OK;
-  PTX_REQUIRE(x && w && (out || split_col == 0), PTX_ERR_BAD_ARG, "linear: null pointer");
-  if (split_col < n_out) {
-    PTX_REQUIRE(out_t, PTX_ERR_BAD_ARG, "linear: out_t is null");
-    PTX_REQUIRE(split_col % 32 == 0 && ldt % 8 == 0 && ldt >= rows && !res, PTX_ERR_BAD_ARG,
-                "linear: transposed tail needs split_col %% 32 == 0, ldt %% 8 == 0, ldt >= rows and "
-                "no residual (split_col=%d ldt=%lld)", split_col, (long long)ldt);
-    PTX_REQUIRE(aligned16(out_t), PTX_ERR_BAD_ARG, "linear: out_t must be 16-byte aligned");
+  if (rows > 0 && n_out > 0) {
+    PTX_REQUIRE(x && w && (out || split_col == 0), PTX_ERR_BAD_ARG, "linear: null pointer");
+    if (split_col < n_out) {
+      PTX_REQUIRE(out_t, PTX_ERR_BAD_ARG, "linear: out_t is null");
+      PTX_REQUIRE(split_col % 32 == 0 && ldt % 8 == 0 && ldt >= rows && !res && !w2, PTX_ERR_BAD_ARG,
+                  "linear: transposed tail needs split_col %% 32 == 0, ldt %% 8 == 0, ldt >= rows and "
+                  "no residual (split_col=%d ldt=%lld)", split_col, (long long)ldt);
+      PTX_REQUIRE(aligned16(out_t), PTX_ERR_BAD_ARG, "linear: out_t must be 16-byte aligned");
+    }
+    PTX_REQUIRE(aligned16(x) && aligned16(w) && (!w2 || aligned16(w2)) && (!out || aligned16(out)) && (!res || aligned16(res)),
+                PTX_ERR_BAD_ARG, "linear: pointers must be 16-byte aligned");
   }
-  PTX_REQUIRE(aligned16(x) && aligned16(w) && (!out || aligned16(out)) && (!res || aligned16(res)),
-              PTX_ERR_BAD_ARG, "linear: pointers must be 16-byte aligned");
-  PTX_DISPATCH(dtype, ptx::linear_fwd<T>(x, w, bias, bias ? bias_cols : 0, res, out, out_t,
-                                         split_col, ldt, rows, k, n_out, (hipStream_t)stream));
-  return after_launch("linear");
+  ptx::single_stage_linear((ptx::SingleStage*)stage, x, w, w2, bias, bias ? bias_cols : 0, res, out, out_t, split_col, ldt, rows, k,
+                           n_out, dtype == PTX_BF16, packed);
+  return PTX_OK;
 }
 
-PTX_API int ptx_swiglu_fwd(const void* x, const void* w_a, const void* w_b, void* out, int rows,
-                           int k, int hidden, int dtype, void* stream) {
-  PTX_REQUIRE(dtype_ok(dtype), PTX_ERR_BAD_ARG, "swiglu: unknown dtype %d", dtype);
-  PTX_REQUIRE(rows >= 0 && k > 0 && hidden >= 0, PTX_ERR_BAD_ARG, "swiglu: rows=%d k=%d hidden=%d",
-              rows, k, hidden);
-  PTX_REQUIRE(k % 16 == 0 && hidden % 8 == 0, PTX_ERR_UNSUPPORTED,
-              "swiglu: k must be a multiple of 16 and hidden of 8 (got k=%d hidden=%d)", k, hidden);
-  if (rows == 0 || hidden == 0) return PTX_OK;
-  PTX_REQUIRE(x && w_a && w_b && out, PTX_ERR_BAD_ARG, "swiglu: null pointer");
-  PTX_REQUIRE(aligned16(x) && aligned16(w_a) && aligned16(w_b) && aligned16(out), PTX_ERR_BAD_ARG,
-              "swiglu: pointers must be 16-byte aligned");
-  PTX_DISPATCH(dtype, ptx::swiglu_fwd<T>(x, w_a, w_b, out, rows, k, hidden, (hipStream_t)stream));
-  return after_launch("swiglu");
-}
-
-PTX_API int ptx_single_attention_fwd(const void* q, const void* k, const void* vt, const void* g,
-                                     const void* bias, int bias_f32, void* out, int n, int heads,
-                                     int d, int64_t ld, int64_t ldt, int64_t ldo, float scale,
-                                     int dtype, void* stream) {
+PTX_API int ptx_single_attention_stage(ptx_single_stage* stage, const void* q, const void* k, const void* vt, const void* g,
+                                       const void* bias, int bias_f32, void* out, int n, int heads, int d, int64_t ld,
+                                       int64_t ldt, int64_t ldo, float scale, int dtype) {
   PTX_REQUIRE(dtype_ok(dtype), PTX_ERR_BAD_ARG, "single_attention: unknown dtype %d", dtype);
+  PTX_REQUIRE(stage, PTX_ERR_BAD_ARG, "single_attention: null stage");
   PTX_REQUIRE(n >= 0 && heads >= 0, PTX_ERR_BAD_ARG, "single_attention: n=%d heads=%d", n, heads);
   PTX_REQUIRE(d > 0 && d <= 32 && d % 8 == 0, PTX_ERR_UNSUPPORTED,
               "single_attention: head dim must be 8, 16, 24 or 32 (got %d)", d);
   PTX_REQUIRE(n <= 32768 && heads <= 65535, PTX_ERR_UNSUPPORTED, "single_attention: n=%d heads=%d too large",
               n, heads);
-  if (n == 0 || heads == 0) return PTX_OK;
+  if (n == 0 || heads == 0) {
+    *(ptx::SingleStage*)stage = ptx::SingleStage{};
+    return PTX_OK;
+  }
   PTX_REQUIRE(q && k && vt && out, PTX_ERR_BAD_ARG, "single_attention: null pointer");
   PTX_REQUIRE(ld % 8 == 0 && ldo % 8 == 0 && ldt % 8 == 0 && ldt >= ((n + 31) / 32) * 32 &&
                   ld >= (int64_t)heads * d && ldo >= (int64_t)heads * d,
@@ -843,9 +866,42 @@ PTX_API int ptx_single_attention_fwd(const void* q, const void* k, const void* v
               (long long)ld, (long long)ldt, (long long)ldo);
   PTX_REQUIRE(aligned16(q) && aligned16(k) && aligned16(vt) && aligned16(out) && (!g || aligned16(g)),
               PTX_ERR_BAD_ARG, "single_attention: pointers must be 16-byte aligned");
-  PTX_DISPATCH(dtype, ptx::single_attention_fwd<T>(q, k, vt, g, bias, bias_f32, out, n, heads, d, ld,
-                                                   ldt, ldo, scale, (hipStream_t)stream));
-  return after_launch("single_attention");
+  ptx::single_stage_attention((ptx::SingleStage*)stage, q, k, vt, g, bias, bias_f32, out, n, heads, d, ld, ldt, ldo, scale,
+                              dtype == PTX_BF16);
+  return PTX_OK;
+}
+
+PTX_API int ptx_single_stage_run(const ptx_single_stage* stage, void* stream) {
+  PTX_REQUIRE(stage, PTX_ERR_BAD_ARG, "single_stage_run: null stage");
+  ptx::single_stage_run((const ptx::SingleStage*)stage, (hipStream_t)stream);
+  return after_launch("single_stage_run");
+}
+
+PTX_API int ptx_linear_fwd(const void* x, const void* w, const void* bias, int bias_cols,
+                           const void* res, void* out, void* out_t, int split_col, int64_t ldt,
+                           int rows, int k, int n_out, int dtype, void* stream) {
+  ptx_single_stage st;
+  const int rc = ptx_single_linear_stage(&st, x, w, nullptr, bias, bias_cols, res, out, out_t, split_col,
+                                         ldt, rows, k, n_out, dtype, 0);
+  return rc != PTX_OK ? rc : ptx_single_stage_run(&st, stream);
+}
+
+PTX_API int ptx_swiglu_fwd(const void* x, const void* w_a, const void* w_b, void* out, int rows,
+                           int k, int hidden, int dtype, void* stream) {
+  PTX_REQUIRE(w_b || rows == 0 || hidden == 0, PTX_ERR_BAD_ARG, "swiglu: null pointer");
+  ptx_single_stage st;
+  const int rc = ptx_single_linear_stage(&st, x, w_a, w_b, nullptr, 0, nullptr, out, nullptr, hidden, 0,
+                                         rows, k, hidden, dtype, 0);
+  return rc != PTX_OK ? rc : ptx_single_stage_run(&st, stream);
+}
+
+PTX_API int ptx_single_attention_fwd(const void* q, const void* k, const void* vt, const void* g,
+                                     const void* bias, int bias_f32, void* out, int n, int heads,
+                                     int d, int64_t ld, int64_t ldt, int64_t ldo, float scale,
+                                     int dtype, void* stream) {
+  ptx_single_stage st;
+  const int rc = ptx_single_attention_stage(&st, q, k, vt, g, bias, bias_f32, out, n, heads, d, ld, ldt, ldo, scale, dtype);
+  return rc != PTX_OK ? rc : ptx_single_stage_run(&st, stream);
 }
 
 PTX_API int ptx_pair_bias_fwd(const void* z, const void* ln_w, const void* ln_b, const void* w, void* bias,

@@ -10,7 +10,6 @@
 // The kernels, their order and their arguments are those of ops.py.
 #include <torch/extension.h>
 
-#include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 
 #include "../../include/protenix_amd.h"
@@ -174,26 +173,45 @@ int64_t workspace_bytes(int n, int c_h, int heads, int64_t es) {
 
 constexpr float kEps = 1e-5f;
 
+// The stages of the single tracks of earlier blocks, in order: every pair launch that can carry one takes the
+// first, so that a block's single track runs underneath the next block's pair kernels without launches,
+// streams or waits of its own.
+struct Stages {
+  std::vector<ptx_single_stage> list;
+  size_t next = 0;
+  const ptx_single_stage* take() { return next < list.size() ? &list[next++] : nullptr; }
+  ptx_single_stage* add() {
+    list.emplace_back();
+    return &list.back();
+  }
+  void run_rest(hipStream_t st) {
+    while (const ptx_single_stage* s = take()) check(ptx_single_stage_run(s, st), "single_stage");
+    list.clear();
+    next = 0;
+  }
+};
+
 void run_trimul(const TriMul& w, const void* z, const Tensor& mask, void* out, int n, bool add, int dt, int64_t es, void* ws,
-                hipStream_t st) {
+                Stages& singles, hipStream_t st) {
   Cut c{(char*)ws};
   TriMulWs s(c, n, w.c_h, es);
   const int pitch = ptx_key_pitch(n), ldx = (n + 7) / 8 * 8;
   check(ptx_trimul_project_packed(z, ptr(mask), ptr(w.ln_in_w), ptr(w.ln_in_b), ptr(w.packed), s.a, s.b, n, w.c_z, w.c_h, pitch,
-                                  w.incoming, kEps, dt, st), "trimul_project");
+                                  w.incoming, kEps, dt, singles.take(), st), "trimul_project");
   check(ptx_trimul_contract_ld(s.a, s.b, s.x, n, ldx, w.c_h, pitch, dt, st), "trimul_contract");
   check(ptx_trimul_output_packed(s.x, ldx, z, ptr(w.ln_in_w), ptr(w.ln_in_b), ptr(w.ln_out_w), ptr(w.ln_out_b), ptr(w.packed), out, n,
-                                 w.c_z, w.c_h, add, kEps, dt, st), "trimul_output");
+                                 w.c_z, w.c_h, add, kEps, dt, singles.take(), st), "trimul_output");
 }
 
 // projection and core; the attention output is left in ws.g
-TriAttWs run_triatt_core(const TriAtt& w, const void* z, const Mask& mask, int n, int dt, int64_t es, void* ws, hipStream_t st) {
+TriAttWs run_triatt_core(const TriAtt& w, const void* z, const Mask& mask, int n, int dt, int64_t es, void* ws, Stages& singles,
+                         hipStream_t st) {
   Cut c{(char*)ws};
   TriAttWs s(c, n, w.heads, es);
   const int pitch = ptx_key_pitch(n);
   void* gate = ptx_triattn_late_gate(w.c, w.heads, dt) ? nullptr : s.g;
   check(ptx_triattn_project_packed(z, ptr(w.ln_w), ptr(w.ln_b), ptr(w.packed), s.q, s.k, s.vt, gate, s.tb, n, w.c, w.heads, pitch,
-                                   w.transposed, kEps, dt, st), "triattn_project");
+                                   w.transposed, kEps, dt, singles.take(), st), "triattn_project");
   const void* m = ptr(w.transposed ? mask.mt : mask.m);
   if (m && mask.n_valid >= 0) {
     // padding at the end: valid rows over valid keys without a mask, padded rows with it (ops.py)
@@ -208,21 +226,22 @@ TriAttWs run_triatt_core(const TriAtt& w, const void* z, const Mask& mask, int n
 }
 
 void run_triatt(const TriAtt& w, const void* z, const Mask& mask, void* out, int n, bool add, int dt, int64_t es, void* ws,
-                hipStream_t st) {
-  const TriAttWs s = run_triatt_core(w, z, mask, n, dt, es, ws, st);
+                Stages& singles, hipStream_t st) {
+  const TriAttWs s = run_triatt_core(w, z, mask, n, dt, es, ws, singles, st);
   check(ptx_triattn_output_packed(s.g, z, ptr(w.ln_w), ptr(w.ln_b), ptr(w.packed), out, n, w.c, w.heads, w.transposed, add, kEps, dt,
-                                  st), "triattn_output");
+                                  singles.take(), st), "triattn_output");
 }
 
 // ---- one Pairformer block ----------------------------------------------------------------------
 struct Block {
+  struct SingleWs;
   TriMul out, in;
   TriAtt start, end;
   // pair transition (fused: with the ending node's output stage in front, one launch)
   bool fused;
   Tensor tr_ln_w, tr_ln_b, tr_packed;
-  int n_factor, c_z, c_s;
-  // single track
+  int n_factor, c_z, c_s, hidden = 0;
+  // single track (matrices packed for ptx_single_linear_stage)
   Tensor pb_ln_w, pb_ln_b, pb_w, a_ln_w, a_ln_b, w_in, b_q, w_o, s_ln_w, s_ln_b, s_wa, s_wb, s_wo;
   int heads = 0, d = 0;
   double a_eps = kEps, s_eps = kEps;
@@ -243,6 +262,7 @@ struct Block {
       s_wa = take(d_, "s_wa"); s_wb = take(d_, "s_wb"); s_wo = take(d_, "s_wo");
       heads = take_int(d_, "heads");
       d = take_int(d_, "d");
+      hidden = take_int(d_, "hidden");
       a_eps = d_["a_eps"].cast<double>();
       s_eps = d_["s_eps"].cast<double>();
     }
@@ -252,20 +272,22 @@ struct Block {
 
   // The five pair updates of the pair tensors of z [batch][n][n][c_z] in place; the single attention's pair
   // bias (fp32 [batch][heads][n][n]) of the finished z into `bias` (null: none wanted).
-  void pair_track(const Tensor& z, const std::vector<Mask>& masks, int64_t batch, int n, void* ws, float* bias, hipStream_t st) const {
+  void pair_track(const Tensor& z, const std::vector<Mask>& masks, int64_t batch, int n, void* ws, float* bias, Stages& singles,
+                  hipStream_t st) const {
     const int dt = code_of_rows(z.scalar_type(), compute);
     const int64_t es = at::elementSize(compute), plane = (int64_t)n * n * c_z * z.element_size();
     char* zp = (char*)z.data_ptr();
     static const Mask none;
     auto mask = [&](int64_t b) -> const Mask& { return masks.empty() ? none : masks[b]; };
-    for (int64_t b = 0; b < batch; ++b) run_trimul(out, zp + b * plane, mask(b).m, zp + b * plane, n, true, dt, es, ws, st);
-    for (int64_t b = 0; b < batch; ++b) run_trimul(in, zp + b * plane, mask(b).m, zp + b * plane, n, true, dt, es, ws, st);
-    for (int64_t b = 0; b < batch; ++b) run_triatt(start, zp + b * plane, mask(b), zp + b * plane, n, true, dt, es, ws, st);
+    for (int64_t b = 0; b < batch; ++b) run_trimul(out, zp + b * plane, mask(b).m, zp + b * plane, n, true, dt, es, ws, singles, st);
+    for (int64_t b = 0; b < batch; ++b) run_trimul(in, zp + b * plane, mask(b).m, zp + b * plane, n, true, dt, es, ws, singles, st);
+    for (int64_t b = 0; b < batch; ++b) run_triatt(start, zp + b * plane, mask(b), zp + b * plane, n, true, dt, es, ws, singles, st);
     const int64_t bias_plane = (int64_t)heads * n * n;
     if (fused) {
       for (int64_t b = 0; b < batch; ++b) {
         void* zb = zp + b * plane;
-        const TriAttWs s = run_triatt_core(end, zb, mask(b), n, dt, es, ws, st);
+        const TriAttWs s = run_triatt_core(end, zb, mask(b), n, dt, es, ws, singles, st);
+        if (b == 0) singles.run_rest(st);   // (the bias is about to be rewritten)
         check(ptx_triattn_output_transition_fwd(s.g, zb, ptr(end.ln_w), ptr(end.ln_b), ptr(tr_packed), ptr(tr_ln_w), ptr(tr_ln_b), zb, n,
                                                 c_z, end.heads, end.transposed, n_factor, kEps, kEps, bias ? ptr(pb_ln_w) : nullptr,
                                                 bias ? ptr(pb_ln_b) : nullptr, bias ? ptr(pb_w) : nullptr,
@@ -274,7 +296,8 @@ struct Block {
       }
       return;
     }
-    for (int64_t b = 0; b < batch; ++b) run_triatt(end, zp + b * plane, mask(b), zp + b * plane, n, true, dt, es, ws, st);
+    for (int64_t b = 0; b < batch; ++b) run_triatt(end, zp + b * plane, mask(b), zp + b * plane, n, true, dt, es, ws, singles, st);
+    singles.run_rest(st);   // (the bias is about to be rewritten)
     check(ptx_transition_fwd(zp, ptr(tr_ln_w), ptr(tr_ln_b), ptr(tr_packed), zp, batch * n * n, c_z, n_factor, 1, kEps, dt, st),
           "transition");
     if (bias)
@@ -283,134 +306,96 @@ struct Block {
               "pair_bias");
   }
 
-  // elements of s' type that single_track() wants as scratch
-  int64_t single_elems(int64_t batch, int n) const {
-    const int64_t rows = batch * n, hd = (int64_t)heads * d, ldt = (n + 31) / 32 * 32;
-    auto up = [](int64_t e) { return (e + 63) / 64 * 64; };
-    return up(rows * c_s) + up((int64_t)n * 3 * hd) + up(hd * ldt) + up(rows * hd) + up(rows * s_wa.size(0));
+  // bytes single_track() wants as scratch
+  int64_t single_bytes(int64_t batch, int n, int64_t es) const {
+    Cut c{nullptr};
+    SingleWs(c, *this, batch, n, es);
+    return c.used;
   }
-  // mid = s + attention(s; bias); s_out = mid + transition(mid)
-  void single_track(const void* s, void* mid, void* s_out, const float* bias, at::ScalarType type, int64_t batch, int n, void* ws,
-                    hipStream_t st) const {
-    const int dt = code_of(type), hd = heads * d, ldt = (n + 31) / 32 * 32, hidden = (int)s_wa.size(0);
+  struct SingleWs {
+    char *y, *qkg, *vt, *o, *h;
+    int64_t qkg_plane, vt_plane, o_plane;   // bytes per batch element
+    SingleWs(Cut& c, const Block& b, int64_t batch, int n, int64_t es) {
+      const int64_t hd = (int64_t)b.heads * b.d, ldt = (n + 31) / 32 * 32;
+      qkg_plane = (int64_t)n * 3 * hd * es;
+      vt_plane = hd * ldt * es;
+      o_plane = (int64_t)n * hd * es;
+      y = (char*)c.part(batch * n * b.c_s * es);
+      qkg = (char*)c.part(batch * qkg_plane);
+      vt = (char*)c.part(batch * vt_plane);
+      o = (char*)c.part(batch * o_plane);
+      h = (char*)c.part(batch * n * b.hidden * es);
+    }
+  };
+  // The stages of: mid = s + attention(LN(s); bias); s_out = mid + transition(LN(mid))
+  void single_track(Stages& st, const void* s, void* mid, void* s_out, const float* bias, at::ScalarType type, int64_t batch, int n,
+                    void* ws) const {
+    const int dt = code_of(type), hd = heads * d, ldt = (n + 31) / 32 * 32;
     const int64_t es = at::elementSize(type), rows = batch * n;
     Cut c{(char*)ws};
-    void* y = c.part(rows * c_s * es);
-    void* qkg = c.part((int64_t)n * 3 * hd * es);
-    void* vt = c.part((int64_t)hd * ldt * es);
-    void* o = c.part(rows * hd * es);
-    void* h = c.part(rows * hidden * es);
-    check(ptx_layernorm_fwd(s, ptr(a_ln_w), ptr(a_ln_b), y, nullptr, nullptr, rows, c_s, (float)a_eps, dt, st), "layernorm");
+    const SingleWs w(c, *this, batch, n, es);
+    check(ptx_single_layernorm_stage(st.add(), s, ptr(a_ln_w), ptr(a_ln_b), w.y, (int)rows, c_s, (float)a_eps, dt), "layernorm");
     for (int64_t b = 0; b < batch; ++b) {
-      check(ptx_linear_fwd((char*)y + b * n * c_s * es, ptr(w_in), ptr(b_q), hd, nullptr, qkg, vt, 3 * hd, ldt, n, c_s, 4 * hd, dt, st),
-            "linear");
-      check(ptx_single_attention_fwd(qkg, (char*)qkg + hd * es, vt, (char*)qkg + 2 * (int64_t)hd * es, bias + b * heads * (int64_t)n * n, 1,
-                                     (char*)o + b * n * hd * es, n, heads, d, 3 * hd, ldt, hd, (float)(1.0 / std::sqrt((double)d)), dt, st),
-            "single_attention");
+      char* qkg = w.qkg + b * w.qkg_plane;
+      check(ptx_single_linear_stage(st.add(), w.y + b * n * c_s * es, ptr(w_in), nullptr, ptr(b_q), hd, nullptr, qkg, w.vt + b * w.vt_plane, 3 * hd, ldt, n, c_s, 4 * hd, dt, 1), "linear");
     }
-    check(ptx_linear_fwd(o, ptr(w_o), nullptr, 0, s, mid, nullptr, c_s, 0, (int)rows, hd, c_s, dt, st), "linear");
-    check(ptx_layernorm_fwd(mid, ptr(s_ln_w), ptr(s_ln_b), y, nullptr, nullptr, rows, c_s, (float)s_eps, dt, st), "layernorm");
-    check(ptx_swiglu_fwd(y, ptr(s_wa), ptr(s_wb), h, (int)rows, c_s, hidden, dt, st), "swiglu");
-    check(ptx_linear_fwd(h, ptr(s_wo), nullptr, 0, mid, s_out, nullptr, c_s, 0, (int)rows, hidden, c_s, dt, st), "linear");
+    for (int64_t b = 0; b < batch; ++b) {
+      char* qkg = w.qkg + b * w.qkg_plane;
+      check(ptx_single_attention_stage(st.add(), qkg, qkg + hd * es, w.vt + b * w.vt_plane, qkg + 2 * hd * es,
+                                       bias + b * heads * (int64_t)n * n, 1, w.o + b * w.o_plane, n, heads, d, 3 * hd, ldt, hd,
+                                       (float)(1.0 / std::sqrt((double)d)), dt), "single_attention");
+    }
+    check(ptx_single_linear_stage(st.add(), w.o, ptr(w_o), nullptr, nullptr, 0, s, mid, nullptr, c_s, 0,
+                                  (int)rows, hd, c_s, dt, 1), "linear");
+    check(ptx_single_layernorm_stage(st.add(), mid, ptr(s_ln_w), ptr(s_ln_b), w.y, (int)rows, c_s, (float)s_eps, dt), "layernorm");
+    check(ptx_single_linear_stage(st.add(), w.y, ptr(s_wa), ptr(s_wb), nullptr, 0, nullptr,
+                                  w.h, nullptr, hidden, 0, (int)rows, c_s, hidden, dt, 1), "swiglu");
+    check(ptx_single_linear_stage(st.add(), w.h, ptr(s_wo), nullptr, nullptr, 0, mid, s_out, nullptr, c_s, 0,
+                                  (int)rows, hidden, c_s, dt, 1), "linear");
   }
 };
 
-// Events of one call, each recorded on one stream only; handed back to the runtime at its end.
-struct Event {
-  hipEvent_t e = nullptr;
-  Event() {
-    if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) throw std::runtime_error("hipEventCreate failed");
-  }
-  ~Event() { (void)hipEventDestroy(e); }
-  void record(hipStream_t s) { hip(hipEventRecord(e, s)); }
-  void wait(hipStream_t s) { hip(hipStreamWaitEvent(s, e, 0)); }
-  static void hip(hipError_t r) {
-    if (r != hipSuccess) throw std::runtime_error(std::string("hipEvent: ") + hipGetErrorString(r));
-  }
-};
-
-// The blocks in sequence on z (contiguous, updated in place).  `side` = (stream id, device index, device type) of a second
-// stream for the single track, which then runs underneath the next block's pair kernels, or None.  Returns the
-// new s (undefined for a stack without a single track).  Not for a stream that is being captured (native.py)
-optional<Tensor> run_blocks(const std::vector<const Block*>& blocks, const optional<Tensor>& s_opt, const Tensor& z, const py::list& mask_list,
-                            const py::object& side_obj) {
+// The blocks in sequence on z (contiguous, updated in place).  The single track of a block runs underneath the next
+// block's pair kernels (see Stages).  Returns the new s (undefined for a stack without a single track).
+optional<Tensor> run_blocks(const std::vector<const Block*>& blocks, const optional<Tensor>& s_opt, const Tensor& z, const py::list& mask_list) {
   const std::vector<Mask> masks = masks_of(mask_list);
-  optional<c10::Stream> side_stream;
-  if (!side_obj.is_none()) {
-    py::tuple t = py::reinterpret_borrow<py::tuple>(side_obj);
-    side_stream = c10::Stream::unpack3(t[0].cast<int64_t>(), (c10::DeviceIndex)t[1].cast<int>(), (c10::DeviceType)t[2].cast<int>());
-  }
   py::gil_scoped_release nogil;
   const int n = (int)z.size(-2);
   const int64_t batch = z.numel() / ((int64_t)n * n * z.size(-1));
   at::DeviceGuard dev(z.device());
-  const hipStream_t main = current_stream(z);
-  int64_t ws_bytes = 0;
-  bool single = false;
-  int64_t s_elems = 0, bias_elems = 0;
+  const hipStream_t st = current_stream(z);
+  const bool single = s_opt.has_value() && s_opt->defined() && blocks[0]->c_s > 0;
+  const int64_t es = single ? (int64_t)s_opt->element_size() : 0;
+  int64_t ws_bytes = 0, single_bytes = 0, bias_elems = 0;
   for (const Block* b : blocks) {
     ws_bytes = std::max(ws_bytes, workspace_bytes(n, std::max(b->out.c_h, b->in.c_h), std::max(b->start.heads, b->end.heads),
                                                   at::elementSize(b->compute)));
-    if (b->c_s) {
-      single = true;
-      s_elems = std::max(s_elems, b->single_elems(batch, n));
+    if (single) {
+      single_bytes = std::max(single_bytes, b->single_bytes(batch, n, es));
       bias_elems = std::max(bias_elems, batch * b->heads * (int64_t)n * n);
     }
   }
   const auto bytes = z.options().dtype(at::kByte);
-  Tensor ws = at::empty({ws_bytes}, bytes);
-  if (!single) {
-    for (const Block* b : blocks) b->pair_track(z, masks, batch, n, ws.data_ptr(), nullptr, main);
-    return s_opt;
+  Tensor ws = at::empty({ws_bytes}, bytes), bias, sws, mid, s_out;
+  const void* s = nullptr;
+  if (single) {
+    bias = at::empty({bias_elems}, z.options().dtype(at::kFloat));
+    sws = at::empty({single_bytes}, bytes);
+    mid = at::empty_like(*s_opt);
+    s_out = at::empty_like(*s_opt);
+    s = s_opt->data_ptr();
   }
-  const Tensor& s0 = *s_opt;
-  const int64_t es = s0.element_size();
-  // The pair bias travels from the main stream to the side stream through a ring of two buffers.
-  const int ring = side_stream ? 2 : 1;
-  Tensor bias = at::empty({ring, bias_elems}, z.options().dtype(at::kFloat));
-  optional<c10::hip::HIPStreamMasqueradingAsCUDA> side;
-  hipStream_t ss = main;
-  Tensor sws, mid, s_out;
-  auto alloc_single = [&]() {
-    sws = at::empty({s_elems * es}, bytes);
-    mid = at::empty_like(s0);
-    s_out = at::empty_like(s0);
-  };
-  optional<Event> ready, done[2];
-  if (side_stream) {
-    side.emplace(c10::hip::HIPStreamMasqueradingAsCUDA::UNCHECKED, *side_stream);
-    ss = side->stream();
-    ready.emplace();
-    done[0].emplace();
-    done[1].emplace();
-    ready->record(main);   // everything the inputs depend on
-    ready->wait(ss);
-    c10::hip::HIPStreamGuardMasqueradingAsCUDA on_side(*side_stream);
-    alloc_single();        // (from the side stream's pool)
-  } else {
-    alloc_single();
-  }
-  const void* s = s0.data_ptr();
-  int k = 0;
+  Stages singles;
   for (const Block* b : blocks) {
-    float* bp = (float*)bias.data_ptr() + (int64_t)(k % ring) * bias_elems;
-    if (side_stream && k >= ring) done[k % ring]->wait(main);   // the buffer's last reader
-    b->pair_track(z, masks, batch, n, ws.data_ptr(), bp, main);
-    if (side_stream) {
-      ready->record(main);
-      ready->wait(ss);
+    float* bp = single ? (float*)bias.data_ptr() : nullptr;
+    b->pair_track(z, masks, batch, n, ws.data_ptr(), bp, singles, st);
+    if (single) {
+      b->single_track(singles, s, mid.data_ptr(), s_out.data_ptr(), bp, s_opt->scalar_type(), batch, n, sws.data_ptr());
+      s = s_out.data_ptr();
     }
-    b->single_track(s, mid.data_ptr(), s_out.data_ptr(), bp, s0.scalar_type(), batch, n, sws.data_ptr(), ss);
-    if (side_stream) done[k % ring]->record(ss);
-    s = s_out.data_ptr();
-    ++k;
   }
-  if (side_stream) {
-    done[(k - 1) % ring]->wait(main);
-    c10::Stream m = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(z.device().index()).unwrap();
-    s_out.record_stream(m);   // (the other buffers are free for reuse once main is past this point)
-  }
-  return s_out;
+  singles.run_rest(st);
+  return single ? optional<Tensor>(s_out) : s_opt;
 }
 
 // ---- single updates ----------------------------------------------------------------------------
@@ -438,12 +423,13 @@ struct Update {
     const int64_t es = at::elementSize(compute);
     Tensor ws = at::empty({workspace_bytes(n, mul ? mul->c_h : 0, att ? att->heads : 0, es)}, z.options().dtype(at::kByte));
     static const Mask none;
+    Stages no_singles;
     for (int64_t b = 0; b < batch; ++b) {
       const Mask& m = masks.empty() ? none : masks[b];
       const char* zb = (const char*)z.data_ptr() + b * plane;
       char* ob = (char*)out.data_ptr() + b * plane;
-      if (mul) run_trimul(*mul, zb, m.m, ob, n, add, dt, es, ws.data_ptr(), st);
-      else run_triatt(*att, zb, m, ob, n, add, dt, es, ws.data_ptr(), st);
+      if (mul) run_trimul(*mul, zb, m.m, ob, n, add, dt, es, ws.data_ptr(), no_singles, st);
+      else run_triatt(*att, zb, m, ob, n, add, dt, es, ws.data_ptr(), no_singles, st);
     }
   }
 };

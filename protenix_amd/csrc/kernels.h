@@ -81,7 +81,45 @@ template <typename T, typename TZ = T>
 int pair_bias_fwd(const void* z, const void* ln_w, const void* ln_b, const void* w, void* bias,
                   int n, int c_z, int heads, int out_f32, float eps, hipStream_t stream);
 
-// The row-local stages of the triangle updates on packed weights (pairproj.hip).
+// One stage of the single-representation track (single_stage.h): filled by the functions below, run by single_stage_run
+// in a launch of its own or carried by one of the pp_* launches.
+enum { kStageNone = 0, kStageLinear = 1, kStageSwiGLU = 2, kStageAttention = 3, kStageLayerNorm = 4 };
+struct SingleStage {
+  int kind, n_work;       // n_work workgroups
+  int packed;             // linear: w, w2 in fragment order (single_stage.h; n_out % 16 == 0, k % 32 == 0)
+  int tile, row_blocks;   // linear: tiles of 16 x 16, 16 x 32, 32 x 32 (1, 2, 3); tiles over the rows
+  int bits16;             // operands bf16, else fp32
+  int rows;               // layernorm, linear: rows of x; attention: queries = keys
+  const void* x;          // layernorm, linear: [rows][k]; attention: q, rows of pitch ld
+  const void* w;          // layernorm: gamma or null; linear: [n_out][k]; attention: k, rows of pitch ld
+  const void* w2;         // layernorm: beta or null; SwiGLU: the second matrix; attention: V^T [heads * d][ldt], keys beyond `rows` hold zeros
+  const void* bias;       // linear: [bias_cols] or null, added to output columns < bias_cols; attention: [heads][n][n] or null
+  const void* res;        // [rows][n_out] or null
+  const void* gate;       // attention: gate logits, rows of pitch ld, or null
+  void* out;              // rows of pitch ldo: output columns < split_col
+  void* out_t;            // [n_out - split_col][ldt]: output columns >= split_col, transposed; rows in [rows, ldt) written as zeros
+  int64_t ld, ldo, ldt;
+  int k, n_out, split_col, bias_cols;   // split_col: a multiple of 32, or n_out (nothing is transposed)
+  int ln_g, ln_nc;        // layernorm: how rows lie over lanes (lnrow.h)
+  float eps;
+  int heads, d, bias_f32, bias_vec;     // bias_vec: rows of the bias can be read as 16-byte vectors
+  float scale;
+};
+// workgroups a launch gives the stage: whole rounds over the 8 XCDs, so that the others keep their places
+inline unsigned single_stage_groups(const SingleStage* s) { return s && s->kind ? (unsigned)(s->n_work + 7) / 8 * 8 : 0u; }
+// 0, or -1 where the rows do not fit the stage
+int single_stage_layernorm(SingleStage* s, const void* x, const void* gamma, const void* beta, void* y, int rows, int cols,
+                           float eps, bool bits16);
+void single_stage_linear(SingleStage* s, const void* x, const void* w, const void* w2, const void* bias, int bias_cols,
+                         const void* res, void* out, void* out_t, int split_col, int64_t ldt, int rows, int k, int n_out,
+                         bool bits16, int packed);
+void single_stage_attention(SingleStage* s, const void* q, const void* k, const void* vt, const void* gate, const void* bias,
+                            int bias_f32, void* out, int n, int heads, int d, int64_t ld, int64_t ldt, int64_t ldo,
+                            float scale, bool bits16);
+int single_stage_run(const SingleStage* s, hipStream_t stream);
+
+// The row-local stages of the triangle updates on packed weights (pairproj.hip).  carry: null, or a stage of the single
+// track on operands of type TZ that this launch's first workgroups run (it must not depend on the launch).
 // Whether the attention's gate is formed by the output stage (no gate tensor exists then).
 inline bool pp_late_gate(int c_z, int heads, bool bits16) { return c_z == 128 && heads == 4 && bits16; }
 int64_t pp_trimul_packed_elems(int c_z, int hidden);
@@ -94,38 +132,20 @@ int pp_triattn_pack(const void* w_q, const void* w_k, const void* w_v, const voi
                     const void* w_o, void* packed, int c_z, int heads, hipStream_t stream);
 template <typename T, typename TZ = T>
 int pp_trimul_in(const void* z, const void* mask, const void* ln_w, const void* ln_b, const void* packed, void* a,
-                 void* b, int n, int c_z, int k_pitch, int incoming, float eps, hipStream_t stream);
+                 void* b, int n, int c_z, int k_pitch, int incoming, float eps, const SingleStage* carry, hipStream_t stream);
 template <typename T, typename TZ = T>
 int pp_triattn_in(const void* z, const void* ln_w, const void* ln_b, const void* packed, void* q, void* k, void* vt,
                   void* g, void* tri_bias, int n, int c_z, int heads, int key_pitch, int transposed, float eps,
-                  hipStream_t stream);
+                  const SingleStage* carry, hipStream_t stream);
 // x [hidden][n][ldx]: ldx = n, or n rounded up to a multiple of 8 (rows of any n then start aligned)
 template <typename T, typename TZ = T>
 int pp_trimul_out(const void* x, int ldx, const void* z, const void* ln_in_w, const void* ln_in_b,
                   const void* ln_out_w, const void* ln_out_b, const void* packed, void* out, int n, int c_z,
-                  int hidden, int add_residual, float eps, hipStream_t stream);
+                  int hidden, int add_residual, float eps, const SingleStage* carry, hipStream_t stream);
 template <typename T, typename TZ = T>
 int pp_triattn_out(const void* o, const void* z, const void* ln_w, const void* ln_b, const void* packed, void* out,
-                   int n, int c_z, int heads, int transposed, int add_residual, float eps, hipStream_t stream);
-
-// Small linear layers of the single-representation track (single.hip):
-//   out[rows][n_out] = [res +] x[rows][k] w[n_out][k]^T [+ bias on columns < bias_cols];
-//   output columns >= split_col go, transposed, to out_t[n_out - split_col][ldt] instead
-//   (rows in [rows, ldt) written as zeros); out then has split_col columns.
-template <typename T>
-int linear_fwd(const void* x, const void* w, const void* bias, int bias_cols, const void* res,
-               void* out, void* out_t, int split_col, int64_t ldt, int rows, int k, int n_out,
-               hipStream_t stream);
-//   out[rows][hidden] = silu(x w_a^T) * (x w_b^T)
-template <typename T>
-int swiglu_fwd(const void* x, const void* w_a, const void* w_b, void* out, int rows, int k,
-               int hidden, hipStream_t stream);
-// out[n][heads*d] = sigmoid(g) * softmax_k(q k^T * scale + bias[h]) v per head; q, k, g rows of
-// pitch ld, vt [heads*d][ldt] (keys beyond n hold zeros), bias [heads][n][n] fp32 or T.
-template <typename T>
-int single_attention_fwd(const void* q, const void* k, const void* vt, const void* g,
-                         const void* bias, int bias_f32, void* out, int n, int heads, int d,
-                         int64_t ld, int64_t ldt, int64_t ldo, float scale, hipStream_t stream);
+                   int n, int c_z, int heads, int transposed, int add_residual, float eps, const SingleStage* carry,
+                   hipStream_t stream);
 
 // x[c][i][j] = sum_k a[c][i][k] * b[c][j][k] for `batch` independent products;
 // a, b rows have pitch k_pitch (a multiple of 64, >= n), x is [batch][n][ldx].

@@ -13,6 +13,7 @@
 
 #include "common.h"
 #include "kernels.h"
+#include "lnrow.h"
 
 namespace ptx {
 
@@ -121,7 +122,7 @@ __global__ __launch_bounds__(256) void layernorm_fwd_kernel(
 #pragma unroll
           for (int e = 0; e < VEC; ++e) {
             const float d = v[c][e] - mean;
-            q += d * d;
+            q = __builtin_fmaf(d, d, q);
           }
         }
       }
@@ -136,24 +137,21 @@ __global__ __launch_bounds__(256) void layernorm_fwd_kernel(
         for (int c = 0; c < NCHUNK; ++c) {
           const int col = (c * G + sub) * VEC;
           if (col < cols) {
-            F o;
-#pragma unroll
-            for (int e = 0; e < VEC; ++e) o[e] = (v[c][e] - mean) * rstd;
+            F o, g1, b1;
             if (HOIST) {
-#pragma unroll
-              for (int e = 0; e < VEC; ++e) o[e] = o[e] * gm[c][e] + bt[c][e];
+              g1 = gm[c];
+              b1 = bt[c];
             } else {
-              if (gamma) {
-                F g1 = __builtin_convertvector(*reinterpret_cast<const V*>(gamma + col), F);
 #pragma unroll
-                for (int e = 0; e < VEC; ++e) o[e] *= g1[e];
+              for (int e = 0; e < VEC; ++e) {
+                g1[e] = 1.0f;
+                b1[e] = 0.0f;
               }
-              if (beta) {
-                F b1 = __builtin_convertvector(*reinterpret_cast<const V*>(beta + col), F);
-#pragma unroll
-                for (int e = 0; e < VEC; ++e) o[e] += b1[e];
-              }
+              if (gamma) g1 = __builtin_convertvector(*reinterpret_cast<const V*>(gamma + col), F);
+              if (beta) b1 = __builtin_convertvector(*reinterpret_cast<const V*>(beta + col), F);
             }
+#pragma unroll
+            for (int e = 0; e < VEC; ++e) o[e] = ln_affine(v[c][e], mean, rstd, g1[e], b1[e]);
             V* p = reinterpret_cast<V*>(y + row * cols + col);
             const V ov = __builtin_convertvector(o, V);
             if (NT) __builtin_nontemporal_store(ov, p); else *p = ov;
@@ -249,9 +247,7 @@ static bool dispatch_ln_vec(const T* x, const T* gamma, const T* beta, T* y, flo
     launch_ln<T, VEC, G, NC>(x, gamma, beta, y, mean, rstd, rows, cols, eps, stream);       \
     return true;                                                                            \
   }
-  PTX_LN_CASE(1, 1) PTX_LN_CASE(2, 1) PTX_LN_CASE(4, 1) PTX_LN_CASE(8, 1) PTX_LN_CASE(16, 1)
-  PTX_LN_CASE(32, 1) PTX_LN_CASE(16, 2) PTX_LN_CASE(16, 3) PTX_LN_CASE(64, 1) PTX_LN_CASE(64, 2) PTX_LN_CASE(64, 4)
-  PTX_LN_CASE(64, 8)
+  PTX_LN_LAYOUTS(PTX_LN_CASE)
 #undef PTX_LN_CASE
   return false;
 }

@@ -17,6 +17,7 @@
 #include "common.h"
 #include "kernels.h"
 #include "rowpieces.h"
+#include "single_stage.h"
 #include <algorithm>
 #include <type_traits>
 
@@ -25,6 +26,18 @@ namespace ptx {
 namespace {
 
 constexpr int kPpWaves = 4;
+static_assert(kPpWaves == kStageWaves, "workgroups of both kinds in one launch");
+constexpr int cmax(int a, int b) { return a > b ? a : b; }
+// The launch's first `carried` workgroups run a stage of the single track (not on rows of 64 channels: no stack
+// of that width has one, and the attention's kernel would spill).
+#define PTX_CARRIED_STAGE()                          \
+  if constexpr (KS > 4) {                            \
+    if (blockIdx.x < carried) {                      \
+      single_stage<TZ>(carry, blockIdx.x, smem);     \
+      return;                                        \
+    }                                                \
+  }                                                  \
+  const uint32_t block = blockIdx.x - carried, blocks = gridDim.x - carried
 
 // Hidden widths (see Widths in rowgemm.hip): 128 for rows of at most 128 channels, else the row width.
 template <int KS> struct PpWidths {
@@ -86,22 +99,25 @@ struct ProjInParams {
 // a, b[c][i][k] = mask * sigmoid(gate) * projection in the contraction's fragment order.  Tile: a patch of 4 * RBW
 // outer indices i x 8 inner indices k, which makes a row block's 32 values of one channel 64 contiguous bytes.
 template <typename T, typename TZ, int KS, int RBW>
-__global__ __launch_bounds__(kPpWaves * 64, (sizeof(T) == 2 && KS <= 8 ? 3 : 1)) void pp_trimul_in_kernel(ProjInParams p) {
+__global__ __launch_bounds__(kPpWaves * 64, (sizeof(T) == 2 && KS <= 8 ? 3 : 1)) void pp_trimul_in_kernel(ProjInParams p, SingleStage carry, unsigned carried) {
   typedef typename Vec8<T>::type V8;
   typedef typename VecE<T>::type VE_t;
   typedef Cfg<T> C;
   constexpr int CPM = PpWidths<KS>::HIDDEN / 32;    // chunks (of 32 channels) per operand
   constexpr int CHW = 2 * CPM / kPpWaves;           // chunks per wave
-  __shared__ __attribute__((aligned(16))) char frag[RBW * FragLds<T, KS>::ROWBLOCK];
-  __shared__ __attribute__((aligned(16))) T stage[kPpWaves][32 * C::PITCH];
-  __shared__ __attribute__((aligned(16))) float lmask[32 * RBW];
+  constexpr int kFrag = RBW * FragLds<T, KS>::ROWBLOCK, kStage = kPpWaves * 32 * C::PITCH * (int)sizeof(T);
+  __shared__ __attribute__((aligned(16))) char smem[cmax(kFrag + kStage + 128 * RBW, kStageLds)];
+  PTX_CARRIED_STAGE();
+  char* const frag = smem;
+  T (*stage)[32 * C::PITCH] = reinterpret_cast<T (*)[32 * C::PITCH]>(smem + kFrag);
+  float* const lmask = reinterpret_cast<float*>(smem + kFrag + kStage);
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int g = lane >> 5;
   const int n = p.n;
   const uint32_t n_kb = (uint32_t)p.pitch >> 3, n_ip = (uint32_t)(n + 4 * RBW - 1) / (4 * RBW);
   // Patches in the order of the memory rows they read, back to front behind a kernel that wrote the pair tensor
   // front to back (the tail is what the memory-side cache still holds).
-  const uint32_t bx = xcd_run(blockIdx.x, gridDim.x), tile = p.backward ? gridDim.x - 1 - bx : bx;
+  const uint32_t bx = xcd_run(block, blocks), tile = p.backward ? blocks - 1 - bx : bx;
   int pi0, pk0;
   if (p.backward) {   // incoming: the inner index is the slow one of z
     const uint32_t kb = tile / n_ip;
@@ -190,19 +206,22 @@ __global__ __launch_bounds__(kPpWaves * 64, (sizeof(T) == 2 && KS <= 8 ? 3 : 1))
 
 // q (scaled), K, V^T, triangle bias and (GATE) sigmoid(gate) in the attention core's layouts.
 template <typename T, typename TZ, int KS, int RBW, bool GATE>
-__global__ __launch_bounds__(kPpWaves * 64, (sizeof(T) == 2 && KS <= 8 ? 3 : 1)) void pp_triattn_in_kernel(ProjInParams p) {
+__global__ __launch_bounds__(kPpWaves * 64, (sizeof(T) == 2 && KS <= 8 ? 3 : 1)) void pp_triattn_in_kernel(ProjInParams p, SingleStage carry, unsigned carried) {
   typedef typename Vec8<T>::type V8;
   typedef typename VecE<T>::type VE_t;
   typedef Cfg<T> C;
   constexpr int HP = PpWidths<KS>::HEADS / 2;            // pairs of heads
   constexpr int NPAIR = (GATE ? 4 : 3) * HP + 1;         // q, k, v (, gate): HP pairs of tiles each; the bias: one tile
-  __shared__ __attribute__((aligned(16))) char frag[RBW * FragLds<T, KS>::ROWBLOCK];
-  __shared__ __attribute__((aligned(16))) T stage[kPpWaves][2][32 * C::PITCH];
+  constexpr int kFrag = RBW * FragLds<T, KS>::ROWBLOCK, kStage = kPpWaves * 2 * 32 * C::PITCH * (int)sizeof(T);
+  __shared__ __attribute__((aligned(16))) char smem[cmax(kFrag + kStage, kStageLds)];
+  PTX_CARRIED_STAGE();
+  char* const frag = smem;
+  T (*stage)[2][32 * C::PITCH] = reinterpret_cast<T (*)[2][32 * C::PITCH]>(smem + kFrag);
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int n = p.n;
   const int64_t n_rows = (int64_t)n * n;
-  const uint32_t bx = xcd_run(blockIdx.x, gridDim.x);
-  const int64_t tile = p.backward ? gridDim.x - 1 - bx : bx;
+  const uint32_t bx = xcd_run(block, blocks);
+  const int64_t tile = p.backward ? blocks - 1 - bx : bx;
   const TileRows tr = tile_rows(tile, 32 * RBW, n, p.tiles_per_i);
   const T* packed = (const T*)p.packed;
   V8 w[2][KS];
@@ -340,19 +359,22 @@ struct ProjOutParams {
 
 // out = [z +] (W_z LN_out(x)) * sigmoid(W_g LN_in(z)); out may be z.
 template <typename T, typename TZ, int KS, int RBW>
-__global__ __launch_bounds__(kPpWaves * 64, (sizeof(T) == 2 && KS <= 8 ? 3 : 1)) void pp_trimul_out_kernel(ProjOutParams p) {
+__global__ __launch_bounds__(kPpWaves * 64, (sizeof(T) == 2 && KS <= 8 ? 3 : 1)) void pp_trimul_out_kernel(ProjOutParams p, SingleStage carry, unsigned carried) {
   typedef typename Vec8<T>::type V8;
   typedef typename VecE<T>::type VE_t;
   typedef Cfg<T> C;
   constexpr int SL = PpWidths<KS>::SL, HIDDEN = PpWidths<KS>::HIDDEN, NOB = KS / 2;
   constexpr int XP = 32 * RBW + 4;   // pitch of the triangle product's tile (elements)
-  constexpr size_t kXt = sizeof(T) * HIDDEN * XP, kUpd = sizeof(T) * 32 * RBW * kUpdPitch<KS>;
-  __shared__ __attribute__((aligned(16))) char frag[RBW * FragLds<T, KS>::ROWBLOCK];
-  __shared__ __attribute__((aligned(16))) char frag2[RBW * FragLds<T, SL>::ROWBLOCK];
-  __shared__ __attribute__((aligned(16))) char scratch[kXt > kUpd ? kXt : kUpd];
+  constexpr int kXt = (int)sizeof(T) * HIDDEN * XP, kUpd = (int)sizeof(T) * 32 * RBW * kUpdPitch<KS>;
+  constexpr int kFrag = RBW * FragLds<T, KS>::ROWBLOCK, kFrag2 = RBW * FragLds<T, SL>::ROWBLOCK;
+  __shared__ __attribute__((aligned(16))) char smem[cmax(kFrag + kFrag2 + cmax(kXt, kUpd), kStageLds)];
+  PTX_CARRIED_STAGE();
+  char* const frag = smem;
+  char* const frag2 = smem + kFrag;
+  char* const scratch = smem + kFrag + kFrag2;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int n = p.n;
-  const TileRows tr = tile_rows(xcd_run(blockIdx.x, gridDim.x), 32 * RBW, n, p.tiles_per_i);
+  const TileRows tr = tile_rows(xcd_run(block, blocks), 32 * RBW, n, p.tiles_per_i);
   const T* packed = (const T*)p.packed;
 
   // the triangle product's rows of every channel: vectors of VE rows
@@ -442,17 +464,20 @@ __global__ __launch_bounds__(kPpWaves * 64, (sizeof(T) == 2 && KS <= 8 ? 3 : 1))
 // out = [z +] W_o (gate * o): GATE: gate = sigmoid(W_g LN(z)) formed here (16-bit arithmetic, rows of 128 channels,
 // 4 heads: wave = head), otherwise o arrives gated.  out may be z.
 template <typename T, typename TZ, int KS, bool GATE, int RBW>
-__global__ __launch_bounds__(kPpWaves * 64, (sizeof(T) == 2 && KS <= 8 ? 3 : 1)) void pp_triattn_out_kernel(ProjOutParams p) {
+__global__ __launch_bounds__(kPpWaves * 64, (sizeof(T) == 2 && KS <= 8 ? 3 : 1)) void pp_triattn_out_kernel(ProjOutParams p, SingleStage carry, unsigned carried) {
   typedef typename Vec8<T>::type V8;
   constexpr int SL = PpWidths<KS>::SL, NOB = KS / 2;
   static_assert(!GATE || (KS == 8 && sizeof(T) == 2), "gate formed here: rows of 128 channels, 16-bit arithmetic");
-  constexpr size_t kFrag = GATE ? RBW * FragLds<T, KS>::ROWBLOCK : 16, kUpd = sizeof(T) * 32 * RBW * kUpdPitch<KS>;
-  __shared__ __attribute__((aligned(16))) char scratch[kFrag > kUpd ? kFrag : kUpd];   // the normalised rows, then the update
-  __shared__ __attribute__((aligned(16))) char fo[RBW * FragLds<T, SL>::ROWBLOCK];
+  constexpr int kFrag = GATE ? RBW * FragLds<T, KS>::ROWBLOCK : 16, kUpd = (int)sizeof(T) * 32 * RBW * kUpdPitch<KS>;
+  constexpr int kScratch = cmax(kFrag, kUpd);   // the normalised rows, then the update
+  __shared__ __attribute__((aligned(16))) char smem[cmax(kScratch + RBW * FragLds<T, SL>::ROWBLOCK, kStageLds)];
+  PTX_CARRIED_STAGE();
+  char* const scratch = smem;
+  char* const fo = smem + kScratch;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int n = p.n, nl = lane & 31, g = lane >> 5;
   const int64_t n_rows = (int64_t)n * n;
-  const TileRows tr = tile_rows(xcd_run(blockIdx.x, gridDim.x), 32 * RBW, n, 0);
+  const TileRows tr = tile_rows(xcd_run(block, blocks), 32 * RBW, n, 0);
   const T* packed = (const T*)p.packed;
   V8 w[SL];
   auto load_w = [&](int ob) {
@@ -654,26 +679,30 @@ static int out_row_blocks(int64_t rows, int ks, bool attention) {
 }
 
 template <typename T, typename TZ, int KS>
-static int pp_trimul_in_ks(ProjInParams p, hipStream_t stream) {
+static int pp_trimul_in_ks(ProjInParams p, const SingleStage* carry, hipStream_t stream) {
   const int rbw = sizeof(T) == 2 ? in_row_blocks((int64_t)p.n * p.n, KS, false) : 1;
-  const dim3 grid((unsigned)((p.n + 4 * rbw - 1) / (4 * rbw)) * (unsigned)(p.pitch / 8)), block(kPpWaves * 64);
+  static const SingleStage none = {};
+  if (carry && KS <= 4) single_stage_run(carry, stream);
+  if (!carry || KS <= 4) carry = &none;
+  const unsigned carried = single_stage_groups(carry);
+  const dim3 grid(carried + (unsigned)((p.n + 4 * rbw - 1) / (4 * rbw)) * (unsigned)(p.pitch / 8)), block(kPpWaves * 64);
   if constexpr (sizeof(T) == 2) {
     if (rbw == 4) {
-      pp_trimul_in_kernel<T, TZ, KS, 4><<<grid, block, 0, stream>>>(p);
+      pp_trimul_in_kernel<T, TZ, KS, 4><<<grid, block, 0, stream>>>(p, *carry, carried);
       return 0;
     }
     if (rbw == 2) {
-      pp_trimul_in_kernel<T, TZ, KS, 2><<<grid, block, 0, stream>>>(p);
+      pp_trimul_in_kernel<T, TZ, KS, 2><<<grid, block, 0, stream>>>(p, *carry, carried);
       return 0;
     }
   }
-  pp_trimul_in_kernel<T, TZ, KS, 1><<<grid, block, 0, stream>>>(p);
+  pp_trimul_in_kernel<T, TZ, KS, 1><<<grid, block, 0, stream>>>(p, *carry, carried);
   return 0;
 }
 
 template <typename T, typename TZ>
 int pp_trimul_in(const void* z, const void* mask, const void* ln_w, const void* ln_b, const void* packed, void* a,
-                 void* b, int n, int c_z, int k_pitch, int incoming, float eps, hipStream_t stream) {
+                 void* b, int n, int c_z, int k_pitch, int incoming, float eps, const SingleStage* carry, hipStream_t stream) {
   ProjInParams p = {};
   p.x = z;
   p.si = incoming ? c_z : (int64_t)n * c_z;
@@ -690,41 +719,45 @@ int pp_trimul_in(const void* z, const void* mask, const void* ln_w, const void* 
   p.n = n;
   p.pitch = k_pitch;
   p.backward = incoming != 0;
-  if (c_z == 64) return pp_trimul_in_ks<T, TZ, 4>(p, stream);
+  if (c_z == 64) return pp_trimul_in_ks<T, TZ, 4>(p, carry, stream);
   if (c_z == 256) {
-    if constexpr (sizeof(T) == 2) return pp_trimul_in_ks<T, TZ, 16>(p, stream);
+    if constexpr (sizeof(T) == 2) return pp_trimul_in_ks<T, TZ, 16>(p, carry, stream);
     else return -1;
   }
-  return pp_trimul_in_ks<T, TZ, 8>(p, stream);
+  return pp_trimul_in_ks<T, TZ, 8>(p, carry, stream);
 }
 
 template <typename T, typename TZ, int KS, bool GATE>
-static int pp_triattn_in_ks(ProjInParams p, hipStream_t stream) {
+static int pp_triattn_in_ks(ProjInParams p, const SingleStage* carry, hipStream_t stream) {
   const int rbw = sizeof(T) == 2 ? in_row_blocks((int64_t)p.n * p.n, KS, true) : 1;
   const int rows = 32 * rbw;
   p.tiles_per_i = p.n % Cfg<T>::VE == 0 ? 0 : (p.n + rows - 1) / rows;
   const int64_t tiles = p.tiles_per_i ? (int64_t)p.n * p.tiles_per_i : ((int64_t)p.n * p.n + rows - 1) / rows;
-  const dim3 grid((unsigned)tiles), block(kPpWaves * 64);
+  static const SingleStage none = {};
+  if (carry && KS <= 4) single_stage_run(carry, stream);
+  if (!carry || KS <= 4) carry = &none;
+  const unsigned carried = single_stage_groups(carry);
+  const dim3 grid(carried + (unsigned)tiles), block(kPpWaves * 64);
   if constexpr (sizeof(T) == 2) {
     if constexpr (KS == 4) {
       if (rbw == 4) {
-        pp_triattn_in_kernel<T, TZ, KS, 4, GATE><<<grid, block, 0, stream>>>(p);
+        pp_triattn_in_kernel<T, TZ, KS, 4, GATE><<<grid, block, 0, stream>>>(p, *carry, carried);
         return 0;
       }
     }
     if (rbw == 2) {
-      pp_triattn_in_kernel<T, TZ, KS, 2, GATE><<<grid, block, 0, stream>>>(p);
+      pp_triattn_in_kernel<T, TZ, KS, 2, GATE><<<grid, block, 0, stream>>>(p, *carry, carried);
       return 0;
     }
   }
-  pp_triattn_in_kernel<T, TZ, KS, 1, GATE><<<grid, block, 0, stream>>>(p);
+  pp_triattn_in_kernel<T, TZ, KS, 1, GATE><<<grid, block, 0, stream>>>(p, *carry, carried);
   return 0;
 }
 
 template <typename T, typename TZ>
 int pp_triattn_in(const void* z, const void* ln_w, const void* ln_b, const void* packed, void* q, void* k, void* vt,
                   void* g, void* tri_bias, int n, int c_z, int heads, int key_pitch, int transposed, float eps,
-                  hipStream_t stream) {
+                  const SingleStage* carry, hipStream_t stream) {
   ProjInParams p = {};
   p.x = z;
   p.si = transposed ? c_z : (int64_t)n * c_z;
@@ -739,49 +772,57 @@ int pp_triattn_in(const void* z, const void* ln_w, const void* ln_b, const void*
   p.backward = 1;
   p.heads = heads;
   p.q_scale = 1.4426950408889634f / sqrtf(32.0f);   // log2(e) / sqrt(d), see triattn.hip
-  if (c_z == 64) return pp_triattn_in_ks<T, TZ, 4, true>(p, stream);
+  if (c_z == 64) return pp_triattn_in_ks<T, TZ, 4, true>(p, carry, stream);
   if (c_z == 256) {
-    if constexpr (sizeof(T) == 2) return pp_triattn_in_ks<T, TZ, 16, true>(p, stream);
+    if constexpr (sizeof(T) == 2) return pp_triattn_in_ks<T, TZ, 16, true>(p, carry, stream);
     else return -1;
   }
-  if constexpr (sizeof(T) == 2) return pp_triattn_in_ks<T, TZ, 8, false>(p, stream);
-  else return pp_triattn_in_ks<T, TZ, 8, true>(p, stream);
+  if constexpr (sizeof(T) == 2) return pp_triattn_in_ks<T, TZ, 8, false>(p, carry, stream);
+  else return pp_triattn_in_ks<T, TZ, 8, true>(p, carry, stream);
 }
 
 template <typename T, typename TZ, int KS>
-static int pp_trimul_out_ks(ProjOutParams p, hipStream_t stream) {
+static int pp_trimul_out_ks(ProjOutParams p, const SingleStage* carry, hipStream_t stream) {
   const int rbw = sizeof(T) == 2 ? out_row_blocks((int64_t)p.n * p.n, KS, false) : 1, rows = 32 * rbw;
   p.tiles_per_i = p.ldx == p.n && p.n % Cfg<T>::VE == 0 ? 0 : (p.n + rows - 1) / rows;
   const int64_t tiles = p.tiles_per_i ? (int64_t)p.n * p.tiles_per_i : ((int64_t)p.n * p.n + rows - 1) / rows;
-  const dim3 grid((unsigned)tiles), block(kPpWaves * 64);
+  static const SingleStage none = {};
+  if (carry && KS <= 4) single_stage_run(carry, stream);
+  if (!carry || KS <= 4) carry = &none;
+  const unsigned carried = single_stage_groups(carry);
+  const dim3 grid(carried + (unsigned)tiles), block(kPpWaves * 64);
   if constexpr (sizeof(T) == 2 && KS == 8) {
     if (rbw == 2) {
-      pp_trimul_out_kernel<T, TZ, KS, 2><<<grid, block, 0, stream>>>(p);
+      pp_trimul_out_kernel<T, TZ, KS, 2><<<grid, block, 0, stream>>>(p, *carry, carried);
       return 0;
     }
   }
-  pp_trimul_out_kernel<T, TZ, KS, 1><<<grid, block, 0, stream>>>(p);
+  pp_trimul_out_kernel<T, TZ, KS, 1><<<grid, block, 0, stream>>>(p, *carry, carried);
   return 0;
 }
 
 template <typename T, typename TZ, int KS, bool GATE>
-static int pp_triattn_out_ks(const ProjOutParams& p, hipStream_t stream) {
+static int pp_triattn_out_ks(const ProjOutParams& p, const SingleStage* carry, hipStream_t stream) {
   const int rbw = sizeof(T) == 2 ? out_row_blocks((int64_t)p.n * p.n, KS, true) : 1, rows = 32 * rbw;
-  const dim3 grid((unsigned)(((int64_t)p.n * p.n + rows - 1) / rows)), block(kPpWaves * 64);
+  static const SingleStage none = {};
+  if (carry && KS <= 4) single_stage_run(carry, stream);
+  if (!carry || KS <= 4) carry = &none;
+  const unsigned carried = single_stage_groups(carry);
+  const dim3 grid(carried + (unsigned)(((int64_t)p.n * p.n + rows - 1) / rows)), block(kPpWaves * 64);
   if constexpr (sizeof(T) == 2 && KS == 8) {
     if (rbw == 2) {
-      pp_triattn_out_kernel<T, TZ, KS, GATE, 2><<<grid, block, 0, stream>>>(p);
+      pp_triattn_out_kernel<T, TZ, KS, GATE, 2><<<grid, block, 0, stream>>>(p, *carry, carried);
       return 0;
     }
   }
-  pp_triattn_out_kernel<T, TZ, KS, GATE, 1><<<grid, block, 0, stream>>>(p);
+  pp_triattn_out_kernel<T, TZ, KS, GATE, 1><<<grid, block, 0, stream>>>(p, *carry, carried);
   return 0;
 }
 
 template <typename T, typename TZ>
 int pp_trimul_out(const void* x, int ldx, const void* z, const void* ln_in_w, const void* ln_in_b,
                   const void* ln_out_w, const void* ln_out_b, const void* packed, void* out, int n, int c_z,
-                  int hidden, int add_residual, float eps, hipStream_t stream) {
+                  int hidden, int add_residual, float eps, const SingleStage* carry, hipStream_t stream) {
   ProjOutParams p = {};
   p.z = z;
   p.si = (int64_t)n * c_z;
@@ -797,17 +838,17 @@ int pp_trimul_out(const void* x, int ldx, const void* z, const void* ln_in_w, co
   p.out = out;
   p.n = n;
   p.add_residual = add_residual;
-  if (c_z == 64) return pp_trimul_out_ks<T, TZ, 4>(p, stream);
+  if (c_z == 64) return pp_trimul_out_ks<T, TZ, 4>(p, carry, stream);
   if (c_z == 256) {
-    if constexpr (sizeof(T) == 2) return pp_trimul_out_ks<T, TZ, 16>(p, stream);
+    if constexpr (sizeof(T) == 2) return pp_trimul_out_ks<T, TZ, 16>(p, carry, stream);
     else return -1;
   }
-  return pp_trimul_out_ks<T, TZ, 8>(p, stream);
+  return pp_trimul_out_ks<T, TZ, 8>(p, carry, stream);
 }
 
 template <typename T, typename TZ>
 int pp_triattn_out(const void* o, const void* z, const void* ln_w, const void* ln_b, const void* packed, void* out,
-                   int n, int c_z, int heads, int transposed, int add_residual, float eps, hipStream_t stream) {
+                   int n, int c_z, int heads, int transposed, int add_residual, float eps, const SingleStage* carry, hipStream_t stream) {
   ProjOutParams p = {};
   p.z = z;
   p.si = transposed ? c_z : (int64_t)n * c_z;
@@ -821,12 +862,12 @@ int pp_triattn_out(const void* o, const void* z, const void* ln_w, const void* l
   p.out = out;
   p.n = n;
   p.add_residual = add_residual;
-  if (c_z == 64) return pp_triattn_out_ks<T, TZ, 4, false>(p, stream);
+  if (c_z == 64) return pp_triattn_out_ks<T, TZ, 4, false>(p, carry, stream);
   if (c_z == 256) {
-    if constexpr (sizeof(T) == 2) return pp_triattn_out_ks<T, TZ, 16, false>(p, stream);
+    if constexpr (sizeof(T) == 2) return pp_triattn_out_ks<T, TZ, 16, false>(p, carry, stream);
     else return -1;
   }
-  return pp_triattn_out_ks<T, TZ, 8, sizeof(T) == 2>(p, stream);
+  return pp_triattn_out_ks<T, TZ, 8, sizeof(T) == 2>(p, carry, stream);
 }
 
 #define PTX_INSTANTIATE_PACK(T)                                                                                        \
@@ -839,13 +880,13 @@ PTX_INSTANTIATE_PACK(bf16_t)
 #undef PTX_INSTANTIATE_PACK
 #define PTX_INSTANTIATE(T, TZ)                                                                                        \
   template int pp_trimul_in<T, TZ>(const void*, const void*, const void*, const void*, const void*, void*, void*,    \
-                                   int, int, int, int, float, hipStream_t);                                          \
+                                   int, int, int, int, float, const SingleStage*, hipStream_t);                                          \
   template int pp_triattn_in<T, TZ>(const void*, const void*, const void*, const void*, void*, void*, void*, void*,  \
-                                    void*, int, int, int, int, int, float, hipStream_t);                             \
+                                    void*, int, int, int, int, int, float, const SingleStage*, hipStream_t);                             \
   template int pp_trimul_out<T, TZ>(const void*, int, const void*, const void*, const void*, const void*,            \
-                                    const void*, const void*, void*, int, int, int, int, float, hipStream_t);        \
+                                    const void*, const void*, void*, int, int, int, int, float, const SingleStage*, hipStream_t);        \
   template int pp_triattn_out<T, TZ>(const void*, const void*, const void*, const void*, const void*, void*, int,    \
-                                     int, int, int, int, float, hipStream_t);
+                                     int, int, int, int, float, const SingleStage*, hipStream_t);
 PTX_INSTANTIATE(float, float)
 PTX_INSTANTIATE(bf16_t, bf16_t)
 PTX_INSTANTIATE(bf16_t, float)

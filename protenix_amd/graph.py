@@ -25,7 +25,7 @@ from typing import Dict, Optional, Tuple
 import torch
 import torch.nn as nn
 
-from . import native, ops
+from . import ops
 
 
 class Graphed:
@@ -63,7 +63,7 @@ class Graphed:
         # allocator, and loads every kernel, none of which may happen while capturing.
         side = torch.cuda.Stream(device=z.device)
         side.wait_stream(torch.cuda.current_stream(z.device))
-        with torch.cuda.stream(side), torch.no_grad(), native.off():
+        with torch.cuda.stream(side), torch.no_grad():
             for _ in range(self.warmup):
                 z_io.copy_(z)
                 self.module(s_in, z_io, m_in, inplace_safe=True)
@@ -73,7 +73,7 @@ class Graphed:
         graph = torch.cuda.CUDAGraph()
         ops.capture_mask_class = self._mask_class(z, pair_mask)
         try:
-            with torch.no_grad(), native.off(), torch.cuda.graph(graph):
+            with torch.no_grad(), torch.cuda.graph(graph):
                 s_out, z_out = self.module(s_in, z_io, m_in, inplace_safe=True)
         finally:
             ops.capture_mask_class = None

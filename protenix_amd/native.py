@@ -8,8 +8,6 @@ the Python path, which has the same kernels in the same order and all the error 
 """
 from __future__ import annotations
 
-import contextlib
-import threading
 import weakref
 from typing import Optional
 
@@ -20,19 +18,6 @@ from . import ops
 
 _plans: "weakref.WeakKeyDictionary" = weakref.WeakKeyDictionary()
 _host = None
-_local = threading.local()
-
-
-@contextlib.contextmanager
-def off():
-    """This thread takes the Python path inside."""
-    keep = getattr(_local, "off", False)
-    _local.off = True
-    try:
-        yield
-    finally:
-        _local.off = keep
-
 # plain attributes of the modules that the plans depend on
 _ATTRS = ["inf", "no_heads", "c_hidden", "n", "n_heads", "num_heads", "c_in", "c_z", "c_s", "eps", "starting", "_outgoing",
           "precision"]
@@ -56,7 +41,7 @@ def host():
 
 
 def _usable(z: torch.Tensor) -> bool:
-    return (ops.use_native() and not getattr(_local, "off", False) and z.is_cuda and not torch.is_grad_enabled() and z.dim() >= 3 and z.shape[-2] == z.shape[-3]
+    return (ops.use_native() and z.is_cuda and not torch.is_grad_enabled() and z.dim() >= 3 and z.shape[-2] == z.shape[-3]
             and z.numel() > 0 and z.dtype in (torch.float32, torch.bfloat16)
             and not _nn_module._global_forward_hooks and not _nn_module._global_forward_pre_hooks)
 
@@ -91,6 +76,13 @@ def _att_spec(a, cd, device, transposed: bool) -> Optional[dict]:
             "transposed": int(transposed)}
 
 
+def _fragments(w: torch.Tensor) -> torch.Tensor:
+    """[n_out][k] in the fragment order of ptx_single_linear_stage."""
+    n, k = w.shape
+    v = 16 // w.element_size()
+    return w.view(n // 16, 16, k // 32, 8 // v, 4, v).permute(0, 2, 3, 4, 1, 5).contiguous()
+
+
 def _block_spec(blk, z: torch.Tensor, cd: torch.dtype, sd: Optional[torch.dtype]) -> Optional[dict]:
     from .primitives import _cv
     dev, c, tr, end = z.device, z.shape[-1], blk.pair_transition, blk.tri_att_end
@@ -117,10 +109,11 @@ def _block_spec(blk, z: torch.Tensor, cd: torch.dtype, sd: Optional[torch.dtype]
         H, d = att.num_heads, att.c_hidden
         lins = (att.linear_q, att.linear_k, att.linear_v, att.linear_g, att.linear_o, st.linear_no_bias_a, st.linear_no_bias_b,
                 st.linear_no_bias)
-        if not (sd in (torch.float32, torch.bfloat16) and c in (128, 256) and 1 <= apb.n_heads <= 32 and apb.n_heads == H
+        # (the single track's stages ride on the pair kernels: same storage type, LayerNorm rows of whole vectors)
+        if not (sd == z.dtype and cs % 16 == 0 and cs * z.element_size() <= 2048 and c in (128, 256) and 1 <= apb.n_heads <= 32 and apb.n_heads == H
                 and all(l is not None and l.precision is None for l in lins)
                 and att.c_q == att.c_k == att.c_v == cs == st.c_in and cs % 16 == 0 and cs not in (64, 128, 256)
-                and d % 8 == 0 and d <= 32 and (3 * H * d) % 32 == 0 and (st.n * cs) % 16 == 0):
+                and d % 8 == 0 and d <= 32 and (H * d) % 32 == 0 and cs % 32 == 0):
             return None
         pw = apb.pair_bias_weights(z)
         w_in, b_q = att._fused_in(sd, dev)
@@ -128,9 +121,10 @@ def _block_spec(blk, z: torch.Tensor, cd: torch.dtype, sd: Optional[torch.dtype]
         s_wa, s_wb, s_wo = st._cache_ab.get(st_ps, sd, dev, lambda: tuple(_cv(p, sd, dev) for p in st_ps))
         w_o = att._cache_out.get((att.linear_o.weight,), sd, dev, lambda: _cv(att.linear_o.weight, sd, dev))
         spec.update(pb_ln_w=pw[0], pb_ln_b=pw[1], pb_w=pw[2], a_ln_w=_cv(apb.layernorm_a.weight, sd, dev),
-                    a_ln_b=_cv(apb.layernorm_a.bias, sd, dev), a_eps=float(apb.layernorm_a.eps), w_in=w_in, b_q=b_q, w_o=w_o,
+                    a_ln_b=_cv(apb.layernorm_a.bias, sd, dev), a_eps=float(apb.layernorm_a.eps), w_in=_fragments(w_in), b_q=b_q, w_o=_fragments(w_o),
                     s_ln_w=_cv(st.layernorm1.weight, sd, dev), s_ln_b=_cv(st.layernorm1.bias, sd, dev),
-                    s_eps=float(st.layernorm1.eps), s_wa=s_wa, s_wb=s_wb, s_wo=s_wo, heads=H, d=d)
+                    s_eps=float(st.layernorm1.eps), s_wa=_fragments(s_wa), s_wb=_fragments(s_wb), s_wo=_fragments(s_wo),
+                    heads=H, d=d, hidden=st.n * cs)
     return spec
 
 
@@ -148,13 +142,10 @@ def _block_plan(blk, z, cd, sd):
     return plan
 
 
-def run_blocks(owner, blocks, s: Optional[torch.Tensor], z: torch.Tensor, pair_mask: Optional[torch.Tensor], side):
+def run_blocks(owner, blocks, s: Optional[torch.Tensor], z: torch.Tensor, pair_mask: Optional[torch.Tensor]):
     """The blocks on (s, z), z contiguous and updated in place: the new s (None without a single track), or NotImplemented
-    where the Python path is to be taken.  `owner`: the module the list of plans is kept with; `side`: None or a callable
-    that returns the second stream for the single track."""
-    # A recording is made by the Python path: its time does not count, and a recording in which the two
-    # streams wait for each other in both directions (the ring of bias buffers) is none this code relies on.
-    if not _usable(z) or not z.is_contiguous() or torch.cuda.is_current_stream_capturing():
+    where the Python path is to be taken.  `owner`: the module the list of plans is kept with."""
+    if not _usable(z) or not z.is_contiguous():
         return NotImplemented
     ac = ops.autocast_compute_dtype(z)
     cd = ops.compute_dtype(z)
@@ -191,11 +182,7 @@ def run_blocks(owner, blocks, s: Optional[torch.Tensor], z: torch.Tensor, pair_m
             plans.append(plan)
         _plans[owner][("stack", key)] = ([weakref.ref(b) for b in blocks], plans)
     masks = _masks(z, pair_mask, cd)
-    stream = None
-    if side is not None and single:
-        st = side()
-        stream = (st.stream_id, st.device_index, st.device_type)
-    return host().run_blocks(plans, s.contiguous() if single else s, z, masks, stream)
+    return host().run_blocks(plans, s.contiguous() if single else s, z, masks)
 
 
 def run_update(module, z: torch.Tensor, cd: torch.dtype, mask: Optional[torch.Tensor], out: torch.Tensor, add: bool,

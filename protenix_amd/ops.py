@@ -383,7 +383,7 @@ def triangle_multiplication(z: torch.Tensor, mask: Optional[torch.Tensor], w: di
     with torch.cuda.device(z.device):
         if packed is not None:
             _call("trimul_project", lib.ptx_trimul_project_packed, _ptr(z), _ptr(mask), _ptr(w["ln_in_w"]),
-                  _ptr(w["ln_in_b"]), _ptr(packed), _ptr(a), _ptr(b), n, c_z, c_h, pitch, int(incoming), eps, dt, st)
+                  _ptr(w["ln_in_b"]), _ptr(packed), _ptr(a), _ptr(b), n, c_z, c_h, pitch, int(incoming), eps, dt, None, st)
         else:
             _call("trimul_project", lib.ptx_trimul_project, _ptr(z), _ptr(mask), _ptr(w["ln_in_w"]), _ptr(w["ln_in_b"]), _ptr(w["w_ap"]),
                 _ptr(w["w_ag"]), _ptr(w["w_bp"]), _ptr(w["w_bg"]), _ptr(a), _ptr(b), n, c_z, c_h, pitch,
@@ -396,7 +396,7 @@ def triangle_multiplication(z: torch.Tensor, mask: Optional[torch.Tensor], w: di
         if packed is not None:
             _call("trimul_output", lib.ptx_trimul_output_packed, _ptr(x), ldx, _ptr(z), _ptr(w["ln_in_w"]),
                   _ptr(w["ln_in_b"]), _ptr(w["ln_out_w"]), _ptr(w["ln_out_b"]), _ptr(packed), _ptr(out), n, c_z, c_h,
-                  int(add_residual), eps, dt, st)
+                  int(add_residual), eps, dt, None, st)
             return out
         _call("trimul_output", lib.ptx_trimul_output, _ptr(x), _ptr(z), _ptr(w["ln_in_w"]), _ptr(w["ln_in_b"]), _ptr(w["ln_out_w"]),
             _ptr(w["ln_out_b"]), _ptr(w["w_z"]), _ptr(w["w_g"]), _ptr(out), n, c_z, c_h,
@@ -502,7 +502,7 @@ def triangle_attention(z: torch.Tensor, mask: Optional[torch.Tensor], w: dict, h
         if packed is not None:
             _call("triattn_project", lib.ptx_triattn_project_packed, _ptr(z), _ptr(w["ln_w"]), _ptr(w["ln_b"]),
                   _ptr(packed), _ptr(q), _ptr(k), _ptr(vt), None if late_gate else _ptr(g), _ptr(tb),
-                  n, c, heads, pitch, int(transposed), eps, dt, st)
+                  n, c, heads, pitch, int(transposed), eps, dt, None, st)
         else:
             _call("triattn_project", lib.ptx_triattn_project, _ptr(z), _ptr(w["ln_w"]),
                   _ptr(w["ln_b"]), _ptr(w["w_q"]), _ptr(w["w_k"]), _ptr(w["w_v"]), _ptr(w["w_g"]),
@@ -541,7 +541,7 @@ def triangle_attention(z: torch.Tensor, mask: Optional[torch.Tensor], w: dict, h
             return out, bias
         if packed is not None:
             _call("triattn_output", lib.ptx_triattn_output_packed, _ptr(g), _ptr(z), _ptr(w["ln_w"]), _ptr(w["ln_b"]),
-                  _ptr(packed), _ptr(out), n, c, heads, int(transposed), int(add_residual), eps, dt, st)
+                  _ptr(packed), _ptr(out), n, c, heads, int(transposed), int(add_residual), eps, dt, None, st)
         elif late_gate:
             _call("triattn_output", lib.ptx_triattn_gate_output, _ptr(g), _ptr(z), _ptr(w["ln_w"]),
                   _ptr(w["ln_b"]), _ptr(w["w_g"]), _ptr(w["w_o"]), _ptr(out), n, c, heads,

@@ -114,7 +114,7 @@ class PairformerBlock(nn.Module):
             return s, pad.result(z if inplace_safe else None)
         if not inplace_safe or not z.is_contiguous():
             z = z.clone(memory_format=torch.contiguous_format)
-        s_new = native.run_blocks(self, (self,), s, z, pair_mask, None)
+        s_new = native.run_blocks(self, (self,), s, z, pair_mask)
         if s_new is not NotImplemented:
             return s_new, z
         return self._forward_unpadded(s, z, pair_mask, None)
@@ -260,7 +260,7 @@ class PairformerStack(nn.Module):
                 f"{triangle_multiplicative}")
         assert triangle_attention in ("torch", "deepspeed", "triattention", "cuequivariance")
         if pad is None and len(self.blocks) > 0:
-            s_new = native.run_blocks(self, tuple(self.blocks), s, z, pair_mask, lambda: self._side_stream(z.device))
+            s_new = native.run_blocks(self, tuple(self.blocks), s, z, pair_mask)
             if s_new is not NotImplemented:
                 return s_new, z
         ac = ops.autocast_compute_dtype(z)
