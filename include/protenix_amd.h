@@ -34,7 +34,7 @@
 extern "C" {
 #endif
 
-#define PTX_ABI_VERSION 4
+#define PTX_ABI_VERSION 5
 #define PTX_API __attribute__((visibility("default")))
 
 /*
@@ -339,6 +339,15 @@ PTX_API int ptx_triattn_core_bwd(const void* q, const void* k, const void* v, co
                          const void* bias2, const void* o, const float* lse, const void* dout,
                          void* dq, void* dk, void* dv, void* dbias2, float* delta, int batch,
                          int n_rows, int s, int heads, int d, int dtype, void* stream);
+/* The same with scratch for dBias2: partials (or NULL: as above) is an uninitialised, 16-byte aligned fp32
+ * buffer of ptx_triattn_core_bwd_partial_elems(n_rows, s, heads) elements (0: none of use), at most 128 MB.
+ * With it the rows dBias2 sums over are cut into slices where few tokens would leave the machine idle;
+ * their sums are added in a fixed order. */
+PTX_API int64_t ptx_triattn_core_bwd_partial_elems(int n_rows, int s, int heads);
+PTX_API int ptx_triattn_core_bwd_sliced(const void* q, const void* k, const void* v, const void* bias1,
+                         const void* bias2, const void* o, const float* lse, const void* dout,
+                         void* dq, void* dk, void* dv, void* dbias2, float* delta, float* partials,
+                         int batch, int n_rows, int s, int heads, int d, int dtype, void* stream);
 
 /*
  * Triangle attention, stage 3 (layers.py:392-396 + the caller's residual add,

@@ -14,7 +14,7 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libprotenix_amd.so")
 
 PTX_F32, PTX_BF16, PTX_MIXED, PTX_F16 = 0, 1, 2, 3
-ABI_VERSION = 4
+ABI_VERSION = 5
 
 _p = ctypes.c_void_p
 _i = ctypes.c_int
@@ -55,6 +55,8 @@ SIGNATURES = {
     "ptx_triattn_core_workspace_elems": (_l, [_i, _i, _i]),
     "ptx_triattn_core_fwd": (_i, [_p] * 8 + [_i, _i, _i, _i, _i, _i, _p]),
     "ptx_triattn_core_bwd": (_i, [_p] * 13 + [_i, _i, _i, _i, _i, _i, _p]),
+    "ptx_triattn_core_bwd_partial_elems": (_l, [_i, _i, _i]),
+    "ptx_triattn_core_bwd_sliced": (_i, [_p] * 14 + [_i, _i, _i, _i, _i, _i, _p]),
     "ptx_triattn_gate_output": (_i, [_p] * 7 + [_i, _i, _i, _i, _i, _f, _i, _p]),
     "ptx_transition_packed_elems": (_l, [_i, _i]),
     "ptx_transition_pack": (_i, [_p, _p, _p, _p, _i, _i, _i, _p]),

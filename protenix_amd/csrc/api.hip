@@ -585,6 +585,20 @@ PTX_API int ptx_triattn_core_bwd(const void* q, const void* k, const void* v, co
                                  const void* dout, void* dq, void* dk, void* dv, void* dbias2,
                                  float* delta, int batch, int n_rows, int s, int heads, int d,
                                  int dtype, void* stream) {
+  return ptx_triattn_core_bwd_sliced(q, k, v, bias1, bias2, o, lse, dout, dq, dk, dv, dbias2, delta, nullptr, batch,
+                                     n_rows, s, heads, d, dtype, stream);
+}
+
+PTX_API int64_t ptx_triattn_core_bwd_partial_elems(int n_rows, int s, int heads) {
+  if (n_rows <= 0 || s <= 0 || heads <= 0 || s > 8192 || heads > 64) return 0;
+  const int slices = ptx::triattn_bwd_slices(n_rows, s, heads);
+  return slices > 1 ? (int64_t)slices * heads * s * s : 0;
+}
+
+PTX_API int ptx_triattn_core_bwd_sliced(const void* q, const void* k, const void* v, const void* bias1,
+                                        const void* bias2, const void* o, const float* lse, const void* dout,
+                                        void* dq, void* dk, void* dv, void* dbias2, float* delta, float* partials,
+                                        int batch, int n_rows, int s, int heads, int d, int dtype, void* stream) {
   PTX_REQUIRE(dtype_ok(dtype), PTX_ERR_BAD_ARG, "triattn_core_bwd: unknown dtype %d", dtype);
   PTX_REQUIRE(batch >= 0 && n_rows >= 0 && s >= 0 && heads >= 0, PTX_ERR_BAD_ARG,
               "triattn_core_bwd: batch=%d n_rows=%d s=%d heads=%d", batch, n_rows, s, heads);
@@ -595,7 +609,7 @@ PTX_API int ptx_triattn_core_bwd(const void* q, const void* k, const void* v, co
   PTX_REQUIRE(q && k && v && bias2 && o && lse && dout && dq && dk && dv && delta, PTX_ERR_BAD_ARG,
               "triattn_core_bwd: null pointer");
   PTX_REQUIRE(aligned16(q) && aligned16(k) && aligned16(v) && aligned16(o) && aligned16(dout) &&
-                  aligned16(dq) && aligned16(dk) && aligned16(dv),
+                  aligned16(dq) && aligned16(dk) && aligned16(dv) && (!partials || aligned16(partials)),
               PTX_ERR_BAD_ARG, "triattn_core_bwd: pointers must be 16-byte aligned");
   const int64_t n_q = (int64_t)n_rows * s * heads * 32, n_l = (int64_t)n_rows * s * heads;
   const int64_t n_b2 = (int64_t)heads * s * s, n_b1 = (int64_t)n_rows * s;
@@ -608,7 +622,7 @@ PTX_API int ptx_triattn_core_bwd(const void* q, const void* k, const void* v, co
                             (const char*)q + oq, (const char*)k + oq, (const char*)v + oq, b1,
                             (const char*)bias2 + b * n_b2 * es, (const char*)o + oq, lse + b * n_l,
                             (const char*)dout + oq, (char*)dq + oq, (char*)dk + oq, (char*)dv + oq,
-                            db2, delta, n_rows, s, heads, (hipStream_t)stream));
+                            db2, delta, partials, n_rows, s, heads, (hipStream_t)stream));
   }
   return after_launch("triattn_core_bwd");
 }

@@ -18,6 +18,7 @@
 // its MFMA fragments from there - also those a product needs with the walking index in the K
 // slots (K^T for dQ, Q^T and dO^T for dK / dV), which 16-bit tiles give through the
 // transposing LDS load and fp32 tiles through a transposed copy.
+#include <algorithm>
 #include <type_traits>
 #include "common.h"
 #include "kernels.h"
@@ -27,6 +28,7 @@ namespace ptx {
 namespace {
 
 constexpr float kBwdLog2e = 1.4426950408889634f;
+constexpr int64_t kDb2Workgroups = 1024;   // what the machine holds of dBias2's at once (triattn_bwd_slices)
 constexpr int kTP = 40;   // pitch of the LDS tiles (elements): 16-byte aligned rows, spread over banks
 
 struct BwdParams {
@@ -35,7 +37,16 @@ struct BwdParams {
   float* delta;
   void *dq, *dk, *dv, *db2;
   int n_rows, s, heads;
+  float* parts;     // dBias2's partial sums [slice][H][S][S], or null: one slice, written as it is
+  int slices;
 };
+
+// Work item of this workgroup in a grid of `items` rounded up to a multiple of 8: one contiguous span per XCD
+// (workgroups are dealt round-robin to the 8 XCDs), so that the heads and blocks of a row, which read the same
+// cache lines, share an L2.
+__device__ __forceinline__ uint32_t xcd_item(uint32_t items) {
+  return (blockIdx.x & 7) * ((items + 7) / 8) + (blockIdx.x >> 3);
+}
 
 __device__ __forceinline__ int perm_row(int m) {   // MFMA row m of a 32-block <-> index in the block
   return 16 * (m >> 4) + 8 * ((m >> 2) & 1) + 4 * ((m >> 3) & 1) + (m & 3);
@@ -143,8 +154,10 @@ __global__ __launch_bounds__(256, (BwdCfg<T, VEC>::kMinWaves)) void attn_bwd_dq_
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, ln = lane & 31, g = lane >> 5;
   const int s = p.s, H = p.heads;
   constexpr bool vec = VEC;   // rows of s keys are 8-aligned
-  const int h = blockIdx.y, i = blockIdx.z;
-  const int q0 = (blockIdx.x * 4 + wave) * 32;
+  const uint32_t n_wg = ((uint32_t)s + 127) / 128, items = n_wg * (uint32_t)H * (uint32_t)p.n_rows, item = xcd_item(items);
+  if (item >= items) return;
+  const int wg = item % n_wg, h = item / n_wg % H, i = item / n_wg / H;
+  const int q0 = (wg * 4 + wave) * 32;
   const int qi = min(q0 + ln, s - 1);
   const bool q_ok = q0 + ln < s;
   // (without a Bias1 the loads go to a row of Bias2 and count for nothing: a load under a
@@ -201,7 +214,7 @@ __global__ __launch_bounds__(256, (BwdCfg<T, VEC>::kMinWaves)) void attn_bwd_dq_
   const T* b2rows[2];
 #pragma unroll
   for (int j = 0; j < 2; ++j)
-    b2rows[j] = (const T*)p.b2 + ((int64_t)h * s + min((int)blockIdx.x * 128 + 64 * j + (tid >> 2), s - 1)) * s;
+    b2rows[j] = (const T*)p.b2 + ((int64_t)h * s + min(wg * 128 + 64 * j + (tid >> 2), s - 1)) * s;
   // (the compiler barriers keep the loads where they are written, a step ahead of their use:
   // left alone, the compiler moves them down to the use and waits there)
   auto fetch = [&](int key0) {
@@ -340,8 +353,10 @@ __global__ __launch_bounds__(256, (BwdCfg<T, VEC>::kMinWaves)) void attn_bwd_kv_
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, ln = lane & 31, g = lane >> 5;
   const int s = p.s, H = p.heads;
   constexpr bool vec = VEC;
-  const int h = blockIdx.y, i = blockIdx.z;
-  const int key0 = (blockIdx.x * 4 + wave) * 32;
+  const uint32_t n_wg = ((uint32_t)s + 127) / 128, items = n_wg * (uint32_t)H * (uint32_t)p.n_rows, item = xcd_item(items);
+  if (item >= items) return;
+  const int wg = item % n_wg, h = item / n_wg % H, i = item / n_wg / H;
+  const int key0 = (wg * 4 + wave) * 32;
   const int kc = min(key0 + ln, s - 1);
   const bool k_ok = key0 + ln < s;
   V8 kf[2], vf[2];
@@ -364,7 +379,7 @@ __global__ __launch_bounds__(256, (BwdCfg<T, VEC>::kMinWaves)) void attn_bwd_kv_
   // touches as many lines per load as it has lanes).
   V8 b2a, b2b;
   const int b2q = TURN ? tid >> 3 : ln;
-  const int b2k = TURN ? (int)blockIdx.x * 128 + 8 * (tid & 7) : key0 + 16 * g;
+  const int b2k = TURN ? wg * 128 + 8 * (tid & 7) : key0 + 16 * g;
   auto fetch = [&](int q0) {
     piece.fetch(p, p.q, p.dout, i, q0, h, tid);
     stat = stat_src[((int64_t)i * s + min(q0 + ln, s - 1)) * H + h];
@@ -483,6 +498,12 @@ __global__ __launch_bounds__(256, (BwdCfg<T, VEC>::kMinWaves)) void attn_bwd_kv_
 // a row's Bias1 is added to it for the initial value of the S^T accumulator, -Delta is that of
 // dP^T.  Nothing in the walk looks at s: queries and keys beyond it repeat the last one, and
 // what accumulates for them is not stored.
+// The walk is cut into slices of rows: 384 tokens and 4 heads are 144 workgroups for 256 compute units that
+// hold four each, every one a serial chain over 384 rows.  Slices write fp32 partial sums that
+// attn_bwd_db2_sum_kernel adds in order (no atomics).  A slice's workgroups all go to one XCD
+// (workgroups are dealt to the XCDs in turn, and the slice is the fastest index), whose L2 then fetches the slice's rows
+// once; with a slice's workgroups on all eight the rows come through the memory-side cache eight times.  us at 384 rows,
+// 384 tokens, 4 heads, bf16: one slice 312; seven slices, spread 165 with the sum; eight, one per XCD, 107 + 4.
 template <typename T, bool VEC>
 __global__ __launch_bounds__(256, (BwdCfg<T, VEC>::kMinWaves)) void attn_bwd_db2_kernel(BwdParams p) {
   typedef typename Vec8<T>::type V8;
@@ -491,8 +512,9 @@ __global__ __launch_bounds__(256, (BwdCfg<T, VEC>::kMinWaves)) void attn_bwd_db2
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, ln = lane & 31, g = lane >> 5;
   const int s = p.s, H = p.heads;
   constexpr bool vec = VEC;
-  const int h = blockIdx.y;
-  const int qs0 = blockIdx.x * 64, ks0 = blockIdx.z * 64;
+  const int slice = blockIdx.x % p.slices, pair = blockIdx.x / p.slices, tiles_s = (s + 63) / 64;
+  const int row_begin = (int)((int64_t)p.n_rows * slice / p.slices), row_end = (int)((int64_t)p.n_rows * (slice + 1) / p.slices);
+  const int qs0 = pair % tiles_s * 64, ks0 = pair / tiles_s % tiles_s * 64, h = pair / tiles_s / tiles_s;
   const int wq = wave >> 1, wk = wave & 1;
   const int q0 = qs0 + 32 * wq, key0 = ks0 + 32 * wk;
   const int qi = min(q0 + ln, s - 1);
@@ -551,15 +573,15 @@ __global__ __launch_bounds__(256, (BwdCfg<T, VEC>::kMinWaves)) void attn_bwd_db2
   };
   // Row i is computed out of buffer i % NB while row i + 1, fetched a step earlier, is parked
   // (two buffers: into the other one, which every wave left at the last barrier).
-  const int last = p.n_rows - 1;
-  fetch(0);
+  const int last = row_end - 1;
+  fetch(row_begin);
 #pragma unroll
-  for (int w = 0; w < 4; ++w) store8<T>(&tiles[0][w][crow * kTP + cc], piece[w]);
+  for (int w = 0; w < 4; ++w) store8<T>(&tiles[row_begin % NB][w][crow * kTP + cc], piece[w]);
   float neg_mq = -mq_n, neg_dq = -dq_n;
   V8 b1c[2] = {b1n[0], b1n[1]};
   T b1m = b1m_n;
   __syncthreads();
-  for (int i = 0; i < p.n_rows; ++i) {
+  for (int i = row_begin; i < row_end; ++i) {
     const int buf = i % NB;
     fetch(min(i + 1, last));
     asm volatile("" ::: "memory");   // the loads are issued here, a step ahead of their use
@@ -603,7 +625,25 @@ __global__ __launch_bounds__(256, (BwdCfg<T, VEC>::kMinWaves)) void attn_bwd_db2
     b1m = b1m_n;
     __syncthreads();
   }
-  if (q_ok) {
+  if (q_ok && p.parts) {
+    float* dst = p.parts + (((int64_t)slice * H + h) * s + qi) * s;
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+      const int kb = key0 + 16 * ks + 8 * g;
+      if (vec) {
+        if (kb < s) {
+#pragma unroll
+          for (int c = 0; c < 2; ++c)
+            *reinterpret_cast<f32x4*>(dst + kb + 4 * c) =
+                f32x4{acc[8 * ks + 4 * c], acc[8 * ks + 4 * c + 1], acc[8 * ks + 4 * c + 2], acc[8 * ks + 4 * c + 3]};
+        }
+      } else {
+#pragma unroll
+        for (int t = 0; t < 8; ++t)
+          if (kb + t < s) dst[kb + t] = acc[8 * ks + t];
+      }
+    }
+  } else if (q_ok) {
     T* dst = (T*)p.db2 + ((int64_t)h * s + qi) * s;
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks) {
@@ -622,14 +662,52 @@ __global__ __launch_bounds__(256, (BwdCfg<T, VEC>::kMinWaves)) void attn_bwd_db2
   }
 }
 
+// dBias2 = the slices' partial sums added in order, V values per thread (4 where the values of a slice are
+// whole vectors).  Reads what the kernel before it left in the caches: 19 MB at 384 tokens, 4 us.
+template <typename T, int V>
+__global__ __launch_bounds__(256) void attn_bwd_db2_sum_kernel(const float* __restrict__ parts, T* __restrict__ db2, int slices, int64_t n) {
+  const int64_t e = ((int64_t)blockIdx.x * 256 + threadIdx.x) * V;
+  if (e >= n) return;
+  if constexpr (V == 4) {
+    f32x4 sum = *reinterpret_cast<const f32x4*>(parts + e);
+    for (int sl = 1; sl < slices; ++sl) sum += *reinterpret_cast<const f32x4*>(parts + sl * n + e);
+    *reinterpret_cast<typename Vec4<T>::type*>(db2 + e) = from_f32<T>(sum);
+  } else {
+    float sum = parts[e];
+    for (int sl = 1; sl < slices; ++sl) sum += parts[sl * n + e];
+    db2[e] = from_f32<T>(sum);
+  }
+}
+
+// Slices of rows of dBias2's walk: eight, one per XCD, or as many more as give every compute unit its four
+// workgroups at once, of at least 8 rows, as long as the partial sums (4 S^2 H bytes per slice, written and
+// read once) stay within 128 MB.
+int triattn_bwd_slices(int n_rows, int s, int heads) {
+  const int64_t tiles = (s + 63) / 64, pairs = tiles * tiles * heads;
+  if (pairs <= 0 || n_rows <= 0) return 1;
+  int64_t want = std::min<int64_t>(std::max<int64_t>(8, kDb2Workgroups / pairs), n_rows / 8);
+  if (want > 8) want &= ~(int64_t)7;
+  return want > 1 && want * heads * s * s * 4 <= (int64_t)128 << 20 ? (int)want : 1;
+}
+
+template <typename T>
+static void db2_sum(const BwdParams& p, int slices, hipStream_t stream) {
+  const int64_t n = (int64_t)p.heads * p.s * p.s;
+  const bool vec = n % 4 == 0 && (uintptr_t)p.db2 % (4 * sizeof(T)) == 0 && (uintptr_t)p.parts % 16 == 0;
+  const unsigned blocks = (unsigned)((n / (vec ? 4 : 1) + 255) / 256);
+  if (vec) attn_bwd_db2_sum_kernel<T, 4><<<dim3(blocks), dim3(256), 0, stream>>>(p.parts, (T*)p.db2, slices, n);
+  else attn_bwd_db2_sum_kernel<T, 1><<<dim3(blocks), dim3(256), 0, stream>>>(p.parts, (T*)p.db2, slices, n);
+}
+
 template <typename T>
 int triattn_bwd(const void* q, const void* k, const void* v, const void* b1, const void* b2,
                 const void* o, const float* lse, const void* dout, void* dq, void* dk, void* dv,
-                void* db2, float* delta, int n_rows, int s, int heads, hipStream_t stream) {
+                void* db2, float* delta, float* parts, int n_rows, int s, int heads, hipStream_t stream) {
   if (n_rows == 0 || s == 0 || heads == 0) return 0;
-  BwdParams p = {q, k, v, o, dout, b1, b2, lse, delta, dq, dk, dv, db2, n_rows, s, heads};
-  const unsigned blocks = (unsigned)((s + 31) / 32);
-  const dim3 walk((blocks + 3) / 4, heads, n_rows), pairs((blocks + 1) / 2, heads, (blocks + 1) / 2);
+  const int slices = parts && db2 ? triattn_bwd_slices(n_rows, s, heads) : 1;
+  BwdParams p = {q, k, v, o, dout, b1, b2, lse, delta, dq, dk, dv, db2, n_rows, s, heads, slices > 1 ? parts : nullptr, slices};
+  const unsigned tiles = (unsigned)((s + 63) / 64);
+  const dim3 walk(((unsigned)((s + 127) / 128) * heads * n_rows + 7) / 8 * 8), pairs(tiles * tiles * heads * slices);
   if ((s & 7) == 0) {
     attn_bwd_dq_kernel<T, true><<<walk, dim3(256), 0, stream>>>(p);   // (writes Delta: first)
     attn_bwd_kv_kernel<T, true><<<walk, dim3(256), 0, stream>>>(p);
@@ -639,14 +717,15 @@ int triattn_bwd(const void* q, const void* k, const void* v, const void* b1, con
     attn_bwd_kv_kernel<T, false><<<walk, dim3(256), 0, stream>>>(p);
     if (db2) attn_bwd_db2_kernel<T, false><<<pairs, dim3(256), 0, stream>>>(p);
   }
+  if (slices > 1) db2_sum<T>(p, slices, stream);
   return 0;
 }
 
 template int triattn_bwd<float>(const void*, const void*, const void*, const void*, const void*,
                                 const void*, const float*, const void*, void*, void*, void*, void*,
-                                float*, int, int, int, hipStream_t);
+                                float*, float*, int, int, int, hipStream_t);
 template int triattn_bwd<bf16_t>(const void*, const void*, const void*, const void*, const void*,
                                  const void*, const float*, const void*, void*, void*, void*, void*,
-                                 float*, int, int, int, hipStream_t);
+                                 float*, float*, int, int, int, hipStream_t);
 
 }  // namespace ptx

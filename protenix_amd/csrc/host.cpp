@@ -523,9 +523,11 @@ struct TriAttentionFn : torch::autograd::Function<TriAttentionFn> {
     const bool want_b2 = ctx->needs_input_grad(ctx->saved_data["b2i"].toInt());
     Tensor dq = at::empty_like(q), dk = at::empty_like(k), dv = at::empty_like(v), db2 = want_b2 ? at::empty_like(b2) : Tensor();
     Tensor delta = at::empty({N * S * H}, q.options().dtype(at::kFloat));
-    check(ptx_triattn_core_bwd(ptr(q), ptr(k), ptr(v), ptr(b1), ptr(b2), ptr(o), (const float*)ptr(m), ptr(dout), ptr(dq), ptr(dk), ptr(dv),
-                               ptr(db2), (float*)ptr(delta), (int)B, (int)N, (int)S, (int)H, (int)D, code_of(q.scalar_type()),
-                               current_stream(q)), "triattn_core_bwd");
+    const int64_t n_parts = want_b2 ? ptx_triattn_core_bwd_partial_elems((int)N, (int)S, (int)H) : 0;
+    Tensor parts = n_parts ? at::empty({n_parts}, q.options().dtype(at::kFloat)) : Tensor();
+    check(ptx_triattn_core_bwd_sliced(ptr(q), ptr(k), ptr(v), ptr(b1), ptr(b2), ptr(o), (const float*)ptr(m), ptr(dout), ptr(dq), ptr(dk), ptr(dv),
+                                      ptr(db2), (float*)ptr(delta), (float*)ptr(parts), (int)B, (int)N, (int)S, (int)H, (int)D,
+                                      code_of(q.scalar_type()), current_stream(q)), "triattn_core_bwd");
     if (want_b2) {
       const auto shape = ctx->saved_data["b2s"].toIntVector();
       if (db2.sizes() != c10::IntArrayRef(shape)) db2 = at::sum_to(db2, shape);

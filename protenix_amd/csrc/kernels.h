@@ -177,11 +177,13 @@ int triattn_pack(const T* q, const T* k, const T* v, const T* bias2, T* qs, T* k
                  int n_rows, int n, int heads, int key_pitch, hipStream_t stream);
 // Backward of the standard-layout attention operator: dQ, dK, dV [n_rows][s][heads][32] and,
 // when db2 is given, dBias2 [heads][s][s], from Q (scaled), K, V, O, dO, the biases and the
-// forward's log2-sum-exp2; delta [n_rows][s][heads] is fp32 scratch.
+// forward's log2-sum-exp2; delta [n_rows][s][heads] is fp32 scratch; parts: fp32 scratch of
+// triattn_bwd_slices() * heads * s * s elements for the partial sums of dBias2, or null (one slice).
+int triattn_bwd_slices(int n_rows, int s, int heads);
 template <typename T>
 int triattn_bwd(const void* q, const void* k, const void* v, const void* b1, const void* b2,
                 const void* o, const float* lse, const void* dout, void* dq, void* dk, void* dv,
-                void* db2, float* delta, int n_rows, int s, int heads, hipStream_t stream);
+                void* db2, float* delta, float* parts, int n_rows, int s, int heads, hipStream_t stream);
 
 // Streams `bytes` (a multiple of 16) from src to dst; src null: write-only, dst null: read-only.
 int hbm_stream(const void* src, void* dst, int64_t bytes, int nontemporal, hipStream_t stream);

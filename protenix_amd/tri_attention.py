@@ -84,10 +84,12 @@ class TriAttentionFunction(torch.autograd.Function):
         DB2 = torch.empty_like(b2) if want_b2 else None
         delta = ops._workspace((N * S * H,), torch.float32, q.device)
         lib = _lib.load()
+        n_parts = lib.ptx_triattn_core_bwd_partial_elems(N, S, H) if want_b2 else 0
+        parts = ops._workspace((n_parts,), torch.float32, q.device) if n_parts else None
         with torch.cuda.device(q.device):
-            ops._call("triattn_core_bwd", lib.ptx_triattn_core_bwd, ops._ptr(q), ops._ptr(k),
+            ops._call("triattn_core_bwd", lib.ptx_triattn_core_bwd_sliced, ops._ptr(q), ops._ptr(k),
                       ops._ptr(v), ops._ptr(b1), ops._ptr(b2), ops._ptr(O), ops._ptr(M), ops._ptr(DO),
-                      ops._ptr(DQ), ops._ptr(DK), ops._ptr(DV), ops._ptr(DB2), ops._ptr(delta),
+                      ops._ptr(DQ), ops._ptr(DK), ops._ptr(DV), ops._ptr(DB2), ops._ptr(delta), ops._ptr(parts),
                       B, N, S, H, D, ops._dt(q), ops._stream())
         dq_t, dk_t, dv_t, db2_t = ctx.in_dtypes
         if want_b2:

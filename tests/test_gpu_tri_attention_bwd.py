@@ -134,3 +134,32 @@ def test_full_size_invariants(dtype):
     want = _autograd_reference(q[:, sl], k[:, sl], v[:, sl], b1[:, sl], b2, do[:, sl])
     for g, w in zip((dq, dk, dv), want[1:4]):
         assert rel_err(g[:, sl], w) <= tol(dtype)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("N,S,H", [(15, 64, 1), (16, 64, 1), (65, 33, 3), (131, 72, 2), (300, 65, 1)])
+def test_sliced_dbias2_equals_one_slice(dtype, N, S, H):
+    """dBias2's rows in one walk (no scratch given) and in slices whose sums are added: 2 (from 16 rows on) to 32
+    slices of unequal length, sizes off the vector lengths.  Two fp32 sums of N terms in another
+    order differ by at most N 2^-24 of the sum of magnitudes, here below 2e-4 of the largest element; then one
+    rounding to the output type.  The other outputs do not depend on it."""
+    from protenix_amd import _lib
+    lib = _lib.load()
+    n_parts = lib.ptx_triattn_core_bwd_partial_elems(N, S, H)
+    assert (n_parts == 0) == (N < 16) and n_parts % (H * S * S) == 0
+    q, k, v, b1, b2, do = (t.cuda() for t in _operands(1, N, S, H, dtype, seed=N))
+    o, lse = P.tri_attention_forward(q, k, v, b1, b2, return_lse=True)
+
+    def run(parts):
+        outs = [torch.full_like(t, float("nan")) for t in (q, k, v, b2)]
+        delta = torch.empty(N * S * H, device="cuda")
+        _lib.check(lib.ptx_triattn_core_bwd_sliced(
+            *(t.data_ptr() for t in (q, k, v, b1, b2, o, lse, do, *outs, delta)), parts, 1, N, S, H, 32,
+            {torch.float32: 0, torch.bfloat16: 1}[dtype], torch.cuda.current_stream().cuda_stream), "bwd")
+        return outs
+    one = run(None)
+    parts = torch.full((n_parts + 64,), float("nan"), device="cuda")
+    sliced = run(parts.data_ptr())
+    assert torch.isnan(parts[n_parts:]).all()            # nothing beyond the scratch that was asked for
+    assert all(torch.equal(a, b) for a, b in zip(one[:3], sliced[:3]))
+    assert rel_err(sliced[3], one[3]) <= (2e-4 if dtype == torch.float32 else 2e-4 + 2.0 ** -8)
