@@ -39,6 +39,12 @@ constexpr int cmax(int a, int b) { return a > b ? a : b; }
   }                                                  \
   const uint32_t block = blockIdx.x - carried, blocks = gridDim.x - carried
 
+// Waves per SIMD that the register allocator leaves room for: three in 16-bit arithmetic (168 registers; the carried
+// stages alone take 148), two on rows of 256 channels and in fp32.  Without that bound the carried stages take 32
+// registers of the accumulation file on top of the kernel's 240 and one workgroup is left per compute unit
+// (triattn_in on rows of 256 channels, 600 tokens: 566 us per launch; with two 377).
+template <typename T, int KS> constexpr int kPpMinWaves = sizeof(T) == 2 && KS <= 8 ? 3 : 2;
+
 // Hidden widths (see Widths in rowgemm.hip): 128 for rows of at most 128 channels, else the row width.
 template <int KS> struct PpWidths {
   static constexpr int SL = KS > 8 ? KS : 8;
@@ -99,7 +105,7 @@ struct ProjInParams {
 // a, b[c][i][k] = mask * sigmoid(gate) * projection in the contraction's fragment order.  Tile: a patch of 4 * RBW
 // outer indices i x 8 inner indices k, which makes a row block's 32 values of one channel 64 contiguous bytes.
 template <typename T, typename TZ, int KS, int RBW>
-__global__ __launch_bounds__(kPpWaves * 64, (sizeof(T) == 2 && KS <= 8 ? 3 : 1)) void pp_trimul_in_kernel(ProjInParams p, SingleStage carry, unsigned carried) {
+__global__ __launch_bounds__(kPpWaves * 64, (kPpMinWaves<T, KS>)) void pp_trimul_in_kernel(ProjInParams p, SingleStage carry, unsigned carried) {
   typedef typename Vec8<T>::type V8;
   typedef typename VecE<T>::type VE_t;
   typedef Cfg<T> C;
@@ -206,7 +212,7 @@ __global__ __launch_bounds__(kPpWaves * 64, (sizeof(T) == 2 && KS <= 8 ? 3 : 1))
 
 // q (scaled), K, V^T, triangle bias and (GATE) sigmoid(gate) in the attention core's layouts.
 template <typename T, typename TZ, int KS, int RBW, bool GATE>
-__global__ __launch_bounds__(kPpWaves * 64, (sizeof(T) == 2 && KS <= 8 ? 3 : 1)) void pp_triattn_in_kernel(ProjInParams p, SingleStage carry, unsigned carried) {
+__global__ __launch_bounds__(kPpWaves * 64, (kPpMinWaves<T, KS>)) void pp_triattn_in_kernel(ProjInParams p, SingleStage carry, unsigned carried) {
   typedef typename Vec8<T>::type V8;
   typedef typename VecE<T>::type VE_t;
   typedef Cfg<T> C;
@@ -359,7 +365,7 @@ struct ProjOutParams {
 
 // out = [z +] (W_z LN_out(x)) * sigmoid(W_g LN_in(z)); out may be z.
 template <typename T, typename TZ, int KS, int RBW>
-__global__ __launch_bounds__(kPpWaves * 64, (sizeof(T) == 2 && KS <= 8 ? 3 : 1)) void pp_trimul_out_kernel(ProjOutParams p, SingleStage carry, unsigned carried) {
+__global__ __launch_bounds__(kPpWaves * 64, (kPpMinWaves<T, KS>)) void pp_trimul_out_kernel(ProjOutParams p, SingleStage carry, unsigned carried) {
   typedef typename Vec8<T>::type V8;
   typedef typename VecE<T>::type VE_t;
   typedef Cfg<T> C;
@@ -464,7 +470,7 @@ __global__ __launch_bounds__(kPpWaves * 64, (sizeof(T) == 2 && KS <= 8 ? 3 : 1))
 // out = [z +] W_o (gate * o): GATE: gate = sigmoid(W_g LN(z)) formed here (16-bit arithmetic, rows of 128 channels,
 // 4 heads: wave = head), otherwise o arrives gated.  out may be z.
 template <typename T, typename TZ, int KS, bool GATE, int RBW>
-__global__ __launch_bounds__(kPpWaves * 64, (sizeof(T) == 2 && KS <= 8 ? 3 : 1)) void pp_triattn_out_kernel(ProjOutParams p, SingleStage carry, unsigned carried) {
+__global__ __launch_bounds__(kPpWaves * 64, (kPpMinWaves<T, KS>)) void pp_triattn_out_kernel(ProjOutParams p, SingleStage carry, unsigned carried) {
   typedef typename Vec8<T>::type V8;
   constexpr int SL = PpWidths<KS>::SL, NOB = KS / 2;
   static_assert(!GATE || (KS == 8 && sizeof(T) == 2), "gate formed here: rows of 128 channels, 16-bit arithmetic");
