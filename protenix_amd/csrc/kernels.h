@@ -121,7 +121,7 @@ int single_stage_run(const SingleStage* s, hipStream_t stream);
 // The row-local stages of the triangle updates on packed weights (pairproj.hip).  carry: null, or a stage of the single
 // track on operands of type TZ that this launch's first workgroups run (it must not depend on the launch).
 // Whether the attention's gate is formed by the output stage (no gate tensor exists then).
-inline bool pp_late_gate(int c_z, int heads, bool bits16) { return c_z == 128 && heads == 4 && bits16; }
+inline bool pp_late_gate(int c_z, int heads, bool bits16) { return bits16 && heads == (c_z == 256 ? 8 : 4); }
 int64_t pp_trimul_packed_elems(int c_z, int hidden);
 template <typename T>
 int pp_trimul_pack(const void* w_ap, const void* w_ag, const void* w_bp, const void* w_bg, const void* w_z,

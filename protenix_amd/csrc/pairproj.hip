@@ -467,13 +467,17 @@ __global__ __launch_bounds__(kPpWaves * 64, (kPpMinWaves<T, KS>)) void pp_trimul
   store_rows<T, TZ, KS, RBW>((TZ*)p.out, z_row, upd, wave, lane, p.add_residual, raw);
 }
 
-// out = [z +] W_o (gate * o): GATE: gate = sigmoid(W_g LN(z)) formed here (16-bit arithmetic, rows of 128 channels,
-// 4 heads: wave = head), otherwise o arrives gated.  out may be z.
+// out = [z +] W_o (gate * o): GATE: gate = sigmoid(W_g LN(z)) formed here (16-bit arithmetic; wave = head, and head + 4
+// on rows of 256 channels), otherwise o arrives gated.  out may be z.  The gate formed here is neither written nor
+// read: on rows of 64 / 256 channels, whose gates are twice / as wide as their rows, one update (projection, core,
+// output) takes 270
+// instead of 281 us at 512 tokens / 1139 instead of 1147 at 600 (per launch: 63 + 156 + 51, was 80 + 165 + 36; 304 + 543 + 292,
+// was 377 + 560 + 210).
 template <typename T, typename TZ, int KS, bool GATE, int RBW>
 __global__ __launch_bounds__(kPpWaves * 64, (kPpMinWaves<T, KS>)) void pp_triattn_out_kernel(ProjOutParams p, SingleStage carry, unsigned carried) {
   typedef typename Vec8<T>::type V8;
   constexpr int SL = PpWidths<KS>::SL, NOB = KS / 2;
-  static_assert(!GATE || (KS == 8 && sizeof(T) == 2), "gate formed here: rows of 128 channels, 16-bit arithmetic");
+  static_assert(!GATE || sizeof(T) == 2, "gate formed here: 16-bit arithmetic");
   constexpr int kFrag = GATE ? RBW * FragLds<T, KS>::ROWBLOCK : 16, kUpd = (int)sizeof(T) * 32 * RBW * kUpdPitch<KS>;
   constexpr int kScratch = cmax(kFrag, kUpd);   // the normalised rows, then the update
   __shared__ __attribute__((aligned(16))) char smem[cmax(kScratch + RBW * FragLds<T, SL>::ROWBLOCK, kStageLds)];
@@ -512,11 +516,16 @@ __global__ __launch_bounds__(kPpWaves * 64, (kPpMinWaves<T, KS>)) void pp_triatt
   typename RowPieces<TZ, KS>::V raw[RBW][RowPieces<TZ, KS>::NP];
   if constexpr (GATE) {
     V8 wg[KS];
+    auto load_wg = [&](int head) {
 #pragma unroll
-    for (int kk = 0; kk < KS; ++kk) wg[kk] = packed_frag<T>((const T*)p.packed_g, wave * KS + kk, lane);
+      for (int kk = 0; kk < KS; ++kk) wg[kk] = packed_frag<T>((const T*)p.packed_g, head * KS + kk, lane);
+    };
+    load_wg(wave);
     norm_rows<T, TZ, KS, RBW>(scratch, (const TZ*)p.z, z_row0, (const T*)p.gamma, (const T*)p.beta, p.eps, wave, lane, raw);
-    load_w(wave);
+    if (HPW == 1 && wave < NOB) load_w(wave);
     __syncthreads();
+#pragma unroll
+    for (int q = 0; q < HPW; ++q)
 #pragma unroll
     for (int rb = 0; rb < RBW; ++rb) {
       f32x16 ag;
@@ -524,17 +533,19 @@ __global__ __launch_bounds__(kPpWaves * 64, (kPpMinWaves<T, KS>)) void pp_triatt
       for (int r = 0; r < 16; ++r) ag[r] = 0.0f;
 #pragma unroll
       for (int kk = 0; kk < KS; ++kk) mma32(ag, wg[kk], FragLds<T, KS>::get(scratch, rb, kk, lane));
+      if (rb == RBW - 1 && q + 1 < HPW) load_wg(wave + 4 * (q + 1));
       // (weight rows packed so that registers 8 u + t are the channels 16 u + 8 g + t of the lane's own fragments;
       // gate and gated output rounded to T like the reference's sigmoid(linear_g(x)) and o * g)
 #pragma unroll
       for (int u = 0; u < 2; ++u) {
-        const f32x8 ov = to_f32(of[rb][0][u]);
+        const f32x8 ov = to_f32(of[rb][q][u]);
         f32x8 gated;
 #pragma unroll
         for (int t = 0; t < 8; ++t) gated[t] = ov[t] * to_f32(from_f32<T>(sigmoidf_fast(ag[8 * u + t])));
-        of[rb][0][u] = from_f32<T>(gated);
+        of[rb][q][u] = from_f32<T>(gated);
       }
     }
+    if (HPW > 1) load_w(wave);
   } else {
     if (wave < NOB) load_w(wave);
     if (p.add_residual) {
@@ -778,9 +789,9 @@ int pp_triattn_in(const void* z, const void* ln_w, const void* ln_b, const void*
   p.backward = 1;
   p.heads = heads;
   p.q_scale = 1.4426950408889634f / sqrtf(32.0f);   // log2(e) / sqrt(d), see triattn.hip
-  if (c_z == 64) return pp_triattn_in_ks<T, TZ, 4, true>(p, carry, stream);
+  if (c_z == 64) return pp_triattn_in_ks<T, TZ, 4, sizeof(T) == 4>(p, carry, stream);
   if (c_z == 256) {
-    if constexpr (sizeof(T) == 2) return pp_triattn_in_ks<T, TZ, 16, true>(p, carry, stream);
+    if constexpr (sizeof(T) == 2) return pp_triattn_in_ks<T, TZ, 16, false>(p, carry, stream);
     else return -1;
   }
   if constexpr (sizeof(T) == 2) return pp_triattn_in_ks<T, TZ, 8, false>(p, carry, stream);
@@ -868,9 +879,9 @@ int pp_triattn_out(const void* o, const void* z, const void* ln_w, const void* l
   p.out = out;
   p.n = n;
   p.add_residual = add_residual;
-  if (c_z == 64) return pp_triattn_out_ks<T, TZ, 4, false>(p, carry, stream);
+  if (c_z == 64) return pp_triattn_out_ks<T, TZ, 4, sizeof(T) == 2>(p, carry, stream);
   if (c_z == 256) {
-    if constexpr (sizeof(T) == 2) return pp_triattn_out_ks<T, TZ, 16, false>(p, carry, stream);
+    if constexpr (sizeof(T) == 2) return pp_triattn_out_ks<T, TZ, 16, true>(p, carry, stream);
     else return -1;
   }
   return pp_triattn_out_ks<T, TZ, 8, sizeof(T) == 2>(p, carry, stream);

@@ -428,8 +428,8 @@ def triangle_multiplicative_update(x: torch.Tensor, incoming: bool, mask: Option
     return out
 
 
-# Triangle attention on rows of 128 channels in bf16 arithmetic: the gate is formed by the output
-# kernel (ptx_triattn_gate_output) instead of travelling through memory.  False restores the
+# Triangle attention in bf16 arithmetic: the gate is formed by the output kernel
+# (ptx_triattn_output_packed, ptx_triattn_gate_output) instead of travelling through memory.  False restores the
 # three stages with a stored gate (tests compare the two).
 late_gate_enabled = True
 
@@ -489,10 +489,13 @@ def triangle_attention(z: torch.Tensor, mask: Optional[torch.Tensor], w: dict, h
     # attention-core layouts (see include/protenix_amd.h): q, gate, output head-major; K, V^T
     # and the triangle bias in fragment-ordered key tiles
     n_kv, n_tb = lib.ptx_triattn_kv_elems(n, heads), lib.ptx_triattn_bias_elems(n, heads)
-    # rows of 128 channels in bf16 arithmetic: no gate tensor, the output kernel forms the gate
+    # bf16 arithmetic (without packed weights, on rows of 128 channels): no gate tensor, the output
+    # kernel forms the gate
     late_gate = late_gate_enabled and c == 128 and heads == 4 and d == 32 and cd == torch.bfloat16
     # (the packed weights are laid out for the gate's place: not with the switch thrown)
     packed = w.get("packed") if late_gate_enabled else None
+    if packed is not None:
+        late_gate = bool(lib.ptx_triattn_late_gate(c, heads, dt))
     q = _workspace((heads, n, n, d), cd, dev)
     g = _workspace((heads, n, n, d), cd, dev)     # the gate, then (or only) the attention output
     k = _workspace((n_kv,), cd, dev)
