@@ -64,17 +64,22 @@ template <typename T> __device__ __forceinline__ typename Vec8<T>::type zero_fra
   return z;
 }
 
-// 8 consecutive bias values starting at key block `kb` (a multiple of 8) of a row of `s` keys,
-// one vector load where rows are 8-aligned (s % 8 == 0: a block of 8 keys is then
-// inside the row or outside as a whole, and an outside block is read from the row's last one;
-// the caller masks it), scalar loads with clamped keys otherwise.
+// 8 consecutive bias values starting at key block `kb` (a multiple of 8) of a row of `s` keys.
+// vec (s % 8 == 0): a block of 8 keys is inside the row or outside as a whole, and an outside block is
+// read from the row's last one (the caller masks it).  Otherwise rows start at any element: a whole block is one load
+// of the element type's alignment (the hardware's vector loads take any; eight loads of one element
+// took dQ 595 us and dK/dV 551 at 500 tokens, 4 heads, bf16, now 323 and 395), the row's last, partial block one load per element.
 template <typename T>
 __device__ __forceinline__ typename Vec8<T>::type load_bias8_raw(const T* row, int kb, int s,
                                                                 bool vec) {
   if (vec) return load8<T>(row + min(kb, s - 8));
   typename Vec8<T>::type v;
+  if (kb + 8 <= s) {
+    __builtin_memcpy(&v, row + kb, sizeof(v));
+  } else {
 #pragma unroll
-  for (int t = 0; t < 8; ++t) v[t] = row[min(kb + t, s - 1)];
+    for (int t = 0; t < 8; ++t) v[t] = row[min(kb + t, s - 1)];
+  }
   return v;
 }
 template <typename T>
@@ -85,12 +90,12 @@ __device__ __forceinline__ f32x8 load_bias8(const T* row, int kb, int s, bool ve
 }  // namespace
 
 // 16-bit kernels double-buffer their shared tiles (one barrier a step) and are held to the
-// registers of three waves per SIMD where rows are 8-aligned; fp32 tiles are twice as
+// registers of three waves per SIMD; fp32 tiles are twice as
 // large and stay single-buffered (two barriers a step).
 template <typename T, bool VEC> struct BwdCfg {
   static constexpr int kBuffers = sizeof(T) == 2 ? 2 : 1;
   // (the second argument of __launch_bounds__: waves per SIMD the register budget allows for)
-  static constexpr int kMinWaves = sizeof(T) == 2 ? (VEC ? 3 : 2) : 1;
+  static constexpr int kMinWaves = sizeof(T) == 2 ? 3 : 1;
 };
 
 // 16-bit tiles are parked in LDS row-major only; an operand that a product needs with the
