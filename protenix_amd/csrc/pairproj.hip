@@ -471,8 +471,9 @@ __global__ __launch_bounds__(kPpWaves * 64, (kPpMinWaves<T, KS>)) void pp_trimul
 // on rows of 256 channels), otherwise o arrives gated.  out may be z.  The gate formed here is neither written nor
 // read: on rows of 64 / 256 channels, whose gates are twice / as wide as their rows, one update (projection, core,
 // output) takes 270
-// instead of 281 us at 512 tokens / 1139 instead of 1147 at 600 (per launch: 63 + 156 + 51, was 80 + 165 + 36; 304 + 543 + 292,
-// was 377 + 560 + 210).
+// instead of 281 us at 512 tokens / 1169 instead of 1207 at 600 (per launch: 63 + 156 + 51, was 80 + 165 + 36; 323 + 571 + 275,
+// was 392 + 603 + 212; 256 channels at 96 / 200 / 400 / 800 tokens: 43 / 118 / 481 / 2242, was 44 / 113 / 487 / 2349).  Two row
+// blocks per workgroup on 256 channels: 292 us at 600, 43 instead of 32 at 200.
 template <typename T, typename TZ, int KS, bool GATE, int RBW>
 __global__ __launch_bounds__(kPpWaves * 64, (kPpMinWaves<T, KS>)) void pp_triattn_out_kernel(ProjOutParams p, SingleStage carry, unsigned carried) {
   typedef typename Vec8<T>::type V8;
@@ -515,12 +516,13 @@ __global__ __launch_bounds__(kPpWaves * 64, (kPpMinWaves<T, KS>)) void pp_triatt
   auto z_row0 = [&](int r) { return max(z_row(r), (int64_t)0); };
   typename RowPieces<TZ, KS>::V raw[RBW][RowPieces<TZ, KS>::NP];
   if constexpr (GATE) {
-    V8 wg[KS];
-    auto load_wg = [&](int head) {
+    // (all of a wave's gate weights under the LayerNorm, the output's first under the last head's products: fetched
+    // when needed, one after the other, they cost rows of 256 channels three waits instead of one)
+    V8 wg[HPW][KS];
 #pragma unroll
-      for (int kk = 0; kk < KS; ++kk) wg[kk] = packed_frag<T>((const T*)p.packed_g, head * KS + kk, lane);
-    };
-    load_wg(wave);
+    for (int q = 0; q < HPW; ++q)
+#pragma unroll
+      for (int kk = 0; kk < KS; ++kk) wg[q][kk] = packed_frag<T>((const T*)p.packed_g, (wave + 4 * q) * KS + kk, lane);
     norm_rows<T, TZ, KS, RBW>(scratch, (const TZ*)p.z, z_row0, (const T*)p.gamma, (const T*)p.beta, p.eps, wave, lane, raw);
     if (HPW == 1 && wave < NOB) load_w(wave);
     __syncthreads();
@@ -532,8 +534,8 @@ __global__ __launch_bounds__(kPpWaves * 64, (kPpMinWaves<T, KS>)) void pp_triatt
 #pragma unroll
       for (int r = 0; r < 16; ++r) ag[r] = 0.0f;
 #pragma unroll
-      for (int kk = 0; kk < KS; ++kk) mma32(ag, wg[kk], FragLds<T, KS>::get(scratch, rb, kk, lane));
-      if (rb == RBW - 1 && q + 1 < HPW) load_wg(wave + 4 * (q + 1));
+      for (int kk = 0; kk < KS; ++kk) mma32(ag, wg[q][kk], FragLds<T, KS>::get(scratch, rb, kk, lane));
+      if (HPW > 1 && rb == RBW - 1 && q == HPW - 2) load_w(wave);
       // (weight rows packed so that registers 8 u + t are the channels 16 u + 8 g + t of the lane's own fragments;
       // gate and gated output rounded to T like the reference's sigmoid(linear_g(x)) and o * g)
 #pragma unroll
@@ -545,7 +547,6 @@ __global__ __launch_bounds__(kPpWaves * 64, (kPpMinWaves<T, KS>)) void pp_triatt
         of[rb][q][u] = from_f32<T>(gated);
       }
     }
-    if (HPW > 1) load_w(wave);
   } else {
     if (wave < NOB) load_w(wave);
     if (p.add_residual) {
