@@ -3,8 +3,7 @@
 Below a few hundred tokens the forward pass is bound by the host: a block issues about forty
 kernel launches and the GPU finishes them faster than Python can enqueue them.  `Graphed`
 records one forward pass of a `PairformerBlock` / `PairformerStack` into a HIP graph (through
-`torch.cuda.CUDAGraph`, which also captures the second stream the stack uses for the single
-track) and replays it for every later call with the same shapes and dtypes (and, for a single
+`torch.cuda.CUDAGraph`) and replays it for every later call with the same shapes and dtypes (and, for a single
 pair mask, the same class of mask: padding at the end with the same number of valid tokens, or
 any other mask - the class decides which attention kernels a forward pass launches).
 
