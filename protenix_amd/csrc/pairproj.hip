@@ -595,6 +595,7 @@ namespace {
 struct PackTile {
   const void* w;
   int row0, n_out, ldw, ksteps, frag0, perm;
+  int raw;   // where the matrix is also kept row-major (elements; 0: not kept)
 };
 constexpr int kMaxPackTiles = 52;
 struct PackList {
@@ -618,11 +619,20 @@ __global__ __launch_bounds__(256) void pair_pack_kernel(PackList list, T* __rest
     u32x4_t* d = reinterpret_cast<u32x4_t*>(packed + (int64_t)(t.frag0 + kk) * kFragElems) + lane;
 #pragma unroll
     for (int pc = 0; pc < PIECES; ++pc) d[pc * kWave] = s[pc];
+    if (t.raw && t.row0 + m < t.n_out)
+      store8<T>(packed + t.raw + (int64_t)(t.row0 + m) * t.ldw + 16 * kk + 8 * (lane >> 5), v);
   }
 }
 
+// On rows of 128 channels the packed weights are followed by the matrices as they are, for the kernels of rowgemm.hip
+// and attnout.hip, which keep them in LDS (resident_rows).
+static int64_t trimul_frag_elems(int c_z, int hidden) { return 5 * (int64_t)c_z * hidden + (int64_t)c_z * c_z; }
+static int64_t triattn_frag_elems(int c_z, int heads) { return (int64_t)(4 * heads + 1) * 32 * c_z + (int64_t)c_z * heads * 32; }
+static bool keeps_rows(int c_z, int hidden) { return c_z == 128 && hidden == 128; }
+constexpr int kMat = 128 * 128;   // such a matrix
+
 int64_t pp_trimul_packed_elems(int c_z, int hidden) {
-  return 5 * (int64_t)c_z * hidden + (int64_t)c_z * c_z;
+  return trimul_frag_elems(c_z, hidden) + (keeps_rows(c_z, hidden) ? 6 * kMat : 0);
 }
 
 template <typename T>
@@ -630,16 +640,17 @@ int pp_trimul_pack(const void* w_ap, const void* w_ag, const void* w_bp, const v
                    const void* w_g, void* packed, int c_z, int hidden, hipStream_t stream) {
   PackList l;
   int nt = 0, f = 0;
-  const int ks = c_z / 16, sl = hidden / 16;
+  const int ks = c_z / 16, sl = hidden / 16, rows0 = (int)trimul_frag_elems(c_z, hidden);
+  auto raw = [&](int i) { return sizeof(T) == 2 && keeps_rows(c_z, hidden) ? rows0 + i * kMat : 0; };
   for (int op = 0; op < 2; ++op)
     for (int cb = 0; cb < hidden / 32; ++cb)
       for (int t = 0; t < 2; ++t) {
-        l.t[nt++] = PackTile{op ? (t ? w_bg : w_bp) : (t ? w_ag : w_ap), 32 * cb, hidden, c_z, ks, f, 0};
+        l.t[nt++] = PackTile{op ? (t ? w_bg : w_bp) : (t ? w_ag : w_ap), 32 * cb, hidden, c_z, ks, f, 0, raw(2 * op + t)};
         f += ks;
       }
   for (int ob = 0; ob < c_z / 32; ++ob) {
-    l.t[nt++] = PackTile{w_z, 32 * ob, c_z, hidden, sl, f, 0};
-    l.t[nt++] = PackTile{w_g, 32 * ob, c_z, c_z, ks, f + sl, 0};
+    l.t[nt++] = PackTile{w_z, 32 * ob, c_z, hidden, sl, f, 0, raw(4)};
+    l.t[nt++] = PackTile{w_g, 32 * ob, c_z, c_z, ks, f + sl, 0, raw(5)};
     f += sl + ks;
   }
   pair_pack_kernel<T><<<dim3(nt), dim3(256), 0, stream>>>(l, (T*)packed);
@@ -647,7 +658,7 @@ int pp_trimul_pack(const void* w_ap, const void* w_ag, const void* w_bp, const v
 }
 
 int64_t pp_triattn_packed_elems(int c_z, int heads) {
-  return (int64_t)(4 * heads + 1) * 32 * c_z + (int64_t)c_z * heads * 32;
+  return triattn_frag_elems(c_z, heads) + (keeps_rows(c_z, heads * 32) ? 5 * kMat + 4 * 128 : 0);
 }
 
 template <typename T>
@@ -655,19 +666,20 @@ int pp_triattn_pack(const void* w_q, const void* w_k, const void* w_v, const voi
                     const void* w_o, void* packed, int c_z, int heads, hipStream_t stream) {
   PackList l;
   int nt = 0, f = 0;
-  const int ks = c_z / 16, sl = heads * 2;
+  const int ks = c_z / 16, sl = heads * 2, rows0 = (int)triattn_frag_elems(c_z, heads);
+  auto raw = [&](int i) { return sizeof(T) == 2 && keeps_rows(c_z, heads * 32) ? rows0 + i * kMat : 0; };   // q, k, v, g, o, bias
   // (the gate formed in the output kernel: its rows permuted, see pp_triattn_out_kernel)
   const bool late = pp_late_gate(c_z, heads, sizeof(T) == 2);
   const void* m[4] = {w_q, w_k, w_v, w_g};
   for (int which = 0; which < 4; ++which)
     for (int h = 0; h < heads; ++h) {
-      l.t[nt++] = PackTile{m[which], 32 * h, heads * 32, c_z, ks, f, which == 3 && late};
+      l.t[nt++] = PackTile{m[which], 32 * h, heads * 32, c_z, ks, f, which == 3 && late, raw(which)};
       f += ks;
     }
-  l.t[nt++] = PackTile{w_b, 0, heads, c_z, ks, f, 0};
+  l.t[nt++] = PackTile{w_b, 0, heads, c_z, ks, f, 0, raw(5)};
   f += ks;
   for (int ob = 0; ob < c_z / 32; ++ob) {
-    l.t[nt++] = PackTile{w_o, 32 * ob, c_z, heads * 32, sl, f, 0};
+    l.t[nt++] = PackTile{w_o, 32 * ob, c_z, heads * 32, sl, f, 0, raw(4)};
     f += sl;
   }
   pair_pack_kernel<T><<<dim3(nt), dim3(256), 0, stream>>>(l, (T*)packed);
@@ -696,6 +708,21 @@ static int out_row_blocks(int64_t rows, int ks, bool attention) {
   return ks == 8 && rows >= (attention ? 320 * 320 : 448 * 448) ? 2 : 1;
 }
 
+// Large calls on 16-bit rows of 128 channels take the kernels that keep all of the weights in LDS, one workgroup per
+// compute unit (rowgemm.hip, attnout.hip): there the rows are half as long and the weights, which every tile here
+// fetches from the L2, weigh twice as much against them.  Only where 8 divides n (their 16-byte accesses) and no stage of
+// the single track rides along.  us per launch, here / resident: trimul_in 640 tokens 94 / 100, 768 132 / 127, 1024 264 / 219,
+// 1536 523 / 478; trimul_out 448 44.1 / 43.5, 512 55 / 52, 768 121 / 113, 1536 465 / 426; triattn_in 256 21.5 / 23.2, 384
+// 34.8 / 33.6, 512 74 / 62, 768 162 / 149, 1536 632 / 592; triattn_out 640 75 / 78, 768 106 / 106, 1024 186 / 182, 1536 415 / 399.
+// (fp32 rows: 768 tokens 139 / 166, 143 / 164, 164 / 172, 133 / 152.)
+enum RowStage { kTriMulInStage, kTriMulOutStage, kTriAttnInStage, kTriAttnOutStage };
+template <typename T, typename TZ>
+static bool resident_rows(RowStage stage, int n, int c_z, int hidden, const SingleStage* carry) {
+  constexpr int kFrom[4] = {704, 480, 352, 896};
+  return sizeof(T) == 2 && std::is_same<T, TZ>::value && keeps_rows(c_z, hidden) && n % 8 == 0 && n >= kFrom[stage] &&
+         !(carry && carry->kind != kStageNone);
+}
+
 template <typename T, typename TZ, int KS>
 static int pp_trimul_in_ks(ProjInParams p, const SingleStage* carry, hipStream_t stream) {
   const int rbw = sizeof(T) == 2 ? in_row_blocks((int64_t)p.n * p.n, KS, false) : 1;
@@ -721,6 +748,13 @@ static int pp_trimul_in_ks(ProjInParams p, const SingleStage* carry, hipStream_t
 template <typename T, typename TZ>
 int pp_trimul_in(const void* z, const void* mask, const void* ln_w, const void* ln_b, const void* packed, void* a,
                  void* b, int n, int c_z, int k_pitch, int incoming, float eps, const SingleStage* carry, hipStream_t stream) {
+  if constexpr (sizeof(T) == 2) {
+    if (resident_rows<T, TZ>(kTriMulInStage, n, c_z, 128, carry)) {
+      const T* m = (const T*)packed + trimul_frag_elems(128, 128);
+      return trimul_project<T, TZ>(z, mask, ln_w, ln_b, m, m + kMat, m + 2 * kMat, m + 3 * kMat, a, b, n, c_z, k_pitch, incoming,
+                                   eps, stream);
+    }
+  }
   ProjInParams p = {};
   p.x = z;
   p.si = incoming ? c_z : (int64_t)n * c_z;
@@ -776,6 +810,13 @@ template <typename T, typename TZ>
 int pp_triattn_in(const void* z, const void* ln_w, const void* ln_b, const void* packed, void* q, void* k, void* vt,
                   void* g, void* tri_bias, int n, int c_z, int heads, int key_pitch, int transposed, float eps,
                   const SingleStage* carry, hipStream_t stream) {
+  if constexpr (sizeof(T) == 2) {
+    if (resident_rows<T, TZ>(kTriAttnInStage, n, c_z, heads * 32, carry)) {
+      const T* m = (const T*)packed + triattn_frag_elems(128, 4);
+      return triattn_project<T, TZ>(z, ln_w, ln_b, m, m + kMat, m + 2 * kMat, m + 3 * kMat, m + 5 * kMat, q, k, vt, nullptr,
+                                    tri_bias, n, c_z, heads, 32, key_pitch, transposed, eps, stream);
+    }
+  }
   ProjInParams p = {};
   p.x = z;
   p.si = transposed ? c_z : (int64_t)n * c_z;
@@ -841,6 +882,13 @@ template <typename T, typename TZ>
 int pp_trimul_out(const void* x, int ldx, const void* z, const void* ln_in_w, const void* ln_in_b,
                   const void* ln_out_w, const void* ln_out_b, const void* packed, void* out, int n, int c_z,
                   int hidden, int add_residual, float eps, const SingleStage* carry, hipStream_t stream) {
+  if constexpr (sizeof(T) == 2) {
+    if (ldx == n && resident_rows<T, TZ>(kTriMulOutStage, n, c_z, hidden, carry)) {
+      const T* m = (const T*)packed + trimul_frag_elems(128, 128);
+      return trimul_output<T, TZ>(x, z, ln_in_w, ln_in_b, ln_out_w, ln_out_b, m + 4 * kMat, m + 5 * kMat, out, n, c_z,
+                                  add_residual, eps, stream);
+    }
+  }
   ProjOutParams p = {};
   p.z = z;
   p.si = (int64_t)n * c_z;
@@ -867,6 +915,12 @@ int pp_trimul_out(const void* x, int ldx, const void* z, const void* ln_in_w, co
 template <typename T, typename TZ>
 int pp_triattn_out(const void* o, const void* z, const void* ln_w, const void* ln_b, const void* packed, void* out,
                    int n, int c_z, int heads, int transposed, int add_residual, float eps, const SingleStage* carry, hipStream_t stream) {
+  if constexpr (sizeof(T) == 2) {
+    if (resident_rows<T, TZ>(kTriAttnOutStage, n, c_z, heads * 32, carry)) {
+      const T* m = (const T*)packed + triattn_frag_elems(128, 4);
+      return triattn_gate_output<TZ>(o, z, ln_w, ln_b, m + 3 * kMat, m + 4 * kMat, out, n, transposed, add_residual, eps, stream);
+    }
+  }
   ProjOutParams p = {};
   p.z = z;
   p.si = transposed ? c_z : (int64_t)n * c_z;

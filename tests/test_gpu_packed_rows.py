@@ -26,6 +26,9 @@ def _call(mod, args, mode):
 
 # (sizes around the lines of in_row_blocks / out_row_blocks, and both kinds of tiles: n a multiple of 8 or not)
 SIZES = ([(128, m, n) for m in ("amp", "bf16") for n in (159, 160, 161, 319, 320, 447, 448, 449)]
+         # (from 352, 480, 704 and 896 on, rows in bf16 take the kernels with all weights in LDS, out of the same packed
+         # buffer; 360 has some of the four stages there, 904 all, 903 none)
+         + [(128, "bf16", n) for n in (344, 352, 360, 480, 704, 903, 904)] + [(128, "amp", 704)]
          + [(128, "fp32", n) for n in (31, 33, 160, 323)]
          + [(64, m, n) for m in ("amp", "fp32") for n in (32, 161, 399, 400, 450)]
          + [(256, m, n) for m in ("amp", "bf16") for n in (33, 95, 96, 97, 199, 200, 203)])
