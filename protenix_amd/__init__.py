@@ -19,6 +19,9 @@ from .triangular import (
     kernel_triangular_mult,
     triangle_multiplicative_update,
 )
+from . import native as _native
+
+_native._own_classes()      # (the classes as they are here, before anybody can have changed them)
 
 __all__ = [
     "Graphed",

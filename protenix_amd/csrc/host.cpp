@@ -52,7 +52,17 @@ Tensor take(const py::dict& d, const char* key) {
 int take_int(const py::dict& d, const char* key) { return d.contains(key) ? d[key].cast<int>() : 0; }
 
 // ---- what a plan's weights were made from ---------------------------------------------------
+// A plan stands in for a tree of modules only while every one of them is of a class it knows and runs that class's
+// own forward; a sub-module of another type, a class changed under way or a `forward` set on an instance makes
+// it stale.
 struct Guard {
+  struct Module {
+    py::object dict;            // m.__dict__
+    PyObject* m;                // (held by its parent's entry, or by the caller)
+    py::object type;
+  };
+  std::vector<Module> modules;
+  bool foreign = false;            // a module of a class that is not among `classes`
   struct Entry {
     py::object dict, key, value;   // dict[key] is value
     int64_t version = -1;          // of a parameter
@@ -74,8 +84,15 @@ struct Guard {
     entries.push_back(std::move(e));
   }
   // `m` and everything below it; the plain attributes named in `attrs` where they exist
-  void walk(const py::object& m, const py::list& attrs) {
+  Guard(const py::object& m, const py::list& attrs, const py::set& classes) { walk(m, attrs, classes); }
+  void walk(const py::object& m, const py::list& attrs, const py::set& classes) {
     py::dict d = m.attr("__dict__");
+    py::object type = py::reinterpret_borrow<py::object>((PyObject*)Py_TYPE(m.ptr()));
+    if (!classes.contains(type)) {
+      foreign = true;
+      return;
+    }
+    modules.push_back(Module{d, m.ptr(), std::move(type)});
     py::dict params = d["_parameters"], mods = d["_modules"];
     for (auto item : params) add(params, item.first);
     empty.push_back(d["_forward_hooks"]);
@@ -84,10 +101,12 @@ struct Guard {
       if (d.contains(a)) add(d, a);
     for (auto item : mods) {
       add(mods, item.first);
-      if (!item.second.is_none()) walk(py::reinterpret_borrow<py::object>(item.second), attrs);
+      if (!item.second.is_none()) walk(py::reinterpret_borrow<py::object>(item.second), attrs, classes);
     }
   }
   bool valid() const {
+    static PyObject* const forward = PyUnicode_InternFromString("forward");
+    if (foreign) return false;
     for (const Entry& e : entries) {
       PyObject* now = PyDict_GetItem(e.dict.ptr(), e.key.ptr());   // borrowed
       if (now != e.value.ptr()) return false;
@@ -98,6 +117,8 @@ struct Guard {
     }
     for (const py::object& d : empty)
       if (PyDict_Size(d.ptr()) != 0) return false;
+    for (const Module& m : modules)   // (the entries hold: every module is still where it was)
+      if ((PyObject*)Py_TYPE(m.m) != m.type.ptr() || PyDict_GetItem(m.dict.ptr(), forward)) return false;
     return true;
   }
 };
@@ -246,13 +267,13 @@ struct Block {
   int heads = 0, d = 0;
   double a_eps = kEps, s_eps = kEps;
   at::ScalarType compute;
-  Guard guard;
+  std::shared_ptr<const Guard> guard;
 
-  Block(const py::object& module, const py::dict& d_, const py::list& attrs)
+  Block(std::shared_ptr<const Guard> guard_, const py::dict& d_)
       : out(d_["tri_mul_out"].cast<py::dict>()), in(d_["tri_mul_in"].cast<py::dict>()), start(d_["tri_att_start"].cast<py::dict>()),
         end(d_["tri_att_end"].cast<py::dict>()), fused(take_int(d_, "fused") != 0), tr_ln_w(take(d_, "tr_ln_w")),
         tr_ln_b(take(d_, "tr_ln_b")), tr_packed(take(d_, "tr_packed")), n_factor(take_int(d_, "n_factor")), c_z(take_int(d_, "c_z")),
-        c_s(take_int(d_, "c_s")) {
+        c_s(take_int(d_, "c_s")), guard(std::move(guard_)) {
     compute = tr_packed.scalar_type();
     if (c_s) {
       pb_ln_w = take(d_, "pb_ln_w"); pb_ln_b = take(d_, "pb_ln_b"); pb_w = take(d_, "pb_w");
@@ -266,9 +287,8 @@ struct Block {
       a_eps = d_["a_eps"].cast<double>();
       s_eps = d_["s_eps"].cast<double>();
     }
-    guard.walk(module, attrs);
   }
-  bool valid() const { return guard.valid(); }
+  bool valid() const { return guard->valid(); }
 
   // The five pair updates of the pair tensors of z [batch][n][n][c_z] in place; the single attention's pair
   // bias (fp32 [batch][heads][n][n]) of the finished z into `bias` (null: none wanted).
@@ -403,14 +423,13 @@ struct Update {
   optional<TriMul> mul;
   optional<TriAtt> att;
   at::ScalarType compute;
-  Guard guard;
-  Update(const py::object& module, const py::dict& d, const py::list& attrs) {
+  std::shared_ptr<const Guard> guard;
+  Update(std::shared_ptr<const Guard> guard_, const py::dict& d) : guard(std::move(guard_)) {
     if (d.contains("heads")) att.emplace(d);
     else mul.emplace(d);
     compute = (att ? att->packed : mul->packed).scalar_type();
-    guard.walk(module, attrs);
   }
-  bool valid() const { return guard.valid(); }
+  bool valid() const { return guard->valid(); }
   // out = [z +] update for every pair tensor of z (contiguous); out may be z
   void run(const Tensor& z, const Tensor& out, const py::list& mask_list, bool add) const {
     const std::vector<Mask> masks = masks_of(mask_list);
@@ -547,11 +566,14 @@ Tensor tri_attention(const Tensor& q, const Tensor& k, const Tensor& v, const op
 PYBIND11_MODULE(_host, m) {
   m.doc() = "native host path of protenix_amd (see csrc/host.cpp)";
   m.def("abi_version", []() { return ptx_version(); });
+  py::class_<Guard, std::shared_ptr<Guard>>(m, "Guard")
+      .def(py::init<const py::object&, const py::list&, const py::set&>(), py::arg("module"), py::arg("attrs"), py::arg("classes"))
+      .def("valid", &Guard::valid);
   py::class_<Block>(m, "Block")
-      .def(py::init<const py::object&, const py::dict&, const py::list&>())
+      .def(py::init<std::shared_ptr<Guard>, const py::dict&>())
       .def("valid", &Block::valid);
   py::class_<Update>(m, "Update")
-      .def(py::init<const py::object&, const py::dict&, const py::list&>())
+      .def(py::init<std::shared_ptr<Guard>, const py::dict&>())
       .def("valid", &Update::valid)
       .def("run", &Update::run);
   m.def("first_stale", [](const std::vector<const Block*>& blocks) {

@@ -2,9 +2,11 @@
 laid out for the kernels, with a record of the parameters they came from - it takes them with.
 
 Plans live here, keyed weakly by module: they are built on a module's first call, checked on every call
-(a replaced or modified parameter, a replaced sub-module or a registered hook makes a plan stale)
-and go away with the module.  What the native path does not cover returns None here and runs through
-the Python path, which has the same kernels in the same order and all the error messages.
+(a replaced or modified parameter, a replaced sub-module, another class, a replaced `forward` or a
+registered hook makes a plan stale) and go away with the module.  A plan stands for this package's own
+classes only, each running its own `forward`.  What the native path does not cover is refused here
+(run_blocks returns NotImplemented, run_update False) and runs through the Python path, which has the same kernels
+in the same order and all the error messages.
 """
 from __future__ import annotations
 
@@ -40,10 +42,43 @@ def host():
     return _host
 
 
+_own: Optional[tuple] = None
+
+
+def _own_classes() -> tuple:
+    """(the classes a plan may stand for, as a set; each with the function that was its forward when this
+    was first asked for)."""
+    global _own
+    if _own is None:
+        from . import layer_norm, pairformer, primitives, transformer, triangular as tri
+        classes = [layer_norm.FusedLayerNorm, primitives.Linear, primitives.Transition, tri.TriangleMultiplicativeUpdate,
+                   tri.TriangleMultiplicationOutgoing, tri.TriangleMultiplicationIncoming, tri.Attention,
+                   tri.TriangleAttention, tri.TriangleAttentionEndingNode, transformer.Attention,
+                   transformer.AttentionPairBias, pairformer.PairformerBlock, torch.nn.Sigmoid]
+        _own = (set(classes), [(c, c.forward) for c in classes])
+    return _own
+
+
+def runs_own_forward(module) -> bool:
+    """Whether calling `module` runs the forward its class in this package has, and nothing else (no `forward` of a
+    subclass, of the instance or put into the class, no hooks): its kernels may then be issued without the call."""
+    classes, forwards = _own_classes()
+    return (type(module) in classes and "forward" not in module.__dict__ and not module._forward_hooks
+            and not module._forward_pre_hooks and all(c.forward is f for c, f in forwards))
+
+
 def _usable(z: torch.Tensor) -> bool:
     return (ops.use_native() and z.is_cuda and not torch.is_grad_enabled() and z.dim() >= 3 and z.shape[-2] == z.shape[-3]
             and z.numel() > 0 and z.dtype in (torch.float32, torch.bfloat16)
-            and not _nn_module._global_forward_hooks and not _nn_module._global_forward_pre_hooks)
+            and not _nn_module._global_forward_hooks and not _nn_module._global_forward_pre_hooks
+            and all(c.forward is f for c, f in _own_classes()[1]))
+
+
+def _guard(module):
+    """A record of what the module's plans are made from, or None where it cannot be relied on (hooks, other
+    classes, parameters without version counters)."""
+    g = host().Guard(module, _ATTRS, _own_classes()[0])
+    return g if g.valid() else None
 
 
 def _masks(z: torch.Tensor, mask: Optional[torch.Tensor], cd: torch.dtype) -> list:
@@ -134,11 +169,9 @@ def _block_plan(blk, z, cd, sd):
     plans = _plans.setdefault(blk, {})
     plan = plans.get(key)
     if plan is None or not plan.valid():
-        spec = _block_spec(blk, z, cd, sd)
-        plan = None if spec is None else host().Block(blk, spec, _ATTRS)
-        if plan is not None and not plan.valid():      # hooks, or parameters without version counters
-            plan = None
-        plans[key] = plan
+        guard = _guard(blk)
+        spec = None if guard is None else _block_spec(blk, z, cd, sd)
+        plan = plans[key] = None if spec is None else host().Block(guard, spec)
     return plan
 
 
@@ -195,12 +228,12 @@ def run_update(module, z: torch.Tensor, cd: torch.dtype, mask: Optional[torch.Te
     plans = _plans.setdefault(module, {})
     plan = plans.get(key)
     if plan is None or not plan.valid():
+        guard = _guard(module)
+        if guard is None:
+            return False
         spec = _mul_spec(module, cd, z.device) if transposed is None else _att_spec(module, cd, z.device, transposed)
         if spec is None or z.shape[-1] != spec.get("c_z", spec.get("c")):
             return False
-        plan = host().Update(module, spec, _ATTRS)
-        if not plan.valid():
-            return False
-        plans[key] = plan
+        plan = plans[key] = host().Update(guard, spec)
     plan.run(z, out, _masks(z, mask, cd), add)
     return True

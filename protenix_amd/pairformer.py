@@ -126,6 +126,12 @@ class PairformerBlock(nn.Module):
             return self._forward_autocast_unfused(s, z, pair_mask, ac, pad)
         # (fp32 z under bf16 autocast: the same fused kernels, reading and updating the fp32
         # rows in place with bf16 arithmetic)
+        if self.c_s > 0 and not native.runs_own_forward(self.attention_pair_bias):
+            # another module in its place: called as the reference calls it (pairformer.py:216-224)
+            self._pair_track(z, pair_mask)
+            zc = z if pad is None else z[..., :pad.n, :pad.n, :].contiguous()
+            s = s + self.attention_pair_bias(s, None, zc).to(s.dtype)
+            return self._single_transition(s), z
         bias = self._pair_track(z, pair_mask, want_bias=self.c_s > 0)
         if self.c_s > 0:
             s = self._single_track(s, bias if pad is None else pad.crop_bias(bias))
@@ -150,14 +156,17 @@ class PairformerBlock(nn.Module):
         `want_bias`, also the pair bias of the single attention, read off the finished z: in
         the transition's own epilogue where that kernel has one, by a kernel of its own
         otherwise."""
-        self.tri_mul_out(z, mask=pair_mask, inplace_safe=True, _add_with_inplace=True)
-        self.tri_mul_in(z, mask=pair_mask, inplace_safe=True, _add_with_inplace=True)
-        self.tri_att_start._run(z, pair_mask, transposed=False, residual_inplace=True)
+        for mul in (self.tri_mul_out, self.tri_mul_in):
+            z_new = mul(z, mask=pair_mask, inplace_safe=True, _add_with_inplace=True)
+            if z_new is not z:      # (another module in its place may return z + update in a new tensor)
+                z.copy_(z_new)
+        self._add_attention(self.tri_att_start, z, pair_mask, transposed=False)
         # ending node: the starting-node module of the reference applied to z^T with
         # mask^T, expressed through transposed addressing of z and mask
         apb = self.attention_pair_bias if want_bias else None
         att, tr = self.tri_att_end, self.pair_transition
-        if (z.is_contiguous() and tr.c_in == att.c_in
+        own_att, own_tr = native.runs_own_forward(att), native.runs_own_forward(tr)
+        if (own_att and own_tr and z.is_contiguous() and tr.c_in == att.c_in
                 and ops.fuses_attention_transition(z, att.no_heads, att.c_hidden, tr.n)
                 and (apb is None or apb.n_heads <= 32)):
             # the ending node's last stage and the transition (and the pair bias) in one launch:
@@ -173,11 +182,13 @@ class PairformerBlock(nn.Module):
             n = z.shape[-2]
             bias = biases[0] if len(biases) == 1 else torch.stack(biases)
             return bias.view(*z.shape[:-3], apb.n_heads, n, n)
-        self.tri_att_end._run(z, pair_mask, transposed=True, residual_inplace=True)
+        self._add_attention(att, z, pair_mask, transposed=True)
+        if not own_tr:
+            z.add_(tr(z))
+            return apb.pair_bias(z) if want_bias else None
         if not want_bias:
             self.pair_transition(z, _residual_out=z)
             return None
-        apb = self.attention_pair_bias
         n = z.shape[-2]
         if z.is_contiguous() and self.pair_transition.fuses_pair_bias(z, apb.n_heads):
             # (one launch per pair tensor of a batch: the epilogue writes [heads][rows])
@@ -188,6 +199,25 @@ class PairformerBlock(nn.Module):
             return bias.view(*z.shape[:-3], apb.n_heads, n, n)
         self.pair_transition(z, _residual_out=z)
         return apb.pair_bias(z)
+
+    @staticmethod
+    def _add_attention(att, z: torch.Tensor, pair_mask: Optional[torch.Tensor], transposed: bool,
+                       rows: Optional[torch.Tensor] = None, rows_mask: Optional[torch.Tensor] = None) -> None:
+        """z += att(z), or for the ending node att(z^T)^T (in place; `rows`: what the update is computed from in
+        z's place).  The package's own module reads and writes z through transposed addressing; any
+        other (a sub-class, a `forward` put in its place, hooks) is called as the module it is,
+        on z and mask as the reference hands them over (pairformer.py:190-214)."""
+        x, mask = (z, pair_mask) if rows is None else (rows, rows_mask)
+        if native.runs_own_forward(att):
+            if rows is None:
+                att._run(x, mask, transposed=transposed, residual_inplace=True)
+            else:
+                z.add_(att._run(x, mask, transposed=transposed, residual_inplace=False))
+        elif transposed:
+            z.add_(att(x.transpose(-2, -3).contiguous(),
+                       mask=None if mask is None else mask.transpose(-1, -2)).transpose(-2, -3))
+        else:
+            z.add_(att(x, mask=mask))
 
     def _forward_autocast_unfused(self, s: Optional[torch.Tensor], z: torch.Tensor,
                                   pair_mask: Optional[torch.Tensor], ac: torch.dtype, pad=None
@@ -201,8 +231,8 @@ class PairformerBlock(nn.Module):
         m = None if pair_mask is None else pair_mask.to(ac)
         z.add_(self.tri_mul_out(z.to(ac), mask=m))
         z.add_(self.tri_mul_in(z.to(ac), mask=m))
-        z.add_(self.tri_att_start._run(z.to(ac), m, transposed=False, residual_inplace=False))
-        z.add_(self.tri_att_end._run(z.to(ac), m, transposed=True, residual_inplace=False))
+        self._add_attention(self.tri_att_start, z, None, False, z.to(ac), m)
+        self._add_attention(self.tri_att_end, z, None, True, z.to(ac), m)
         z.add_(self.pair_transition(z.to(ac)))
         if self.c_s > 0:
             bias = self.attention_pair_bias.pair_bias(z.to(ac))
@@ -217,7 +247,13 @@ class PairformerBlock(nn.Module):
         transition, costs s a 2.4e-2 relative error against 5e-3 this way)."""
         with torch.autocast("cuda", enabled=False):
             s = self.attention_pair_bias.forward_with_bias(s, bias, residual=s)
-            return self.single_transition(s, _residual_new=True)
+        return self._single_transition(s)
+
+    def _single_transition(self, s: torch.Tensor) -> torch.Tensor:
+        with torch.autocast("cuda", enabled=False):
+            if native.runs_own_forward(self.single_transition):
+                return self.single_transition(s, _residual_new=True)
+            return s + self.single_transition(s)
 
 
 class PairformerStack(nn.Module):
@@ -245,7 +281,8 @@ class PairformerStack(nn.Module):
                 raise RuntimeError("protenix_amd.PairformerStack is inference-only: call .eval()")
         pad = None
         z_caller = z
-        if _wants_padding(z, pair_mask) and len(self.blocks) > 0:
+        own = all(native.runs_own_forward(b) for b in self.blocks)
+        if own and _wants_padding(z, pair_mask) and len(self.blocks) > 0:
             # (one padded copy for the whole stack, see pad_tokens_to)
             pad = _Padded(z)
             z, pair_mask = pad.z, pad.mask
@@ -264,7 +301,8 @@ class PairformerStack(nn.Module):
             if s_new is not NotImplemented:
                 return s_new, z
         ac = ops.autocast_compute_dtype(z)
-        if (not z.is_cuda or s is None or any(b.c_s == 0 for b in self.blocks)
+        if (not own or not z.is_cuda or s is None
+                or any(b.c_s == 0 or not native.runs_own_forward(b.attention_pair_bias) for b in self.blocks)
                 or (ac is not None and ops.compute_dtype(z) == z.dtype)):
             for blk in self.blocks:
                 if pad is None:
