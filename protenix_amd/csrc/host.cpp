@@ -377,7 +377,10 @@ struct Block {
 
 // The blocks in sequence on z (contiguous, updated in place).  The single track of a block runs underneath the next
 // block's pair kernels (see Stages).  Returns the new s (undefined for a stack without a single track).
-optional<Tensor> run_blocks(const std::vector<const Block*>& blocks, const optional<Tensor>& s_opt, const Tensor& z, const py::list& mask_list) {
+// Owns the blocks it was given until it returns: the caller's list is shared, and another thread may
+// put a new plan into it while this one runs without the interpreter's lock.
+using Blocks = std::vector<std::shared_ptr<Block>>;
+optional<Tensor> run_blocks(const Blocks& blocks, const optional<Tensor>& s_opt, const Tensor& z, const py::list& mask_list) {
   const std::vector<Mask> masks = masks_of(mask_list);
   py::gil_scoped_release nogil;
   const int n = (int)z.size(-2);
@@ -387,7 +390,7 @@ optional<Tensor> run_blocks(const std::vector<const Block*>& blocks, const optio
   const bool single = s_opt.has_value() && s_opt->defined() && blocks[0]->c_s > 0;
   const int64_t es = single ? (int64_t)s_opt->element_size() : 0;
   int64_t ws_bytes = 0, single_bytes = 0, bias_elems = 0;
-  for (const Block* b : blocks) {
+  for (const auto& b : blocks) {
     ws_bytes = std::max(ws_bytes, workspace_bytes(n, std::max(b->out.c_h, b->in.c_h), std::max(b->start.heads, b->end.heads),
                                                   at::elementSize(b->compute)));
     if (single) {
@@ -406,7 +409,7 @@ optional<Tensor> run_blocks(const std::vector<const Block*>& blocks, const optio
     s = s_opt->data_ptr();
   }
   Stages singles;
-  for (const Block* b : blocks) {
+  for (const auto& b : blocks) {
     float* bp = single ? (float*)bias.data_ptr() : nullptr;
     b->pair_track(z, masks, batch, n, ws.data_ptr(), bp, singles, st);
     if (single) {
@@ -569,14 +572,14 @@ PYBIND11_MODULE(_host, m) {
   py::class_<Guard, std::shared_ptr<Guard>>(m, "Guard")
       .def(py::init<const py::object&, const py::list&, const py::set&>(), py::arg("module"), py::arg("attrs"), py::arg("classes"))
       .def("valid", &Guard::valid);
-  py::class_<Block>(m, "Block")
+  py::class_<Block, std::shared_ptr<Block>>(m, "Block")
       .def(py::init<std::shared_ptr<Guard>, const py::dict&>())
       .def("valid", &Block::valid);
   py::class_<Update>(m, "Update")
       .def(py::init<std::shared_ptr<Guard>, const py::dict&>())
       .def("valid", &Update::valid)
       .def("run", &Update::run);
-  m.def("first_stale", [](const std::vector<const Block*>& blocks) {
+  m.def("first_stale", [](const Blocks& blocks) {
     for (size_t i = 0; i < blocks.size(); ++i)
       if (!blocks[i]->valid()) return (int64_t)i;
     return (int64_t)-1;

@@ -1,0 +1,84 @@
+"""A call owns the plans it was given until it returns, whatever becomes of the list they came in."""
+import collections.abc
+import sys
+import threading
+
+import pytest
+import torch
+
+import protenix_amd as P
+from protenix_amd import native
+from oracle import pairformer_oracle as O
+from tests.util import oracle_and_product
+
+
+class Key(str):
+    """A parameter's name whose look-up can be watched (a plan is examined by looking its parameters up)."""
+    seen = None
+
+    def __hash__(self):
+        if Key.seen is not None:
+            Key.seen()
+        return str.__hash__(self)
+
+    def __eq__(self, other):
+        return str.__eq__(self, other)
+
+
+def test_plans_outlive_the_sequence_they_came_in():
+    ln = P.FusedLayerNorm(8)
+    weight = ln._parameters.pop("weight")
+    ln._parameters[Key("weight")] = weight
+    spec = {"packed": torch.zeros(1)}
+    spec = {k: spec for k in ("tri_mul_out", "tri_mul_in")} | {k: spec | {"inf": 1.0} for k in ("tri_att_start", "tri_att_end")}
+    spec["tr_packed"] = torch.zeros(1)
+
+    def block():
+        return native.host().Block(native._guard(ln), spec)
+    kept = block()
+
+    class Handed(collections.abc.Sequence):        # nobody else holds what it hands out
+        def __len__(self):
+            return 3
+
+        def __getitem__(self, i):
+            if i >= 3:
+                raise IndexError
+            return block()
+    held = []
+    Key.seen = lambda: held.append(sys.getrefcount(weight))
+    try:
+        assert native.host().first_stale([kept]) == -1 and len(held) == 1
+        alone = held.pop()
+        assert native.host().first_stale(Handed()) == -1
+    finally:
+        Key.seen = None
+    assert max(held) == alone + 3       # all three records hold the parameter while they are examined
+
+
+@pytest.mark.gpu
+def test_a_stack_called_by_two_threads_while_its_parameters_change():
+    """A parameter is replaced between calls by equal values, so that every call finds some plans stale and all
+    results are the same."""
+    _, prod = oracle_and_product(O.PairformerStack, P.PairformerStack, n_blocks=4)
+    s, z, pm = (t.cuda() for t in O.make_inputs(40, n_pad=3))
+    with torch.no_grad():
+        s0, z0 = prod(s, z, pm)
+    torch.cuda.synchronize()
+    wrong, lock = [], threading.Lock()
+
+    def work(k):
+        with torch.no_grad():
+            for i in range(12):
+                lin = prod.blocks[(i + k) % 4].tri_mul_in.linear_g
+                with lock:
+                    lin.weight = torch.nn.Parameter(lin.weight.detach())
+                s1, z1 = prod(s, z, pm)
+                if not (torch.equal(s1, s0) and torch.equal(z1, z0)):
+                    wrong.append((k, i))
+    ts = [threading.Thread(target=work, args=(k,)) for k in range(2)]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    assert not wrong
