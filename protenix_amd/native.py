@@ -118,6 +118,12 @@ def _fragments(w: torch.Tensor) -> torch.Tensor:
     return w.view(n // 16, 16, k // 32, 8 // v, 4, v).permute(0, 2, 3, 4, 1, 5).contiguous()
 
 
+def _aligned(t: Optional[torch.Tensor]) -> Optional[torch.Tensor]:
+    """t, or a copy of it where it does not start at a multiple of 16 bytes (a view into a flat buffer): the
+    single track's stages read whole vectors, unlike the stand-alone kernels of the Python path."""
+    return t if t is None or t.data_ptr() % 16 == 0 else t.clone()
+
+
 def _block_spec(blk, z: torch.Tensor, cd: torch.dtype, sd: Optional[torch.dtype]) -> Optional[dict]:
     from .primitives import _cv
     dev, c, tr, end = z.device, z.shape[-1], blk.pair_transition, blk.tri_att_end
@@ -155,9 +161,9 @@ def _block_spec(blk, z: torch.Tensor, cd: torch.dtype, sd: Optional[torch.dtype]
         st_ps = (st.linear_no_bias_a.weight, st.linear_no_bias_b.weight, st.linear_no_bias.weight)
         s_wa, s_wb, s_wo = st._cache_ab.get(st_ps, sd, dev, lambda: tuple(_cv(p, sd, dev) for p in st_ps))
         w_o = att._cache_out.get((att.linear_o.weight,), sd, dev, lambda: _cv(att.linear_o.weight, sd, dev))
-        spec.update(pb_ln_w=pw[0], pb_ln_b=pw[1], pb_w=pw[2], a_ln_w=_cv(apb.layernorm_a.weight, sd, dev),
-                    a_ln_b=_cv(apb.layernorm_a.bias, sd, dev), a_eps=float(apb.layernorm_a.eps), w_in=_fragments(w_in), b_q=b_q, w_o=_fragments(w_o),
-                    s_ln_w=_cv(st.layernorm1.weight, sd, dev), s_ln_b=_cv(st.layernorm1.bias, sd, dev),
+        spec.update(pb_ln_w=pw[0], pb_ln_b=pw[1], pb_w=pw[2], a_ln_w=_aligned(_cv(apb.layernorm_a.weight, sd, dev)),
+                    a_ln_b=_aligned(_cv(apb.layernorm_a.bias, sd, dev)), a_eps=float(apb.layernorm_a.eps), w_in=_fragments(w_in), b_q=b_q, w_o=_fragments(w_o),
+                    s_ln_w=_aligned(_cv(st.layernorm1.weight, sd, dev)), s_ln_b=_aligned(_cv(st.layernorm1.bias, sd, dev)),
                     s_eps=float(st.layernorm1.eps), s_wa=_fragments(s_wa), s_wb=_fragments(s_wb), s_wo=_fragments(s_wo),
                     heads=H, d=d, hidden=st.n * cs)
     return spec
@@ -215,7 +221,7 @@ def run_blocks(owner, blocks, s: Optional[torch.Tensor], z: torch.Tensor, pair_m
             plans.append(plan)
         _plans[owner][("stack", key)] = ([weakref.ref(b) for b in blocks], plans)
     masks = _masks(z, pair_mask, cd)
-    return host().run_blocks(plans, s.contiguous() if single else s, z, masks)
+    return host().run_blocks(plans, _aligned(s.contiguous()) if single else s, z, masks)
 
 
 def run_update(module, z: torch.Tensor, cd: torch.dtype, mask: Optional[torch.Tensor], out: torch.Tensor, add: bool,
