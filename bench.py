@@ -489,12 +489,12 @@ def main() -> int:
                     return st_odd(s7, zw7, None, inplace_safe=True)
             odd = {}
             for pad_to in (8, 0):
-                keep_pad = pf.pad_tokens_to, pf.pad_tokens_end_n
-                pf.pad_tokens_to, pf.pad_tokens_end_n = pad_to, 1 << 30
+                keep_pad = pf.pad_tokens_to, pf.pad_tokens_min_n
+                pf.pad_tokens_to, pf.pad_tokens_min_n = pad_to, 0
                 try:
                     _, per_odd, out_odd = timed(step_odd, 2, 5)
                 finally:
-                    pf.pad_tokens_to, pf.pad_tokens_end_n = keep_pad
+                    pf.pad_tokens_to, pf.pad_tokens_min_n = keep_pad
                 odd[pad_to] = (statistics.median(per_odd) / 4, out_odd[1].clone())
             shapes["odd_size_n700_4_blocks"] = {
                 "ms_per_block": round(odd[8][0], 3), "ms_per_block_unpadded": round(odd[0][0], 3),

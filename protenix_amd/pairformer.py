@@ -23,12 +23,11 @@ from .triangular import (TriangleAttention, TriangleMultiplicationIncoming,
 
 
 # Pair tensors whose N_token is not a multiple of pad_tokens_to can be worked on as the next multiple
-# with the extra tokens masked out, from pad_tokens_min_n tokens up to below pad_tokens_end_n.  The
-# row-local kernels on packed weights take any N with 16-byte accesses (tiles that stay inside one row
-# of the pair tensor, a padded pitch of the triangle product), and rows as they are now beat padded
-# ones at every size and width measured (us per block, padded / as they are: c_z = 128 at 363 tokens
-# 780 / 715, 501 1319 / 1226, 1021 5748 / 5521; c_z = 64 at 501 932 / 862; c_z = 256 at 501 3522 / 3406;
-# fp32 at 403 3619 / 3396), so the band is a token one.
+# with the extra tokens masked out, from pad_tokens_min_n tokens on.  Not by default: the row-local
+# kernels on packed weights take any N with 16-byte accesses (tiles that stay inside one row of the pair
+# tensor, a padded pitch of the triangle product), and rows as they are beat padded ones at every size
+# and width measured (us per block, padded / as they are: c_z = 128 at 363 tokens 780 / 715, 501 1319 / 1226,
+# 1021 5748 / 5521; c_z = 64 at 501 932 / 862; c_z = 256 at 501 3522 / 3406; fp32 at 403 3619 / 3396).
 # Masked tokens take no part in either triangle update and every other operation on the pair tensor
 # is local to a pair, so the N x N corner of the result is what the unpadded tensor gives; the single
 # representation is not padded (its attention has no mask), it reads the corner of the pair bias.
@@ -36,8 +35,7 @@ from .triangular import (TriangleAttention, TriangleMultiplicationIncoming,
 # are all masked, the reference gives such a row the mean of V over all N keys, and with more keys
 # that mean would be another.
 pad_tokens_to = 8
-pad_tokens_min_n = 320
-pad_tokens_end_n = 328
+pad_tokens_min_n = 1 << 30
 
 
 class _Padded:
@@ -65,7 +63,7 @@ class _Padded:
 
 def _wants_padding(z: torch.Tensor, pair_mask: Optional[torch.Tensor]) -> bool:
     return (pad_tokens_to > 1 and z.is_cuda and z.dim() >= 3 and z.shape[-2] == z.shape[-3]
-            and z.shape[-2] % pad_tokens_to != 0 and pad_tokens_min_n <= z.shape[-2] < pad_tokens_end_n
+            and z.shape[-2] % pad_tokens_to != 0 and pad_tokens_min_n <= z.shape[-2]
             and (pair_mask is None or (pair_mask.is_cuda and ops.mask_class(pair_mask)[0])))
 
 
