@@ -198,59 +198,129 @@ constexpr float kEps = 1e-5f;
 // first, so that a block's single track runs underneath the next block's pair kernels without launches,
 // streams or waits of its own.
 struct Stages {
-  std::vector<ptx_single_stage> list;
+  struct Named {
+    ptx_single_stage stage;
+    const char* name;
+  };
+  std::vector<Named> list;
   size_t next = 0;
-  const ptx_single_stage* take() { return next < list.size() ? &list[next++] : nullptr; }
-  ptx_single_stage* add() {
-    list.emplace_back();
-    return &list.back();
+  const ptx_single_stage* take() { return next < list.size() ? &list[next++].stage : nullptr; }
+  ptx_single_stage* add(const char* name) {
+    list.push_back(Named{{}, name});
+    return &list.back().stage;
   }
-  void run_rest(hipStream_t st) {
-    while (const ptx_single_stage* s = take()) check(ptx_single_stage_run(s, st), "single_stage");
+  void clear() {
     list.clear();
     next = 0;
   }
 };
 
+// A point on a stream, for timing.
+struct Mark {
+  hipEvent_t e = nullptr;
+  explicit Mark(hipStream_t st) {
+    if (hipEventCreate(&e) != hipSuccess || hipEventRecord(e, st) != hipSuccess) throw std::runtime_error("cannot record an event");
+  }
+  Mark(const Mark&) = delete;
+  ~Mark() { (void)hipEventDestroy(e); }
+  float elapsed_time(const Mark& end) const {
+    float ms = 0;
+    if (hipEventElapsedTime(&ms, e, end.e) != hipSuccess) throw std::runtime_error("hipEventElapsedTime failed (synchronize first)");
+    return ms;
+  }
+};
+
+// One call: its stream, the single-track stages that wait for a launch to ride on, and what the caller
+// wants to look at (ops.py): every launch bracketed by events, and workspaces filled with NaN first.
+struct Run {
+  hipStream_t st;
+  Stages singles;
+  bool poison = false, timing = false;
+  struct Span {
+    const char* name;
+    std::shared_ptr<Mark> begin, end;
+  };
+  std::vector<Span> spans;
+
+  template <typename F> void launch(const char* name, F&& f) {
+    if (!timing) return check(f(), name);
+    Span s{name, std::make_shared<Mark>(st), nullptr};
+    check(f(), name);
+    s.end = std::make_shared<Mark>(st);
+    spans.push_back(std::move(s));
+  }
+  void run_rest() {
+    while (singles.next < singles.list.size()) {
+      const char* name = singles.list[singles.next].name;
+      const ptx_single_stage* s = singles.take();
+      launch(name, [&] { return ptx_single_stage_run(s, st); });
+    }
+    singles.clear();
+  }
+  // (0xff bytes are NaNs in every type)
+  Tensor workspace(int64_t bytes, const at::TensorOptions& like) const {
+    Tensor t = at::empty({bytes}, like.dtype(at::kByte));
+    return poison ? t.fill_(255) : t;
+  }
+  // name -> [(begin, end)], appended to the caller's dict; with the interpreter's lock
+  void hand_over(const py::object& timer) const {
+    for (const Span& s : spans)
+      py::reinterpret_borrow<py::dict>(timer).attr("setdefault")(s.name, py::list()).attr("append")(py::make_tuple(s.begin, s.end));
+  }
+};
+
 void run_trimul(const TriMul& w, const void* z, const Tensor& mask, void* out, int n, bool add, int dt, int64_t es, void* ws,
-                Stages& singles, hipStream_t st) {
+                Run& run) {
   Cut c{(char*)ws};
   TriMulWs s(c, n, w.c_h, es);
   const int pitch = ptx_key_pitch(n), ldx = (n + 7) / 8 * 8;
-  check(ptx_trimul_project_packed(z, ptr(mask), ptr(w.ln_in_w), ptr(w.ln_in_b), ptr(w.packed), s.a, s.b, n, w.c_z, w.c_h, pitch,
-                                  w.incoming, kEps, dt, singles.take(), st), "trimul_project");
-  check(ptx_trimul_contract_ld(s.a, s.b, s.x, n, ldx, w.c_h, pitch, dt, st), "trimul_contract");
-  check(ptx_trimul_output_packed(s.x, ldx, z, ptr(w.ln_in_w), ptr(w.ln_in_b), ptr(w.ln_out_w), ptr(w.ln_out_b), ptr(w.packed), out, n,
-                                 w.c_z, w.c_h, add, kEps, dt, singles.take(), st), "trimul_output");
+  run.launch("trimul_project", [&] {
+    return ptx_trimul_project_packed(z, ptr(mask), ptr(w.ln_in_w), ptr(w.ln_in_b), ptr(w.packed), s.a, s.b, n, w.c_z, w.c_h, pitch,
+                                     w.incoming, kEps, dt, run.singles.take(), run.st);
+  });
+  run.launch("trimul_contract", [&] { return ptx_trimul_contract_ld(s.a, s.b, s.x, n, ldx, w.c_h, pitch, dt, run.st); });
+  run.launch("trimul_output", [&] {
+    return ptx_trimul_output_packed(s.x, ldx, z, ptr(w.ln_in_w), ptr(w.ln_in_b), ptr(w.ln_out_w), ptr(w.ln_out_b), ptr(w.packed), out,
+                                    n, w.c_z, w.c_h, add, kEps, dt, run.singles.take(), run.st);
+  });
 }
 
 // projection and core; the attention output is left in ws.g
-TriAttWs run_triatt_core(const TriAtt& w, const void* z, const Mask& mask, int n, int dt, int64_t es, void* ws, Stages& singles,
-                         hipStream_t st) {
+TriAttWs run_triatt_core(const TriAtt& w, const void* z, const Mask& mask, int n, int dt, int64_t es, void* ws, Run& run) {
   Cut c{(char*)ws};
   TriAttWs s(c, n, w.heads, es);
   const int pitch = ptx_key_pitch(n);
   void* gate = ptx_triattn_late_gate(w.c, w.heads, dt) ? nullptr : s.g;
-  check(ptx_triattn_project_packed(z, ptr(w.ln_w), ptr(w.ln_b), ptr(w.packed), s.q, s.k, s.vt, gate, s.tb, n, w.c, w.heads, pitch,
-                                   w.transposed, kEps, dt, singles.take(), st), "triattn_project");
+  run.launch("triattn_project", [&] {
+    return ptx_triattn_project_packed(z, ptr(w.ln_w), ptr(w.ln_b), ptr(w.packed), s.q, s.k, s.vt, gate, s.tb, n, w.c, w.heads, pitch,
+                                      w.transposed, kEps, dt, run.singles.take(), run.st);
+  });
   const void* m = ptr(w.transposed ? mask.mt : mask.m);
   if (m && mask.n_valid >= 0) {
     // padding at the end: valid rows over valid keys without a mask, padded rows with it (ops.py)
-    check(ptx_triattn_fwd_rows(s.q, s.k, s.vt, gate, s.tb, nullptr, s.g, n, w.heads, 32, pitch, 0, w.inf, 0, mask.n_valid,
-                               mask.n_valid, dt, st), "triattn_fwd");
-    check(ptx_triattn_fwd_rows(s.q, s.k, s.vt, gate, s.tb, m, s.g, n, w.heads, 32, pitch, 0, w.inf, mask.n_valid,
-                               n - mask.n_valid, n, dt, st), "triattn_fwd_padded_rows");
+    run.launch("triattn_fwd", [&] {
+      return ptx_triattn_fwd_rows(s.q, s.k, s.vt, gate, s.tb, nullptr, s.g, n, w.heads, 32, pitch, 0, w.inf, 0, mask.n_valid,
+                                  mask.n_valid, dt, run.st);
+    });
+    run.launch("triattn_fwd_padded_rows", [&] {
+      return ptx_triattn_fwd_rows(s.q, s.k, s.vt, gate, s.tb, m, s.g, n, w.heads, 32, pitch, 0, w.inf, mask.n_valid, n - mask.n_valid, n,
+                                  dt, run.st);
+    });
   } else {
-    check(ptx_triattn_fwd(s.q, s.k, s.vt, gate, s.tb, m, s.g, n, w.heads, 32, pitch, 0, w.inf, dt, st), "triattn_fwd");
+    run.launch("triattn_fwd", [&] {
+      return ptx_triattn_fwd(s.q, s.k, s.vt, gate, s.tb, m, s.g, n, w.heads, 32, pitch, 0, w.inf, dt, run.st);
+    });
   }
   return s;
 }
 
 void run_triatt(const TriAtt& w, const void* z, const Mask& mask, void* out, int n, bool add, int dt, int64_t es, void* ws,
-                Stages& singles, hipStream_t st) {
-  const TriAttWs s = run_triatt_core(w, z, mask, n, dt, es, ws, singles, st);
-  check(ptx_triattn_output_packed(s.g, z, ptr(w.ln_w), ptr(w.ln_b), ptr(w.packed), out, n, w.c, w.heads, w.transposed, add, kEps, dt,
-                                  singles.take(), st), "triattn_output");
+                Run& run) {
+  const TriAttWs s = run_triatt_core(w, z, mask, n, dt, es, ws, run);
+  run.launch("triattn_output", [&] {
+    return ptx_triattn_output_packed(s.g, z, ptr(w.ln_w), ptr(w.ln_b), ptr(w.packed), out, n, w.c, w.heads, w.transposed, add, kEps, dt,
+                                     run.singles.take(), run.st);
+  });
 }
 
 // ---- one Pairformer block ----------------------------------------------------------------------
@@ -292,38 +362,41 @@ struct Block {
 
   // The five pair updates of the pair tensors of z [batch][n][n][c_z] in place; the single attention's pair
   // bias (fp32 [batch][heads][n][n]) of the finished z into `bias` (null: none wanted).
-  void pair_track(const Tensor& z, const std::vector<Mask>& masks, int64_t batch, int n, void* ws, float* bias, Stages& singles,
-                  hipStream_t st) const {
+  void pair_track(const Tensor& z, const std::vector<Mask>& masks, int64_t batch, int n, void* ws, float* bias, Run& run) const {
     const int dt = code_of_rows(z.scalar_type(), compute);
     const int64_t es = at::elementSize(compute), plane = (int64_t)n * n * c_z * z.element_size();
     char* zp = (char*)z.data_ptr();
     static const Mask none;
     auto mask = [&](int64_t b) -> const Mask& { return masks.empty() ? none : masks[b]; };
-    for (int64_t b = 0; b < batch; ++b) run_trimul(out, zp + b * plane, mask(b).m, zp + b * plane, n, true, dt, es, ws, singles, st);
-    for (int64_t b = 0; b < batch; ++b) run_trimul(in, zp + b * plane, mask(b).m, zp + b * plane, n, true, dt, es, ws, singles, st);
-    for (int64_t b = 0; b < batch; ++b) run_triatt(start, zp + b * plane, mask(b), zp + b * plane, n, true, dt, es, ws, singles, st);
+    for (int64_t b = 0; b < batch; ++b) run_trimul(out, zp + b * plane, mask(b).m, zp + b * plane, n, true, dt, es, ws, run);
+    for (int64_t b = 0; b < batch; ++b) run_trimul(in, zp + b * plane, mask(b).m, zp + b * plane, n, true, dt, es, ws, run);
+    for (int64_t b = 0; b < batch; ++b) run_triatt(start, zp + b * plane, mask(b), zp + b * plane, n, true, dt, es, ws, run);
     const int64_t bias_plane = (int64_t)heads * n * n;
     if (fused) {
       for (int64_t b = 0; b < batch; ++b) {
         void* zb = zp + b * plane;
-        const TriAttWs s = run_triatt_core(end, zb, mask(b), n, dt, es, ws, singles, st);
-        if (b == 0) singles.run_rest(st);   // (the bias is about to be rewritten)
-        check(ptx_triattn_output_transition_fwd(s.g, zb, ptr(end.ln_w), ptr(end.ln_b), ptr(tr_packed), ptr(tr_ln_w), ptr(tr_ln_b), zb, n,
-                                                c_z, end.heads, end.transposed, n_factor, kEps, kEps, bias ? ptr(pb_ln_w) : nullptr,
-                                                bias ? ptr(pb_ln_b) : nullptr, bias ? ptr(pb_w) : nullptr,
-                                                bias ? bias + b * bias_plane : nullptr, bias ? heads : 0, 1, kEps, dt, st),
-              "triattn_output_transition");
+        const TriAttWs s = run_triatt_core(end, zb, mask(b), n, dt, es, ws, run);
+        if (b == 0) run.run_rest();   // (the bias is about to be rewritten)
+        run.launch("triattn_output_transition", [&] {
+          return ptx_triattn_output_transition_fwd(s.g, zb, ptr(end.ln_w), ptr(end.ln_b), ptr(tr_packed), ptr(tr_ln_w), ptr(tr_ln_b), zb, n,
+                                                   c_z, end.heads, end.transposed, n_factor, kEps, kEps, bias ? ptr(pb_ln_w) : nullptr,
+                                                   bias ? ptr(pb_ln_b) : nullptr, bias ? ptr(pb_w) : nullptr,
+                                                   bias ? bias + b * bias_plane : nullptr, bias ? heads : 0, 1, kEps, dt, run.st);
+        });
       }
       return;
     }
-    for (int64_t b = 0; b < batch; ++b) run_triatt(end, zp + b * plane, mask(b), zp + b * plane, n, true, dt, es, ws, singles, st);
-    singles.run_rest(st);   // (the bias is about to be rewritten)
-    check(ptx_transition_fwd(zp, ptr(tr_ln_w), ptr(tr_ln_b), ptr(tr_packed), zp, batch * n * n, c_z, n_factor, 1, kEps, dt, st),
-          "transition");
+    for (int64_t b = 0; b < batch; ++b) run_triatt(end, zp + b * plane, mask(b), zp + b * plane, n, true, dt, es, ws, run);
+    run.run_rest();   // (the bias is about to be rewritten)
+    run.launch("transition", [&] {
+      return ptx_transition_fwd(zp, ptr(tr_ln_w), ptr(tr_ln_b), ptr(tr_packed), zp, batch * n * n, c_z, n_factor, 1, kEps, dt, run.st);
+    });
     if (bias)
       for (int64_t b = 0; b < batch; ++b)
-        check(ptx_pair_bias_fwd(zp + b * plane, ptr(pb_ln_w), ptr(pb_ln_b), ptr(pb_w), bias + b * bias_plane, n, c_z, heads, 1, kEps, dt, st),
-              "pair_bias");
+        run.launch("pair_bias", [&] {
+          return ptx_pair_bias_fwd(zp + b * plane, ptr(pb_ln_w), ptr(pb_ln_b), ptr(pb_w), bias + b * bias_plane, n, c_z, heads, 1, kEps, dt,
+                                   run.st);
+        });
   }
 
   // bytes single_track() wants as scratch
@@ -354,39 +427,37 @@ struct Block {
     const int64_t es = at::elementSize(type), rows = batch * n;
     Cut c{(char*)ws};
     const SingleWs w(c, *this, batch, n, es);
-    check(ptx_single_layernorm_stage(st.add(), s, ptr(a_ln_w), ptr(a_ln_b), w.y, (int)rows, c_s, (float)a_eps, dt), "layernorm");
+    check(ptx_single_layernorm_stage(st.add("layernorm"), s, ptr(a_ln_w), ptr(a_ln_b), w.y, (int)rows, c_s, (float)a_eps, dt), "layernorm");
     for (int64_t b = 0; b < batch; ++b) {
       char* qkg = w.qkg + b * w.qkg_plane;
-      check(ptx_single_linear_stage(st.add(), w.y + b * n * c_s * es, ptr(w_in), nullptr, ptr(b_q), hd, nullptr, qkg, w.vt + b * w.vt_plane, 3 * hd, ldt, n, c_s, 4 * hd, dt, 1), "linear");
+      check(ptx_single_linear_stage(st.add("linear"), w.y + b * n * c_s * es, ptr(w_in), nullptr, ptr(b_q), hd, nullptr, qkg, w.vt + b * w.vt_plane, 3 * hd, ldt, n, c_s, 4 * hd, dt, 1), "linear");
     }
     for (int64_t b = 0; b < batch; ++b) {
       char* qkg = w.qkg + b * w.qkg_plane;
-      check(ptx_single_attention_stage(st.add(), qkg, qkg + hd * es, w.vt + b * w.vt_plane, qkg + 2 * hd * es,
+      check(ptx_single_attention_stage(st.add("single_attention"), qkg, qkg + hd * es, w.vt + b * w.vt_plane, qkg + 2 * hd * es,
                                        bias + b * heads * (int64_t)n * n, 1, w.o + b * w.o_plane, n, heads, d, 3 * hd, ldt, hd,
                                        (float)(1.0 / std::sqrt((double)d)), dt), "single_attention");
     }
-    check(ptx_single_linear_stage(st.add(), w.o, ptr(w_o), nullptr, nullptr, 0, s, mid, nullptr, c_s, 0,
+    check(ptx_single_linear_stage(st.add("linear"), w.o, ptr(w_o), nullptr, nullptr, 0, s, mid, nullptr, c_s, 0,
                                   (int)rows, hd, c_s, dt, 1), "linear");
-    check(ptx_single_layernorm_stage(st.add(), mid, ptr(s_ln_w), ptr(s_ln_b), w.y, (int)rows, c_s, (float)s_eps, dt), "layernorm");
-    check(ptx_single_linear_stage(st.add(), w.y, ptr(s_wa), ptr(s_wb), nullptr, 0, nullptr,
+    check(ptx_single_layernorm_stage(st.add("layernorm"), mid, ptr(s_ln_w), ptr(s_ln_b), w.y, (int)rows, c_s, (float)s_eps, dt), "layernorm");
+    check(ptx_single_linear_stage(st.add("swiglu"), w.y, ptr(s_wa), ptr(s_wb), nullptr, 0, nullptr,
                                   w.h, nullptr, hidden, 0, (int)rows, c_s, hidden, dt, 1), "swiglu");
-    check(ptx_single_linear_stage(st.add(), w.h, ptr(s_wo), nullptr, nullptr, 0, mid, s_out, nullptr, c_s, 0,
+    check(ptx_single_linear_stage(st.add("linear"), w.h, ptr(s_wo), nullptr, nullptr, 0, mid, s_out, nullptr, c_s, 0,
                                   (int)rows, hidden, c_s, dt, 1), "linear");
   }
 };
 
-// The blocks in sequence on z (contiguous, updated in place).  The single track of a block runs underneath the next
-// block's pair kernels (see Stages).  Returns the new s (undefined for a stack without a single track).
 // Owns the blocks it was given until it returns: the caller's list is shared, and another thread may
 // put a new plan into it while this one runs without the interpreter's lock.
 using Blocks = std::vector<std::shared_ptr<Block>>;
-optional<Tensor> run_blocks(const Blocks& blocks, const optional<Tensor>& s_opt, const Tensor& z, const py::list& mask_list) {
-  const std::vector<Mask> masks = masks_of(mask_list);
-  py::gil_scoped_release nogil;
+
+// The blocks in sequence on z (contiguous, updated in place).  The single track of a block runs underneath the next
+// block's pair kernels (see Stages).  Returns the new s (undefined for a stack without a single track).
+optional<Tensor> run_blocks_on(Run& run, const Blocks& blocks, const optional<Tensor>& s_opt, const Tensor& z,
+                               const std::vector<Mask>& masks) {
   const int n = (int)z.size(-2);
   const int64_t batch = z.numel() / ((int64_t)n * n * z.size(-1));
-  at::DeviceGuard dev(z.device());
-  const hipStream_t st = current_stream(z);
   const bool single = s_opt.has_value() && s_opt->defined() && blocks[0]->c_s > 0;
   const int64_t es = single ? (int64_t)s_opt->element_size() : 0;
   int64_t ws_bytes = 0, single_bytes = 0, bias_elems = 0;
@@ -398,27 +469,41 @@ optional<Tensor> run_blocks(const Blocks& blocks, const optional<Tensor>& s_opt,
       bias_elems = std::max(bias_elems, batch * b->heads * (int64_t)n * n);
     }
   }
-  const auto bytes = z.options().dtype(at::kByte);
-  Tensor ws = at::empty({ws_bytes}, bytes), bias, sws, mid, s_out;
+  Tensor ws = run.workspace(ws_bytes, z.options()), bias, sws, mid, s_out;
   const void* s = nullptr;
   if (single) {
-    bias = at::empty({bias_elems}, z.options().dtype(at::kFloat));
-    sws = at::empty({single_bytes}, bytes);
+    bias = run.workspace(bias_elems * 4, z.options());
+    sws = run.workspace(single_bytes, z.options());
     mid = at::empty_like(*s_opt);
     s_out = at::empty_like(*s_opt);
     s = s_opt->data_ptr();
   }
-  Stages singles;
   for (const auto& b : blocks) {
     float* bp = single ? (float*)bias.data_ptr() : nullptr;
-    b->pair_track(z, masks, batch, n, ws.data_ptr(), bp, singles, st);
+    b->pair_track(z, masks, batch, n, ws.data_ptr(), bp, run);
     if (single) {
-      b->single_track(singles, s, mid.data_ptr(), s_out.data_ptr(), bp, s_opt->scalar_type(), batch, n, sws.data_ptr());
+      b->single_track(run.singles, s, mid.data_ptr(), s_out.data_ptr(), bp, s_opt->scalar_type(), batch, n, sws.data_ptr());
       s = s_out.data_ptr();
     }
   }
-  singles.run_rest(st);
+  run.run_rest();
   return single ? optional<Tensor>(s_out) : s_opt;
+}
+// timer: None, or the dict that gets the launches' times; poison: see Run.
+optional<Tensor> run_blocks(const Blocks& blocks, const optional<Tensor>& s_opt, const Tensor& z, const py::list& mask_list,
+                            const py::object& timer, bool poison) {
+  const std::vector<Mask> masks = masks_of(mask_list);
+  at::DeviceGuard dev(z.device());
+  Run run{current_stream(z)};
+  run.poison = poison;
+  run.timing = !timer.is_none();
+  optional<Tensor> s_out;
+  {
+    py::gil_scoped_release nogil;
+    s_out = run_blocks_on(run, blocks, s_opt, z, masks);
+  }
+  run.hand_over(timer);
+  return s_out;
 }
 
 // ---- single updates ----------------------------------------------------------------------------
@@ -434,24 +519,33 @@ struct Update {
   }
   bool valid() const { return guard->valid(); }
   // out = [z +] update for every pair tensor of z (contiguous); out may be z
-  void run(const Tensor& z, const Tensor& out, const py::list& mask_list, bool add) const {
+  void run(const Tensor& z, const Tensor& out, const py::list& mask_list, bool add, const py::object& timer, bool poison) const {
     const std::vector<Mask> masks = masks_of(mask_list);
-    py::gil_scoped_release nogil;
+    at::DeviceGuard dev(z.device());
+    Run run{current_stream(z)};
+    run.poison = poison;
+    run.timing = !timer.is_none();
+    {
+      py::gil_scoped_release nogil;
+      run_on(run, z, out, masks, add);
+    }
+    run.hand_over(timer);
+  }
+
+ private:
+  void run_on(Run& run, const Tensor& z, const Tensor& out, const std::vector<Mask>& masks, bool add) const {
     const int n = (int)z.size(-2), c = (int)z.size(-1);
     const int64_t batch = n ? z.numel() / ((int64_t)n * n * c) : 0, plane = (int64_t)n * n * c * z.element_size();
-    at::DeviceGuard dev(z.device());
-    const hipStream_t st = current_stream(z);
     const int dt = code_of_rows(z.scalar_type(), compute);
     const int64_t es = at::elementSize(compute);
-    Tensor ws = at::empty({workspace_bytes(n, mul ? mul->c_h : 0, att ? att->heads : 0, es)}, z.options().dtype(at::kByte));
+    Tensor ws = run.workspace(workspace_bytes(n, mul ? mul->c_h : 0, att ? att->heads : 0, es), z.options());
     static const Mask none;
-    Stages no_singles;
     for (int64_t b = 0; b < batch; ++b) {
       const Mask& m = masks.empty() ? none : masks[b];
       const char* zb = (const char*)z.data_ptr() + b * plane;
       char* ob = (char*)out.data_ptr() + b * plane;
-      if (mul) run_trimul(*mul, zb, m.m, ob, n, add, dt, es, ws.data_ptr(), no_singles, st);
-      else run_triatt(*att, zb, m, ob, n, add, dt, es, ws.data_ptr(), no_singles, st);
+      if (mul) run_trimul(*mul, zb, m.m, ob, n, add, dt, es, ws.data_ptr(), run);
+      else run_triatt(*att, zb, m, ob, n, add, dt, es, ws.data_ptr(), run);
     }
   }
 };
@@ -578,13 +672,16 @@ PYBIND11_MODULE(_host, m) {
   py::class_<Update>(m, "Update")
       .def(py::init<std::shared_ptr<Guard>, const py::dict&>())
       .def("valid", &Update::valid)
-      .def("run", &Update::run);
+      .def("run", &Update::run, py::arg("z"), py::arg("out"), py::arg("masks"), py::arg("add"), py::arg("timer") = py::none(),
+           py::arg("poison") = false);
   m.def("first_stale", [](const Blocks& blocks) {
     for (size_t i = 0; i < blocks.size(); ++i)
       if (!blocks[i]->valid()) return (int64_t)i;
     return (int64_t)-1;
   }, "index of the first block whose weights are no longer the module's, or -1");
-  m.def("run_blocks", &run_blocks);
+  m.def("run_blocks", &run_blocks, py::arg("blocks"), py::arg("s"), py::arg("z"), py::arg("masks"), py::arg("timer") = py::none(),
+        py::arg("poison") = false);
+  py::class_<Mark, std::shared_ptr<Mark>>(m, "Mark").def("elapsed_time", &Mark::elapsed_time);
   m.def("layer_norm", &layer_norm);
   m.def("tri_attention", &tri_attention);
 }

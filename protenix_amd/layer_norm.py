@@ -84,7 +84,7 @@ class FusedLayerNorm(nn.Module):
                 f"expected last dimension {self.normalized_shape[0]}, got {tuple(input.shape)}")
         grad = torch.is_grad_enabled() and any(
             t is not None and t.requires_grad for t in (input, self.weight, self.bias))
-        if ops.use_native() and input.is_cuda and input.numel() > 0:
+        if ops.use_native_operators() and input.is_cuda and input.numel() > 0:
             return native.host().layer_norm(input, self.weight, self.bias, self.eps, grad)
         if grad:
             return FusedLayerNormAffineFunction.apply(input, self.weight, self.bias,

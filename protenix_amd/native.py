@@ -221,7 +221,7 @@ def run_blocks(owner, blocks, s: Optional[torch.Tensor], z: torch.Tensor, pair_m
             plans.append(plan)
         _plans[owner][("stack", key)] = ([weakref.ref(b) for b in blocks], plans)
     masks = _masks(z, pair_mask, cd)
-    return host().run_blocks(plans, _aligned(s.contiguous()) if single else s, z, masks)
+    return host().run_blocks(plans, _aligned(s.contiguous()) if single else s, z, masks, ops.kernel_timer, ops.poison_workspaces)
 
 
 def run_update(module, z: torch.Tensor, cd: torch.dtype, mask: Optional[torch.Tensor], out: torch.Tensor, add: bool,
@@ -241,5 +241,5 @@ def run_update(module, z: torch.Tensor, cd: torch.dtype, mask: Optional[torch.Te
         if spec is None or z.shape[-1] != spec.get("c_z", spec.get("c")):
             return False
         plan = plans[key] = host().Update(guard, spec)
-    plan.run(z, out, _masks(z, mask, cd), add)
+    plan.run(z, out, _masks(z, mask, cd), add, ops.kernel_timer, ops.poison_workspaces)
     return True

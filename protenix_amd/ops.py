@@ -44,21 +44,27 @@ def _stream() -> int:
     return torch.cuda.current_stream().cuda_stream
 
 
-# Optional per-kernel timing: while `kernel_timer` is a dict, every C-ABI call
-# is bracketed by HIP events on the stream it is launched on and the pairs are
-# appended under the entry point's name; read them with kernel_times().
+# Optional per-kernel timing: while `kernel_timer` is a dict, every C-ABI call (those of the native host
+# path included) is bracketed by HIP events on the stream it is launched on and the pairs are
+# appended under the entry point's name; read them with kernel_times().  A stage of the single track
+# that rides on a pair kernel is part of that kernel's time and has no entry of its own.
 kernel_timer: Optional[dict] = None
 
 
 # The native host path (native.py): whole stacks, updates and the differentiable operators in one
-# call each.  Off while kernels are timed one by one or one of the switches below that tests throw
-# is thrown; False takes the Python path always (tests compare the two, bit for bit).
+# call each.  False takes the Python path always (tests compare the two, bit for bit).
 native_enabled = True
 
 
 def use_native() -> bool:
-    return (native_enabled and kernel_timer is None and not poison_workspaces and late_gate_enabled
-            and fuse_attention_transition)
+    """Stacks, blocks and updates: not with a switch below thrown that changes which kernels run."""
+    return native_enabled and late_gate_enabled and fuse_attention_transition
+
+
+def use_native_operators() -> bool:
+    """LayerNorm and the attention operator, of one launch or two each: not while kernels are timed or
+    workspaces poisoned, which their Python side does around the same entry points and buffers."""
+    return native_enabled and kernel_timer is None and not poison_workspaces
 
 
 def _call(name: str, fn, *args) -> None:
@@ -179,7 +185,8 @@ def layer_norm_backward(dout: torch.Tensor, x: torch.Tensor, mean: torch.Tensor,
 
 
 # Workspaces are handed to the kernels uninitialised.  With `poison_workspaces` set (tests),
-# they are filled with NaN first: no result may depend on what a workspace held before.
+# they are filled with NaN first, those of the native host path included: no result may depend on what a
+# workspace held before.
 poison_workspaces = False
 
 

@@ -57,7 +57,7 @@ class TriAttentionFunction(torch.autograd.Function):
     @classmethod
     def apply(cls, Q, K, V, Bias1, Bias2, deterministic=False):
         # the same function as a C++ autograd node where nothing is to be refused
-        if (ops.use_native() and Q.is_cuda and Q.dim() == 5 and K.shape == Q.shape and V.shape == Q.shape and Q.numel() > 0
+        if (ops.use_native_operators() and Q.is_cuda and Q.dim() == 5 and K.shape == Q.shape and V.shape == Q.shape and Q.numel() > 0
                 and Q.dtype in (torch.float32, torch.bfloat16) and not (Bias1 is not None and Bias1.requires_grad)):
             return native.host().tri_attention(Q, K, V, Bias1, Bias2)
         return super().apply(Q, K, V, Bias1, Bias2, deterministic)
