@@ -34,7 +34,7 @@
 extern "C" {
 #endif
 
-#define PTX_ABI_VERSION 5
+#define PTX_ABI_VERSION 6
 #define PTX_API __attribute__((visibility("default")))
 
 /*
@@ -120,7 +120,7 @@ PTX_API int ptx_layernorm_fwd(const void* x, const void* gamma, const void* beta
 typedef struct ptx_single_stage {
   int64_t opaque[32];
 } ptx_single_stage;
-PTX_API int64_t ptx_trimul_packed_elems(int c_z, int c_hidden);
+PTX_API int64_t ptx_trimul_packed_elems(int c_z, int c_hidden, int dtype);
 PTX_API int ptx_trimul_pack(const void* w_ap, const void* w_ag, const void* w_bp, const void* w_bg,
                       const void* w_z, const void* w_g, void* packed, int c_z, int c_hidden, int dtype,
                       void* stream);
@@ -135,7 +135,7 @@ PTX_API int ptx_trimul_output_packed(const void* x, int ldx, const void* z, cons
                       const void* packed, void* out, int n, int c_z, int c_hidden, int add_residual,
                       float eps, int dtype,
                       const ptx_single_stage* carry, void* stream);
-PTX_API int64_t ptx_triattn_packed_elems(int c_in, int heads);
+PTX_API int64_t ptx_triattn_packed_elems(int c_in, int heads, int dtype);
 PTX_API int ptx_triattn_late_gate(int c_in, int heads, int dtype);
 PTX_API int ptx_triattn_pack(const void* w_q, const void* w_k, const void* w_v, const void* w_g,
                       const void* w_b, const void* w_o, void* packed, int c_in, int heads, int dtype,

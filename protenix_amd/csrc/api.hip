@@ -391,8 +391,8 @@ PTX_API int ptx_triattn_fwd_rows(const void* q, const void* k, const void* vt, c
 }
 
 // ---- the row-local stages on packed weights (pairproj.hip) ----
-PTX_API int64_t ptx_trimul_packed_elems(int c_z, int c_hidden) {
-  return c_z > 0 && c_hidden > 0 ? ptx::pp_trimul_packed_elems(c_z, c_hidden) : 0;
+PTX_API int64_t ptx_trimul_packed_elems(int c_z, int c_hidden, int dtype) {
+  return c_z > 0 && c_hidden > 0 ? ptx::pp_trimul_packed_elems(c_z, c_hidden, dtype != PTX_F32) : 0;
 }
 
 PTX_API int ptx_trimul_pack(const void* w_ap, const void* w_ag, const void* w_bp, const void* w_bg,
@@ -460,8 +460,8 @@ PTX_API int ptx_trimul_output_packed(const void* x, int ldx, const void* z, cons
   return after_launch("trimul_output_packed");
 }
 
-PTX_API int64_t ptx_triattn_packed_elems(int c_in, int heads) {
-  return c_in > 0 && heads > 0 ? ptx::pp_triattn_packed_elems(c_in, heads) : 0;
+PTX_API int64_t ptx_triattn_packed_elems(int c_in, int heads, int dtype) {
+  return c_in > 0 && heads > 0 ? ptx::pp_triattn_packed_elems(c_in, heads, dtype != PTX_F32) : 0;
 }
 
 PTX_API int ptx_triattn_late_gate(int c_in, int heads, int dtype) {

@@ -122,11 +122,11 @@ int single_stage_run(const SingleStage* s, hipStream_t stream);
 // track on operands of type TZ that this launch's first workgroups run (it must not depend on the launch).
 // Whether the attention's gate is formed by the output stage (no gate tensor exists then).
 inline bool pp_late_gate(int c_z, int heads, bool bits16) { return bits16 && heads == (c_z == 256 ? 8 : 4); }
-int64_t pp_trimul_packed_elems(int c_z, int hidden);
+int64_t pp_trimul_packed_elems(int c_z, int hidden, bool bits16);
 template <typename T>
 int pp_trimul_pack(const void* w_ap, const void* w_ag, const void* w_bp, const void* w_bg, const void* w_z,
                    const void* w_g, void* packed, int c_z, int hidden, hipStream_t stream);
-int64_t pp_triattn_packed_elems(int c_z, int heads);
+int64_t pp_triattn_packed_elems(int c_z, int heads, bool bits16);
 template <typename T>
 int pp_triattn_pack(const void* w_q, const void* w_k, const void* w_v, const void* w_g, const void* w_b,
                     const void* w_o, void* packed, int c_z, int heads, hipStream_t stream);

@@ -624,15 +624,15 @@ __global__ __launch_bounds__(256) void pair_pack_kernel(PackList list, T* __rest
   }
 }
 
-// On rows of 128 channels the packed weights are followed by the matrices as they are, for the kernels of rowgemm.hip
-// and attnout.hip, which keep them in LDS (resident_rows).
+// On rows of 128 channels in 16-bit arithmetic the packed weights are followed by the matrices as they are, for the
+// kernels of rowgemm.hip and attnout.hip, which keep them in LDS (resident_rows): as many bytes again.
 static int64_t trimul_frag_elems(int c_z, int hidden) { return 5 * (int64_t)c_z * hidden + (int64_t)c_z * c_z; }
 static int64_t triattn_frag_elems(int c_z, int heads) { return (int64_t)(4 * heads + 1) * 32 * c_z + (int64_t)c_z * heads * 32; }
-static bool keeps_rows(int c_z, int hidden) { return c_z == 128 && hidden == 128; }
+static bool keeps_rows(int c_z, int hidden, bool bits16) { return bits16 && c_z == 128 && hidden == 128; }
 constexpr int kMat = 128 * 128;   // such a matrix
 
-int64_t pp_trimul_packed_elems(int c_z, int hidden) {
-  return trimul_frag_elems(c_z, hidden) + (keeps_rows(c_z, hidden) ? 6 * kMat : 0);
+int64_t pp_trimul_packed_elems(int c_z, int hidden, bool bits16) {
+  return trimul_frag_elems(c_z, hidden) + (keeps_rows(c_z, hidden, bits16) ? 6 * kMat : 0);
 }
 
 template <typename T>
@@ -641,7 +641,7 @@ int pp_trimul_pack(const void* w_ap, const void* w_ag, const void* w_bp, const v
   PackList l;
   int nt = 0, f = 0;
   const int ks = c_z / 16, sl = hidden / 16, rows0 = (int)trimul_frag_elems(c_z, hidden);
-  auto raw = [&](int i) { return sizeof(T) == 2 && keeps_rows(c_z, hidden) ? rows0 + i * kMat : 0; };
+  auto raw = [&](int i) { return keeps_rows(c_z, hidden, sizeof(T) == 2) ? rows0 + i * kMat : 0; };
   for (int op = 0; op < 2; ++op)
     for (int cb = 0; cb < hidden / 32; ++cb)
       for (int t = 0; t < 2; ++t) {
@@ -657,8 +657,8 @@ int pp_trimul_pack(const void* w_ap, const void* w_ag, const void* w_bp, const v
   return 0;
 }
 
-int64_t pp_triattn_packed_elems(int c_z, int heads) {
-  return triattn_frag_elems(c_z, heads) + (keeps_rows(c_z, heads * 32) ? 5 * kMat + 4 * 128 : 0);
+int64_t pp_triattn_packed_elems(int c_z, int heads, bool bits16) {
+  return triattn_frag_elems(c_z, heads) + (keeps_rows(c_z, heads * 32, bits16) ? 5 * kMat + 4 * 128 : 0);
 }
 
 template <typename T>
@@ -667,7 +667,7 @@ int pp_triattn_pack(const void* w_q, const void* w_k, const void* w_v, const voi
   PackList l;
   int nt = 0, f = 0;
   const int ks = c_z / 16, sl = heads * 2, rows0 = (int)triattn_frag_elems(c_z, heads);
-  auto raw = [&](int i) { return sizeof(T) == 2 && keeps_rows(c_z, heads * 32) ? rows0 + i * kMat : 0; };   // q, k, v, g, o, bias
+  auto raw = [&](int i) { return keeps_rows(c_z, heads * 32, sizeof(T) == 2) ? rows0 + i * kMat : 0; };   // q, k, v, g, o, bias
   // (the gate formed in the output kernel: its rows permuted, see pp_triattn_out_kernel)
   const bool late = pp_late_gate(c_z, heads, sizeof(T) == 2);
   const void* m[4] = {w_q, w_k, w_v, w_g};
@@ -719,7 +719,7 @@ enum RowStage { kTriMulInStage, kTriMulOutStage, kTriAttnInStage, kTriAttnOutSta
 template <typename T, typename TZ>
 static bool resident_rows(RowStage stage, int n, int c_z, int hidden, const SingleStage* carry) {
   constexpr int kFrom[4] = {704, 480, 352, 896};
-  return sizeof(T) == 2 && std::is_same<T, TZ>::value && keeps_rows(c_z, hidden) && n % 8 == 0 && n >= kFrom[stage] &&
+  return std::is_same<T, TZ>::value && keeps_rows(c_z, hidden, sizeof(T) == 2) && n % 8 == 0 && n >= kFrom[stage] &&
          !(carry && carry->kind != kStageNone);
 }
 

@@ -349,7 +349,8 @@ def trimul_pack(w: dict) -> torch.Tensor:
     _dev(w["w_ap"], "w_ap")
     lib = _lib.load()
     c_h, c_z = w["w_ap"].shape
-    packed = torch.empty((lib.ptx_trimul_packed_elems(c_z, c_h),), dtype=w["w_ap"].dtype, device=w["w_ap"].device)
+    packed = torch.empty((lib.ptx_trimul_packed_elems(c_z, c_h, _dt(w["w_ap"])),), dtype=w["w_ap"].dtype,
+                         device=w["w_ap"].device)
     with torch.cuda.device(packed.device):
         _call("trimul_pack", lib.ptx_trimul_pack, *(_ptr(w[k]) for k in ("w_ap", "w_ag", "w_bp", "w_bg", "w_z", "w_g")),
               _ptr(packed), c_z, c_h, _dt(packed), _stream())
@@ -361,7 +362,8 @@ def triattn_pack(w: dict) -> torch.Tensor:
     _dev(w["w_q"], "w_q")
     lib = _lib.load()
     heads, c_in = w["w_b"].shape
-    packed = torch.empty((lib.ptx_triattn_packed_elems(c_in, heads),), dtype=w["w_q"].dtype, device=w["w_q"].device)
+    packed = torch.empty((lib.ptx_triattn_packed_elems(c_in, heads, _dt(w["w_q"])),), dtype=w["w_q"].dtype,
+                         device=w["w_q"].device)
     with torch.cuda.device(packed.device):
         _call("triattn_pack", lib.ptx_triattn_pack, *(_ptr(w[k]) for k in ("w_q", "w_k", "w_v", "w_g", "w_b", "w_o")),
               _ptr(packed), c_in, heads, _dt(packed), _stream())
