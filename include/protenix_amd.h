@@ -150,6 +150,21 @@ PTX_API int ptx_triattn_output_packed(const void* o, const void* z, const void* 
                       const ptx_single_stage* carry, void* stream);
 
 /*
+ * Parameters converted and laid out for the kernels, any number in one launch: dst[rows][cols] = src[rows][cols] in
+ * dst_dtype (PTX_F32 or PTX_BF16, as src_dtype; rounded to nearest even), or with `fragments` in the
+ * order that ptx_single_linear_stage takes as packed weights (rows % 16 == 0, cols % 32 == 0):
+ * [rows / 16][cols / 32][16-byte piece][lane][elements of a piece], lane 16 g + r <-> row r, column
+ * (4 piece + g) * elements per piece + e.  `params` is read before the call returns.
+ */
+typedef struct ptx_param {
+  const void* src;
+  void* dst;
+  int64_t rows;
+  int cols, src_dtype, dst_dtype, fragments;
+} ptx_param;
+PTX_API int ptx_param_pack(const ptx_param* params, int count, void* stream);
+
+/*
  * LayerNorm backward.  Replaces fast_layer_norm_cuda_v2.backward_{none,with_bias,with_weight,
  * with_both}_affine (layer_norm_cuda.cpp:159-178; kernels layer_norm_cuda_kernel.cu:395-760,
  * host :860-990), fp32 arithmetic, with xc = x - mean and gd = gamma * dout:

@@ -390,6 +390,28 @@ PTX_API int ptx_triattn_fwd_rows(const void* q, const void* k, const void* vt, c
                              stream);
 }
 
+// ---- parameters laid out for the kernels (params.hip) ----
+PTX_API int ptx_param_pack(const ptx_param* params, int count, void* stream) {
+  PTX_REQUIRE(count >= 0 && (params || count == 0), PTX_ERR_BAD_ARG, "param_pack: count=%d", count);
+  ptx::Param list[64];
+  for (int i = 0; i < count;) {
+    int m = 0;
+    for (; i < count && m < 64; ++i, ++m) {
+      const ptx_param& p = params[i];
+      PTX_REQUIRE(dtype_ok(p.src_dtype) && dtype_ok(p.dst_dtype), PTX_ERR_BAD_ARG, "param_pack: unknown dtype %d or %d", p.src_dtype,
+                  p.dst_dtype);
+      PTX_REQUIRE(p.rows >= 0 && p.cols >= 0 && p.rows * p.cols <= INT32_MAX, PTX_ERR_BAD_ARG, "param_pack: rows=%lld cols=%d",
+                  (long long)p.rows, p.cols);
+      PTX_REQUIRE((p.src && p.dst) || p.rows * p.cols == 0, PTX_ERR_BAD_ARG, "param_pack: null pointer");
+      PTX_REQUIRE(!p.fragments || (p.rows % 16 == 0 && p.cols % 32 == 0), PTX_ERR_UNSUPPORTED,
+                  "param_pack: fragments need rows %% 16 == 0 and cols %% 32 == 0 (got rows=%lld cols=%d)", (long long)p.rows, p.cols);
+      list[m] = ptx::Param{p.src, p.dst, p.rows, p.cols, p.src_dtype == PTX_BF16, p.dst_dtype == PTX_BF16, p.fragments != 0};
+    }
+    ptx::param_pack(list, m, (hipStream_t)stream);
+  }
+  return after_launch("param_pack");
+}
+
 // ---- the row-local stages on packed weights (pairproj.hip) ----
 PTX_API int64_t ptx_trimul_packed_elems(int c_z, int c_hidden, int dtype) {
   return c_z > 0 && c_hidden > 0 ? ptx::pp_trimul_packed_elems(c_z, c_hidden, dtype != PTX_F32) : 0;

@@ -4,8 +4,8 @@
 // hundred tokens the GPU finishes a block's kernels faster than Python can enqueue them (93 tokens:
 // 390 us of Python per block against about 110 us of kernels).
 //
-// Weights are laid out by Python (the modules' caches) and handed over once as a Plan, with a record of
-// the parameters, sub-modules and hooks they came from: valid() compares identities and version
+// Weights are laid out here, from the modules' parameters, once per weight set (a plan), with a record of the
+// parameters, sub-modules and hooks they came from: valid() compares identities and version
 // counters, so that a parameter that was replaced or changed in place is noticed on the next call.
 // The kernels, their order and their arguments are those of ops.py.
 #include <torch/extension.h>
@@ -43,13 +43,6 @@ void* ptr(const Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; }
 hipStream_t current_stream(const Tensor& t) {
   return c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(t.device().index()).stream();
 }
-
-Tensor take(const py::dict& d, const char* key) {
-  if (!d.contains(key)) return Tensor();
-  py::object o = d[key];
-  return o.is_none() ? Tensor() : o.cast<Tensor>();
-}
-int take_int(const py::dict& d, const char* key) { return d.contains(key) ? d[key].cast<int>() : 0; }
 
 // ---- what a plan's weights were made from ---------------------------------------------------
 // A plan stands in for a tree of modules only while every one of them is of a class it knows and runs that class's
@@ -123,22 +116,187 @@ struct Guard {
   }
 };
 
+// What all plans are.
+struct Plan {
+  std::shared_ptr<const Guard> guard;
+  explicit Plan(std::shared_ptr<const Guard> g) : guard(std::move(g)) {}
+  bool valid() const { return guard->valid(); }
+};
+
+// ---- a plan's weights ----------------------------------------------------------------------
+// A configuration without a native path: the call goes to Python, which has it or the error message.
+struct NotCovered {};
+void require(bool ok) {
+  if (!ok) throw NotCovered{};
+}
+
+// A module as Python holds it: plain attributes, sub-modules and parameters out of its dicts.  (Every class in the tree is
+// one of this package's, see Guard.)
+struct Module {
+  py::dict d;
+  explicit Module(const py::handle& m) : d(m.attr("__dict__")) {}
+  py::object item(const char* name) const {
+    require(d.contains(name));
+    return d[name];
+  }
+  int number(const char* name) const { return item(name).cast<int>(); }
+  double real(const char* name) const { return item(name).cast<double>(); }
+  Module operator[](const char* name) const {
+    const py::dict mods = d["_modules"];
+    require(mods.contains(name) && !mods[name].is_none());
+    return Module(mods[name]);
+  }
+  Tensor parameter(const char* name) const {   // undefined for None
+    const py::dict params = d["_parameters"];
+    require(params.contains(name));
+    const py::object p = params[name];
+    return p.is_none() ? Tensor() : p.cast<Tensor>();
+  }
+  // a linear layer's weight, of the size the kernels will take it for
+  Tensor matrix(int64_t n_out, int64_t n_in) const {
+    const Tensor w = parameter("weight");
+    require(w.defined() && w.dim() == 2 && w.size(0) == n_out && w.size(1) == n_in);
+    return w;
+  }
+  Tensor vector(const char* name, int64_t n) const {
+    const Tensor v = parameter(name);
+    require(!v.defined() || (v.dim() == 1 && v.size(0) == n));
+    return v;
+  }
+};
+
+// Parameters in the type and place the kernels want them: as they are where they qualify (dense, at a multiple of 16 bytes),
+// otherwise converted, all of a plan's in one launch.
+struct Weights {
+  std::vector<Tensor> kept;        // what the pointers handed out point into
+  Weights(at::Device device, hipStream_t stream) : device_(device), st_(stream) {}
+
+  // *out: the parameter in `type` (null for none); valid after settle().  temporary: until done().
+  void want(const void** out, const Tensor& t, at::ScalarType type, bool temporary = false) { add(out, t, type, temporary, false); }
+  // *out: the matrices one below the other, packed for ptx_single_linear_stage
+  void want_fragments(const void** out, std::initializer_list<Tensor> matrices, at::ScalarType type) {
+    for (const Tensor& t : matrices) {
+      add(out, t, type, false, true);
+      out = nullptr;    // (it follows the one before)
+    }
+  }
+  void settle() {
+    int64_t bytes[2] = {0, 0};
+    for (Wanted& w : wanted_) {
+      w.at = bytes[w.temporary];
+      bytes[w.temporary] += w.t.numel() * (int64_t)at::elementSize(w.type);
+      if (!w.fragments) bytes[w.temporary] = (bytes[w.temporary] + 15) / 16 * 16;
+    }
+    const auto options = at::TensorOptions().dtype(at::kByte).device(device_);
+    char* base[2];
+    for (int k = 0; k < 2; ++k) {
+      Tensor buffer = at::empty({bytes[k]}, options);
+      base[k] = (char*)buffer.data_ptr();
+      (k ? temporaries_ : kept).push_back(std::move(buffer));
+    }
+    std::vector<ptx_param> list;
+    for (const Wanted& w : wanted_) {
+      char* dst = base[w.temporary] + w.at;
+      if (w.out) *w.out = dst;
+      const int64_t cols = w.t.dim() == 2 ? w.t.size(1) : w.t.numel();
+      list.push_back(ptx_param{w.t.data_ptr(), dst, cols ? w.t.numel() / cols : 0, (int)cols, code_of(w.t.scalar_type()), code_of(w.type),
+                               w.fragments});
+    }
+    check(ptx_param_pack(list.data(), (int)list.size(), st_), "param_pack");
+    wanted_.clear();
+  }
+  // room for `elems` elements, kept
+  void* room(int64_t elems, at::ScalarType type) {
+    kept.push_back(at::empty({elems}, at::TensorOptions().dtype(type).device(device_)));
+    return kept.back().data_ptr();
+  }
+  hipStream_t stream() const { return st_; }
+  void done() { temporaries_.clear(); }   // (their memory is used again behind the launches on this stream)
+
+ private:
+  struct Wanted {
+    Tensor t;
+    const void** out;
+    at::ScalarType type;
+    bool temporary, fragments;
+    int64_t at = 0;
+  };
+  void add(const void** out, const Tensor& p, at::ScalarType type, bool temporary, bool fragments) {
+    if (!p.defined()) {
+      *out = nullptr;
+      return;
+    }
+    Tensor t = p.detach();
+    if (t.device() != device_ || (t.scalar_type() != at::kFloat && t.scalar_type() != at::kBFloat16)) t = t.to(device_, type);
+    t = t.contiguous();
+    if (!fragments && t.scalar_type() == type && ((uintptr_t)t.data_ptr() & 15) == 0) {
+      *out = t.data_ptr();
+      (temporary ? temporaries_ : kept).push_back(std::move(t));
+      return;
+    }
+    wanted_.push_back(Wanted{std::move(t), out, type, temporary, fragments});
+  }
+  at::Device device_;
+  hipStream_t st_;
+  std::vector<Wanted> wanted_;
+  std::vector<Tensor> temporaries_;
+};
+
+// rows of c channels with this hidden width and arithmetic on the packed kernels
+void require_width(int c, int hidden, at::ScalarType compute) {
+  require((compute == at::kFloat || compute == at::kBFloat16) &&
+          (((c == 64 || c == 128) && hidden == 128) || (c == 256 && hidden == 256 && compute == at::kBFloat16)));
+}
+
 struct TriMul {
-  Tensor ln_in_w, ln_in_b, ln_out_w, ln_out_b, packed;
-  int c_z = 0, c_h = 0;
-  bool incoming = false;
-  explicit TriMul(const py::dict& d)
-      : ln_in_w(take(d, "ln_in_w")), ln_in_b(take(d, "ln_in_b")), ln_out_w(take(d, "ln_out_w")), ln_out_b(take(d, "ln_out_b")),
-        packed(take(d, "packed")), c_z(take_int(d, "c_z")), c_h(take_int(d, "c_h")), incoming(take_int(d, "incoming") != 0) {}
+  const void *ln_in_w, *ln_in_b, *ln_out_w, *ln_out_b, *packed = nullptr;
+  int c_z, c_h;
+  bool incoming;
+  const void* w[6];     // while the plan is made
+  TriMul(const Module& m, Weights& ws, at::ScalarType type) : c_z(m.number("c_z")), c_h(m.number("c_hidden")) {
+    require_width(c_z, c_h, type);
+    incoming = !m.item("_outgoing").cast<bool>();
+    const Module in = m["layer_norm_in"], out = m["layer_norm_out"];
+    ws.want(&ln_in_w, in.vector("weight", c_z), type);
+    ws.want(&ln_in_b, in.vector("bias", c_z), type);
+    ws.want(&ln_out_w, out.vector("weight", c_h), type);
+    ws.want(&ln_out_b, out.vector("bias", c_h), type);
+    const char* const names[4] = {"linear_a_p", "linear_a_g", "linear_b_p", "linear_b_g"};
+    for (int i = 0; i < 4; ++i) ws.want(&w[i], m[names[i]].matrix(c_h, c_z), type, true);
+    ws.want(&w[4], m["linear_z"].matrix(c_z, c_h), type, true);
+    ws.want(&w[5], m["linear_g"].matrix(c_z, c_z), type, true);
+  }
+  void pack(Weights& ws, at::ScalarType type) {
+    const int dt = code_of(type);
+    void* p = ws.room(ptx_trimul_packed_elems(c_z, c_h, dt), type);
+    check(ptx_trimul_pack(w[0], w[1], w[2], w[3], w[4], w[5], p, c_z, c_h, dt, ws.stream()), "trimul_pack");
+    packed = p;
+  }
 };
 struct TriAtt {
-  Tensor ln_w, ln_b, packed;
-  int c = 0, heads = 0;
-  float inf = 0;
-  bool transposed = false;
-  explicit TriAtt(const py::dict& d)
-      : ln_w(take(d, "ln_w")), ln_b(take(d, "ln_b")), packed(take(d, "packed")), c(take_int(d, "c")), heads(take_int(d, "heads")),
-        inf((float)d["inf"].cast<double>()), transposed(take_int(d, "transposed") != 0) {}
+  const void *ln_w, *ln_b, *packed = nullptr;
+  int c, heads;
+  float inf;
+  bool transposed;
+  const void* w[6];     // while the plan is made: q, k, v, gate, bias, output
+  TriAtt(const Module& m, Weights& ws, at::ScalarType type, bool transposed_)
+      : c(m.number("c_in")), heads(m.number("no_heads")), inf((float)m.real("inf")), transposed(transposed_) {
+    require(m.number("c_hidden") == 32);
+    require_width(c, heads * 32, type);
+    const Module ln = m["layer_norm"], mha = m["mha"];
+    ws.want(&ln_w, ln.vector("weight", c), type);
+    ws.want(&ln_b, ln.vector("bias", c), type);
+    const char* const names[4] = {"linear_q", "linear_k", "linear_v", "linear_g"};
+    for (int i = 0; i < 4; ++i) ws.want(&w[i], mha[names[i]].matrix(heads * 32, c), type, true);
+    ws.want(&w[4], m["linear"].matrix(heads, c), type, true);
+    ws.want(&w[5], mha["linear_o"].matrix(c, heads * 32), type, true);
+  }
+  void pack(Weights& ws, at::ScalarType type) {
+    const int dt = code_of(type);
+    void* p = ws.room(ptx_triattn_packed_elems(c, heads, dt), type);
+    check(ptx_triattn_pack(w[0], w[1], w[2], w[3], w[4], w[5], p, c, heads, dt, ws.stream()), "triattn_pack");
+    packed = p;
+  }
 };
 struct Mask {   // of one pair tensor: as the triangle multiplications / the starting node read it, transposed, valid tokens
   Tensor m, mt;
@@ -275,12 +433,12 @@ void run_trimul(const TriMul& w, const void* z, const Tensor& mask, void* out, i
   TriMulWs s(c, n, w.c_h, es);
   const int pitch = ptx_key_pitch(n), ldx = (n + 7) / 8 * 8;
   run.launch("trimul_project", [&] {
-    return ptx_trimul_project_packed(z, ptr(mask), ptr(w.ln_in_w), ptr(w.ln_in_b), ptr(w.packed), s.a, s.b, n, w.c_z, w.c_h, pitch,
+    return ptx_trimul_project_packed(z, ptr(mask), w.ln_in_w, w.ln_in_b, w.packed, s.a, s.b, n, w.c_z, w.c_h, pitch,
                                      w.incoming, kEps, dt, run.singles.take(), run.st);
   });
   run.launch("trimul_contract", [&] { return ptx_trimul_contract_ld(s.a, s.b, s.x, n, ldx, w.c_h, pitch, dt, run.st); });
   run.launch("trimul_output", [&] {
-    return ptx_trimul_output_packed(s.x, ldx, z, ptr(w.ln_in_w), ptr(w.ln_in_b), ptr(w.ln_out_w), ptr(w.ln_out_b), ptr(w.packed), out,
+    return ptx_trimul_output_packed(s.x, ldx, z, w.ln_in_w, w.ln_in_b, w.ln_out_w, w.ln_out_b, w.packed, out,
                                     n, w.c_z, w.c_h, add, kEps, dt, run.singles.take(), run.st);
   });
 }
@@ -292,7 +450,7 @@ TriAttWs run_triatt_core(const TriAtt& w, const void* z, const Mask& mask, int n
   const int pitch = ptx_key_pitch(n);
   void* gate = ptx_triattn_late_gate(w.c, w.heads, dt) ? nullptr : s.g;
   run.launch("triattn_project", [&] {
-    return ptx_triattn_project_packed(z, ptr(w.ln_w), ptr(w.ln_b), ptr(w.packed), s.q, s.k, s.vt, gate, s.tb, n, w.c, w.heads, pitch,
+    return ptx_triattn_project_packed(z, w.ln_w, w.ln_b, w.packed, s.q, s.k, s.vt, gate, s.tb, n, w.c, w.heads, pitch,
                                       w.transposed, kEps, dt, run.singles.take(), run.st);
   });
   const void* m = ptr(w.transposed ? mask.mt : mask.m);
@@ -318,47 +476,99 @@ void run_triatt(const TriAtt& w, const void* z, const Mask& mask, void* out, int
                 Run& run) {
   const TriAttWs s = run_triatt_core(w, z, mask, n, dt, es, ws, run);
   run.launch("triattn_output", [&] {
-    return ptx_triattn_output_packed(s.g, z, ptr(w.ln_w), ptr(w.ln_b), ptr(w.packed), out, n, w.c, w.heads, w.transposed, add, kEps, dt,
+    return ptx_triattn_output_packed(s.g, z, w.ln_w, w.ln_b, w.packed, out, n, w.c, w.heads, w.transposed, add, kEps, dt,
                                      run.singles.take(), run.st);
   });
 }
 
 // ---- one Pairformer block ----------------------------------------------------------------------
-struct Block {
+struct Block : Plan {
   struct SingleWs;
+  Weights weights;
+  at::ScalarType compute;
+  int c_z, c_s;
   TriMul out, in;
   TriAtt start, end;
   // pair transition (fused: with the ending node's output stage in front, one launch)
+  int n_factor;
   bool fused;
-  Tensor tr_ln_w, tr_ln_b, tr_packed;
-  int n_factor, c_z, c_s, hidden = 0;
+  const void *tr_ln_w, *tr_ln_b, *tr_packed;
   // single track (matrices packed for ptx_single_linear_stage)
-  Tensor pb_ln_w, pb_ln_b, pb_w, a_ln_w, a_ln_b, w_in, b_q, w_o, s_ln_w, s_ln_b, s_wa, s_wb, s_wo;
-  int heads = 0, d = 0;
+  int heads = 0, d = 0, hidden = 0;
   double a_eps = kEps, s_eps = kEps;
-  at::ScalarType compute;
-  std::shared_ptr<const Guard> guard;
+  const void *pb_ln_w = nullptr, *pb_ln_b = nullptr, *pb_w = nullptr, *a_ln_w, *a_ln_b, *w_in, *b_q, *w_o, *s_ln_w, *s_ln_b, *s_wa, *s_wb,
+      *s_wo;
 
-  Block(std::shared_ptr<const Guard> guard_, const py::dict& d_)
-      : out(d_["tri_mul_out"].cast<py::dict>()), in(d_["tri_mul_in"].cast<py::dict>()), start(d_["tri_att_start"].cast<py::dict>()),
-        end(d_["tri_att_end"].cast<py::dict>()), fused(take_int(d_, "fused") != 0), tr_ln_w(take(d_, "tr_ln_w")),
-        tr_ln_b(take(d_, "tr_ln_b")), tr_packed(take(d_, "tr_packed")), n_factor(take_int(d_, "n_factor")), c_z(take_int(d_, "c_z")),
-        c_s(take_int(d_, "c_s")), guard(std::move(guard_)) {
-    compute = tr_packed.scalar_type();
-    if (c_s) {
-      pb_ln_w = take(d_, "pb_ln_w"); pb_ln_b = take(d_, "pb_ln_b"); pb_w = take(d_, "pb_w");
-      a_ln_w = take(d_, "a_ln_w"); a_ln_b = take(d_, "a_ln_b");
-      w_in = take(d_, "w_in"); b_q = take(d_, "b_q"); w_o = take(d_, "w_o");
-      s_ln_w = take(d_, "s_ln_w"); s_ln_b = take(d_, "s_ln_b");
-      s_wa = take(d_, "s_wa"); s_wb = take(d_, "s_wb"); s_wo = take(d_, "s_wo");
-      heads = take_int(d_, "heads");
-      d = take_int(d_, "d");
-      hidden = take_int(d_, "hidden");
-      a_eps = d_["a_eps"].cast<double>();
-      s_eps = d_["s_eps"].cast<double>();
-    }
+  // `module` on pair tensors like z (compute: their kernels' arithmetic) and single representations of type s_type; throws
+  // NotCovered
+  Block(std::shared_ptr<const Guard> guard_, const Module& m, const Tensor& z, at::ScalarType compute_, optional<at::ScalarType> s_type)
+      : Plan(std::move(guard_)), weights(z.device(), current_stream(z)), compute(compute_), c_z((int)z.size(-1)), c_s(m.number("c_s")),
+        out(m["tri_mul_out"], weights, compute), in(m["tri_mul_in"], weights, compute), start(m["tri_att_start"], weights, compute, false),
+        end(m["tri_att_end"], weights, compute, true) {
+    require(out.c_z == c_z && in.c_z == c_z && start.c == c_z && end.c == c_z);
+    const Module tr = m["pair_transition"], tr_ln = tr["layernorm1"];
+    n_factor = tr.number("n");
+    require(tr.number("c_in") == c_z && n_factor > 0 && n_factor <= 64 && (n_factor * c_z) % 64 == 0);
+    fused = c_z == 128 && end.heads == 4 && compute == at::kBFloat16;
+    weights.want(&tr_ln_w, tr_ln.vector("weight", c_z), compute);
+    weights.want(&tr_ln_b, tr_ln.vector("bias", c_z), compute);
+    const void* w_tr[3];
+    const int n_hidden = n_factor * c_z;
+    weights.want(&w_tr[0], tr["linear_no_bias_a"].matrix(n_hidden, c_z), compute, true);
+    weights.want(&w_tr[1], tr["linear_no_bias_b"].matrix(n_hidden, c_z), compute, true);
+    weights.want(&w_tr[2], tr["linear_no_bias"].matrix(c_z, n_hidden), compute, true);
+    if (c_s > 0) take_single(m, z, s_type);
+    weights.settle();
+    out.pack(weights, compute);
+    in.pack(weights, compute);
+    start.pack(weights, compute);
+    end.pack(weights, compute);
+    const int dt = code_of(compute);
+    void* p = weights.room(fused ? ptx_triattn_output_transition_packed_elems(n_factor) : ptx_transition_packed_elems(c_z, n_factor), compute);
+    if (fused)
+      check(ptx_triattn_output_transition_pack(end.w[3], end.w[5], w_tr[0], w_tr[1], w_tr[2], p, n_factor, dt, weights.stream()), "transition_pack");
+    else
+      check(ptx_transition_pack(w_tr[0], w_tr[1], w_tr[2], p, c_z, n_factor, dt, weights.stream()), "transition_pack");
+    tr_packed = p;
+    weights.done();
   }
-  bool valid() const { return guard->valid(); }
+  // The single track's stages ride on the pair kernels: same storage type, LayerNorm rows of whole vectors, on rows
+  // of 128 or 256 channels; and not on widths that have a fused pair transition (64, 128, 256).
+  void take_single(const Module& m, const Tensor& z, optional<at::ScalarType> s_type) {
+    require(s_type && *s_type == z.scalar_type());
+    const at::ScalarType type = *s_type;
+    const Module apb = m["attention_pair_bias"], att = apb["attention"], st = m["single_transition"], ln_a = apb["layernorm_a"],
+                 ln_z = apb["layernorm_z"], ln_s = st["layernorm1"];
+    heads = att.number("num_heads");
+    d = att.number("c_hidden");
+    hidden = st.number("n") * c_s;
+    const int hd = heads * d;
+    require(c_s % 32 == 0 && c_s * (int64_t)at::elementSize(type) <= 2048 && c_s != 64 && c_s != 128 && c_s != 256 &&
+            (c_z == 128 || c_z == 256) && heads >= 1 && heads <= 32 && apb.number("n_heads") == heads && att.number("c_q") == c_s &&
+            att.number("c_k") == c_s && att.number("c_v") == c_s && st.number("c_in") == c_s && d > 0 && d % 8 == 0 && d <= 32 && hd % 32 == 0 &&
+            hidden > 0);
+    auto matrix = [&](const Module& parent, const char* name, int64_t n_out, int64_t n_in) {
+      const Module l = parent[name];
+      require(l.item("precision").is_none());
+      return l.matrix(n_out, n_in);
+    };
+    weights.want(&pb_ln_w, ln_z.vector("weight", c_z), compute);
+    weights.want(&pb_ln_b, ln_z.vector("bias", c_z), compute);
+    weights.want(&pb_w, apb["linear_nobias_z"].matrix(heads, c_z), compute);
+    weights.want(&a_ln_w, ln_a.vector("weight", c_s), type);
+    weights.want(&a_ln_b, ln_a.vector("bias", c_s), type);
+    weights.want(&s_ln_w, ln_s.vector("weight", c_s), type);
+    weights.want(&s_ln_b, ln_s.vector("bias", c_s), type);
+    weights.want(&b_q, att["linear_q"].vector("bias", hd), type);
+    a_eps = ln_a.real("eps");
+    s_eps = ln_s.real("eps");
+    weights.want_fragments(&w_in, {matrix(att, "linear_q", hd, c_s), matrix(att, "linear_k", hd, c_s), matrix(att, "linear_g", hd, c_s),
+                                   matrix(att, "linear_v", hd, c_s)}, type);
+    weights.want_fragments(&w_o, {matrix(att, "linear_o", c_s, hd)}, type);
+    weights.want_fragments(&s_wa, {matrix(st, "linear_no_bias_a", hidden, c_s)}, type);
+    weights.want_fragments(&s_wb, {matrix(st, "linear_no_bias_b", hidden, c_s)}, type);
+    weights.want_fragments(&s_wo, {matrix(st, "linear_no_bias", c_s, hidden)}, type);
+  }
 
   // The five pair updates of the pair tensors of z [batch][n][n][c_z] in place; the single attention's pair
   // bias (fp32 [batch][heads][n][n]) of the finished z into `bias` (null: none wanted).
@@ -378,9 +588,9 @@ struct Block {
         const TriAttWs s = run_triatt_core(end, zb, mask(b), n, dt, es, ws, run);
         if (b == 0) run.run_rest();   // (the bias is about to be rewritten)
         run.launch("triattn_output_transition", [&] {
-          return ptx_triattn_output_transition_fwd(s.g, zb, ptr(end.ln_w), ptr(end.ln_b), ptr(tr_packed), ptr(tr_ln_w), ptr(tr_ln_b), zb, n,
-                                                   c_z, end.heads, end.transposed, n_factor, kEps, kEps, bias ? ptr(pb_ln_w) : nullptr,
-                                                   bias ? ptr(pb_ln_b) : nullptr, bias ? ptr(pb_w) : nullptr,
+          return ptx_triattn_output_transition_fwd(s.g, zb, end.ln_w, end.ln_b, tr_packed, tr_ln_w, tr_ln_b, zb, n,
+                                                   c_z, end.heads, end.transposed, n_factor, kEps, kEps, bias ? pb_ln_w : nullptr,
+                                                   bias ? pb_ln_b : nullptr, bias ? pb_w : nullptr,
                                                    bias ? bias + b * bias_plane : nullptr, bias ? heads : 0, 1, kEps, dt, run.st);
         });
       }
@@ -389,12 +599,12 @@ struct Block {
     for (int64_t b = 0; b < batch; ++b) run_triatt(end, zp + b * plane, mask(b), zp + b * plane, n, true, dt, es, ws, run);
     run.run_rest();   // (the bias is about to be rewritten)
     run.launch("transition", [&] {
-      return ptx_transition_fwd(zp, ptr(tr_ln_w), ptr(tr_ln_b), ptr(tr_packed), zp, batch * n * n, c_z, n_factor, 1, kEps, dt, run.st);
+      return ptx_transition_fwd(zp, tr_ln_w, tr_ln_b, tr_packed, zp, batch * n * n, c_z, n_factor, 1, kEps, dt, run.st);
     });
     if (bias)
       for (int64_t b = 0; b < batch; ++b)
         run.launch("pair_bias", [&] {
-          return ptx_pair_bias_fwd(zp + b * plane, ptr(pb_ln_w), ptr(pb_ln_b), ptr(pb_w), bias + b * bias_plane, n, c_z, heads, 1, kEps, dt,
+          return ptx_pair_bias_fwd(zp + b * plane, pb_ln_w, pb_ln_b, pb_w, bias + b * bias_plane, n, c_z, heads, 1, kEps, dt,
                                    run.st);
         });
   }
@@ -427,10 +637,10 @@ struct Block {
     const int64_t es = at::elementSize(type), rows = batch * n;
     Cut c{(char*)ws};
     const SingleWs w(c, *this, batch, n, es);
-    check(ptx_single_layernorm_stage(st.add("layernorm"), s, ptr(a_ln_w), ptr(a_ln_b), w.y, (int)rows, c_s, (float)a_eps, dt), "layernorm");
+    check(ptx_single_layernorm_stage(st.add("layernorm"), s, a_ln_w, a_ln_b, w.y, (int)rows, c_s, (float)a_eps, dt), "layernorm");
     for (int64_t b = 0; b < batch; ++b) {
       char* qkg = w.qkg + b * w.qkg_plane;
-      check(ptx_single_linear_stage(st.add("linear"), w.y + b * n * c_s * es, ptr(w_in), nullptr, ptr(b_q), hd, nullptr, qkg, w.vt + b * w.vt_plane, 3 * hd, ldt, n, c_s, 4 * hd, dt, 1), "linear");
+      check(ptx_single_linear_stage(st.add("linear"), w.y + b * n * c_s * es, w_in, nullptr, b_q, hd, nullptr, qkg, w.vt + b * w.vt_plane, 3 * hd, ldt, n, c_s, 4 * hd, dt, 1), "linear");
     }
     for (int64_t b = 0; b < batch; ++b) {
       char* qkg = w.qkg + b * w.qkg_plane;
@@ -438,12 +648,12 @@ struct Block {
                                        bias + b * heads * (int64_t)n * n, 1, w.o + b * w.o_plane, n, heads, d, 3 * hd, ldt, hd,
                                        (float)(1.0 / std::sqrt((double)d)), dt), "single_attention");
     }
-    check(ptx_single_linear_stage(st.add("linear"), w.o, ptr(w_o), nullptr, nullptr, 0, s, mid, nullptr, c_s, 0,
+    check(ptx_single_linear_stage(st.add("linear"), w.o, w_o, nullptr, nullptr, 0, s, mid, nullptr, c_s, 0,
                                   (int)rows, hd, c_s, dt, 1), "linear");
-    check(ptx_single_layernorm_stage(st.add("layernorm"), mid, ptr(s_ln_w), ptr(s_ln_b), w.y, (int)rows, c_s, (float)s_eps, dt), "layernorm");
-    check(ptx_single_linear_stage(st.add("swiglu"), w.y, ptr(s_wa), ptr(s_wb), nullptr, 0, nullptr,
+    check(ptx_single_layernorm_stage(st.add("layernorm"), mid, s_ln_w, s_ln_b, w.y, (int)rows, c_s, (float)s_eps, dt), "layernorm");
+    check(ptx_single_linear_stage(st.add("swiglu"), w.y, s_wa, s_wb, nullptr, 0, nullptr,
                                   w.h, nullptr, hidden, 0, (int)rows, c_s, hidden, dt, 1), "swiglu");
-    check(ptx_single_linear_stage(st.add("linear"), w.h, ptr(s_wo), nullptr, nullptr, 0, mid, s_out, nullptr, c_s, 0,
+    check(ptx_single_linear_stage(st.add("linear"), w.h, s_wo, nullptr, nullptr, 0, mid, s_out, nullptr, c_s, 0,
                                   (int)rows, hidden, c_s, dt, 1), "linear");
   }
 };
@@ -507,17 +717,22 @@ optional<Tensor> run_blocks(const Blocks& blocks, const optional<Tensor>& s_opt,
 }
 
 // ---- single updates ----------------------------------------------------------------------------
-struct Update {
+struct Update : Plan {
+  Weights weights;
+  at::ScalarType compute;
   optional<TriMul> mul;
   optional<TriAtt> att;
-  at::ScalarType compute;
-  std::shared_ptr<const Guard> guard;
-  Update(std::shared_ptr<const Guard> guard_, const py::dict& d) : guard(std::move(guard_)) {
-    if (d.contains("heads")) att.emplace(d);
-    else mul.emplace(d);
-    compute = (att ? att->packed : mul->packed).scalar_type();
+  // transposed: None for a triangle multiplication
+  Update(std::shared_ptr<const Guard> guard_, const Module& m, const Tensor& z, at::ScalarType compute_, optional<bool> transposed)
+      : Plan(std::move(guard_)), weights(z.device(), current_stream(z)), compute(compute_) {
+    if (transposed) att.emplace(m, weights, compute, *transposed);
+    else mul.emplace(m, weights, compute);
+    require((att ? att->c : mul->c_z) == z.size(-1));
+    weights.settle();
+    if (att) att->pack(weights, compute);
+    else mul->pack(weights, compute);
+    weights.done();
   }
-  bool valid() const { return guard->valid(); }
   // out = [z +] update for every pair tensor of z (contiguous); out may be z
   void run(const Tensor& z, const Tensor& out, const py::list& mask_list, bool add, const py::object& timer, bool poison) const {
     const std::vector<Mask> masks = masks_of(mask_list);
@@ -549,6 +764,16 @@ struct Update {
     }
   }
 };
+
+template <typename Plan, typename Kind>
+std::shared_ptr<Plan> make_plan(std::shared_ptr<Guard> guard, const py::object& module, const Tensor& z, at::ScalarType compute, Kind kind) {
+  at::DeviceGuard dev(z.device());
+  try {
+    return std::make_shared<Plan>(std::move(guard), Module(module), z, compute, kind);
+  } catch (const NotCovered&) {
+    return nullptr;
+  }
+}
 
 // ---- LayerNorm ---------------------------------------------------------------------------------
 Tensor same_as(const optional<Tensor>& t, const Tensor& x) {
@@ -666,15 +891,16 @@ PYBIND11_MODULE(_host, m) {
   py::class_<Guard, std::shared_ptr<Guard>>(m, "Guard")
       .def(py::init<const py::object&, const py::list&, const py::set&>(), py::arg("module"), py::arg("attrs"), py::arg("classes"))
       .def("valid", &Guard::valid);
-  py::class_<Block, std::shared_ptr<Block>>(m, "Block")
-      .def(py::init<std::shared_ptr<Guard>, const py::dict&>())
-      .def("valid", &Block::valid);
-  py::class_<Update>(m, "Update")
-      .def(py::init<std::shared_ptr<Guard>, const py::dict&>())
-      .def("valid", &Update::valid)
+  py::class_<Plan, std::shared_ptr<Plan>>(m, "Plan").def(py::init<std::shared_ptr<Guard>>()).def("valid", &Plan::valid);
+  py::class_<Block, Plan, std::shared_ptr<Block>>(m, "Block");
+  m.def("make_block", &make_plan<Block, optional<at::ScalarType>>, py::arg("guard"), py::arg("module"), py::arg("z"), py::arg("compute"),
+        py::arg("s_type"), "a plan of the block `module` for pair tensors like z, or None where the Python path is to be taken");
+  m.def("make_update", &make_plan<Update, optional<bool>>, py::arg("guard"), py::arg("module"), py::arg("z"), py::arg("compute"),
+        py::arg("transposed"), "a plan of one triangle update; transposed: None for a multiplication");
+  py::class_<Update, Plan, std::shared_ptr<Update>>(m, "Update")
       .def("run", &Update::run, py::arg("z"), py::arg("out"), py::arg("masks"), py::arg("add"), py::arg("timer") = py::none(),
            py::arg("poison") = false);
-  m.def("first_stale", [](const Blocks& blocks) {
+  m.def("first_stale", [](const std::vector<std::shared_ptr<Plan>>& blocks) {
     for (size_t i = 0; i < blocks.size(); ++i)
       if (!blocks[i]->valid()) return (int64_t)i;
     return (int64_t)-1;

@@ -118,6 +118,17 @@ void single_stage_attention(SingleStage* s, const void* q, const void* k, const 
                             float scale, bool bits16);
 int single_stage_run(const SingleStage* s, hipStream_t stream);
 
+// A parameter on its way into the kernels (params.hip): src, dst bf16 or fp32 as the flags say, dst [rows][cols] like src or,
+// fragments, in the order of a linear stage's packed weights (rows % 16 == 0, cols % 32 == 0).
+struct Param {
+  const void* src;
+  void* dst;
+  int64_t rows;
+  int cols;
+  bool src_bits16, dst_bits16, fragments;
+};
+int param_pack(const Param* p, int count, hipStream_t stream);
+
 // The row-local stages of the triangle updates on packed weights (pairproj.hip).  carry: null, or a stage of the single
 // track on operands of type TZ that this launch's first workgroups run (it must not depend on the launch).
 // Whether the attention's gate is formed by the output stage (no gate tensor exists then).

@@ -95,78 +95,10 @@ def _masks(z: torch.Tensor, mask: Optional[torch.Tensor], cd: torch.dtype) -> li
     return out
 
 
-def _mul_spec(m, cd, device) -> Optional[dict]:
-    w = m._weights(cd, device)
-    if "packed" not in w:
-        return None
-    return {**{k: w[k] for k in ("ln_in_w", "ln_in_b", "ln_out_w", "ln_out_b", "packed")}, "c_z": m.c_z, "c_h": m.c_hidden,
-            "incoming": int(not m._outgoing)}
-
-
-def _att_spec(a, cd, device, transposed: bool) -> Optional[dict]:
-    w = a._weights(cd, device)
-    if "packed" not in w:
-        return None
-    return {"ln_w": w["ln_w"], "ln_b": w["ln_b"], "packed": w["packed"], "c": a.c_in, "heads": a.no_heads, "inf": float(a.inf),
-            "transposed": int(transposed)}
-
-
-def _fragments(w: torch.Tensor) -> torch.Tensor:
-    """[n_out][k] in the fragment order of ptx_single_linear_stage."""
-    n, k = w.shape
-    v = 16 // w.element_size()
-    return w.view(n // 16, 16, k // 32, 8 // v, 4, v).permute(0, 2, 3, 4, 1, 5).contiguous()
-
-
-def _aligned(t: Optional[torch.Tensor]) -> Optional[torch.Tensor]:
-    """t, or a copy of it where it does not start at a multiple of 16 bytes (a view into a flat buffer): the
-    single track's stages read whole vectors, unlike the stand-alone kernels of the Python path."""
-    return t if t is None or t.data_ptr() % 16 == 0 else t.clone()
-
-
-def _block_spec(blk, z: torch.Tensor, cd: torch.dtype, sd: Optional[torch.dtype]) -> Optional[dict]:
-    from .primitives import _cv
-    dev, c, tr, end = z.device, z.shape[-1], blk.pair_transition, blk.tri_att_end
-    if not (c in (64, 128) or (c == 256 and cd == torch.bfloat16)):
-        return None
-    if not (tr.c_in == c and (tr.n * c) % 64 == 0 and 0 < tr.n <= 64
-            and all(m.c_z == c for m in (blk.tri_mul_out, blk.tri_mul_in))
-            and all(a.c_in == c and a.c_hidden == 32 for a in (blk.tri_att_start, end))):
-        return None
-    spec = {"tri_mul_out": _mul_spec(blk.tri_mul_out, cd, dev), "tri_mul_in": _mul_spec(blk.tri_mul_in, cd, dev),
-            "tri_att_start": _att_spec(blk.tri_att_start, cd, dev, False), "tri_att_end": _att_spec(end, cd, dev, True),
-            "c_z": c, "c_s": blk.c_s, "n_factor": tr.n}
-    if any(v is None for v in spec.values()):
-        return None
-    spec["fused"] = int(ops.fuses_attention_transition(z, end.no_heads, end.c_hidden, tr.n))
-    if spec["fused"]:
-        t = blk._fused_weights(cd, dev)
-    else:
-        t = tr._weights(cd, dev)
-    spec.update(tr_ln_w=t["ln_w"], tr_ln_b=t["ln_b"], tr_packed=t["packed"])
-    if blk.c_s > 0:
-        apb, st = blk.attention_pair_bias, blk.single_transition
-        att, cs = apb.attention, blk.c_s
-        H, d = att.num_heads, att.c_hidden
-        lins = (att.linear_q, att.linear_k, att.linear_v, att.linear_g, att.linear_o, st.linear_no_bias_a, st.linear_no_bias_b,
-                st.linear_no_bias)
-        # (the single track's stages ride on the pair kernels: same storage type, LayerNorm rows of whole vectors)
-        if not (sd == z.dtype and cs % 16 == 0 and cs * z.element_size() <= 2048 and c in (128, 256) and 1 <= apb.n_heads <= 32 and apb.n_heads == H
-                and all(l is not None and l.precision is None for l in lins)
-                and att.c_q == att.c_k == att.c_v == cs == st.c_in and cs % 16 == 0 and cs not in (64, 128, 256)
-                and d % 8 == 0 and d <= 32 and (H * d) % 32 == 0 and cs % 32 == 0):
-            return None
-        pw = apb.pair_bias_weights(z)
-        w_in, b_q = att._fused_in(sd, dev)
-        st_ps = (st.linear_no_bias_a.weight, st.linear_no_bias_b.weight, st.linear_no_bias.weight)
-        s_wa, s_wb, s_wo = st._cache_ab.get(st_ps, sd, dev, lambda: tuple(_cv(p, sd, dev) for p in st_ps))
-        w_o = att._cache_out.get((att.linear_o.weight,), sd, dev, lambda: _cv(att.linear_o.weight, sd, dev))
-        spec.update(pb_ln_w=pw[0], pb_ln_b=pw[1], pb_w=pw[2], a_ln_w=_aligned(_cv(apb.layernorm_a.weight, sd, dev)),
-                    a_ln_b=_aligned(_cv(apb.layernorm_a.bias, sd, dev)), a_eps=float(apb.layernorm_a.eps), w_in=_fragments(w_in), b_q=b_q, w_o=_fragments(w_o),
-                    s_ln_w=_aligned(_cv(st.layernorm1.weight, sd, dev)), s_ln_b=_aligned(_cv(st.layernorm1.bias, sd, dev)),
-                    s_eps=float(st.layernorm1.eps), s_wa=_fragments(s_wa), s_wb=_fragments(s_wb), s_wo=_fragments(s_wo),
-                    heads=H, d=d, hidden=st.n * cs)
-    return spec
+def _aligned(t: torch.Tensor) -> torch.Tensor:
+    """t, or a copy of it where it does not start at a multiple of 16 bytes: the single track's stages read whole
+    vectors, unlike the stand-alone kernels of the Python path."""
+    return t if t.data_ptr() % 16 == 0 else t.clone()
 
 
 def _block_plan(blk, z, cd, sd):
@@ -176,8 +108,7 @@ def _block_plan(blk, z, cd, sd):
     plan = plans.get(key)
     if plan is None or not plan.valid():
         guard = _guard(blk)
-        spec = None if guard is None else _block_spec(blk, z, cd, sd)
-        plan = plans[key] = None if spec is None else host().Block(guard, spec)
+        plan = plans[key] = None if guard is None else host().make_block(guard, blk, z, cd, sd)
     return plan
 
 
@@ -237,9 +168,9 @@ def run_update(module, z: torch.Tensor, cd: torch.dtype, mask: Optional[torch.Te
         guard = _guard(module)
         if guard is None:
             return False
-        spec = _mul_spec(module, cd, z.device) if transposed is None else _att_spec(module, cd, z.device, transposed)
-        if spec is None or z.shape[-1] != spec.get("c_z", spec.get("c")):
+        plan = host().make_update(guard, module, z, cd, transposed)
+        if plan is None:
             return False
-        plan = plans[key] = host().Update(guard, spec)
+        plans[key] = plan
     plan.run(z, out, _masks(z, mask, cd), add, ops.kernel_timer, ops.poison_workspaces)
     return True

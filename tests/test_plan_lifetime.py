@@ -29,13 +29,10 @@ def test_plans_outlive_the_sequence_they_came_in():
     ln = P.FusedLayerNorm(8)
     weight = ln._parameters.pop("weight")
     ln._parameters[Key("weight")] = weight
-    spec = {"packed": torch.zeros(1)}
-    spec = {k: spec for k in ("tri_mul_out", "tri_mul_in")} | {k: spec | {"inf": 1.0} for k in ("tri_att_start", "tri_att_end")}
-    spec["tr_packed"] = torch.zeros(1)
 
-    def block():
-        return native.host().Block(native._guard(ln), spec)
-    kept = block()
+    def plan():
+        return native.host().Plan(native._guard(ln))
+    kept = plan()
 
     class Handed(collections.abc.Sequence):        # nobody else holds what it hands out
         def __len__(self):
@@ -44,7 +41,7 @@ def test_plans_outlive_the_sequence_they_came_in():
         def __getitem__(self, i):
             if i >= 3:
                 raise IndexError
-            return block()
+            return plan()
     held = []
     Key.seen = lambda: held.append(sys.getrefcount(weight))
     try:
