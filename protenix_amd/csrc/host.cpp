@@ -658,63 +658,77 @@ struct Block : Plan {
   }
 };
 
-// Owns the blocks it was given until it returns: the caller's list is shared, and another thread may
+// Owns the blocks it is given until the call ends: the caller's list is shared, and another thread may
 // put a new plan into it while this one runs without the interpreter's lock.
 using Blocks = std::vector<std::shared_ptr<Block>>;
 
-// The blocks in sequence on z (contiguous, updated in place).  The single track of a block runs underneath the next
-// block's pair kernels (see Stages).  Returns the new s (undefined for a stack without a single track).
-optional<Tensor> run_blocks_on(Run& run, const Blocks& blocks, const optional<Tensor>& s_opt, const Tensor& z,
-                               const std::vector<Mask>& masks) {
-  const int n = (int)z.size(-2);
-  const int64_t batch = z.numel() / ((int64_t)n * n * z.size(-1));
-  const bool single = s_opt.has_value() && s_opt->defined() && blocks[0]->c_s > 0;
-  const int64_t es = single ? (int64_t)s_opt->element_size() : 0;
-  int64_t ws_bytes = 0, single_bytes = 0, bias_elems = 0;
-  for (const auto& b : blocks) {
-    ws_bytes = std::max(ws_bytes, workspace_bytes(n, std::max(b->out.c_h, b->in.c_h), std::max(b->start.heads, b->end.heads),
-                                                  at::elementSize(b->compute)));
-    if (single) {
-      single_bytes = std::max(single_bytes, b->single_bytes(batch, n, es));
-      bias_elems = std::max(bias_elems, batch * b->heads * (int64_t)n * n);
-    }
+// Blocks in sequence on z (contiguous, updated in place).  The single track of a block runs underneath the next
+// block's pair kernels (see Stages), the last one's in finish().  The blocks may come in several lots: on new weights
+// a plan is made while the kernels of the blocks before it run.
+struct Call {
+  // timer: None, or the dict that gets the launches' times; poison: see Run.
+  Call(const optional<Tensor>& s, const Tensor& z, const py::list& masks, const py::object& timer, bool poison)
+      : z_(z), s_(s), masks_(masks_of(masks)), timer_(timer), run_{current_stream(z)} {
+    run_.poison = poison;
+    run_.timing = !timer.is_none();
+    n_ = (int)z.size(-2);
+    batch_ = z.numel() / ((int64_t)n_ * n_ * z.size(-1));
   }
-  Tensor ws = run.workspace(ws_bytes, z.options()), bias, sws, mid, s_out;
-  const void* s = nullptr;
-  if (single) {
-    bias = run.workspace(bias_elems * 4, z.options());
-    sws = run.workspace(single_bytes, z.options());
-    mid = at::empty_like(*s_opt);
-    s_out = at::empty_like(*s_opt);
-    s = s_opt->data_ptr();
-  }
-  for (const auto& b : blocks) {
-    float* bp = single ? (float*)bias.data_ptr() : nullptr;
-    b->pair_track(z, masks, batch, n, ws.data_ptr(), bp, run);
-    if (single) {
-      b->single_track(run.singles, s, mid.data_ptr(), s_out.data_ptr(), bp, s_opt->scalar_type(), batch, n, sws.data_ptr());
-      s = s_out.data_ptr();
-    }
-  }
-  run.run_rest();
-  return single ? optional<Tensor>(s_out) : s_opt;
-}
-// timer: None, or the dict that gets the launches' times; poison: see Run.
-optional<Tensor> run_blocks(const Blocks& blocks, const optional<Tensor>& s_opt, const Tensor& z, const py::list& mask_list,
-                            const py::object& timer, bool poison) {
-  const std::vector<Mask> masks = masks_of(mask_list);
-  at::DeviceGuard dev(z.device());
-  Run run{current_stream(z)};
-  run.poison = poison;
-  run.timing = !timer.is_none();
-  optional<Tensor> s_out;
-  {
+  void blocks(const Blocks& list) {
+    held_.insert(held_.end(), list.begin(), list.end());
     py::gil_scoped_release nogil;
-    s_out = run_blocks_on(run, blocks, s_opt, z, masks);
+    at::DeviceGuard dev(z_.device());
+    for (const auto& b : list) make_room(*b);   // (one allocation for all of a stack's)
+    for (const auto& b : list) {
+      make_room(*b);
+      const bool single = b->c_s > 0;
+      float* bias = single ? (float*)bias_.data_ptr() : nullptr;
+      b->pair_track(z_, masks_, batch_, n_, ws_.data_ptr(), bias, run_);
+      if (single) {
+        b->single_track(run_.singles, s_now_, mid_.data_ptr(), s_out_.data_ptr(), bias, s_->scalar_type(), batch_, n_, sws_.data_ptr());
+        s_now_ = s_out_.data_ptr();
+      }
+    }
   }
-  run.hand_over(timer);
-  return s_out;
-}
+  // the new s (what was given, for blocks without a single track)
+  optional<Tensor> finish() {
+    {
+      py::gil_scoped_release nogil;
+      at::DeviceGuard dev(z_.device());
+      run_.run_rest();
+    }
+    run_.hand_over(timer_);
+    return s_out_.defined() ? optional<Tensor>(s_out_) : s_;
+  }
+
+ private:
+  void make_room(const Block& b) {
+    enlarge(ws_, workspace_bytes(n_, std::max(b.out.c_h, b.in.c_h), std::max(b.start.heads, b.end.heads), at::elementSize(b.compute)));
+    if (b.c_s == 0) return;
+    enlarge(bias_, batch_ * b.heads * (int64_t)n_ * n_ * 4);
+    enlarge(sws_, b.single_bytes(batch_, n_, (int64_t)s_->element_size()));
+    if (s_out_.defined()) return;
+    mid_ = at::empty_like(*s_);
+    s_out_ = at::empty_like(*s_);
+    s_now_ = s_->data_ptr();
+  }
+  void enlarge(Tensor& t, int64_t bytes) {
+    if (t.defined() && t.numel() >= bytes) return;
+    if (t.defined()) outgrown_.push_back(t);   // (stages that wait for a launch point into it)
+    t = run_.workspace(bytes, z_.options());
+  }
+  Tensor z_;
+  optional<Tensor> s_;
+  std::vector<Mask> masks_;
+  py::object timer_;
+  Run run_;
+  int n_ = 0;
+  int64_t batch_ = 0;
+  Blocks held_;
+  Tensor ws_, bias_, sws_, mid_, s_out_;
+  std::vector<Tensor> outgrown_;
+  const void* s_now_ = nullptr;
+};
 
 // ---- single updates ----------------------------------------------------------------------------
 struct Update : Plan {
@@ -905,8 +919,11 @@ PYBIND11_MODULE(_host, m) {
       if (!blocks[i]->valid()) return (int64_t)i;
     return (int64_t)-1;
   }, "index of the first block whose weights are no longer the module's, or -1");
-  m.def("run_blocks", &run_blocks, py::arg("blocks"), py::arg("s"), py::arg("z"), py::arg("masks"), py::arg("timer") = py::none(),
-        py::arg("poison") = false);
+  py::class_<Call>(m, "Call")
+      .def(py::init<const optional<Tensor>&, const Tensor&, const py::list&, const py::object&, bool>(), py::arg("s"), py::arg("z"),
+           py::arg("masks"), py::arg("timer") = py::none(), py::arg("poison") = false)
+      .def("blocks", &Call::blocks)
+      .def("finish", &Call::finish);
   py::class_<Mark, std::shared_ptr<Mark>>(m, "Mark").def("elapsed_time", &Mark::elapsed_time);
   m.def("layer_norm", &layer_norm);
   m.def("tri_attention", &tri_attention);

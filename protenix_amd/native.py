@@ -5,7 +5,7 @@ Plans live here, keyed weakly by module: they are built on a module's first call
 (a replaced or modified parameter, a replaced sub-module, another class, a replaced `forward` or a
 registered hook makes a plan stale) and go away with the module.  A plan stands for this package's own
 classes only, each running its own `forward`.  What the native path does not cover is refused here
-(run_blocks returns NotImplemented, run_update False) and runs through the Python path, which has the same kernels
+(run_blocks says how many blocks it ran, run_update returns False) and runs through the Python path, which has the same kernels
 in the same order and all the error messages.
 """
 from __future__ import annotations
@@ -113,46 +113,52 @@ def _block_plan(blk, z, cd, sd):
 
 
 def run_blocks(owner, blocks, s: Optional[torch.Tensor], z: torch.Tensor, pair_mask: Optional[torch.Tensor]):
-    """The blocks on (s, z), z contiguous and updated in place: the new s (None without a single track), or NotImplemented
-    where the Python path is to be taken.  `owner`: the module the list of plans is kept with."""
+    """The blocks on (s, z), z contiguous and updated in place: (the new s - None without a single track -, how many of the
+    blocks were run).  What follows the first block without a plan is left to the caller, as is everything where the
+    count is 0.  `owner`: the module the list of plans is kept with."""
     if not _usable(z) or not z.is_contiguous():
-        return NotImplemented
+        return s, 0
     ac = ops.autocast_compute_dtype(z)
     cd = ops.compute_dtype(z)
     if ac is not None and cd == z.dtype:
-        return NotImplemented
+        return s, 0
     if pair_mask is not None and not (pair_mask.is_cuda and pair_mask.dim() >= 2):
-        return NotImplemented
+        return s, 0
     single = any(b.c_s > 0 for b in blocks)
     sd = None
     if single:
         n = z.shape[-2]
         if s is None or not s.is_cuda or s.dim() < 2 or s.shape[-2] != n or s.numel() // (n * s.shape[-1]) != z.numel() // (
                 n * n * z.shape[-1]) or any(b.c_s != s.shape[-1] for b in blocks):
-            return NotImplemented
+            return s, 0
         sd = s.dtype
-    key = (cd, sd, z.device.index, z.dtype)
-    kept = _plans.setdefault(owner, {}).get(("stack", key))
-    plans = None
-    if kept is not None and len(kept[0]) == len(blocks) and all(a() is b for a, b in zip(kept[0], blocks)):
+    key = ("stack", cd, sd, z.device.index, z.dtype)
+    kept = _plans.setdefault(owner, {}).get(key)
+    if (kept is not None and len(kept[0]) == len(blocks) and all(a() is b for a, b in zip(kept[0], blocks))
+            and host().first_stale(kept[1]) < 0):
         plans = kept[1]
-        stale = host().first_stale(plans)
-        while stale >= 0:
-            plan = _block_plan(blocks[stale], z, cd, sd)
-            if plan is None:
-                return NotImplemented
-            plans[stale] = plan
-            stale = host().first_stale(plans)
+        call = _call(s, z, pair_mask, cd, single)
+        call.blocks(plans)
     else:
-        plans = []
+        # a plan is made while the kernels of the blocks before it run
+        plans, call = [], None
         for b in blocks:
             plan = _block_plan(b, z, cd, sd)
             if plan is None:
-                return NotImplemented
+                break
             plans.append(plan)
-        _plans[owner][("stack", key)] = ([weakref.ref(b) for b in blocks], plans)
-    masks = _masks(z, pair_mask, cd)
-    return host().run_blocks(plans, _aligned(s.contiguous()) if single else s, z, masks, ops.kernel_timer, ops.poison_workspaces)
+            call = call or _call(s, z, pair_mask, cd, single)
+            call.blocks([plan])
+        if call is None:
+            return s, 0
+        if len(plans) == len(blocks):
+            _plans[owner][key] = ([weakref.ref(b) for b in blocks], plans)
+    return call.finish(), len(plans)
+
+
+def _call(s, z, pair_mask, cd, single):
+    return host().Call(_aligned(s.contiguous()) if single else s, z, _masks(z, pair_mask, cd), ops.kernel_timer,
+                       ops.poison_workspaces)
 
 
 def run_update(module, z: torch.Tensor, cd: torch.dtype, mask: Optional[torch.Tensor], out: torch.Tensor, add: bool,

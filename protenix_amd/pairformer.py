@@ -112,8 +112,8 @@ class PairformerBlock(nn.Module):
             return s, pad.result(z if inplace_safe else None)
         if not inplace_safe or not z.is_contiguous():
             z = z.clone(memory_format=torch.contiguous_format)
-        s_new = native.run_blocks(self, (self,), s, z, pair_mask)
-        if s_new is not NotImplemented:
+        s_new, done = native.run_blocks(self, (self,), s, z, pair_mask)
+        if done:
             return s_new, z
         return self._forward_unpadded(s, z, pair_mask, None)
 
@@ -295,9 +295,11 @@ class PairformerStack(nn.Module):
                 f"{triangle_multiplicative}")
         assert triangle_attention in ("torch", "deepspeed", "triattention", "cuequivariance")
         if pad is None and len(self.blocks) > 0:
-            s_new = native.run_blocks(self, tuple(self.blocks), s, z, pair_mask)
-            if s_new is not NotImplemented:
-                return s_new, z
+            s, done = native.run_blocks(self, tuple(self.blocks), s, z, pair_mask)
+            if done:
+                for blk in self.blocks[done:]:
+                    s, z = blk(s, z, pair_mask, inplace_safe=True)
+                return s, z
         ac = ops.autocast_compute_dtype(z)
         if (not own or not z.is_cuda or s is None
                 or any(b.c_s == 0 or not native.runs_own_forward(b.attention_pair_bias) for b in self.blocks)
