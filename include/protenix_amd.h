@@ -116,10 +116,14 @@ PTX_API int ptx_layernorm_fwd(const void* x, const void* gamma, const void* beta
  *   carry: NULL, or a stage of the single-representation track (ptx_single_*_stage, operands of
  *     the pair rows' storage type) that the launch runs along: on workgroups of its own, so it
  *     must not depend on this launch nor this launch on it.
+ *   ptx_row_stage_resident: 1 where the launch, if it carries nothing, takes a kernel that holds all weights
+ *     in LDS and is the faster for it (it cannot carry).  stage: 0 trimul_project, 1 trimul_output,
+ *     2 triattn_project, 3 triattn_output.
  */
 typedef struct ptx_single_stage {
   int64_t opaque[32];
 } ptx_single_stage;
+PTX_API int ptx_row_stage_resident(int stage, int n, int c_z, int c_hidden, int dtype);
 PTX_API int64_t ptx_trimul_packed_elems(int c_z, int c_hidden, int dtype);
 PTX_API int ptx_trimul_pack(const void* w_ap, const void* w_ag, const void* w_bp, const void* w_bg,
                       const void* w_z, const void* w_g, void* packed, int c_z, int c_hidden, int dtype,

@@ -36,6 +36,7 @@ SIGNATURES = {
     "ptx_trimul_project": (_i, [_p] * 10 + [_i, _i, _i, _i, _i, _f, _i, _p]),
     "ptx_trimul_contract": (_i, [_p, _p, _p, _i, _i, _i, _i, _p]),
     "ptx_param_pack": (_i, [_p, _i, _p]),
+    "ptx_row_stage_resident": (_i, [_i, _i, _i, _i, _i]),
     "ptx_trimul_packed_elems": (_l, [_i, _i, _i]),
     "ptx_trimul_pack": (_i, [_p] * 7 + [_i, _i, _i, _p]),
     "ptx_trimul_project_packed": (_i, [_p] * 7 + [_i, _i, _i, _i, _i, _f, _i, _p, _p]),

@@ -417,6 +417,10 @@ PTX_API int64_t ptx_trimul_packed_elems(int c_z, int c_hidden, int dtype) {
   return c_z > 0 && c_hidden > 0 ? ptx::pp_trimul_packed_elems(c_z, c_hidden, dtype != PTX_F32) : 0;
 }
 
+PTX_API int ptx_row_stage_resident(int stage, int n, int c_z, int c_hidden, int dtype) {
+  return stage >= 0 && stage < 4 && ptx::pp_resident((ptx::RowStage)stage, n, c_z, c_hidden, dtype != PTX_F32, dtype == PTX_BF16);
+}
+
 PTX_API int ptx_trimul_pack(const void* w_ap, const void* w_ag, const void* w_bp, const void* w_bg,
                             const void* w_z, const void* w_g, void* packed, int c_z, int c_hidden, int dtype,
                             void* stream) {

@@ -12,6 +12,8 @@
 
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 
+#include <cstring>
+
 #include "../../include/protenix_amd.h"
 
 namespace {
@@ -354,17 +356,19 @@ constexpr float kEps = 1e-5f;
 
 // The stages of the single tracks of earlier blocks, in order: every pair launch that can carry one takes the
 // first, so that a block's single track runs underneath the next block's pair kernels without launches,
-// streams or waits of its own.
+// streams or waits of its own.  A block has seven of each; where one of its projections is faster without (see Run::carry),
+// the two LayerNorms, 5 us each, are launched by themselves.
 struct Stages {
   struct Named {
     ptx_single_stage stage;
     const char* name;
+    bool layernorm;
   };
   std::vector<Named> list;
   size_t next = 0;
   const ptx_single_stage* take() { return next < list.size() ? &list[next++].stage : nullptr; }
   ptx_single_stage* add(const char* name) {
-    list.push_back(Named{{}, name});
+    list.push_back(Named{{}, name, std::strcmp(name, "layernorm") == 0});
     return &list.back().stage;
   }
   void clear() {
@@ -407,12 +411,28 @@ struct Run {
     s.end = std::make_shared<Mark>(st);
     spans.push_back(std::move(s));
   }
+  // What a pair launch carries: the next stage, or none for a projection (stage 0: of the triangle multiplications, 2: of the
+  // attentions) that has a faster kernel for it; on fp32 rows that is one of the two kinds at most, which leaves
+  // five launches for the five other stages, on 16-bit rows it may be both, and stages left over are
+  // launched.  us per block with a single track, always carrying / so: fp32 rows, 512 tokens 1107 / 1092, 640 1814 / 1785, 768
+  // 2615 / 2595, 1024 5090 / 5047, 2048 28073 / 27832; 16-bit rows, 768 2403 / 2339, 1024 4656 / 4517, 1536 12661 / 12403.
+  bool mul_alone = false, att_alone = false;
+  void row_stages(int n, int c_z, int hidden, int dt) {
+    mul_alone = ptx_row_stage_resident(0, n, c_z, hidden, dt);
+    att_alone = ptx_row_stage_resident(2, n, c_z, hidden, dt);
+  }
+  const ptx_single_stage* carry(int stage) {
+    if ((stage == 0 && mul_alone) || (stage == 2 && att_alone)) return nullptr;
+    if ((mul_alone || att_alone) && singles.next < singles.list.size() && singles.list[singles.next].layernorm) run_next();
+    return singles.take();
+  }
+  void run_next() {
+    const char* name = singles.list[singles.next].name;
+    const ptx_single_stage* s = singles.take();
+    launch(name, [&] { return ptx_single_stage_run(s, st); });
+  }
   void run_rest() {
-    while (singles.next < singles.list.size()) {
-      const char* name = singles.list[singles.next].name;
-      const ptx_single_stage* s = singles.take();
-      launch(name, [&] { return ptx_single_stage_run(s, st); });
-    }
+    while (singles.next < singles.list.size()) run_next();
     singles.clear();
   }
   // (0xff bytes are NaNs in every type)
@@ -432,14 +452,16 @@ void run_trimul(const TriMul& w, const void* z, const Tensor& mask, void* out, i
   Cut c{(char*)ws};
   TriMulWs s(c, n, w.c_h, es);
   const int pitch = ptx_key_pitch(n), ldx = (n + 7) / 8 * 8;
+  const ptx_single_stage* carry0 = run.carry(0);
   run.launch("trimul_project", [&] {
     return ptx_trimul_project_packed(z, ptr(mask), w.ln_in_w, w.ln_in_b, w.packed, s.a, s.b, n, w.c_z, w.c_h, pitch,
-                                     w.incoming, kEps, dt, run.singles.take(), run.st);
+                                     w.incoming, kEps, dt, carry0, run.st);
   });
   run.launch("trimul_contract", [&] { return ptx_trimul_contract_ld(s.a, s.b, s.x, n, ldx, w.c_h, pitch, dt, run.st); });
+  const ptx_single_stage* carry1 = run.carry(1);
   run.launch("trimul_output", [&] {
     return ptx_trimul_output_packed(s.x, ldx, z, w.ln_in_w, w.ln_in_b, w.ln_out_w, w.ln_out_b, w.packed, out,
-                                    n, w.c_z, w.c_h, add, kEps, dt, run.singles.take(), run.st);
+                                    n, w.c_z, w.c_h, add, kEps, dt, carry1, run.st);
   });
 }
 
@@ -449,9 +471,10 @@ TriAttWs run_triatt_core(const TriAtt& w, const void* z, const Mask& mask, int n
   TriAttWs s(c, n, w.heads, es);
   const int pitch = ptx_key_pitch(n);
   void* gate = ptx_triattn_late_gate(w.c, w.heads, dt) ? nullptr : s.g;
+  const ptx_single_stage* carry2 = run.carry(2);
   run.launch("triattn_project", [&] {
     return ptx_triattn_project_packed(z, w.ln_w, w.ln_b, w.packed, s.q, s.k, s.vt, gate, s.tb, n, w.c, w.heads, pitch,
-                                      w.transposed, kEps, dt, run.singles.take(), run.st);
+                                      w.transposed, kEps, dt, carry2, run.st);
   });
   const void* m = ptr(w.transposed ? mask.mt : mask.m);
   if (m && mask.n_valid >= 0) {
@@ -475,9 +498,10 @@ TriAttWs run_triatt_core(const TriAtt& w, const void* z, const Mask& mask, int n
 void run_triatt(const TriAtt& w, const void* z, const Mask& mask, void* out, int n, bool add, int dt, int64_t es, void* ws,
                 Run& run) {
   const TriAttWs s = run_triatt_core(w, z, mask, n, dt, es, ws, run);
+  const ptx_single_stage* carry3 = run.carry(3);
   run.launch("triattn_output", [&] {
     return ptx_triattn_output_packed(s.g, z, w.ln_w, w.ln_b, w.packed, out, n, w.c, w.heads, w.transposed, add, kEps, dt,
-                                     run.singles.take(), run.st);
+                                     carry3, run.st);
   });
 }
 
@@ -683,6 +707,7 @@ struct Call {
       make_room(*b);
       const bool single = b->c_s > 0;
       float* bias = single ? (float*)bias_.data_ptr() : nullptr;
+      run_.row_stages(n_, b->c_z, b->out.c_h, code_of_rows(z_.scalar_type(), b->compute));
       b->pair_track(z_, masks_, batch_, n_, ws_.data_ptr(), bias, run_);
       if (single) {
         b->single_track(run_.singles, s_now_, mid_.data_ptr(), s_out_.data_ptr(), bias, s_->scalar_type(), batch_, n_, sws_.data_ptr());

@@ -133,6 +133,9 @@ int param_pack(const Param* p, int count, hipStream_t stream);
 // track on operands of type TZ that this launch's first workgroups run (it must not depend on the launch).
 // Whether the attention's gate is formed by the output stage (no gate tensor exists then).
 inline bool pp_late_gate(int c_z, int heads, bool bits16) { return bits16 && heads == (c_z == 256 ? 8 : 4); }
+// Whether such a stage, with nothing to carry, takes the kernel that holds all of its weights in LDS.
+enum RowStage { kTriMulInStage, kTriMulOutStage, kTriAttnInStage, kTriAttnOutStage };
+bool pp_resident(RowStage stage, int n, int c_z, int hidden, bool bits16, bool rows16);
 int64_t pp_trimul_packed_elems(int c_z, int hidden, bool bits16);
 template <typename T>
 int pp_trimul_pack(const void* w_ap, const void* w_ag, const void* w_bp, const void* w_bg, const void* w_z,

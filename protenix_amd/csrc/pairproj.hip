@@ -11,15 +11,15 @@
 // the 120 us that the pair tensor's own bytes take.  Read from row-major weights, a fragment touches 32
 // cache lines per load instruction and costs the first-level cache four times as much.)
 // Short workgroups, three or four of them per compute unit at different points of their lives,
-// take the place of the resident kernels of rowgemm.hip (which still serve callers that hand in
-// row-major weights): those hold 128 KB of weights per compute unit and two waves per SIMD, need eight row
-// tiles per compute unit to have something for every wave, and end in a partial round of tiles.
+// take the place of the resident kernels of rowgemm.hip: those hold 128 KB of weights per compute unit
+// and two waves per SIMD, need eight row tiles per compute unit to have something for every wave, and end
+// in a partial round of tiles.  They serve callers that hand in row-major weights and, out of the packed
+// buffer, the large calls named at pp_resident().
 #include "common.h"
 #include "kernels.h"
 #include "rowpieces.h"
 #include "single_stage.h"
 #include <algorithm>
-#include <type_traits>
 
 namespace ptx {
 
@@ -708,19 +708,25 @@ static int out_row_blocks(int64_t rows, int ks, bool attention) {
   return ks == 8 && rows >= (attention ? 320 * 320 : 448 * 448) ? 2 : 1;
 }
 
-// Large calls on 16-bit rows of 128 channels take the kernels that keep all of the weights in LDS, one workgroup per
-// compute unit (rowgemm.hip, attnout.hip): there the rows are half as long and the weights, which every tile here
-// fetches from the L2, weigh twice as much against them.  Only where 8 divides n (their 16-byte accesses) and no stage of
-// the single track rides along.  us per launch, here / resident: trimul_in 640 tokens 94 / 100, 768 132 / 127, 1024 264 / 219,
-// 1536 523 / 478; trimul_out 448 44.1 / 43.5, 512 55 / 52, 768 121 / 113, 1536 465 / 426; triattn_in 256 21.5 / 23.2, 384
-// 34.8 / 33.6, 512 74 / 62, 768 162 / 149, 1536 632 / 592; triattn_out 640 75 / 78, 768 106 / 106, 1024 186 / 182, 1536 415 / 399.
-// (fp32 rows: 768 tokens 139 / 166, 143 / 164, 164 / 172, 133 / 152.)
-enum RowStage { kTriMulInStage, kTriMulOutStage, kTriAttnInStage, kTriAttnOutStage };
+// Large calls on rows of 128 channels in 16-bit arithmetic take the kernels that keep all of the weights in LDS, one
+// workgroup per compute unit (rowgemm.hip, attnout.hip), where those are faster: there the weights, which every tile here
+// fetches from the L2, weigh as much as the rows. Only where 8 divides n (their 16-byte accesses) and no stage of the
+// single track rides along.  us per launch, here / resident.  16-bit rows: trimul_in 640 tokens 94 / 100, 768 132 / 127, 1024
+// 264 / 219, 1536 523 / 478; trimul_out 448 44.1 / 43.5, 512 55 / 52, 768 121 / 113, 1536 465 / 426; triattn_in 256 21.5 / 23.2,
+// 384 34.8 / 33.6, 512 74 / 62, 768 162 / 149, 1536 632 / 592; triattn_out 640 75 / 78, 768 106 / 106, 1024 186 / 182, 1536
+// 415 / 399.
+// fp32 rows (within a stack): triattn_in 448 62 / 62, 512 86 / 78, 640 125 / 112, 768 182 / 167, 1024 324 / 299, 1536 722 / 694,
+// 2048 1243 / 1262; trimul_in 1024 272 / 271, 1536 571 / 594, 2048 1183 / 1066 (1984 and 2304: the same block either way);
+// trimul_out and triattn_out are faster here at every size (768: 151 / 154, 132 / 145).
+bool pp_resident(RowStage stage, int n, int c_z, int hidden, bool bits16, bool rows16) {
+  constexpr int kFrom16[4] = {704, 480, 352, 896};
+  if (!keeps_rows(c_z, hidden, bits16) || n % 8 != 0) return false;
+  if (rows16) return n >= kFrom16[stage];
+  return stage == kTriAttnInStage ? n >= 480 && n < 1792 : stage == kTriMulInStage && n >= 2048;
+}
 template <typename T, typename TZ>
 static bool resident_rows(RowStage stage, int n, int c_z, int hidden, const SingleStage* carry) {
-  constexpr int kFrom[4] = {704, 480, 352, 896};
-  return std::is_same<T, TZ>::value && keeps_rows(c_z, hidden, sizeof(T) == 2) && n % 8 == 0 && n >= kFrom[stage] &&
-         !(carry && carry->kind != kStageNone);
+  return pp_resident(stage, n, c_z, hidden, sizeof(T) == 2, sizeof(TZ) == 2) && !(carry && carry->kind != kStageNone);
 }
 
 template <typename T, typename TZ, int KS>
