@@ -13,6 +13,8 @@
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 
 #include <cstring>
+#include <mutex>
+#include <set>
 
 #include "../../include/protenix_amd.h"
 
@@ -118,11 +120,60 @@ struct Guard {
   }
 };
 
-// What all plans are.
+// A point on a stream, to be waited for or timed.
+struct Mark {
+  hipEvent_t e = nullptr;
+  explicit Mark(hipStream_t st, unsigned flags = hipEventDefault) {
+    if (hipEventCreateWithFlags(&e, flags) != hipSuccess || hipEventRecord(e, st) != hipSuccess) throw std::runtime_error("cannot record an event");
+  }
+  Mark(const Mark&) = delete;
+  ~Mark() { (void)hipEventDestroy(e); }
+  float elapsed_time(const Mark& end) const {
+    float ms = 0;
+    if (hipEventElapsedTime(&ms, e, end.e) != hipSuccess) throw std::runtime_error("hipEventElapsedTime failed (synchronize first)");
+    return ms;
+  }
+};
+
+bool capturing(hipStream_t stream) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  return hipStreamIsCapturing(stream, &status) != hipSuccess || status != hipStreamCaptureStatusNone;
+}
+
+// What all plans are.  Weights are laid out on the stream of the call that made the plan; a call on another stream waits for
+// them once, and they are not handed out again while that stream may still read them.
 struct Plan {
   std::shared_ptr<const Guard> guard;
   explicit Plan(std::shared_ptr<const Guard> g) : guard(std::move(g)) {}
+  Plan(const Plan&) = delete;
+  virtual ~Plan() = default;
   bool valid() const { return guard->valid(); }
+  // before this plan's launches on `st` (not while a graph is recorded, which takes no waits from outside: the recording's
+  // owner has synchronised)
+  void used_on(const c10::Stream& st, hipStream_t stream) const {
+    if (!ready_ || stream == made_on_) return;
+    const std::lock_guard<std::mutex> lock(mutex_);
+    if (others_.count(stream) || capturing(stream)) return;
+    others_.insert(stream);
+    if (hipStreamWaitEvent(stream, ready_->e, 0) != hipSuccess) throw std::runtime_error("hipStreamWaitEvent failed");
+    for (const Tensor& t : *weights_) t.record_stream(st);
+  }
+
+ protected:
+  // all weights have been laid out, on `stream`
+  void made(hipStream_t stream, const std::vector<Tensor>& weights) {
+    if (capturing(stream)) return;   // (part of the recording)
+    made_on_ = stream;
+    weights_ = &weights;
+    ready_ = std::make_unique<Mark>(stream, hipEventDisableTiming);
+  }
+
+ private:
+  std::unique_ptr<Mark> ready_;
+  hipStream_t made_on_ = nullptr;
+  const std::vector<Tensor>* weights_ = nullptr;
+  mutable std::mutex mutex_;
+  mutable std::set<hipStream_t> others_;
 };
 
 // ---- a plan's weights ----------------------------------------------------------------------
@@ -377,24 +428,10 @@ struct Stages {
   }
 };
 
-// A point on a stream, for timing.
-struct Mark {
-  hipEvent_t e = nullptr;
-  explicit Mark(hipStream_t st) {
-    if (hipEventCreate(&e) != hipSuccess || hipEventRecord(e, st) != hipSuccess) throw std::runtime_error("cannot record an event");
-  }
-  Mark(const Mark&) = delete;
-  ~Mark() { (void)hipEventDestroy(e); }
-  float elapsed_time(const Mark& end) const {
-    float ms = 0;
-    if (hipEventElapsedTime(&ms, e, end.e) != hipSuccess) throw std::runtime_error("hipEventElapsedTime failed (synchronize first)");
-    return ms;
-  }
-};
-
 // One call: its stream, the single-track stages that wait for a launch to ride on, and what the caller
 // wants to look at (ops.py): every launch bracketed by events, and workspaces filled with NaN first.
 struct Run {
+  c10::Stream stream;
   hipStream_t st;
   Stages singles;
   bool poison = false, timing = false;
@@ -403,6 +440,9 @@ struct Run {
     std::shared_ptr<Mark> begin, end;
   };
   std::vector<Span> spans;
+
+  explicit Run(const Tensor& z)
+      : stream(c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(z.device().index()).unwrap()), st(current_stream(z)) {}
 
   template <typename F> void launch(const char* name, F&& f) {
     if (!timing) return check(f(), name);
@@ -555,6 +595,7 @@ struct Block : Plan {
       check(ptx_transition_pack(w_tr[0], w_tr[1], w_tr[2], p, c_z, n_factor, dt, weights.stream()), "transition_pack");
     tr_packed = p;
     weights.done();
+    made(weights.stream(), weights.kept);
   }
   // The single track's stages ride on the pair kernels: same storage type, LayerNorm rows of whole vectors, on rows
   // of 128 or 256 channels; and not on widths that have a fused pair transition (64, 128, 256).
@@ -692,7 +733,7 @@ using Blocks = std::vector<std::shared_ptr<Block>>;
 struct Call {
   // timer: None, or the dict that gets the launches' times; poison: see Run.
   Call(const optional<Tensor>& s, const Tensor& z, const py::list& masks, const py::object& timer, bool poison)
-      : z_(z), s_(s), masks_(masks_of(masks)), timer_(timer), run_{current_stream(z)} {
+      : z_(z), s_(s), masks_(masks_of(masks)), timer_(timer), run_(z) {
     run_.poison = poison;
     run_.timing = !timer.is_none();
     n_ = (int)z.size(-2);
@@ -702,7 +743,10 @@ struct Call {
     held_.insert(held_.end(), list.begin(), list.end());
     py::gil_scoped_release nogil;
     at::DeviceGuard dev(z_.device());
-    for (const auto& b : list) make_room(*b);   // (one allocation for all of a stack's)
+    for (const auto& b : list) {
+      make_room(*b);   // (one allocation for all of a stack's)
+      b->used_on(run_.stream, run_.st);
+    }
     for (const auto& b : list) {
       make_room(*b);
       const bool single = b->c_s > 0;
@@ -771,16 +815,18 @@ struct Update : Plan {
     if (att) att->pack(weights, compute);
     else mul->pack(weights, compute);
     weights.done();
+    made(weights.stream(), weights.kept);
   }
   // out = [z +] update for every pair tensor of z (contiguous); out may be z
   void run(const Tensor& z, const Tensor& out, const py::list& mask_list, bool add, const py::object& timer, bool poison) const {
     const std::vector<Mask> masks = masks_of(mask_list);
     at::DeviceGuard dev(z.device());
-    Run run{current_stream(z)};
+    Run run(z);
     run.poison = poison;
     run.timing = !timer.is_none();
     {
       py::gil_scoped_release nogil;
+      used_on(run.stream, run.st);
       run_on(run, z, out, masks, add);
     }
     run.hand_over(timer);

@@ -79,3 +79,32 @@ def test_a_stack_called_by_two_threads_while_its_parameters_change():
     for t in ts:
         t.join()
     assert not wrong
+
+
+@pytest.mark.gpu
+def test_a_plan_made_on_one_stream_and_used_on_another():
+    """The weights are still to be laid out when the second stream's call is issued, and the plan goes away while
+    that call may still read them."""
+    _, prod = oracle_and_product(O.PairformerStack, P.PairformerStack, n_blocks=3)
+    s, z, pm = (t.cuda() for t in O.make_inputs(40, n_pad=3))
+    mul = prod.blocks[0].tri_mul_out
+    with torch.no_grad():
+        s0, z0 = prod(s, z, pm)
+        u0 = mul(z, pm)
+    a, b = torch.cuda.Stream(), torch.cuda.Stream()
+    for _ in range(3):
+        native._plans.clear()
+        torch.cuda.synchronize()
+        with torch.no_grad():
+            with torch.cuda.stream(a):
+                torch.cuda._sleep(20_000_000)       # (some 10 ms, then the weights)
+                prod(s, z, pm)
+                mul(z, pm)
+            with torch.cuda.stream(b):
+                s1, z1 = prod(s, z, pm)
+                u1 = mul(z, pm)
+                native._plans.clear()               # (the weights' memory goes back)
+            with torch.cuda.stream(a):
+                torch.full((4_000_000,), float("nan"), device="cuda")
+        torch.cuda.synchronize()
+        assert bool(torch.equal(s1, s0)) and bool(torch.equal(z1, z0)) and bool(torch.equal(u1, u0))
