@@ -380,7 +380,7 @@ rowgemm_in_kernel(RowGemmInParams p) {
       const int i = min(pi0 + 4 * rb + (n >> 3), p.n - 1), k = min(pk0 + (n & 7), p.n - 1);
       off[rb] = (int64_t)i * p.xmap.stride_outer + (int64_t)k * p.xmap.stride_inner;
     }
-    load_rows_at<T, RB, true>(xf, (const TZ*)p.x, off, gamma, beta, p.eps, lane);
+    load_rows_at<T, RB, true, KS, T, true, TZ, sizeof(TZ) == 2>(xf, (const TZ*)p.x, off, gamma, beta, p.eps, lane);
   } else if constexpr (kRegRes) {
     // (the fp32 rows are requested further down, once the triangle product's rows are on
     // their way through the staging tile: both sets of raw rows at once do not fit the

@@ -60,7 +60,16 @@ template <typename T> __device__ __forceinline__ const T* default_beta() {
 template <typename TZ> __device__ __forceinline__ int row_sum_chain(int kk, int t) {
   return sizeof(TZ) == 4 ? (kk & 1) * 2 + (t >> 2) : kk & 3;
 }
-template <typename TZ> __device__ __forceinline__ float row_sum4(const float (&s)[4]) {
+// VIA_LDS (16-bit rows): the halves met through ds_bpermute, the same sums.  For trimul_project, whose LDS pipe has room: on the
+// incoming product's rows at 768 tokens 132.6 us with permlane swaps, 129.1 so; the transition takes 390.4 / 392.5.
+template <typename TZ, bool VIA_LDS = false> __device__ __forceinline__ float row_sum4(const float (&s)[4]) {
+  if constexpr (VIA_LDS) {
+    static_assert(sizeof(TZ) == 2, "16-bit rows");
+    float w[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) w[c] = s[c] + swap32(s[c]);
+    return (w[0] + w[1]) + (w[2] + w[3]);
+  }
   auto halves = [](float a, float b) {   // lower half-wave: a.lower + a.upper; upper: b.lower + b.upper
     const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b),
                                                     false, false);
@@ -78,7 +87,7 @@ template <typename TZ> __device__ __forceinline__ float row_sum4(const float (&s
 // gamma / beta are read as type P: T from global memory (null: the stand-ins above), or float
 // from a copy the caller keeps in LDS (P = float, DEFAULTS = false: never null).
 // TZ: the type the row is stored in (it decides how the sums associate).
-template <typename T, typename TZ, int KS, typename P = T, bool DEFAULTS = true>
+template <typename T, typename TZ, int KS, typename P = T, bool DEFAULTS = true, bool VIA_LDS = false>
 __device__ __forceinline__ void normalize_row(f32x8 (&v)[KS], const P* __restrict__ gamma,
                                               const P* __restrict__ beta, float eps, int g,
                                               typename Vec8<T>::type (&out)[KS]) {
@@ -89,7 +98,7 @@ __device__ __forceinline__ void normalize_row(f32x8 (&v)[KS], const P* __restric
   for (int kk = 0; kk < KS; ++kk)
 #pragma unroll
     for (int t = 0; t < 8; ++t) s[row_sum_chain<TZ>(kk, t)] += v[kk][t];
-  const float mean = row_sum4<TZ>(s) * (1.0f / (16 * KS));
+  const float mean = row_sum4<TZ, VIA_LDS>(s) * (1.0f / (16 * KS));
   float q[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
   for (int kk = 0; kk < KS; ++kk)
@@ -98,7 +107,7 @@ __device__ __forceinline__ void normalize_row(f32x8 (&v)[KS], const P* __restric
       const float d = v[kk][t] - mean;
       q[row_sum_chain<TZ>(kk, t)] += d * d;
     }
-  const float rstd = rsqrtf(row_sum4<TZ>(q) * (1.0f / (16 * KS)) + eps);
+  const float rstd = rsqrtf(row_sum4<TZ, VIA_LDS>(q) * (1.0f / (16 * KS)) + eps);
 #pragma unroll
   for (int kk = 0; kk < KS; ++kk) {
     // (no branch around these loads, so the compiler may issue them as early as registers allow)
@@ -153,7 +162,7 @@ __device__ __forceinline__ void normalize_raw(const typename Vec8<T>::type (&raw
 // and, if LN, normalise them.
 // TZ: storage type of the rows (T, or float for an fp32 residual stream normalised and
 // rounded to T here; LN only).
-template <typename T, int RB, bool LN, int KS, typename P = T, bool DEFAULTS = true, typename TZ = T>
+template <typename T, int RB, bool LN, int KS, typename P = T, bool DEFAULTS = true, typename TZ = T, bool VIA_LDS = false>
 __device__ __forceinline__ void load_rows_at(RowFrags<T, RB, KS>& out, const TZ* __restrict__ x,
                                              const int64_t (&off)[RB], const P* __restrict__ gamma,
                                              const P* __restrict__ beta, float eps, int lane) {
@@ -169,7 +178,7 @@ __device__ __forceinline__ void load_rows_at(RowFrags<T, RB, KS>& out, const TZ*
       f32x8 v[KS];
 #pragma unroll
       for (int kk = 0; kk < KS; ++kk) v[kk] = to_f32(load8<TZ>(rp + 16 * kk));
-      normalize_row<T, TZ, KS, P, DEFAULTS>(v, gamma, beta, eps, g, out.f[rb]);
+      normalize_row<T, TZ, KS, P, DEFAULTS, VIA_LDS>(v, gamma, beta, eps, g, out.f[rb]);
     }
   }
 }
