@@ -1,7 +1,7 @@
 """HIP-graph replay of a Pairformer block or stack for repeated calls at one shape.
 
-Below a few hundred tokens the forward pass is bound by the host: a block issues about forty
-kernel launches and the GPU finishes them faster than Python can enqueue them.  `Graphed`
+A block is some twelve dependent launches of 10 us each at small sizes, and what the host does between
+them (checking plans and masks, allocating, launching) is paid on every call.  `Graphed`
 records one forward pass of a `PairformerBlock` / `PairformerStack` into a HIP graph (through
 `torch.cuda.CUDAGraph`) and replays it for every later call with the same shapes and dtypes (and, for a single
 pair mask, the same class of mask: padding at the end with the same number of valid tokens, or
@@ -15,7 +15,8 @@ is an optional wrapper and the modules themselves are unchanged.  Inputs are cop
 graph's static buffers and the results are copied out, so the caller's tensors are never
 aliased; parameters are baked in by address, so weights must not be replaced (in-place updates
 of the same storage are picked up only by the kernels that read parameters directly: re-create
-the wrapper after loading new weights).  Every captured shape keeps its workspaces alive.
+the wrapper after loading new weights).  Every captured shape keeps its workspaces and the packed
+weights it was recorded with alive.
 """
 from __future__ import annotations
 
@@ -24,7 +25,7 @@ from typing import Dict, Optional, Tuple
 import torch
 import torch.nn as nn
 
-from . import ops
+from . import native, ops
 
 
 class Graphed:
@@ -76,7 +77,8 @@ class Graphed:
                 s_out, z_out = self.module(s_in, z_io, m_in, inplace_safe=True)
         finally:
             ops.capture_mask_class = None
-        return graph, s_in, z_io, m_in, s_out, z_out
+        # (with the plans it was recorded with: the graph has the addresses of their packed weights)
+        return graph, s_in, z_io, m_in, s_out, z_out, native.plans_of(self.module)
 
     def __call__(self, s: Optional[torch.Tensor], z: torch.Tensor,
                  pair_mask: Optional[torch.Tensor] = None
@@ -88,7 +90,7 @@ class Graphed:
         if entry is None:
             entry = self._capture(s, z, pair_mask)
             self._entries[key] = entry
-        graph, s_in, z_io, m_in, s_out, z_out = entry
+        graph, s_in, z_io, m_in, s_out, z_out, _ = entry
         z_io.copy_(z)
         if s_in is not None:
             s_in.copy_(s)

@@ -112,6 +112,12 @@ def _block_plan(blk, z, cd, sd):
     return plan
 
 
+def plans_of(module) -> list:
+    """Every plan kept for `module` and what is below it: a recorded graph holds them, since it has their weights'
+    addresses and a plan is replaced when a parameter is."""
+    return [plan for m in module.modules() for plan in _plans.get(m, {}).values()]
+
+
 def run_blocks(owner, blocks, s: Optional[torch.Tensor], z: torch.Tensor, pair_mask: Optional[torch.Tensor]):
     """The blocks on (s, z), z contiguous and updated in place: (the new s - None without a single track -, how many of the
     blocks were run).  What follows the first block without a plan is left to the caller, as is everything where the

@@ -82,6 +82,26 @@ def test_a_stack_called_by_two_threads_while_its_parameters_change():
 
 
 @pytest.mark.gpu
+def test_a_recording_outlives_the_plans_it_was_made_with():
+    """A parameter replaced by equal values makes the plan stale; the eager call that follows makes another, and the
+    memory of the first must still be the recording's."""
+    _, prod = oracle_and_product(O.PairformerStack, P.PairformerStack, n_blocks=2)
+    s, z, pm = (t.cuda() for t in O.make_inputs(40, n_pad=3))
+    fast = P.Graphed(prod)
+    s0, z0 = fast(s, z, pm)
+    with torch.no_grad():
+        for b in prod.blocks:
+            b.tri_mul_in.linear_g.weight = torch.nn.Parameter(b.tri_mul_in.linear_g.weight.detach())
+        prod(s, z, pm)
+        torch.cuda.synchronize()
+        junk = [torch.full((n,), float("nan"), device="cuda") for n in (98304, 131072, 1 << 20, 1 << 21, 1 << 22) for _ in range(4)]
+        for _ in range(2):
+            s1, z1 = fast(s, z, pm)
+            assert bool(torch.equal(s1, s0)) and bool(torch.equal(z1, z0))
+    del junk
+
+
+@pytest.mark.gpu
 def test_a_plan_made_on_one_stream_and_used_on_another():
     """The weights are still to be laid out when the second stream's call is issued, and the plan goes away while
     that call may still read them."""
