@@ -2,12 +2,13 @@
 // libprotenix_amd.so (allocation, argument lists, streams, autograd bookkeeping), in C++.  One call
 // per stack, update or operator instead of some twenty Python-level calls per block: below a few
 // hundred tokens the GPU finishes a block's kernels faster than Python can enqueue them (93 tokens:
-// 390 us of Python per block against about 110 us of kernels).
+// 390 us of Python per block against 130 us of kernels).
 //
 // Weights are laid out here, from the modules' parameters, once per weight set (a plan), with a record of the
 // parameters, sub-modules and hooks they came from: valid() compares identities and version
 // counters, so that a parameter that was replaced or changed in place is noticed on the next call.
-// The kernels, their order and their arguments are those of ops.py.
+// The kernels and their arguments are those of ops.py; in a stack the single track's stages ride on the next block's
+// pair kernels (Stages), where the Python path launches them on a second stream.
 #include <torch/extension.h>
 
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
