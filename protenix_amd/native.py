@@ -62,9 +62,20 @@ def _own_classes() -> tuple:
 def runs_own_forward(module) -> bool:
     """Whether calling `module` runs the forward its class in this package has, and nothing else (no `forward` of a
     subclass, of the instance or put into the class, no hooks): its kernels may then be issued without the call."""
+    return leading_own((module,)) == 1
+
+
+def leading_own(modules) -> int:
+    """How many of `modules`, from the first on, run their own forward (see runs_own_forward)."""
     classes, forwards = _own_classes()
-    return (type(module) in classes and "forward" not in module.__dict__ and not module._forward_hooks
-            and not module._forward_pre_hooks and all(c.forward is f for c, f in forwards))
+    if not all(c.forward is f for c, f in forwards):
+        return 0
+    count = 0
+    for m in modules:
+        if type(m) not in classes or "forward" in m.__dict__ or m._forward_hooks or m._forward_pre_hooks:
+            break
+        count += 1
+    return count
 
 
 def _usable(z: torch.Tensor) -> bool:

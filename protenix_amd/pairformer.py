@@ -279,7 +279,8 @@ class PairformerStack(nn.Module):
                 raise RuntimeError("protenix_amd.PairformerStack is inference-only: call .eval()")
         pad = None
         z_caller = z
-        own = all(native.runs_own_forward(b) for b in self.blocks)
+        lead = native.leading_own(self.blocks)
+        own = lead == len(self.blocks)
         if own and _wants_padding(z, pair_mask) and len(self.blocks) > 0:
             # (one padded copy for the whole stack, see pad_tokens_to)
             pad = _Padded(z)
@@ -294,8 +295,8 @@ class PairformerStack(nn.Module):
                 "triangle_multiplicative must be 'cuequivariance' or 'torch', but got "
                 f"{triangle_multiplicative}")
         assert triangle_attention in ("torch", "deepspeed", "triattention", "cuequivariance")
-        if pad is None and len(self.blocks) > 0:
-            s, done = native.run_blocks(self, tuple(self.blocks), s, z, pair_mask)
+        if pad is None and lead > 0:
+            s, done = native.run_blocks(self, tuple(self.blocks)[:lead], s, z, pair_mask)
             if done:
                 for blk in self.blocks[done:]:
                     s, z = blk(s, z, pair_mask, inplace_safe=True)

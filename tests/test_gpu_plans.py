@@ -167,7 +167,7 @@ def test_weights_of_another_shape_are_left_to_the_python_path():
 
 
 @pytest.mark.parametrize("at", [0, 1, 2, 3])
-@pytest.mark.parametrize("how", ["hook", "other"])
+@pytest.mark.parametrize("how", ["hook", "other", "another class"])
 def test_a_block_without_a_plan_leaves_the_rest_to_python(at, how):
     """The blocks before it have run natively by then, on the caller's z and s."""
     _, prod = oracle_and_product(O.PairformerStack, P.PairformerStack, n_blocks=4)
@@ -178,6 +178,16 @@ def test_a_block_without_a_plan_leaves_the_rest_to_python(at, how):
         blk = prod.blocks[at]
         if how == "hook":
             blk.tri_mul_in.register_forward_hook(lambda *_: seen.append(1))
+        elif how == "another class":
+            class Wrapped(torch.nn.Module):
+                def __init__(self, blk):
+                    super().__init__()
+                    self.inner = blk
+
+                def forward(self, *a, **k):
+                    seen.append(1)
+                    return self.inner(*a, **k)
+            prod.blocks[at] = Wrapped(blk).eval()
         else:
             fwd = blk.forward
             blk.forward = lambda *a, **k: (seen.append(1), fwd(*a, **k))[1]
