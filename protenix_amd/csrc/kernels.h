@@ -88,6 +88,7 @@ struct SingleStage {
   int kind, n_work;       // n_work workgroups
   int packed;             // linear: w, w2 in fragment order (single_stage.h; n_out % 16 == 0, k % 32 == 0)
   int tile, row_blocks;   // linear: tiles of 16 x 16, 16 x 32, 32 x 32 (1, 2, 3); tiles over the rows
+  int set_shift;          // linear: column tiles go to the XCDs in sets of 1 << set_shift
   int bits16;             // operands bf16, else fp32
   int rows;               // layernorm, linear: rows of x; attention: queries = keys
   const void* x;          // layernorm, linear: [rows][k]; attention: q, rows of pitch ld

@@ -63,6 +63,7 @@ void single_stage_linear(SingleStage* s, const void* x, const void* w, const voi
     s->row_blocks = (int)((span + rm - 1) / rm);
     const int cols = (n_out + cn - 1) / cn;
     s->n_work = cols * s->row_blocks;
+    for (s->set_shift = 3; s->set_shift > 0 && cols % (1 << s->set_shift); --s->set_shift) {}
     if (s->tile == 3 || (cols + 7) / 8 * 8 * s->row_blocks <= kStageTiles) break;
   }
   s->kind = s->n_work == 0 || rows == 0 ? kStageNone : w2 ? kStageSwiGLU : kStageLinear;

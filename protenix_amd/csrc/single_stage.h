@@ -49,11 +49,11 @@ __device__ __forceinline__ void linear_stage(const SingleStage& p, int wg, char*
   float (*part)[4 * NM * NB][kWave] = reinterpret_cast<float (*)[4 * NM * NB][kWave]>(smem);       // [wave][register][lane]
   const int lane = threadIdx.x & 63, ln = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  // All row blocks of a column block on one XCD, whose L2 then fetches those weights once: sets of eight column
-  // blocks, the last one of what is left.
-  const int row_blocks = p.row_blocks, col_blocks = (p.n_out + 16 * CN - 1) / (16 * CN);
-  const int set = wg / (8 * row_blocks), in_set = wg - set * (8 * row_blocks), width = min(8, col_blocks - 8 * set);
-  const int rb = width == 8 ? in_set >> 3 : in_set / width, cb = set * 8 + in_set - rb * width;
+  // Sets of eight column blocks (or fewer, see single_stage_linear): all row blocks of a column block on one XCD, whose L2 then
+  // fetches those weights once.
+  const int per_set = p.row_blocks << p.set_shift;
+  const int set = wg / per_set, in_set = wg - set * per_set;
+  const int rb = in_set >> p.set_shift, cb = (set << p.set_shift) + in_set - (rb << p.set_shift);
   const int row0 = rb * 16 * RM, col0 = cb * 16 * CN;
   const bool transposed = !SWIGLU && col0 >= p.split_col;   // the same for the whole workgroup
   // K steps of 32 (k is a multiple of 16), an equal share per wave.  A lane's 8 elements of a step are 16-byte pieces

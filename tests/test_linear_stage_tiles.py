@@ -28,10 +28,10 @@ def test_one_workgroup_per_tile(rows, n_out):
     assert n_work == cols * row_blocks
     # the mapping of linear_stage(): every tile once
     seen = set()
+    width = next(w for w in (8, 4, 2, 1) if cols % w == 0)
     for wg in range(n_work):
-        group, i = divmod(wg, 8 * row_blocks)
-        width = min(8, cols - 8 * group)
-        seen.add((i // width, 8 * group + i % width))
+        group, i = divmod(wg, width * row_blocks)
+        seen.add((i // width, width * group + i % width))
     assert seen == {(r, c) for r in range(row_blocks) for c in range(cols)}
 
 
