@@ -237,9 +237,10 @@ struct Weights {
   void settle() {
     int64_t bytes[2] = {0, 0};
     for (Wanted& w : wanted_) {
-      w.at = bytes[w.temporary];
-      bytes[w.temporary] += w.t.numel() * (int64_t)at::elementSize(w.type);
-      if (!w.fragments) bytes[w.temporary] = (bytes[w.temporary] + 15) / 16 * 16;
+      int64_t& used = bytes[w.temporary];
+      if (w.out) used = (used + 255) / 256 * 256;   // (whole cache lines; a matrix below another follows it)
+      w.at = used;
+      used += w.t.numel() * (int64_t)at::elementSize(w.type);
     }
     const auto options = at::TensorOptions().dtype(at::kByte).device(device_);
     char* base[2];
