@@ -454,14 +454,15 @@ struct Run {
     spans.push_back(std::move(s));
   }
   // What a pair launch carries: the next stage, or none for a projection (stage 0: of the triangle multiplications, 2: of the
-  // attentions) that has a faster kernel for it; on fp32 rows that is one of the two kinds at most, which leaves
+  // attentions) that has a faster kernel for it - from 480 tokens on, below that the LayerNorms' launches cost what it saves
+  // (16-bit rows, 384 tokens 528 us carrying / 533, 448 711 / 716, 480 881 / 872). On fp32 rows that is one of the two kinds at most, which leaves
   // five launches for the five other stages, on 16-bit rows it may be both, and stages left over are
   // launched.  us per block with a single track, always carrying / so: fp32 rows, 512 tokens 1107 / 1092, 640 1814 / 1785, 768
   // 2615 / 2595, 1024 5090 / 5047, 2048 28073 / 27832; 16-bit rows, 768 2403 / 2339, 1024 4656 / 4517, 1536 12661 / 12403.
   bool mul_alone = false, att_alone = false;
   void row_stages(int n, int c_z, int hidden, int dt) {
     mul_alone = ptx_row_stage_resident(0, n, c_z, hidden, dt);
-    att_alone = ptx_row_stage_resident(2, n, c_z, hidden, dt);
+    att_alone = n >= 480 && ptx_row_stage_resident(2, n, c_z, hidden, dt);
   }
   const ptx_single_stage* carry(int stage) {
     if ((stage == 0 && mul_alone) || (stage == 2 && att_alone)) return nullptr;

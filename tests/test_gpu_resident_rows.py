@@ -52,7 +52,7 @@ def test_fp32_rows_equal_the_general_kernels(kind, n, monkeypatch):
         assert ((got - want).abs().max() / want.abs().max()).item() <= 4e-3
 
 
-@pytest.mark.parametrize("mode,n", [("amp", 472), ("amp", 480), ("amp", 520), ("amp", 2048), ("bf16", 352), ("bf16", 704)])
+@pytest.mark.parametrize("mode,n", [("amp", 472), ("amp", 480), ("amp", 520), ("amp", 2048), ("bf16", 352), ("bf16", 480), ("bf16", 704)])
 def test_stages_that_do_not_ride(mode, n):
     _, prod = oracle_and_product(O.PairformerStack, P.PairformerStack, n_blocks=3 if n < 1000 else 2, dtype=BF16)
     dt = BF16 if mode == "bf16" else torch.float32
