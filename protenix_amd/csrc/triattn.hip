@@ -1,7 +1,7 @@
 // Triangle attention core: flash-style online softmax on MFMA, the N^3 logits
 // are never written anywhere.
 //
-// One workgroup (4 waves) owns one (row i, head h) pair and 128 queries; each
+// One workgroup (4 or 8 waves) owns one row i, or two, of one head h and 128 or 256 queries; each
 // wave owns 32 queries and walks over the keys in staged tiles of 64, which it
 // processes as two halves of 32 keys (16 logit registers at a time: four waves
 // fit a SIMD).  Per half:
@@ -17,8 +17,8 @@
 // is stored in 16 bits).  q and the bias are stored multiplied by log2(e) (by the projection
 // kernel), so on the common path the vector ALU executes per logit one conversion, one exp2,
 // half a packed bf16 convert and half a dot2 (the row sum).
-// K and V^T tiles are shared by the 4 waves through LDS in fragment order
-// (a ring of three tiles, one barrier per tile); the bias tile is private to a wave
+// K and V^T tiles are shared by the waves through LDS in fragment order (two tiles, one barrier per
+// tile; 16-bit tiles arrive by direct-to-LDS loads); the bias tile is private to a wave
 // and read straight from global (L2-resident: workgroups are numbered so that
 // one XCD works on one head at a time).
 //
@@ -73,16 +73,16 @@ struct AttnAux {
 // n_keys set to -inf (kMaskTail; kMaskNone where the keys fill whole tiles).
 enum { kMaskNone = 0, kMaskTail = 1, kMaskGiven = 2 };
 template <typename T, int R, int NWQ, int MK>
-__global__ __launch_bounds__((NWQ * 64), (sizeof(T) == 2 ? (R == 1 ? 16 / NWQ : (NWQ == 8 ? (MK == kMaskTail ? 4 : 2) : 3)) : 2)) void triattn_fwd_kernel(
+__global__ __launch_bounds__((NWQ * 64), (sizeof(T) == 2 ? (R == 1 ? 16 / NWQ : 4) : 2)) void triattn_fwd_kernel(
     const T* __restrict__ q, const T* __restrict__ k, const T* __restrict__ vt,
     const T* gate, const T* __restrict__ bias, const T* __restrict__ mask,
     T* o, int n, int heads, int key_pitch, int mask_transposed, float inf,
     int n_qtiles, int n_rowgroups, int64_t total_items, AttnAux ax) {
   typedef typename Vec8<T>::type V8;
   typedef typename Vec4<T>::type V4;
-  // ring of 3 key tiles x R rows: iteration t reads tile t while tile t+2 is written
-  __shared__ V8 lds_kv[3][R][8][kWave];     // fragments 0-3: K (u,kk); 4-7: V^T (u,s)
-  __shared__ __attribute__((aligned(16))) float lds_mb[3][R][kKeyTile];  // mask bias per key
+  // two key tiles x R rows: iteration t reads tile t while tile t+1 is written
+  __shared__ V8 lds_kv[2][R][8][kWave];     // fragments 0-3: K (u,kk); 4-7: V^T (u,s)
+  __shared__ __attribute__((aligned(16))) float lds_mb[2][R][kKeyTile];  // mask bias per key
 
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int ln = lane & 31, g = lane >> 5;
@@ -126,31 +126,35 @@ __global__ __launch_bounds__((NWQ * 64), (sizeof(T) == 2 ? (R == 1 ? 16 / NWQ : 
     for (int kk = 0; kk < 2; ++kk) qf[r][kk] = load8<T>(q + qrow[r] + 16 * kk + 8 * g);
   }
 
-  // ---- cooperative tile loader: 8*R fragments per key tile, 2*R per wave ----
-  // `tile` may run past the last tile: the pipeline below never branches around a load, so
-  // that the compiler can count the outstanding loads exactly.  Addresses use the clamped
-  // tile; the mask bias and the V^T zeroing use the real key index, which makes a phantom
-  // tile contribute exactly nothing.  Keys beyond n_keys hold garbage (or, below n, keys that
-  // are left out) in K, removed by the -inf mask bias, and are zeroed in V^T (0 * garbage must
-  // stay 0).
-  // fetch() only issues loads; everything that consumes a loaded value (mask -> additive
-  // bias, zeroing of V^T beyond n) happens in stash(), one tile of work later, so no wait
-  // for memory sits in the issue path.
-  constexpr int FPW = 8 * R / NWQ;   // fragments each wave moves per tile
-  V8 pre[FPW];
+  // ---- cooperative tile loader: 8*R fragments per key tile, 8*R / NWQ per wave ----
+  // 16-bit: direct-to-LDS loads (a fragment's LDS image is its global image: no registers, no LDS writes and, with
+  // a scalar base, no vector arithmetic); fp32: through registers.  fetch() only issues loads; what looks at a loaded value
+  // (mask -> additive bias, zeroing of V^T beyond n_keys) happens in stash(), one tile of work later.
+  // Keys beyond n_keys hold garbage (or, below n, keys that are left out) in K, removed by the -inf mask bias, and
+  // are zeroed in V^T (0 * garbage must stay 0).
+  constexpr bool kDirect = sizeof(T) == 2;
+  constexpr int FPW = 8 * R / NWQ;   // fragments each wave moves per tile, of one operand and row
+  static_assert(FPW >= 1 && FPW <= 4, "a wave's fragments are consecutive in memory");
+  const int fid0 = wave * FPW, fr = fid0 >> 3, f0 = fid0 & 7;   // row, first fragment
+  const T* const kv_base = (f0 < 4 ? k : vt) + ((int64_t)h * n_rows + min(i0 + fr, n_rows - 1)) * key_tiles * kAttnTileElems + (f0 & 3) * 512;
+  V8 pre[kDirect ? 1 : FPW];
   T pre_mv;
   // mask value of key kc for this wave's row: m_base[kc * m_stride]
   const int m_row = min(i0 + min(wave, R - 1), n_rows - 1);
   const unsigned m_stride = mask_transposed ? n : 1;
   const T* m_base = has_mask ? mask + (mask_transposed ? (int64_t)m_row : (int64_t)m_row * n) : nullptr;
   auto fetch = [&](int tile) {
-    const int64_t atile = min(tile, n_tiles - 1);
+    const T* src = kv_base + (int64_t)tile * kAttnTileElems;
+    if constexpr (kDirect) {
+      const uint64_t base = uniform64((uint64_t)src);
+      const uint32_t dst = lds_address(&lds_kv[tile & 1][fr][f0][0]), off = lane * 16;
+      load_to_lds16_s<0>(base, off, dst);
+      if constexpr (FPW > 1) load_to_lds16_s<1024>(base, off, dst);
+      if constexpr (FPW > 2) load_to_lds16_s<2048>(base, off, dst);
+      if constexpr (FPW > 3) load_to_lds16_s<3072>(base, off, dst);
+    } else {
 #pragma unroll
-    for (int j = 0; j < FPW; ++j) {
-      const int fid = wave * FPW + j;              // row = fid / 8, fragment = fid % 8
-      const int r = fid >> 3, f = fid & 7;
-      const int64_t rowtiles = ((int64_t)h * n_rows + min(i0 + r, n_rows - 1)) * key_tiles + atile;
-      pre[j] = load8<T>((f < 4 ? k : vt) + rowtiles * kAttnTileElems + (f & 3) * 512 + lane * 8);
+      for (int j = 0; j < FPW; ++j) pre[j] = load8<T>(src + j * 512 + lane * 8);
     }
     // wave w < R publishes the mask bias of row i0 + w; all waves load (uniform load count)
     if constexpr (has_mask) {
@@ -159,21 +163,24 @@ __global__ __launch_bounds__((NWQ * 64), (sizeof(T) == 2 ? (R == 1 ? 16 / NWQ : 
     }
   };
   auto stash = [&](int tile) {
-    const int buf = tile % 3;
+    const int buf = tile & 1;
     const int key0 = tile * kKeyTile;
     const bool tail = MK != kMaskNone && key0 + kKeyTile > nk;   // uniform (kMaskNone: whole tiles only)
+    if constexpr (kDirect) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // (nothing younger than the tile's loads is under way)
+    if (!kDirect || tail) {
 #pragma unroll
-    for (int j = 0; j < FPW; ++j) {
-      const int fid = wave * FPW + j;
-      const int f = fid & 7;
-      V8 v = pre[j];
-      if (tail && f >= 4) {
-        // V^T fragment (u, s): slots <-> keys 32g + 16u + 8s + t
-        const int koff = key0 + 32 * g + 16 * ((f >> 1) & 1) + 8 * (f & 1);
+      for (int j = 0; j < FPW; ++j) {
+        V8 v;
+        if constexpr (kDirect) v = lds_kv[buf][fr][f0 + j][lane];
+        else v = pre[j];
+        if (tail && f0 >= 4) {
+          // V^T fragment (u, s): slots <-> keys 32g + 16u + 8s + t
+          const int f = f0 + j, koff = key0 + 32 * g + 16 * ((f >> 1) & 1) + 8 * (f & 1);
 #pragma unroll
-        for (int t = 0; t < 8; ++t) v[t] = koff + t < nk ? v[t] : (T)0.0f;
+          for (int t = 0; t < 8; ++t) v[t] = koff + t < nk ? v[t] : (T)0.0f;
+        }
+        lds_kv[buf][fr][f0 + j][lane] = v;
       }
-      lds_kv[buf][fid >> 3][f][lane] = v;
     }
     if constexpr (has_mask) {
       if (wave < R) {
@@ -193,6 +200,7 @@ __global__ __launch_bounds__((NWQ * 64), (sizeof(T) == 2 ? (R == 1 ? 16 / NWQ : 
   };
 
   f32x16 acc_o[R];                // O^T per row
+  bool zero_reference = false;    // (uniform) every row's softmax reference is 0
   float m_run[R], l_run[R];       // running max (natural units) and denominator (this lane's keys)
 #pragma unroll
   for (int r = 0; r < R; ++r) {
@@ -228,6 +236,33 @@ __global__ __launch_bounds__((NWQ * 64), (sizeof(T) == 2 ? (R == 1 ? 16 / NWQ : 
   struct HalfOut {
     V8 pf[2];
     float psum, alpha;
+  };
+  // P^T of a half from its exponentials, and their sum over this lane's keys.
+  auto probabilities = [&](const f32x16& s, V8 (&pf)[2]) -> float {
+    float psum = 0.0f;
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      f32x8 p8;
+#pragma unroll
+      for (int t = 0; t < 8; ++t) p8[t] = s[8 * c + t];
+      pf[c] = from_f32<T>(p8);
+      if constexpr (sizeof(T) == 2) {
+        bf16x2 ones;
+        ones[0] = (__bf16)1.0f;
+        ones[1] = (__bf16)1.0f;
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+          bf16x2 pr;
+          pr[0] = pf[c][2 * t];
+          pr[1] = pf[c][2 * t + 1];
+          psum = __builtin_amdgcn_fdot2_f32_bf16(pr, ones, psum, false);
+        }
+      } else {
+#pragma unroll
+        for (int t = 0; t < 8; ++t) psum += p8[t];
+      }
+    }
+    return psum;
   };
   // TAIL: the tile holds keys beyond n_keys; their logits, whatever was made of the K rows and
   // mask values found there, are replaced by -inf before the softmax (weight zero).  The other
@@ -302,30 +337,7 @@ __global__ __launch_bounds__((NWQ * 64), (sizeof(T) == 2 ? (R == 1 ? 16 / NWQ : 
 #pragma unroll
       for (int e = 0; e < 16; ++e) s[e] = fast_exp2((s[e] - mref) * kLog2e);
     }
-    float psum = 0.0f;
-#pragma unroll
-    for (int c = 0; c < 2; ++c) {
-      f32x8 p8;
-#pragma unroll
-      for (int t = 0; t < 8; ++t) p8[t] = s[8 * c + t];
-      out.pf[c] = from_f32<T>(p8);
-      if constexpr (sizeof(T) == 2) {
-        typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2_t;
-        bf16x2_t ones;
-        ones[0] = (__bf16)1.0f;
-        ones[1] = (__bf16)1.0f;
-#pragma unroll
-        for (int t = 0; t < 4; ++t) {
-          bf16x2_t pr;
-          pr[0] = out.pf[c][2 * t];
-          pr[1] = out.pf[c][2 * t + 1];
-          psum = __builtin_amdgcn_fdot2_f32_bf16(pr, ones, psum, false);
-        }
-      } else {
-#pragma unroll
-        for (int t = 0; t < 8; ++t) psum += p8[t];
-      }
-    }
+    const float psum = probabilities(s, out.pf);
     if constexpr (MODE == kOptimistic || MODE == kOptimisticZero) {
       if ((__builtin_amdgcn_ballot_w64(!(psum < kOptimisticLimit)) & q_ok_mask) != 0ull) return false;
     }
@@ -335,7 +347,7 @@ __global__ __launch_bounds__((NWQ * 64), (sizeof(T) == 2 ? (R == 1 ? 16 / NWQ : 
   };
   auto process_tile = [&](auto tail_tag, int tile, V8 (&tb)[2][2]) {
     constexpr bool LAST_PARTIAL = decltype(tail_tag)::value;   // the one tile with keys beyond n_keys
-    const int buf = tile % 3;
+    const int buf = tile & 1;
     const int key0 = tile * kKeyTile;
     // keys of the tile with a non-zero mask bias, per row, as a lane mask (key <-> lane); half
     // u's keys are the lanes with bit 4 == u
@@ -356,10 +368,54 @@ __global__ __launch_bounds__((NWQ * 64), (sizeof(T) == 2 ? (R == 1 ? 16 / NWQ : 
     for (int u = 0; u < 2; ++u) {
       const bool tail_tile = LAST_PARTIAL && tile_keys < 48 + 16 * u;
       if (LAST_PARTIAL && tile_keys <= 16 * u) continue;
-      const f32x8 b0 = to_f32(tb[u][0]), b1 = to_f32(tb[u][1]);
-      const f32x16 tbf = __builtin_shufflevector(b0, b1, 0, 1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15);
+      auto bias_of = [](const V8 (&raw)[2]) {
+        const f32x8 b0 = to_f32(raw[0]), b1 = to_f32(raw[1]);
+        return __builtin_shufflevector(b0, b1, 0, 1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15);
+      };
+      // The common path of two rows: the reference is 0, no key is left out.  Both rows' logits are formed before the first
+      // row's exponentials, which run under the second row's products (the second takes the bias' registers), and the
+      // second's under the first's P.V (768 tokens 375 -> 363 us, 2048 6315 -> 6160).  What a row does is what half_row's
+      // kOptimisticZero does.  A probability sum out of range leaves this row, and the second one behind it, to the
+      // paths below (r_begin: rows that are done).
+      int r_begin = 0;
+      if constexpr (R == 2 && !has_mask) {
+        if (zero_reference && !tail_tile) {
+          const f32x16 tbf = bias_of(tb[u]);
+          V8 kf[2][2];
+          f32x16 s[2];
+#pragma unroll
+          for (int r = 0; r < 2; ++r)
+#pragma unroll
+            for (int kk = 0; kk < 2; ++kk) kf[r][kk] = lds_kv[buf][r][u * 2 + kk][lane];
+#pragma unroll
+          for (int r = 0; r < 2; ++r) {
+            s[r] = tbf;
+#pragma unroll
+            for (int kk = 0; kk < 2; ++kk) mma32(s[r], kf[r][kk], qf[r][kk]);
+          }
+#pragma unroll
+          for (int r = 0; r < 2; ++r) {
+            if (r_begin != r) break;
+            V8 vf[2], pf[2];
+#pragma unroll
+            for (int c = 0; c < 2; ++c) vf[c] = lds_kv[buf][r][4 + u * 2 + c][lane];
+#pragma unroll
+            for (int e = 0; e < 16; ++e) s[r][e] = fast_exp2(s[r][e]);
+            const float psum = probabilities(s[r], pf);
+            if ((__builtin_amdgcn_ballot_w64(!(psum < kOptimisticLimit)) & q_ok_mask) != 0ull) break;
+            l_run[r] += psum;
+#pragma unroll
+            for (int c = 0; c < 2; ++c) mma32(acc_o[r], vf[c], pf[c]);
+            r_begin = r + 1;
+          }
+          if (r_begin == 2) continue;
+        }
+        asm volatile("" : "+v"(tb[u][0]), "+v"(tb[u][1]));   // (the bias is converted again: no registers for it on the common path)
+      }
+      const f32x16 tbf = bias_of(tb[u]);
 #pragma unroll
       for (int r = 0; r < R; ++r) {
+        if (r < r_begin) continue;
         // the unmasked paths of one half: optimistic against the reference the earlier tiles
         // left, classic if there is none yet or the optimistic one had to give up
         auto unmasked_half = [&](auto ttag, HalfOut& out) -> bool {
@@ -393,26 +449,30 @@ __global__ __launch_bounds__((NWQ * 64), (sizeof(T) == 2 ? (R == 1 ? 16 / NWQ : 
 #pragma unroll
         for (int c = 0; c < 2; ++c) mma32(acc_o[r], lds_kv[buf][r][4 + u * 2 + c][lane], out.pf[c]);
       }
+      if constexpr (R == 2 && !has_mask)
+        zero_reference = ((__builtin_amdgcn_ballot_w64(m_run[0] != 0.0f) | __builtin_amdgcn_ballot_w64(m_run[1] != 0.0f)) & q_ok_mask) == 0ull;
     }
     }
-    fetch_bias(tile + 1, tb);
   };
-  // Tile t+2 travels global -> registers -> LDS while tile t is processed; the bias tile of
-  // t+1 is requested into the bias registers once tile t has consumed them.
+  // Tile t+1 travels while tile t is processed; its bias tile is requested into the bias registers once tile t has
+  // consumed them, behind the wait for tile t+1.
   V8 tbias[2][2];
+  auto barrier = [] { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
   auto step = [&](auto tail_tag, int tile) {
-    fetch(tile + 2);
+    const bool more = tile + 1 < n_tiles;
+    if (more) fetch(tile + 1);
     process_tile(tail_tag, tile, tbias);
-    stash(tile + 2);
-    __syncthreads();
+    if (more) {
+      stash(tile + 1);
+      fetch_bias(tile + 1, tbias);
+    }
+    barrier();
   };
 
   fetch(0);
   fetch_bias(0, tbias);
   stash(0);
-  fetch(1);
-  stash(1);
-  __syncthreads();
+  barrier();
   // the tiles whose keys all take part, in a loop that knows nothing of a partial tile (with
   // its tests in the loop every tile was 7 % slower), then the partial one if there is one
   const int n_full = MK == kMaskNone ? n_tiles : nk / kKeyTile;
@@ -481,63 +541,49 @@ int triattn_fwd_ex(const T* q, const T* k, const T* vt, const T* g, const T* tri
                    int row_count, int n_keys, hipStream_t stream) {
   if (n == 0 || n_rows == 0 || row_count == 0) return 0;
   AttnAux ax = {sh, si, sj, n_rows, mask_is_bias, lse, lh, li, lj, row_begin, row_begin + row_count, n_keys, 0, n};
-  // 8-wave workgroups for long rows (measured: +2 % at n = 768, even at 1024, -2.6 % at 1536,
-  // -2.2 % at 2048), where their 256 queries divide n or n is large enough for the idle waves
-  // of the last one not to matter
-  const bool wide = sizeof(T) == 2 && ((n % 256 == 0 && n >= 1536) || n >= 2048);
-  // Two rows per wave, in 8-wave workgroups (16-bit, no mask): the two rows
-  // share the query block and with it the bias tile - one load and one conversion per logit for
-  // both, half the bias stream from the L2 - at 123 registers, so that four waves still share a
-  // SIMD (with a partial last key tile the register allocator is held to 128 by the kernel's
-  // launch bounds and gets there without spills; with a mask the kernel needs 160 and loses a
-  // wave; with four waves per workgroup the K / V tiles of two rows leave room for three
-  // workgroups only: no gain).  Per launch: 395 -> 356 us at n = 768 in the trunk; in a loop of attention updates
-  // -7 % at n = 512, -3 % at 768, -11 % at 1536, -13 % at 2048.  Where 256 queries do not divide
-  // n, the waves of a row's last workgroup that have no queries skip the arithmetic and only
-  // help to stage the K / V tiles; such a workgroup still holds its place for as long as the
-  // staging takes (n = 776 against 768, same keys: +11 %), but a second launch for the
-  // remaining queries - one row per wave, two or four waves per workgroup - was no better
-  // (per update, against the split launches with every wave computing: 520 214 -> 208 us,
-  // 640 270 -> 255, 704 369 -> 332, 800 592 -> 550, 1032 1127 -> 1055, 1100 1239 -> 1214).
-  const bool r2 = sizeof(T) == 2 && !mask && n >= 512 && row_count >= 2;
+  // Two rows per wave (16-bit, no mask): the two rows share the query block and with it the bias tile - one load
+  // and one conversion per logit for both, half the bias stream from the L2 - at 128 registers, so that four waves
+  // still share a SIMD (with a mask the kernel needs 160 and loses a wave).  Below 352 tokens the pairs of rows leave too few
+  // workgroups.  us per launch, 4 heads, one row (four waves) / two rows (four waves) / two rows (eight): n = 256 23.3 / 24.8 /
+  // 24.6, 320 39.9 / 40.0 / 47.8, 384 63 / 60 / 68, 387 86 / 78 / 83, 448 94 / 89 / 91, 480 128 / 118 / 120, 600 234 / 211 / 223, 768
+  // 395 / 363 / 366, 776 481 / 432 / 474, 1024 895 / 833 / 825, 1100 1215 / 1105 / 1105, 1536 3041 / 2707 / 2680, 2048 7157 / 6418 / 6150.
+  // (Before direct-to-LDS loads and two tiles in LDS instead of three, which made room for four workgroups of four waves per
+  // compute unit, and before two rows' products ran next to each other's exponentials: 384 67, 387 94, 600 233, 768 385, 776
+  // 494, 1024 856, 2048 6410.)
+  const bool two_rows = sizeof(T) == 2 && !mask && n >= 352 && row_count >= 2;
+  // Eight waves share the staged K / V tiles of long rows: +2 % at n = 768 with one row per wave, even at 1024, -2.6 % at 1536; with
+  // two rows the figures above.  Where 256 queries do not divide n, the waves of a row's last workgroup that have no queries
+  // skip the arithmetic and only help to stage the tiles.
+  const bool wide = sizeof(T) == 2 && (two_rows ? n > 1056 : (n % 256 == 0 && n >= 1536) || n >= 2048);
   const int mk = mask ? kMaskGiven : n_keys % kKeyTile ? kMaskTail : kMaskNone;
-  // one launch over the queries q_begin .. q_end-1 of the launch's rows
-  auto launch = [&](int q_begin, int q_end, bool two_rows, bool wide8) {
-    ax.q_begin = q_begin;
-    ax.q_end = q_end;
-    const int nq = q_end - q_begin;
-    const int n_qtiles = (two_rows || wide8) ? (nq + 255) / 256 : (nq + 127) / 128;
-    const int R = two_rows ? 2 : 1;
-    const int n_rowgroups = (row_count + R - 1) / R;
-    const int64_t total = (int64_t)heads * n_rowgroups * n_qtiles;
-    const int64_t per_xcd = (total + 7) / 8;
+  const int n_qtiles = wide ? (n + 255) / 256 : (n + 127) / 128;
+  const int R = two_rows ? 2 : 1;
+  const int n_rowgroups = (row_count + R - 1) / R;
+  const int64_t total = (int64_t)heads * n_rowgroups * n_qtiles;
+  const int64_t per_xcd = (total + 7) / 8;
 #define PTX_ATTN_LAUNCH_R(RR, NWQ, MK)                                                            \
   triattn_fwd_kernel<T, RR, NWQ, MK><<<dim3((unsigned)(per_xcd * 8)), dim3(NWQ * 64), 0, stream>>>( \
       q, k, vt, g, tri_bias, mask, o, n, heads, key_pitch, mask_transposed, inf, n_qtiles,        \
       n_rowgroups, total, ax)
-#define PTX_ATTN_LAUNCH(NWQ, MK) PTX_ATTN_LAUNCH_R(1, NWQ, MK)
-    if (two_rows) {
-      if constexpr (sizeof(T) == 2) {
-        if (mk == kMaskTail) PTX_ATTN_LAUNCH_R(2, 8, kMaskTail);
-        else PTX_ATTN_LAUNCH_R(2, 8, kMaskNone);
-      }
-    } else if (wide8) {
-      if (mk == kMaskGiven) PTX_ATTN_LAUNCH(8, kMaskGiven);
-      else if (mk == kMaskTail) PTX_ATTN_LAUNCH(8, kMaskTail);
-      else PTX_ATTN_LAUNCH(8, kMaskNone);
-    } else {
-      if (mk == kMaskGiven) PTX_ATTN_LAUNCH(4, kMaskGiven);
-      else if (mk == kMaskTail) PTX_ATTN_LAUNCH(4, kMaskTail);
-      else PTX_ATTN_LAUNCH(4, kMaskNone);
+#define PTX_ATTN_LAUNCH(RR, MK)                \
+  do {                                         \
+    if (wide) PTX_ATTN_LAUNCH_R(RR, 8, MK);    \
+    else PTX_ATTN_LAUNCH_R(RR, 4, MK);         \
+  } while (0)
+  if (two_rows) {
+    if constexpr (sizeof(T) == 2) {
+      if (mk == kMaskTail) PTX_ATTN_LAUNCH(2, kMaskTail);
+      else PTX_ATTN_LAUNCH(2, kMaskNone);
     }
+  } else if (mk == kMaskGiven) {
+    PTX_ATTN_LAUNCH(1, kMaskGiven);
+  } else if (mk == kMaskTail) {
+    PTX_ATTN_LAUNCH(1, kMaskTail);
+  } else {
+    PTX_ATTN_LAUNCH(1, kMaskNone);
+  }
 #undef PTX_ATTN_LAUNCH
 #undef PTX_ATTN_LAUNCH_R
-  };
-  if (r2) {
-    launch(0, n, true, false);
-  } else {
-    launch(0, n, false, wide);
-  }
   return 0;
 }
 

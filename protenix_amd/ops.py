@@ -206,12 +206,12 @@ _mask_cache: list = []
 
 # Pair masks of padded batches are m (x) m with the padding at the end: the triangle attention
 # then runs its valid rows over the valid keys without a mask (see triangle_attention).  False
-# hands every mask to the kernels as it is (tests compare the two).  Below some 480 tokens the
-# second launch costs what the first one saves (measured per update, two launches against the
-# masked kernel: 170 against 157 us at N = 384 with 32 padded tokens, 237 = 237 at 448, 293
-# against 305 at 512, 390 against 411 at 576, 1.42 against 1.59 ms at 1024).
+# hands every mask to the kernels as it is (tests compare the two).  From 352 tokens on, where the unmasked
+# kernel takes two rows per wave; below, the second launch costs what the first one saves (us per update, two launches
+# against the masked kernel: 106 = 106 at N = 320 with 20 padded tokens, 118 against 126 at 352, 170 against 190 at 416 with 50,
+# 189 against 200 at 448; 384 with 32, whose keys fill whole tiles either way: 134 against 135).
 prefix_mask_enabled = True
-prefix_mask_min_n = 480
+prefix_mask_min_n = 352
 
 
 _CACHE_ENTRIES = 64      # masks kept per cache: a batch of pair masks has one entry per element

@@ -1,0 +1,59 @@
+"""The triangle-attention core where its workgroups change: two rows per wave from 352 tokens on, eight waves from 1057 on, odd
+numbers of rows and of query blocks, last key tiles of one key to a whole tile; and logits that leave the range of the
+reference 0, which take rows off the common path in the middle of a wave's work."""
+import math
+
+import pytest
+import torch
+
+from protenix_amd import _lib
+
+
+def _core(n, heads, scale, g, n_keys=None):
+    """q, K, V^T, bias in the core's layouts from random plain tensors, and the plain tensors."""
+    lib = _lib.load()
+    q, k, v = (torch.randn(heads, n, n, 32, generator=g).bfloat16() for _ in range(3))
+    b = (scale * torch.randn(heads, n, n, generator=g)).bfloat16()
+    pitch = lib.ptx_key_pitch(n)
+    tiles, qb = pitch // 64, (n + 31) // 32
+    j = torch.arange(n)
+    gg, u, r = (j % 64) // 32, (j % 32) // 16, j % 16
+    kd = torch.full((heads, n, tiles, 2, 2, 2, 32, 8), float("nan")).bfloat16()      # u, kk, lane half, MFMA row, d
+    kd[:, :, j // 64, u, :, :, 8 * (r // 4) + 4 * gg + r % 4] = k.view(heads, n, n, 2, 2, 8).permute(2, 0, 1, 3, 4, 5)
+    vd = torch.full((heads, n, tiles, 2, 2, 2, 32, 8), float("nan")).bfloat16()      # u, key group, lane half, d, key
+    vd[:, :, j // 64, u, r // 8, gg, :, j % 8] = v.permute(2, 0, 1, 3)
+    bd = torch.zeros(heads, qb, tiles, 2, 2, 2, 32, 8).bfloat16()
+    qi = torch.arange(n)[:, None].expand(n, n)
+    jj = j[None, :].expand(n, n)
+    bd[:, qi // 32, jj // 64, (jj % 32) // 16, (jj % 16) // 8, (jj % 64) // 32, qi % 32, jj % 8] = b
+    return (q, kd, vd, bd), (q, k, v, b), pitch
+
+
+def _reference(q, k, v, b, rows, n_keys):
+    # the core works in log2 units: probabilities 2^(q.k + b)
+    s = torch.einsum("hiqd,hikd->hiqk", q[:, rows].float(), k[:, rows].float()) + b[:, None].float()
+    p = torch.softmax(s[..., :n_keys] * math.log(2.0), dim=-1)
+    return torch.einsum("hiqk,hikd->hiqd", p, v[:, rows, :n_keys].float())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [33, 351, 352, 353, 385, 417, 1057])
+@pytest.mark.parametrize("scale", [1.0, 40.0])
+def test_core(n, scale):
+    lib, heads = _lib.load(), 1
+    g = torch.Generator().manual_seed(n)
+    dev, plain, pitch = _core(n, heads, scale, g)
+    dq, dk, dv, db = (t.cuda() for t in dev)
+    st = torch.cuda.current_stream().cuda_stream
+    for row0, count, n_keys in ((0, n, n), (2, n - 3, n - 1)):
+        o = torch.full((heads, n, n, 32), 7.0, dtype=torch.bfloat16, device="cuda")
+        rc = lib.ptx_triattn_fwd_rows(dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), None, db.data_ptr(), None, o.data_ptr(), n, heads, 32,
+                                      pitch, 0, 1e9, row0, count, n_keys, 1, st)
+        assert rc == 0
+        o = o.cpu()
+        rows = sorted({row0, row0 + 1, row0 + count // 2, row0 + count - 2, row0 + count - 1})
+        # (probabilities and outputs are rounded to 8 significant bits: 2^-8 each of a weighted mean of |v| < 5)
+        err = (o[:, rows].float() - _reference(*plain, rows, n_keys)).abs().max().item()
+        assert err <= 2 * 2.0 ** -8 * plain[2].abs().max().item(), (n, scale, row0, err)
+        outside = [r for r in range(n) if not row0 <= r < row0 + count]
+        assert bool((o[:, outside] == 7.0).all())
