@@ -97,6 +97,9 @@ struct ProjInParams {
   int n, pitch, backward;
   int tiles_per_i;        // triattn_in: 0 = linear tiles
   int heads;
+  int slices;             // workgroups per tile, each with its share of the output columns (see in_slices)
+  unsigned tiles;
+  int share;              // trimul_in: a wave's chunks per slice
   float q_scale;
 };
 
@@ -110,7 +113,7 @@ __global__ __launch_bounds__(kPpWaves * 64, (kPpMinWaves<T, KS>)) void pp_trimul
   typedef typename VecE<T>::type VE_t;
   typedef Cfg<T> C;
   constexpr int CPM = PpWidths<KS>::HIDDEN / 32;    // chunks (of 32 channels) per operand
-  constexpr int CHW = 2 * CPM / kPpWaves;           // chunks per wave
+  constexpr int CHW = 2 * CPM / kPpWaves;           // chunks per wave, all slices
   constexpr int kFrag = RBW * FragLds<T, KS>::ROWBLOCK, kStage = kPpWaves * 32 * C::PITCH * (int)sizeof(T);
   __shared__ __attribute__((aligned(16))) char smem[cmax(kFrag + kStage + 128 * RBW, kStageLds)];
   PTX_CARRIED_STAGE();
@@ -123,7 +126,8 @@ __global__ __launch_bounds__(kPpWaves * 64, (kPpMinWaves<T, KS>)) void pp_trimul
   const uint32_t n_kb = (uint32_t)p.pitch >> 3, n_ip = (uint32_t)(n + 4 * RBW - 1) / (4 * RBW);
   // Patches in the order of the memory rows they read, back to front behind a kernel that wrote the pair tensor
   // front to back (the tail is what the memory-side cache still holds).
-  const uint32_t bx = xcd_run(block, blocks), tile = p.backward ? blocks - 1 - bx : bx;
+  const uint32_t tiles = p.tiles, slice = (block >= tiles) + (block >= 2 * tiles) + (block >= 3 * tiles);
+  const uint32_t bx = xcd_run(block - slice * tiles, tiles), tile = p.backward ? tiles - 1 - bx : bx;
   int pi0, pk0;
   if (p.backward) {   // incoming: the inner index is the slow one of z
     const uint32_t kb = tile / n_ip;
@@ -150,7 +154,8 @@ __global__ __launch_bounds__(kPpWaves * 64, (kPpMinWaves<T, KS>)) void pp_trimul
         return i * p.si + k * p.sj;
       },
       (const T*)p.gamma, (const T*)p.beta, p.eps, wave, lane, raw);
-  load_w(wave * CHW);
+  const int c_begin = slice * p.share, c_end = c_begin + p.share;   // this slice's chunks of every wave
+  load_w(wave * CHW + c_begin);
   if (threadIdx.x < 32 * RBW) {
     const int i = min(pi0 + (int)(threadIdx.x >> 3), n - 1), k = pk0 + (int)(threadIdx.x & 7);
     float mv = 1.0f;
@@ -172,6 +177,7 @@ __global__ __launch_bounds__(kPpWaves * 64, (kPpMinWaves<T, KS>)) void pp_trimul
   }
 #pragma unroll
   for (int c = 0; c < CHW; ++c) {
+    if (c < c_begin || c >= c_end) continue;
     const int ch = wave * CHW + c;
     T* outp = (T*)p.out[ch / CPM] + trimul_frag_offset((ch % CPM) * 32, 0, 0, n_rb, n_ks);
 #pragma unroll
@@ -185,7 +191,7 @@ __global__ __launch_bounds__(kPpWaves * 64, (kPpMinWaves<T, KS>)) void pp_trimul
         mma32(acc[0], xv, w[0][kk]);   // lane <-> channel, register <-> row
         mma32(acc[1], xv, w[1][kk]);
       }
-      if (rb == RBW - 1 && c + 1 < CHW) load_w(ch + 1);
+      if (rb == RBW - 1 && c + 1 < CHW && c + 1 < c_end) load_w(ch + 1);
       float vals[16];
 #pragma unroll
       for (int qd = 0; qd < 4; ++qd) {
@@ -226,8 +232,9 @@ __global__ __launch_bounds__(kPpWaves * 64, (kPpMinWaves<T, KS>)) void pp_triatt
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int n = p.n;
   const int64_t n_rows = (int64_t)n * n;
-  const uint32_t bx = xcd_run(block, blocks);
-  const int64_t tile = p.backward ? blocks - 1 - bx : bx;
+  const uint32_t tiles = p.tiles, slice = (block >= tiles) + (block >= 2 * tiles) + (block >= 3 * tiles);
+  const uint32_t bx = xcd_run(block - slice * tiles, tiles);
+  const int64_t tile = p.backward ? tiles - 1 - bx : bx;
   const TileRows tr = tile_rows(tile, 32 * RBW, n, p.tiles_per_i);
   const T* packed = (const T*)p.packed;
   V8 w[2][KS];
@@ -248,13 +255,14 @@ __global__ __launch_bounds__(kPpWaves * 64, (kPpMinWaves<T, KS>)) void pp_triatt
         return i * p.si + j * p.sj;
       },
       (const T*)p.gamma, (const T*)p.beta, p.eps, wave, lane, raw);
-  load_w(wave);
+  const int step = kPpWaves * p.slices;
+  load_w(min(wave + kPpWaves * (int)slice, NPAIR - 1));
   __syncthreads();
 
   const int key_tiles = p.pitch >> 6, q_blocks = (n + 31) >> 5;
   const int64_t head_plane = (int64_t)n * key_tiles * kAttnTileElems;
 #pragma unroll 1
-  for (int pair = wave; pair < NPAIR; pair += kPpWaves) {
+  for (int pair = wave + kPpWaves * slice; pair < NPAIR; pair += step) {
     const int which = pair < NPAIR - 1 ? pair / HP : 4;   // 0 q, 1 k, 2 v, 3 gate, 4 bias
     const int h0 = (pair % HP) * 2;
 #pragma unroll
@@ -277,7 +285,7 @@ __global__ __launch_bounds__(kPpWaves * 64, (kPpMinWaves<T, KS>)) void pp_triatt
           mma32(acc[1], w[1][kk], xv);
         }
       }
-      if (rb == RBW - 1 && pair + kPpWaves < NPAIR) load_w(pair + kPpWaves);
+      if (rb == RBW - 1 && pair + step < NPAIR) load_w(pair + step);
       wave_lds_sync();
 #pragma unroll
       for (int t = 0; t < 2; ++t) {
@@ -729,6 +737,18 @@ static bool resident_rows(RowStage stage, int n, int c_z, int hidden, const Sing
   return pp_resident(stage, n, c_z, hidden, sizeof(T) == 2, sizeof(TZ) == 2) && !(carry && carry->kind != kStageNone);
 }
 
+// Workgroups per tile of a projection.  Where the tiles leave compute units idle, each takes a share of the output
+// columns (and normalises the rows again): a wave then works through one set of columns instead of two or three.  fp32,
+// whose sets take 4 us of matrix pipe each, up to three and a half workgroups per compute unit.  us, without / with: one
+// fp32 block at 48 tokens 209 / 181, 64 215 / 195, 93 333 / 317 (128, which stays as it is: 347 / 352); two blocks of 256 channels at 64
+// tokens 342 / 316; 16 blocks under autocast at 40 tokens 1230 / 1209, 64 1328 / 1316 (up to four workgroups per compute unit: 128
+// 2000 / 2030, 160 2789 / 2843).
+static int in_slices(int64_t tiles, int most, bool bits16) {
+  int s = 1;
+  while (s < most && tiles * (s + 1) <= (bits16 ? 256 : 900)) ++s;
+  return s;
+}
+
 template <typename T, typename TZ, int KS>
 static int pp_trimul_in_ks(ProjInParams p, const SingleStage* carry, hipStream_t stream) {
   const int rbw = sizeof(T) == 2 ? in_row_blocks((int64_t)p.n * p.n, KS, false) : 1;
@@ -736,7 +756,13 @@ static int pp_trimul_in_ks(ProjInParams p, const SingleStage* carry, hipStream_t
   if (carry && KS <= 4) single_stage_run(carry, stream);
   if (!carry || KS <= 4) carry = &none;
   const unsigned carried = single_stage_groups(carry);
-  const dim3 grid(carried + (unsigned)((p.n + 4 * rbw - 1) / (4 * rbw)) * (unsigned)(p.pitch / 8)), block(kPpWaves * 64);
+  const unsigned tiles = (unsigned)((p.n + 4 * rbw - 1) / (4 * rbw)) * (unsigned)(p.pitch / 8);
+  constexpr int kChunks = PpWidths<KS>::HIDDEN / 64;   // per wave
+  p.slices = in_slices(tiles, kChunks, sizeof(T) == 2);
+  if (kChunks % p.slices) --p.slices;   // (2 or 4 chunks: equal shares)
+  p.tiles = tiles;
+  p.share = kChunks / p.slices;
+  const dim3 grid(carried + tiles * p.slices), block(kPpWaves * 64);
   if constexpr (sizeof(T) == 2) {
     if (rbw == 4) {
       pp_trimul_in_kernel<T, TZ, KS, 4><<<grid, block, 0, stream>>>(p, *carry, carried);
@@ -795,7 +821,9 @@ static int pp_triattn_in_ks(ProjInParams p, const SingleStage* carry, hipStream_
   if (carry && KS <= 4) single_stage_run(carry, stream);
   if (!carry || KS <= 4) carry = &none;
   const unsigned carried = single_stage_groups(carry);
-  const dim3 grid(carried + (unsigned)tiles), block(kPpWaves * 64);
+  p.slices = in_slices(tiles, ((GATE ? 4 : 3) * PpWidths<KS>::HEADS / 2 + kPpWaves) / kPpWaves, sizeof(T) == 2);
+  p.tiles = (unsigned)tiles;
+  const dim3 grid(carried + p.tiles * p.slices), block(kPpWaves * 64);
   if constexpr (sizeof(T) == 2) {
     if constexpr (KS == 4) {
       if (rbw == 4) {
