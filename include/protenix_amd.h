@@ -34,7 +34,7 @@
 extern "C" {
 #endif
 
-#define PTX_ABI_VERSION 6
+#define PTX_ABI_VERSION 7
 #define PTX_API __attribute__((visibility("default")))
 
 /*
@@ -116,6 +116,13 @@ PTX_API int ptx_layernorm_fwd(const void* x, const void* gamma, const void* beta
  *   carry: NULL, or a stage of the single-representation track (ptx_single_*_stage, operands of
  *     the pair rows' storage type) that the launch runs along: on workgroups of its own, so it
  *     must not depend on this launch nor this launch on it.
+ *   ptx_trimul_contract_carry: ptx_trimul_contract_ld that carries a stage (of the pair rows' storage type: dtype PTX_MIXED
+ *     for fp32 rows), along its own workgroups where ptx_trimul_contract_carries says 1, else in a launch in front.
+ *   ptx_trimul_output_triattn_project, ptx_triattn_output_triattn_project: an output stage (residual added) and, of the rows it
+ *     stores, the projection that follows it in a block, in one launch: the incoming triangle multiplication and the starting
+ *     node, the starting and the ending node.  dtype PTX_BF16 or PTX_MIXED; the same bits as the two calls; q, k, vt,
+ *     tri_bias must not overlap x / o.  ptx_row_stages_joined: 1 where that is the faster way (attention: 0 for the
+ *     first, 1 for the second pair).
  *   ptx_row_stage_resident: 1 where the launch, if it carries nothing, takes a kernel that holds all weights
  *     in LDS and is the faster for it (it cannot carry).  stage: 0 trimul_project, 1 trimul_output,
  *     2 triattn_project, 3 triattn_output.
@@ -152,6 +159,20 @@ PTX_API int ptx_triattn_output_packed(const void* o, const void* z, const void* 
                       const void* packed, void* out, int n, int c_in, int heads, int transposed,
                       int add_residual, float eps, int dtype,
                       const ptx_single_stage* carry, void* stream);
+PTX_API int ptx_trimul_contract_carry(const void* a, const void* b, void* x, int n, int ldx, int c, int k_pitch, int dtype,
+                      const ptx_single_stage* carry, void* stream);
+PTX_API int ptx_trimul_contract_carries(int n, int dtype);
+PTX_API int ptx_row_stages_joined(int attention, int n, int c_z, int c_hidden, int dtype);
+PTX_API int ptx_trimul_output_triattn_project(const void* x, int ldx, const void* z, const void* ln_in_w,
+                      const void* ln_in_b, const void* ln_out_w, const void* ln_out_b, const void* packed,
+                      void* out, const void* att_ln_w, const void* att_ln_b, const void* att_packed, void* q,
+                      void* k, void* vt, void* tri_bias, int n, int c_z, int c_hidden, int heads,
+                      int key_pitch, float eps, int dtype, const ptx_single_stage* carry, void* stream);
+PTX_API int ptx_triattn_output_triattn_project(const void* o, const void* z, const void* ln_w, const void* ln_b,
+                      const void* packed, void* out, const void* next_ln_w, const void* next_ln_b,
+                      const void* next_packed, void* q, void* k, void* vt, void* tri_bias, int n, int c_in,
+                      int heads, int key_pitch, float eps, int dtype, const ptx_single_stage* carry,
+                      void* stream);
 
 /*
  * Parameters converted and laid out for the kernels, any number in one launch: dst[rows][cols] = src[rows][cols] in

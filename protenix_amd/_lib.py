@@ -14,7 +14,7 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libprotenix_amd.so")
 
 PTX_F32, PTX_BF16, PTX_MIXED, PTX_F16 = 0, 1, 2, 3
-ABI_VERSION = 6
+ABI_VERSION = 7
 
 _p = ctypes.c_void_p
 _i = ctypes.c_int
@@ -41,6 +41,11 @@ SIGNATURES = {
     "ptx_trimul_pack": (_i, [_p] * 7 + [_i, _i, _i, _p]),
     "ptx_trimul_project_packed": (_i, [_p] * 7 + [_i, _i, _i, _i, _i, _f, _i, _p, _p]),
     "ptx_trimul_contract_ld": (_i, [_p, _p, _p, _i, _i, _i, _i, _i, _p]),
+    "ptx_trimul_contract_carry": (_i, [_p, _p, _p, _i, _i, _i, _i, _i, _p, _p]),
+    "ptx_trimul_contract_carries": (_i, [_i, _i]),
+    "ptx_row_stages_joined": (_i, [_i, _i, _i, _i, _i]),
+    "ptx_trimul_output_triattn_project": (_i, [_p, _i] + [_p] * 14 + [_i, _i, _i, _i, _i, _f, _i, _p, _p]),
+    "ptx_triattn_output_triattn_project": (_i, [_p] * 13 + [_i, _i, _i, _i, _f, _i, _p, _p]),
     "ptx_trimul_output_packed": (_i, [_p, _i] + [_p] * 7 + [_i, _i, _i, _i, _f, _i, _p, _p]),
     "ptx_triattn_packed_elems": (_l, [_i, _i, _i]),
     "ptx_triattn_late_gate": (_i, [_i, _i, _i]),

@@ -235,8 +235,18 @@ PTX_API int ptx_trimul_contract(const void* a, const void* b, void* x, int n, in
   return ptx_trimul_contract_ld(a, b, x, n, n, c, k_pitch, dtype, stream);
 }
 
+static bool carry_ok(const ptx_single_stage* carry, int dtype);
+
 PTX_API int ptx_trimul_contract_ld(const void* a, const void* b, void* x, int n, int ldx, int c, int k_pitch,
                                    int dtype, void* stream) {
+  return ptx_trimul_contract_carry(a, b, x, n, ldx, c, k_pitch, dtype, nullptr, stream);
+}
+
+PTX_API int ptx_trimul_contract_carries(int n, int dtype) { return ptx::nt_gemm_carries(n, dtype != PTX_F32); }
+
+PTX_API int ptx_trimul_contract_carry(const void* a, const void* b, void* x, int n, int ldx, int c, int k_pitch, int dtype,
+                                      const ptx_single_stage* carry, void* stream) {
+  PTX_REQUIRE(carry_ok(carry, dtype), PTX_ERR_BAD_ARG, "trimul_contract: the carried stage must be of the pair tensor's type");
   if (dtype == PTX_MIXED) dtype = PTX_BF16;   // no residual-stream tensor here
   PTX_REQUIRE(dtype_ok(dtype), PTX_ERR_BAD_ARG, "trimul_contract: unknown dtype %d", dtype);
   PTX_REQUIRE(n >= 0 && c >= 0, PTX_ERR_BAD_ARG, "trimul_contract: n=%d c=%d", n, c);
@@ -245,12 +255,12 @@ PTX_API int ptx_trimul_contract_ld(const void* a, const void* b, void* x, int n,
   PTX_REQUIRE(n < 32768, PTX_ERR_UNSUPPORTED, "trimul_contract: n=%d too large", n);
   PTX_REQUIRE(ldx >= n && (ldx == n || ldx % 8 == 0), PTX_ERR_BAD_ARG,
               "trimul_contract: ldx=%d (n=%d, or a multiple of 8 above it)", ldx, n);
-  if (n == 0 || c == 0) return PTX_OK;
-  PTX_REQUIRE(a && b && x, PTX_ERR_BAD_ARG, "trimul_contract: null pointer");
+  if ((n == 0 || c == 0) && !carry) return PTX_OK;
+  PTX_REQUIRE((a && b && x) || n == 0 || c == 0, PTX_ERR_BAD_ARG, "trimul_contract: null pointer");
   PTX_REQUIRE(aligned16(a) && aligned16(b), PTX_ERR_BAD_ARG,
               "trimul_contract: a and b must be 16-byte aligned");
   PTX_DISPATCH(dtype, ptx::nt_gemm_batched<T>((const T*)a, (const T*)b, (T*)x, n, ldx, k_pitch, c,
-                                              (hipStream_t)stream));
+                                              (const ptx::SingleStage*)carry, (hipStream_t)stream));
   return after_launch("trimul_contract");
 }
 
@@ -550,6 +560,70 @@ PTX_API int ptx_triattn_output_packed(const void* o, const void* z, const void* 
                                                      add_residual, eps, (const ptx::SingleStage*)carry,
                                                    (hipStream_t)stream));
   return after_launch("triattn_output_packed");
+}
+
+PTX_API int ptx_row_stages_joined(int attention, int n, int c_z, int c_hidden, int dtype) {
+  return (dtype == PTX_BF16 || dtype == PTX_MIXED) && pair_width_ok(c_z, c_hidden, dtype) &&
+         ptx::pp_joined(attention != 0, n, c_z, c_hidden, dtype == PTX_BF16);
+}
+
+PTX_API int ptx_trimul_output_triattn_project(const void* x, int ldx, const void* z, const void* ln_in_w, const void* ln_in_b,
+                                              const void* ln_out_w, const void* ln_out_b, const void* packed, void* out,
+                                              const void* att_ln_w, const void* att_ln_b, const void* att_packed, void* q, void* k,
+                                              void* vt, void* tri_bias, int n, int c_z, int c_hidden, int heads, int key_pitch, float eps,
+                                              int dtype, const ptx_single_stage* carry, void* stream) {
+  PTX_REQUIRE(dtype == PTX_BF16 || dtype == PTX_MIXED, PTX_ERR_BAD_ARG, "trimul_output_triattn_project: dtype %d", dtype);
+  PTX_REQUIRE(n >= 0, PTX_ERR_BAD_ARG, "trimul_output_triattn_project: n=%d", n);
+  PTX_REQUIRE(pair_width_ok(c_z, c_hidden, dtype) && pair_width_ok(c_z, heads * 32, dtype) && ptx::pp_late_gate(c_z, heads, true),
+              PTX_ERR_UNSUPPORTED, "trimul_output_triattn_project: %s (got c_z=%d c_hidden=%d heads=%d)", kWidthMsg, c_z, c_hidden, heads);
+  PTX_REQUIRE(key_pitch == ptx_key_pitch(n), PTX_ERR_BAD_ARG, "trimul_output_triattn_project: key_pitch=%d, expected %d", key_pitch,
+              ptx_key_pitch(n));
+  PTX_REQUIRE(n <= 8192, PTX_ERR_UNSUPPORTED, "trimul_output_triattn_project: n=%d too large (8192 at most)", n);
+  PTX_REQUIRE(ldx >= n && ldx % 8 == 0, PTX_ERR_BAD_ARG, "trimul_output_triattn_project: ldx=%d (a multiple of 8, >= n=%d)", ldx, n);
+  if (n == 0) return PTX_OK;
+  PTX_REQUIRE(x && z && packed && out && att_packed && q && k && vt && tri_bias, PTX_ERR_BAD_ARG, "trimul_output_triattn_project: null pointer");
+  PTX_REQUIRE(aligned16(x) && aligned16(out) && aligned16(z) && aligned16(packed) && (!ln_out_w || aligned16(ln_out_w)) &&
+                  (!ln_out_b || aligned16(ln_out_b)) && (!ln_in_w || aligned16(ln_in_w)) && (!ln_in_b || aligned16(ln_in_b)) &&
+                  aligned16(att_packed) && aligned16(q) && aligned16(k) && aligned16(vt) && aligned16(tri_bias) &&
+                  (!att_ln_w || aligned16(att_ln_w)) && (!att_ln_b || aligned16(att_ln_b)),
+              PTX_ERR_BAD_ARG, "trimul_output_triattn_project: pointers must be 16-byte aligned");
+  PTX_REQUIRE(carry_ok(carry, dtype), PTX_ERR_BAD_ARG, "trimul_output_triattn_project: the carried stage must be of the pair tensor's type");
+  if (dtype == PTX_MIXED)
+    ptx::pp_trimul_out_triattn_in<float>(x, ldx, z, ln_in_w, ln_in_b, ln_out_w, ln_out_b, packed, out, att_ln_w, att_ln_b, att_packed, q, k, vt,
+                                         tri_bias, n, c_z, c_hidden, heads, key_pitch, eps, (const ptx::SingleStage*)carry, (hipStream_t)stream);
+  else
+    ptx::pp_trimul_out_triattn_in<ptx::bf16_t>(x, ldx, z, ln_in_w, ln_in_b, ln_out_w, ln_out_b, packed, out, att_ln_w, att_ln_b, att_packed, q,
+                                               k, vt, tri_bias, n, c_z, c_hidden, heads, key_pitch, eps, (const ptx::SingleStage*)carry,
+                                               (hipStream_t)stream);
+  return after_launch("trimul_output_triattn_project");
+}
+
+PTX_API int ptx_triattn_output_triattn_project(const void* o, const void* z, const void* ln_w, const void* ln_b, const void* packed,
+                                               void* out, const void* next_ln_w, const void* next_ln_b, const void* next_packed, void* q,
+                                               void* k, void* vt, void* tri_bias, int n, int c_in, int heads, int key_pitch, float eps,
+                                               int dtype, const ptx_single_stage* carry, void* stream) {
+  PTX_REQUIRE(dtype == PTX_BF16 || dtype == PTX_MIXED, PTX_ERR_BAD_ARG, "triattn_output_triattn_project: dtype %d", dtype);
+  PTX_REQUIRE(n >= 0, PTX_ERR_BAD_ARG, "triattn_output_triattn_project: n=%d", n);
+  PTX_REQUIRE(heads > 0 && heads <= 8 && pair_width_ok(c_in, heads * 32, dtype) && ptx::pp_late_gate(c_in, heads, true), PTX_ERR_UNSUPPORTED,
+              "triattn_output_triattn_project: %s (got c_in=%d heads=%d)", kWidthMsg, c_in, heads);
+  PTX_REQUIRE(key_pitch == ptx_key_pitch(n), PTX_ERR_BAD_ARG, "triattn_output_triattn_project: key_pitch=%d, expected %d", key_pitch,
+              ptx_key_pitch(n));
+  PTX_REQUIRE(n <= 8192, PTX_ERR_UNSUPPORTED, "triattn_output_triattn_project: n=%d too large (8192 at most)", n);
+  if (n == 0) return PTX_OK;
+  PTX_REQUIRE(o && z && packed && out && next_packed && q && k && vt && tri_bias, PTX_ERR_BAD_ARG, "triattn_output_triattn_project: null pointer");
+  PTX_REQUIRE(o != q && o != k && o != vt, PTX_ERR_BAD_ARG, "triattn_output_triattn_project: o must not be one of the outputs");
+  PTX_REQUIRE(aligned16(o) && aligned16(z) && aligned16(packed) && aligned16(out) && (!ln_w || aligned16(ln_w)) && (!ln_b || aligned16(ln_b)) &&
+                  aligned16(next_packed) && aligned16(q) && aligned16(k) && aligned16(vt) && aligned16(tri_bias) &&
+                  (!next_ln_w || aligned16(next_ln_w)) && (!next_ln_b || aligned16(next_ln_b)),
+              PTX_ERR_BAD_ARG, "triattn_output_triattn_project: pointers must be 16-byte aligned");
+  PTX_REQUIRE(carry_ok(carry, dtype), PTX_ERR_BAD_ARG, "triattn_output_triattn_project: the carried stage must be of the pair tensor's type");
+  if (dtype == PTX_MIXED)
+    ptx::pp_triattn_out_triattn_in<float>(o, z, ln_w, ln_b, packed, out, next_ln_w, next_ln_b, next_packed, q, k, vt, tri_bias, n, c_in, heads,
+                                          key_pitch, eps, (const ptx::SingleStage*)carry, (hipStream_t)stream);
+  else
+    ptx::pp_triattn_out_triattn_in<ptx::bf16_t>(o, z, ln_w, ln_b, packed, out, next_ln_w, next_ln_b, next_packed, q, k, vt, tri_bias, n, c_in,
+                                                heads, key_pitch, eps, (const ptx::SingleStage*)carry, (hipStream_t)stream);
+  return after_launch("triattn_output_triattn_project");
 }
 
 PTX_API int64_t ptx_triattn_core_workspace_elems(int n_rows, int s, int heads) {

@@ -404,6 +404,25 @@ int64_t workspace_bytes(int n, int c_h, int heads, int64_t es) {
   if (heads) TriAttWs(a, n, heads, es);
   return std::max(m.used, a.used);
 }
+// The same for updates whose output stage also projects for the next one (no gate tensors): what such a launch reads,
+// x or o, lies apart from what it writes.
+struct ChainWs {
+  void *a, *b, *x, *q, *k, *vt, *tb, *o;
+  ChainWs(Cut& c, int n, int c_h, int heads, int64_t es) {
+    const int64_t ab = ptx_trimul_operand_elems(n, c_h) * es, row = (int64_t)heads * n * n * 32 * es;
+    const int64_t kv = ptx_triattn_kv_elems(n, heads) * es;
+    a = q = c.part(std::max(ab, row));
+    b = k = c.part(std::max(ab, kv));
+    vt = c.part(kv);
+    tb = c.part(ptx_triattn_bias_elems(n, heads) * es);
+    x = o = c.part(std::max((int64_t)c_h * n * ((n + 7) / 8 * 8) * es, row));
+  }
+};
+int64_t chain_bytes(int n, int c_h, int heads, int64_t es) {
+  Cut c{nullptr};
+  ChainWs(c, n, c_h, heads, es);
+  return c.used;
+}
 
 constexpr float kEps = 1e-5f;
 
@@ -459,14 +478,18 @@ struct Run {
   // five launches for the five other stages, on 16-bit rows it may be both, and stages left over are
   // launched.  us per block with a single track, always carrying / so: fp32 rows, 512 tokens 1107 / 1092, 640 1814 / 1785, 768
   // 2615 / 2595, 1024 5090 / 5047, 2048 28073 / 27832; 16-bit rows, 768 2403 / 2339, 1024 4656 / 4517, 1536 12661 / 12403.
-  bool mul_alone = false, att_alone = false;
+  // Chained updates (Block::chain) have two launches fewer to carry: small products carry then, elsewhere the LayerNorms
+  // are launched by themselves too.
+  bool mul_alone = false, att_alone = false, contract_carries = false, chained = false;
   void row_stages(int n, int c_z, int hidden, int dt) {
     mul_alone = ptx_row_stage_resident(0, n, c_z, hidden, dt);
     att_alone = n >= 480 && ptx_row_stage_resident(2, n, c_z, hidden, dt);
+    contract_carries = ptx_trimul_contract_carries(n, dt);
   }
+  // stage 4: of the contractions, which take part where the updates are chained (two launches fewer to carry)
   const ptx_single_stage* carry(int stage) {
-    if ((stage == 0 && mul_alone) || (stage == 2 && att_alone)) return nullptr;
-    if ((mul_alone || att_alone) && singles.next < singles.list.size() && singles.list[singles.next].layernorm) run_next();
+    if ((stage == 0 && mul_alone) || (stage == 2 && att_alone) || (stage == 4 && !(chained && contract_carries))) return nullptr;
+    if ((mul_alone || att_alone || (chained && !contract_carries)) && singles.next < singles.list.size() && singles.list[singles.next].layernorm) run_next();
     return singles.take();
   }
   void run_next() {
@@ -490,51 +513,67 @@ struct Run {
   }
 };
 
+// projection and product; the product is left in x
+void run_trimul_product(const TriMul& w, const void* z, const Tensor& mask, int n, int dt, void* a, void* b, void* x, Run& run) {
+  const int pitch = ptx_key_pitch(n), ldx = (n + 7) / 8 * 8;
+  const ptx_single_stage* carry0 = run.carry(0);
+  run.launch("trimul_project", [&] {
+    return ptx_trimul_project_packed(z, ptr(mask), w.ln_in_w, w.ln_in_b, w.packed, a, b, n, w.c_z, w.c_h, pitch,
+                                     w.incoming, kEps, dt, carry0, run.st);
+  });
+  const ptx_single_stage* carry4 = run.carry(4);
+  run.launch("trimul_contract", [&] { return ptx_trimul_contract_carry(a, b, x, n, ldx, w.c_h, pitch, dt, carry4, run.st); });
+}
+
+void run_trimul_output(const TriMul& w, const void* x, const void* z, void* out, int n, bool add, int dt, Run& run) {
+  const ptx_single_stage* carry1 = run.carry(1);
+  run.launch("trimul_output", [&] {
+    return ptx_trimul_output_packed(x, (n + 7) / 8 * 8, z, w.ln_in_w, w.ln_in_b, w.ln_out_w, w.ln_out_b, w.packed, out,
+                                    n, w.c_z, w.c_h, add, kEps, dt, carry1, run.st);
+  });
+}
+
 void run_trimul(const TriMul& w, const void* z, const Tensor& mask, void* out, int n, bool add, int dt, int64_t es, void* ws,
                 Run& run) {
   Cut c{(char*)ws};
   TriMulWs s(c, n, w.c_h, es);
-  const int pitch = ptx_key_pitch(n), ldx = (n + 7) / 8 * 8;
-  const ptx_single_stage* carry0 = run.carry(0);
-  run.launch("trimul_project", [&] {
-    return ptx_trimul_project_packed(z, ptr(mask), w.ln_in_w, w.ln_in_b, w.packed, s.a, s.b, n, w.c_z, w.c_h, pitch,
-                                     w.incoming, kEps, dt, carry0, run.st);
-  });
-  run.launch("trimul_contract", [&] { return ptx_trimul_contract_ld(s.a, s.b, s.x, n, ldx, w.c_h, pitch, dt, run.st); });
-  const ptx_single_stage* carry1 = run.carry(1);
-  run.launch("trimul_output", [&] {
-    return ptx_trimul_output_packed(s.x, ldx, z, w.ln_in_w, w.ln_in_b, w.ln_out_w, w.ln_out_b, w.packed, out,
-                                    n, w.c_z, w.c_h, add, kEps, dt, carry1, run.st);
-  });
+  run_trimul_product(w, z, mask, n, dt, s.a, s.b, s.x, run);
+  run_trimul_output(w, s.x, z, out, n, add, dt, run);
+}
+
+// the attention of projected operands, gated unless the gate is null, into o
+void run_attention(const TriAtt& w, const void* q, const void* k, const void* vt, const void* gate, const void* tb, void* o, const Mask& mask,
+                   int n, int dt, Run& run) {
+  const int pitch = ptx_key_pitch(n);
+  const void* m = ptr(w.transposed ? mask.mt : mask.m);
+  if (m && mask.n_valid >= 0) {
+    // padding at the end: valid rows over valid keys without a mask, padded rows with it (ops.py)
+    run.launch("triattn_fwd", [&] {
+      return ptx_triattn_fwd_rows(q, k, vt, gate, tb, nullptr, o, n, w.heads, 32, pitch, 0, w.inf, 0, mask.n_valid,
+                                  mask.n_valid, dt, run.st);
+    });
+    run.launch("triattn_fwd_padded_rows", [&] {
+      return ptx_triattn_fwd_rows(q, k, vt, gate, tb, m, o, n, w.heads, 32, pitch, 0, w.inf, mask.n_valid, n - mask.n_valid, n,
+                                  dt, run.st);
+    });
+  } else {
+    run.launch("triattn_fwd", [&] {
+      return ptx_triattn_fwd(q, k, vt, gate, tb, m, o, n, w.heads, 32, pitch, 0, w.inf, dt, run.st);
+    });
+  }
 }
 
 // projection and core; the attention output is left in ws.g
 TriAttWs run_triatt_core(const TriAtt& w, const void* z, const Mask& mask, int n, int dt, int64_t es, void* ws, Run& run) {
   Cut c{(char*)ws};
   TriAttWs s(c, n, w.heads, es);
-  const int pitch = ptx_key_pitch(n);
   void* gate = ptx_triattn_late_gate(w.c, w.heads, dt) ? nullptr : s.g;
   const ptx_single_stage* carry2 = run.carry(2);
   run.launch("triattn_project", [&] {
-    return ptx_triattn_project_packed(z, w.ln_w, w.ln_b, w.packed, s.q, s.k, s.vt, gate, s.tb, n, w.c, w.heads, pitch,
+    return ptx_triattn_project_packed(z, w.ln_w, w.ln_b, w.packed, s.q, s.k, s.vt, gate, s.tb, n, w.c, w.heads, ptx_key_pitch(n),
                                       w.transposed, kEps, dt, carry2, run.st);
   });
-  const void* m = ptr(w.transposed ? mask.mt : mask.m);
-  if (m && mask.n_valid >= 0) {
-    // padding at the end: valid rows over valid keys without a mask, padded rows with it (ops.py)
-    run.launch("triattn_fwd", [&] {
-      return ptx_triattn_fwd_rows(s.q, s.k, s.vt, gate, s.tb, nullptr, s.g, n, w.heads, 32, pitch, 0, w.inf, 0, mask.n_valid,
-                                  mask.n_valid, dt, run.st);
-    });
-    run.launch("triattn_fwd_padded_rows", [&] {
-      return ptx_triattn_fwd_rows(s.q, s.k, s.vt, gate, s.tb, m, s.g, n, w.heads, 32, pitch, 0, w.inf, mask.n_valid, n - mask.n_valid, n,
-                                  dt, run.st);
-    });
-  } else {
-    run.launch("triattn_fwd", [&] {
-      return ptx_triattn_fwd(s.q, s.k, s.vt, gate, s.tb, m, s.g, n, w.heads, 32, pitch, 0, w.inf, dt, run.st);
-    });
-  }
+  run_attention(w, s.q, s.k, s.vt, gate, s.tb, s.g, mask, n, dt, run);
   return s;
 }
 
@@ -646,25 +685,34 @@ struct Block : Plan {
     char* zp = (char*)z.data_ptr();
     static const Mask none;
     auto mask = [&](int64_t b) -> const Mask& { return masks.empty() ? none : masks[b]; };
-    for (int64_t b = 0; b < batch; ++b) run_trimul(out, zp + b * plane, mask(b).m, zp + b * plane, n, true, dt, es, ws, run);
-    for (int64_t b = 0; b < batch; ++b) run_trimul(in, zp + b * plane, mask(b).m, zp + b * plane, n, true, dt, es, ws, run);
-    for (int64_t b = 0; b < batch; ++b) run_triatt(start, zp + b * plane, mask(b), zp + b * plane, n, true, dt, es, ws, run);
     const int64_t bias_plane = (int64_t)heads * n * n;
-    if (fused) {
+    if (run.chained) {
       for (int64_t b = 0; b < batch; ++b) {
         void* zb = zp + b * plane;
-        const TriAttWs s = run_triatt_core(end, zb, mask(b), n, dt, es, ws, run);
-        if (b == 0) run.run_rest();   // (the bias is about to be rewritten)
-        run.launch("triattn_output_transition", [&] {
-          return ptx_triattn_output_transition_fwd(s.g, zb, end.ln_w, end.ln_b, tr_packed, tr_ln_w, tr_ln_b, zb, n,
-                                                   c_z, end.heads, end.transposed, n_factor, kEps, kEps, bias ? pb_ln_w : nullptr,
-                                                   bias ? pb_ln_b : nullptr, bias ? pb_w : nullptr,
-                                                   bias ? bias + b * bias_plane : nullptr, bias ? heads : 0, 1, kEps, dt, run.st);
-        });
+        chain(zb, mask(b), n, dt, es, ws, run);
+        if (fused) {
+          if (b == 0) run.run_rest();   // (the bias is about to be rewritten)
+          output_transition(zb, attention_output(n, es, ws), n, dt, bias ? bias + b * bias_plane : nullptr, run);
+        } else {
+          output(end, zb, attention_output(n, es, ws), n, dt, run);
+        }
       }
-      return;
+      if (fused) return;
+    } else {
+      for (int64_t b = 0; b < batch; ++b) run_trimul(out, zp + b * plane, mask(b).m, zp + b * plane, n, true, dt, es, ws, run);
+      for (int64_t b = 0; b < batch; ++b) run_trimul(in, zp + b * plane, mask(b).m, zp + b * plane, n, true, dt, es, ws, run);
+      for (int64_t b = 0; b < batch; ++b) run_triatt(start, zp + b * plane, mask(b), zp + b * plane, n, true, dt, es, ws, run);
+      if (fused) {
+        for (int64_t b = 0; b < batch; ++b) {
+          void* zb = zp + b * plane;
+          const TriAttWs s = run_triatt_core(end, zb, mask(b), n, dt, es, ws, run);
+          if (b == 0) run.run_rest();   // (the bias is about to be rewritten)
+          output_transition(zb, s.g, n, dt, bias ? bias + b * bias_plane : nullptr, run);
+        }
+        return;
+      }
+      for (int64_t b = 0; b < batch; ++b) run_triatt(end, zp + b * plane, mask(b), zp + b * plane, n, true, dt, es, ws, run);
     }
-    for (int64_t b = 0; b < batch; ++b) run_triatt(end, zp + b * plane, mask(b), zp + b * plane, n, true, dt, es, ws, run);
     run.run_rest();   // (the bias is about to be rewritten)
     run.launch("transition", [&] {
       return ptx_transition_fwd(zp, tr_ln_w, tr_ln_b, tr_packed, zp, batch * n * n, c_z, n_factor, 1, kEps, dt, run.st);
@@ -675,6 +723,66 @@ struct Block : Plan {
           return ptx_pair_bias_fwd(zp + b * plane, pb_ln_w, pb_ln_b, pb_w, bias + b * bias_plane, n, c_z, heads, 1, kEps, dt,
                                    run.st);
         });
+  }
+
+  // Whether an output stage projects for the update behind it (16-bit arithmetic; not where launches are timed one by one).
+  bool chains(const Run& run, int n, int dt) const {
+    return !run.timing && out.c_h == in.c_h && start.heads == end.heads && ptx_triattn_late_gate(c_z, start.heads, dt) &&
+           ptx_row_stages_joined(0, n, c_z, out.c_h, dt);
+  }
+  // The block up to the ending node's attention output.
+  void chain(void* z, const Mask& mask, int n, int dt, int64_t es, void* ws, Run& run) const {
+    Cut c{(char*)ws};
+    const ChainWs s(c, n, out.c_h, start.heads, es);
+    const int ldx = (n + 7) / 8 * 8, pitch = ptx_key_pitch(n);
+    run_trimul_product(out, z, mask.m, n, dt, s.a, s.b, s.x, run);
+    run_trimul_output(out, s.x, z, z, n, true, dt, run);
+    run_trimul_product(in, z, mask.m, n, dt, s.a, s.b, s.x, run);
+    const ptx_single_stage* carry1 = run.carry(1);
+    run.launch("trimul_output_triattn_project", [&] {
+      return ptx_trimul_output_triattn_project(s.x, ldx, z, in.ln_in_w, in.ln_in_b, in.ln_out_w, in.ln_out_b, in.packed, z, start.ln_w,
+                                               start.ln_b, start.packed, s.q, s.k, s.vt, s.tb, n, c_z, in.c_h, start.heads, pitch, kEps, dt,
+                                               carry1, run.st);
+    });
+    run_attention(start, s.q, s.k, s.vt, nullptr, s.tb, s.o, mask, n, dt, run);
+    if (ptx_row_stages_joined(1, n, c_z, out.c_h, dt)) {
+      const ptx_single_stage* carry3 = run.carry(3);
+      run.launch("triattn_output_triattn_project", [&] {
+        return ptx_triattn_output_triattn_project(s.o, z, start.ln_w, start.ln_b, start.packed, z, end.ln_w, end.ln_b, end.packed, s.q, s.k,
+                                                  s.vt, s.tb, n, c_z, start.heads, pitch, kEps, dt, carry3, run.st);
+      });
+    } else {
+      output(start, z, s.o, n, dt, run);
+      project(end, z, s, n, dt, run);
+    }
+    run_attention(end, s.q, s.k, s.vt, nullptr, s.tb, s.o, mask, n, dt, run);
+  }
+  void project(const TriAtt& w, const void* z, const ChainWs& s, int n, int dt, Run& run) const {
+    const ptx_single_stage* carry2 = run.carry(2);
+    run.launch("triattn_project", [&] {
+      return ptx_triattn_project_packed(z, w.ln_w, w.ln_b, w.packed, s.q, s.k, s.vt, nullptr, s.tb, n, w.c, w.heads, ptx_key_pitch(n),
+                                        w.transposed, kEps, dt, carry2, run.st);
+    });
+  }
+  const void* attention_output(int n, int64_t es, void* ws) const {
+    Cut c{(char*)ws};
+    return ChainWs(c, n, out.c_h, start.heads, es).o;
+  }
+  void output(const TriAtt& w, void* z, const void* o, int n, int dt, Run& run) const {
+    const ptx_single_stage* carry3 = run.carry(3);
+    run.launch("triattn_output", [&] {
+      return ptx_triattn_output_packed(o, z, w.ln_w, w.ln_b, w.packed, z, n, w.c, w.heads, w.transposed, true, kEps, dt,
+                                       carry3, run.st);
+    });
+  }
+  // the ending node's output stage and the transition, with the pair bias where one is wanted
+  void output_transition(void* z, const void* o, int n, int dt, float* bias, Run& run) const {
+    run.launch("triattn_output_transition", [&] {
+      return ptx_triattn_output_transition_fwd(o, z, end.ln_w, end.ln_b, tr_packed, tr_ln_w, tr_ln_b, z, n,
+                                               c_z, end.heads, end.transposed, n_factor, kEps, kEps, bias ? pb_ln_w : nullptr,
+                                               bias ? pb_ln_b : nullptr, bias ? pb_w : nullptr, bias,
+                                               bias ? heads : 0, 1, kEps, dt, run.st);
+    });
   }
 
   // bytes single_track() wants as scratch
@@ -754,7 +862,9 @@ struct Call {
       make_room(*b);
       const bool single = b->c_s > 0;
       float* bias = single ? (float*)bias_.data_ptr() : nullptr;
-      run_.row_stages(n_, b->c_z, b->out.c_h, code_of_rows(z_.scalar_type(), b->compute));
+      const int dt = code_of_rows(z_.scalar_type(), b->compute);
+      run_.row_stages(n_, b->c_z, b->out.c_h, dt);
+      run_.chained = b->chains(run_, n_, dt);
       b->pair_track(z_, masks_, batch_, n_, ws_.data_ptr(), bias, run_);
       if (single) {
         b->single_track(run_.singles, s_now_, mid_.data_ptr(), s_out_.data_ptr(), bias, s_->scalar_type(), batch_, n_, sws_.data_ptr());
@@ -775,7 +885,9 @@ struct Call {
 
  private:
   void make_room(const Block& b) {
-    enlarge(ws_, workspace_bytes(n_, std::max(b.out.c_h, b.in.c_h), std::max(b.start.heads, b.end.heads), at::elementSize(b.compute)));
+    const int c_h = std::max(b.out.c_h, b.in.c_h), pair_heads = std::max(b.start.heads, b.end.heads);
+    const int64_t es = at::elementSize(b.compute);
+    enlarge(ws_, std::max(workspace_bytes(n_, c_h, pair_heads, es), chain_bytes(n_, c_h, pair_heads, es)));
     if (b.c_s == 0) return;
     enlarge(bias_, batch_ * b.heads * (int64_t)n_ * n_ * 4);
     enlarge(sws_, b.single_bytes(batch_, n_, (int64_t)s_->element_size()));

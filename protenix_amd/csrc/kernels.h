@@ -119,6 +119,12 @@ void single_stage_attention(SingleStage* s, const void* q, const void* k, const 
                             float scale, bool bits16);
 int single_stage_run(const SingleStage* s, hipStream_t stream);
 
+// carry: null, or a stage of the single track that the launch's first workgroups run (it must not depend on the launch), where
+// nt_gemm_carries(); elsewhere the stage is launched in front.
+bool nt_gemm_carries(int n, bool bits16);
+template <typename T>
+int nt_gemm_batched(const T* a, const T* b, T* x, int n, int ldx, int k_pitch, int batch, const SingleStage* carry, hipStream_t stream);
+
 // A parameter on its way into the kernels (params.hip): src, dst bf16 or fp32 as the flags say, dst [rows][cols] like src or,
 // fragments, in the order of a linear stage's packed weights (rows % 16 == 0, cols % 32 == 0).
 struct Param {
@@ -161,12 +167,27 @@ template <typename T, typename TZ = T>
 int pp_triattn_out(const void* o, const void* z, const void* ln_w, const void* ln_b, const void* packed, void* out,
                    int n, int c_z, int heads, int transposed, int add_residual, float eps, const SingleStage* carry,
                    hipStream_t stream);
+// Whether a triangle multiplication's (attention: a starting node's) output stage and the projection behind it are faster in
+// one launch, in 16-bit arithmetic.
+bool pp_joined(bool attention, int n, int c_z, int hidden, bool rows16);
+// An output stage and the projection of the attention that reads its rows next, in one launch (16-bit arithmetic, residual
+// added; the projection writes no gate): the incoming triangle multiplication -> the starting node, the starting -> the
+// ending node.
+template <typename TZ>
+int pp_trimul_out_triattn_in(const void* x, int ldx, const void* z, const void* ln_in_w, const void* ln_in_b, const void* ln_out_w,
+                             const void* ln_out_b, const void* packed, void* out, const void* att_ln_w, const void* att_ln_b,
+                             const void* att_packed, void* q, void* k, void* vt, void* tri_bias, int n, int c_z, int hidden, int heads,
+                             int key_pitch, float eps, const SingleStage* carry, hipStream_t stream);
+template <typename TZ>
+int pp_triattn_out_triattn_in(const void* o, const void* z, const void* ln_w, const void* ln_b, const void* packed, void* out,
+                              const void* next_ln_w, const void* next_ln_b, const void* next_packed, void* q, void* k, void* vt,
+                              void* tri_bias, int n, int c_z, int heads, int key_pitch, float eps, const SingleStage* carry,
+                              hipStream_t stream);
+
 
 // x[c][i][j] = sum_k a[c][i][k] * b[c][j][k] for `batch` independent products;
 // a, b rows have pitch k_pitch (a multiple of 64, >= n), x is [batch][n][ldx].
-template <typename T>
-int nt_gemm_batched(const T* a, const T* b, T* x, int n, int ldx, int k_pitch, int batch,
-                    hipStream_t stream);
+
 
 // Flash-style triangle attention core (see triattn.hip).
 template <typename T>

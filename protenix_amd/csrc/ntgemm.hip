@@ -40,6 +40,7 @@
 
 #include "common.h"
 #include "kernels.h"
+#include "single_stage.h"
 
 namespace ptx {
 
@@ -327,9 +328,9 @@ __global__ __launch_bounds__(256) void nt_gemm_batched_kernel(const T* __restric
 // channels c = 8 q + xcd, all tiles of one in a row (see above).
 struct ChannelTile {
   int c, tile;
-  __device__ explicit ChannelTile(int tiles) {
-    const int local = blockIdx.x >> 3, q = local / tiles;
-    c = q * 8 + (blockIdx.x & 7);
+  __device__ ChannelTile(unsigned block, int tiles) {
+    const int local = block >> 3, q = local / tiles;
+    c = q * 8 + (block & 7);
     tile = local - q * tiles;
   }
 };
@@ -340,18 +341,27 @@ struct ChannelTile {
 // bytes per product grow as the tile shrinks: 768 tokens by itself, 128 channels, tiles 64 x 64 / 128 x 128 / 128 x 256 / 192 x
 // 192 / 256 x 256 (the kernel above): 237 / 160 / 141 / 133 / 137 us.  Small tensors are chains of
 // latencies: 93 tokens 8.4 (above) -> 3.1 us, 128 tokens 8.9 -> 3.6, 200 tokens 12.8 -> 9.3.
-template <int RM, int RN>
+// TS: the launch's first `carried` workgroups run a stage of the single track on operands of that type (void: none).
+template <int RM, int RN, typename TS>
 __global__ __launch_bounds__(256) void nt_gemm_ring_kernel(const bf16_t* __restrict__ a, const bf16_t* __restrict__ b,
                                                            bf16_t* __restrict__ x, int n, int ldx, int k_pitch, int batch,
-                                                           int tiles, int tiles_j) {
+                                                           int tiles, int tiles_j, SingleStage carry, unsigned carried) {
   typedef Vec8<bf16_t>::type V8;
   constexpr int KK = 2, NBUF = 3, NRUN = 2 * (RM + RN), RUNS = NRUN / 4;   // runs: (operand, row block), KK fragments each
   constexpr int kFragBytes = kFragElems * (int)sizeof(bf16_t);
   static_assert(NRUN % 4 == 0, "the same number of loads for each of the four waves");
-  __shared__ u32x4_t lds_f[NBUF][NRUN * KK][kWave];
+  constexpr bool kCarries = !std::is_void<TS>::value;
+  constexpr int kBufs = kCarries ? std::max(NBUF, (kStageLds + NRUN * KK * 1024 - 1) / (NRUN * KK * 1024)) : NBUF;
+  __shared__ u32x4_t lds_f[kBufs][NRUN * KK][kWave];
+  if constexpr (kCarries) {
+    if (blockIdx.x < carried) {
+      single_stage<TS>(carry, blockIdx.x, reinterpret_cast<char*>(lds_f));
+      return;
+    }
+  }
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int ln = lane & 31, g = lane >> 5, wi = wave >> 1, wj = wave & 1;
-  const ChannelTile w(tiles);
+  const ChannelTile w(blockIdx.x - carried, tiles);
   if (w.c >= batch) return;
   const int ti = w.tile / tiles_j, tj = w.tile - ti * tiles_j;
   // (K steps that hold nothing but the zeros up to k_pitch are left out: a multiple of 64, so stages of 32 fit)
@@ -424,7 +434,7 @@ __global__ __launch_bounds__(256) void nt_gemm_direct_kernel(const float* __rest
   typedef Vec8<float>::type V8;
   constexpr int U = 2;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const ChannelTile w(tiles);
+  const ChannelTile w(blockIdx.x, tiles);
   const int n_rb = (n + 31) >> 5, n_ks = k_pitch >> 4, steps = (n + 15) >> 4;
   const int ib = (w.tile / tiles_j) * 2 + (wave >> 1), jb = (w.tile % tiles_j) * 2 + (wave & 1);
   if (w.c >= batch || ib >= n_rb || jb >= n_rb) return;
@@ -482,21 +492,35 @@ static int contraction_grid() {
 // 57 / 51 / 42, 600 204 / 176 / 182, 768 259 / 279 / 267.  Both triangle multiplications of bf16 rows, persistent / the better of
 // the other two: 576 473 / 430, 600 520 / 503, 768 749 / 772, 832 983 / 976, 960 1248 / 1253, 1056 1725 / 1624, 1344 2815 / 2643, 1632 4380 / 4405.
 template <int RM, int RN>
-static void launch_ring(const bf16_t* a, const bf16_t* b, bf16_t* x, int n, int ldx, int k_pitch, int batch, hipStream_t stream) {
+static void launch_ring(const bf16_t* a, const bf16_t* b, bf16_t* x, int n, int ldx, int k_pitch, int batch, const SingleStage* carry,
+                        hipStream_t stream) {
   const int tiles_i = (n + 64 * RM - 1) / (64 * RM), tiles_j = (n + 64 * RN - 1) / (64 * RN), tiles = tiles_i * tiles_j;
-  nt_gemm_ring_kernel<RM, RN><<<dim3((unsigned)((batch + 7) / 8 * 8 * tiles)), dim3(256), 0, stream>>>(a, b, x, n, ldx, k_pitch, batch, tiles,
-                                                                                                      tiles_j);
+  const unsigned carried = single_stage_groups(carry), groups = (unsigned)((batch + 7) / 8 * 8 * tiles);
+  if constexpr (RM * RN <= 4) {
+    if (carried) {
+      if (carry->bits16)
+        nt_gemm_ring_kernel<RM, RN, bf16_t><<<dim3(carried + groups), dim3(256), 0, stream>>>(a, b, x, n, ldx, k_pitch, batch, tiles, tiles_j,
+                                                                                             *carry, carried);
+      else
+        nt_gemm_ring_kernel<RM, RN, float><<<dim3(carried + groups), dim3(256), 0, stream>>>(a, b, x, n, ldx, k_pitch, batch, tiles, tiles_j,
+                                                                                            *carry, carried);
+      return;
+    }
+  }
+  nt_gemm_ring_kernel<RM, RN, void><<<dim3(groups), dim3(256), 0, stream>>>(a, b, x, n, ldx, k_pitch, batch, tiles, tiles_j, SingleStage{}, 0u);
 }
-static bool ring_takes(const bf16_t* a, const bf16_t* b, bf16_t* x, int n, int ldx, int k_pitch, int batch, hipStream_t stream) {
+bool nt_gemm_carries(int n, bool bits16) { return bits16 && n <= 256; }
+static bool ring_takes(const bf16_t* a, const bf16_t* b, bf16_t* x, int n, int ldx, int k_pitch, int batch, const SingleStage* carry,
+                       hipStream_t stream) {
   // us, persistent / 64 x 64 / 128 x 128 (128 channels): n = 64 6.7 / 2.5 / 3.3, 160 10.9 / 6.3 / 6.6, 192 11.2 / 7.7 / 8.1, 224 13.1 / 10.3 / 9.4,
   // 256 14.6 / 12.3 / 10.6; 256 channels: 128 10.6 / - / 6.6, 224 19.2 / - / 15.8, 256 24.4 / - / 24.7
-  if (n <= 192) return launch_ring<1, 1>(a, b, x, n, ldx, k_pitch, batch, stream), true;
-  if (n <= 256) return launch_ring<2, 2>(a, b, x, n, ldx, k_pitch, batch, stream), true;
+  if (n <= 192) return launch_ring<1, 1>(a, b, x, n, ldx, k_pitch, batch, carry, stream), true;
+  if (n <= 256) return launch_ring<2, 2>(a, b, x, n, ldx, k_pitch, batch, carry, stream), true;
   auto tiles = [n](int ti, int tj) { return (double)((n + ti - 1) / ti) * ((n + tj - 1) / tj); };
   const double whole = tiles(256, 256), wide = 0.58 * tiles(128, 256), square = 0.64 * tiles(192, 192);
   if (whole <= wide && whole <= square) return false;
-  if (wide < square) launch_ring<2, 4>(a, b, x, n, ldx, k_pitch, batch, stream);
-  else launch_ring<3, 3>(a, b, x, n, ldx, k_pitch, batch, stream);
+  if (wide < square) launch_ring<2, 4>(a, b, x, n, ldx, k_pitch, batch, nullptr, stream);
+  else launch_ring<3, 3>(a, b, x, n, ldx, k_pitch, batch, nullptr, stream);
   return true;
 }
 // fp32: a tile of the persistent kernel costs what 215 x 215 results cost the direct one (us, 128 channels: n = 384 208 / 171, 512
@@ -510,11 +534,15 @@ static bool direct_takes(const float* a, const float* b, float* x, int n, int ld
 }
 
 template <typename T>
-int nt_gemm_batched(const T* a, const T* b, T* x, int n, int ldx, int k_pitch, int batch,
+int nt_gemm_batched(const T* a, const T* b, T* x, int n, int ldx, int k_pitch, int batch, const SingleStage* carry,
                     hipStream_t stream) {
+  if (carry && (n == 0 || batch == 0 || !nt_gemm_carries(n, sizeof(T) == 2))) {
+    single_stage_run(carry, stream);
+    carry = nullptr;
+  }
   if (n == 0 || batch == 0) return 0;
   if constexpr (sizeof(T) == 2) {
-    if (ring_takes(a, b, x, n, ldx, k_pitch, batch, stream)) return 0;
+    if (ring_takes(a, b, x, n, ldx, k_pitch, batch, carry, stream)) return 0;
   } else {
     if (direct_takes(a, b, x, n, ldx, k_pitch, batch, stream)) return 0;
   }
@@ -528,8 +556,8 @@ int nt_gemm_batched(const T* a, const T* b, T* x, int n, int ldx, int k_pitch, i
   return 0;
 }
 
-template int nt_gemm_batched<float>(const float*, const float*, float*, int, int, int, int, hipStream_t);
-template int nt_gemm_batched<bf16_t>(const bf16_t*, const bf16_t*, bf16_t*, int, int, int, int,
+template int nt_gemm_batched<float>(const float*, const float*, float*, int, int, int, int, const SingleStage*, hipStream_t);
+template int nt_gemm_batched<bf16_t>(const bf16_t*, const bf16_t*, bf16_t*, int, int, int, int, const SingleStage*,
                                      hipStream_t);
 
 }  // namespace ptx

@@ -216,36 +216,146 @@ __global__ __launch_bounds__(kPpWaves * 64, (kPpMinWaves<T, KS>)) void pp_trimul
   }
 }
 
-// q (scaled), K, V^T, triangle bias and (GATE) sigmoid(gate) in the attention core's layouts.
-template <typename T, typename TZ, int KS, int RBW, bool GATE>
-__global__ __launch_bounds__(kPpWaves * 64, (kPpMinWaves<T, KS>)) void pp_triattn_in_kernel(ProjInParams p, SingleStage carry, unsigned carried) {
+// The output columns of an attention projection: q (scaled), K, V^T, triangle bias and (GATE) sigmoid(gate) in the attention
+// core's layouts, from a tile's normalised rows in LDS.  The waves take pairs of 32-column tiles in turn.  Rows: where
+// the tile's rows lie, at(row, i, j); runs of VE rows from a multiple of VE on are consecutive j of one i.
+template <typename T, int KS, int RBW, bool GATE>
+struct AttnColumns {
   typedef typename Vec8<T>::type V8;
   typedef typename VecE<T>::type VE_t;
   typedef Cfg<T> C;
-  constexpr int HP = PpWidths<KS>::HEADS / 2;            // pairs of heads
-  constexpr int NPAIR = (GATE ? 4 : 3) * HP + 1;         // q, k, v (, gate): HP pairs of tiles each; the bias: one tile
-  constexpr int kFrag = RBW * FragLds<T, KS>::ROWBLOCK, kStage = kPpWaves * 2 * 32 * C::PITCH * (int)sizeof(T);
-  __shared__ __attribute__((aligned(16))) char smem[cmax(kFrag + kStage, kStageLds)];
-  PTX_CARRIED_STAGE();
-  char* const frag = smem;
-  T (*stage)[2][32 * C::PITCH] = reinterpret_cast<T (*)[2][32 * C::PITCH]>(smem + kFrag);
-  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int n = p.n;
-  const int64_t n_rows = (int64_t)n * n;
-  const uint32_t tiles = p.tiles, slice = (block >= tiles) + (block >= 2 * tiles) + (block >= 3 * tiles);
-  const uint32_t bx = xcd_run(block - slice * tiles, tiles);
-  const int64_t tile = p.backward ? tiles - 1 - bx : bx;
-  const TileRows tr = tile_rows(tile, 32 * RBW, n, p.tiles_per_i);
-  const T* packed = (const T*)p.packed;
+  static constexpr int HP = PpWidths<KS>::HEADS / 2;            // pairs of heads
+  static constexpr int NPAIR = (GATE ? 4 : 3) * HP + 1;         // q, k, v (, gate): HP pairs of tiles each; the bias: one tile
+  static constexpr int kStage = kPpWaves * 2 * 32 * C::PITCH * (int)sizeof(T);   // LDS beside the rows'
   V8 w[2][KS];
-  auto load_w = [&](int pair) {   // pair -> tiles 2 pair, 2 pair + 1 (the bias' tile twice)
+  __device__ __forceinline__ void load_w(const ProjInParams& p, int pair, int lane) {   // pair -> tiles 2 pair, 2 pair + 1 (the bias' tile twice)
+    const T* packed = (const T*)p.packed;
     const int t0 = pair < NPAIR - 1 ? 2 * pair : 8 * HP, t1 = pair < NPAIR - 1 ? t0 + 1 : t0;
 #pragma unroll
     for (int kk = 0; kk < KS; ++kk) {
       w[0][kk] = packed_frag<T>(packed, t0 * KS + kk, lane);
       w[1][kk] = packed_frag<T>(packed, t1 * KS + kk, lane);
     }
-  };
+  }
+  // (the weights of pair `first` have been requested)
+  template <typename Rows>
+  __device__ __forceinline__ void run(const ProjInParams& p, const char* frag, char* stage_lds, const Rows tr, int first, int step, int wave, int lane) {
+    T* const q_out = (T*)p.out[0];
+    T* const gate_out = (T*)p.out[3];
+    T (*stage)[2][32 * C::PITCH] = reinterpret_cast<T (*)[2][32 * C::PITCH]>(stage_lds);
+    const int n = p.n;
+    const int64_t n_rows = (int64_t)n * n;
+    const int key_tiles = p.pitch >> 6, q_blocks = (n + 31) >> 5;
+    const int64_t head_plane = (int64_t)n * key_tiles * kAttnTileElems;
+#pragma unroll 1
+    for (int pair = first; pair < NPAIR; pair += step) {
+      const int which = pair < NPAIR - 1 ? pair / HP : 4;   // 0 q, 1 k, 2 v, 3 gate, 4 bias
+      const int h0 = (pair % HP) * 2;
+#pragma unroll
+      for (int rb = 0; rb < RBW; ++rb) {
+        f32x16 acc[2];
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[0][r] = acc[1][r] = 0.0f;
+        if (which == 2 || which == 4) {
+#pragma unroll
+          for (int kk = 0; kk < KS; ++kk) {
+            const V8 xv = FragLds<T, KS>::get(frag, rb, kk, lane);
+            mma32(acc[0], xv, w[0][kk]);   // lane <-> channel, register <-> row
+            mma32(acc[1], xv, w[1][kk]);
+          }
+        } else {
+#pragma unroll
+          for (int kk = 0; kk < KS; ++kk) {
+            const V8 xv = FragLds<T, KS>::get(frag, rb, kk, lane);
+            mma32(acc[0], w[0][kk], xv);   // lane <-> row, register <-> channel
+            mma32(acc[1], w[1][kk], xv);
+          }
+        }
+        if (rb == RBW - 1 && pair + step < NPAIR) load_w(p, pair + step, lane);
+        wave_lds_sync();
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+          float vals[16];
+          if (which == 0) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) vals[r] = to_f32(from_f32<T>(acc[t][r])) * p.q_scale;
+          } else if (which == 4) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) vals[r] = acc[t][r] * 1.4426950408889634f;   // the core works in log2 units
+          } else if (GATE && which == 3) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) vals[r] = sigmoidf_fast(acc[t][r]);
+          } else {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) vals[r] = acc[t][r];
+          }
+          stage_put<T>(stage[wave][t], vals, lane);
+        }
+        wave_lds_sync();
+        if (which == 2 || which == 4) {
+          // vectors of VE consecutive keys of one i
+          const int v0 = (lane % C::LPM) * C::VE;
+          int i, j;
+          const bool ok = tr.at(rb * 32 + v0, i, j);
+          if (which == 2) {
+            T* outp = (T*)p.out[2] + attn_v_offset(0, i, j, 0, n, key_tiles);
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+#pragma unroll
+              for (int ps = 0; ps < C::NPASS; ++ps) {
+                int chn, r0;
+                stage_coord<T>(ps, lane, chn, r0);
+                if (ok) *reinterpret_cast<VE_t*>(outp + (h0 + t) * head_plane + chn * 8) = stage_get_vec<T>(stage[wave][t], chn, r0);
+              }
+          } else {
+            T* outp = (T*)p.out[4];
+#pragma unroll
+            for (int ps = 0; ps < C::NPASS; ++ps) {
+              int chn, r0;
+              stage_coord<T>(ps, lane, chn, r0);
+              if (ok && chn < p.heads)
+                *reinterpret_cast<VE_t*>(outp + attn_b_offset(chn, i, j, q_blocks, key_tiles)) = stage_get_vec<T>(stage[wave][0], chn, r0);
+            }
+          }
+        } else {
+#pragma unroll
+          for (int ps = 0; ps < C::NPASS; ++ps) {
+            int mj, m0;
+            stage_coord<T>(ps, lane, mj, m0);
+            int i, j;
+            const bool ok = tr.at(rb * 32 + mj, i, j);
+            if (which == 1) {
+              T* outp = (T*)p.out[1] + attn_k_offset(0, i, j, m0, n, key_tiles);
+#pragma unroll
+              for (int t = 0; t < 2; ++t)
+                if (ok) *reinterpret_cast<VE_t*>(outp + (h0 + t) * head_plane) = stage_get_vec<T>(stage[wave][t], mj, m0);
+            } else {
+              T* outp = (GATE && which == 3 ? gate_out : q_out) + ((int64_t)i * n + j) * 32 + m0;
+#pragma unroll
+              for (int t = 0; t < 2; ++t)
+                if (ok) *reinterpret_cast<VE_t*>(outp + (int64_t)(h0 + t) * n_rows * 32) = stage_get_vec<T>(stage[wave][t], mj, m0);
+            }
+          }
+        }
+      }
+    }
+  }
+};
+
+// q (scaled), K, V^T, triangle bias and (GATE) sigmoid(gate) in the attention core's layouts.
+template <typename T, typename TZ, int KS, int RBW, bool GATE>
+__global__ __launch_bounds__(kPpWaves * 64, (kPpMinWaves<T, KS>)) void pp_triattn_in_kernel(ProjInParams p, SingleStage carry, unsigned carried) {
+  typedef AttnColumns<T, KS, RBW, GATE> Columns;
+  constexpr int kFrag = RBW * FragLds<T, KS>::ROWBLOCK;
+  __shared__ __attribute__((aligned(16))) char smem[cmax(kFrag + Columns::kStage, kStageLds)];
+  PTX_CARRIED_STAGE();
+  char* const frag = smem;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t tiles = p.tiles, slice = (block >= tiles) + (block >= 2 * tiles) + (block >= 3 * tiles);
+  const uint32_t bx = xcd_run(block - slice * tiles, tiles);
+  const int64_t tile = p.backward ? tiles - 1 - bx : bx;
+  const TileRows tr = tile_rows(tile, 32 * RBW, p.n, p.tiles_per_i);
+  Columns columns;
   typename RowPieces<TZ, KS>::V raw[RBW][RowPieces<TZ, KS>::NP];
   norm_rows<T, TZ, KS, RBW>(
       frag, (const TZ*)p.x,
@@ -255,104 +365,10 @@ __global__ __launch_bounds__(kPpWaves * 64, (kPpMinWaves<T, KS>)) void pp_triatt
         return i * p.si + j * p.sj;
       },
       (const T*)p.gamma, (const T*)p.beta, p.eps, wave, lane, raw);
-  const int step = kPpWaves * p.slices;
-  load_w(min(wave + kPpWaves * (int)slice, NPAIR - 1));
+  const int first = wave + kPpWaves * (int)slice;
+  columns.load_w(p, min(first, Columns::NPAIR - 1), lane);
   __syncthreads();
-
-  const int key_tiles = p.pitch >> 6, q_blocks = (n + 31) >> 5;
-  const int64_t head_plane = (int64_t)n * key_tiles * kAttnTileElems;
-#pragma unroll 1
-  for (int pair = wave + kPpWaves * slice; pair < NPAIR; pair += step) {
-    const int which = pair < NPAIR - 1 ? pair / HP : 4;   // 0 q, 1 k, 2 v, 3 gate, 4 bias
-    const int h0 = (pair % HP) * 2;
-#pragma unroll
-    for (int rb = 0; rb < RBW; ++rb) {
-      f32x16 acc[2];
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[0][r] = acc[1][r] = 0.0f;
-      if (which == 2 || which == 4) {
-#pragma unroll
-        for (int kk = 0; kk < KS; ++kk) {
-          const V8 xv = FragLds<T, KS>::get(frag, rb, kk, lane);
-          mma32(acc[0], xv, w[0][kk]);   // lane <-> channel, register <-> row
-          mma32(acc[1], xv, w[1][kk]);
-        }
-      } else {
-#pragma unroll
-        for (int kk = 0; kk < KS; ++kk) {
-          const V8 xv = FragLds<T, KS>::get(frag, rb, kk, lane);
-          mma32(acc[0], w[0][kk], xv);   // lane <-> row, register <-> channel
-          mma32(acc[1], w[1][kk], xv);
-        }
-      }
-      if (rb == RBW - 1 && pair + step < NPAIR) load_w(pair + step);
-      wave_lds_sync();
-#pragma unroll
-      for (int t = 0; t < 2; ++t) {
-        float vals[16];
-        if (which == 0) {
-#pragma unroll
-          for (int r = 0; r < 16; ++r) vals[r] = to_f32(from_f32<T>(acc[t][r])) * p.q_scale;
-        } else if (which == 4) {
-#pragma unroll
-          for (int r = 0; r < 16; ++r) vals[r] = acc[t][r] * 1.4426950408889634f;   // the core works in log2 units
-        } else if (GATE && which == 3) {
-#pragma unroll
-          for (int r = 0; r < 16; ++r) vals[r] = sigmoidf_fast(acc[t][r]);
-        } else {
-#pragma unroll
-          for (int r = 0; r < 16; ++r) vals[r] = acc[t][r];
-        }
-        stage_put<T>(stage[wave][t], vals, lane);
-      }
-      wave_lds_sync();
-      if (which == 2 || which == 4) {
-        // vectors of VE consecutive keys of one i
-        const int v0 = (lane % C::LPM) * C::VE;
-        int i, j;
-        const bool ok = tr.at(rb * 32 + v0, i, j);
-        if (which == 2) {
-          T* outp = (T*)p.out[2] + attn_v_offset(0, i, j, 0, n, key_tiles);
-#pragma unroll
-          for (int t = 0; t < 2; ++t)
-#pragma unroll
-            for (int ps = 0; ps < C::NPASS; ++ps) {
-              int chn, r0;
-              stage_coord<T>(ps, lane, chn, r0);
-              if (ok) *reinterpret_cast<VE_t*>(outp + (h0 + t) * head_plane + chn * 8) = stage_get_vec<T>(stage[wave][t], chn, r0);
-            }
-        } else {
-          T* outp = (T*)p.out[4];
-#pragma unroll
-          for (int ps = 0; ps < C::NPASS; ++ps) {
-            int chn, r0;
-            stage_coord<T>(ps, lane, chn, r0);
-            if (ok && chn < p.heads)
-              *reinterpret_cast<VE_t*>(outp + attn_b_offset(chn, i, j, q_blocks, key_tiles)) = stage_get_vec<T>(stage[wave][0], chn, r0);
-          }
-        }
-      } else {
-#pragma unroll
-        for (int ps = 0; ps < C::NPASS; ++ps) {
-          int mj, m0;
-          stage_coord<T>(ps, lane, mj, m0);
-          int i, j;
-          const bool ok = tr.at(rb * 32 + mj, i, j);
-          if (which == 1) {
-            T* outp = (T*)p.out[1] + attn_k_offset(0, i, j, m0, n, key_tiles);
-#pragma unroll
-            for (int t = 0; t < 2; ++t)
-              if (ok) *reinterpret_cast<VE_t*>(outp + (h0 + t) * head_plane) = stage_get_vec<T>(stage[wave][t], mj, m0);
-          } else {
-            T* outp = (T*)(which == 0 ? p.out[0] : p.out[3]) + ((int64_t)i * n + j) * 32 + m0;
-#pragma unroll
-            for (int t = 0; t < 2; ++t)
-              if (ok) *reinterpret_cast<VE_t*>(outp + (int64_t)(h0 + t) * n_rows * 32) = stage_get_vec<T>(stage[wave][t], mj, m0);
-          }
-        }
-      }
-    }
-  }
+  columns.run(p, frag, smem + kFrag, tr, first, kPpWaves * p.slices, wave, lane);
 }
 
 namespace {
@@ -371,230 +387,348 @@ struct ProjOutParams {
 };
 }  // namespace
 
-// out = [z +] (W_z LN_out(x)) * sigmoid(W_g LN_in(z)); out may be z.
-template <typename T, typename TZ, int KS, int RBW>
-__global__ __launch_bounds__(kPpWaves * 64, (kPpMinWaves<T, KS>)) void pp_trimul_out_kernel(ProjOutParams p, SingleStage carry, unsigned carried) {
-  typedef typename Vec8<T>::type V8;
-  typedef typename VecE<T>::type VE_t;
-  typedef Cfg<T> C;
-  constexpr int SL = PpWidths<KS>::SL, HIDDEN = PpWidths<KS>::HIDDEN, NOB = KS / 2;
-  constexpr int XP = 32 * RBW + 4;   // pitch of the triangle product's tile (elements)
-  constexpr int kXt = (int)sizeof(T) * HIDDEN * XP, kUpd = (int)sizeof(T) * 32 * RBW * kUpdPitch<KS>;
-  constexpr int kFrag = RBW * FragLds<T, KS>::ROWBLOCK, kFrag2 = RBW * FragLds<T, SL>::ROWBLOCK;
-  __shared__ __attribute__((aligned(16))) char smem[cmax(kFrag + kFrag2 + cmax(kXt, kUpd), kStageLds)];
-  PTX_CARRIED_STAGE();
-  char* const frag = smem;
-  char* const frag2 = smem + kFrag;
-  char* const scratch = smem + kFrag + kFrag2;
-  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int n = p.n;
-  const TileRows tr = tile_rows(xcd_run(block, blocks), 32 * RBW, n, p.tiles_per_i);
-  const T* packed = (const T*)p.packed;
-
-  // the triangle product's rows of every channel: vectors of VE rows
-  constexpr int VPC = 32 * RBW / C::VE, NV = HIDDEN * VPC / (kPpWaves * 64);
-  const int v0 = (threadIdx.x % VPC) * C::VE, c0 = threadIdx.x / VPC;
-  VE_t xv[NV];
-  {
-    int i, j;
-    tr.at(v0, i, j);
-    // (a tile past the end of a plane re-reads its last vector: those rows are not stored)
-    const int64_t off = min((int64_t)i * p.ldx + j, (int64_t)n * p.ldx - C::VE) & ~(int64_t)(C::VE - 1);
-    const T* src = (const T*)p.x + off;
-    const int64_t plane = (int64_t)n * p.ldx;
-#pragma unroll
-    for (int q = 0; q < NV; ++q) xv[q] = *reinterpret_cast<const VE_t*>(src + (c0 + q * (kPpWaves * 64 / VPC)) * plane);
-  }
-  auto z_row = [&](int r) {
+// Element offset of a tile's row in z and out, or -1.
+template <typename Rows> struct ZRow {
+  const ProjOutParams& p;
+  const Rows& tr;
+  __device__ __forceinline__ int64_t operator()(int r) const {
     int i, j;
     const bool ok = tr.at(r, i, j);
     const int64_t o = i * p.si + j * p.sj;
     return ok ? o : -1;
-  };
+  }
+};
+
+// The update (W_z LN_out(x)) * sigmoid(W_g LN_in(z)) of a tile, left in LDS (returned) with the raw rows of z in registers;
+// a barrier is due before it is read.
+template <typename T, typename TZ, int KS, int RBW> struct MulOut {
+  static constexpr int SL = PpWidths<KS>::SL, HIDDEN = PpWidths<KS>::HIDDEN, NOB = KS / 2;
+  static constexpr int XP = 32 * RBW + 4;   // pitch of the triangle product's tile (elements)
+  static constexpr int kXt = (int)sizeof(T) * HIDDEN * XP, kUpd = (int)sizeof(T) * 32 * RBW * kUpdPitch<KS>;
+  static constexpr int kFrag = RBW * FragLds<T, KS>::ROWBLOCK, kFrag2 = RBW * FragLds<T, SL>::ROWBLOCK;
+  static constexpr int kLds = kFrag + kFrag2 + cmax(kXt, kUpd);
+  template <typename Rows>
+  static __device__ __forceinline__ T* run(const ProjOutParams& p, const Rows& tr, char* smem, int wave, int lane,
+                                           typename RowPieces<TZ, KS>::V (&raw)[RBW][RowPieces<TZ, KS>::NP]) {
+    typedef typename Vec8<T>::type V8;
+    typedef typename VecE<T>::type VE_t;
+    typedef Cfg<T> C;
+    char* const frag = smem;
+    char* const frag2 = smem + kFrag;
+    char* const scratch = smem + kFrag + kFrag2;
+    const int n = p.n;
+    const T* packed = (const T*)p.packed;
+
+    // the triangle product's rows of every channel: vectors of VE rows
+    constexpr int VPC = 32 * RBW / C::VE, NV = HIDDEN * VPC / (kPpWaves * 64);
+    const int v0 = (threadIdx.x % VPC) * C::VE, c0 = threadIdx.x / VPC;
+    VE_t xv[NV];
+    {
+      int i, j;
+      tr.at(v0, i, j);
+      // (a tile past the end of a plane re-reads its last vector: those rows are not stored)
+      const int64_t off = min((int64_t)i * p.ldx + j, (int64_t)n * p.ldx - C::VE) & ~(int64_t)(C::VE - 1);
+      const T* src = (const T*)p.x + off;
+      const int64_t plane = (int64_t)n * p.ldx;
+#pragma unroll
+      for (int q = 0; q < NV; ++q) xv[q] = *reinterpret_cast<const VE_t*>(src + (c0 + q * (kPpWaves * 64 / VPC)) * plane);
+    }
+    const ZRow<Rows> z_row{p, tr};
+    norm_rows<T, TZ, KS, RBW>(
+        frag, (const TZ*)p.z, [&](int r) { return max(z_row(r), (int64_t)0); }, (const T*)p.gamma, (const T*)p.beta, p.eps,
+        wave, lane, raw);
+    T* xt = reinterpret_cast<T*>(scratch);
+#pragma unroll
+    for (int q = 0; q < NV; ++q) {
+      u32x2* d = reinterpret_cast<u32x2*>(xt + (c0 + q * (kPpWaves * 64 / VPC)) * XP + v0);
+      const u32x2* s = reinterpret_cast<const u32x2*>(&xv[q]);
+      d[0] = s[0];
+      d[1] = s[1];
+    }
+    __syncthreads();
+    {
+      typedef RowPieces<T, SL> RP;
+      constexpr int PE = RP::PE, NP = RP::NP;
+      const int j = lane & 7, r8 = wave * 8 + (lane >> 3);
+      float gm[NP][PE], bt[NP][PE];
+      load_affine_pieces<T, PE, NP>((const T*)p.gamma2, (const T*)p.beta2, j, gm, bt);
+#pragma unroll
+      for (int rb = 0; rb < RBW; ++rb) {
+        float v[NP][PE];
+#pragma unroll
+        for (int q = 0; q < NP; ++q)
+#pragma unroll
+          for (int t = 0; t < PE; ++t) v[q][t] = to_f32(xt[(PE * (j + 8 * q) + t) * XP + rb * 32 + r8]);
+        normalize_pieces<PE, NP>(v, gm, bt, p.eps);
+#pragma unroll
+        for (int q = 0; q < NP; ++q) put_piece<T, SL, PE>(frag2, rb, r8, j + 8 * q, v[q]);
+      }
+    }
+    V8 wz[SL], wg[KS];
+    auto load_w = [&](int ob) {
+#pragma unroll
+      for (int kk = 0; kk < SL; ++kk) wz[kk] = packed_frag<T>(packed, ob * (SL + KS) + kk, lane);
+#pragma unroll
+      for (int kk = 0; kk < KS; ++kk) wg[kk] = packed_frag<T>(packed, ob * (SL + KS) + SL + kk, lane);
+    };
+    if (wave < NOB) load_w(wave);
+    __syncthreads();   // both operand tiles are complete, and the product's tile has been read
+    T* upd = reinterpret_cast<T*>(scratch);
+#pragma unroll
+    for (int ob = wave; ob < NOB; ob += kPpWaves) {
+#pragma unroll
+      for (int rb = 0; rb < RBW; ++rb) {
+        f32x16 az, ag;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) az[r] = ag[r] = 0.0f;
+#pragma unroll
+        for (int kk = 0; kk < SL; ++kk) mma32(az, wz[kk], FragLds<T, SL>::get(frag2, rb, kk, lane));
+#pragma unroll
+        for (int kk = 0; kk < KS; ++kk) mma32(ag, wg[kk], FragLds<T, KS>::get(frag, rb, kk, lane));
+        if (rb == RBW - 1 && ob + kPpWaves < NOB) load_w(ob + kPpWaves);
+        float vals[16];
+#pragma unroll
+        for (int r = 0; r < 16; ++r)   // linear_z's output rounded to T, times the gate, rounded to T
+          vals[r] = to_f32(from_f32<T>(az[r])) * sigmoidf_fast(ag[r]);
+        put_update<T, KS>(upd, rb, ob, vals, lane);
+      }
+    }
+    return upd;
+  }
+};
+
+// out = [z +] (W_z LN_out(x)) * sigmoid(W_g LN_in(z)); out may be z.
+template <typename T, typename TZ, int KS, int RBW>
+__global__ __launch_bounds__(kPpWaves * 64, (kPpMinWaves<T, KS>)) void pp_trimul_out_kernel(ProjOutParams p, SingleStage carry, unsigned carried) {
+  typedef MulOut<T, TZ, KS, RBW> Out;
+  __shared__ __attribute__((aligned(16))) char smem[cmax(Out::kLds, kStageLds)];
+  PTX_CARRIED_STAGE();
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const TileRows tr = tile_rows(xcd_run(block, blocks), 32 * RBW, p.n, p.tiles_per_i);
   typename RowPieces<TZ, KS>::V raw[RBW][RowPieces<TZ, KS>::NP];
-  norm_rows<T, TZ, KS, RBW>(
-      frag, (const TZ*)p.z, [&](int r) { return max(z_row(r), (int64_t)0); }, (const T*)p.gamma, (const T*)p.beta, p.eps,
-      wave, lane, raw);
-  T* xt = reinterpret_cast<T*>(scratch);
-#pragma unroll
-  for (int q = 0; q < NV; ++q) {
-    u32x2* d = reinterpret_cast<u32x2*>(xt + (c0 + q * (kPpWaves * 64 / VPC)) * XP + v0);
-    const u32x2* s = reinterpret_cast<const u32x2*>(&xv[q]);
-    d[0] = s[0];
-    d[1] = s[1];
-  }
+  const T* upd = Out::run(p, tr, smem, wave, lane, raw);
   __syncthreads();
-  {
-    typedef RowPieces<T, SL> RP;
-    constexpr int PE = RP::PE, NP = RP::NP;
-    const int j = lane & 7, r8 = wave * 8 + (lane >> 3);
-    float gm[NP][PE], bt[NP][PE];
-    load_affine_pieces<T, PE, NP>((const T*)p.gamma2, (const T*)p.beta2, j, gm, bt);
-#pragma unroll
-    for (int rb = 0; rb < RBW; ++rb) {
-      float v[NP][PE];
-#pragma unroll
-      for (int q = 0; q < NP; ++q)
-#pragma unroll
-        for (int t = 0; t < PE; ++t) v[q][t] = to_f32(xt[(PE * (j + 8 * q) + t) * XP + rb * 32 + r8]);
-      normalize_pieces<PE, NP>(v, gm, bt, p.eps);
-#pragma unroll
-      for (int q = 0; q < NP; ++q) put_piece<T, SL, PE>(frag2, rb, r8, j + 8 * q, v[q]);
-    }
-  }
-  V8 wz[SL], wg[KS];
-  auto load_w = [&](int ob) {
-#pragma unroll
-    for (int kk = 0; kk < SL; ++kk) wz[kk] = packed_frag<T>(packed, ob * (SL + KS) + kk, lane);
-#pragma unroll
-    for (int kk = 0; kk < KS; ++kk) wg[kk] = packed_frag<T>(packed, ob * (SL + KS) + SL + kk, lane);
-  };
-  if (wave < NOB) load_w(wave);
-  __syncthreads();   // both operand tiles are complete, and the product's tile has been read
-  T* upd = reinterpret_cast<T*>(scratch);
-#pragma unroll
-  for (int ob = wave; ob < NOB; ob += kPpWaves) {
-#pragma unroll
-    for (int rb = 0; rb < RBW; ++rb) {
-      f32x16 az, ag;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) az[r] = ag[r] = 0.0f;
-#pragma unroll
-      for (int kk = 0; kk < SL; ++kk) mma32(az, wz[kk], FragLds<T, SL>::get(frag2, rb, kk, lane));
-#pragma unroll
-      for (int kk = 0; kk < KS; ++kk) mma32(ag, wg[kk], FragLds<T, KS>::get(frag, rb, kk, lane));
-      if (rb == RBW - 1 && ob + kPpWaves < NOB) load_w(ob + kPpWaves);
-      float vals[16];
-#pragma unroll
-      for (int r = 0; r < 16; ++r)   // linear_z's output rounded to T, times the gate, rounded to T
-        vals[r] = to_f32(from_f32<T>(az[r])) * sigmoidf_fast(ag[r]);
-      put_update<T, KS>(upd, rb, ob, vals, lane);
-    }
-  }
-  __syncthreads();
-  store_rows<T, TZ, KS, RBW>((TZ*)p.out, z_row, upd, wave, lane, p.add_residual, raw);
+  store_rows<T, TZ, KS, RBW>((TZ*)p.out, ZRow<TileRows>{p, tr}, upd, wave, lane, p.add_residual, raw);
 }
 
-// out = [z +] W_o (gate * o): GATE: gate = sigmoid(W_g LN(z)) formed here (16-bit arithmetic; wave = head, and head + 4
+// Row of the attention output that belongs to a tile's row (past the end: a valid one).
+__device__ __forceinline__ int64_t o_row(const TileRows& tr, int r, int n) { return min(tr.p0 + r, (int64_t)n * n - 1); }
+
+// The update W_o (gate * o) of a tile, as above.
+// GATE: gate = sigmoid(W_g LN(z)) formed here (16-bit arithmetic; wave = head, and head + 4
 // on rows of 256 channels), otherwise o arrives gated.  out may be z.  The gate formed here is neither written nor
 // read: on rows of 64 / 256 channels, whose gates are twice / as wide as their rows, one update (projection, core,
 // output) takes 270
 // instead of 281 us at 512 tokens / 1169 instead of 1207 at 600 (per launch: 63 + 156 + 51, was 80 + 165 + 36; 323 + 571 + 275,
 // was 392 + 603 + 212; 256 channels at 96 / 200 / 400 / 800 tokens: 43 / 118 / 481 / 2242, was 44 / 113 / 487 / 2349).  Two row
 // blocks per workgroup on 256 channels: 292 us at 600, 43 instead of 32 at 200.
-template <typename T, typename TZ, int KS, bool GATE, int RBW>
-__global__ __launch_bounds__(kPpWaves * 64, (kPpMinWaves<T, KS>)) void pp_triattn_out_kernel(ProjOutParams p, SingleStage carry, unsigned carried) {
-  typedef typename Vec8<T>::type V8;
-  constexpr int SL = PpWidths<KS>::SL, NOB = KS / 2;
+template <typename T, typename TZ, int KS, bool GATE, int RBW> struct AttnOut {
+  static constexpr int SL = PpWidths<KS>::SL, NOB = KS / 2;
   static_assert(!GATE || sizeof(T) == 2, "gate formed here: 16-bit arithmetic");
-  constexpr int kFrag = GATE ? RBW * FragLds<T, KS>::ROWBLOCK : 16, kUpd = (int)sizeof(T) * 32 * RBW * kUpdPitch<KS>;
-  constexpr int kScratch = cmax(kFrag, kUpd);   // the normalised rows, then the update
-  __shared__ __attribute__((aligned(16))) char smem[cmax(kScratch + RBW * FragLds<T, SL>::ROWBLOCK, kStageLds)];
-  PTX_CARRIED_STAGE();
-  char* const scratch = smem;
-  char* const fo = smem + kScratch;
-  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int n = p.n, nl = lane & 31, g = lane >> 5;
-  const int64_t n_rows = (int64_t)n * n;
-  const TileRows tr = tile_rows(xcd_run(block, blocks), 32 * RBW, n, 0);
-  const T* packed = (const T*)p.packed;
-  V8 w[SL];
-  auto load_w = [&](int ob) {
+  static constexpr int kFrag = GATE ? RBW * FragLds<T, KS>::ROWBLOCK : 16, kUpd = (int)sizeof(T) * 32 * RBW * kUpdPitch<KS>;
+  static constexpr int kScratch = cmax(kFrag, kUpd);   // the normalised rows, then the update
+  static constexpr int kLds = kScratch + RBW * FragLds<T, SL>::ROWBLOCK;
+  template <typename Rows>
+  static __device__ __forceinline__ T* run(const ProjOutParams& p, const Rows& tr, char* smem, int wave, int lane,
+                                           typename RowPieces<TZ, KS>::V (&raw)[RBW][RowPieces<TZ, KS>::NP]) {
+    typedef typename Vec8<T>::type V8;
+    char* const scratch = smem;
+    char* const fo = smem + kScratch;
+    const int n = p.n, nl = lane & 31, g = lane >> 5;
+    const int64_t n_rows = (int64_t)n * n;
+    const T* packed = (const T*)p.packed;
+    V8 w[SL];
+    auto load_w = [&](int ob) {
 #pragma unroll
-    for (int kk = 0; kk < SL; ++kk) w[kk] = packed_frag<T>(packed, ob * SL + kk, lane);
-  };
-  // this wave's share of the attention output: heads wave, wave + 4, .. as fragments
-  constexpr int HPW = PpWidths<KS>::HEADS / kPpWaves;
-  V8 of[RBW][HPW][2];
-#pragma unroll
-  for (int rb = 0; rb < RBW; ++rb) {
-    const int64_t pr = min(tr.p0 + rb * 32 + nl, n_rows - 1);
-#pragma unroll
-    for (int q = 0; q < HPW; ++q)
-#pragma unroll
-      for (int u = 0; u < 2; ++u)
-        of[rb][q][u] = load8<T>((const T*)p.x + ((int64_t)(wave + 4 * q) * n_rows + pr) * 32 + 16 * u + 8 * g);
-  }
-  auto z_row = [&](int r) {
-    int i, j;
-    const bool ok = tr.at(r, i, j);
-    const int64_t o = i * p.si + j * p.sj;
-    return ok ? o : -1;
-  };
-  auto z_row0 = [&](int r) { return max(z_row(r), (int64_t)0); };
-  typename RowPieces<TZ, KS>::V raw[RBW][RowPieces<TZ, KS>::NP];
-  if constexpr (GATE) {
-    // (all of a wave's gate weights under the LayerNorm, the output's first under the last head's products: fetched
-    // when needed, one after the other, they cost rows of 256 channels three waits instead of one)
-    V8 wg[HPW][KS];
-#pragma unroll
-    for (int q = 0; q < HPW; ++q)
-#pragma unroll
-      for (int kk = 0; kk < KS; ++kk) wg[q][kk] = packed_frag<T>((const T*)p.packed_g, (wave + 4 * q) * KS + kk, lane);
-    norm_rows<T, TZ, KS, RBW>(scratch, (const TZ*)p.z, z_row0, (const T*)p.gamma, (const T*)p.beta, p.eps, wave, lane, raw);
-    if (HPW == 1 && wave < NOB) load_w(wave);
-    __syncthreads();
-#pragma unroll
-    for (int q = 0; q < HPW; ++q)
+      for (int kk = 0; kk < SL; ++kk) w[kk] = packed_frag<T>(packed, ob * SL + kk, lane);
+    };
+    // this wave's share of the attention output: heads wave, wave + 4, .. as fragments
+    constexpr int HPW = PpWidths<KS>::HEADS / kPpWaves;
+    V8 of[RBW][HPW][2];
 #pragma unroll
     for (int rb = 0; rb < RBW; ++rb) {
-      f32x16 ag;
+      const int64_t pr = o_row(tr, rb * 32 + nl, p.n);
 #pragma unroll
-      for (int r = 0; r < 16; ++r) ag[r] = 0.0f;
+      for (int q = 0; q < HPW; ++q)
 #pragma unroll
-      for (int kk = 0; kk < KS; ++kk) mma32(ag, wg[q][kk], FragLds<T, KS>::get(scratch, rb, kk, lane));
-      if (HPW > 1 && rb == RBW - 1 && q == HPW - 2) load_w(wave);
-      // (weight rows packed so that registers 8 u + t are the channels 16 u + 8 g + t of the lane's own fragments;
-      // gate and gated output rounded to T like the reference's sigmoid(linear_g(x)) and o * g)
-#pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        const f32x8 ov = to_f32(of[rb][q][u]);
-        f32x8 gated;
-#pragma unroll
-        for (int t = 0; t < 8; ++t) gated[t] = ov[t] * to_f32(from_f32<T>(sigmoidf_fast(ag[8 * u + t])));
-        of[rb][q][u] = from_f32<T>(gated);
-      }
+        for (int u = 0; u < 2; ++u)
+          of[rb][q][u] = load8<T>((const T*)p.x + ((int64_t)(wave + 4 * q) * n_rows + pr) * 32 + 16 * u + 8 * g);
     }
-  } else {
-    if (wave < NOB) load_w(wave);
-    if (p.add_residual) {
-      typedef RowPieces<TZ, KS> RP;
+    const ZRow<Rows> z_row{p, tr};
+    auto z_row0 = [&](int r) { return max(z_row(r), (int64_t)0); };
+    if constexpr (GATE) {
+      // (all of a wave's gate weights under the LayerNorm, the output's first under the last head's products: fetched
+      // when needed, one after the other, they cost rows of 256 channels three waits instead of one)
+      V8 wg[HPW][KS];
+#pragma unroll
+      for (int q = 0; q < HPW; ++q)
+#pragma unroll
+        for (int kk = 0; kk < KS; ++kk) wg[q][kk] = packed_frag<T>((const T*)p.packed_g, (wave + 4 * q) * KS + kk, lane);
+      norm_rows<T, TZ, KS, RBW>(scratch, (const TZ*)p.z, z_row0, (const T*)p.gamma, (const T*)p.beta, p.eps, wave, lane, raw);
+      if (HPW == 1 && wave < NOB) load_w(wave);
+      __syncthreads();
+#pragma unroll
+      for (int q = 0; q < HPW; ++q)
 #pragma unroll
       for (int rb = 0; rb < RBW; ++rb) {
-        const TZ* rp = (const TZ*)p.z + z_row0(rb * 32 + wave * 8 + (lane >> 3)) + RP::PE * (lane & 7);
+        f32x16 ag;
 #pragma unroll
-        for (int q = 0; q < RP::NP; ++q) raw[rb][q] = *reinterpret_cast<const typename RP::V*>(rp + 8 * RP::PE * q);
+        for (int r = 0; r < 16; ++r) ag[r] = 0.0f;
+#pragma unroll
+        for (int kk = 0; kk < KS; ++kk) mma32(ag, wg[q][kk], FragLds<T, KS>::get(scratch, rb, kk, lane));
+        if (HPW > 1 && rb == RBW - 1 && q == HPW - 2) load_w(wave);
+        // (weight rows packed so that registers 8 u + t are the channels 16 u + 8 g + t of the lane's own fragments;
+        // gate and gated output rounded to T like the reference's sigmoid(linear_g(x)) and o * g)
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          const f32x8 ov = to_f32(of[rb][q][u]);
+          f32x8 gated;
+#pragma unroll
+          for (int t = 0; t < 8; ++t) gated[t] = ov[t] * to_f32(from_f32<T>(sigmoidf_fast(ag[8 * u + t])));
+          of[rb][q][u] = from_f32<T>(gated);
+        }
+      }
+    } else {
+      if (wave < NOB) load_w(wave);
+      if (p.add_residual) {
+        typedef RowPieces<TZ, KS> RP;
+#pragma unroll
+        for (int rb = 0; rb < RBW; ++rb) {
+          const TZ* rp = (const TZ*)p.z + z_row0(rb * 32 + wave * 8 + (lane >> 3)) + RP::PE * (lane & 7);
+#pragma unroll
+          for (int q = 0; q < RP::NP; ++q) raw[rb][q] = *reinterpret_cast<const typename RP::V*>(rp + 8 * RP::PE * q);
+        }
       }
     }
-  }
 #pragma unroll
-  for (int rb = 0; rb < RBW; ++rb)
+    for (int rb = 0; rb < RBW; ++rb)
 #pragma unroll
-    for (int q = 0; q < HPW; ++q)
+      for (int q = 0; q < HPW; ++q)
 #pragma unroll
-      for (int u = 0; u < 2; ++u) FragLds<T, SL>::put(fo, rb, nl, 2 * (2 * (wave + 4 * q) + u) + g, of[rb][q][u]);
-  __syncthreads();   // (and the normalised rows have been read)
-  T* upd = reinterpret_cast<T*>(scratch);
+        for (int u = 0; u < 2; ++u) FragLds<T, SL>::put(fo, rb, nl, 2 * (2 * (wave + 4 * q) + u) + g, of[rb][q][u]);
+    __syncthreads();   // (and the normalised rows have been read)
+    T* upd = reinterpret_cast<T*>(scratch);
 #pragma unroll
-  for (int ob = wave; ob < NOB; ob += kPpWaves) {
+    for (int ob = wave; ob < NOB; ob += kPpWaves) {
 #pragma unroll
-    for (int rb = 0; rb < RBW; ++rb) {
-      f32x16 acc;
+      for (int rb = 0; rb < RBW; ++rb) {
+        f32x16 acc;
 #pragma unroll
-      for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
+        for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
 #pragma unroll
-      for (int kk = 0; kk < SL; ++kk) mma32(acc, w[kk], FragLds<T, SL>::get(fo, rb, kk, lane));
-      if (rb == RBW - 1 && ob + kPpWaves < NOB) load_w(ob + kPpWaves);
-      float vals[16];
+        for (int kk = 0; kk < SL; ++kk) mma32(acc, w[kk], FragLds<T, SL>::get(fo, rb, kk, lane));
+        if (rb == RBW - 1 && ob + kPpWaves < NOB) load_w(ob + kPpWaves);
+        float vals[16];
 #pragma unroll
-      for (int r = 0; r < 16; ++r) vals[r] = acc[r];
-      put_update<T, KS>(upd, rb, ob, vals, lane);   // (rounded to T, as the module's output is)
+        for (int r = 0; r < 16; ++r) vals[r] = acc[r];
+        put_update<T, KS>(upd, rb, ob, vals, lane);   // (rounded to T, as the module's output is)
+      }
     }
+    return upd;
   }
+};
+
+template <typename T, typename TZ, int KS, bool GATE, int RBW>
+__global__ __launch_bounds__(kPpWaves * 64, (kPpMinWaves<T, KS>)) void pp_triattn_out_kernel(ProjOutParams p, SingleStage carry, unsigned carried) {
+  typedef AttnOut<T, TZ, KS, GATE, RBW> Out;
+  __shared__ __attribute__((aligned(16))) char smem[cmax(Out::kLds, kStageLds)];
+  PTX_CARRIED_STAGE();
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const TileRows tr = tile_rows(xcd_run(block, blocks), 32 * RBW, p.n, 0);
+  typename RowPieces<TZ, KS>::V raw[RBW][RowPieces<TZ, KS>::NP];
+  const T* upd = Out::run(p, tr, smem, wave, lane, raw);
   __syncthreads();
-  store_rows<T, TZ, KS, RBW>((TZ*)p.out, z_row, upd, wave, lane, p.add_residual, raw);
+  store_rows<T, TZ, KS, RBW>((TZ*)p.out, ZRow<TileRows>{p, tr}, upd, wave, lane, p.add_residual, raw);
 }
 
+// ---- an output stage and the projection that reads its rows next, in one launch -------------------------
+// A patch of 8 x 4 * RBW positions for the projection of an ending node behind a starting node's output: logical rows (i, j) of the
+// ending node are z[j][i]; 8 consecutive j of one i follow each other.
+struct PatchRows {
+  int i0, j0, n;
+  __device__ __forceinline__ bool at(int r, int& i, int& j) const {   // of the ending node
+    i = min(i0 + (r >> 3), n - 1);
+    j = min(j0 + (r & 7), n - 1);
+    return i0 + (r >> 3) < n && j0 + (r & 7) < n;
+  }
+};
+struct PatchRowsT {   // the same positions of the starting node
+  PatchRows t;
+  __device__ __forceinline__ bool at(int r, int& i, int& j) const { return t.at(r, j, i); }
+};
+__device__ __forceinline__ int64_t o_row(const PatchRowsT& tr, int r, int n) {
+  int i, j;
+  tr.at(r, i, j);
+  return (int64_t)i * n + j;
+}
+
+// z' = z + update (stored), and its rows, as stored, normalised with the next stage's parameters into `frag`.
+template <typename T, typename TZ, int KS, int RBW, typename Off>
+__device__ __forceinline__ void store_and_norm_rows(char* frag, TZ* out, Off off, const T* upd, const T* gamma, const T* beta, float eps, int wave,
+                                                    int lane, typename RowPieces<TZ, KS>::V (&raw)[RBW][RowPieces<TZ, KS>::NP]) {
+  typedef RowPieces<TZ, KS> RP;
+  constexpr int PE = RP::PE, NP = RP::NP;
+  const int j = lane & 7, r8 = wave * 8 + (lane >> 3);
+  float gm[NP][PE], bt[NP][PE];
+  load_affine_pieces<T, PE, NP>(gamma, beta, j, gm, bt);
+  __syncthreads();   // (the update is complete, and what lay in `frag` has been read)
+  store_rows<T, TZ, KS, RBW>(out, off, upd, wave, lane, 1, raw);
+#pragma unroll
+  for (int rb = 0; rb < RBW; ++rb) {
+    float v[NP][PE];
+#pragma unroll
+    for (int q = 0; q < NP; ++q)
+#pragma unroll
+      for (int t = 0; t < PE; ++t) v[q][t] = to_f32(raw[rb][q][t]);
+    normalize_pieces<PE, NP>(v, gm, bt, eps);
+#pragma unroll
+    for (int q = 0; q < NP; ++q) put_piece<T, KS, PE>(frag, rb, r8, j + 8 * q, v[q]);
+  }
+}
+
+// The output stage of a triangle multiplication and the projection of the starting node behind it: z' is read by nothing in
+// between.
+template <typename T, typename TZ, int KS, int RBW>
+__global__ __launch_bounds__(kPpWaves * 64, (kPpMinWaves<T, KS>)) void pp_mul_out_attn_in_kernel(ProjOutParams p, ProjInParams pi, SingleStage carry,
+                                                                                                unsigned carried) {
+  typedef MulOut<T, TZ, KS, RBW> Out;
+  typedef AttnColumns<T, KS, RBW, false> Columns;
+  __shared__ __attribute__((aligned(16))) char smem[cmax(cmax(Out::kLds, Out::kFrag + Columns::kStage), kStageLds)];
+  PTX_CARRIED_STAGE();
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const TileRows tr = tile_rows(xcd_run(block, blocks), 32 * RBW, p.n, p.tiles_per_i);
+  typename RowPieces<TZ, KS>::V raw[RBW][RowPieces<TZ, KS>::NP];
+  const T* upd = Out::run(p, tr, smem, wave, lane, raw);
+  store_and_norm_rows<T, TZ, KS, RBW>(smem, (TZ*)p.out, ZRow<TileRows>{p, tr}, upd, (const T*)pi.gamma, (const T*)pi.beta, pi.eps, wave, lane, raw);
+  Columns columns;
+  columns.load_w(pi, wave, lane);
+  __syncthreads();
+  columns.run(pi, smem, smem + Out::kFrag, tr, wave, kPpWaves, wave, lane);
+}
+
+// The output stage of a starting node and the projection of the ending node behind it.
+template <typename T, typename TZ, int KS, int RBW>
+__global__ __launch_bounds__(kPpWaves * 64, (kPpMinWaves<T, KS>)) void pp_attn_out_attn_in_kernel(ProjOutParams p, ProjInParams pi, SingleStage carry,
+                                                                                                 unsigned carried) {
+  typedef AttnOut<T, TZ, KS, true, RBW> Out;
+  typedef AttnColumns<T, KS, RBW, false> Columns;
+  // the next stage's rows: behind the update, which other waves may still read, and the staging tiles
+  constexpr int kNorm = cmax(Out::kScratch, Columns::kStage);
+  __shared__ __attribute__((aligned(16))) char smem[cmax(kNorm + RBW * FragLds<T, KS>::ROWBLOCK, cmax(Out::kLds, kStageLds))];
+  PTX_CARRIED_STAGE();
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t n_ip = (uint32_t)(p.n + 4 * RBW - 1) / (4 * RBW), tile = xcd_run(block, blocks), jb = tile / n_ip;
+  const PatchRows tr = {(int)(tile - jb * n_ip) * (4 * RBW), (int)jb * 8, p.n};
+  const PatchRowsT trt = {tr};
+  typename RowPieces<TZ, KS>::V raw[RBW][RowPieces<TZ, KS>::NP];
+  const T* upd = Out::run(p, trt, smem, wave, lane, raw);
+  store_and_norm_rows<T, TZ, KS, RBW>(smem + kNorm, (TZ*)p.out, ZRow<PatchRowsT>{p, trt}, upd, (const T*)pi.gamma, (const T*)pi.beta, pi.eps,
+                                      wave, lane, raw);
+  Columns columns;
+  columns.load_w(pi, wave, lane);
+  __syncthreads();
+  columns.run(pi, smem + kNorm, smem, tr, wave, kPpWaves, wave, lane);
+}
 // ---------------------------------------------------------------------------
 // Weight packing: every 32-row tile of the matrices as KS (or more) fragments, one lane's 8
 // elements in 16-byte pieces [fragment][piece][lane].
@@ -975,6 +1109,137 @@ int pp_triattn_out(const void* o, const void* z, const void* ln_w, const void* l
   }
   return pp_triattn_out_ks<T, TZ, 8, sizeof(T) == 2>(p, carry, stream);
 }
+
+// ---- an output stage with the next projection ----
+// Where the two stages are faster in one launch.  They save a launch, its wait for the rows and one reading of the pair
+// tensor, and give up the kernel with all weights in LDS that a projection by itself may take (pp_resident), on rows of 64 and 128
+// channels tiles of four row blocks, on 256 tiles of two; the ending node's patches read the attention output and the rows in
+// shorter runs.  us per block, no / the first / both pairs joined: 128 channels, fp32 rows, 64 tokens 85.1 / 84.1 / 79.2, 93 119 / 116 / 110, 160 173
+// / 169 / 164, 256 300 / 290 / 278, 387 739 / 723 / 714, 512 1115 / 1109 / 1102, 576 1421 / 1409 / 1429, 640 1774 / 1775 / 1789, 768 2601 / 2596 /
+// 2613, 1500 (no such kernel) 13264 / 13160 / 13226, 2048 27462 / 27528 / 27682; 16-bit rows, 256 262 / 259 / 251, 440 769 / 750 / 747, 480 918 / 922 / 924, 768
+// 2354 / 2402 / 2437; 64 channels, 128 101 / 97 / 94, 512 790 / 792 / 790, 1200 6191 / 6171 / 6147, 1500 10724 / 10774 / 10803; 256 channels, 96 240 / 234 / 228, 256
+// 715 / 715 / 714, 300 1114 / 1133 / 1139.
+bool pp_joined(bool attention, int n, int c_z, int hidden, bool rows16) {
+  if (c_z == 256) return n <= 256;
+  if (c_z == 64) return n <= 1280;
+  const bool first = n < (rows16 ? 480 : 528) || (n < 1792 && !pp_resident(kTriAttnInStage, n, c_z, hidden, true, rows16));
+  return first && (!attention || n < 600);
+}
+static int merged_row_blocks(int64_t rows, int ks) { return ks <= 8 && rows >= 160 * 160 ? 2 : 1; }
+
+static void attn_in_params(ProjInParams& p, const void* ln_w, const void* ln_b, const void* packed, void* q, void* k, void* vt, void* tri_bias,
+                           int n, int heads, int key_pitch, float eps) {
+  p.gamma = ln_w;
+  p.beta = ln_b;
+  p.eps = eps;
+  p.packed = packed;
+  p.out[0] = q; p.out[1] = k; p.out[2] = vt; p.out[4] = tri_bias;
+  p.n = n;
+  p.pitch = key_pitch;
+  p.heads = heads;
+  p.q_scale = 1.4426950408889634f / sqrtf(32.0f);   // log2(e) / sqrt(d), see triattn.hip
+}
+
+template <typename TZ, int KS>
+static void mul_out_attn_in_ks(ProjOutParams p, const ProjInParams& pi, const SingleStage* carry, hipStream_t stream) {
+  const int rbw = merged_row_blocks((int64_t)p.n * p.n, KS), rows = 32 * rbw;
+  p.tiles_per_i = p.ldx == p.n && p.n % Cfg<bf16_t>::VE == 0 ? 0 : (p.n + rows - 1) / rows;
+  const int64_t tiles = p.tiles_per_i ? (int64_t)p.n * p.tiles_per_i : ((int64_t)p.n * p.n + rows - 1) / rows;
+  static const SingleStage none = {};
+  if (carry && KS <= 4) single_stage_run(carry, stream);
+  if (!carry || KS <= 4) carry = &none;
+  const unsigned carried = single_stage_groups(carry);
+  const dim3 grid(carried + (unsigned)tiles), block(kPpWaves * 64);
+  if constexpr (KS <= 8) {
+    if (rbw == 2) {
+      pp_mul_out_attn_in_kernel<bf16_t, TZ, KS, 2><<<grid, block, 0, stream>>>(p, pi, *carry, carried);
+      return;
+    }
+  }
+  pp_mul_out_attn_in_kernel<bf16_t, TZ, KS, 1><<<grid, block, 0, stream>>>(p, pi, *carry, carried);
+}
+
+template <typename TZ, int KS>
+static void attn_out_attn_in_ks(const ProjOutParams& p, const ProjInParams& pi, const SingleStage* carry, hipStream_t stream) {
+  const int rbw = merged_row_blocks((int64_t)p.n * p.n, KS);
+  static const SingleStage none = {};
+  if (carry && KS <= 4) single_stage_run(carry, stream);
+  if (!carry || KS <= 4) carry = &none;
+  const unsigned carried = single_stage_groups(carry);
+  const dim3 grid(carried + (unsigned)((p.n + 4 * rbw - 1) / (4 * rbw)) * (unsigned)((p.n + 7) / 8)), block(kPpWaves * 64);
+  if constexpr (KS <= 8) {
+    if (rbw == 2) {
+      pp_attn_out_attn_in_kernel<bf16_t, TZ, KS, 2><<<grid, block, 0, stream>>>(p, pi, *carry, carried);
+      return;
+    }
+  }
+  pp_attn_out_attn_in_kernel<bf16_t, TZ, KS, 1><<<grid, block, 0, stream>>>(p, pi, *carry, carried);
+}
+
+template <typename TZ>
+int pp_trimul_out_triattn_in(const void* x, int ldx, const void* z, const void* ln_in_w, const void* ln_in_b, const void* ln_out_w,
+                             const void* ln_out_b, const void* packed, void* out, const void* att_ln_w, const void* att_ln_b,
+                             const void* att_packed, void* q, void* k, void* vt, void* tri_bias, int n, int c_z, int hidden, int heads,
+                             int key_pitch, float eps, const SingleStage* carry, hipStream_t stream) {
+  ProjOutParams p = {};
+  p.z = z;
+  p.si = (int64_t)n * c_z;
+  p.sj = c_z;
+  p.gamma = ln_in_w;
+  p.beta = ln_in_b;
+  p.gamma2 = ln_out_w;
+  p.beta2 = ln_out_b;
+  p.eps = eps;
+  p.packed = (const bf16_t*)packed + (int64_t)4 * c_z * hidden;
+  p.x = x;
+  p.ldx = ldx;
+  p.out = out;
+  p.n = n;
+  p.add_residual = 1;
+  ProjInParams pi = {};
+  attn_in_params(pi, att_ln_w, att_ln_b, att_packed, q, k, vt, tri_bias, n, heads, key_pitch, eps);
+  if (c_z == 64) mul_out_attn_in_ks<TZ, 4>(p, pi, carry, stream);
+  else if (c_z == 256) mul_out_attn_in_ks<TZ, 16>(p, pi, carry, stream);
+  else mul_out_attn_in_ks<TZ, 8>(p, pi, carry, stream);
+  return 0;
+}
+
+template <typename TZ>
+int pp_triattn_out_triattn_in(const void* o, const void* z, const void* ln_w, const void* ln_b, const void* packed, void* out,
+                              const void* next_ln_w, const void* next_ln_b, const void* next_packed, void* q, void* k, void* vt,
+                              void* tri_bias, int n, int c_z, int heads, int key_pitch, float eps, const SingleStage* carry,
+                              hipStream_t stream) {
+  ProjOutParams p = {};
+  p.z = z;
+  p.si = (int64_t)n * c_z;
+  p.sj = c_z;
+  p.gamma = ln_w;
+  p.beta = ln_b;
+  p.eps = eps;
+  p.packed = (const bf16_t*)packed + (int64_t)(4 * heads + 1) * 32 * c_z;
+  p.packed_g = (const bf16_t*)packed + (int64_t)3 * heads * 32 * c_z;
+  p.x = o;
+  p.out = out;
+  p.n = n;
+  p.add_residual = 1;
+  ProjInParams pi = {};
+  attn_in_params(pi, next_ln_w, next_ln_b, next_packed, q, k, vt, tri_bias, n, heads, key_pitch, eps);
+  if (c_z == 64) attn_out_attn_in_ks<TZ, 4>(p, pi, carry, stream);
+  else if (c_z == 256) attn_out_attn_in_ks<TZ, 16>(p, pi, carry, stream);
+  else attn_out_attn_in_ks<TZ, 8>(p, pi, carry, stream);
+  return 0;
+}
+#define PTX_INSTANTIATE_MERGED(TZ)                                                                                    \
+  template int pp_trimul_out_triattn_in<TZ>(const void*, int, const void*, const void*, const void*, const void*,     \
+                                            const void*, const void*, void*, const void*, const void*, const void*,   \
+                                            void*, void*, void*, void*, int, int, int, int, int, float,               \
+                                            const SingleStage*, hipStream_t);                                         \
+  template int pp_triattn_out_triattn_in<TZ>(const void*, const void*, const void*, const void*, const void*, void*,  \
+                                             const void*, const void*, const void*, void*, void*, void*, void*, int,  \
+                                             int, int, int, float, const SingleStage*, hipStream_t);
+PTX_INSTANTIATE_MERGED(float)
+PTX_INSTANTIATE_MERGED(bf16_t)
+#undef PTX_INSTANTIATE_MERGED
 
 #define PTX_INSTANTIATE_PACK(T)                                                                                        \
   template int pp_trimul_pack<T>(const void*, const void*, const void*, const void*, const void*, const void*, void*, \

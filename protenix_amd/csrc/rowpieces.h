@@ -143,11 +143,11 @@ __device__ __forceinline__ void norm_rows(char* frag, const TZ* x, Off off, cons
 }
 
 // The update of the tile's rows (T, [32 RBW][16 KS] at a pitch of kUpdPitch<KS>) added to the raw rows norm_rows() left
-// in registers (or stored as it is) and written in the same layout: whole lines.
+// in registers (or stored as it is) and written in the same layout: whole lines.  `raw` then holds the rows as stored.
 template <int KS> constexpr int kUpdPitch = 16 * KS + 8;
 template <typename T, typename TZ, int KS, int RBW, typename Off>
 __device__ __forceinline__ void store_rows(TZ* out, Off off, const T* upd, int wave, int lane, int add,
-                                           const typename RowPieces<TZ, KS>::V (&raw)[RBW][RowPieces<TZ, KS>::NP]) {
+                                           typename RowPieces<TZ, KS>::V (&raw)[RBW][RowPieces<TZ, KS>::NP]) {
   typedef RowPieces<TZ, KS> RP;
   constexpr int PE = RP::PE, NP = RP::NP;
   const int j = lane & 7, r8 = wave * 8 + (lane >> 3);
@@ -166,6 +166,7 @@ __device__ __forceinline__ void store_rows(TZ* out, Off off, const T* upd, int w
           for (int t = 0; t < 4; ++t) v[e + t] = from_f32<TZ>(add ? to_f32(raw[rb][q][e + t]) + u[t] : u[t]);
         }
         *reinterpret_cast<typename RP::V*>(out + o + PE * j + 8 * PE * q) = v;
+        raw[rb][q] = v;
       }
     }
   }
