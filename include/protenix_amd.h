@@ -118,11 +118,11 @@ PTX_API int ptx_layernorm_fwd(const void* x, const void* gamma, const void* beta
  *     must not depend on this launch nor this launch on it.
  *   ptx_trimul_contract_carry: ptx_trimul_contract_ld that carries a stage (of the pair rows' storage type: dtype PTX_MIXED
  *     for fp32 rows), along its own workgroups where ptx_trimul_contract_carries says 1, else in a launch in front.
- *   ptx_trimul_output_triattn_project, ptx_triattn_output_triattn_project: an output stage (residual added) and, of the rows it
- *     stores, the projection that follows it in a block, in one launch: the incoming triangle multiplication and the starting
- *     node, the starting and the ending node.  dtype PTX_BF16 or PTX_MIXED; the same bits as the two calls; q, k, vt,
- *     tri_bias must not overlap x / o.  ptx_row_stages_joined: 1 where that is the faster way (attention: 0 for the
- *     first, 1 for the second pair).
+ *   ptx_trimul_output_trimul_project, ptx_trimul_output_triattn_project, ptx_triattn_output_triattn_project: an output stage
+ *     (residual added) and, of the rows it stores, the projection that follows it in a block, in one launch: pair 0, the
+ *     outgoing and the incoming triangle multiplication (rows of 64 and 128 channels); 1, the incoming one and the starting node;
+ *     2, the starting and the ending node.  dtype PTX_BF16 or PTX_MIXED; the same bits as the two calls; the projection's results
+ *     must not overlap x / o.  ptx_row_stages_joined: 1 where that is the faster way.
  *   ptx_row_stage_resident: 1 where the launch, if it carries nothing, takes a kernel that holds all weights
  *     in LDS and is the faster for it (it cannot carry).  stage: 0 trimul_project, 1 trimul_output,
  *     2 triattn_project, 3 triattn_output.
@@ -162,7 +162,12 @@ PTX_API int ptx_triattn_output_packed(const void* o, const void* z, const void* 
 PTX_API int ptx_trimul_contract_carry(const void* a, const void* b, void* x, int n, int ldx, int c, int k_pitch, int dtype,
                       const ptx_single_stage* carry, void* stream);
 PTX_API int ptx_trimul_contract_carries(int n, int dtype);
-PTX_API int ptx_row_stages_joined(int attention, int n, int c_z, int c_hidden, int dtype);
+PTX_API int ptx_row_stages_joined(int pair, int n, int c_z, int c_hidden, int dtype);
+PTX_API int ptx_trimul_output_trimul_project(const void* x, int ldx, const void* z, const void* mask, const void* ln_in_w,
+                      const void* ln_in_b, const void* ln_out_w, const void* ln_out_b, const void* packed,
+                      void* out, const void* next_ln_w, const void* next_ln_b, const void* next_packed, void* a,
+                      void* b, int n, int c_z, int c_hidden, int k_pitch, float eps, int dtype,
+                      const ptx_single_stage* carry, void* stream);
 PTX_API int ptx_trimul_output_triattn_project(const void* x, int ldx, const void* z, const void* ln_in_w,
                       const void* ln_in_b, const void* ln_out_w, const void* ln_out_b, const void* packed,
                       void* out, const void* att_ln_w, const void* att_ln_b, const void* att_packed, void* q,
@@ -335,6 +340,13 @@ PTX_API int ptx_triattn_fwd_rows(const void* q, const void* k, const void* vt, c
                                  const void* tri_bias, const void* mask, void* o, int n, int heads,
                                  int d, int key_pitch, int mask_transposed, float inf, int row_begin,
                                  int row_count, int n_keys, int dtype, void* stream);
+/* ptx_triattn_fwd with a stage of the single track (see ptx_single_stage; operands of the pair rows' storage type, dtype
+ * PTX_MIXED for fp32 rows), run along the launch's own workgroups where ptx_triattn_fwd_carries says 1, else in front. */
+PTX_API int ptx_triattn_fwd_carries(int n, int dtype);
+PTX_API int ptx_triattn_fwd_carry(const void* q, const void* k, const void* vt, const void* g,
+                                  const void* tri_bias, const void* mask, void* o, int n, int heads,
+                                  int d, int key_pitch, int mask_transposed, float inf, int dtype,
+                                  const ptx_single_stage* carry, void* stream);
 
 /*
  * The fused attention operator on standard-layout tensors: the contract of
@@ -475,6 +487,16 @@ PTX_API int ptx_triattn_output_transition_fwd(const void* o, const void* z, cons
                                       const void* pb_ln_w, const void* pb_ln_b, const void* pb_w,
                                       void* bias, int pb_heads, int bias_f32, float pb_eps,
                                       int dtype, void* stream);
+/* The same with a stage of the single track (see ptx_single_stage; operands of the rows' storage type), run along the
+ * launch's own workgroups where ptx_triattn_output_transition_carries says 1 and a pair bias is formed, else in front. */
+PTX_API int ptx_triattn_output_transition_carries(int n);
+PTX_API int ptx_triattn_output_transition_carry(const void* o, const void* z, const void* att_ln_w,
+                                      const void* att_ln_b, const void* packed, const void* ln_w,
+                                      const void* ln_b, void* out, int n, int c_in, int heads,
+                                      int transposed, int n_factor, float att_eps, float eps,
+                                      const void* pb_ln_w, const void* pb_ln_b, const void* pb_w,
+                                      void* bias, int pb_heads, int bias_f32, float pb_eps,
+                                      int dtype, const ptx_single_stage* carry, void* stream);
 
 /*
  * Pair bias of the single-representation attention (transformer.py:191-194):

@@ -44,6 +44,7 @@ SIGNATURES = {
     "ptx_trimul_contract_carry": (_i, [_p, _p, _p, _i, _i, _i, _i, _i, _p, _p]),
     "ptx_trimul_contract_carries": (_i, [_i, _i]),
     "ptx_row_stages_joined": (_i, [_i, _i, _i, _i, _i]),
+    "ptx_trimul_output_trimul_project": (_i, [_p, _i] + [_p] * 13 + [_i, _i, _i, _i, _f, _i, _p, _p]),
     "ptx_trimul_output_triattn_project": (_i, [_p, _i] + [_p] * 14 + [_i, _i, _i, _i, _i, _f, _i, _p, _p]),
     "ptx_triattn_output_triattn_project": (_i, [_p] * 13 + [_i, _i, _i, _i, _f, _i, _p, _p]),
     "ptx_trimul_output_packed": (_i, [_p, _i] + [_p] * 7 + [_i, _i, _i, _i, _f, _i, _p, _p]),
@@ -58,6 +59,8 @@ SIGNATURES = {
     "ptx_triattn_project": (_i, [_p] * 13 + [_i, _i, _i, _i, _i, _i, _f, _i, _p]),
     "ptx_triattn_fwd": (_i, [_p] * 7 + [_i, _i, _i, _i, _i, _f, _i, _p]),
     "ptx_triattn_fwd_rows": (_i, [_p] * 7 + [_i, _i, _i, _i, _i, _f, _i, _i, _i, _i, _p]),
+    "ptx_triattn_fwd_carries": (_i, [_i, _i]),
+    "ptx_triattn_fwd_carry": (_i, [_p] * 7 + [_i, _i, _i, _i, _i, _f, _i, _p, _p]),
     "ptx_triattn_output": (_i, [_p, _p, _p, _p, _i, _i, _i, _i, _i, _p]),
     "ptx_triattn_core_workspace_elems": (_l, [_i, _i, _i]),
     "ptx_triattn_core_fwd": (_i, [_p] * 8 + [_i, _i, _i, _i, _i, _i, _p]),
@@ -72,6 +75,9 @@ SIGNATURES = {
     "ptx_triattn_output_transition_pack": (_i, [_p] * 6 + [_i, _i, _p]),
     "ptx_triattn_output_transition_fwd": (_i, [_p] * 8 + [_i, _i, _i, _i, _i, _f, _f, _p, _p, _p, _p, _i, _i,
                                                _f, _i, _p]),
+    "ptx_triattn_output_transition_carries": (_i, [_i]),
+    "ptx_triattn_output_transition_carry": (_i, [_p] * 8 + [_i, _i, _i, _i, _i, _f, _f, _p, _p, _p, _p, _i, _i,
+                                                 _f, _i, _p, _p]),
     "ptx_transition_pair_bias_fwd": (_i, [_p] * 5 + [_l, _i, _i, _i, _f, _p, _p, _p, _p, _i, _i, _f, _i, _p]),
     "ptx_single_layernorm_stage": (_i, [_p, _p, _p, _p, _p, _i, _i, _f, _i]),
     "ptx_single_linear_stage": (_i, [_p, _p, _p, _p, _p, _i, _p, _p, _p, _i, _l, _i, _i, _i, _i, _i]),

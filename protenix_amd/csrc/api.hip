@@ -361,7 +361,9 @@ PTX_API int ptx_triattn_project(const void* z, const void* ln_w, const void* ln_
 static int triattn_fwd_checked(const char* what, const void* q, const void* k, const void* vt,
                                const void* g, const void* tri_bias, const void* mask, void* o, int n,
                                int heads, int d, int key_pitch, int mask_transposed, float inf,
-                               int row_begin, int row_count, int n_keys, int dtype, void* stream) {
+                               int row_begin, int row_count, int n_keys, int dtype, void* stream,
+                               const ptx_single_stage* carry = nullptr) {
+  PTX_REQUIRE(carry_ok(carry, dtype), PTX_ERR_BAD_ARG, "%s: the carried stage must be of the pair tensor's type", what);
   if (dtype == PTX_MIXED) dtype = PTX_BF16;   // no residual-stream tensor here
   PTX_REQUIRE(dtype_ok(dtype), PTX_ERR_BAD_ARG, "%s: unknown dtype %d", what, dtype);
   PTX_REQUIRE(n >= 0 && heads >= 0, PTX_ERR_BAD_ARG, "%s: n=%d heads=%d", what, n, heads);
@@ -372,16 +374,25 @@ static int triattn_fwd_checked(const char* what, const void* q, const void* k, c
   PTX_REQUIRE(row_begin >= 0 && row_count >= 0 && row_begin <= n - row_count, PTX_ERR_BAD_ARG,
               "%s: rows %d .. +%d of %d", what, row_begin, row_count, n);
   PTX_REQUIRE(n_keys >= (n > 0) && n_keys <= n, PTX_ERR_BAD_ARG, "%s: n_keys=%d of %d", what, n_keys, n);
-  if (n == 0 || heads == 0 || row_count == 0) return PTX_OK;
-  PTX_REQUIRE(q && k && vt && tri_bias && o, PTX_ERR_BAD_ARG, "%s: null pointer", what);
+  if ((n == 0 || heads == 0 || row_count == 0) && !carry) return PTX_OK;
+  PTX_REQUIRE((q && k && vt && tri_bias && o) || n == 0 || heads == 0, PTX_ERR_BAD_ARG, "%s: null pointer", what);
   PTX_REQUIRE(aligned16(q) && aligned16(k) && aligned16(vt) && (!g || aligned16(g)) &&
                   aligned16(tri_bias) && aligned16(o),
               PTX_ERR_BAD_ARG, "%s: pointers must be 16-byte aligned", what);
   PTX_DISPATCH(dtype, ptx::triattn_fwd<T>((const T*)q, (const T*)k, (const T*)vt, (const T*)g,
                                           (const T*)tri_bias, (const T*)mask, (T*)o, n, heads,
                                           key_pitch, mask_transposed, inf, row_begin, row_count,
-                                          n_keys, (hipStream_t)stream));
+                                          n_keys, (const ptx::SingleStage*)carry, (hipStream_t)stream));
   return after_launch(what);
+}
+
+PTX_API int ptx_triattn_fwd_carries(int n, int dtype) { return ptx::triattn_fwd_carries(n, dtype != PTX_F32); }
+
+PTX_API int ptx_triattn_fwd_carry(const void* q, const void* k, const void* vt, const void* g, const void* tri_bias, const void* mask,
+                                  void* o, int n, int heads, int d, int key_pitch, int mask_transposed, float inf, int dtype,
+                                  const ptx_single_stage* carry, void* stream) {
+  return triattn_fwd_checked("triattn_fwd", q, k, vt, g, tri_bias, mask, o, n, heads, d, key_pitch,
+                             mask_transposed, inf, 0, n, n, dtype, stream, carry);
 }
 
 PTX_API int ptx_triattn_fwd(const void* q, const void* k, const void* vt, const void* g,
@@ -562,9 +573,39 @@ PTX_API int ptx_triattn_output_packed(const void* o, const void* z, const void* 
   return after_launch("triattn_output_packed");
 }
 
-PTX_API int ptx_row_stages_joined(int attention, int n, int c_z, int c_hidden, int dtype) {
-  return (dtype == PTX_BF16 || dtype == PTX_MIXED) && pair_width_ok(c_z, c_hidden, dtype) &&
-         ptx::pp_joined(attention != 0, n, c_z, c_hidden, dtype == PTX_BF16);
+PTX_API int ptx_row_stages_joined(int pair, int n, int c_z, int c_hidden, int dtype) {
+  return pair >= 0 && pair < 3 && (dtype == PTX_BF16 || dtype == PTX_MIXED) && pair_width_ok(c_z, c_hidden, dtype) &&
+         ptx::pp_joined(pair, n, c_z, c_hidden, dtype == PTX_BF16);
+}
+
+PTX_API int ptx_trimul_output_trimul_project(const void* x, int ldx, const void* z, const void* mask, const void* ln_in_w, const void* ln_in_b,
+                                             const void* ln_out_w, const void* ln_out_b, const void* packed, void* out,
+                                             const void* next_ln_w, const void* next_ln_b, const void* next_packed, void* a, void* b, int n,
+                                             int c_z, int c_hidden, int k_pitch, float eps, int dtype, const ptx_single_stage* carry,
+                                             void* stream) {
+  PTX_REQUIRE(dtype == PTX_BF16 || dtype == PTX_MIXED, PTX_ERR_BAD_ARG, "trimul_output_trimul_project: dtype %d", dtype);
+  PTX_REQUIRE(n >= 0, PTX_ERR_BAD_ARG, "trimul_output_trimul_project: n=%d", n);
+  PTX_REQUIRE(pair_width_ok(c_z, c_hidden, dtype) && c_z <= 128, PTX_ERR_UNSUPPORTED,
+              "trimul_output_trimul_project: rows of 64 or 128 channels (got c_z=%d c_hidden=%d)", c_z, c_hidden);
+  PTX_REQUIRE(k_pitch == ptx_key_pitch(n), PTX_ERR_BAD_ARG, "trimul_output_trimul_project: k_pitch=%d, expected %d", k_pitch, ptx_key_pitch(n));
+  PTX_REQUIRE(n <= 8192, PTX_ERR_UNSUPPORTED, "trimul_output_trimul_project: n=%d too large (8192 at most)", n);
+  PTX_REQUIRE(ldx >= n && ldx % 8 == 0, PTX_ERR_BAD_ARG, "trimul_output_trimul_project: ldx=%d (a multiple of 8, >= n=%d)", ldx, n);
+  if (n == 0) return PTX_OK;
+  PTX_REQUIRE(x && z && packed && out && next_packed && a && b, PTX_ERR_BAD_ARG, "trimul_output_trimul_project: null pointer");
+  PTX_REQUIRE(aligned16(x) && aligned16(out) && aligned16(z) && aligned16(packed) && (!ln_out_w || aligned16(ln_out_w)) &&
+                  (!ln_out_b || aligned16(ln_out_b)) && (!ln_in_w || aligned16(ln_in_w)) && (!ln_in_b || aligned16(ln_in_b)) &&
+                  aligned16(next_packed) && aligned16(a) && aligned16(b) && (!next_ln_w || aligned16(next_ln_w)) &&
+                  (!next_ln_b || aligned16(next_ln_b)),
+              PTX_ERR_BAD_ARG, "trimul_output_trimul_project: pointers must be 16-byte aligned");
+  PTX_REQUIRE(carry_ok(carry, dtype), PTX_ERR_BAD_ARG, "trimul_output_trimul_project: the carried stage must be of the pair tensor's type");
+  if (dtype == PTX_MIXED)
+    ptx::pp_trimul_out_trimul_in<float>(x, ldx, z, mask, ln_in_w, ln_in_b, ln_out_w, ln_out_b, packed, out, next_ln_w, next_ln_b, next_packed, a,
+                                        b, n, c_z, c_hidden, k_pitch, eps, (const ptx::SingleStage*)carry, (hipStream_t)stream);
+  else
+    ptx::pp_trimul_out_trimul_in<ptx::bf16_t>(x, ldx, z, mask, ln_in_w, ln_in_b, ln_out_w, ln_out_b, packed, out, next_ln_w, next_ln_b,
+                                              next_packed, a, b, n, c_z, c_hidden, k_pitch, eps, (const ptx::SingleStage*)carry,
+                                              (hipStream_t)stream);
+  return after_launch("trimul_output_trimul_project");
 }
 
 PTX_API int ptx_trimul_output_triattn_project(const void* x, int ldx, const void* z, const void* ln_in_w, const void* ln_in_b,
@@ -674,7 +715,7 @@ PTX_API int ptx_triattn_core_fwd(const void* q, const void* k, const void* v, co
       ptx::triattn_fwd_ex<T>((const T*)qs, (const T*)kf, (const T*)vtf, (const T*)nullptr,
                              (const T*)bf, (const T*)b1, (T*)ob, n_rows, s, heads, pitch, 0, 0.0f, 1,
                              32, (int64_t)s * heads * 32, (int64_t)heads * 32, lb, 1,
-                             (int64_t)s * heads, heads, 0, n_rows, s, (hipStream_t)stream);
+                             (int64_t)s * heads, heads, 0, n_rows, s, nullptr, (hipStream_t)stream);
     });
   }
   return after_launch("triattn_core_fwd");
@@ -874,14 +915,14 @@ PTX_API int ptx_triattn_output_transition_pack(const void* w_g, const void* w_o,
   return after_launch("triattn_output_transition_pack");
 }
 
-PTX_API int ptx_triattn_output_transition_fwd(const void* o, const void* z, const void* att_ln_w,
+PTX_API int ptx_triattn_output_transition_carry(const void* o, const void* z, const void* att_ln_w,
                                               const void* att_ln_b, const void* packed,
                                               const void* ln_w, const void* ln_b, void* out, int n,
                                               int c_in, int heads, int transposed, int n_factor,
                                               float att_eps, float eps, const void* pb_ln_w,
                                               const void* pb_ln_b, const void* pb_w, void* bias,
                                               int pb_heads, int bias_f32, float pb_eps, int dtype,
-                                              void* stream) {
+                                              const ptx_single_stage* carry, void* stream) {
   PTX_REQUIRE(dtype == PTX_BF16 || dtype == PTX_MIXED, PTX_ERR_UNSUPPORTED,
               "triattn_output_transition: built for PTX_BF16 and PTX_MIXED only (got dtype %d)", dtype);
   PTX_REQUIRE(n >= 0, PTX_ERR_BAD_ARG, "triattn_output_transition: n=%d", n);
@@ -893,8 +934,9 @@ PTX_API int ptx_triattn_output_transition_fwd(const void* o, const void* z, cons
   PTX_REQUIRE(n < 32768, PTX_ERR_UNSUPPORTED, "triattn_output_transition: n=%d too large", n);
   PTX_REQUIRE(!pb_w || (pb_heads >= 1 && pb_heads <= 32), PTX_ERR_UNSUPPORTED,
               "triattn_output_transition: pair-bias heads=%d (1..32)", pb_heads);
-  if (n == 0) return PTX_OK;
-  PTX_REQUIRE(o && z && packed && out && (!pb_w || bias), PTX_ERR_BAD_ARG,
+  PTX_REQUIRE(carry_ok(carry, dtype), PTX_ERR_BAD_ARG, "triattn_output_transition: the carried stage must be of the pair tensor's type");
+  if (n == 0 && !carry) return PTX_OK;
+  PTX_REQUIRE(n == 0 || (o && z && packed && out && (!pb_w || bias)), PTX_ERR_BAD_ARG,
               "triattn_output_transition: null pointer");
   PTX_REQUIRE(aligned16(o) && aligned16(z) && aligned16(packed) && aligned16(out) &&
                   (!att_ln_w || aligned16(att_ln_w)) && (!att_ln_b || aligned16(att_ln_b)) &&
@@ -906,13 +948,27 @@ PTX_API int ptx_triattn_output_transition_fwd(const void* o, const void* z, cons
   if (dtype == PTX_MIXED)
     rc = ptx::triattn_output_transition_fwd<ptx::bf16_t, float>(
         o, z, att_ln_w, att_ln_b, packed, ln_w, ln_b, out, n, transposed, n_factor, att_eps, eps, pb_ln_w,
-        pb_ln_b, pb_w, bias, pb_heads, bias_f32, pb_eps, (hipStream_t)stream);
+        pb_ln_b, pb_w, bias, pb_heads, bias_f32, pb_eps, (hipStream_t)stream, (const ptx::SingleStage*)carry);
   else
     rc = ptx::triattn_output_transition_fwd<ptx::bf16_t, ptx::bf16_t>(
         o, z, att_ln_w, att_ln_b, packed, ln_w, ln_b, out, n, transposed, n_factor, att_eps, eps, pb_ln_w,
-        pb_ln_b, pb_w, bias, pb_heads, bias_f32, pb_eps, (hipStream_t)stream);
+        pb_ln_b, pb_w, bias, pb_heads, bias_f32, pb_eps, (hipStream_t)stream, (const ptx::SingleStage*)carry);
   PTX_REQUIRE(rc == 0, PTX_ERR_UNSUPPORTED, "triattn_output_transition: not built for this type");
   return after_launch("triattn_output_transition");
+}
+
+PTX_API int ptx_triattn_output_transition_carries(int n) { return n >= 0 && n < 32768 && ptx::transition_carries((int64_t)n * n); }
+
+PTX_API int ptx_triattn_output_transition_fwd(const void* o, const void* z, const void* att_ln_w,
+                                              const void* att_ln_b, const void* packed,
+                                              const void* ln_w, const void* ln_b, void* out, int n,
+                                              int c_in, int heads, int transposed, int n_factor,
+                                              float att_eps, float eps, const void* pb_ln_w,
+                                              const void* pb_ln_b, const void* pb_w, void* bias,
+                                              int pb_heads, int bias_f32, float pb_eps, int dtype,
+                                              void* stream) {
+  return ptx_triattn_output_transition_carry(o, z, att_ln_w, att_ln_b, packed, ln_w, ln_b, out, n, c_in, heads, transposed, n_factor,
+                                             att_eps, eps, pb_ln_w, pb_ln_b, pb_w, bias, pb_heads, bias_f32, pb_eps, dtype, nullptr, stream);
 }
 
 static_assert(sizeof(ptx::SingleStage) <= sizeof(ptx_single_stage), "ptx_single_stage is too small");

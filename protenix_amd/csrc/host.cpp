@@ -480,15 +480,18 @@ struct Run {
   // 2615 / 2595, 1024 5090 / 5047, 2048 28073 / 27832; 16-bit rows, 768 2403 / 2339, 1024 4656 / 4517, 1536 12661 / 12403.
   // Chained updates (Block::chain) have two launches fewer to carry: small products carry then, elsewhere the LayerNorms
   // are launched by themselves too.
-  bool mul_alone = false, att_alone = false, contract_carries = false, chained = false;
+  bool mul_alone = false, att_alone = false, contract_carries = false, chained = false, core_carries = false;
   void row_stages(int n, int c_z, int hidden, int dt) {
     mul_alone = ptx_row_stage_resident(0, n, c_z, hidden, dt);
     att_alone = n >= 480 && ptx_row_stage_resident(2, n, c_z, hidden, dt);
     contract_carries = ptx_trimul_contract_carries(n, dt);
   }
-  // stage 4: of the contractions, which take part where the updates are chained (two launches fewer to carry)
+  // stage 4: of the contractions, which take part where the updates are chained (two launches fewer to carry), 5: of the
+  // attention cores, see Block::joins_products
   const ptx_single_stage* carry(int stage) {
-    if ((stage == 0 && mul_alone) || (stage == 2 && att_alone) || (stage == 4 && !(chained && contract_carries))) return nullptr;
+    if ((stage == 0 && mul_alone) || (stage == 2 && att_alone) || (stage == 4 && !(chained && contract_carries)) ||
+        (stage == 5 && !core_carries))
+      return nullptr;
     if ((mul_alone || att_alone || (chained && !contract_carries)) && singles.next < singles.list.size() && singles.list[singles.next].layernorm) run_next();
     return singles.take();
   }
@@ -500,6 +503,15 @@ struct Run {
   void run_rest() {
     while (singles.next < singles.list.size()) run_next();
     singles.clear();
+  }
+  // The same in front of a launch that rewrites the pair bias but can carry a stage: the last one, which does not read it, is
+  // left to it.
+  optional<ptx_single_stage> run_rest_but_last() {
+    optional<ptx_single_stage> last;
+    while (singles.next + 1 < singles.list.size()) run_next();
+    if (singles.next < singles.list.size()) last = *singles.take();
+    singles.clear();
+    return last;
   }
   // (0xff bytes are NaNs in every type)
   Tensor workspace(int64_t bytes, const at::TensorOptions& like) const {
@@ -513,16 +525,21 @@ struct Run {
   }
 };
 
+void run_contraction(const TriMul& w, const void* a, const void* b, void* x, int n, int dt, Run& run) {
+  const ptx_single_stage* carry4 = run.carry(4);
+  run.launch("trimul_contract", [&] {
+    return ptx_trimul_contract_carry(a, b, x, n, (n + 7) / 8 * 8, w.c_h, ptx_key_pitch(n), dt, carry4, run.st);
+  });
+}
+
 // projection and product; the product is left in x
 void run_trimul_product(const TriMul& w, const void* z, const Tensor& mask, int n, int dt, void* a, void* b, void* x, Run& run) {
-  const int pitch = ptx_key_pitch(n), ldx = (n + 7) / 8 * 8;
   const ptx_single_stage* carry0 = run.carry(0);
   run.launch("trimul_project", [&] {
-    return ptx_trimul_project_packed(z, ptr(mask), w.ln_in_w, w.ln_in_b, w.packed, a, b, n, w.c_z, w.c_h, pitch,
+    return ptx_trimul_project_packed(z, ptr(mask), w.ln_in_w, w.ln_in_b, w.packed, a, b, n, w.c_z, w.c_h, ptx_key_pitch(n),
                                      w.incoming, kEps, dt, carry0, run.st);
   });
-  const ptx_single_stage* carry4 = run.carry(4);
-  run.launch("trimul_contract", [&] { return ptx_trimul_contract_carry(a, b, x, n, ldx, w.c_h, pitch, dt, carry4, run.st); });
+  run_contraction(w, a, b, x, n, dt, run);
 }
 
 void run_trimul_output(const TriMul& w, const void* x, const void* z, void* out, int n, bool add, int dt, Run& run) {
@@ -557,8 +574,9 @@ void run_attention(const TriAtt& w, const void* q, const void* k, const void* vt
                                   dt, run.st);
     });
   } else {
+    const ptx_single_stage* carry5 = run.carry(5);
     run.launch("triattn_fwd", [&] {
-      return ptx_triattn_fwd(q, k, vt, gate, tb, m, o, n, w.heads, 32, pitch, 0, w.inf, dt, run.st);
+      return ptx_triattn_fwd_carry(q, k, vt, gate, tb, m, o, n, w.heads, 32, pitch, 0, w.inf, dt, carry5, run.st);
     });
   }
 }
@@ -691,8 +709,10 @@ struct Block : Plan {
         void* zb = zp + b * plane;
         chain(zb, mask(b), n, dt, es, ws, run);
         if (fused) {
-          if (b == 0) run.run_rest();   // (the bias is about to be rewritten)
-          output_transition(zb, attention_output(n, es, ws), n, dt, bias ? bias + b * bias_plane : nullptr, run);
+          optional<ptx_single_stage> last;
+          if (b == 0 && bias && ptx_triattn_output_transition_carries(n)) last = run.run_rest_but_last();
+          else if (b == 0) run.run_rest();   // (the bias is about to be rewritten)
+          output_transition(zb, attention_output(n, es, ws), n, dt, bias ? bias + b * bias_plane : nullptr, last ? &*last : nullptr, run);
         } else {
           output(end, zb, attention_output(n, es, ws), n, dt, run);
         }
@@ -707,7 +727,7 @@ struct Block : Plan {
           void* zb = zp + b * plane;
           const TriAttWs s = run_triatt_core(end, zb, mask(b), n, dt, es, ws, run);
           if (b == 0) run.run_rest();   // (the bias is about to be rewritten)
-          output_transition(zb, s.g, n, dt, bias ? bias + b * bias_plane : nullptr, run);
+          output_transition(zb, s.g, n, dt, bias ? bias + b * bias_plane : nullptr, nullptr, run);
         }
         return;
       }
@@ -728,7 +748,16 @@ struct Block : Plan {
   // Whether an output stage projects for the update behind it (16-bit arithmetic; not where launches are timed one by one).
   bool chains(const Run& run, int n, int dt) const {
     return !run.timing && out.c_h == in.c_h && start.heads == end.heads && ptx_triattn_late_gate(c_z, start.heads, dt) &&
-           ptx_row_stages_joined(0, n, c_z, out.c_h, dt);
+           ptx_row_stages_joined(1, n, c_z, out.c_h, dt);
+  }
+  // With a single track only where the block's other launches can carry its seven stages: two projections and output stages
+  // and the two products carry six, the transition the last one or else an attention core one more.
+  bool joins_products(int n, int dt) const {
+    return ptx_row_stages_joined(0, n, c_z, out.c_h, dt) &&
+           (c_s == 0 || (fused && ptx_trimul_contract_carries(n, dt) && (ptx_triattn_output_transition_carries(n) || ptx_triattn_fwd_carries(n, dt))));
+  }
+  bool core_carries(int n, int dt) const {
+    return c_s > 0 && joins_products(n, dt) && !ptx_triattn_output_transition_carries(n);
   }
   // The block up to the ending node's attention output.
   void chain(void* z, const Mask& mask, int n, int dt, int64_t es, void* ws, Run& run) const {
@@ -736,8 +765,17 @@ struct Block : Plan {
     const ChainWs s(c, n, out.c_h, start.heads, es);
     const int ldx = (n + 7) / 8 * 8, pitch = ptx_key_pitch(n);
     run_trimul_product(out, z, mask.m, n, dt, s.a, s.b, s.x, run);
-    run_trimul_output(out, s.x, z, z, n, true, dt, run);
-    run_trimul_product(in, z, mask.m, n, dt, s.a, s.b, s.x, run);
+    if (joins_products(n, dt)) {
+      const ptx_single_stage* carry0 = run.carry(1);
+      run.launch("trimul_output_trimul_project", [&] {
+        return ptx_trimul_output_trimul_project(s.x, ldx, z, ptr(mask.m), out.ln_in_w, out.ln_in_b, out.ln_out_w, out.ln_out_b, out.packed, z,
+                                                in.ln_in_w, in.ln_in_b, in.packed, s.a, s.b, n, c_z, out.c_h, pitch, kEps, dt, carry0, run.st);
+      });
+      run_contraction(in, s.a, s.b, s.x, n, dt, run);
+    } else {
+      run_trimul_output(out, s.x, z, z, n, true, dt, run);
+      run_trimul_product(in, z, mask.m, n, dt, s.a, s.b, s.x, run);
+    }
     const ptx_single_stage* carry1 = run.carry(1);
     run.launch("trimul_output_triattn_project", [&] {
       return ptx_trimul_output_triattn_project(s.x, ldx, z, in.ln_in_w, in.ln_in_b, in.ln_out_w, in.ln_out_b, in.packed, z, start.ln_w,
@@ -745,7 +783,7 @@ struct Block : Plan {
                                                carry1, run.st);
     });
     run_attention(start, s.q, s.k, s.vt, nullptr, s.tb, s.o, mask, n, dt, run);
-    if (ptx_row_stages_joined(1, n, c_z, out.c_h, dt)) {
+    if (ptx_row_stages_joined(2, n, c_z, out.c_h, dt)) {
       const ptx_single_stage* carry3 = run.carry(3);
       run.launch("triattn_output_triattn_project", [&] {
         return ptx_triattn_output_triattn_project(s.o, z, start.ln_w, start.ln_b, start.packed, z, end.ln_w, end.ln_b, end.packed, s.q, s.k,
@@ -776,12 +814,12 @@ struct Block : Plan {
     });
   }
   // the ending node's output stage and the transition, with the pair bias where one is wanted
-  void output_transition(void* z, const void* o, int n, int dt, float* bias, Run& run) const {
+  void output_transition(void* z, const void* o, int n, int dt, float* bias, const ptx_single_stage* carry, Run& run) const {
     run.launch("triattn_output_transition", [&] {
-      return ptx_triattn_output_transition_fwd(o, z, end.ln_w, end.ln_b, tr_packed, tr_ln_w, tr_ln_b, z, n,
-                                               c_z, end.heads, end.transposed, n_factor, kEps, kEps, bias ? pb_ln_w : nullptr,
-                                               bias ? pb_ln_b : nullptr, bias ? pb_w : nullptr, bias,
-                                               bias ? heads : 0, 1, kEps, dt, run.st);
+      return ptx_triattn_output_transition_carry(o, z, end.ln_w, end.ln_b, tr_packed, tr_ln_w, tr_ln_b, z, n,
+                                                 c_z, end.heads, end.transposed, n_factor, kEps, kEps, bias ? pb_ln_w : nullptr,
+                                                 bias ? pb_ln_b : nullptr, bias ? pb_w : nullptr, bias,
+                                                 bias ? heads : 0, 1, kEps, dt, carry, run.st);
     });
   }
 
@@ -865,6 +903,7 @@ struct Call {
       const int dt = code_of_rows(z_.scalar_type(), b->compute);
       run_.row_stages(n_, b->c_z, b->out.c_h, dt);
       run_.chained = b->chains(run_, n_, dt);
+      run_.core_carries = run_.chained && b->core_carries(n_, dt);
       b->pair_track(z_, masks_, batch_, n_, ws_.data_ptr(), bias, run_);
       if (single) {
         b->single_track(run_.singles, s_now_, mid_.data_ptr(), s_out_.data_ptr(), bias, s_->scalar_type(), batch_, n_, sws_.data_ptr());

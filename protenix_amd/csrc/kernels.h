@@ -52,6 +52,7 @@ template <typename T, typename TZ = T>
 int transition_fwd(const void* x, const void* ln_w, const void* ln_b, const void* packed,
                    void* out, int64_t rows, int c, int n_factor, int add_residual, float eps,
                    hipStream_t stream);
+struct SingleStage;
 // The transition on rows of 128 channels (16-bit arithmetic) with the pair bias of the single
 // attention, bias[h][row] = (W LN_pb(out[row]))[h], formed from the finished rows in its epilogue.
 template <typename T, typename TZ = T>
@@ -76,7 +77,9 @@ int triattn_output_transition_fwd(const void* o, const void* z, const void* att_
                                   const void* ln_b, void* out, int n, int transposed, int n_factor,
                                   float att_eps, float eps, const void* pb_ln_w, const void* pb_ln_b,
                                   const void* pb_w, void* bias, int heads, int bias_f32, float pb_eps,
-                                  hipStream_t stream);
+                                  hipStream_t stream, const SingleStage* carry = nullptr);
+// Whether that launch, with a pair bias, runs a carried stage along its own workgroups (else in front).
+bool transition_carries(int64_t n_rows);
 template <typename T, typename TZ = T>
 int pair_bias_fwd(const void* z, const void* ln_w, const void* ln_b, const void* w, void* bias,
                   int n, int c_z, int heads, int out_f32, float eps, hipStream_t stream);
@@ -122,6 +125,8 @@ int single_stage_run(const SingleStage* s, hipStream_t stream);
 // carry: null, or a stage of the single track that the launch's first workgroups run (it must not depend on the launch), where
 // nt_gemm_carries(); elsewhere the stage is launched in front.
 bool nt_gemm_carries(int n, bool bits16);
+// How far the product reads its operands' K for n tokens: what the projections write, zeros from n on.
+int nt_gemm_k_extent(int n, bool bits16);
 template <typename T>
 int nt_gemm_batched(const T* a, const T* b, T* x, int n, int ldx, int k_pitch, int batch, const SingleStage* carry, hipStream_t stream);
 
@@ -167,12 +172,17 @@ template <typename T, typename TZ = T>
 int pp_triattn_out(const void* o, const void* z, const void* ln_w, const void* ln_b, const void* packed, void* out,
                    int n, int c_z, int heads, int transposed, int add_residual, float eps, const SingleStage* carry,
                    hipStream_t stream);
-// Whether a triangle multiplication's (attention: a starting node's) output stage and the projection behind it are faster in
-// one launch, in 16-bit arithmetic.
-bool pp_joined(bool attention, int n, int c_z, int hidden, bool rows16);
-// An output stage and the projection of the attention that reads its rows next, in one launch (16-bit arithmetic, residual
-// added; the projection writes no gate): the incoming triangle multiplication -> the starting node, the starting -> the
-// ending node.
+// Whether a triangle update's output stage and the projection behind it are faster in
+// one launch, in 16-bit arithmetic; pair: 0 the outgoing multiplication -> the incoming one, 1 the incoming multiplication -> the
+// starting node, 2 the starting -> the ending node.
+bool pp_joined(int pair, int n, int c_z, int hidden, bool rows16);
+// An output stage and the projection that reads its rows next, in one launch (16-bit arithmetic, residual added; attentions'
+// projections write no gate): these pairs.
+template <typename TZ>
+int pp_trimul_out_trimul_in(const void* x, int ldx, const void* z, const void* mask, const void* ln_in_w, const void* ln_in_b,
+                            const void* ln_out_w, const void* ln_out_b, const void* packed, void* out, const void* next_ln_w,
+                            const void* next_ln_b, const void* next_packed, void* a, void* b, int n, int c_z, int hidden, int k_pitch,
+                            float eps, const SingleStage* carry, hipStream_t stream);
 template <typename TZ>
 int pp_trimul_out_triattn_in(const void* x, int ldx, const void* z, const void* ln_in_w, const void* ln_in_b, const void* ln_out_w,
                              const void* ln_out_b, const void* packed, void* out, const void* att_ln_w, const void* att_ln_b,
@@ -193,7 +203,10 @@ int pp_triattn_out_triattn_in(const void* o, const void* z, const void* ln_w, co
 template <typename T>
 int triattn_fwd(const T* q, const T* k, const T* vt, const T* g, const T* tri_bias, const T* mask,
                 T* o, int n, int heads, int key_pitch, int mask_transposed, float inf,
-                int row_begin, int row_count, int n_keys, hipStream_t stream);
+                int row_begin, int row_count, int n_keys, const SingleStage* carry, hipStream_t stream);
+// carry: null, or a stage of the single track that the launch's first workgroups run where triattn_fwd_carries(); elsewhere it
+// is launched in front.
+bool triattn_fwd_carries(int n, bool bits16);
 // The same core on n_rows rows of n queries / keys, with q / g / o addressed through element
 // strides (head, row, query), an optional gate (g may be null), the mask either 0/1 values or
 // (mask_is_bias) an additive bias per (row, key), and an optional log2-sum-exp2 output.
@@ -204,7 +217,7 @@ int triattn_fwd_ex(const T* q, const T* k, const T* vt, const T* g, const T* tri
                    const T* mask, T* o, int n_rows, int n, int heads, int key_pitch,
                    int mask_transposed, float inf, int mask_is_bias, int64_t sh, int64_t si,
                    int64_t sj, float* lse, int64_t lh, int64_t li, int64_t lj, int row_begin,
-                   int row_count, int n_keys, hipStream_t stream);
+                   int row_count, int n_keys, const SingleStage* carry, hipStream_t stream);
 // Standard-layout K, V [n_rows][n][heads][32] and bias [heads][n][n] -> the core's fragment-
 // ordered K, V^T and bias (bias and nothing else multiplied by log2(e)); q [n_rows][n][heads][32]
 // -> qs, the same layout multiplied by log2(e).

@@ -56,6 +56,7 @@ template <int KS> struct PpWidths {
 // of the 16-byte vector length, so that vectors of consecutive rows stay inside one i); otherwise ROWS
 // positions j of one i, the last tile of an i partial.
 struct TileRows {
+  static constexpr bool kPatch = false;
   int64_t p0;
   int i0, j0, n;
   int64_t n_rows;
@@ -99,33 +100,115 @@ struct ProjInParams {
   int heads;
   int slices;             // workgroups per tile, each with its share of the output columns (see in_slices)
   unsigned tiles;
+  unsigned n_kb;          // trimul_in: blocks of 8 inner indices
   int share;              // trimul_in: a wave's chunks per slice
   float q_scale;
 };
 
 }  // namespace
 
-// a, b[c][i][k] = mask * sigmoid(gate) * projection in the contraction's fragment order.  Tile: a patch of 4 * RBW
-// outer indices i x 8 inner indices k, which makes a row block's 32 values of one channel 64 contiguous bytes.
-template <typename T, typename TZ, int KS, int RBW>
-__global__ __launch_bounds__(kPpWaves * 64, (kPpMinWaves<T, KS>)) void pp_trimul_in_kernel(ProjInParams p, SingleStage carry, unsigned carried) {
+// The output columns of a triangle multiplication's projection: a, b[c][i][k] = mask * sigmoid(gate) * projection in the
+// contraction's fragment order, from the normalised rows in LDS of a patch of 4 * RBW outer indices i x 8 inner indices
+// k, which makes a row block's 32 values of one channel 64 contiguous bytes.
+template <typename T, int KS, int RBW>
+struct MulColumns {
   typedef typename Vec8<T>::type V8;
   typedef typename VecE<T>::type VE_t;
   typedef Cfg<T> C;
-  constexpr int CPM = PpWidths<KS>::HIDDEN / 32;    // chunks (of 32 channels) per operand
-  constexpr int CHW = 2 * CPM / kPpWaves;           // chunks per wave, all slices
-  constexpr int kFrag = RBW * FragLds<T, KS>::ROWBLOCK, kStage = kPpWaves * 32 * C::PITCH * (int)sizeof(T);
-  __shared__ __attribute__((aligned(16))) char smem[cmax(kFrag + kStage + 128 * RBW, kStageLds)];
+  static constexpr int CPM = PpWidths<KS>::HIDDEN / 32;    // chunks (of 32 channels) per operand
+  static constexpr int CHW = 2 * CPM / kPpWaves;           // chunks per wave, all slices
+  static constexpr int kStage = kPpWaves * 32 * C::PITCH * (int)sizeof(T) + 128 * RBW;   // LDS beside the rows': staging tiles, mask
+  V8 w[2][KS];
+  __device__ __forceinline__ void load_w(const ProjInParams& p, int ch, int lane) {
+    const T* packed = (const T*)p.packed;
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int kk = 0; kk < KS; ++kk) w[t][kk] = packed_frag<T>(packed, (ch * 2 + t) * KS + kk, lane);
+  }
+  static __device__ __forceinline__ float* mask_of(char* stage_lds) { return reinterpret_cast<float*>(stage_lds + kStage - 128 * RBW); }
+  // the patch's mask into LDS
+  static __device__ __forceinline__ void put_mask(const ProjInParams& p, char* stage_lds, int pi0, int pk0) {
+    if (threadIdx.x < 32 * RBW) {
+      const int n = p.n, i = min(pi0 + (int)(threadIdx.x >> 3), n - 1), k = pk0 + (int)(threadIdx.x & 7);
+      float mv = 1.0f;
+      if (p.mask) mv = to_f32(((const T*)p.mask)[i * p.mi + min(k, n - 1) * p.mk]);
+      mask_of(stage_lds)[threadIdx.x] = k < n ? mv : 0.0f;   // (the contraction relies on zeros between n and the pitch)
+    }
+  }
+  // chunks c_begin .. c_end - 1 of the wave's; the first one's weights have been requested
+  __device__ __forceinline__ void run(const ProjInParams& p, const char* frag, char* stage_lds, int pi0, int pk0, int c_begin, int c_end, int wave,
+                                      int lane) {
+    T (*stage)[32 * C::PITCH] = reinterpret_cast<T (*)[32 * C::PITCH]>(stage_lds);
+    const float* const lmask = mask_of(stage_lds);
+    T* const out_a = (T*)p.out[0];
+    T* const out_b = (T*)p.out[1];
+    const int n = p.n, g = lane >> 5;
+    T* st = stage[wave];
+    const int n_rb = (n + 31) >> 5, n_ks = p.pitch >> 4;
+    // this lane's vector of row block 0 inside a channel block's planes
+    uint32_t rel[C::NPASS];
+#pragma unroll
+    for (int ps = 0; ps < C::NPASS; ++ps) {
+      int chn, r0;
+      stage_coord<T>(ps, lane, chn, r0);
+      const int i = pi0 + (r0 >> 3);
+      rel[ps] = (uint32_t)(trimul_frag_offset(chn, i >> 5, pk0 >> 4, n_rb, n_ks) + ((pk0 >> 3) & 1) * 256 + (i & 31) * 8 + (r0 & 7));
+    }
+#pragma unroll
+    for (int c = 0; c < CHW; ++c) {
+      if (c < c_begin || c >= c_end) continue;
+      const int ch = wave * CHW + c;
+      T* outp = (ch < CPM ? out_a : out_b) + trimul_frag_offset((ch % CPM) * 32, 0, 0, n_rb, n_ks);
+#pragma unroll
+      for (int rb = 0; rb < RBW; ++rb) {
+        f32x16 acc[2];
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[0][r] = acc[1][r] = 0.0f;
+#pragma unroll
+        for (int kk = 0; kk < KS; ++kk) {
+          const V8 xv = FragLds<T, KS>::get(frag, rb, kk, lane);
+          mma32(acc[0], xv, w[0][kk]);   // lane <-> channel, register <-> row
+          mma32(acc[1], xv, w[1][kk]);
+        }
+        if (rb == RBW - 1 && c + 1 < CHW && c + 1 < c_end) load_w(p, ch + 1, lane);
+        float vals[16];
+#pragma unroll
+        for (int qd = 0; qd < 4; ++qd) {
+          const f32x4 m4 = *reinterpret_cast<const f32x4*>(&lmask[rb * 32 + 8 * qd + 4 * g]);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const int r = 4 * qd + e;
+            vals[r] = m4[e] * sigmoidf_fast(acc[1][r]) * acc[0][r];
+          }
+        }
+        wave_lds_sync();
+        stage_put<T>(st, vals, lane);
+        wave_lds_sync();
+        // row block rb: outer indices 4 rb .. 4 rb + 3 further on; a patch of 4 RBW outer indices lies in one block of 32
+#pragma unroll
+        for (int ps = 0; ps < C::NPASS; ++ps) {
+          int chn, r0;
+          stage_coord<T>(ps, lane, chn, r0);
+          *reinterpret_cast<VE_t*>(outp + rel[ps] + rb * 32) = stage_get_vec<T>(st, chn, r0);
+        }
+      }
+    }
+  }
+};
+
+// Tiles in the order of the memory rows they read.
+template <typename T, typename TZ, int KS, int RBW>
+__global__ __launch_bounds__(kPpWaves * 64, (kPpMinWaves<T, KS>)) void pp_trimul_in_kernel(ProjInParams p, SingleStage carry, unsigned carried) {
+  typedef MulColumns<T, KS, RBW> Columns;
+  constexpr int kFrag = RBW * FragLds<T, KS>::ROWBLOCK;
+  __shared__ __attribute__((aligned(16))) char smem[cmax(kFrag + Columns::kStage, kStageLds)];
   PTX_CARRIED_STAGE();
   char* const frag = smem;
-  T (*stage)[32 * C::PITCH] = reinterpret_cast<T (*)[32 * C::PITCH]>(smem + kFrag);
-  float* const lmask = reinterpret_cast<float*>(smem + kFrag + kStage);
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int g = lane >> 5;
   const int n = p.n;
-  const uint32_t n_kb = (uint32_t)p.pitch >> 3, n_ip = (uint32_t)(n + 4 * RBW - 1) / (4 * RBW);
-  // Patches in the order of the memory rows they read, back to front behind a kernel that wrote the pair tensor
-  // front to back (the tail is what the memory-side cache still holds).
+  const uint32_t n_kb = p.n_kb, n_ip = (uint32_t)(n + 4 * RBW - 1) / (4 * RBW);
+  // back to front behind a kernel that wrote the pair tensor front to back (the tail is what the memory-side cache still holds)
   const uint32_t tiles = p.tiles, slice = (block >= tiles) + (block >= 2 * tiles) + (block >= 3 * tiles);
   const uint32_t bx = xcd_run(block - slice * tiles, tiles), tile = p.backward ? tiles - 1 - bx : bx;
   int pi0, pk0;
@@ -138,14 +221,7 @@ __global__ __launch_bounds__(kPpWaves * 64, (kPpMinWaves<T, KS>)) void pp_trimul
     pi0 = ip * (4 * RBW);
     pk0 = (tile - ip * n_kb) * 8;
   }
-  const T* packed = (const T*)p.packed;
-  V8 w[2][KS];
-  auto load_w = [&](int ch) {
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-      for (int kk = 0; kk < KS; ++kk) w[t][kk] = packed_frag<T>(packed, (ch * 2 + t) * KS + kk, lane);
-  };
+  Columns columns;
   typename RowPieces<TZ, KS>::V raw[RBW][RowPieces<TZ, KS>::NP];
   norm_rows<T, TZ, KS, RBW>(
       frag, (const TZ*)p.x,
@@ -155,65 +231,10 @@ __global__ __launch_bounds__(kPpWaves * 64, (kPpMinWaves<T, KS>)) void pp_trimul
       },
       (const T*)p.gamma, (const T*)p.beta, p.eps, wave, lane, raw);
   const int c_begin = slice * p.share, c_end = c_begin + p.share;   // this slice's chunks of every wave
-  load_w(wave * CHW + c_begin);
-  if (threadIdx.x < 32 * RBW) {
-    const int i = min(pi0 + (int)(threadIdx.x >> 3), n - 1), k = pk0 + (int)(threadIdx.x & 7);
-    float mv = 1.0f;
-    if (p.mask) mv = to_f32(((const T*)p.mask)[i * p.mi + min(k, n - 1) * p.mk]);
-    lmask[threadIdx.x] = k < n ? mv : 0.0f;   // (the contraction relies on zeros between n and the pitch)
-  }
+  columns.load_w(p, wave * Columns::CHW + c_begin, lane);
+  Columns::put_mask(p, smem + kFrag, pi0, pk0);
   __syncthreads();
-
-  T* st = stage[wave];
-  const int n_rb = (n + 31) >> 5, n_ks = p.pitch >> 4;
-  // this lane's vector of row block 0 inside a channel block's planes
-  uint32_t rel[C::NPASS];
-#pragma unroll
-  for (int ps = 0; ps < C::NPASS; ++ps) {
-    int chn, r0;
-    stage_coord<T>(ps, lane, chn, r0);
-    const int i = pi0 + (r0 >> 3);
-    rel[ps] = (uint32_t)(trimul_frag_offset(chn, i >> 5, pk0 >> 4, n_rb, n_ks) + ((pk0 >> 3) & 1) * 256 + (i & 31) * 8 + (r0 & 7));
-  }
-#pragma unroll
-  for (int c = 0; c < CHW; ++c) {
-    if (c < c_begin || c >= c_end) continue;
-    const int ch = wave * CHW + c;
-    T* outp = (T*)p.out[ch / CPM] + trimul_frag_offset((ch % CPM) * 32, 0, 0, n_rb, n_ks);
-#pragma unroll
-    for (int rb = 0; rb < RBW; ++rb) {
-      f32x16 acc[2];
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[0][r] = acc[1][r] = 0.0f;
-#pragma unroll
-      for (int kk = 0; kk < KS; ++kk) {
-        const V8 xv = FragLds<T, KS>::get(frag, rb, kk, lane);
-        mma32(acc[0], xv, w[0][kk]);   // lane <-> channel, register <-> row
-        mma32(acc[1], xv, w[1][kk]);
-      }
-      if (rb == RBW - 1 && c + 1 < CHW && c + 1 < c_end) load_w(ch + 1);
-      float vals[16];
-#pragma unroll
-      for (int qd = 0; qd < 4; ++qd) {
-        const f32x4 m4 = *reinterpret_cast<const f32x4*>(&lmask[rb * 32 + 8 * qd + 4 * g]);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int r = 4 * qd + e;
-          vals[r] = m4[e] * sigmoidf_fast(acc[1][r]) * acc[0][r];
-        }
-      }
-      wave_lds_sync();
-      stage_put<T>(st, vals, lane);
-      wave_lds_sync();
-      // row block rb: outer indices 4 rb .. 4 rb + 3 further on; a patch of 4 RBW outer indices lies in one block of 32
-#pragma unroll
-      for (int ps = 0; ps < C::NPASS; ++ps) {
-        int chn, r0;
-        stage_coord<T>(ps, lane, chn, r0);
-        *reinterpret_cast<VE_t*>(outp + rel[ps] + rb * 32) = stage_get_vec<T>(st, chn, r0);
-      }
-    }
-  }
+  columns.run(p, frag, smem + kFrag, pi0, pk0, c_begin, c_end, wave, lane);
 }
 
 // The output columns of an attention projection: q (scaled), K, V^T, triangle bias and (GATE) sigmoid(gate) in the attention
@@ -387,7 +408,7 @@ struct ProjOutParams {
 };
 }  // namespace
 
-// Element offset of a tile's row in z and out, or -1.
+// Element offset of a tile's row in z and out, or -1; clamped: past the end that of a row the tile has.
 template <typename Rows> struct ZRow {
   const ProjOutParams& p;
   const Rows& tr;
@@ -396,6 +417,11 @@ template <typename Rows> struct ZRow {
     const bool ok = tr.at(r, i, j);
     const int64_t o = i * p.si + j * p.sj;
     return ok ? o : -1;
+  }
+  __device__ __forceinline__ int64_t clamped(int r) const {
+    int i, j;
+    tr.at(r, i, j);
+    return i * p.si + j * p.sj;
   }
 };
 
@@ -419,23 +445,30 @@ template <typename T, typename TZ, int KS, int RBW> struct MulOut {
     const int n = p.n;
     const T* packed = (const T*)p.packed;
 
-    // the triangle product's rows of every channel: vectors of VE rows
-    constexpr int VPC = 32 * RBW / C::VE, NV = HIDDEN * VPC / (kPpWaves * 64);
-    const int v0 = (threadIdx.x % VPC) * C::VE, c0 = threadIdx.x / VPC;
-    VE_t xv[NV];
+    // the triangle product's rows of every channel: vectors of VE rows, or for a patch of 8 i x 4 * RBW j of XE of
+    // an i's j, in which order they then lie in LDS
+    constexpr bool kPatch = Rows::kPatch;
+    constexpr int JW = 4 * RBW, XE = kPatch && JW < C::VE ? JW : C::VE;
+    typedef typename std::conditional<XE == C::VE, VE_t, u32x2>::type X_t;
+    static_assert(sizeof(X_t) == XE * sizeof(T), "one vector");
+    auto x_pos = [](int r) { return kPatch ? (r & 7) * JW + (r >> 3) : r; };
+    constexpr int VPC = 32 * RBW / XE, NV = HIDDEN * VPC / (kPpWaves * 64);
+    const int v0 = (threadIdx.x % VPC) * XE, c0 = threadIdx.x / VPC;
+    X_t xv[NV];
     {
       int i, j;
-      tr.at(v0, i, j);
+      tr.at(kPatch ? (v0 % JW) * 8 + v0 / JW : v0, i, j);
+      if (kPatch) j &= ~(XE - 1);   // (clamped to n - 1: the vector that holds it)
       // (a tile past the end of a plane re-reads its last vector: those rows are not stored)
-      const int64_t off = min((int64_t)i * p.ldx + j, (int64_t)n * p.ldx - C::VE) & ~(int64_t)(C::VE - 1);
+      const int64_t off = min((int64_t)i * p.ldx + j, (int64_t)n * p.ldx - XE) & ~(int64_t)(XE - 1);
       const T* src = (const T*)p.x + off;
       const int64_t plane = (int64_t)n * p.ldx;
 #pragma unroll
-      for (int q = 0; q < NV; ++q) xv[q] = *reinterpret_cast<const VE_t*>(src + (c0 + q * (kPpWaves * 64 / VPC)) * plane);
+      for (int q = 0; q < NV; ++q) xv[q] = *reinterpret_cast<const X_t*>(src + (c0 + q * (kPpWaves * 64 / VPC)) * plane);
     }
     const ZRow<Rows> z_row{p, tr};
     norm_rows<T, TZ, KS, RBW>(
-        frag, (const TZ*)p.z, [&](int r) { return max(z_row(r), (int64_t)0); }, (const T*)p.gamma, (const T*)p.beta, p.eps,
+        frag, (const TZ*)p.z, [&](int r) { return z_row.clamped(r); }, (const T*)p.gamma, (const T*)p.beta, p.eps,
         wave, lane, raw);
     T* xt = reinterpret_cast<T*>(scratch);
 #pragma unroll
@@ -443,7 +476,7 @@ template <typename T, typename TZ, int KS, int RBW> struct MulOut {
       u32x2* d = reinterpret_cast<u32x2*>(xt + (c0 + q * (kPpWaves * 64 / VPC)) * XP + v0);
       const u32x2* s = reinterpret_cast<const u32x2*>(&xv[q]);
       d[0] = s[0];
-      d[1] = s[1];
+      if (sizeof(X_t) == 16) d[1] = s[sizeof(X_t) / 8 - 1];
     }
     __syncthreads();
     {
@@ -458,7 +491,7 @@ template <typename T, typename TZ, int KS, int RBW> struct MulOut {
 #pragma unroll
         for (int q = 0; q < NP; ++q)
 #pragma unroll
-          for (int t = 0; t < PE; ++t) v[q][t] = to_f32(xt[(PE * (j + 8 * q) + t) * XP + rb * 32 + r8]);
+          for (int t = 0; t < PE; ++t) v[q][t] = to_f32(xt[(PE * (j + 8 * q) + t) * XP + x_pos(rb * 32 + r8)]);
         normalize_pieces<PE, NP>(v, gm, bt, p.eps);
 #pragma unroll
         for (int q = 0; q < NP; ++q) put_piece<T, SL, PE>(frag2, rb, r8, j + 8 * q, v[q]);
@@ -555,7 +588,7 @@ template <typename T, typename TZ, int KS, bool GATE, int RBW> struct AttnOut {
           of[rb][q][u] = load8<T>((const T*)p.x + ((int64_t)(wave + 4 * q) * n_rows + pr) * 32 + 16 * u + 8 * g);
     }
     const ZRow<Rows> z_row{p, tr};
-    auto z_row0 = [&](int r) { return max(z_row(r), (int64_t)0); };
+    auto z_row0 = [&](int r) { return z_row.clamped(r); };
     if constexpr (GATE) {
       // (all of a wave's gate weights under the LayerNorm, the output's first under the last head's products: fetched
       // when needed, one after the other, they cost rows of 256 channels three waits instead of one)
@@ -642,17 +675,18 @@ __global__ __launch_bounds__(kPpWaves * 64, (kPpMinWaves<T, KS>)) void pp_triatt
 }
 
 // ---- an output stage and the projection that reads its rows next, in one launch -------------------------
-// A patch of 8 x 4 * RBW positions for the projection of an ending node behind a starting node's output: logical rows (i, j) of the
-// ending node are z[j][i]; 8 consecutive j of one i follow each other.
+// A patch of 8 x 4 * RBW positions, for a projection that reads the pair tensor transposed (the ending node, the incoming
+// multiplication): its logical rows (i, j) are z[j][i]; 8 consecutive j of one i follow each other.
 struct PatchRows {
   int i0, j0, n;
-  __device__ __forceinline__ bool at(int r, int& i, int& j) const {   // of the ending node
+  __device__ __forceinline__ bool at(int r, int& i, int& j) const {   // of the projection
     i = min(i0 + (r >> 3), n - 1);
     j = min(j0 + (r & 7), n - 1);
     return i0 + (r >> 3) < n && j0 + (r & 7) < n;
   }
 };
-struct PatchRowsT {   // the same positions of the starting node
+struct PatchRowsT {   // the same positions as rows of z
+  static constexpr bool kPatch = true;
   PatchRows t;
   __device__ __forceinline__ bool at(int r, int& i, int& j) const { return t.at(r, j, i); }
 };
@@ -704,6 +738,29 @@ __global__ __launch_bounds__(kPpWaves * 64, (kPpMinWaves<T, KS>)) void pp_mul_ou
   columns.load_w(pi, wave, lane);
   __syncthreads();
   columns.run(pi, smem, smem + Out::kFrag, tr, wave, kPpWaves, wave, lane);
+}
+
+// The output stage of the outgoing triangle multiplication and the projection of the incoming one behind it.
+template <typename T, typename TZ, int KS, int RBW>
+__global__ __launch_bounds__(kPpWaves * 64, (kPpMinWaves<T, KS>)) void pp_mul_out_mul_in_kernel(ProjOutParams p, ProjInParams pi, SingleStage carry,
+                                                                                               unsigned carried) {
+  typedef MulOut<T, TZ, KS, RBW> Out;
+  typedef MulColumns<T, KS, RBW> Columns;
+  __shared__ __attribute__((aligned(16))) char smem[cmax(cmax(Out::kLds, Out::kFrag + Columns::kStage), kStageLds)];
+  PTX_CARRIED_STAGE();
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t n_ip = (uint32_t)(p.n + 4 * RBW - 1) / (4 * RBW), tile = xcd_run(block, blocks), kb = tile / n_ip;
+  const PatchRows tr = {(int)(tile - kb * n_ip) * (4 * RBW), (int)kb * 8, p.n};
+  const PatchRowsT trt = {tr};
+  typename RowPieces<TZ, KS>::V raw[RBW][RowPieces<TZ, KS>::NP];
+  const T* upd = Out::run(p, trt, smem, wave, lane, raw);
+  store_and_norm_rows<T, TZ, KS, RBW>(smem, (TZ*)p.out, ZRow<PatchRowsT>{p, trt}, upd, (const T*)pi.gamma, (const T*)pi.beta, pi.eps, wave, lane, raw);
+  Columns columns;
+  columns.load_w(pi, wave * Columns::CHW, lane);
+  __syncthreads();
+  Columns::put_mask(pi, smem + Out::kFrag, tr.i0, tr.j0);   // (over the update)
+  __syncthreads();
+  columns.run(pi, smem, smem + Out::kFrag, tr.i0, tr.j0, 0, Columns::CHW, wave, lane);
 }
 
 // The output stage of a starting node and the projection of the ending node behind it.
@@ -890,7 +947,8 @@ static int pp_trimul_in_ks(ProjInParams p, const SingleStage* carry, hipStream_t
   if (carry && KS <= 4) single_stage_run(carry, stream);
   if (!carry || KS <= 4) carry = &none;
   const unsigned carried = single_stage_groups(carry);
-  const unsigned tiles = (unsigned)((p.n + 4 * rbw - 1) / (4 * rbw)) * (unsigned)(p.pitch / 8);
+  p.n_kb = (unsigned)nt_gemm_k_extent(p.n, sizeof(T) == 2) / 8;
+  const unsigned tiles = (unsigned)((p.n + 4 * rbw - 1) / (4 * rbw)) * p.n_kb;
   constexpr int kChunks = PpWidths<KS>::HIDDEN / 64;   // per wave
   p.slices = in_slices(tiles, kChunks, sizeof(T) == 2);
   if (kChunks % p.slices) --p.slices;   // (2 or 4 chunks: equal shares)
@@ -1119,11 +1177,15 @@ int pp_triattn_out(const void* o, const void* z, const void* ln_w, const void* l
 // 2613, 1500 (no such kernel) 13264 / 13160 / 13226, 2048 27462 / 27528 / 27682; 16-bit rows, 256 262 / 259 / 251, 440 769 / 750 / 747, 480 918 / 922 / 924, 768
 // 2354 / 2402 / 2437; 64 channels, 128 101 / 97 / 94, 512 790 / 792 / 790, 1200 6191 / 6171 / 6147, 1500 10724 / 10774 / 10803; 256 channels, 96 240 / 234 / 228, 256
 // 715 / 715 / 714, 300 1114 / 1133 / 1139.
-bool pp_joined(bool attention, int n, int c_z, int hidden, bool rows16) {
+// The two multiplications (up to 256 tokens, where the products take the operands of any patch order from the L2), us per block
+// without / with: 40 tokens 74.5 / 68.6, 93 110 / 102, 128 118 / 115, 200 226 / 216, 256 276 / 275; without a single track 200 221 / 213, 256
+// 263 / 257; 64 channels 64 60 / 57, 200 169 / 165 (zeros beyond n written up to the next 32 tokens only are a part of that).
+bool pp_joined(int pair, int n, int c_z, int hidden, bool rows16) {
+  if (pair == 0) return n <= 256 && c_z <= 128;
   if (c_z == 256) return n <= 256;
   if (c_z == 64) return n <= 1280;
   const bool first = n < (rows16 ? 480 : 528) || (n < 1792 && !pp_resident(kTriAttnInStage, n, c_z, hidden, true, rows16));
-  return first && (!attention || n < 600);
+  return first && (pair == 1 || n < 600);
 }
 static int merged_row_blocks(int64_t rows, int ks) { return ks <= 8 && rows >= 160 * 160 ? 2 : 1; }
 
@@ -1229,7 +1291,60 @@ int pp_triattn_out_triattn_in(const void* o, const void* z, const void* ln_w, co
   else attn_out_attn_in_ks<TZ, 8>(p, pi, carry, stream);
   return 0;
 }
+template <typename TZ, int KS>
+static void mul_out_mul_in_ks(const ProjOutParams& p, const ProjInParams& pi, const SingleStage* carry, hipStream_t stream) {
+  const int rbw = merged_row_blocks((int64_t)p.n * p.n, KS);
+  static const SingleStage none = {};
+  if (carry && KS <= 4) single_stage_run(carry, stream);
+  if (!carry || KS <= 4) carry = &none;
+  const unsigned carried = single_stage_groups(carry);
+  const dim3 grid(carried + (unsigned)((p.n + 4 * rbw - 1) / (4 * rbw)) * (unsigned)(nt_gemm_k_extent(p.n, true) / 8)), block(kPpWaves * 64);
+  if (rbw == 2) pp_mul_out_mul_in_kernel<bf16_t, TZ, KS, 2><<<grid, block, 0, stream>>>(p, pi, *carry, carried);
+  else pp_mul_out_mul_in_kernel<bf16_t, TZ, KS, 1><<<grid, block, 0, stream>>>(p, pi, *carry, carried);
+}
+
+template <typename TZ>
+int pp_trimul_out_trimul_in(const void* x, int ldx, const void* z, const void* mask, const void* ln_in_w, const void* ln_in_b,
+                            const void* ln_out_w, const void* ln_out_b, const void* packed, void* out, const void* next_ln_w,
+                            const void* next_ln_b, const void* next_packed, void* a, void* b, int n, int c_z, int hidden, int k_pitch,
+                            float eps, const SingleStage* carry, hipStream_t stream) {
+  ProjOutParams p = {};
+  p.z = z;
+  p.si = (int64_t)n * c_z;
+  p.sj = c_z;
+  p.gamma = ln_in_w;
+  p.beta = ln_in_b;
+  p.gamma2 = ln_out_w;
+  p.beta2 = ln_out_b;
+  p.eps = eps;
+  p.packed = (const bf16_t*)packed + (int64_t)4 * c_z * hidden;
+  p.x = x;
+  p.ldx = ldx;
+  p.out = out;
+  p.n = n;
+  p.add_residual = 1;
+  ProjInParams pi = {};
+  pi.gamma = next_ln_w;
+  pi.beta = next_ln_b;
+  pi.eps = eps;
+  pi.packed = next_packed;
+  pi.out[0] = a;
+  pi.out[1] = b;
+  pi.mask = mask;
+  pi.mi = 1;
+  pi.mk = n;
+  pi.n = n;
+  pi.pitch = k_pitch;
+  if (c_z == 64) mul_out_mul_in_ks<TZ, 4>(p, pi, carry, stream);
+  else if (c_z == 128) mul_out_mul_in_ks<TZ, 8>(p, pi, carry, stream);
+  else return -1;
+  return 0;
+}
 #define PTX_INSTANTIATE_MERGED(TZ)                                                                                    \
+  template int pp_trimul_out_trimul_in<TZ>(const void*, int, const void*, const void*, const void*, const void*,      \
+                                           const void*, const void*, const void*, void*, const void*, const void*,    \
+                                           const void*, void*, void*, int, int, int, int, float, const SingleStage*,  \
+                                           hipStream_t);                                                              \
   template int pp_trimul_out_triattn_in<TZ>(const void*, int, const void*, const void*, const void*, const void*,     \
                                             const void*, const void*, void*, const void*, const void*, const void*,   \
                                             void*, void*, void*, void*, int, int, int, int, int, float,               \

@@ -1,6 +1,7 @@
 // What the two transition kernels (transition.hip, transition_small.hip) share.
 #pragma once
 #include "common.h"
+#include "kernels.h"
 
 namespace ptx {
 
@@ -20,9 +21,11 @@ struct AttnOutArgs {
 constexpr int kAoChunks = 3;   // chunks of 24 fragments that hold the 64 fragments of W_g and W_o
 
 // The transition on few rows (transition_small.hip); arguments as the fused kernel's.  Returns
-// false where the fused kernel is to be launched instead.
+// false where the fused kernel is to be launched instead.  carry (PB and AO): a stage of the single track on operands of type
+// TZ, run by the launch's first workgroups.
 template <typename T, int KS, typename TZ, bool PB, bool AO>
 bool transition_small(const TZ* x, const T* gamma, const T* beta, const T* packed, TZ* out, int64_t n_rows, int n_chunks,
-                      int add_residual, float eps, const PairBiasArgs& pb, const AttnOutArgs& ao, hipStream_t stream);
+                      int add_residual, float eps, const PairBiasArgs& pb, const AttnOutArgs& ao, hipStream_t stream,
+                      const SingleStage* carry = nullptr);
 
 }  // namespace ptx

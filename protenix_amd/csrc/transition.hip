@@ -686,7 +686,8 @@ int triattn_output_transition_fwd(const void* o, const void* z, const void* att_
                                   const void* ln_b, void* out, int n, int transposed, int n_factor,
                                   float att_eps, float eps, const void* pb_ln_w, const void* pb_ln_b,
                                   const void* pb_w, void* bias, int heads, int bias_f32, float pb_eps,
-                                  hipStream_t stream) {
+                                  hipStream_t stream, const SingleStage* carry) {
+  if (carry && (n == 0 || !pb_w || !transition_carries((int64_t)n * n))) single_stage_run(carry, stream);
   if (n == 0) return 0;
   if constexpr (sizeof(T) == 2) {
     constexpr int KS = 8;
@@ -705,7 +706,7 @@ int triattn_output_transition_fwd(const void* o, const void* z, const void* att_
     if (pb_w) {
       const PairBiasArgs pb = {pb_ln_w, pb_ln_b, pb_w, bias, heads, bias_f32, pb_eps};
       if (transition_small<T, KS, TZ, true, true>((const TZ*)z, (const T*)ln_w, (const T*)ln_b, (const T*)packed, (TZ*)out, rows,
-                                                  n_chunks, 1, eps, pb, ao, stream))
+                                                  n_chunks, 1, eps, pb, ao, stream, carry))
         return 0;
       transition_fused_kernel<T, KS, TZ, true, true><<<dim3((unsigned)blocks), dim3(TrCfg<T, KS>::NW * 64), 0, stream>>>(
           (const TZ*)z, (const T*)ln_w, (const T*)ln_b, (const T*)packed, (TZ*)out, rows, n_chunks, 1, eps,
@@ -751,7 +752,7 @@ template int triattn_output_transition_pack<bf16_t>(const void*, const void*, co
   template int triattn_output_transition_fwd<bf16_t, TZ>(                                          \
       const void*, const void*, const void*, const void*, const void*, const void*, const void*,   \
       void*, int, int, int, float, float, const void*, const void*, const void*, void*, int, int,  \
-      float, hipStream_t);
+      float, hipStream_t, const SingleStage*);
 PTX_INSTANTIATE_AOT(bf16_t)
 PTX_INSTANTIATE_AOT(float)
 #undef PTX_INSTANTIATE_AOT

@@ -10,6 +10,7 @@
 #include "common.h"
 #include "kernels.h"
 #include "rowpieces.h"
+#include "single_stage.h"
 #include "transition.h"
 #include <type_traits>
 
@@ -20,7 +21,7 @@ constexpr int kTsWaves = 4;
 template <typename T, int KS, typename TZ, bool PB, bool AO>
 __global__ __launch_bounds__(kTsWaves * 64, (sizeof(T) == 2 && KS <= 8 ? 2 : 1)) void transition_small_kernel(
     const TZ* x, const T* __restrict__ gamma, const T* __restrict__ beta, const T* __restrict__ packed, TZ* out,
-    int64_t n_rows, int n_chunks, int add_residual, float eps, PairBiasArgs pb, AttnOutArgs ao) {
+    int64_t n_rows, int n_chunks, int add_residual, float eps, PairBiasArgs pb, AttnOutArgs ao, SingleStage carry, unsigned carried) {
   typedef typename Vec8<T>::type V8;
   typedef RowPieces<TZ, KS> RP;
   constexpr int NOB = KS / 2, FRAGS = 3 * KS, kCx = 16 * KS, PE = RP::PE, NP = RP::NP, NW = kTsWaves;
@@ -32,10 +33,19 @@ __global__ __launch_bounds__(kTsWaves * 64, (sizeof(T) == 2 && KS <= 8 ? 2 : 1))
   __shared__ __attribute__((aligned(16))) char frag[kFrag > kUpd ? kFrag : kUpd];
   __shared__ __attribute__((aligned(16))) float part[NW][NOB][16][kWave];
   static_assert(!AO || sizeof(part) >= (size_t)FragLds<T, KS>::ROWBLOCK + kUpd, "the prologue's tiles fit the partial sums' place");
+  // The first `carried` workgroups run a stage of the single track (the form that a block with one launches).
+  if constexpr (PB && AO) {
+    static_assert(!(PB && AO) || sizeof(part) >= kStageLds, "the stage's LDS");
+    if (blockIdx.x < carried) {
+      single_stage<TZ>(carry, blockIdx.x, reinterpret_cast<char*>(part));
+      return;
+    }
+  }
+  const uint32_t block = blockIdx.x - carried, blocks = gridDim.x - carried;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int nl = lane & 31, g = lane >> 5, j8 = lane & 7, r8 = wave * 8 + (lane >> 3);
   // (back to front: the kernel before this one wrote the pair tensor front to back)
-  const int64_t row0 = (int64_t)(gridDim.x - 1 - xcd_run(blockIdx.x, gridDim.x)) * 32;
+  const int64_t row0 = (int64_t)(blocks - 1 - xcd_run(block, blocks)) * 32;
   const T* tpacked = packed + (AO ? (int64_t)kAoChunks * FRAGS * kFragElems : 0);
   auto x_row = [&](int r) -> int64_t { return row0 + r < n_rows ? (row0 + r) * kCx : -1; };
   auto x_row0 = [&](int r) -> int64_t { return min(row0 + r, n_rows - 1) * kCx; };
@@ -227,9 +237,7 @@ __global__ __launch_bounds__(kTsWaves * 64, (sizeof(T) == 2 && KS <= 8 ? 2 : 1))
   }
 }
 
-template <typename T, int KS, typename TZ, bool PB, bool AO>
-bool transition_small(const TZ* x, const T* gamma, const T* beta, const T* packed, TZ* out, int64_t n_rows, int n_chunks,
-                      int add_residual, float eps, const PairBiasArgs& pb, const AttnOutArgs& ao, hipStream_t stream) {
+static bool takes_split(int64_t n_rows, int ks, bool bits16) {
   // us per launch, fused / split (fp32 rows where the arithmetic is 16-bit):
   //   c = 128, 16-bit (with the attention's output and the pair bias): 27.4 / 12.4 at 64^2 rows, 27.6 / 18.9 at 93^2,
   //     28.2 / 20.0 at 128^2, 42.8 / 43.8 at 192^2: the fused kernel is flat up to 256 workgroups of 128 rows
@@ -239,19 +247,34 @@ bool transition_small(const TZ* x, const T* gamma, const T* beta, const T* packe
   //     64^2, 56 / 51 at 128^2, 114 / 117 at 192^2, 128 / 185 at 256^2
   // (Eight waves per workgroup: 14.1 at 64^2, 26.8 at 128^2.)
   const double rounds = (double)((n_rows + 32767) / 32768);
-  bool split;
-  if (sizeof(T) == 4) split = 10.0 + 0.0038 * (double)n_rows < 104.0 * rounds;
-  else if (KS == 16) split = 3.0 + 0.003 * (double)n_rows < 56.0 * rounds;
-  else split = n_rows <= (KS == 4 ? 60000 : 21500);
-  if (!split) return false;
-  transition_small_kernel<T, KS, TZ, PB, AO><<<dim3((unsigned)((n_rows + 31) / 32)), dim3(kTsWaves * 64), 0, stream>>>(
-      x, gamma, beta, packed, out, n_rows, n_chunks, add_residual, eps, pb, ao);
+  if (!bits16) return 10.0 + 0.0038 * (double)n_rows < 104.0 * rounds;
+  if (ks == 16) return 3.0 + 0.003 * (double)n_rows < 56.0 * rounds;
+  return n_rows <= (ks == 4 ? 60000 : 21500);
+}
+
+// Two workgroups per compute unit: where a stage's (some two hundred of its own, with as much LDS) would make another round they
+// are launched apart (128 tokens: a block of 119 us took 125).
+bool transition_carries(int64_t n_rows) {
+  constexpr int64_t kRound = 512, kStage = 200;
+  const int64_t blocks = (n_rows + 31) / 32;
+  return takes_split(n_rows, 8, true) && (blocks + kStage + kRound - 1) / kRound == (blocks + kRound - 1) / kRound;
+}
+
+template <typename T, int KS, typename TZ, bool PB, bool AO>
+bool transition_small(const TZ* x, const T* gamma, const T* beta, const T* packed, TZ* out, int64_t n_rows, int n_chunks,
+                      int add_residual, float eps, const PairBiasArgs& pb, const AttnOutArgs& ao, hipStream_t stream, const SingleStage* carry) {
+  if (!takes_split(n_rows, KS, sizeof(T) == 2)) return false;
+  static const SingleStage none = {};
+  if (!carry) carry = &none;
+  const unsigned carried = PB && AO ? single_stage_groups(carry) : 0u;
+  transition_small_kernel<T, KS, TZ, PB, AO><<<dim3(carried + (unsigned)((n_rows + 31) / 32)), dim3(kTsWaves * 64), 0, stream>>>(
+      x, gamma, beta, packed, out, n_rows, n_chunks, add_residual, eps, pb, ao, *carry, carried);
   return true;
 }
 
 #define PTX_INSTANTIATE(T, KS, TZ, PB, AO)                                                                            \
   template bool transition_small<T, KS, TZ, PB, AO>(const TZ*, const T*, const T*, const T*, TZ*, int64_t, int, int,  \
-                                                    float, const PairBiasArgs&, const AttnOutArgs&, hipStream_t);
+                                                    float, const PairBiasArgs&, const AttnOutArgs&, hipStream_t, const SingleStage*);
 PTX_INSTANTIATE(float, 4, float, false, false)
 PTX_INSTANTIATE(float, 8, float, false, false)
 PTX_INSTANTIATE(bf16_t, 4, bf16_t, false, false)

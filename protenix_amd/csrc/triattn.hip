@@ -31,6 +31,7 @@
 
 #include "common.h"
 #include "kernels.h"
+#include "single_stage.h"
 
 namespace ptx {
 
@@ -72,16 +73,27 @@ struct AttnAux {
 // partial key tile takes the same paths as the others with the logits of the keys beyond
 // n_keys set to -inf (kMaskTail; kMaskNone where the keys fill whole tiles).
 enum { kMaskNone = 0, kMaskTail = 1, kMaskGiven = 2 };
-template <typename T, int R, int NWQ, int MK>
-__global__ __launch_bounds__((NWQ * 64), (sizeof(T) == 2 ? (R == 1 ? 16 / NWQ : 4) : 2)) void triattn_fwd_kernel(
+// TS: the launch's first `carried` workgroups run a stage of the single track on operands of that type (void: none).
+template <typename T, int R, int NWQ, int MK, typename TS>
+__global__ __launch_bounds__((NWQ * 64), (sizeof(T) == 2 ? (!std::is_void<TS>::value ? 3 : R == 1 ? 16 / NWQ : 4) : 2)) void triattn_fwd_kernel(
     const T* __restrict__ q, const T* __restrict__ k, const T* __restrict__ vt,
     const T* gate, const T* __restrict__ bias, const T* __restrict__ mask,
     T* o, int n, int heads, int key_pitch, int mask_transposed, float inf,
-    int n_qtiles, int n_rowgroups, int64_t total_items, AttnAux ax) {
+    int n_qtiles, int n_rowgroups, int64_t total_items, AttnAux ax, SingleStage carry, unsigned carried) {
   typedef typename Vec8<T>::type V8;
   typedef typename Vec4<T>::type V4;
+  constexpr bool kCarries = !std::is_void<TS>::value;
+  static_assert(!kCarries || (sizeof(T) == 2 && R == 1 && NWQ == kStageWaves), "the small launches");
   // two key tiles x R rows: iteration t reads tile t while tile t+1 is written
-  __shared__ V8 lds_kv[2][R][8][kWave];     // fragments 0-3: K (u,kk); 4-7: V^T (u,s)
+  __shared__ V8 lds_kv[kCarries ? 4 : 2][R][8][kWave];     // fragments 0-3: K (u,kk); 4-7: V^T (u,s)
+  if constexpr (kCarries) {
+    static_assert(!kCarries || sizeof(lds_kv) >= kStageLds, "the stage's LDS");
+    if (blockIdx.x < carried) {
+      single_stage<TS>(carry, blockIdx.x, reinterpret_cast<char*>(lds_kv));
+      return;
+    }
+  }
+  const unsigned block = blockIdx.x - carried;
   __shared__ __attribute__((aligned(16))) float lds_mb[2][R][kKeyTile];  // mask bias per key
 
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -90,7 +102,7 @@ __global__ __launch_bounds__((NWQ * 64), (sizeof(T) == 2 ? (R == 1 ? 16 / NWQ : 
   // Work item -> (h, row group, query tile), h-major, one contiguous span per XCD
   // (workgroups are dealt round-robin to the 8 XCDs).
   const int64_t per_xcd = (total_items + 7) / 8;
-  const int64_t item = (int64_t)(blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+  const int64_t item = (int64_t)(block & 7) * per_xcd + (block >> 3);
   if (item >= total_items) return;
   const int qt = (int)(item % n_qtiles);
   const int i0 = ax.row0 + (int)((item / n_qtiles) % n_rowgroups) * R;   // first of this workgroup's R rows
@@ -519,10 +531,13 @@ __global__ __launch_bounds__((NWQ * 64), (sizeof(T) == 2 ? (R == 1 ? 16 / NWQ : 
   }
 }
 
+// (one row and four waves at those sizes, and workgroups to spare)
+bool triattn_fwd_carries(int n, bool bits16) { return bits16 && n <= 256; }
+
 template <typename T>
 int triattn_fwd(const T* q, const T* k, const T* vt, const T* g, const T* tri_bias, const T* mask,
                 T* o, int n, int heads, int key_pitch, int mask_transposed, float inf,
-                int row_begin, int row_count, int n_keys, hipStream_t stream) {
+                int row_begin, int row_count, int n_keys, const SingleStage* carry, hipStream_t stream) {
   // head-major q, gate, o of a whole pair tensor: [heads][n][n][32]
   AttnAux ax = {};
   ax.sh = (int64_t)n * n * kD;
@@ -530,7 +545,7 @@ int triattn_fwd(const T* q, const T* k, const T* vt, const T* g, const T* tri_bi
   ax.sj = kD;
   ax.n_rows = n;
   return triattn_fwd_ex<T>(q, k, vt, g, tri_bias, mask, o, n, n, heads, key_pitch, mask_transposed, inf,
-                           0, ax.sh, ax.si, ax.sj, nullptr, 0, 0, 0, row_begin, row_count, n_keys, stream);
+                           0, ax.sh, ax.si, ax.sj, nullptr, 0, 0, 0, row_begin, row_count, n_keys, carry, stream);
 }
 
 template <typename T>
@@ -538,8 +553,13 @@ int triattn_fwd_ex(const T* q, const T* k, const T* vt, const T* g, const T* tri
                    const T* mask, T* o, int n_rows, int n, int heads, int key_pitch,
                    int mask_transposed, float inf, int mask_is_bias, int64_t sh, int64_t si,
                    int64_t sj, float* lse, int64_t lh, int64_t li, int64_t lj, int row_begin,
-                   int row_count, int n_keys, hipStream_t stream) {
-  if (n == 0 || n_rows == 0 || row_count == 0) return 0;
+                   int row_count, int n_keys, const SingleStage* carry, hipStream_t stream) {
+  const bool empty = n == 0 || n_rows == 0 || row_count == 0 || heads == 0;
+  if (carry && (empty || !triattn_fwd_carries(n, sizeof(T) == 2))) {
+    single_stage_run(carry, stream);
+    carry = nullptr;
+  }
+  if (empty) return 0;
   AttnAux ax = {sh, si, sj, n_rows, mask_is_bias, lse, lh, li, lj, row_begin, row_begin + row_count, n_keys, 0, n};
   // Two rows per wave (16-bit, no mask): the two rows share the query block and with it the bias tile - one load
   // and one conversion per logit for both, half the bias stream from the L2 - at 128 registers, so that four waves
@@ -561,10 +581,26 @@ int triattn_fwd_ex(const T* q, const T* k, const T* vt, const T* g, const T* tri
   const int n_rowgroups = (row_count + R - 1) / R;
   const int64_t total = (int64_t)heads * n_rowgroups * n_qtiles;
   const int64_t per_xcd = (total + 7) / 8;
-#define PTX_ATTN_LAUNCH_R(RR, NWQ, MK)                                                            \
-  triattn_fwd_kernel<T, RR, NWQ, MK><<<dim3((unsigned)(per_xcd * 8)), dim3(NWQ * 64), 0, stream>>>( \
-      q, k, vt, g, tri_bias, mask, o, n, heads, key_pitch, mask_transposed, inf, n_qtiles,        \
-      n_rowgroups, total, ax)
+#define PTX_ATTN_LAUNCH_T(RR, NWQ, MK, TS)                                                                   \
+  triattn_fwd_kernel<T, RR, NWQ, MK, TS><<<dim3(carried + (unsigned)(per_xcd * 8)), dim3(NWQ * 64), 0, stream>>>( \
+      q, k, vt, g, tri_bias, mask, o, n, heads, key_pitch, mask_transposed, inf, n_qtiles,                   \
+      n_rowgroups, total, ax, carried ? *carry : SingleStage{}, carried)
+#define PTX_ATTN_LAUNCH_R(RR, NWQ, MK) PTX_ATTN_LAUNCH_T(RR, NWQ, MK, void)
+  const unsigned carried = single_stage_groups(carry);
+  if constexpr (sizeof(T) == 2) {
+    if (carried) {
+#define PTX_ATTN_LAUNCH_C(TS)                                              \
+  do {                                                                     \
+    if (mk == kMaskGiven) PTX_ATTN_LAUNCH_T(1, 4, kMaskGiven, TS);         \
+    else if (mk == kMaskTail) PTX_ATTN_LAUNCH_T(1, 4, kMaskTail, TS);      \
+    else PTX_ATTN_LAUNCH_T(1, 4, kMaskNone, TS);                           \
+  } while (0)
+      if (carry->bits16) PTX_ATTN_LAUNCH_C(bf16_t);
+      else PTX_ATTN_LAUNCH_C(float);
+#undef PTX_ATTN_LAUNCH_C
+      return 0;
+    }
+  }
 #define PTX_ATTN_LAUNCH(RR, MK)                \
   do {                                         \
     if (wide) PTX_ATTN_LAUNCH_R(RR, 8, MK);    \
@@ -584,21 +620,22 @@ int triattn_fwd_ex(const T* q, const T* k, const T* vt, const T* g, const T* tri
   }
 #undef PTX_ATTN_LAUNCH
 #undef PTX_ATTN_LAUNCH_R
+#undef PTX_ATTN_LAUNCH_T
   return 0;
 }
 
 #define PTX_INSTANTIATE_EX(T)                                                                     \
   template int triattn_fwd_ex<T>(const T*, const T*, const T*, const T*, const T*, const T*, T*,  \
                                  int, int, int, int, int, float, int, int64_t, int64_t, int64_t,  \
-                                 float*, int64_t, int64_t, int64_t, int, int, int, hipStream_t);
+                                 float*, int64_t, int64_t, int64_t, int, int, int, const SingleStage*, hipStream_t);
 PTX_INSTANTIATE_EX(float)
 PTX_INSTANTIATE_EX(bf16_t)
 #undef PTX_INSTANTIATE_EX
 template int triattn_fwd<float>(const float*, const float*, const float*, const float*,
                                 const float*, const float*, float*, int, int, int, int, float,
-                                int, int, int, hipStream_t);
+                                int, int, int, const SingleStage*, hipStream_t);
 template int triattn_fwd<bf16_t>(const bf16_t*, const bf16_t*, const bf16_t*, const bf16_t*,
                                  const bf16_t*, const bf16_t*, bf16_t*, int, int, int, int, float,
-                                 int, int, int, hipStream_t);
+                                 int, int, int, const SingleStage*, hipStream_t);
 
 }  // namespace ptx

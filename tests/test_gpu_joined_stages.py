@@ -15,7 +15,8 @@ BF16 = torch.bfloat16
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("mode,c_z,n,batch,pad", [
-    ("amp", 128, 1, 1, 0), ("amp", 128, 7, 2, 1), ("bf16", 128, 9, 1, 0), ("amp", 128, 159, 1, 3), ("bf16", 128, 160, 1, 0),
+    ("amp", 128, 1, 1, 0), ("amp", 128, 7, 2, 1), ("bf16", 128, 31, 2, 0), ("amp", 128, 93, 1, 6), ("amp", 128, 101, 1, 0), ("amp", 128, 102, 1, 0), ("bf16", 128, 128, 1, 3), ("amp", 128, 128, 2, 0), ("amp", 128, 146, 1, 0),
+    ("amp", 128, 147, 1, 0), ("bf16", 64, 255, 1, 3), ("amp", 64, 256, 1, 0), ("bf16", 128, 9, 1, 0), ("amp", 128, 159, 1, 3), ("bf16", 128, 160, 1, 0),
     ("amp", 128, 161, 1, 5), ("amp", 128, 193, 1, 0), ("amp", 128, 256, 1, 9), ("amp", 128, 257, 1, 0), ("bf16", 128, 355, 1, 0),
     ("bf16", 128, 479, 1, 0), ("bf16", 128, 484, 1, 0), ("amp", 128, 527, 1, 17), ("amp", 128, 528, 1, 0), ("amp", 128, 596, 1, 0),
     ("amp", 128, 601, 1, 4), ("amp", 64, 5, 2, 1), ("bf16", 64, 158, 1, 0), ("amp", 64, 165, 1, 2), ("amp", 64, 396, 1, 0),
@@ -35,3 +36,17 @@ def test_joined_equal_separate(mode, c_z, n, batch, pad):
             return prod(s, z, m)
     (s1, z1), (s2, z2) = both(run)
     assert torch.equal(z1, z2) and (s1 is s2 if s is None else torch.equal(s1, s2))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [30, 129, 200])
+def test_without_a_single_track(n):
+    _, prod = oracle_and_product(O.PairformerStack, P.PairformerStack, n_blocks=2, dtype=BF16, c_s=0)
+    z = torch.randn(1, n, n, 128, generator=torch.Generator().manual_seed(n)).cuda()
+    m = (torch.rand(1, n, n, generator=torch.Generator().manual_seed(n)) > 0.3).float().cuda()
+
+    def run():
+        with torch.no_grad(), torch.autocast("cuda", dtype=BF16):
+            return prod(None, z, m)
+    (_, z1), (_, z2) = both(run)
+    assert torch.equal(z1, z2)
