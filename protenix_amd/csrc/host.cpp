@@ -695,19 +695,20 @@ struct Block : Plan {
     weights.want_fragments(&s_wo, {matrix(st, "linear_no_bias", c_s, hidden)}, type);
   }
 
-  // The five pair updates of the pair tensors of z [batch][n][n][c_z] in place; the single attention's pair
+  // The five pair updates of the pair tensors `from` (like z; may be z) into z [batch][n][n][c_z]; the single attention's pair
   // bias (fp32 [batch][heads][n][n]) of the finished z into `bias` (null: none wanted).
-  void pair_track(const Tensor& z, const std::vector<Mask>& masks, int64_t batch, int n, void* ws, float* bias, Run& run) const {
+  void pair_track(const void* from, const Tensor& z, const std::vector<Mask>& masks, int64_t batch, int n, void* ws, float* bias, Run& run) const {
     const int dt = code_of_rows(z.scalar_type(), compute);
     const int64_t es = at::elementSize(compute), plane = (int64_t)n * n * c_z * z.element_size();
     char* zp = (char*)z.data_ptr();
+    const char* fp = (const char*)from;
     static const Mask none;
     auto mask = [&](int64_t b) -> const Mask& { return masks.empty() ? none : masks[b]; };
     const int64_t bias_plane = (int64_t)heads * n * n;
     if (run.chained) {
       for (int64_t b = 0; b < batch; ++b) {
         void* zb = zp + b * plane;
-        chain(zb, mask(b), n, dt, es, ws, run);
+        chain(fp + b * plane, zb, mask(b), n, dt, es, ws, run);
         if (fused) {
           optional<ptx_single_stage> last;
           if (b == 0 && bias && ptx_triattn_output_transition_carries(n)) last = run.run_rest_but_last();
@@ -719,7 +720,7 @@ struct Block : Plan {
       }
       if (fused) return;
     } else {
-      for (int64_t b = 0; b < batch; ++b) run_trimul(out, zp + b * plane, mask(b).m, zp + b * plane, n, true, dt, es, ws, run);
+      for (int64_t b = 0; b < batch; ++b) run_trimul(out, fp + b * plane, mask(b).m, zp + b * plane, n, true, dt, es, ws, run);
       for (int64_t b = 0; b < batch; ++b) run_trimul(in, zp + b * plane, mask(b).m, zp + b * plane, n, true, dt, es, ws, run);
       for (int64_t b = 0; b < batch; ++b) run_triatt(start, zp + b * plane, mask(b), zp + b * plane, n, true, dt, es, ws, run);
       if (fused) {
@@ -759,21 +760,21 @@ struct Block : Plan {
   bool core_carries(int n, int dt) const {
     return c_s > 0 && joins_products(n, dt) && !ptx_triattn_output_transition_carries(n);
   }
-  // The block up to the ending node's attention output.
-  void chain(void* z, const Mask& mask, int n, int dt, int64_t es, void* ws, Run& run) const {
+  // The block up to the ending node's attention output: pair tensor `from` (may be z) into z.
+  void chain(const void* from, void* z, const Mask& mask, int n, int dt, int64_t es, void* ws, Run& run) const {
     Cut c{(char*)ws};
     const ChainWs s(c, n, out.c_h, start.heads, es);
     const int ldx = (n + 7) / 8 * 8, pitch = ptx_key_pitch(n);
-    run_trimul_product(out, z, mask.m, n, dt, s.a, s.b, s.x, run);
+    run_trimul_product(out, from, mask.m, n, dt, s.a, s.b, s.x, run);
     if (joins_products(n, dt)) {
       const ptx_single_stage* carry0 = run.carry(1);
       run.launch("trimul_output_trimul_project", [&] {
-        return ptx_trimul_output_trimul_project(s.x, ldx, z, ptr(mask.m), out.ln_in_w, out.ln_in_b, out.ln_out_w, out.ln_out_b, out.packed, z,
+        return ptx_trimul_output_trimul_project(s.x, ldx, from, ptr(mask.m), out.ln_in_w, out.ln_in_b, out.ln_out_w, out.ln_out_b, out.packed, z,
                                                 in.ln_in_w, in.ln_in_b, in.packed, s.a, s.b, n, c_z, out.c_h, pitch, kEps, dt, carry0, run.st);
       });
       run_contraction(in, s.a, s.b, s.x, n, dt, run);
     } else {
-      run_trimul_output(out, s.x, z, z, n, true, dt, run);
+      run_trimul_output(out, s.x, from, z, n, true, dt, run);
       run_trimul_product(in, z, mask.m, n, dt, s.a, s.b, s.x, run);
     }
     const ptx_single_stage* carry1 = run.carry(1);
@@ -844,9 +845,9 @@ struct Block : Plan {
       h = (char*)c.part(batch * n * b.hidden * es);
     }
   };
-  // The stages of: mid = s + attention(LN(s); bias); s_out = mid + transition(LN(mid))
-  void single_track(Stages& st, const void* s, void* mid, void* s_out, const float* bias, at::ScalarType type, int64_t batch, int n,
-                    void* ws) const {
+  // The stages of: mid = s + attention(LN(s); bias); s_out = mid + transition(LN(mid)).  The first two, which do not need the
+  // pair bias:
+  void single_projection(Stages& st, const void* s, at::ScalarType type, int64_t batch, int n, void* ws) const {
     const int dt = code_of(type), hd = heads * d, ldt = (n + 31) / 32 * 32;
     const int64_t es = at::elementSize(type), rows = batch * n;
     Cut c{(char*)ws};
@@ -856,6 +857,14 @@ struct Block : Plan {
       char* qkg = w.qkg + b * w.qkg_plane;
       check(ptx_single_linear_stage(st.add("linear"), w.y + b * n * c_s * es, w_in, nullptr, b_q, hd, nullptr, qkg, w.vt + b * w.vt_plane, 3 * hd, ldt, n, c_s, 4 * hd, dt, 1), "linear");
     }
+  }
+  // the others
+  void single_track(Stages& st, const void* s, void* mid, void* s_out, const float* bias, at::ScalarType type, int64_t batch, int n,
+                    void* ws) const {
+    const int dt = code_of(type), hd = heads * d, ldt = (n + 31) / 32 * 32;
+    const int64_t es = at::elementSize(type), rows = batch * n;
+    Cut c{(char*)ws};
+    const SingleWs w(c, *this, batch, n, es);
     for (int64_t b = 0; b < batch; ++b) {
       char* qkg = w.qkg + b * w.qkg_plane;
       check(ptx_single_attention_stage(st.add("single_attention"), qkg, qkg + hd * es, w.vt + b * w.vt_plane, qkg + 2 * hd * es,
@@ -876,13 +885,13 @@ struct Block : Plan {
 // put a new plan into it while this one runs without the interpreter's lock.
 using Blocks = std::vector<std::shared_ptr<Block>>;
 
-// Blocks in sequence on z (contiguous, updated in place).  The single track of a block runs underneath the next
+// Blocks in sequence on the pair tensors `from` into z (contiguous; the same tensor: in place).  The single track of a block runs underneath the next
 // block's pair kernels (see Stages), the last one's in finish().  The blocks may come in several lots: on new weights
 // a plan is made while the kernels of the blocks before it run.
 struct Call {
   // timer: None, or the dict that gets the launches' times; poison: see Run.
-  Call(const optional<Tensor>& s, const Tensor& z, const py::list& masks, const py::object& timer, bool poison)
-      : z_(z), s_(s), masks_(masks_of(masks)), timer_(timer), run_(z) {
+  Call(const optional<Tensor>& s, const Tensor& z, const Tensor& from, const py::list& masks, const py::object& timer, bool poison)
+      : z_(z), from_(from), s_(s), masks_(masks_of(masks)), timer_(timer), run_(z) {
     run_.poison = poison;
     run_.timing = !timer.is_none();
     n_ = (int)z.size(-2);
@@ -904,8 +913,13 @@ struct Call {
       run_.row_stages(n_, b->c_z, b->out.c_h, dt);
       run_.chained = b->chains(run_, n_, dt);
       run_.core_carries = run_.chained && b->core_carries(n_, dt);
-      b->pair_track(z_, masks_, batch_, n_, ws_.data_ptr(), bias, run_);
+      // (a first block's projection rides on its own pair kernels, where nothing waits from a block before)
+      const bool early = single && run_.singles.list.empty();
+      if (early) b->single_projection(run_.singles, s_now_, s_->scalar_type(), batch_, n_, sws_.data_ptr());
+      b->pair_track(from_.data_ptr(), z_, masks_, batch_, n_, ws_.data_ptr(), bias, run_);
+      from_ = z_;
       if (single) {
+        if (!early) b->single_projection(run_.singles, s_now_, s_->scalar_type(), batch_, n_, sws_.data_ptr());
         b->single_track(run_.singles, s_now_, mid_.data_ptr(), s_out_.data_ptr(), bias, s_->scalar_type(), batch_, n_, sws_.data_ptr());
         s_now_ = s_out_.data_ptr();
       }
@@ -940,7 +954,7 @@ struct Call {
     if (t.defined()) outgrown_.push_back(t);   // (stages that wait for a launch point into it)
     t = run_.workspace(bytes, z_.options());
   }
-  Tensor z_;
+  Tensor z_, from_;   // (from_: until the first block has read it)
   optional<Tensor> s_;
   std::vector<Mask> masks_;
   py::object timer_;
@@ -1145,8 +1159,8 @@ PYBIND11_MODULE(_host, m) {
     return (int64_t)-1;
   }, "index of the first block whose weights are no longer the module's, or -1");
   py::class_<Call>(m, "Call")
-      .def(py::init<const optional<Tensor>&, const Tensor&, const py::list&, const py::object&, bool>(), py::arg("s"), py::arg("z"),
-           py::arg("masks"), py::arg("timer") = py::none(), py::arg("poison") = false)
+      .def(py::init<const optional<Tensor>&, const Tensor&, const Tensor&, const py::list&, const py::object&, bool>(), py::arg("s"),
+           py::arg("z"), py::arg("from_"), py::arg("masks"), py::arg("timer") = py::none(), py::arg("poison") = false)
       .def("blocks", &Call::blocks)
       .def("finish", &Call::finish);
   py::class_<Mark, std::shared_ptr<Mark>>(m, "Mark").def("elapsed_time", &Mark::elapsed_time);

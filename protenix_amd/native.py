@@ -129,32 +129,33 @@ def plans_of(module) -> list:
     return [plan for m in module.modules() for plan in _plans.get(m, {}).values()]
 
 
-def run_blocks(owner, blocks, s: Optional[torch.Tensor], z: torch.Tensor, pair_mask: Optional[torch.Tensor]):
-    """The blocks on (s, z), z contiguous and updated in place: (the new s - None without a single track -, how many of the
+def run_blocks(owner, blocks, s: Optional[torch.Tensor], z: torch.Tensor, pair_mask: Optional[torch.Tensor], in_place: bool):
+    """The blocks on (s, z): (the new s - None without a single track -, the new z - z itself if `in_place` -, how many of the
     blocks were run).  What follows the first block without a plan is left to the caller, as is everything where the
-    count is 0.  `owner`: the module the list of plans is kept with."""
+    count is 0.  z is contiguous, and at a multiple of 16 bytes if it is not to be changed (the first block then reads it
+    and writes another tensor).  `owner`: the module the list of plans is kept with."""
     if not _usable(z) or not z.is_contiguous():
-        return s, 0
+        return s, z, 0
     ac = ops.autocast_compute_dtype(z)
     cd = ops.compute_dtype(z)
     if ac is not None and cd == z.dtype:
-        return s, 0
+        return s, z, 0
     if pair_mask is not None and not (pair_mask.is_cuda and pair_mask.dim() >= 2):
-        return s, 0
+        return s, z, 0
     single = any(b.c_s > 0 for b in blocks)
     sd = None
     if single:
         n = z.shape[-2]
         if s is None or not s.is_cuda or s.dim() < 2 or s.shape[-2] != n or s.numel() // (n * s.shape[-1]) != z.numel() // (
                 n * n * z.shape[-1]) or any(b.c_s != s.shape[-1] for b in blocks):
-            return s, 0
+            return s, z, 0
         sd = s.dtype
     key = ("stack", cd, sd, z.device.index, z.dtype)
     kept = _plans.setdefault(owner, {}).get(key)
     if (kept is not None and len(kept[0]) == len(blocks) and all(a() is b for a, b in zip(kept[0], blocks))
             and host().first_stale(kept[1]) < 0):
         plans = kept[1]
-        call = _call(s, z, pair_mask, cd, single)
+        call, out = _call(s, z, pair_mask, cd, single, in_place)
         call.blocks(plans)
     else:
         # a plan is made while the kernels of the blocks before it run
@@ -164,18 +165,20 @@ def run_blocks(owner, blocks, s: Optional[torch.Tensor], z: torch.Tensor, pair_m
             if plan is None:
                 break
             plans.append(plan)
-            call = call or _call(s, z, pair_mask, cd, single)
+            if call is None:
+                call, out = _call(s, z, pair_mask, cd, single, in_place)
             call.blocks([plan])
         if call is None:
-            return s, 0
+            return s, z, 0
         if len(plans) == len(blocks):
             _plans[owner][key] = ([weakref.ref(b) for b in blocks], plans)
-    return call.finish(), len(plans)
+    return call.finish(), out, len(plans)
 
 
-def _call(s, z, pair_mask, cd, single):
-    return host().Call(_aligned(s.contiguous()) if single else s, z, _masks(z, pair_mask, cd), ops.kernel_timer,
-                       ops.poison_workspaces)
+def _call(s, z, pair_mask, cd, single, in_place):
+    out = z if in_place else torch.empty_like(z)
+    return host().Call(_aligned(s.contiguous()) if single else s, out, z, _masks(z, pair_mask, cd), ops.kernel_timer,
+                       ops.poison_workspaces), out
 
 
 def run_update(module, z: torch.Tensor, cd: torch.dtype, mask: Optional[torch.Tensor], out: torch.Tensor, add: bool,

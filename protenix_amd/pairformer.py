@@ -61,6 +61,14 @@ class _Padded:
         return corner.contiguous() if z_out is None else z_out.copy_(corner)
 
 
+def _own_copy(z: torch.Tensor, in_place: bool) -> Tuple[torch.Tensor, bool]:
+    """(z or a copy of it, whether blocks may work on that in place): contiguous, and without a copy where the first
+    block can read the caller's tensor and write another one (the native path: dense rows at a multiple of 16 bytes)."""
+    if z.is_contiguous() and (in_place or (z.is_cuda and not z.is_neg() and z.data_ptr() % 16 == 0)):
+        return z, in_place
+    return z.clone(memory_format=torch.contiguous_format), True
+
+
 def _wants_padding(z: torch.Tensor, pair_mask: Optional[torch.Tensor]) -> bool:
     return (pad_tokens_to > 1 and z.is_cuda and z.dim() >= 3 and z.shape[-2] == z.shape[-3]
             and z.shape[-2] % pad_tokens_to != 0 and pad_tokens_min_n <= z.shape[-2]
@@ -110,12 +118,11 @@ class PairformerBlock(nn.Module):
             pad = _Padded(z)
             s, _ = self._forward_unpadded(s, pad.z, pad.mask, pad)
             return s, pad.result(z if inplace_safe else None)
-        if not inplace_safe or not z.is_contiguous():
-            z = z.clone(memory_format=torch.contiguous_format)
-        s_new, done = native.run_blocks(self, (self,), s, z, pair_mask)
+        z, in_place = _own_copy(z, inplace_safe)
+        s_new, z_new, done = native.run_blocks(self, (self,), s, z, pair_mask, in_place)
         if done:
-            return s_new, z
-        return self._forward_unpadded(s, z, pair_mask, None)
+            return s_new, z_new
+        return self._forward_unpadded(s, z if in_place else z.clone(), pair_mask, None)
 
     def _forward_unpadded(self, s, z, pair_mask, pad):
         """z: contiguous, updated in place; pad: the _Padded that made it, or None."""
@@ -285,22 +292,23 @@ class PairformerStack(nn.Module):
             # (one padded copy for the whole stack, see pad_tokens_to)
             pad = _Padded(z)
             z, pair_mask = pad.z, pad.mask
-        elif not inplace_safe and len(self.blocks) > 0:
-            # one private copy for the whole stack; the blocks then work in place
-            z = z.clone(memory_format=torch.contiguous_format)
-        if not z.is_contiguous():
-            z = z.contiguous()
+        in_place = True
+        if pad is None:
+            # one private copy for the whole stack at most; the blocks then work in place
+            z, in_place = _own_copy(z, inplace_safe or len(self.blocks) == 0)
         if triangle_multiplicative not in ("torch", "cuequivariance"):
             raise ValueError(
                 "triangle_multiplicative must be 'cuequivariance' or 'torch', but got "
                 f"{triangle_multiplicative}")
         assert triangle_attention in ("torch", "deepspeed", "triattention", "cuequivariance")
         if pad is None and lead > 0:
-            s, done = native.run_blocks(self, tuple(self.blocks)[:lead], s, z, pair_mask)
+            s, z, done = native.run_blocks(self, tuple(self.blocks)[:lead], s, z, pair_mask, in_place)
             if done:
                 for blk in self.blocks[done:]:
                     s, z = blk(s, z, pair_mask, inplace_safe=True)
                 return s, z
+        if not in_place:
+            z = z.clone()
         ac = ops.autocast_compute_dtype(z)
         if (not own or not z.is_cuda or s is None
                 or any(b.c_s == 0 or not native.runs_own_forward(b.attention_pair_bias) for b in self.blocks)
