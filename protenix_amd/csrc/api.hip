@@ -708,14 +708,17 @@ PTX_API int ptx_triattn_core_fwd(const void* q, const void* k, const void* v, co
     const char* b1 = bias1 ? (const char*)bias1 + b * n_b1 * es : nullptr;
     char* ob = (char*)o + b * n_q * es;
     float* lb = lse ? lse + (int64_t)b * n_rows * s * heads : nullptr;
+    // 16-bit: q, K and V are read as they are, as long as the output does not overwrite them under way
+    auto apart = [&](const char* t) { return ob + n_q * es <= t || t + n_q * es <= ob; };
+    const bool as_is = dtype == PTX_BF16 && ptx::triattn_fwd_standard(s, b1 != nullptr) && apart(qb) && apart(kb) && apart(vb);
     PTX_DISPATCH(dtype, {
-      ptx::triattn_pack<T>((const T*)qb, (const T*)kb, (const T*)vb, (const T*)b2, (T*)qs, (T*)kf,
+      ptx::triattn_pack<T>(as_is ? nullptr : (const T*)qb, (const T*)kb, (const T*)vb, (const T*)b2, (T*)qs, (T*)kf,
                            (T*)vtf, (T*)bf, n_rows, s, heads, pitch, (hipStream_t)stream);
       // standard layout [row][position][head][32]; no gate; bias1 is an additive bias per key
-      ptx::triattn_fwd_ex<T>((const T*)qs, (const T*)kf, (const T*)vtf, (const T*)nullptr,
+      ptx::triattn_fwd_ex<T>((const T*)(as_is ? qb : qs), (const T*)(as_is ? kb : kf), (const T*)(as_is ? vb : vtf), (const T*)nullptr,
                              (const T*)bf, (const T*)b1, (T*)ob, n_rows, s, heads, pitch, 0, 0.0f, 1,
                              32, (int64_t)s * heads * 32, (int64_t)heads * 32, lb, 1,
-                             (int64_t)s * heads, heads, 0, n_rows, s, nullptr, (hipStream_t)stream);
+                             (int64_t)s * heads, heads, 0, n_rows, s, nullptr, (hipStream_t)stream, as_is);
     });
   }
   return after_launch("triattn_core_fwd");

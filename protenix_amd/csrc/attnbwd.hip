@@ -99,24 +99,11 @@ template <typename T, bool VEC> struct BwdCfg {
 };
 
 // 16-bit tiles are parked in LDS row-major only; an operand that a product needs with the
-// tile's rows in the K slots is read with the transposing LDS load of gfx950
-// (ds_read_b64_tr_b16: the 16 lanes of a block hand in the addresses of 4 x 16 elements, 4
-// lanes per row, and lane j of the block gets column j of the 4 rows).  Two of them: the lane
-// gets column col0 + lane % 16 of rows row0 .. row0 + 7.  fp32 has no such load and keeps
-// transposed copies of its tiles.
+// tile's rows in the K slots is read with the transposing LDS load of gfx950 (load8_turned in
+// common.h).  fp32 has no such load and keeps transposed copies of its tiles.
 template <typename T> struct Turned {
   static constexpr bool value = sizeof(T) == 2;
 };
-__device__ __forceinline__ bf16x8 load8_turned(const bf16_t* tile, int pitch, int row0, int col0, int lane) {
-  typedef short v4s __attribute__((ext_vector_type(4)));
-  typedef short v8s __attribute__((ext_vector_type(8)));
-  typedef __attribute__((address_space(3))) v4s* LdsV4;
-  const int i = lane & 15;
-  const bf16_t* a = tile + (row0 + (i >> 2)) * pitch + col0 + 4 * (i & 3);
-  const v4s lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsV4)a);
-  const v4s hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsV4)(a + 4 * pitch));
-  return __builtin_bit_cast(bf16x8, (v8s)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-}
 __device__ __forceinline__ f32x8 load8_turned(const float*, int, int, int, int) { return f32x8{}; }   // (never called)
 
 // The workgroup's 256 threads load two [32 rows][32 channels] tiles (rows `pos0 ..` of tensors

@@ -1,7 +1,8 @@
 // Repack of standard-layout attention operands into the layouts of the triangle-attention
 // core (common.h): K and V [rows][n][heads][32] -> fragment-ordered K and V^T key tiles, the
 // pair bias [heads][n][n] -> fragment-ordered bias tiles in log2 units, q -> q * log2(e).
-// One thread per 16-byte destination vector; plain gathers, bandwidth-bound.
+// One thread per 16-byte destination vector; plain gathers, bandwidth-bound.  16-bit operands need the bias' part only:
+// the core reads q, K and V as they are (triattn.hip, STD), unless its output overlaps them.
 #include "common.h"
 #include "kernels.h"
 
@@ -82,12 +83,14 @@ int triattn_pack(const T* q, const T* k, const T* v, const T* bias2, T* qs, T* k
                  int n_rows, int n, int heads, int key_pitch, hipStream_t stream) {
   if (n_rows == 0 || n == 0 || heads == 0) return 0;
   const int key_tiles = key_pitch >> 6;
-  const int64_t nqk = (int64_t)n_rows * n * heads * 4;
-  attn_pack_qk_kernel<T><<<dim3((unsigned)((nqk + 255) / 256)), dim3(256), 0, stream>>>(
-      q, k, qs, kf, n_rows, n, heads, key_tiles);
-  const int64_t nv = (int64_t)n_rows * key_tiles * 8 * heads * 32;
-  attn_pack_v_kernel<T><<<dim3((unsigned)((nv + 255) / 256)), dim3(256), 0, stream>>>(
-      v, vtf, n_rows, n, heads, key_tiles);
+  if (q) {
+    const int64_t nqk = (int64_t)n_rows * n * heads * 4;
+    attn_pack_qk_kernel<T><<<dim3((unsigned)((nqk + 255) / 256)), dim3(256), 0, stream>>>(
+        q, k, qs, kf, n_rows, n, heads, key_tiles);
+    const int64_t nv = (int64_t)n_rows * key_tiles * 8 * heads * 32;
+    attn_pack_v_kernel<T><<<dim3((unsigned)((nv + 255) / 256)), dim3(256), 0, stream>>>(
+        v, vtf, n_rows, n, heads, key_tiles);
+  }
   const int64_t nb = (int64_t)heads * n * key_tiles * 8;
   attn_pack_bias_kernel<T><<<dim3((unsigned)((nb + 255) / 256)), dim3(256), 0, stream>>>(
       bias2, bf, n, heads, key_tiles);

@@ -87,6 +87,20 @@ __device__ __forceinline__ void store8(T* p, typename Vec8<T>::type v) {
   *reinterpret_cast<typename Vec8<T>::type*>(p) = v;
 }
 
+// Eight 16-bit elements of one column out of a row-major LDS tile: column col0 + lane % 16 of rows row0 .. row0 + 7, by two
+// of gfx950's transposing LDS loads (ds_read_b64_tr_b16: the 16 lanes of a block hand in the addresses of 4 x 16
+// elements, 4 lanes per row, and lane j of the block gets column j of the 4 rows).
+__device__ __forceinline__ bf16x8 load8_turned(const bf16_t* tile, int pitch, int row0, int col0, int lane) {
+  typedef short v4s __attribute__((ext_vector_type(4)));
+  typedef short v8s __attribute__((ext_vector_type(8)));
+  typedef __attribute__((address_space(3))) v4s* LdsV4;
+  const int i = lane & 15;
+  const bf16_t* a = tile + (row0 + (i >> 2)) * pitch + col0 + 4 * (i & 3);
+  const v4s lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsV4)a);
+  const v4s hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsV4)(a + 4 * pitch));
+  return __builtin_bit_cast(bf16x8, (v8s)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+}
+
 typedef __attribute__((ext_vector_type(4))) uint32_t u32x4_t;
 
 // Direct-to-LDS load: every lane moves 16 bytes from its own global address to LDS address

@@ -211,16 +211,18 @@ bool triattn_fwd_carries(int n, bool bits16);
 // strides (head, row, query), an optional gate (g may be null), the mask either 0/1 values or
 // (mask_is_bias) an additive bias per (row, key), and an optional log2-sum-exp2 output.
 // The launch covers rows row_begin .. row_begin + row_count - 1 and lets keys 0 .. n_keys - 1
-// take part (keys beyond count as masked: weight exactly zero).
+// take part (keys beyond count as masked: weight exactly zero).  standard (16-bit): k and vt are K and V addressed by q's
+// strides, and q is not yet in log2 units; where triattn_fwd_standard().
+bool triattn_fwd_standard(int n, bool masked);
 template <typename T>
 int triattn_fwd_ex(const T* q, const T* k, const T* vt, const T* g, const T* tri_bias,
                    const T* mask, T* o, int n_rows, int n, int heads, int key_pitch,
                    int mask_transposed, float inf, int mask_is_bias, int64_t sh, int64_t si,
                    int64_t sj, float* lse, int64_t lh, int64_t li, int64_t lj, int row_begin,
-                   int row_count, int n_keys, const SingleStage* carry, hipStream_t stream);
+                   int row_count, int n_keys, const SingleStage* carry, hipStream_t stream, bool standard = false);
 // Standard-layout K, V [n_rows][n][heads][32] and bias [heads][n][n] -> the core's fragment-
 // ordered K, V^T and bias (bias and nothing else multiplied by log2(e)); q [n_rows][n][heads][32]
-// -> qs, the same layout multiplied by log2(e).
+// -> qs, the same layout multiplied by log2(e).  q = null: the bias only.
 template <typename T>
 int triattn_pack(const T* q, const T* k, const T* v, const T* bias2, T* qs, T* kf, T* vtf, T* bf,
                  int n_rows, int n, int heads, int key_pitch, hipStream_t stream);

@@ -74,7 +74,11 @@ struct AttnAux {
 // n_keys set to -inf (kMaskTail; kMaskNone where the keys fill whole tiles).
 enum { kMaskNone = 0, kMaskTail = 1, kMaskGiven = 2 };
 // TS: the launch's first `carried` workgroups run a stage of the single track on operands of that type (void: none).
-template <typename T, int R, int NWQ, int MK, typename TS>
+// STD: K and V as the operator's callers have them, [row][position][head][32] (addressed like q), and q not yet multiplied by
+// log2 e: K rows find their fragments by the lanes' addresses, V tiles lie row-major in LDS and are turned when they
+// are read.  (Repacked by kernels of their own, q, K and V cost 44 us at 384 rows of 384 positions and 4 heads, next to 86 of
+// the core.)
+template <typename T, int R, int NWQ, int MK, typename TS, bool STD = false>
 __global__ __launch_bounds__((NWQ * 64), (sizeof(T) == 2 ? (!std::is_void<TS>::value ? 3 : R == 1 ? 16 / NWQ : 4) : 2)) void triattn_fwd_kernel(
     const T* __restrict__ q, const T* __restrict__ k, const T* __restrict__ vt,
     const T* gate, const T* __restrict__ bias, const T* __restrict__ mask,
@@ -135,7 +139,15 @@ __global__ __launch_bounds__((NWQ * 64), (sizeof(T) == 2 ? (!std::is_void<TS>::v
   for (int r = 0; r < R; ++r) {
     qrow[r] = h * ax.sh + min(i0 + r, n_rows - 1) * ax.si + qi * ax.sj;
 #pragma unroll
-    for (int kk = 0; kk < 2; ++kk) qf[r][kk] = load8<T>(q + qrow[r] + 16 * kk + 8 * g);
+    for (int kk = 0; kk < 2; ++kk) {
+      qf[r][kk] = load8<T>(q + qrow[r] + 16 * kk + 8 * g);
+      if constexpr (STD) {
+        f32x8 v = to_f32(qf[r][kk]);
+#pragma unroll
+        for (int t = 0; t < 8; ++t) v[t] *= kLog2e;
+        qf[r][kk] = from_f32<T>(v);
+      }
+    }
   }
 
   // ---- cooperative tile loader: 8*R fragments per key tile, 8*R / NWQ per wave ----
@@ -148,7 +160,21 @@ __global__ __launch_bounds__((NWQ * 64), (sizeof(T) == 2 ? (!std::is_void<TS>::v
   constexpr int FPW = 8 * R / NWQ;   // fragments each wave moves per tile, of one operand and row
   static_assert(FPW >= 1 && FPW <= 4, "a wave's fragments are consecutive in memory");
   const int fid0 = wave * FPW, fr = fid0 >> 3, f0 = fid0 & 7;   // row, first fragment
-  const T* const kv_base = (f0 < 4 ? k : vt) + ((int64_t)h * n_rows + min(i0 + fr, n_rows - 1)) * key_tiles * kAttnTileElems + (f0 & 3) * 512;
+  static_assert(!STD || kDirect, "standard layouts: 16-bit");
+  const T* const kv_base = STD ? (f0 < 4 ? k : vt) + h * ax.sh + min(i0 + fr, n_rows - 1) * ax.si
+                               : (f0 < 4 ? k : vt) + ((int64_t)h * n_rows + min(i0 + fr, n_rows - 1)) * key_tiles * kAttnTileElems + (f0 & 3) * 512;
+  // STD: this lane's key within the tile and its channels, of the wave's fragment j
+  auto std_place = [&](int j, int& key, int& d) {
+    const int f = (f0 + j) & 3;
+    if (f0 < 4) {   // K fragment (u, kk) = f: MFMA row lane % 32 (see the top), half-wave's channels
+      const int m = lane & 31;
+      key = 32 * ((m >> 2) & 1) + 16 * (f >> 1) + 4 * (m >> 3) + (m & 3);
+      d = 16 * (f & 1) + 8 * g;
+    } else {        // V: 16 rows of 64 bytes
+      key = 16 * f + (lane >> 2);
+      d = 8 * (lane & 3);
+    }
+  };
   V8 pre[kDirect ? 1 : FPW];
   T pre_mv;
   // mask value of key kc for this wave's row: m_base[kc * m_stride]
@@ -157,7 +183,16 @@ __global__ __launch_bounds__((NWQ * 64), (sizeof(T) == 2 ? (!std::is_void<TS>::v
   const T* m_base = has_mask ? mask + (mask_transposed ? (int64_t)m_row : (int64_t)m_row * n) : nullptr;
   auto fetch = [&](int tile) {
     const T* src = kv_base + (int64_t)tile * kAttnTileElems;
-    if constexpr (kDirect) {
+    if constexpr (STD) {
+      const uint64_t base = uniform64((uint64_t)kv_base);
+      const uint32_t dst = lds_address(&lds_kv[tile & 1][fr][f0][0]);
+#pragma unroll
+      for (int j = 0; j < FPW; ++j) {
+        int key, d;
+        std_place(j, key, d);   // (keys beyond n: the last one, left out below)
+        load_to_lds16_s<0>(base, (uint32_t)(min(tile * kKeyTile + key, n - 1) * (int)ax.sj + d) * (uint32_t)sizeof(T), dst + j * 1024);
+      }
+    } else if constexpr (kDirect) {
       const uint64_t base = uniform64((uint64_t)src);
       const uint32_t dst = lds_address(&lds_kv[tile & 1][fr][f0][0]), off = lane * 16;
       load_to_lds16_s<0>(base, off, dst);
@@ -185,7 +220,12 @@ __global__ __launch_bounds__((NWQ * 64), (sizeof(T) == 2 ? (!std::is_void<TS>::v
         V8 v;
         if constexpr (kDirect) v = lds_kv[buf][fr][f0 + j][lane];
         else v = pre[j];
-        if (tail && f0 >= 4) {
+        if (STD && tail && f0 >= 4) {
+          int key, d;
+          std_place(j, key, d);
+#pragma unroll
+          for (int t = 0; t < 8; ++t) v[t] = key0 + key < nk ? v[t] : (T)0.0f;
+        } else if (tail && f0 >= 4) {
           // V^T fragment (u, s): slots <-> keys 32g + 16u + 8s + t
           const int f = f0 + j, koff = key0 + 32 * g + 16 * ((f >> 1) & 1) + 8 * (f & 1);
 #pragma unroll
@@ -211,6 +251,13 @@ __global__ __launch_bounds__((NWQ * 64), (sizeof(T) == 2 ? (!std::is_void<TS>::v
       for (int c = 0; c < 2; ++c) dst[u][c] = load8<T>(bp + (u * 2 + c) * 512);
   };
 
+  // V^T fragment (u, c) of row r: keys 32g + 16u + 8c .. + 7 of channel lane % 32
+  auto v_frag = [&](int buf, int r, int u, int c) -> V8 {
+    if constexpr (STD)
+      return load8_turned(reinterpret_cast<const T*>(&lds_kv[buf][r][4][0]), 32, 32 * g + 16 * u + 8 * c, 16 * ((lane >> 4) & 1), lane);
+    else
+      return lds_kv[buf][r][4 + u * 2 + c][lane];
+  };
   f32x16 acc_o[R];                // O^T per row
   bool zero_reference = false;    // (uniform) every row's softmax reference is 0
   float m_run[R], l_run[R];       // running max (natural units) and denominator (this lane's keys)
@@ -410,7 +457,7 @@ __global__ __launch_bounds__((NWQ * 64), (sizeof(T) == 2 ? (!std::is_void<TS>::v
             if (r_begin != r) break;
             V8 vf[2], pf[2];
 #pragma unroll
-            for (int c = 0; c < 2; ++c) vf[c] = lds_kv[buf][r][4 + u * 2 + c][lane];
+            for (int c = 0; c < 2; ++c) vf[c] = v_frag(buf, r, u, c);
 #pragma unroll
             for (int e = 0; e < 16; ++e) s[r][e] = fast_exp2(s[r][e]);
             const float psum = probabilities(s[r], pf);
@@ -459,7 +506,7 @@ __global__ __launch_bounds__((NWQ * 64), (sizeof(T) == 2 ? (!std::is_void<TS>::v
         }
         l_run[r] += out.psum;
 #pragma unroll
-        for (int c = 0; c < 2; ++c) mma32(acc_o[r], lds_kv[buf][r][4 + u * 2 + c][lane], out.pf[c]);
+        for (int c = 0; c < 2; ++c) mma32(acc_o[r], v_frag(buf, r, u, c), out.pf[c]);
       }
       if constexpr (R == 2 && !has_mask)
         zero_reference = ((__builtin_amdgcn_ballot_w64(m_run[0] != 0.0f) | __builtin_amdgcn_ballot_w64(m_run[1] != 0.0f)) & q_ok_mask) == 0ull;
@@ -531,6 +578,12 @@ __global__ __launch_bounds__((NWQ * 64), (sizeof(T) == 2 ? (!std::is_void<TS>::v
   }
 }
 
+constexpr int kTwoRowsFrom = 352;   // (see triattn_fwd_ex)
+
+// Where the core reads standard layouts: with one row per wave (with two, the lanes' addresses take registers that it does not
+// have).
+bool triattn_fwd_standard(int n, bool masked) { return masked || n < kTwoRowsFrom; }
+
 // (one row and four waves at those sizes, and workgroups to spare)
 bool triattn_fwd_carries(int n, bool bits16) { return bits16 && n <= 256; }
 
@@ -553,7 +606,7 @@ int triattn_fwd_ex(const T* q, const T* k, const T* vt, const T* g, const T* tri
                    const T* mask, T* o, int n_rows, int n, int heads, int key_pitch,
                    int mask_transposed, float inf, int mask_is_bias, int64_t sh, int64_t si,
                    int64_t sj, float* lse, int64_t lh, int64_t li, int64_t lj, int row_begin,
-                   int row_count, int n_keys, const SingleStage* carry, hipStream_t stream) {
+                   int row_count, int n_keys, const SingleStage* carry, hipStream_t stream, bool standard) {
   const bool empty = n == 0 || n_rows == 0 || row_count == 0 || heads == 0;
   if (carry && (empty || !triattn_fwd_carries(n, sizeof(T) == 2))) {
     single_stage_run(carry, stream);
@@ -570,7 +623,7 @@ int triattn_fwd_ex(const T* q, const T* k, const T* vt, const T* g, const T* tri
   // (Before direct-to-LDS loads and two tiles in LDS instead of three, which made room for four workgroups of four waves per
   // compute unit, and before two rows' products ran next to each other's exponentials: 384 67, 387 94, 600 233, 768 385, 776
   // 494, 1024 856, 2048 6410.)
-  const bool two_rows = sizeof(T) == 2 && !mask && n >= 352 && row_count >= 2;
+  const bool two_rows = sizeof(T) == 2 && !mask && n >= kTwoRowsFrom && row_count >= 2 && !standard;
   // Eight waves share the staged K / V tiles of long rows: +2 % at n = 768 with one row per wave, even at 1024, -2.6 % at 1536; with
   // two rows the figures above.  Where 256 queries do not divide n, the waves of a row's last workgroup that have no queries
   // skip the arithmetic and only help to stage the tiles.
@@ -581,8 +634,8 @@ int triattn_fwd_ex(const T* q, const T* k, const T* vt, const T* g, const T* tri
   const int n_rowgroups = (row_count + R - 1) / R;
   const int64_t total = (int64_t)heads * n_rowgroups * n_qtiles;
   const int64_t per_xcd = (total + 7) / 8;
-#define PTX_ATTN_LAUNCH_T(RR, NWQ, MK, TS)                                                                   \
-  triattn_fwd_kernel<T, RR, NWQ, MK, TS><<<dim3(carried + (unsigned)(per_xcd * 8)), dim3(NWQ * 64), 0, stream>>>( \
+#define PTX_ATTN_LAUNCH_T(RR, NWQ, MK, ...)                                                                  \
+  triattn_fwd_kernel<T, RR, NWQ, MK, __VA_ARGS__><<<dim3(carried + (unsigned)(per_xcd * 8)), dim3(NWQ * 64), 0, stream>>>( \
       q, k, vt, g, tri_bias, mask, o, n, heads, key_pitch, mask_transposed, inf, n_qtiles,                   \
       n_rowgroups, total, ax, carried ? *carry : SingleStage{}, carried)
 #define PTX_ATTN_LAUNCH_R(RR, NWQ, MK) PTX_ATTN_LAUNCH_T(RR, NWQ, MK, void)
@@ -598,6 +651,20 @@ int triattn_fwd_ex(const T* q, const T* k, const T* vt, const T* g, const T* tri
       if (carry->bits16) PTX_ATTN_LAUNCH_C(bf16_t);
       else PTX_ATTN_LAUNCH_C(float);
 #undef PTX_ATTN_LAUNCH_C
+      return 0;
+    }
+  }
+  if constexpr (sizeof(T) == 2) {
+    if (standard) {
+#define PTX_ATTN_LAUNCH_S(RR, MK)                                    \
+  do {                                                               \
+    if (wide) PTX_ATTN_LAUNCH_T(RR, 8, MK, void, true);              \
+    else PTX_ATTN_LAUNCH_T(RR, 4, MK, void, true);                   \
+  } while (0)
+      if (mk == kMaskGiven) PTX_ATTN_LAUNCH_S(1, kMaskGiven);
+      else if (mk == kMaskTail) PTX_ATTN_LAUNCH_S(1, kMaskTail);
+      else PTX_ATTN_LAUNCH_S(1, kMaskNone);
+#undef PTX_ATTN_LAUNCH_S
       return 0;
     }
   }
@@ -627,7 +694,7 @@ int triattn_fwd_ex(const T* q, const T* k, const T* vt, const T* g, const T* tri
 #define PTX_INSTANTIATE_EX(T)                                                                     \
   template int triattn_fwd_ex<T>(const T*, const T*, const T*, const T*, const T*, const T*, T*,  \
                                  int, int, int, int, int, float, int, int64_t, int64_t, int64_t,  \
-                                 float*, int64_t, int64_t, int64_t, int, int, int, const SingleStage*, hipStream_t);
+                                 float*, int64_t, int64_t, int64_t, int, int, int, const SingleStage*, hipStream_t, bool);
 PTX_INSTANTIATE_EX(float)
 PTX_INSTANTIATE_EX(bf16_t)
 #undef PTX_INSTANTIATE_EX

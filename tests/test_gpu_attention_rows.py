@@ -57,3 +57,28 @@ def test_core(n, scale):
         assert err <= 2 * 2.0 ** -8 * plain[2].abs().max().item(), (n, scale, row0, err)
         outside = [r for r in range(n) if not row0 <= r < row0 + count]
         assert bool((o[:, outside] == 7.0).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,s,heads,with_b1", [(1, 1, 1, True), (3, 31, 4, True), (2, 64, 2, False), (5, 65, 4, True), (4, 100, 3, False),
+                                                  (3, 352, 4, False), (2, 353, 4, False), (5, 385, 4, True), (2, 500, 1, True),
+                                                  (2, 1057, 2, False), (1, 2056, 1, True)])
+def test_standard_layouts_equal_the_repacked_operands(rows, s, heads, with_b1):
+    """16-bit operands read as they are, and repacked where the output would overwrite V: the same products, bit for bit."""
+    lib = _lib.load()
+    g = torch.Generator().manual_seed(rows * s)
+    q, k, v = (torch.randn(rows, s, heads, 32, generator=g).bfloat16().cuda() for _ in range(3))
+    b2 = torch.randn(heads, s, s, generator=g).bfloat16().cuda()
+    b1 = (-1e9 * (torch.rand(rows, s, generator=g) > 0.8).float()).bfloat16().cuda() if with_b1 else None
+    ws = torch.empty(lib.ptx_triattn_core_workspace_elems(rows, s, heads), dtype=torch.bfloat16, device="cuda")
+    st = torch.cuda.current_stream().cuda_stream
+    outs = []
+    for o in (torch.empty_like(v), v.clone()):
+        lse = torch.empty(rows, s, heads, device="cuda")
+        src = v if not outs else o
+        rc = lib.ptx_triattn_core_fwd(q.data_ptr(), k.data_ptr(), src.data_ptr(), None if b1 is None else b1.data_ptr(), b2.data_ptr(),
+                                      o.data_ptr(), lse.data_ptr(), ws.fill_(float("nan")).data_ptr(), 1, rows, s, heads, 32, 1, st)
+        assert rc == 0
+        outs.append((o, lse))
+    assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
+    assert bool(torch.isfinite(outs[0][0]).all())
