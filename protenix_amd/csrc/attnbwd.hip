@@ -5,8 +5,8 @@
 //   P = 2^(S log2 e - M),  S = Q K^T + Bias1 + Bias2,  Delta = rowsum(O * dO),
 //   dS = P * (dO V^T - Delta)
 // it produces  dV = P^T dO,  dK = dS^T Q,  dQ = dS K,  dBias2[h] = sum over rows of dS.
-// Three kernels - dQ, which also forms Delta (the reference's preprocess kernel) and leaves it
-// for the others, dK/dV, dBias2 - where the reference has four; P is recomputed, the
+// Two kernels where a workgroup can take a whole row (rows_at_once) - dQ, dK and dV, and dBias2 -, else three: dQ, dK / dV, dBias2.
+// The first forms Delta (the reference's preprocess kernel) and leaves it for the others; P is recomputed, the
 // logits are never stored.  One wave owns a 32 x 32 block of (query, key) pairs and walks over
 // the other index; every product runs on MFMA with fp32 accumulation (conventions of
 // common.h).  The register <-> index permutation of single.hip makes the recomputed P and dS
@@ -22,6 +22,7 @@
 #include <type_traits>
 #include "common.h"
 #include "kernels.h"
+#include "rowtile.h"
 
 namespace ptx {
 
@@ -484,6 +485,260 @@ __global__ __launch_bounds__(256, (BwdCfg<T, VEC>::kMinWaves)) void attn_bwd_kv_
   }
 }
 
+// LDS tiles of 32 x 32 elements: rows of 64 bytes, their four 16-byte pieces exchanged by bits 2 and 3 of the row, so that
+// neither eight rows' pieces (vector reads and writes) nor four rows' halves (turning reads) meet in a bank.
+__device__ __forceinline__ int piece_at(int row, int piece) { return row * 32 + ((piece ^ ((row >> 2) & 3)) << 3); }
+
+// Eight elements of this lane's column out of such a tile, rows 16 ks + 8 g .. + 7 (g = lane / 32), column 16 (lane / 16 % 2) + lane % 16
+struct TurnedAt {
+  int lo, hi;   // of the rows' first and second four
+  __device__ explicit TurnedAt(int lane) {
+    const int row = 8 * (lane >> 5) + ((lane & 15) >> 2), piece = 2 * ((lane >> 4) & 1) + ((lane & 3) >> 1), e = 4 * (lane & 1);
+    lo = piece_at(row, piece) + e;
+    hi = piece_at(row + 4, piece) + e;
+  }
+  __device__ __forceinline__ bf16x8 load(const bf16_t* tile, int ks) const {
+    typedef short v4s __attribute__((ext_vector_type(4)));
+    typedef short v8s __attribute__((ext_vector_type(8)));
+    typedef __attribute__((address_space(3))) v4s* LdsV4;
+    const v4s a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsV4)(tile + lo + 512 * ks));
+    const v4s b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsV4)(tile + hi + 512 * ks));
+    return __builtin_bit_cast(bf16x8, (v8s)__builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7));
+  }
+};
+
+// -inf as the lowest finite value, so that a product with 0 is 0 (a NaN's row is NaN throughout by its log-sum-exp).
+__device__ __forceinline__ Vec8<bf16_t>::type finite_low(Vec8<bf16_t>::type x) {
+  typedef uint16_t U8 __attribute__((ext_vector_type(8)));
+  return __builtin_bit_cast(Vec8<bf16_t>::type, __builtin_elementwise_min(__builtin_bit_cast(U8, x), (U8)0xff7f));
+}
+
+// dQ, dK and dV in one pass, 16-bit, rows of at most 32 NW NBK positions: a workgroup takes one (row, head), a wave NBK blocks of
+// 32 keys (every NW-th), and all walk over the query blocks.  Logits and dP are formed once instead of once for dQ and
+// once for dK / dV.  Works on S like the dK / dV kernel (lane <-> key, register <-> query); dQ contracts over the keys, so
+// a block's dS goes through LDS once more and is turned on its way out, and the waves' dQ of a query block, each over its own
+// keys, are added through LDS in wave order.  Bias2 reaches the S accumulator on the matrix pipe, S += B2 * 1, from fragments
+// loaded along the queries' rows; Bias1 is the accumulator's initial value, and -inf for keys beyond s.
+// Bound by latency: of a wave's time 28 % issues, 52 % waits for LDS and barriers (two waves per SIMD: the accumulators of all its
+// keys are registers); of a SIMD's time 36 % is vector work, 24 % matrix work, and 30 % of the compute unit's is LDS.  Leaving out the
+// exponentials, the exchange of dQ or the spread of Bias2's rows, or three waves of one block each, changes it by 0 - 3 %.
+// 384 rows of 384 positions, 4 heads: dQ 109 us and dK / dV 126 before, 195 now.
+template <int NW, int NBK>
+__global__ __launch_bounds__(NW * 64, NBK == 1 ? 3 : 2) void attn_bwd_row_kernel(BwdParams p) {
+  typedef bf16_t T;
+  typedef Vec8<T>::type V8;
+  typedef Vec4<T>::type V4;
+  constexpr int KB = NW * NBK, kExWave = 16 * kWave * 4;   // bytes of a wave's partial dQ
+  static_assert(1024 * (int)sizeof(T) <= kExWave, "a wave's dS tile fits its place for dQ");
+  __shared__ __attribute__((aligned(32))) T kt[KB][1024];      // K, row-major, read by the wave that owns the block
+  __shared__ __attribute__((aligned(32))) T rm[2][2][1024];      // Q, dO of the step
+  __shared__ f32x8 stats[2][KB * 4];   // -log-sum-exp, -Delta
+  // two of them, for a step and the next: a wave's dS tile, later its partial dQ
+  __shared__ __attribute__((aligned(32))) char ex[2][NW][kExWave];
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, ln = lane & 31, g = lane >> 5;
+  const int s = p.s, H = p.heads;
+  const uint32_t items = (uint32_t)H * (uint32_t)p.n_rows, item = xcd_item(items);
+  if (item >= items) return;
+  const int h = item % H, i = item / H;
+
+  // Delta = sum_d O * dO of every query, four lanes each; left in p.delta for the dBias2 kernel
+  for (int q = tid >> 2; q < KB * 32; q += NW * 16) {
+    const int64_t e = elem(p, i, min(q, s - 1), h) + 8 * (tid & 3);
+    const f32x8 of = to_f32(load8<T>((const T*)p.o + e)), df = to_f32(load8<T>((const T*)p.dout + e));
+    float d = 0.0f;
+#pragma unroll
+    for (int t = 0; t < 8; ++t) d += of[t] * df[t];
+    d += __shfl_xor(d, 1, 64);
+    d += __shfl_xor(d, 2, 64);
+    if ((tid & 3) == 0) {
+      const int64_t st = ((int64_t)i * s + min(q, s - 1)) * H + h;
+      reinterpret_cast<float*>(stats[0])[q] = q < s ? -p.lse[st] : -INFINITY;   // (beyond s: probability 0)
+      reinterpret_cast<float*>(stats[1])[q] = -d;
+      if (q < s) p.delta[st] = d;
+    }
+  }
+  // this wave's keys
+  V8 vf[NBK][2];
+  float b1v[NBK];
+  f32x16 acc_dk[NBK], acc_dv[NBK];
+#pragma unroll
+  for (int b = 0; b < NBK; ++b) {
+    const int key = (b * NW + wave) * 32 + ln, kc = min(key, s - 1);
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) {
+      vf[b][kk] = load8<T>((const T*)p.v + elem(p, i, kc, h) + 16 * kk + 8 * g);
+      store8<T>(&kt[b * NW + wave][piece_at(ln, 2 * kk + g)], load8<T>((const T*)p.k + elem(p, i, kc, h) + 16 * kk + 8 * g));
+    }
+    b1v[b] = key >= s ? -INFINITY : p.b1 ? to_f32(((const T*)p.b1)[(int64_t)i * s + kc]) : 0.0f;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc_dk[b][r] = acc_dv[b][r] = 0.0f;
+  }
+  // the unit matrix as the other operand of Bias2's product (slot <-> key of the block, lane <-> key)
+  V8 one[2];
+#pragma unroll
+  for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+    for (int t = 0; t < 8; ++t) one[kk][t] = (T)(ln == 16 * kk + 8 * g + t ? 1.0f : 0.0f);
+
+  const int n_steps = (s + 31) >> 5;
+  const TurnedAt turned(lane);
+  // Q and dO tiles: the first 256 threads, 8 channels of one row of one tile each, a step ahead (positions of a row times
+  // heads and channels stay below 2^31)
+  V8 piece;
+  const T* const tile_src = (const T*)(tid >> 7 & 1 ? p.dout : p.q) + elem(p, i, 0, h);
+  const int tile_row = (tid & 127) >> 2, tile_col = 8 * (tid & 3), tile_at = piece_at(tile_row, tid & 3);
+  auto fetch = [&](int t) {
+    if (NW == 4 || wave < 4) piece = load8<T>(tile_src + (uint32_t)(min(t * 32 + tile_row, s - 1) * H * 32 + tile_col));
+  };
+  auto park = [&](int t) {
+    if (NW == 4 || wave < 4) store8<T>(&rm[t & 1][tid >> 7 & 1][tile_at], piece);
+  };
+  // Bias2 fragments of block b at step t: lane <-> query perm_row(ln), slots <-> 8 keys; one block ahead.  Rows start at any
+  // element.  The last 8 keys are read again for those beyond, and moved down (zeros above: -inf plus whatever lies there
+  // might not be -inf).
+  const T* b2h = (const T*)p.b2 + (int64_t)h * s * s;
+  const int b2q = perm_row(ln);
+  V8 b2n[2];
+  auto fetch_bias = [&](int t, int b) {
+    const int key0 = (b * NW + wave) * 32;
+    const uint32_t row = (uint32_t)min(t * 32 + b2q, s - 1) * (uint32_t)s;
+    if (key0 + 32 <= s) {   // the same for the whole wave
+#pragma unroll
+      for (int kk = 0; kk < 2; ++kk) __builtin_memcpy(&b2n[kk], b2h + (row + (uint32_t)(key0 + 16 * kk + 8 * g)), sizeof(V8));
+    } else {
+#pragma unroll
+      for (int kk = 0; kk < 2; ++kk) {
+        const int kb = key0 + 16 * kk + 8 * g, from = min(kb, s - 8);
+        unsigned __int128 v;
+        __builtin_memcpy(&v, b2h + (row + (uint32_t)from), sizeof(v));
+        v = kb >= s ? 0 : v >> (16 * (kb - from));
+        __builtin_memcpy(&b2n[kk], &v, sizeof(v));
+      }
+    }
+  };
+  fetch(0);
+  fetch_bias(0, 0);
+  park(0);
+  __syncthreads();
+  for (int t = 0; t < n_steps; ++t) {
+    const int buf = t & 1;
+    fetch(t + 1);
+    asm volatile("" ::: "memory");   // (issued here, a step ahead of their use)
+    T* const ds_tile = reinterpret_cast<T*>(&ex[buf][wave][0]);
+    V8 qf[2], dof[2];
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) {
+      qf[kk] = load8<T>(&rm[buf][0][piece_at(b2q, 2 * kk + g)]);
+      dof[kk] = load8<T>(&rm[buf][1][piece_at(b2q, 2 * kk + g)]);
+    }
+    f32x16 dq;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) dq[r] = 0.0f;
+#pragma unroll
+    for (int b = 0; b < NBK; ++b) {
+      const int blk = b * NW + wave;
+      // (opaque offsets: what all steps or all blocks read alike would be kept in registers that are not there)
+      int kt_off = blk * 1024, rm_off = buf * 2048, st_off = t * 4;
+      asm volatile("" : "+v"(kt_off), "+v"(rm_off), "+v"(st_off));
+      const T* const kb = &kt[0][0] + kt_off;
+      const T* const qd = &rm[0][0][0] + rm_off;
+      f32x16 sm, dp;
+      float b1 = b1v[b];
+      asm volatile("" : "+v"(b1));   // (sixteen registers with the same value, per block)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        sm[r] = b1;
+        dp[r] = stats[1][st_off + 2 * (r >> 3) + g][r & 7];
+      }
+#pragma unroll
+      for (int kk = 0; kk < 2; ++kk) mma32(sm, finite_low(b2n[kk]), one[kk]);   // Bias1 + Bias2
+      __builtin_amdgcn_sched_barrier(0);
+      fetch_bias(b + 1 < NBK ? t : t + 1, b + 1 < NBK ? b + 1 : 0);
+      asm volatile("" ::: "memory");
+#pragma unroll
+      for (int kk = 0; kk < 2; ++kk) {
+        mma32(sm, qf[kk], load8<T>(kb + piece_at(ln, 2 * kk + g)));   // S[query][key] (+ biases)
+        mma32(dp, dof[kk], vf[b][kk]);                                  // dP[query][key] - Delta
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      V8 pf[2], dsf[2];
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks) {
+        const f32x8 nl = stats[0][st_off + 2 * ks + g];
+        f32x8 pv, dv;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const int r = 8 * ks + e;
+          const float pr = fast_exp2(sm[r] * kBwdLog2e + nl[e]);
+          pv[e] = pr;
+          dv[e] = pr * dp[r];
+        }
+        pf[ks] = from_f32<T>(pv);
+        dsf[ks] = from_f32<T>(dv);
+        store8<T>(ds_tile + piece_at(ln, 2 * ks + g), dsf[ks]);   // [key][query]
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks) {
+        mma32(acc_dv[b], turned.load(qd + 1024, ks), pf[ks]);    // dV^T[d][key] += dO^T P
+        mma32(acc_dk[b], turned.load(qd, ks), dsf[ks]);   // dK^T[d][key] += Q^T dS
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      wave_lds_sync();
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks)   // dQ^T[d][query] += K^T dS^T
+        mma32(dq, turned.load(kb, ks), turned.load(ds_tile, ks));
+      wave_lds_sync();
+    }
+    {
+      float* d = reinterpret_cast<float*>(&ex[buf][wave][0]) + lane;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) d[r * kWave] = dq[r];
+    }
+    park(t + 1);
+    // the waves' dQ of this step and the next step's tiles are complete; the other pair of places was read before the
+    // last barrier
+    __syncthreads();
+    if (wave < 4) {   // wave w: registers 4 w .. 4 w + 3, channels 8 w + 4 g .. + 3 of the lane's query
+      f32x4 sum = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int w = 0; w < NW; ++w)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) sum[e] += reinterpret_cast<const float*>(&ex[buf][w][0])[(4 * wave + e) * kWave + lane];
+      const int q = t * 32 + ln;
+      if (q < s) *reinterpret_cast<V4*>((T*)p.dq + elem(p, i, q, h) + 8 * wave + 4 * g) = from_f32<T>(sum);
+    }
+  }
+#pragma unroll
+  for (int b = 0; b < NBK; ++b) {
+    const int key = (b * NW + wave) * 32 + ln;
+    if (key >= s) continue;
+    T* dk = (T*)p.dk + elem(p, i, key, h);
+    T* dv = (T*)p.dv + elem(p, i, key, h);
+#pragma unroll
+    for (int a = 0; a < 4; ++a) {
+      f32x4 x, y;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        x[e] = acc_dk[b][4 * a + e];
+        y[e] = acc_dv[b][4 * a + e];
+      }
+      *reinterpret_cast<V4*>(dk + 8 * a + 4 * g) = from_f32<T>(x);
+      *reinterpret_cast<V4*>(dv + 8 * a + 4 * g) = from_f32<T>(y);
+    }
+  }
+}
+
+// Whether a workgroup takes whole rows (attn_bwd_row_kernel): 16-bit rows whose accumulators for dK and dV fit the registers
+// of eight waves, at least one vector long.  Above 384 positions a workgroup is eight waves that fill a compute unit: from
+// 192 workgroups on.  Both sides, us for the operator forward and backward, 4 heads: 384 rows of 384, 390 | 355; 256 of 65, 95 | 88;
+// 256 of 264, 202 | 180; 48 of 500, 131 | 123; 64 of 768, 267 | 233; 256 of 520, 538 | 517; 768 of 768, 3054 | 2735; and below the
+// line 20 of 520, 93 | 110; 20 of 768, 112 | 158.
+template <typename T>
+bool rows_at_once(const BwdParams& p) {
+  return sizeof(T) == 2 && p.s >= 8 && p.s <= 768 && (p.s <= 384 || (int64_t)p.heads * p.n_rows >= 192);
+}
+
 // dBias2: a workgroup takes 64 queries x 64 keys of one head, a wave one 32 x 32 quadrant, and
 // walks over the rows; the two Q / dO tiles and the two K / V tiles of a row are shared.
 // Works on S^T like dQ.  Bias2 itself does not change along the walk and stays in registers;
@@ -700,7 +955,19 @@ int triattn_bwd(const void* q, const void* k, const void* v, const void* b1, con
   BwdParams p = {q, k, v, o, dout, b1, b2, lse, delta, dq, dk, dv, db2, n_rows, s, heads, slices > 1 ? parts : nullptr, slices};
   const unsigned tiles = (unsigned)((s + 63) / 64);
   const dim3 walk(((unsigned)((s + 127) / 128) * heads * n_rows + 7) / 8 * 8), pairs(tiles * tiles * heads * slices);
-  if ((s & 7) == 0) {
+  const bool joint = rows_at_once<T>(p);
+  if constexpr (sizeof(T) == 2) if (joint) {
+    const dim3 grid(((unsigned)heads * n_rows + 7) / 8 * 8);
+    if (s <= 128) attn_bwd_row_kernel<4, 1><<<grid, dim3(256), 0, stream>>>(p);
+    else if (s <= 256) attn_bwd_row_kernel<4, 2><<<grid, dim3(256), 0, stream>>>(p);
+    else if (s <= 384) attn_bwd_row_kernel<4, 3><<<grid, dim3(256), 0, stream>>>(p);
+    else if (s <= 512) attn_bwd_row_kernel<8, 2><<<grid, dim3(512), 0, stream>>>(p);
+    else attn_bwd_row_kernel<8, 3><<<grid, dim3(512), 0, stream>>>(p);
+  }
+  if (joint) {
+    if (db2 && (s & 7) == 0) attn_bwd_db2_kernel<T, true><<<pairs, dim3(256), 0, stream>>>(p);
+    else if (db2) attn_bwd_db2_kernel<T, false><<<pairs, dim3(256), 0, stream>>>(p);
+  } else if ((s & 7) == 0) {
     attn_bwd_dq_kernel<T, true><<<walk, dim3(256), 0, stream>>>(p);   // (writes Delta: first)
     attn_bwd_kv_kernel<T, true><<<walk, dim3(256), 0, stream>>>(p);
     if (db2) attn_bwd_db2_kernel<T, true><<<pairs, dim3(256), 0, stream>>>(p);
