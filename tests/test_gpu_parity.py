@@ -151,6 +151,22 @@ def test_layernorm_backward_c_abi_options_and_determinism():
     assert all(torch.equal(a, b) for a, b in zip(ones, none))
 
 
+@pytest.mark.parametrize("cols", [1, 15, 16, 17, 128, 384])
+def test_layernorm_backward_parameter_sums_are_complete(cols):
+    """Whole numbers, so that dgamma = sum dout x and dbeta = sum dout are exact in any order: 1 to 1024 rows of partial
+    sums, on both sides of every multiple of what a pass over them takes."""
+    from protenix_amd import ops
+    g = torch.Generator().manual_seed(cols)
+    per = max(4, 4 * (64 // max(1, -(-cols // 4))))      # rows per partial row, up to a factor
+    for parts in (1, 2, 63, 64, 65, 447, 448, 449, 511, 512, 513, 577, 1023, 1024, 1500):
+        rows = parts * per
+        x, dout = (torch.randint(-3, 4, (rows, cols), generator=g).float().cuda() for _ in range(2))
+        mean, rstd = torch.zeros(rows, device="cuda"), torch.ones(rows, device="cuda")
+        _, dg, db = ops.layer_norm_backward(dout, x, mean, rstd, None, True, True)
+        assert torch.equal(dg, (dout * x).double().sum(0).float()), parts
+        assert torch.equal(db, dout.double().sum(0).float()), parts
+
+
 # ------------------------------------------------------------------ TriMul
 @pytest.mark.parametrize("mode", ["fp32", "bf16", "mixed"])
 @pytest.mark.parametrize("direction", ["outgoing", "incoming"])
