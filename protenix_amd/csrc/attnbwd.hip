@@ -485,7 +485,7 @@ __global__ __launch_bounds__(256, (BwdCfg<T, VEC>::kMinWaves)) void attn_bwd_kv_
   }
 }
 
-// LDS tiles of 32 x 32 elements: rows of 64 bytes, their four 16-byte pieces exchanged by bits 2 and 3 of the row, so that
+// LDS tiles of 32 channels, 16-bit: rows of 64 bytes, their four 16-byte pieces exchanged by bits 2 and 3 of the row, so that
 // neither eight rows' pieces (vector reads and writes) nor four rows' halves (turning reads) meet in a bank.
 __device__ __forceinline__ int piece_at(int row, int piece) { return row * 32 + ((piece ^ ((row >> 2) & 3)) << 3); }
 
@@ -739,6 +739,12 @@ bool rows_at_once(const BwdParams& p) {
   return sizeof(T) == 2 && p.s >= 8 && p.s <= 768 && (p.s <= 384 || (int64_t)p.heads * p.n_rows >= 192);
 }
 
+// dBias2's tiles: 16-bit rows as above (padded to 80 bytes a third of the LDS cycles were conflicts: the operator at 768 rows of 768
+// positions, forward and backward, 2735 -> 2640 us, 384 360 -> 357), fp32 ones padded
+template <typename T>
+__device__ __forceinline__ int db2_at(int row, int piece) { return sizeof(T) == 2 ? piece_at(row, piece) : row * kTP + 8 * piece; }
+template <typename T> constexpr int kDb2Tile = 64 * (sizeof(T) == 2 ? 32 : kTP);
+
 // dBias2: a workgroup takes 64 queries x 64 keys of one head, a wave one 32 x 32 quadrant, and
 // walks over the rows; the two Q / dO tiles and the two K / V tiles of a row are shared.
 // Works on S^T like dQ.  Bias2 itself does not change along the walk and stays in registers;
@@ -755,7 +761,7 @@ template <typename T, bool VEC>
 __global__ __launch_bounds__(256, (BwdCfg<T, VEC>::kMinWaves)) void attn_bwd_db2_kernel(BwdParams p) {
   typedef typename Vec8<T>::type V8;
   constexpr int NB = BwdCfg<T, VEC>::kBuffers;
-  __shared__ __attribute__((aligned(32))) T tiles[NB][4][64 * kTP];   // Q, dO (64 queries), K, V (64 keys)
+  __shared__ __attribute__((aligned(32))) T tiles[NB][4][kDb2Tile<T>];   // Q, dO (64 queries), K, V (64 keys)
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, ln = lane & 31, g = lane >> 5;
   const int s = p.s, H = p.heads;
   constexpr bool vec = VEC;
@@ -781,7 +787,7 @@ __global__ __launch_bounds__(256, (BwdCfg<T, VEC>::kMinWaves)) void attn_bwd_db2
   // thread t: 8 channels (t & 3) of row t >> 2 of each of the four 64-row tiles.  Along the
   // walk only the row's base address changes, the same for all lanes: what a lane adds to it
   // is formed once.
-  const int crow = tid >> 2, cc = 8 * (tid & 3);
+  const int crow = tid >> 2, cc = 8 * (tid & 3), park_at = db2_at<T>(crow, tid & 3);
   const unsigned off_q = ((unsigned)min(qs0 + crow, s - 1) * H + h) * 32 + cc;
   const unsigned off_k = ((unsigned)min(ks0 + crow, s - 1) * H + h) * 32 + cc;
   const unsigned off_stat = (unsigned)qi * H + h;
@@ -823,7 +829,7 @@ __global__ __launch_bounds__(256, (BwdCfg<T, VEC>::kMinWaves)) void attn_bwd_db2
   const int last = row_end - 1;
   fetch(row_begin);
 #pragma unroll
-  for (int w = 0; w < 4; ++w) store8<T>(&tiles[row_begin % NB][w][crow * kTP + cc], piece[w]);
+  for (int w = 0; w < 4; ++w) store8<T>(&tiles[row_begin % NB][w][park_at], piece[w]);
   float neg_mq = -mq_n, neg_dq = -dq_n;
   V8 b1c[2] = {b1n[0], b1n[1]};
   T b1m = b1m_n;
@@ -852,10 +858,10 @@ __global__ __launch_bounds__(256, (BwdCfg<T, VEC>::kMinWaves)) void attn_bwd_db2
     }
 #pragma unroll
     for (int kk = 0; kk < 2; ++kk) {
-      const V8 qf = load8<T>(&tiles[buf][0][(32 * wq + ln) * kTP + 16 * kk + 8 * g]);
-      const V8 dof = load8<T>(&tiles[buf][1][(32 * wq + ln) * kTP + 16 * kk + 8 * g]);
-      const V8 kf = load8<T>(&tiles[buf][2][(32 * wk + perm_row(ln)) * kTP + 16 * kk + 8 * g]);
-      const V8 vf = load8<T>(&tiles[buf][3][(32 * wk + perm_row(ln)) * kTP + 16 * kk + 8 * g]);
+      const V8 qf = load8<T>(&tiles[buf][0][db2_at<T>(32 * wq + ln, 2 * kk + g)]);
+      const V8 dof = load8<T>(&tiles[buf][1][db2_at<T>(32 * wq + ln, 2 * kk + g)]);
+      const V8 kf = load8<T>(&tiles[buf][2][db2_at<T>(32 * wk + perm_row(ln), 2 * kk + g)]);
+      const V8 vf = load8<T>(&tiles[buf][3][db2_at<T>(32 * wk + perm_row(ln), 2 * kk + g)]);
       mma32(st, kf, qf);    // S^T[key][query] (+ biases)
       mma32(dp, vf, dof);   // dP^T[key][query] - Delta
     }
@@ -864,7 +870,7 @@ __global__ __launch_bounds__(256, (BwdCfg<T, VEC>::kMinWaves)) void attn_bwd_db2
     if (NB == 1) __syncthreads();
     // the next row: tiles into LDS, its statistics and Bias1 into this step's places
 #pragma unroll
-    for (int w = 0; w < 4; ++w) store8<T>(&tiles[(i + 1) % NB][w][crow * kTP + cc], piece[w]);
+    for (int w = 0; w < 4; ++w) store8<T>(&tiles[(i + 1) % NB][w][park_at], piece[w]);
     neg_mq = -mq_n;
     neg_dq = -dq_n;
 #pragma unroll
