@@ -68,7 +68,7 @@ def _work(n: int, z_bytes: int) -> dict:
 
 def _attn_update_ms(times: dict) -> float:
     """Median time of the attention core per triangle-attention update: a padded batch from
-    480 tokens on runs it as two launches (valid rows, padded rows), timed under two names."""
+    352 tokens on runs it as two launches (valid rows, padded rows), timed under two names."""
     t = statistics.median(times["triattn_fwd"])
     if "triattn_fwd_padded_rows" in times:
         t += statistics.median(times["triattn_fwd_padded_rows"])
@@ -446,9 +446,9 @@ def main() -> int:
                     "bwd_frac_mfma": round(1280.0 * 768 ** 3 / (bm * 1e-3) / 1e12 / PEAK_BF16_TFLOPS, 4),
                     "algorithmic": "backward: 5 products of 2 * 768^3 * 4 * 32 flop (dV, dP, dS^T Q, dS K, "
                                    "and the logits once); the kernels recompute the logits and dP in each of "
-                                   "three passes, 10 products executed, and add the biases on the matrix pipe",
+                                   "two passes, 7 products executed, and add the biases on the matrix pipe",
                     "workload": "TriAttentionFunction.apply + backward (dQ, dK, dV, dBias2); fwd_ms includes "
-                                "the scaling of Q and the repack of the operands into the core's tile order"}
+                                "the scaling of Q and the repack of Bias2 into the core's tile order"}
                 del qkv, qo, ko, vo, do, b1o, b2o, oo
             # the scaled-up model's block (c_z = 256, 8 pair heads, c_hidden_mul = 256), fp32 rows
             # under bf16 autocast: the fused fp32-row kernels of that width

@@ -361,7 +361,7 @@ PTX_API int ptx_triattn_fwd_carry(const void* q, const void* k, const void* vt, 
  *   lse         fp32 [batch][n_rows][s][heads] or NULL: log2 of the sum over keys of
  *               2^(logit * log2 e), the reference's M (forward.py:185-188)
  *   workspace   ptx_triattn_core_workspace_elems(n_rows, s, heads) elements of `dtype`,
- *               uninitialised (the operands repacked into the core's tile order)
+ *               uninitialised (operands repacked into the core's tile order, those that are not read as they are)
  * The logits are formed as (q.k + Bias1) + Bias2 in fp32 wherever Bias1 is non-zero, the
  * order of layers.py:286-289; they are never materialised.  n_rows may differ from s (a chunk
  * of rows).  dtype PTX_F32 or PTX_BF16.

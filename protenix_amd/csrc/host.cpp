@@ -428,8 +428,9 @@ constexpr float kEps = 1e-5f;
 
 // The stages of the single tracks of earlier blocks, in order: every pair launch that can carry one takes the
 // first, so that a block's single track runs underneath the next block's pair kernels without launches,
-// streams or waits of its own.  A block has seven of each; where one of its projections is faster without (see Run::carry),
-// the two LayerNorms, 5 us each, are launched by themselves.
+// streams or waits of its own.  A block has seven stages and, its updates apart, seven such launches; where one of its projections is
+// faster without (see Run::carry), the two LayerNorms, 5 us each, are launched by themselves; chained updates (Block::chain) have fewer
+// launches, and their contractions, cores and transition take stages too.
 struct Stages {
   struct Named {
     ptx_single_stage stage;
