@@ -687,7 +687,10 @@ int triattn_output_transition_fwd(const void* o, const void* z, const void* att_
                                   float att_eps, float eps, const void* pb_ln_w, const void* pb_ln_b,
                                   const void* pb_w, void* bias, int heads, int bias_f32, float pb_eps,
                                   hipStream_t stream, const SingleStage* carry) {
-  if (carry && (n == 0 || !pb_w || !transition_carries((int64_t)n * n))) single_stage_run(carry, stream);
+  if (carry && (n == 0 || !pb_w || !transition_carries((int64_t)n * n))) {
+    single_stage_run(carry, stream);
+    carry = nullptr;
+  }
   if (n == 0) return 0;
   if constexpr (sizeof(T) == 2) {
     constexpr int KS = 8;
