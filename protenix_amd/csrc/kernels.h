@@ -125,8 +125,6 @@ int single_stage_run(const SingleStage* s, hipStream_t stream);
 // carry: null, or a stage of the single track that the launch's first workgroups run (it must not depend on the launch), where
 // nt_gemm_carries(); elsewhere the stage is launched in front.
 bool nt_gemm_carries(int n, bool bits16);
-// How far the product reads its operands' K for n tokens: what the projections write, zeros from n on.
-int nt_gemm_k_extent(int n, bool bits16);
 template <typename T>
 int nt_gemm_batched(const T* a, const T* b, T* x, int n, int ldx, int k_pitch, int batch, const SingleStage* carry, hipStream_t stream);
 

@@ -510,7 +510,6 @@ static void launch_ring(const bf16_t* a, const bf16_t* b, bf16_t* x, int n, int 
   nt_gemm_ring_kernel<RM, RN, void><<<dim3(groups), dim3(256), 0, stream>>>(a, b, x, n, ldx, k_pitch, batch, tiles, tiles_j, SingleStage{}, 0u);
 }
 bool nt_gemm_carries(int n, bool bits16) { return bits16 && n <= 256; }
-int nt_gemm_k_extent(int n, bool bits16) { return bits16 && n <= 256 ? (n + 31) / 32 * 32 : (n + 63) / 64 * 64; }
 static bool ring_takes(const bf16_t* a, const bf16_t* b, bf16_t* x, int n, int ldx, int k_pitch, int batch, const SingleStage* carry,
                        hipStream_t stream) {
   // us, persistent / 64 x 64 / 128 x 128 (128 channels): n = 64 6.7 / 2.5 / 3.3, 160 10.9 / 6.3 / 6.6, 192 11.2 / 7.7 / 8.1, 224 13.1 / 10.3 / 9.4,

@@ -100,7 +100,6 @@ struct ProjInParams {
   int heads;
   int slices;             // workgroups per tile, each with its share of the output columns (see in_slices)
   unsigned tiles;
-  unsigned n_kb;          // trimul_in: blocks of 8 inner indices
   int share;              // trimul_in: a wave's chunks per slice
   float q_scale;
 };
@@ -136,6 +135,28 @@ struct MulColumns {
       mask_of(stage_lds)[threadIdx.x] = k < n ? mv : 0.0f;   // (the contraction relies on zeros between n and the pitch)
     }
   }
+  // this lane's vector of row block 0 of the patch inside a channel block's planes
+  static __device__ __forceinline__ uint32_t vector_at(const ProjInParams& p, int pi0, int pk0, int ps, int lane) {
+    int chn, r0;
+    stage_coord<T>(ps, lane, chn, r0);
+    const int i = pi0 + (r0 >> 3), n_rb = (p.n + 31) >> 5, n_ks = p.pitch >> 4;
+    return (uint32_t)(trimul_frag_offset(chn, i >> 5, pk0 >> 4, n_rb, n_ks) + ((pk0 >> 3) & 1) * 256 + (i & 31) * 8 + (r0 & 7));
+  }
+  // a patch of inner indices that all lie between n and the pitch
+  static __device__ __forceinline__ void put_zeros(const ProjInParams& p, int pi0, int pk0, int c_begin, int c_end, int wave, int lane) {
+    asm volatile("" : "+v"(lane));   // (what it computes stays here: kept for the other patches it would take registers from them)
+    const int n_rb = (p.n + 31) >> 5, n_ks = p.pitch >> 4;
+    VE_t zero;
+#pragma unroll
+    for (int t = 0; t < C::VE; ++t) zero[t] = (T)0.0f;
+    for (int ch = wave * CHW + c_begin; ch < wave * CHW + c_end; ++ch) {
+      T* outp = (T*)(ch < CPM ? p.out[0] : p.out[1]) + trimul_frag_offset((ch % CPM) * 32, 0, 0, n_rb, n_ks);
+#pragma unroll
+      for (int ps = 0; ps < C::NPASS; ++ps)
+#pragma unroll
+        for (int rb = 0; rb < RBW; ++rb) *reinterpret_cast<VE_t*>(outp + vector_at(p, pi0, pk0, ps, lane) + rb * 32) = zero;
+    }
+  }
   // chunks c_begin .. c_end - 1 of the wave's; the first one's weights have been requested
   __device__ __forceinline__ void run(const ProjInParams& p, const char* frag, char* stage_lds, int pi0, int pk0, int c_begin, int c_end, int wave,
                                       int lane) {
@@ -146,15 +167,9 @@ struct MulColumns {
     const int n = p.n, g = lane >> 5;
     T* st = stage[wave];
     const int n_rb = (n + 31) >> 5, n_ks = p.pitch >> 4;
-    // this lane's vector of row block 0 inside a channel block's planes
     uint32_t rel[C::NPASS];
 #pragma unroll
-    for (int ps = 0; ps < C::NPASS; ++ps) {
-      int chn, r0;
-      stage_coord<T>(ps, lane, chn, r0);
-      const int i = pi0 + (r0 >> 3);
-      rel[ps] = (uint32_t)(trimul_frag_offset(chn, i >> 5, pk0 >> 4, n_rb, n_ks) + ((pk0 >> 3) & 1) * 256 + (i & 31) * 8 + (r0 & 7));
-    }
+    for (int ps = 0; ps < C::NPASS; ++ps) rel[ps] = vector_at(p, pi0, pk0, ps, lane);
 #pragma unroll
     for (int c = 0; c < CHW; ++c) {
       if (c < c_begin || c >= c_end) continue;
@@ -207,7 +222,7 @@ __global__ __launch_bounds__(kPpWaves * 64, (kPpMinWaves<T, KS>)) void pp_trimul
   char* const frag = smem;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int n = p.n;
-  const uint32_t n_kb = p.n_kb, n_ip = (uint32_t)(n + 4 * RBW - 1) / (4 * RBW);
+  const uint32_t n_kb = (uint32_t)p.pitch >> 3, n_ip = (uint32_t)(n + 4 * RBW - 1) / (4 * RBW);
   // back to front behind a kernel that wrote the pair tensor front to back (the tail is what the memory-side cache still holds)
   const uint32_t tiles = p.tiles, slice = (block >= tiles) + (block >= 2 * tiles) + (block >= 3 * tiles);
   const uint32_t bx = xcd_run(block - slice * tiles, tiles), tile = p.backward ? tiles - 1 - bx : bx;
@@ -221,6 +236,11 @@ __global__ __launch_bounds__(kPpWaves * 64, (kPpMinWaves<T, KS>)) void pp_trimul
     pi0 = ip * (4 * RBW);
     pk0 = (tile - ip * n_kb) * 8;
   }
+  const int c_begin = slice * p.share, c_end = c_begin + p.share;   // this slice's chunks of every wave
+  if (pk0 >= n) {
+    Columns::put_zeros(p, pi0, pk0, c_begin, c_end, wave, lane);
+    return;
+  }
   Columns columns;
   typename RowPieces<TZ, KS>::V raw[RBW][RowPieces<TZ, KS>::NP];
   norm_rows<T, TZ, KS, RBW>(
@@ -230,7 +250,6 @@ __global__ __launch_bounds__(kPpWaves * 64, (kPpMinWaves<T, KS>)) void pp_trimul
         return i * p.si + k * p.sj;
       },
       (const T*)p.gamma, (const T*)p.beta, p.eps, wave, lane, raw);
-  const int c_begin = slice * p.share, c_end = c_begin + p.share;   // this slice's chunks of every wave
   columns.load_w(p, wave * Columns::CHW + c_begin, lane);
   Columns::put_mask(p, smem + kFrag, pi0, pk0);
   __syncthreads();
@@ -751,6 +770,10 @@ __global__ __launch_bounds__(kPpWaves * 64, (kPpMinWaves<T, KS>)) void pp_mul_ou
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const uint32_t n_ip = (uint32_t)(p.n + 4 * RBW - 1) / (4 * RBW), tile = xcd_run(block, blocks), kb = tile / n_ip;
   const PatchRows tr = {(int)(tile - kb * n_ip) * (4 * RBW), (int)kb * 8, p.n};
+  if (tr.j0 >= p.n) {
+    Columns::put_zeros(pi, tr.i0, tr.j0, 0, Columns::CHW, wave, lane);
+    return;
+  }
   const PatchRowsT trt = {tr};
   typename RowPieces<TZ, KS>::V raw[RBW][RowPieces<TZ, KS>::NP];
   const T* upd = Out::run(p, trt, smem, wave, lane, raw);
@@ -947,8 +970,7 @@ static int pp_trimul_in_ks(ProjInParams p, const SingleStage* carry, hipStream_t
   if (carry && KS <= 4) single_stage_run(carry, stream);
   if (!carry || KS <= 4) carry = &none;
   const unsigned carried = single_stage_groups(carry);
-  p.n_kb = (unsigned)nt_gemm_k_extent(p.n, sizeof(T) == 2) / 8;
-  const unsigned tiles = (unsigned)((p.n + 4 * rbw - 1) / (4 * rbw)) * p.n_kb;
+  const unsigned tiles = (unsigned)((p.n + 4 * rbw - 1) / (4 * rbw)) * (unsigned)(p.pitch / 8);
   constexpr int kChunks = PpWidths<KS>::HIDDEN / 64;   // per wave
   p.slices = in_slices(tiles, kChunks, sizeof(T) == 2);
   if (kChunks % p.slices) --p.slices;   // (2 or 4 chunks: equal shares)
@@ -1179,7 +1201,7 @@ int pp_triattn_out(const void* o, const void* z, const void* ln_w, const void* l
 // 715 / 715 / 714, 300 1114 / 1133 / 1139.
 // The two multiplications (up to 256 tokens, where the products take the operands of any patch order from the L2), us per block
 // without / with: 40 tokens 74.5 / 68.6, 93 110 / 102, 128 118 / 115, 200 226 / 216, 256 276 / 275; without a single track 200 221 / 213, 256
-// 263 / 257; 64 channels 64 60 / 57, 200 169 / 165 (zeros beyond n written up to the next 32 tokens only are a part of that).
+// 263 / 257; 64 channels 64 60 / 57, 200 169 / 165.
 bool pp_joined(int pair, int n, int c_z, int hidden, bool rows16) {
   if (pair == 0) return n <= 256 && c_z <= 128;
   if (c_z == 256) return n <= 256;
@@ -1298,7 +1320,7 @@ static void mul_out_mul_in_ks(const ProjOutParams& p, const ProjInParams& pi, co
   if (carry && KS <= 4) single_stage_run(carry, stream);
   if (!carry || KS <= 4) carry = &none;
   const unsigned carried = single_stage_groups(carry);
-  const dim3 grid(carried + (unsigned)((p.n + 4 * rbw - 1) / (4 * rbw)) * (unsigned)(nt_gemm_k_extent(p.n, true) / 8)), block(kPpWaves * 64);
+  const dim3 grid(carried + (unsigned)((p.n + 4 * rbw - 1) / (4 * rbw)) * (unsigned)(pi.pitch / 8)), block(kPpWaves * 64);
   if (rbw == 2) pp_mul_out_mul_in_kernel<bf16_t, TZ, KS, 2><<<grid, block, 0, stream>>>(p, pi, *carry, carried);
   else pp_mul_out_mul_in_kernel<bf16_t, TZ, KS, 1><<<grid, block, 0, stream>>>(p, pi, *carry, carried);
 }
