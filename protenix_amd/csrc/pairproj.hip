@@ -100,6 +100,7 @@ struct ProjInParams {
   int heads;
   int slices;             // workgroups per tile, each with its share of the output columns (see in_slices)
   unsigned tiles;
+  unsigned work;          // trimul_in: workgroups before those that write zeros only
   int share;              // trimul_in: a wave's chunks per slice
   float q_scale;
 };
@@ -135,26 +136,23 @@ struct MulColumns {
       mask_of(stage_lds)[threadIdx.x] = k < n ? mv : 0.0f;   // (the contraction relies on zeros between n and the pitch)
     }
   }
-  // this lane's vector of row block 0 of the patch inside a channel block's planes
-  static __device__ __forceinline__ uint32_t vector_at(const ProjInParams& p, int pi0, int pk0, int ps, int lane) {
-    int chn, r0;
-    stage_coord<T>(ps, lane, chn, r0);
-    const int i = pi0 + (r0 >> 3), n_rb = (p.n + 31) >> 5, n_ks = p.pitch >> 4;
-    return (uint32_t)(trimul_frag_offset(chn, i >> 5, pk0 >> 4, n_rb, n_ks) + ((pk0 >> 3) & 1) * 256 + (i & 31) * 8 + (r0 & 7));
-  }
-  // a patch of inner indices that all lie between n and the pitch
-  static __device__ __forceinline__ void put_zeros(const ProjInParams& p, int pi0, int pk0, int c_begin, int c_end, int wave, int lane) {
-    asm volatile("" : "+v"(lane));   // (what it computes stays here: kept for the other patches it would take registers from them)
-    const int n_rb = (p.n + 31) >> 5, n_ks = p.pitch >> 4;
+  // Patches along the inner index: whole K steps of the contraction.
+  static __host__ __device__ __forceinline__ uint32_t patches_k(int n) { return 2 * ((uint32_t)(n + 15) >> 4); }
+  // The K steps that hold nothing but the zeros up to the pitch, whole fragments: 16 channels of one operand and row block a
+  // workgroup.  (As patches, which write 64 bytes at a time, they cost both multiplications 3 us of 72 at 200 tokens.)
+  static int zero_groups(int n, int pitch) { return (pitch >> 4) > (n + 15) >> 4 ? ((n + 31) >> 5) * (2 * PpWidths<KS>::HIDDEN / 16) : 0; }
+  static __device__ __forceinline__ void put_zeros(const ProjInParams& p, uint32_t group, int wave, int lane) {
+    const int n_rb = (p.n + 31) >> 5, n_ks = p.pitch >> 4, ks0 = (p.n + 15) >> 4;
+    const uint32_t per_rb = 2 * PpWidths<KS>::HIDDEN / 16, rb = group / per_rb;
+    const int ch0 = (int)(group - rb * per_rb) * 16;
+    T* const operand = (T*)(ch0 < PpWidths<KS>::HIDDEN ? p.out[0] : p.out[1]);
     VE_t zero;
 #pragma unroll
     for (int t = 0; t < C::VE; ++t) zero[t] = (T)0.0f;
-    for (int ch = wave * CHW + c_begin; ch < wave * CHW + c_end; ++ch) {
-      T* outp = (T*)(ch < CPM ? p.out[0] : p.out[1]) + trimul_frag_offset((ch % CPM) * 32, 0, 0, n_rb, n_ks);
-#pragma unroll
-      for (int ps = 0; ps < C::NPASS; ++ps)
-#pragma unroll
-        for (int rb = 0; rb < RBW; ++rb) *reinterpret_cast<VE_t*>(outp + vector_at(p, pi0, pk0, ps, lane) + rb * 32) = zero;
+#pragma unroll 1
+    for (int c = wave; c < 16; c += kPpWaves) {
+      T* dst = operand + trimul_frag_offset((ch0 + c) % PpWidths<KS>::HIDDEN, (int)rb, ks0, n_rb, n_ks) + lane * C::VE;
+      for (int e = 0; e < (n_ks - ks0) * kFragElems; e += kWave * C::VE) *reinterpret_cast<VE_t*>(dst + e) = zero;
     }
   }
   // chunks c_begin .. c_end - 1 of the wave's; the first one's weights have been requested
@@ -167,9 +165,15 @@ struct MulColumns {
     const int n = p.n, g = lane >> 5;
     T* st = stage[wave];
     const int n_rb = (n + 31) >> 5, n_ks = p.pitch >> 4;
+    // this lane's vector of row block 0 inside a channel block's planes
     uint32_t rel[C::NPASS];
 #pragma unroll
-    for (int ps = 0; ps < C::NPASS; ++ps) rel[ps] = vector_at(p, pi0, pk0, ps, lane);
+    for (int ps = 0; ps < C::NPASS; ++ps) {
+      int chn, r0;
+      stage_coord<T>(ps, lane, chn, r0);
+      const int i = pi0 + (r0 >> 3);
+      rel[ps] = (uint32_t)(trimul_frag_offset(chn, i >> 5, pk0 >> 4, n_rb, n_ks) + ((pk0 >> 3) & 1) * 256 + (i & 31) * 8 + (r0 & 7));
+    }
 #pragma unroll
     for (int c = 0; c < CHW; ++c) {
       if (c < c_begin || c >= c_end) continue;
@@ -222,7 +226,11 @@ __global__ __launch_bounds__(kPpWaves * 64, (kPpMinWaves<T, KS>)) void pp_trimul
   char* const frag = smem;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int n = p.n;
-  const uint32_t n_kb = (uint32_t)p.pitch >> 3, n_ip = (uint32_t)(n + 4 * RBW - 1) / (4 * RBW);
+  const uint32_t n_kb = Columns::patches_k(n), n_ip = (uint32_t)(n + 4 * RBW - 1) / (4 * RBW);
+  if (block >= p.work) {
+    Columns::put_zeros(p, block - p.work, wave, lane);
+    return;
+  }
   // back to front behind a kernel that wrote the pair tensor front to back (the tail is what the memory-side cache still holds)
   const uint32_t tiles = p.tiles, slice = (block >= tiles) + (block >= 2 * tiles) + (block >= 3 * tiles);
   const uint32_t bx = xcd_run(block - slice * tiles, tiles), tile = p.backward ? tiles - 1 - bx : bx;
@@ -237,10 +245,6 @@ __global__ __launch_bounds__(kPpWaves * 64, (kPpMinWaves<T, KS>)) void pp_trimul
     pk0 = (tile - ip * n_kb) * 8;
   }
   const int c_begin = slice * p.share, c_end = c_begin + p.share;   // this slice's chunks of every wave
-  if (pk0 >= n) {
-    Columns::put_zeros(p, pi0, pk0, c_begin, c_end, wave, lane);
-    return;
-  }
   Columns columns;
   typename RowPieces<TZ, KS>::V raw[RBW][RowPieces<TZ, KS>::NP];
   norm_rows<T, TZ, KS, RBW>(
@@ -768,12 +772,13 @@ __global__ __launch_bounds__(kPpWaves * 64, (kPpMinWaves<T, KS>)) void pp_mul_ou
   __shared__ __attribute__((aligned(16))) char smem[cmax(cmax(Out::kLds, Out::kFrag + Columns::kStage), kStageLds)];
   PTX_CARRIED_STAGE();
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const uint32_t n_ip = (uint32_t)(p.n + 4 * RBW - 1) / (4 * RBW), tile = xcd_run(block, blocks), kb = tile / n_ip;
-  const PatchRows tr = {(int)(tile - kb * n_ip) * (4 * RBW), (int)kb * 8, p.n};
-  if (tr.j0 >= p.n) {
-    Columns::put_zeros(pi, tr.i0, tr.j0, 0, Columns::CHW, wave, lane);
+  const uint32_t n_ip = (uint32_t)(p.n + 4 * RBW - 1) / (4 * RBW), work = n_ip * Columns::patches_k(p.n);
+  if (block >= work) {
+    Columns::put_zeros(pi, block - work, wave, lane);
     return;
   }
+  const uint32_t tile = xcd_run(block, work), kb = tile / n_ip;
+  const PatchRows tr = {(int)(tile - kb * n_ip) * (4 * RBW), (int)kb * 8, p.n};
   const PatchRowsT trt = {tr};
   typename RowPieces<TZ, KS>::V raw[RBW][RowPieces<TZ, KS>::NP];
   const T* upd = Out::run(p, trt, smem, wave, lane, raw);
@@ -965,18 +970,20 @@ static int in_slices(int64_t tiles, int most, bool bits16) {
 
 template <typename T, typename TZ, int KS>
 static int pp_trimul_in_ks(ProjInParams p, const SingleStage* carry, hipStream_t stream) {
+  typedef MulColumns<T, KS, 1> Columns;   // (its numbers of workgroups do not depend on the row blocks)
   const int rbw = sizeof(T) == 2 ? in_row_blocks((int64_t)p.n * p.n, KS, false) : 1;
   static const SingleStage none = {};
   if (carry && KS <= 4) single_stage_run(carry, stream);
   if (!carry || KS <= 4) carry = &none;
   const unsigned carried = single_stage_groups(carry);
-  const unsigned tiles = (unsigned)((p.n + 4 * rbw - 1) / (4 * rbw)) * (unsigned)(p.pitch / 8);
+  const unsigned tiles = (unsigned)((p.n + 4 * rbw - 1) / (4 * rbw)) * Columns::patches_k(p.n);
   constexpr int kChunks = PpWidths<KS>::HIDDEN / 64;   // per wave
   p.slices = in_slices(tiles, kChunks, sizeof(T) == 2);
   if (kChunks % p.slices) --p.slices;   // (2 or 4 chunks: equal shares)
   p.tiles = tiles;
   p.share = kChunks / p.slices;
-  const dim3 grid(carried + tiles * p.slices), block(kPpWaves * 64);
+  p.work = tiles * p.slices;
+  const dim3 grid(carried + p.work + Columns::zero_groups(p.n, p.pitch)), block(kPpWaves * 64);
   if constexpr (sizeof(T) == 2) {
     if (rbw == 4) {
       pp_trimul_in_kernel<T, TZ, KS, 4><<<grid, block, 0, stream>>>(p, *carry, carried);
@@ -1320,7 +1327,9 @@ static void mul_out_mul_in_ks(const ProjOutParams& p, const ProjInParams& pi, co
   if (carry && KS <= 4) single_stage_run(carry, stream);
   if (!carry || KS <= 4) carry = &none;
   const unsigned carried = single_stage_groups(carry);
-  const dim3 grid(carried + (unsigned)((p.n + 4 * rbw - 1) / (4 * rbw)) * (unsigned)(pi.pitch / 8)), block(kPpWaves * 64);
+  typedef MulColumns<bf16_t, KS, 1> Columns;
+  const unsigned work = (unsigned)((p.n + 4 * rbw - 1) / (4 * rbw)) * Columns::patches_k(p.n);
+  const dim3 grid(carried + work + Columns::zero_groups(pi.n, pi.pitch)), block(kPpWaves * 64);
   if (rbw == 2) pp_mul_out_mul_in_kernel<bf16_t, TZ, KS, 2><<<grid, block, 0, stream>>>(p, pi, *carry, carried);
   else pp_mul_out_mul_in_kernel<bf16_t, TZ, KS, 1><<<grid, block, 0, stream>>>(p, pi, *carry, carried);
 }
