@@ -190,6 +190,10 @@ struct MulColumns {
           mma32(acc[0], xv, w[0][kk]);   // lane <-> channel, register <-> row
           mma32(acc[1], xv, w[1][kk]);
         }
+        // (the products stay together: mixed with the staging below they take 138 registers from two row blocks of 16-bit rows and
+        // leave three waves per SIMD instead of four.  us for both multiplications of bf16 rows, so / as here: 300 tokens 137 / 135, 352
+        // 167 / 163, 387 218 / 214, 440 256 / 251)
+        if constexpr (sizeof(T) == 2 && RBW == 2) __builtin_amdgcn_sched_barrier(0);
         if (rb == RBW - 1 && c + 1 < CHW && c + 1 < c_end) load_w(p, ch + 1, lane);
         float vals[16];
 #pragma unroll
@@ -231,8 +235,10 @@ __global__ __launch_bounds__(kPpWaves * 64, (kPpMinWaves<T, KS>)) void pp_trimul
     Columns::put_zeros(p, block - p.work, wave, lane);
     return;
   }
+  // (slices: of one row block only, see in_slices)
+  constexpr bool kSliced = RBW == 1;
   // back to front behind a kernel that wrote the pair tensor front to back (the tail is what the memory-side cache still holds)
-  const uint32_t tiles = p.tiles, slice = (block >= tiles) + (block >= 2 * tiles) + (block >= 3 * tiles);
+  const uint32_t tiles = p.tiles, slice = kSliced ? (block >= tiles) + (block >= 2 * tiles) + (block >= 3 * tiles) : 0u;
   const uint32_t bx = xcd_run(block - slice * tiles, tiles), tile = p.backward ? tiles - 1 - bx : bx;
   int pi0, pk0;
   if (p.backward) {   // incoming: the inner index is the slow one of z
@@ -244,7 +250,7 @@ __global__ __launch_bounds__(kPpWaves * 64, (kPpMinWaves<T, KS>)) void pp_trimul
     pi0 = ip * (4 * RBW);
     pk0 = (tile - ip * n_kb) * 8;
   }
-  const int c_begin = slice * p.share, c_end = c_begin + p.share;   // this slice's chunks of every wave
+  const int c_begin = kSliced ? slice * p.share : 0, c_end = kSliced ? c_begin + p.share : Columns::CHW;   // this slice's chunks of every wave
   Columns columns;
   typename RowPieces<TZ, KS>::V raw[RBW][RowPieces<TZ, KS>::NP];
   norm_rows<T, TZ, KS, RBW>(
@@ -978,7 +984,7 @@ static int pp_trimul_in_ks(ProjInParams p, const SingleStage* carry, hipStream_t
   const unsigned carried = single_stage_groups(carry);
   const unsigned tiles = (unsigned)((p.n + 4 * rbw - 1) / (4 * rbw)) * Columns::patches_k(p.n);
   constexpr int kChunks = PpWidths<KS>::HIDDEN / 64;   // per wave
-  p.slices = in_slices(tiles, kChunks, sizeof(T) == 2);
+  p.slices = rbw == 1 ? in_slices(tiles, kChunks, sizeof(T) == 2) : 1;
   if (kChunks % p.slices) --p.slices;   // (2 or 4 chunks: equal shares)
   p.tiles = tiles;
   p.share = kChunks / p.slices;
