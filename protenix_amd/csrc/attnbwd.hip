@@ -107,6 +107,12 @@ template <typename T> struct Turned {
 };
 __device__ __forceinline__ f32x8 load8_turned(const float*, int, int, int, int) { return f32x8{}; }   // (never called)
 
+// -inf as the lowest finite value, so that a product with 0 is 0 (a NaN's row is NaN throughout by its log-sum-exp).
+__device__ __forceinline__ Vec8<bf16_t>::type finite_low(Vec8<bf16_t>::type x) {
+  typedef uint16_t U8 __attribute__((ext_vector_type(8)));
+  return __builtin_bit_cast(Vec8<bf16_t>::type, __builtin_elementwise_min(__builtin_bit_cast(U8, x), (U8)0xff7f));
+}
+
 // The workgroup's 256 threads load two [32 rows][32 channels] tiles (rows `pos0 ..` of tensors
 // a and b at (row i, head h)): thread t takes 8 channels of one row of one tile.
 template <typename T> struct TilePiece {
@@ -161,7 +167,7 @@ __global__ __launch_bounds__(256, (BwdCfg<T, VEC>::kMinWaves)) void attn_bwd_dq_
   // idle four fifths of the time, instead of being converted and added on the vector ALU:
   //   Bias2  S^T += E * B2, B2 the block's [key][query] values as they lie in LDS for this
   //          lane's query (B operand: slots <-> keys), E the 0/1 matrix that sends key j to
-  //          the accumulator row that stands for it (row m <-> key perm_row(m));
+  //          the accumulator row that stands for it (row m <-> key perm_row(m)), -inf as the lowest finite value;
   //   Bias1  S^T += b * 1^T: Bias1 of the row's key in K slot 0 of one more product, against
   //          a B operand with 1 in that slot (0 without a Bias1).  Products with 1 are exact.
   constexpr bool MMB = sizeof(T) == 2;
@@ -219,7 +225,10 @@ __global__ __launch_bounds__(256, (BwdCfg<T, VEC>::kMinWaves)) void attn_bwd_dq_
   auto park = [&](int buf) {
     piece.park(rm[buf], tr + (TURN ? 0 : buf * 32 * kTP), TURN ? 0 : 1, tid);
 #pragma unroll
-    for (int j = 0; j < 2; ++j) store8<T>(&b2s[buf][(64 * j + (tid >> 2)) * kTP + b2col], b2n[j]);
+    for (int j = 0; j < 2; ++j) {
+      if constexpr (MMB) b2n[j] = finite_low(b2n[j]);
+      store8<T>(&b2s[buf][(64 * j + (tid >> 2)) * kTP + b2col], b2n[j]);
+    }
   };
   auto fetch_bias = [&](int key0) {
     if (MMB) {
@@ -267,7 +276,7 @@ __global__ __launch_bounds__(256, (BwdCfg<T, VEC>::kMinWaves)) void attn_bwd_dq_
         const f32x8 b1f = to_f32(b1n[ks]);
         const f32x8 b2f = to_f32(load8<T>(&b2s[buf][(32 * wave + ln) * kTP + 16 * ks + 8 * g]));
 #pragma unroll
-        for (int t = 0; t < 8; ++t) st[8 * ks + t] = b1f[t] * b1on + b2f[t];
+        for (int t = 0; t < 8; ++t) st[8 * ks + t] = (b1on != 0.0f ? b1f[t] : 0.0f) + b2f[t];   // (not b1f * b1on: -inf)
       }
       fetch_bias(next_key0);
 #pragma unroll
@@ -506,12 +515,6 @@ struct TurnedAt {
     return __builtin_bit_cast(bf16x8, (v8s)__builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7));
   }
 };
-
-// -inf as the lowest finite value, so that a product with 0 is 0 (a NaN's row is NaN throughout by its log-sum-exp).
-__device__ __forceinline__ Vec8<bf16_t>::type finite_low(Vec8<bf16_t>::type x) {
-  typedef uint16_t U8 __attribute__((ext_vector_type(8)));
-  return __builtin_bit_cast(Vec8<bf16_t>::type, __builtin_elementwise_min(__builtin_bit_cast(U8, x), (U8)0xff7f));
-}
 
 // dQ, dK and dV in one pass, 16-bit, rows of at most 32 NW NBK positions: a workgroup takes one (row, head), a wave NBK blocks of
 // 32 keys (every NW-th), and all walk over the query blocks.  Logits and dP are formed once instead of once for dQ and
@@ -853,7 +856,7 @@ __global__ __launch_bounds__(256, (BwdCfg<T, VEC>::kMinWaves)) void attn_bwd_db2
       for (int ks = 0; ks < 2; ++ks) {
         const f32x8 b1f = to_f32(b1c[ks]);
 #pragma unroll
-        for (int t = 0; t < 8; ++t) st[8 * ks + t] = b1f[t] * b1on + b2f[ks][t];
+        for (int t = 0; t < 8; ++t) st[8 * ks + t] = (b1on != 0.0f ? b1f[t] : 0.0f) + b2f[ks][t];   // (not b1f * b1on: -inf)
       }
     }
 #pragma unroll

@@ -171,9 +171,8 @@ def test_sliced_dbias2_equals_one_slice(dtype, N, S, H):
 def test_whole_rows_at_a_time(N, S, H):
     """16-bit rows of every class of the backward that takes a (row, head) at a time and of its neighbours that do not:
     a vector more and less than a block, the last keys' shifted Bias2 vectors, dQ over one to eight waves.  One row has
-    a Bias1 of -inf for half of its keys, and Bias2 has -inf at one key for one query; the weight there is 0 (the
-    kernels that take dQ by itself add biases as products with 0 and 1, so they get -1e9)."""
-    low = -math.inf if 8 <= S <= 768 and (S <= 384 or N * H >= 192) else -1e9
+    a Bias1 of -inf for half of its keys, and Bias2 has -inf at one key for one query; the weight there is 0."""
+    low = -math.inf
     q, k, v, b1, b2, do = _operands(1, N, S, H, torch.bfloat16, seed=N + S, n_masked=min(3, S - 2))
     b1[:, 0, ..., S // 2:] = low
     b2[..., S - 2, 1] = low
@@ -183,3 +182,19 @@ def test_whole_rows_at_a_time(N, S, H):
     for name, g, w in zip(("dQ", "dK", "dV"), (dq, dk, dv), want[1:4]):
         assert rel_err(g[:, few], w) <= tol(torch.bfloat16), name
     assert (dk[:, 0, S // 2:] == 0).all() and (dv[:, 0, S // 2:] == 0).all()
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("with_bias1", [True, False])
+@pytest.mark.parametrize("N,S,H", [(3, 40, 2), (2, 7, 1), (3, 200, 1), (2, 385, 1), (2, 770, 1)])
+def test_bias2_of_minus_infinity_has_weight_zero(dtype, with_bias1, N, S, H):
+    """In every kernel of the backward, as in the forward: finite gradients, those of the torch path, and none for that logit."""
+    q, k, v, b1, b2, do = _operands(1, N, S, H, dtype, seed=S)
+    b2[..., S - 2, 1] = -math.inf
+    b2[..., 0, S // 2:] = -math.inf
+    want = _autograd_reference(q, k, v, b1, b2, do)
+    qc, kc, vc, b2c = (t.cuda().requires_grad_(True) for t in (q, k, v, b2))
+    P.TriAttentionFunction.apply(qc, kc, vc, b1.cuda() if with_bias1 else None, b2c).backward(do.cuda())
+    for name, g, w in zip(("dQ", "dK", "dV", "dBias2"), (qc.grad, kc.grad, vc.grad, b2c.grad), want[1:]):
+        assert torch.isfinite(g).all() and rel_err(g, w) <= tol(dtype), name
+    assert (b2c.grad[..., S - 2, 1] == 0).all() and (b2c.grad[..., 0, S // 2:] == 0).all()
