@@ -733,13 +733,29 @@ __global__ __launch_bounds__(NW * 64, NBK == 1 ? 3 : 2) void attn_bwd_row_kernel
 }
 
 // Whether a workgroup takes whole rows (attn_bwd_row_kernel): 16-bit rows whose accumulators for dK and dV fit the registers
-// of eight waves, at least one vector long.  Above 384 positions a workgroup is eight waves that fill a compute unit: from
-// 192 workgroups on.  Both sides, us for the operator forward and backward, 4 heads: 384 rows of 384, 390 | 355; 256 of 65, 95 | 88;
-// 256 of 264, 202 | 180; 48 of 500, 131 | 123; 64 of 768, 267 | 233; 256 of 520, 538 | 517; 768 of 768, 3054 | 2735; and below the
-// line 20 of 520, 93 | 110; 20 of 768, 112 | 158.
+// of eight waves, at least one vector long, and enough of them.  A (row, head) is one workgroup, whatever its length: what
+// these cost is rounds of the machine - 512 of four waves with two or three blocks each, 256 of eight waves -, where the kernels
+// of 128 queries or keys a workgroup, two to six of them for a pair, fill it sooner.  So as many pairs are asked for, round by round, as
+// give the others a round more (256 workgroups; three to a pair: from 171 pairs on, from 342).
+// us for dQ, dK and dV, by themselves | so, 4 heads, (rows, positions):
+//   one block a wave: (1, 128) 11.5 | 8.9, (256, 128) 31.8 | 25.0
+//   two: (32, 136) 13.5 | 15.2, (32, 256) 17.4 | 20.7, (34, 136) 17.7 | 15.2, (36, 200) 20.2 | 19.3, (36, 256) 22.7 | 20.9, (112, 200) 38.5 | 29.0,
+//     (130, 200) 43.0 | 45.0, (160, 200) 45.5 | 44.8
+//   three, 8 divides the positions: (1, 384) 20.5 | 38.8, (48, 384) 40 | 46, (84, 264) 41 | 45, (84, 384) 57 | 59, (88, 264) 48.4 | 45.1, (88, 384)
+//     63.3 | 59.9, (130, 384) 86 | 100, (160, 384) 104 | 100, (192, 384) 115 | 101; otherwise: (40, 300) 31.8 | 35.7, (47, 300) 39.9 | 36.7, (72, 300) 54 | 49,
+//     (130, 300) 81.5 | 84.8, (144, 300) 86 | 84
+//   eight waves: (48, 400) 45 | 41, (80, 400) 69 | 78, (96, 400) 81 | 79, (48, 512) 57 | 48, (96, 512) 103 | 93, (48, 520) 70 | 70, (80, 520) 108 | 136, (96, 520)
+//     128 | 137, (112, 520) 141 | 138, (160, 520) 203 | 205, (64, 640) 98 | 86, (96, 640) 153 | 166, (112, 640) 177 | 167, (48, 768) 115 | 99, (80, 768) 184 | 195,
+//     (96, 768) 217 | 196
+// The operator forward and backward: 384 rows of 384, 390 | 355; 768 of 768, 3054 | 2735.
 template <typename T>
 bool rows_at_once(const BwdParams& p) {
-  return sizeof(T) == 2 && p.s >= 8 && p.s <= 768 && (p.s <= 384 || (int64_t)p.heads * p.n_rows >= 192);
+  if (sizeof(T) != 2 || p.s < 8 || p.s > 768) return false;
+  if (p.s <= 128) return true;
+  const int64_t pairs = (int64_t)p.heads * p.n_rows;
+  if (p.s <= 256) return pairs > 128;
+  if (p.s <= 384) return pairs >= (p.s % 8 == 0 ? 342 : 171) + 290 * ((pairs - 1) / 512);
+  return pairs >= (p.s > 512 && p.s <= 640 ? 216 : 192) * ((pairs + 255) / 256);
 }
 
 // dBias2's tiles: 16-bit rows as above (padded to 80 bytes a third of the LDS cycles were conflicts: the operator at 768 rows of 768

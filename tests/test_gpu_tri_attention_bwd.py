@@ -167,21 +167,23 @@ def test_sliced_dbias2_equals_one_slice(dtype, N, S, H):
 
 @pytest.mark.parametrize("N,S,H", [(2, 7, 1), (3, 8, 1), (5, 9, 3), (3, 31, 2), (2, 32, 4), (9, 33, 1), (2, 127, 2), (2, 128, 1), (2, 129, 3),
                                    (3, 255, 1), (2, 256, 2), (2, 257, 1), (2, 383, 2), (3, 384, 1), (64, 385, 3), (47, 391, 4),
-                                   (48, 511, 4), (64, 512, 3), (48, 513, 4), (192, 767, 1), (48, 768, 4), (48, 769, 4)])
+                                   (48, 511, 4), (64, 512, 3), (48, 513, 4), (192, 767, 1), (48, 768, 4), (48, 769, 4),
+                                   (33, 129, 4), (43, 255, 3), (65, 256, 2), (32, 256, 4), (48, 257, 4), (86, 264, 4), (48, 383, 4), (86, 384, 4),
+                                   (129, 384, 4), (54, 513, 4), (54, 640, 4)])
 def test_whole_rows_at_a_time(N, S, H):
-    """16-bit rows of every class of the backward that takes a (row, head) at a time and of its neighbours that do not:
-    a vector more and less than a block, the last keys' shifted Bias2 vectors, dQ over one to eight waves.  One row has
-    a Bias1 of -inf for half of its keys, and Bias2 has -inf at one key for one query; the weight there is 0."""
+    """16-bit rows of every class of the backward that takes a (row, head) at a time and of its neighbours that do not, in length and in
+    number: a vector more and less than a block, the last keys' shifted Bias2 vectors, dQ over one to eight waves.  One row has
+    a Bias1 of -inf for half of its keys, and Bias2 has -inf at one key for one query; the weight there is 0.  The reference is
+    autograd in fp32 on the same device."""
     low = -math.inf
     q, k, v, b1, b2, do = _operands(1, N, S, H, torch.bfloat16, seed=N + S, n_masked=min(3, S - 2))
     b1[:, 0, ..., S // 2:] = low
     b2[..., S - 2, 1] = low
     _, dq, dk, dv, db2 = _product(q, k, v, b1, b2, do)
-    few = slice(0, min(N, 4))
-    want = _autograd_reference(q[:, few], k[:, few], v[:, few], b1[:, few], b2, do[:, few])
-    for name, g, w in zip(("dQ", "dK", "dV"), (dq, dk, dv), want[1:4]):
-        assert rel_err(g[:, few], w) <= tol(torch.bfloat16), name
-    assert (dk[:, 0, S // 2:] == 0).all() and (dv[:, 0, S // 2:] == 0).all()
+    want = _autograd_reference(*(t.cuda() for t in (q, k, v, b1, b2, do)))
+    for name, g, w in zip(("dQ", "dK", "dV", "dBias2"), (dq, dk, dv, db2), want[1:]):
+        assert torch.isfinite(g).all() and rel_err(g, w) <= tol(torch.bfloat16), name
+    assert (dk[:, 0, S // 2:] == 0).all() and (dv[:, 0, S // 2:] == 0).all() and (db2[..., S - 2, 1] == 0).all()
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
