@@ -462,6 +462,14 @@ static bool carry_ok(const ptx_single_stage* carry, int dtype) {
   return !st || st->kind == ptx::kStageNone || (st->bits16 != 0) == (dtype == PTX_BF16);
 }
 
+// A launch over no rows still runs the stage that it was to carry.
+static int only_carried(const char* what, const ptx_single_stage* carry, int dtype, void* stream) {
+  PTX_REQUIRE(carry_ok(carry, dtype), PTX_ERR_BAD_ARG, "%s: the carried stage must be of the pair tensor's type", what);
+  if (!carry) return PTX_OK;
+  ptx::single_stage_run((const ptx::SingleStage*)carry, (hipStream_t)stream);
+  return after_launch(what);
+}
+
 PTX_API int ptx_trimul_project_packed(const void* z, const void* mask, const void* ln_w, const void* ln_b,
                                       const void* packed, void* a, void* b, int n, int c_z, int c_hidden,
                                       int k_pitch, int incoming, float eps, int dtype,
@@ -473,7 +481,7 @@ PTX_API int ptx_trimul_project_packed(const void* z, const void* mask, const voi
   PTX_REQUIRE(k_pitch == ptx_key_pitch(n), PTX_ERR_BAD_ARG, "trimul_project_packed: k_pitch=%d, expected %d", k_pitch,
               ptx_key_pitch(n));
   PTX_REQUIRE(n <= 8192, PTX_ERR_UNSUPPORTED, "trimul_project_packed: n=%d too large (8192 at most)", n);
-  if (n == 0) return PTX_OK;
+  if (n == 0) return only_carried("trimul_project_packed", carry, dtype, stream);
   PTX_REQUIRE(z && packed && a && b, PTX_ERR_BAD_ARG, "trimul_project_packed: null pointer");
   PTX_REQUIRE(aligned16(z) && aligned16(packed) && aligned16(a) && aligned16(b) && (!ln_w || aligned16(ln_w)) &&
                   (!ln_b || aligned16(ln_b)),
@@ -495,7 +503,7 @@ PTX_API int ptx_trimul_output_packed(const void* x, int ldx, const void* z, cons
               "trimul_output_packed: %s (got c_z=%d c_hidden=%d)", kWidthMsg, c_z, c_hidden);
   PTX_REQUIRE(n < 32768, PTX_ERR_UNSUPPORTED, "trimul_output_packed: n=%d too large", n);
   PTX_REQUIRE(ldx >= n && ldx % 8 == 0, PTX_ERR_BAD_ARG, "trimul_output_packed: ldx=%d (a multiple of 8, >= n=%d)", ldx, n);
-  if (n == 0) return PTX_OK;
+  if (n == 0) return only_carried("trimul_output_packed", carry, dtype, stream);
   PTX_REQUIRE(x && z && packed && out, PTX_ERR_BAD_ARG, "trimul_output_packed: null pointer");
   PTX_REQUIRE(aligned16(x) && aligned16(out) && aligned16(z) && aligned16(packed) && (!ln_out_w || aligned16(ln_out_w)) &&
                   (!ln_out_b || aligned16(ln_out_b)) && (!ln_in_w || aligned16(ln_in_w)) && (!ln_in_b || aligned16(ln_in_b)),
@@ -538,7 +546,7 @@ PTX_API int ptx_triattn_project_packed(const void* z, const void* ln_w, const vo
   PTX_REQUIRE(key_pitch == ptx_key_pitch(n), PTX_ERR_BAD_ARG, "triattn_project_packed: key_pitch=%d, expected %d",
               key_pitch, ptx_key_pitch(n));
   PTX_REQUIRE(n <= 8192, PTX_ERR_UNSUPPORTED, "triattn_project_packed: n=%d too large (8192 at most)", n);
-  if (n == 0) return PTX_OK;
+  if (n == 0) return only_carried("triattn_project_packed", carry, dtype, stream);
   const bool late = ptx::pp_late_gate(c_in, heads, dtype != PTX_F32);
   PTX_REQUIRE(z && packed && q && k && vt && tri_bias && (g || late), PTX_ERR_BAD_ARG,
               "triattn_project_packed: null pointer");
@@ -561,7 +569,7 @@ PTX_API int ptx_triattn_output_packed(const void* o, const void* z, const void* 
   PTX_REQUIRE(heads > 0 && heads <= 8 && pair_width_ok(c_in, heads * 32, dtype), PTX_ERR_UNSUPPORTED,
               "triattn_output_packed: %s (got c_in=%d heads=%d)", kWidthMsg, c_in, heads);
   PTX_REQUIRE(n < 32768, PTX_ERR_UNSUPPORTED, "triattn_output_packed: n=%d too large", n);
-  if (n == 0) return PTX_OK;
+  if (n == 0) return only_carried("triattn_output_packed", carry, dtype, stream);
   PTX_REQUIRE(o && z && packed && out, PTX_ERR_BAD_ARG, "triattn_output_packed: null pointer");
   PTX_REQUIRE(aligned16(o) && aligned16(z) && aligned16(packed) && aligned16(out) && (!ln_w || aligned16(ln_w)) &&
                   (!ln_b || aligned16(ln_b)),
@@ -590,7 +598,7 @@ PTX_API int ptx_trimul_output_trimul_project(const void* x, int ldx, const void*
   PTX_REQUIRE(k_pitch == ptx_key_pitch(n), PTX_ERR_BAD_ARG, "trimul_output_trimul_project: k_pitch=%d, expected %d", k_pitch, ptx_key_pitch(n));
   PTX_REQUIRE(n <= 8192, PTX_ERR_UNSUPPORTED, "trimul_output_trimul_project: n=%d too large (8192 at most)", n);
   PTX_REQUIRE(ldx >= n && ldx % 8 == 0, PTX_ERR_BAD_ARG, "trimul_output_trimul_project: ldx=%d (a multiple of 8, >= n=%d)", ldx, n);
-  if (n == 0) return PTX_OK;
+  if (n == 0) return only_carried("trimul_output_trimul_project", carry, dtype, stream);
   PTX_REQUIRE(x && z && packed && out && next_packed && a && b, PTX_ERR_BAD_ARG, "trimul_output_trimul_project: null pointer");
   PTX_REQUIRE(aligned16(x) && aligned16(out) && aligned16(z) && aligned16(packed) && (!ln_out_w || aligned16(ln_out_w)) &&
                   (!ln_out_b || aligned16(ln_out_b)) && (!ln_in_w || aligned16(ln_in_w)) && (!ln_in_b || aligned16(ln_in_b)) &&
@@ -621,7 +629,7 @@ PTX_API int ptx_trimul_output_triattn_project(const void* x, int ldx, const void
               ptx_key_pitch(n));
   PTX_REQUIRE(n <= 8192, PTX_ERR_UNSUPPORTED, "trimul_output_triattn_project: n=%d too large (8192 at most)", n);
   PTX_REQUIRE(ldx >= n && ldx % 8 == 0, PTX_ERR_BAD_ARG, "trimul_output_triattn_project: ldx=%d (a multiple of 8, >= n=%d)", ldx, n);
-  if (n == 0) return PTX_OK;
+  if (n == 0) return only_carried("trimul_output_triattn_project", carry, dtype, stream);
   PTX_REQUIRE(x && z && packed && out && att_packed && q && k && vt && tri_bias, PTX_ERR_BAD_ARG, "trimul_output_triattn_project: null pointer");
   PTX_REQUIRE(aligned16(x) && aligned16(out) && aligned16(z) && aligned16(packed) && (!ln_out_w || aligned16(ln_out_w)) &&
                   (!ln_out_b || aligned16(ln_out_b)) && (!ln_in_w || aligned16(ln_in_w)) && (!ln_in_b || aligned16(ln_in_b)) &&
@@ -650,7 +658,7 @@ PTX_API int ptx_triattn_output_triattn_project(const void* o, const void* z, con
   PTX_REQUIRE(key_pitch == ptx_key_pitch(n), PTX_ERR_BAD_ARG, "triattn_output_triattn_project: key_pitch=%d, expected %d", key_pitch,
               ptx_key_pitch(n));
   PTX_REQUIRE(n <= 8192, PTX_ERR_UNSUPPORTED, "triattn_output_triattn_project: n=%d too large (8192 at most)", n);
-  if (n == 0) return PTX_OK;
+  if (n == 0) return only_carried("triattn_output_triattn_project", carry, dtype, stream);
   PTX_REQUIRE(o && z && packed && out && next_packed && q && k && vt && tri_bias, PTX_ERR_BAD_ARG, "triattn_output_triattn_project: null pointer");
   PTX_REQUIRE(o != q && o != k && o != vt, PTX_ERR_BAD_ARG, "triattn_output_triattn_project: o must not be one of the outputs");
   PTX_REQUIRE(aligned16(o) && aligned16(z) && aligned16(packed) && aligned16(out) && (!ln_w || aligned16(ln_w)) && (!ln_b || aligned16(ln_b)) &&

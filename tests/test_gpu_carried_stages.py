@@ -89,3 +89,22 @@ def test_attention_core(mode, n, carries, masked):
     _both(lambda stage, st: lib.ptx_triattn_fwd_carry(q.data_ptr(), k.data_ptr(), vt.data_ptr(), None, tb.data_ptr(),
                                                       None if mask is None else mask.data_ptr(), o.data_ptr(), n, 4, 32, lib.ptx_key_pitch(n), 0, 1e9,
                                                       code, stage, st), mode, [o])
+
+
+@pytest.mark.parametrize("mode", ["bf16", "amp"])
+def test_no_rows(mode):
+    """Every launch that takes a stage along runs it where it has no rows of its own."""
+    lib = _lib.load()
+    code, _ = MODES[mode]
+    calls = [lambda s, st: lib.ptx_trimul_project_packed(*[None] * 7, 0, 128, 128, 0, 0, 1e-5, code, s, st),
+             lambda s, st: lib.ptx_trimul_contract_carry(None, None, None, 0, 0, 128, 0, code, s, st),
+             lambda s, st: lib.ptx_trimul_output_packed(None, 0, *[None] * 7, 0, 128, 128, 1, 1e-5, code, s, st),
+             lambda s, st: lib.ptx_triattn_project_packed(*[None] * 9, 0, 128, 4, 0, 0, 1e-5, code, s, st),
+             lambda s, st: lib.ptx_triattn_fwd_carry(*[None] * 7, 0, 4, 32, 0, 0, 1e9, code, s, st),
+             lambda s, st: lib.ptx_triattn_output_packed(*[None] * 6, 0, 128, 4, 0, 1, 1e-5, code, s, st),
+             lambda s, st: lib.ptx_trimul_output_trimul_project(None, 0, *[None] * 13, 0, 128, 128, 0, 1e-5, code, s, st),
+             lambda s, st: lib.ptx_trimul_output_triattn_project(None, 0, *[None] * 14, 0, 128, 128, 4, 0, 1e-5, code, s, st),
+             lambda s, st: lib.ptx_triattn_output_triattn_project(*[None] * 13, 0, 128, 4, 0, 1e-5, code, s, st),
+             lambda s, st: lib.ptx_triattn_output_transition_carry(*[None] * 8, 0, 128, 4, 1, 2, 1e-5, 1e-5, *[None] * 4, 0, 1, 1e-5, code, s, st)]
+    for call in calls:
+        _both(call, mode, [])
