@@ -110,7 +110,7 @@ struct ProjInParams {
 // The output columns of a triangle multiplication's projection: a, b[c][i][k] = mask * sigmoid(gate) * projection in the
 // contraction's fragment order, from the normalised rows in LDS of a patch of 4 * RBW outer indices i x 8 inner indices
 // k, which makes a row block's 32 values of one channel 64 contiguous bytes.
-template <typename T, int KS, int RBW>
+template <typename T, int KS, int RBW, bool APART = false>
 struct MulColumns {
   typedef typename Vec8<T>::type V8;
   typedef typename VecE<T>::type VE_t;
@@ -190,10 +190,10 @@ struct MulColumns {
           mma32(acc[0], xv, w[0][kk]);   // lane <-> channel, register <-> row
           mma32(acc[1], xv, w[1][kk]);
         }
-        // (the products stay together: mixed with the staging below they take 138 registers from two row blocks of 16-bit rows and
+        // (APART: the products stay together; mixed with the staging below they take 138 registers from two row blocks of 16-bit rows and
         // leave three waves per SIMD instead of four.  us for both multiplications of bf16 rows, so / as here: 300 tokens 137 / 135, 352
         // 167 / 163, 387 218 / 214, 440 256 / 251)
-        if constexpr (sizeof(T) == 2 && RBW == 2) __builtin_amdgcn_sched_barrier(0);
+        if constexpr (APART) __builtin_amdgcn_sched_barrier(0);
         if (rb == RBW - 1 && c + 1 < CHW && c + 1 < c_end) load_w(p, ch + 1, lane);
         float vals[16];
 #pragma unroll
@@ -223,7 +223,7 @@ struct MulColumns {
 // Tiles in the order of the memory rows they read.
 template <typename T, typename TZ, int KS, int RBW>
 __global__ __launch_bounds__(kPpWaves * 64, (kPpMinWaves<T, KS>)) void pp_trimul_in_kernel(ProjInParams p, SingleStage carry, unsigned carried) {
-  typedef MulColumns<T, KS, RBW> Columns;
+  typedef MulColumns<T, KS, RBW, sizeof(T) == 2 && sizeof(TZ) == 2 && RBW == 2> Columns;
   constexpr int kFrag = RBW * FragLds<T, KS>::ROWBLOCK;
   __shared__ __attribute__((aligned(16))) char smem[cmax(kFrag + Columns::kStage, kStageLds)];
   PTX_CARRIED_STAGE();
@@ -235,8 +235,8 @@ __global__ __launch_bounds__(kPpWaves * 64, (kPpMinWaves<T, KS>)) void pp_trimul
     Columns::put_zeros(p, block - p.work, wave, lane);
     return;
   }
-  // (slices: of one row block only, see in_slices)
-  constexpr bool kSliced = RBW == 1;
+  // (slices: of one row block only, see in_slices; fp32 rows keep their bounds, which cost them no wave: 440 tokens 351 us with, 356 without)
+  constexpr bool kSliced = RBW == 1 || sizeof(TZ) == 4;
   // back to front behind a kernel that wrote the pair tensor front to back (the tail is what the memory-side cache still holds)
   const uint32_t tiles = p.tiles, slice = kSliced ? (block >= tiles) + (block >= 2 * tiles) + (block >= 3 * tiles) : 0u;
   const uint32_t bx = xcd_run(block - slice * tiles, tiles), tile = p.backward ? tiles - 1 - bx : bx;
