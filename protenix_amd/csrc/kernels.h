@@ -122,6 +122,8 @@ void single_stage_attention(SingleStage* s, const void* q, const void* k, const 
                             float scale, bool bits16);
 int single_stage_run(const SingleStage* s, hipStream_t stream);
 
+// x[c][i][j] = sum_k a[c][i][k] * b[c][j][k] for `batch` independent products;
+// a, b rows have pitch k_pitch (a multiple of 64, >= n), x is [batch][n][ldx].
 // carry: null, or a stage of the single track that the launch's first workgroups run (it must not depend on the launch), where
 // nt_gemm_carries(); elsewhere the stage is launched in front.
 bool nt_gemm_carries(int n, bool bits16);
@@ -191,11 +193,6 @@ int pp_triattn_out_triattn_in(const void* o, const void* z, const void* ln_w, co
                               const void* next_ln_w, const void* next_ln_b, const void* next_packed, void* q, void* k, void* vt,
                               void* tri_bias, int n, int c_z, int heads, int key_pitch, float eps, const SingleStage* carry,
                               hipStream_t stream);
-
-
-// x[c][i][j] = sum_k a[c][i][k] * b[c][j][k] for `batch` independent products;
-// a, b rows have pitch k_pitch (a multiple of 64, >= n), x is [batch][n][ldx].
-
 
 // Flash-style triangle attention core (see triattn.hip).
 template <typename T>

@@ -56,7 +56,6 @@ struct AttnAux {
   int64_t lh, li, lj;     // element strides of lse: head, row, query
   int row0, row_end;      // rows row0 .. row_end-1 are this launch's (a launch may cover a range)
   int n_keys;             // keys 0 .. n_keys-1 take part (n_keys <= n; the rest count as masked)
-  int q_begin, q_end;     // queries q_begin .. q_end-1 of every row are this launch's (q_begin % 32 == 0)
 };
 
 // Rows of the pair tensor handled by one wave: R = 1 or 2, chosen per launch (triattn_fwd_ex).
@@ -73,7 +72,8 @@ struct AttnAux {
 // partial key tile takes the same paths as the others with the logits of the keys beyond
 // n_keys set to -inf (kMaskTail; kMaskNone where the keys fill whole tiles).
 enum { kMaskNone = 0, kMaskTail = 1, kMaskGiven = 2 };
-// TS: the launch's first `carried` workgroups run a stage of the single track on operands of that type (void: none).
+// TS: the launch's first `carried` workgroups run a stage of the single track on operands of that type (void: none; with one three waves
+// per SIMD instead of four).
 // STD: K and V as the operator's callers have them, [row][position][head][32] (addressed like q), and q not yet multiplied by
 // log2 e: K rows find their fragments by the lanes' addresses, V tiles lie row-major in LDS and are turned when they
 // are read.  (Repacked by kernels of their own, q, K and V cost 44 us at 384 rows of 384 positions and 4 heads, next to 86 of
@@ -112,7 +112,7 @@ __global__ __launch_bounds__((NWQ * 64), (sizeof(T) == 2 ? (!std::is_void<TS>::v
   const int i0 = ax.row0 + (int)((item / n_qtiles) % n_rowgroups) * R;   // first of this workgroup's R rows
   const int h = (int)(item / ((int64_t)n_qtiles * n_rowgroups));
 
-  const int q0 = ax.q_begin + (qt * NWQ + wave) * 32;   // first query of this wave
+  const int q0 = (qt * NWQ + wave) * 32;   // first query of this wave
   const int key_tiles = key_pitch >> 6;
   const int q_blocks = (n + 31) >> 5;
   const int nk = ax.n_keys;
@@ -127,7 +127,7 @@ __global__ __launch_bounds__((NWQ * 64), (sizeof(T) == 2 ? (!std::is_void<TS>::v
   // Lanes whose query lies beyond n compute on whatever the bias workspace holds there; they
   // store nothing, and they are kept out of the wave-wide decisions below so that the path a
   // wave takes (and with it the rounding of its valid queries) never depends on that content.
-  const bool q_ok = q0 + ln < ax.q_end;
+  const bool q_ok = q0 + ln < n;
   // (as a lane mask: wave-wide decisions are ballots of the condition alone, combined with this
   // mask on the scalar unit)
   const uint64_t q_ok_mask = __builtin_amdgcn_ballot_w64(q_ok);
@@ -560,10 +560,10 @@ __global__ __launch_bounds__((NWQ * 64), (sizeof(T) == 2 ? (!std::is_void<TS>::v
   for (int r = 0; r < R; ++r) {
     const float l_tot = l_run[r] + swap32(l_run[r]);
     const float inv = fast_rcp(l_tot);
-    if (ax.lse && g == 0 && q0 + ln < ax.q_end && i0 + r < ax.row_end)
+    if (ax.lse && g == 0 && q0 + ln < n && i0 + r < ax.row_end)
       ax.lse[h * ax.lh + (int64_t)(i0 + r) * ax.li + (int64_t)qi_again * ax.lj] =
           m_run[r] * kLog2e + __builtin_amdgcn_logf(l_tot);   // v_log_f32 is log2
-    if (q0 + ln < ax.q_end && i0 + r < ax.row_end) {
+    if (q0 + ln < n && i0 + r < ax.row_end) {
 #pragma unroll
       for (int c = 0; c < 4; ++c) {
         f32x4 ov;
@@ -613,7 +613,7 @@ int triattn_fwd_ex(const T* q, const T* k, const T* vt, const T* g, const T* tri
     carry = nullptr;
   }
   if (empty) return 0;
-  AttnAux ax = {sh, si, sj, n_rows, mask_is_bias, lse, lh, li, lj, row_begin, row_begin + row_count, n_keys, 0, n};
+  AttnAux ax = {sh, si, sj, n_rows, mask_is_bias, lse, lh, li, lj, row_begin, row_begin + row_count, n_keys};
   // Two rows per wave (16-bit, no mask): the two rows share the query block and with it the bias tile - one load
   // and one conversion per logit for both, half the bias stream from the L2 - at 128 registers, so that four waves
   // still share a SIMD (with a mask the kernel needs 160 and loses a wave).  Below 352 tokens the pairs of rows leave too few
