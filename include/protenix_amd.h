@@ -237,7 +237,7 @@ PTX_API int ptx_layernorm_bwd_static(const void* dout, const void* x, const floa
  *   z [n][n][c_z], mask [n][n] in `dtype` or NULL (= ones),
  *   w_* [c_hidden][c_z]; a, b: workspaces of ptx_trimul_operand_elems(n, c_hidden)
  *   elements each, written in the contraction's operand order (K between n and
- *   k_pitch is written as zeros, rows beyond n stay unwritten);
+ *   k_pitch is written as zeros, rows beyond n hold nothing that counts);
  *   k_pitch = ptx_key_pitch(n).  Widths: c_z = 64 or 128 with c_hidden = 128, or
  *   (PTX_BF16, PTX_MIXED) c_z = c_hidden = 256.
  */

@@ -5,7 +5,7 @@
 //   P = 2^(S log2 e - M),  S = Q K^T + Bias1 + Bias2,  Delta = rowsum(O * dO),
 //   dS = P * (dO V^T - Delta)
 // it produces  dV = P^T dO,  dK = dS^T Q,  dQ = dS K,  dBias2[h] = sum over rows of dS.
-// Two kernels where a workgroup can take a whole row (rows_at_once) - dQ, dK and dV, and dBias2 -, else three: dQ, dK / dV, dBias2.
+// Two kernels where a workgroup takes a whole row (rows_at_once) - dQ, dK and dV, and dBias2 -, else three: dQ, dK / dV, dBias2.
 // The first forms Delta (the reference's preprocess kernel) and leaves it for the others; P is recomputed, the
 // logits are never stored.  One wave owns a 32 x 32 block of (query, key) pairs and walks over
 // the other index; every product runs on MFMA with fp32 accumulation (conventions of
@@ -525,7 +525,8 @@ struct TurnedAt {
 // Bound by latency: of a wave's time 28 % issues, 52 % waits for LDS and barriers (two waves per SIMD: the accumulators of all its
 // keys are registers); of a SIMD's time 36 % is vector work, 24 % matrix work, and 30 % of the compute unit's is LDS.  Leaving out the
 // exponentials, the exchange of dQ or the spread of Bias2's rows, or three waves of one block each, changes it by 0 - 3 %.
-// 384 rows of 384 positions, 4 heads: dQ 109 us and dK / dV 126 before, 195 now.
+// 384 rows of 384 positions, 4 heads: dQ 109 us and dK / dV 126 before, 195 now.  The forms with three blocks a wave are at the limit of 256
+// registers and spill: ten (44 bytes of scratch a lane) with four waves, eight with eight; with two blocks 218 and none, with one 164.
 template <int NW, int NBK>
 __global__ __launch_bounds__(NW * 64, NBK == 1 ? 3 : 2) void attn_bwd_row_kernel(BwdParams p) {
   typedef bf16_t T;

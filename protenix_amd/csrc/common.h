@@ -173,7 +173,7 @@ struct RowMap {
 // and K in steps of 16; one (row block, K step) fragment is stored in MFMA
 // operand order, 64 lanes x 8 elements = 512 contiguous elements: lane
 // 32*g + r holds K = 16*ks + 8*g .. +7 of row 32*rb + r.  A channel has
-// ceil(n/32) row blocks (rows beyond n are never written) and k_pitch/16 K steps
+// ceil(n/32) row blocks (rows beyond n hold nothing that counts) and k_pitch/16 K steps
 // (K between n and k_pitch is written as zeros: the contraction runs over it).
 // ---------------------------------------------------------------------------
 constexpr int kFragElems = 512;

@@ -341,7 +341,9 @@ struct ChannelTile {
 // bytes per product grow as the tile shrinks: 768 tokens by itself, 128 channels, tiles 64 x 64 / 128 x 128 / 128 x 256 / 192 x
 // 192 / 256 x 256 (the kernel above): 237 / 160 / 141 / 133 / 137 us.  Small tensors are chains of
 // latencies: 93 tokens 8.4 (above) -> 3.1 us, 128 tokens 8.9 -> 3.6, 200 tokens 12.8 -> 9.3.
-// TS: the launch's first `carried` workgroups run a stage of the single track on operands of that type (void: none).
+// TS: the launch's first `carried` workgroups run a stage of the single track on operands of that type (void: none).  The stage's
+// registers are the kernel's then: 64 x 64 tiles go from 36 and six waves per SIMD to 179 and two with an fp32 stage, 131 and three with a
+// 16-bit one, and the stage sets the launch's length (93 tokens 3.1 us without, 7 - 8 with).
 template <int RM, int RN, typename TS>
 __global__ __launch_bounds__(256) void nt_gemm_ring_kernel(const bf16_t* __restrict__ a, const bf16_t* __restrict__ b,
                                                            bf16_t* __restrict__ x, int n, int ldx, int k_pitch, int batch,

@@ -47,7 +47,9 @@ def _stream() -> int:
 # Optional per-kernel timing: while `kernel_timer` is a dict, every C-ABI call (those of the native host
 # path included) is bracketed by HIP events on the stream it is launched on and the pairs are
 # appended under the entry point's name; read them with kernel_times().  A stage of the single track
-# that rides on a pair kernel is part of that kernel's time and has no entry of its own.
+# that rides on a pair kernel is part of that kernel's time and has no entry of its own.  Launches are timed one by one: where
+# a stack would join an output stage with the projection behind it (below some 500 tokens, ptx_row_stages_joined), a timed call makes the two
+# launches instead, and what it reports there is theirs; the results are the same bits.
 kernel_timer: Optional[dict] = None
 
 
@@ -209,7 +211,9 @@ _mask_cache: list = []
 # hands every mask to the kernels as it is (tests compare the two).  From 352 tokens on, where the unmasked
 # kernel takes two rows per wave; below, the second launch costs what the first one saves (us per update, two launches
 # against the masked kernel: 106 = 106 at N = 320 with 20 padded tokens, 118 against 126 at 352, 170 against 190 at 416 with 50,
-# 189 against 200 at 448; 384 with 32, whose keys fill whole tiles either way: 134 against 135).
+# 189 against 200 at 448; no gain at 352 with 1 padded token and at 384 with 32, whose keys fill whole tiles either way: 134 against 135).
+# The two differ by the rounding of 16-bit probabilities (a relative 2e-3 of the update): the masked kernel moves the softmax reference to
+# the running maximum in a row's last tiles, the valid rows' does not.
 prefix_mask_enabled = True
 prefix_mask_min_n = 352
 
