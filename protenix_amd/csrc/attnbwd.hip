@@ -522,11 +522,14 @@ struct TurnedAt {
 // a block's dS goes through LDS once more and is turned on its way out, and the waves' dQ of a query block, each over its own
 // keys, are added through LDS in wave order.  Bias2 reaches the S accumulator on the matrix pipe, S += B2 * 1, from fragments
 // loaded along the queries' rows; Bias1 is the accumulator's initial value, and -inf for keys beyond s.
-// Bound by latency: of a wave's time 28 % issues, 52 % waits for LDS and barriers (two waves per SIMD: the accumulators of all its
-// keys are registers); of a SIMD's time 36 % is vector work, 24 % matrix work, and 30 % of the compute unit's is LDS.  Leaving out the
-// exponentials, the exchange of dQ or the spread of Bias2's rows, or three waves of one block each, changes it by 0 - 3 %.
-// 384 rows of 384 positions, 4 heads: dQ 109 us and dK / dV 126 before, 195 now.  The forms with three blocks a wave are at the limit of 256
-// registers and spill: ten (44 bytes of scratch a lane) with four waves, eight with eight; with two blocks 218 and none, with one 164.
+// At 384 rows of 384 positions and 4 heads (us per launch, parts left out in turn): 42 are the workgroups' beginnings and ends, K, V, dK and dV
+// at the memory's rate; of the 135 of the walk the products alone take 40, Bias2's loads 28, the operands out of LDS 24, the
+// statistics 11, the exponentials 7, dS' way through LDS 5: two waves per SIMD (the accumulators of all its keys are registers) hide
+// little of one under the other.  Hence: O and the log-sum-exp come in along the walk, where Delta is formed, and not ahead of it (O, dO
+// and 384 log-sum-exps first: 75 us of beginnings and ends); K and V are requested in one go; dK and dV leave as whole rows of 64
+// bytes through LDS (as pieces of 8 bytes from the accumulators 56); Q and dO fragments are read again for every block, since kept across
+// the blocks they spill.  203 us before, 177 with these; 109 + 126 in two kernels.  Tried without gain: V out of the caches instead of
+// registers, dQ's product a block behind, Bias2 laid out in fragments by a launch of its own (170 + 5 us).
 template <int NW, int NBK>
 __global__ __launch_bounds__(NW * 64, NBK == 1 ? 3 : 2) void attn_bwd_row_kernel(BwdParams p) {
   typedef bf16_t T;
@@ -536,7 +539,7 @@ __global__ __launch_bounds__(NW * 64, NBK == 1 ? 3 : 2) void attn_bwd_row_kernel
   static_assert(1024 * (int)sizeof(T) <= kExWave, "a wave's dS tile fits its place for dQ");
   __shared__ __attribute__((aligned(32))) T kt[KB][1024];      // K, row-major, read by the wave that owns the block
   __shared__ __attribute__((aligned(32))) T rm[2][2][1024];      // Q, dO of the step
-  __shared__ f32x8 stats[2][KB * 4];   // -log-sum-exp, -Delta
+  __shared__ f32x8 stats[2][2][4];   // -log-sum-exp, -Delta of the step's queries
   // two of them, for a step and the next: a wave's dS tile, later its partial dQ
   __shared__ __attribute__((aligned(32))) char ex[2][NW][kExWave];
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, ln = lane & 31, g = lane >> 5;
@@ -545,35 +548,28 @@ __global__ __launch_bounds__(NW * 64, NBK == 1 ? 3 : 2) void attn_bwd_row_kernel
   if (item >= items) return;
   const int h = item % H, i = item / H;
 
-  // Delta = sum_d O * dO of every query, four lanes each; left in p.delta for the dBias2 kernel
-  for (int q = tid >> 2; q < KB * 32; q += NW * 16) {
-    const int64_t e = elem(p, i, min(q, s - 1), h) + 8 * (tid & 3);
-    const f32x8 of = to_f32(load8<T>((const T*)p.o + e)), df = to_f32(load8<T>((const T*)p.dout + e));
-    float d = 0.0f;
-#pragma unroll
-    for (int t = 0; t < 8; ++t) d += of[t] * df[t];
-    d += __shfl_xor(d, 1, 64);
-    d += __shfl_xor(d, 2, 64);
-    if ((tid & 3) == 0) {
-      const int64_t st = ((int64_t)i * s + min(q, s - 1)) * H + h;
-      reinterpret_cast<float*>(stats[0])[q] = q < s ? -p.lse[st] : -INFINITY;   // (beyond s: probability 0)
-      reinterpret_cast<float*>(stats[1])[q] = -d;
-      if (q < s) p.delta[st] = d;
-    }
-  }
-  // this wave's keys
-  V8 vf[NBK][2];
+  // this wave's keys (all loads in front of the first wait; without a Bias1 they read Bias2, which counts for nothing)
+  V8 vf[NBK][2], k_in[NBK][2];
+  T b1_in[NBK];
   float b1v[NBK];
   f32x16 acc_dk[NBK], acc_dv[NBK];
+  const T* const b1_src = p.b1 ? (const T*)p.b1 + (int64_t)i * s : (const T*)p.b2;
 #pragma unroll
   for (int b = 0; b < NBK; ++b) {
-    const int key = (b * NW + wave) * 32 + ln, kc = min(key, s - 1);
+    const int kc = min((b * NW + wave) * 32 + ln, s - 1);
 #pragma unroll
     for (int kk = 0; kk < 2; ++kk) {
+      k_in[b][kk] = load8<T>((const T*)p.k + elem(p, i, kc, h) + 16 * kk + 8 * g);
       vf[b][kk] = load8<T>((const T*)p.v + elem(p, i, kc, h) + 16 * kk + 8 * g);
-      store8<T>(&kt[b * NW + wave][piece_at(ln, 2 * kk + g)], load8<T>((const T*)p.k + elem(p, i, kc, h) + 16 * kk + 8 * g));
     }
-    b1v[b] = key >= s ? -INFINITY : p.b1 ? to_f32(((const T*)p.b1)[(int64_t)i * s + kc]) : 0.0f;
+    b1_in[b] = b1_src[kc];
+  }
+  asm volatile("" ::: "memory");
+#pragma unroll
+  for (int b = 0; b < NBK; ++b) {
+    b1v[b] = (b * NW + wave) * 32 + ln >= s ? -INFINITY : p.b1 ? to_f32(b1_in[b]) : 0.0f;
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) store8<T>(&kt[b * NW + wave][piece_at(ln, 2 * kk + g)], k_in[b][kk]);
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc_dk[b][r] = acc_dv[b][r] = 0.0f;
   }
@@ -587,15 +583,42 @@ __global__ __launch_bounds__(NW * 64, NBK == 1 ? 3 : 2) void attn_bwd_row_kernel
   const int n_steps = (s + 31) >> 5;
   const TurnedAt turned(lane);
   // Q and dO tiles: the first 256 threads, 8 channels of one row of one tile each, a step ahead (positions of a row times
-  // heads and channels stay below 2^31)
-  V8 piece;
-  const T* const tile_src = (const T*)(tid >> 7 & 1 ? p.dout : p.q) + elem(p, i, 0, h);
+  // heads and channels stay below 2^31).  The threads of dO also take O and form Delta = sum_d O * dO on the way, four lanes
+  // to a query, left in p.delta for the dBias2 kernel.
+  const bool of_dout = wave >> 1 & 1;   // (the same for a wave)
+  V8 piece, o_piece;
+  float lse_piece;
+  const int64_t row_at = elem(p, i, 0, h);
+  const T* const tile_src = (const T*)(of_dout ? p.dout : p.q) + row_at;
+  const T* const o_src = (const T*)(of_dout ? p.o : p.q) + row_at;
+  const int64_t stat_at = (int64_t)i * s * H + h;
   const int tile_row = (tid & 127) >> 2, tile_col = 8 * (tid & 3), tile_at = piece_at(tile_row, tid & 3);
   auto fetch = [&](int t) {
-    if (NW == 4 || wave < 4) piece = load8<T>(tile_src + (uint32_t)(min(t * 32 + tile_row, s - 1) * H * 32 + tile_col));
+    if (NW == 4 || wave < 4) {
+      const uint32_t at = (uint32_t)min(t * 32 + tile_row, s - 1) * (uint32_t)H;
+      piece = load8<T>(tile_src + (at * 32 + tile_col));
+      o_piece = load8<T>(o_src + (at * 32 + tile_col));
+      lse_piece = p.lse[stat_at + at];
+    }
   };
   auto park = [&](int t) {
-    if (NW == 4 || wave < 4) store8<T>(&rm[t & 1][tid >> 7 & 1][tile_at], piece);
+    if (NW == 4 || wave < 4) {
+      store8<T>(&rm[t & 1][of_dout][tile_at], piece);
+      if (of_dout) {
+        const f32x8 of = to_f32(o_piece), df = to_f32(piece);
+        float d = 0.0f;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) d += of[e] * df[e];
+        d += __shfl_xor(d, 1, 64);
+        d += __shfl_xor(d, 2, 64);
+        const int q = t * 32 + tile_row;
+        if ((tid & 3) == 0) {
+          reinterpret_cast<float*>(stats[t & 1][0])[tile_row] = q < s ? -lse_piece : -INFINITY;   // (beyond s: probability 0)
+          reinterpret_cast<float*>(stats[t & 1][1])[tile_row] = -d;
+          if (q < s) p.delta[stat_at + (uint32_t)q * (uint32_t)H] = d;
+        }
+      }
+    }
   };
   // Bias2 fragments of block b at step t: lane <-> query perm_row(ln), slots <-> 8 keys; one block ahead.  Rows start at any
   // element.  The last 8 keys are read again for those beyond, and moved down (zeros above: -inf plus whatever lies there
@@ -610,9 +633,11 @@ __global__ __launch_bounds__(NW * 64, NBK == 1 ? 3 : 2) void attn_bwd_row_kernel
 #pragma unroll
       for (int kk = 0; kk < 2; ++kk) __builtin_memcpy(&b2n[kk], b2h + (row + (uint32_t)(key0 + 16 * kk + 8 * g)), sizeof(V8));
     } else {
+      int part0 = key0;
+      asm volatile("" : "+s"(part0));   // (nothing of it is formed ahead of the walk: no registers for it)
 #pragma unroll
       for (int kk = 0; kk < 2; ++kk) {
-        const int kb = key0 + 16 * kk + 8 * g, from = min(kb, s - 8);
+        const int kb = part0 + 16 * kk + 8 * g, from = min(kb, s - 8);
         unsigned __int128 v;
         __builtin_memcpy(&v, b2h + (row + (uint32_t)from), sizeof(v));
         v = kb >= s ? 0 : v >> (16 * (kb - from));
@@ -629,12 +654,6 @@ __global__ __launch_bounds__(NW * 64, NBK == 1 ? 3 : 2) void attn_bwd_row_kernel
     fetch(t + 1);
     asm volatile("" ::: "memory");   // (issued here, a step ahead of their use)
     T* const ds_tile = reinterpret_cast<T*>(&ex[buf][wave][0]);
-    V8 qf[2], dof[2];
-#pragma unroll
-    for (int kk = 0; kk < 2; ++kk) {
-      qf[kk] = load8<T>(&rm[buf][0][piece_at(b2q, 2 * kk + g)]);
-      dof[kk] = load8<T>(&rm[buf][1][piece_at(b2q, 2 * kk + g)]);
-    }
     f32x16 dq;
 #pragma unroll
     for (int r = 0; r < 16; ++r) dq[r] = 0.0f;
@@ -642,7 +661,7 @@ __global__ __launch_bounds__(NW * 64, NBK == 1 ? 3 : 2) void attn_bwd_row_kernel
     for (int b = 0; b < NBK; ++b) {
       const int blk = b * NW + wave;
       // (opaque offsets: what all steps or all blocks read alike would be kept in registers that are not there)
-      int kt_off = blk * 1024, rm_off = buf * 2048, st_off = t * 4;
+      int kt_off = blk * 1024, rm_off = buf * 2048, st_off = buf * 8;
       asm volatile("" : "+v"(kt_off), "+v"(rm_off), "+v"(st_off));
       const T* const kb = &kt[0][0] + kt_off;
       const T* const qd = &rm[0][0][0] + rm_off;
@@ -652,7 +671,7 @@ __global__ __launch_bounds__(NW * 64, NBK == 1 ? 3 : 2) void attn_bwd_row_kernel
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         sm[r] = b1;
-        dp[r] = stats[1][st_off + 2 * (r >> 3) + g][r & 7];
+        dp[r] = stats[0][1][st_off + 2 * (r >> 3) + g][r & 7];
       }
 #pragma unroll
       for (int kk = 0; kk < 2; ++kk) mma32(sm, finite_low(b2n[kk]), one[kk]);   // Bias1 + Bias2
@@ -661,14 +680,14 @@ __global__ __launch_bounds__(NW * 64, NBK == 1 ? 3 : 2) void attn_bwd_row_kernel
       asm volatile("" ::: "memory");
 #pragma unroll
       for (int kk = 0; kk < 2; ++kk) {
-        mma32(sm, qf[kk], load8<T>(kb + piece_at(ln, 2 * kk + g)));   // S[query][key] (+ biases)
-        mma32(dp, dof[kk], vf[b][kk]);                                  // dP[query][key] - Delta
+        mma32(sm, load8<T>(qd + piece_at(b2q, 2 * kk + g)), load8<T>(kb + piece_at(ln, 2 * kk + g)));   // S[query][key] (+ biases)
+        mma32(dp, load8<T>(qd + 1024 + piece_at(b2q, 2 * kk + g)), vf[b][kk]);                           // dP[query][key] - Delta
       }
       __builtin_amdgcn_sched_barrier(0);
       V8 pf[2], dsf[2];
 #pragma unroll
       for (int ks = 0; ks < 2; ++ks) {
-        const f32x8 nl = stats[0][st_off + 2 * ks + g];
+        const f32x8 nl = stats[0][0][st_off + 2 * ks + g];
         f32x8 pv, dv;
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
@@ -713,12 +732,11 @@ __global__ __launch_bounds__(NW * 64, NBK == 1 ? 3 : 2) void attn_bwd_row_kernel
       if (q < s) *reinterpret_cast<V4*>((T*)p.dq + elem(p, i, q, h) + 8 * wave + 4 * g) = from_f32<T>(sum);
     }
   }
+  // dK and dV, a block at a time through the place of this wave's partial dQ that the last step left alone: four lanes to a
+  // key store its 64 bytes (from the accumulators they would be pieces of 8)
+  T* const out_tile = reinterpret_cast<T*>(&ex[n_steps & 1][wave][0]);
 #pragma unroll
   for (int b = 0; b < NBK; ++b) {
-    const int key = (b * NW + wave) * 32 + ln;
-    if (key >= s) continue;
-    T* dk = (T*)p.dk + elem(p, i, key, h);
-    T* dv = (T*)p.dv + elem(p, i, key, h);
 #pragma unroll
     for (int a = 0; a < 4; ++a) {
       f32x4 x, y;
@@ -727,9 +745,21 @@ __global__ __launch_bounds__(NW * 64, NBK == 1 ? 3 : 2) void attn_bwd_row_kernel
         x[e] = acc_dk[b][4 * a + e];
         y[e] = acc_dv[b][4 * a + e];
       }
-      *reinterpret_cast<V4*>(dk + 8 * a + 4 * g) = from_f32<T>(x);
-      *reinterpret_cast<V4*>(dv + 8 * a + 4 * g) = from_f32<T>(y);
+      *reinterpret_cast<V4*>(out_tile + piece_at(ln, a) + 4 * g) = from_f32<T>(x);
+      *reinterpret_cast<V4*>(out_tile + 1024 + piece_at(ln, a) + 4 * g) = from_f32<T>(y);
     }
+    wave_lds_sync();
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+      const int row = 16 * half + (lane >> 2), key = (b * NW + wave) * 32 + row;
+      const V8 x = load8<T>(out_tile + piece_at(row, lane & 3)), y = load8<T>(out_tile + 1024 + piece_at(row, lane & 3));
+      if (key < s) {
+        const int64_t at = elem(p, i, key, h) + 8 * (lane & 3);
+        store8<T>((T*)p.dk + at, x);
+        store8<T>((T*)p.dv + at, y);
+      }
+    }
+    wave_lds_sync();
   }
 }
 
