@@ -789,32 +789,184 @@ bool rows_at_once(const BwdParams& p) {
   return pairs >= (p.s > 512 && p.s <= 640 ? 216 : 192) * ((pairs + 255) / 256);
 }
 
-// dBias2's tiles: 16-bit rows as above (padded to 80 bytes a third of the LDS cycles were conflicts: the operator at 768 rows of 768
-// positions, forward and backward, 2735 -> 2640 us, 384 360 -> 357), fp32 ones padded
-template <typename T>
-__device__ __forceinline__ int db2_at(int row, int piece) { return sizeof(T) == 2 ? piece_at(row, piece) : row * kTP + 8 * piece; }
-template <typename T> constexpr int kDb2Tile = 64 * (sizeof(T) == 2 ? 32 : kTP);
-
-// dBias2: a workgroup takes 64 queries x 64 keys of one head, a wave one 32 x 32 quadrant, and
-// walks over the rows; the two Q / dO tiles and the two K / V tiles of a row are shared.
-// Works on S^T like dQ.  Bias2 itself does not change along the walk and stays in registers;
-// a row's Bias1 is added to it for the initial value of the S^T accumulator, -Delta is that of
-// dP^T.  Nothing in the walk looks at s: queries and keys beyond it repeat the last one, and
-// what accumulates for them is not stored.
-// The walk is cut into slices of rows: 384 tokens and 4 heads are 144 workgroups for 256 compute units that
+// dBias2, the walk: a workgroup takes a tile of queries x keys of one head and walks over the rows, whose Q, dO, K and V tiles its waves
+// share.  Works on S^T like dQ.  Bias2 itself does not change along the walk and stays in registers; a row's Bias1 is added to it for the
+// initial value of the S^T accumulator, -Delta is that of dP^T.  Nothing in the walk looks at s: queries and keys beyond it repeat the last
+// one, and what accumulates for them is not stored.
+// The walk is cut into slices of rows: 384 tokens and 4 heads are 96 workgroups for 256 compute units that
 // hold four each, every one a serial chain over 384 rows.  Slices write fp32 partial sums that
 // attn_bwd_db2_sum_kernel adds in order (no atomics).  A slice's workgroups all go to one XCD
 // (workgroups are dealt to the XCDs in turn, and the slice is the fastest index), whose L2 then fetches the slice's rows
 // once; with a slice's workgroups on all eight the rows come through the memory-side cache eight times.  us at 384 rows,
-// 384 tokens, 4 heads, bf16: one slice 312; seven slices, spread 165 with the sum; eight, one per XCD, 107 + 4.
-template <typename T, bool VEC>
-__global__ __launch_bounds__(256, (BwdCfg<T, VEC>::kMinWaves)) void attn_bwd_db2_kernel(BwdParams p) {
-  typedef typename Vec8<T>::type V8;
-  constexpr int NB = BwdCfg<T, VEC>::kBuffers;
-  __shared__ __attribute__((aligned(32))) T tiles[NB][4][kDb2Tile<T>];   // Q, dO (64 queries), K, V (64 keys)
+// 384 tokens, 4 heads, bf16, tiles of 64 x 64: one slice 312; seven slices, spread 165 with the sum; eight, one per XCD, 107 + 4.
+
+// What a lane holds of a 32 x 32 block of dBias2: keys key0 + 16 ks + 8 g .. + 7 of query qi, in acc[8 ks ..]
+template <typename T>
+__device__ __forceinline__ void db2_store(const BwdParams& p, int slice, int h, int qi, int key0, int g, const f32x16& acc) {
+  const int s = p.s;
+  const bool vec = (s & 7) == 0;
+#pragma unroll
+  for (int ks = 0; ks < 2; ++ks) {
+    const int kb = key0 + 16 * ks + 8 * g;
+    f32x8 v;
+#pragma unroll
+    for (int t = 0; t < 8; ++t) v[t] = acc[8 * ks + t];
+    if (p.parts) {
+      float* const dst = p.parts + (((int64_t)slice * p.heads + h) * s + qi) * s;
+      if (vec) {
+        if (kb < s) store8<float>(dst + kb, v);
+      } else {
+#pragma unroll
+        for (int t = 0; t < 8; ++t)
+          if (kb + t < s) dst[kb + t] = v[t];
+      }
+    } else {
+      T* const dst = (T*)p.db2 + ((int64_t)h * s + qi) * s;
+      if (vec) {
+        if (kb < s) store8<T>(dst + kb, from_f32<T>(v));
+      } else {
+#pragma unroll
+        for (int t = 0; t < 8; ++t)
+          if (kb + t < s) dst[kb + t] = from_f32<T>(v[t]);
+      }
+    }
+  }
+}
+
+// 16-bit: NWQ waves, each 32 queries x NB blocks of 32 keys that share the query's operands and statistics; the next row's tiles
+// travel by direct-to-LDS loads while a row is computed.  A lane's place in LDS is fixed by the instruction, so the exchange
+// of pieces (piece_at) is one of the global addresses.
+// Bound by what a compute unit issues, its LDS and the way of the tiles there together: with two blocks and four waves 67 vector instructions
+// and 5 MFMA per block, and 9 KB through LDS.  In tiles of 64 x 64, a block a wave, with the tiles through registers, they were 82, 5
+// and 12 KB (figures: db2_walk).  Two waves per SIMD of twice the registers: 123 us against 98 at 384 positions; sixteen slices instead
+// of eight: 100 - 117.
+template <int NWQ, int NB>
+__global__ __launch_bounds__(NWQ * 64, 3) void attn_bwd_db2_kernel(BwdParams p) {
+  typedef bf16_t T;
+  typedef Vec8<T>::type V8;
+  constexpr int kQ = 32 * NWQ, kKeys = 32 * NB;
+  __shared__ __attribute__((aligned(32))) T tiles[2][(2 * kQ + 2 * kKeys) * 32];   // Q, dO, K, V
+  constexpr int kDo = kQ * 32, kK = 2 * kQ * 32, kV = kK + kKeys * 32;               // where they start
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, ln = lane & 31, g = lane >> 5;
+  const int s = p.s, H = p.heads;
+  const int slice = blockIdx.x % p.slices, pair = blockIdx.x / p.slices, q_tiles = (s + kQ - 1) / kQ, k_tiles = (s + kKeys - 1) / kKeys;
+  const int row_begin = (int)((int64_t)p.n_rows * slice / p.slices), row_end = (int)((int64_t)p.n_rows * (slice + 1) / p.slices);
+  const int qs0 = pair % q_tiles * kQ, ks0 = pair / q_tiles % k_tiles * kKeys, h = pair / q_tiles / k_tiles;
+  const int q0 = qs0 + 32 * wave, qi = min(q0 + ln, s - 1);
+  const bool vec = (s & 7) == 0;
+  const T* const b2row = (const T*)p.b2 + ((int64_t)h * s + qi) * s;
+  f32x16 b2acc[NB], acc[NB];
+#pragma unroll
+  for (int b = 0; b < NB; ++b) {
+    const f32x8 lo = load_bias8<T>(b2row, ks0 + 32 * b + 8 * g, s, vec), hi = load_bias8<T>(b2row, ks0 + 32 * b + 16 + 8 * g, s, vec);
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      b2acc[b][r] = r < 8 ? lo[r & 7] : hi[r & 7];
+      acc[b][r] = 0.0f;
+    }
+  }
+  // Bias1 reaches the accumulator on the matrix pipe (see the dQ kernel): one value per lane, that of the key its accumulator row
+  // stands for, in K slot 0 of one more product.  (Without a Bias1 the loads go to Bias2's row and count for nothing.)
+  const T* const b1base = p.b1 ? (const T*)p.b1 : b2row;
+  const int64_t b1pitch = p.b1 ? s : 0;
+  const bool b1on = p.b1 != nullptr;
+  unsigned off_b1[NB];
+#pragma unroll
+  for (int b = 0; b < NB; ++b) off_b1[b] = min(ks0 + 32 * b + perm_row(ln), s - 1);
+  V8 one_frag = zero_frag<T>();
+  one_frag[0] = (T)(g == 0 && b1on ? 1.0f : 0.0f);
+
+  // This wave's share of a row's tiles: 16 rows of 64 bytes an instruction, two of Q's and dO's 2 NWQ, its part of K's and V's four
+  // (three waves load one of those twice, to the same place).  A row moves the base address, the same for all lanes.
+  constexpr int kKv = (2 * NB + NWQ - 1) / NWQ;
+  const int piece8 = 8 * ((lane & 3) ^ ((lane >> 4) & 3));
+  auto tile_offset = [&](int pos) { return (((uint32_t)min(pos + (lane >> 2), s - 1) * H + h) * 32 + piece8) * (uint32_t)sizeof(T); };
+  uint32_t off_q[2], off_k[kKv];
+  int kv_at[kKv];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) off_q[j] = tile_offset(qs0 + 16 * (wave + NWQ * j));
+#pragma unroll
+  for (int j = 0; j < kKv; ++j) {
+    kv_at[j] = min(wave + NWQ * j, 2 * NB - 1);
+    off_k[j] = tile_offset(ks0 + 16 * kv_at[j]);
+  }
+  const int64_t row_elems = (int64_t)s * H * 32, row_stats = (int64_t)s * H;
+  const unsigned off_stat = (unsigned)qi * H + h;
+  float mq_n, dq_n;
+  T b1_n[NB];
+  auto fetch = [&](int i) {
+    T* const t = tiles[i & 1];
+    mq_n = (p.lse + i * row_stats)[off_stat];
+    dq_n = (p.delta + i * row_stats)[off_stat];
+    const T* const b1row = b1base + i * b1pitch;
+#pragma unroll
+    for (int b = 0; b < NB; ++b) b1_n[b] = b1row[off_b1[b]];
+    const uint64_t qa = (uint64_t)((const T*)p.q + i * row_elems), da = (uint64_t)((const T*)p.dout + i * row_elems);
+    const uint64_t ka = (uint64_t)((const T*)p.k + i * row_elems), va = (uint64_t)((const T*)p.v + i * row_elems);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      load_to_lds16_s<0>(qa, off_q[j], lds_address(t + (wave + NWQ * j) * 512));
+      load_to_lds16_s<0>(da, off_q[j], lds_address(t + kDo + (wave + NWQ * j) * 512));
+    }
+#pragma unroll
+    for (int j = 0; j < kKv; ++j) {
+      load_to_lds16_s<0>(ka, off_k[j], lds_address(t + kK + kv_at[j] * 512));
+      load_to_lds16_s<0>(va, off_k[j], lds_address(t + kV + kv_at[j] * 512));
+    }
+  };
+  // Row i is computed out of buffer i & 1 while row i + 1 travels into the other one, which every wave left at the last barrier.
+  const int last = row_end - 1;
+  fetch(row_begin);
+  ring_barrier<0>();
+  for (int i = row_begin; i < row_end; ++i) {
+    const float neg_mq = -mq_n, neg_dq = -dq_n;
+    T b1[NB];
+#pragma unroll
+    for (int b = 0; b < NB; ++b) b1[b] = b1_n[b];
+    if (i < last) fetch(i + 1);
+    const T* const t = tiles[i & 1];
+    V8 qf[2], dof[2];
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) {
+      qf[kk] = load8<T>(t + piece_at(32 * wave + ln, 2 * kk + g));
+      dof[kk] = load8<T>(t + kDo + piece_at(32 * wave + ln, 2 * kk + g));
+    }
+    f32x16 ndq;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) ndq[r] = neg_dq;
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      V8 b1a = zero_frag<T>();
+      b1a[0] = g == 0 && b1on ? b1[b] : (T)0.0f;
+      f32x16 st = b2acc[b], dp = ndq;
+      if (b) __builtin_amdgcn_sched_barrier(0);   // (one block after the other: both blocks' logits at once are registers that are not there)
+      mma32(st, b1a, one_frag);   // Bias2 + Bias1
+#pragma unroll
+      for (int kk = 0; kk < 2; ++kk) {
+        const V8 kf = load8<T>(t + kK + piece_at(32 * b + perm_row(ln), 2 * kk + g));
+        const V8 vf = load8<T>(t + kV + piece_at(32 * b + perm_row(ln), 2 * kk + g));
+        mma32(st, kf, qf[kk]);    // S^T[key][query] (+ biases)
+        mma32(dp, vf, dof[kk]);   // dP^T[key][query] - Delta
+      }
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[b][r] += fast_exp2(st[r] * kBwdLog2e + neg_mq) * dp[r];
+    }
+    ring_barrier<0>();
+  }
+  if (q0 + ln < s) {
+#pragma unroll
+    for (int b = 0; b < NB; ++b) db2_store<T>(p, slice, h, qi, ks0 + 32 * b, g, acc[b]);
+  }
+}
+
+// fp32: four waves, tiles of 64 queries x 64 keys, a 32 x 32 quadrant each; one buffer, through registers.
+template <bool VEC>
+__global__ __launch_bounds__(256, 1) void attn_bwd_db2_fp32_kernel(BwdParams p) {
+  typedef float T;
+  typedef Vec8<T>::type V8;
+  __shared__ __attribute__((aligned(32))) T tiles[4][64 * kTP];   // Q, dO (64 queries), K, V (64 keys)
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, ln = lane & 31, g = lane >> 5;
   const int s = p.s, H = p.heads;
-  constexpr bool vec = VEC;
   const int slice = blockIdx.x % p.slices, pair = blockIdx.x / p.slices, tiles_s = (s + 63) / 64;
   const int row_begin = (int)((int64_t)p.n_rows * slice / p.slices), row_end = (int)((int64_t)p.n_rows * (slice + 1) / p.slices);
   const int qs0 = pair % tiles_s * 64, ks0 = pair / tiles_s % tiles_s * 64, h = pair / tiles_s / tiles_s;
@@ -825,11 +977,11 @@ __global__ __launch_bounds__(256, (BwdCfg<T, VEC>::kMinWaves)) void attn_bwd_db2
   const T* b2row = (const T*)p.b2 + ((int64_t)h * s + qi) * s;
   f32x8 b2f[2];
 #pragma unroll
-  for (int ks = 0; ks < 2; ++ks) b2f[ks] = load_bias8<T>(b2row, key0 + 16 * ks + 8 * g, s, vec);
+  for (int ks = 0; ks < 2; ++ks) b2f[ks] = load_bias8<T>(b2row, key0 + 16 * ks + 8 * g, s, VEC);
   // (without a Bias1 the loads go to Bias2's row and count for nothing: no load under a branch)
   const T* b1base = p.b1 ? (const T*)p.b1 : b2row;
   const int64_t b1pitch = p.b1 ? s : 0;
-  const float b1on = p.b1 ? 1.0f : 0.0f;
+  const bool b1on = p.b1 != nullptr;
   f32x16 acc;
 #pragma unroll
   for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
@@ -837,27 +989,16 @@ __global__ __launch_bounds__(256, (BwdCfg<T, VEC>::kMinWaves)) void attn_bwd_db2
   // thread t: 8 channels (t & 3) of row t >> 2 of each of the four 64-row tiles.  Along the
   // walk only the row's base address changes, the same for all lanes: what a lane adds to it
   // is formed once.
-  const int crow = tid >> 2, cc = 8 * (tid & 3), park_at = db2_at<T>(crow, tid & 3);
+  const int crow = tid >> 2, cc = 8 * (tid & 3), park_at = crow * kTP + cc;
   const unsigned off_q = ((unsigned)min(qs0 + crow, s - 1) * H + h) * 32 + cc;
   const unsigned off_k = ((unsigned)min(ks0 + crow, s - 1) * H + h) * 32 + cc;
   const unsigned off_stat = (unsigned)qi * H + h;
   unsigned off_b1[2];
 #pragma unroll
-  for (int ks = 0; ks < 2; ++ks) off_b1[ks] = vec ? min(key0 + 16 * ks + 8 * g, s - 8) : 0;
+  for (int ks = 0; ks < 2; ++ks) off_b1[ks] = VEC ? min(key0 + 16 * ks + 8 * g, s - 8) : 0;
   const int64_t row_elems = (int64_t)s * H * 32, row_stats = (int64_t)s * H;
   V8 piece[4], b1n[2];
   float mq_n = 0.0f, dq_n = 0.0f;
-  // 16-bit: Bias1 reaches the accumulator on the matrix pipe (see the dQ kernel): one value
-  // per lane, that of the key its accumulator row stands for, in K slot 0 of one more product
-  constexpr bool MMB = sizeof(T) == 2;
-  const unsigned off_b1m = min(key0 + perm_row(ln), s - 1);
-  T b1m_n = (T)0.0f;
-  V8 one_frag;
-#pragma unroll
-  for (int t = 0; t < 8; ++t) one_frag[t] = (T)(t == 0 && g == 0 ? b1on : 0.0f);
-  f32x16 b2acc;
-#pragma unroll
-  for (int r = 0; r < 16; ++r) b2acc[r] = b2f[r >> 3][r & 7];
   auto fetch = [&](int i) {
     piece[0] = load8<T>((const T*)p.q + i * row_elems + off_q);
     piece[1] = load8<T>((const T*)p.dout + i * row_elems + off_q);
@@ -866,103 +1007,50 @@ __global__ __launch_bounds__(256, (BwdCfg<T, VEC>::kMinWaves)) void attn_bwd_db2
     mq_n = (p.lse + i * row_stats)[off_stat];
     dq_n = (p.delta + i * row_stats)[off_stat];
     const T* b1row = b1base + i * b1pitch;
-    if (MMB) {
-      b1m_n = b1row[off_b1m];
-    } else {
 #pragma unroll
-      for (int ks = 0; ks < 2; ++ks)
-        b1n[ks] = vec ? load8<T>(b1row + off_b1[ks]) : load_bias8_raw<T>(b1row, key0 + 16 * ks + 8 * g, s, false);
-    }
+    for (int ks = 0; ks < 2; ++ks)
+      b1n[ks] = VEC ? load8<T>(b1row + off_b1[ks]) : load_bias8_raw<T>(b1row, key0 + 16 * ks + 8 * g, s, false);
   };
-  // Row i is computed out of buffer i % NB while row i + 1, fetched a step earlier, is parked
-  // (two buffers: into the other one, which every wave left at the last barrier).
   const int last = row_end - 1;
   fetch(row_begin);
 #pragma unroll
-  for (int w = 0; w < 4; ++w) store8<T>(&tiles[row_begin % NB][w][park_at], piece[w]);
+  for (int w = 0; w < 4; ++w) store8<T>(&tiles[w][park_at], piece[w]);
   float neg_mq = -mq_n, neg_dq = -dq_n;
   V8 b1c[2] = {b1n[0], b1n[1]};
-  T b1m = b1m_n;
   __syncthreads();
   for (int i = row_begin; i < row_end; ++i) {
-    const int buf = i % NB;
     fetch(min(i + 1, last));
     asm volatile("" ::: "memory");   // the loads are issued here, a step ahead of their use
     f32x16 st, dp;
 #pragma unroll
     for (int r = 0; r < 16; ++r) dp[r] = neg_dq;
-    if constexpr (MMB) {
-      V8 b1a;
 #pragma unroll
-      for (int t = 0; t < 8; ++t) b1a[t] = (T)0.0f;
-      b1a[0] = (g == 0 && b1on != 0.0f) ? b1m : (T)0.0f;
-      st = b2acc;
-      mma32(st, b1a, one_frag);   // Bias2 + Bias1
-    } else {
+    for (int ks = 0; ks < 2; ++ks) {
+      const f32x8 b1f = to_f32(b1c[ks]);
 #pragma unroll
-      for (int ks = 0; ks < 2; ++ks) {
-        const f32x8 b1f = to_f32(b1c[ks]);
-#pragma unroll
-        for (int t = 0; t < 8; ++t) st[8 * ks + t] = (b1on != 0.0f ? b1f[t] : 0.0f) + b2f[ks][t];   // (not b1f * b1on: -inf)
-      }
+      for (int t = 0; t < 8; ++t) st[8 * ks + t] = (b1on ? b1f[t] : 0.0f) + b2f[ks][t];
     }
 #pragma unroll
     for (int kk = 0; kk < 2; ++kk) {
-      const V8 qf = load8<T>(&tiles[buf][0][db2_at<T>(32 * wq + ln, 2 * kk + g)]);
-      const V8 dof = load8<T>(&tiles[buf][1][db2_at<T>(32 * wq + ln, 2 * kk + g)]);
-      const V8 kf = load8<T>(&tiles[buf][2][db2_at<T>(32 * wk + perm_row(ln), 2 * kk + g)]);
-      const V8 vf = load8<T>(&tiles[buf][3][db2_at<T>(32 * wk + perm_row(ln), 2 * kk + g)]);
+      const int c = 16 * kk + 8 * g;
+      const V8 qf = load8<T>(&tiles[0][(32 * wq + ln) * kTP + c]), dof = load8<T>(&tiles[1][(32 * wq + ln) * kTP + c]);
+      const V8 kf = load8<T>(&tiles[2][(32 * wk + perm_row(ln)) * kTP + c]), vf = load8<T>(&tiles[3][(32 * wk + perm_row(ln)) * kTP + c]);
       mma32(st, kf, qf);    // S^T[key][query] (+ biases)
       mma32(dp, vf, dof);   // dP^T[key][query] - Delta
     }
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[r] += fast_exp2(st[r] * kBwdLog2e + neg_mq) * dp[r];
-    if (NB == 1) __syncthreads();
+    __syncthreads();
     // the next row: tiles into LDS, its statistics and Bias1 into this step's places
 #pragma unroll
-    for (int w = 0; w < 4; ++w) store8<T>(&tiles[(i + 1) % NB][w][park_at], piece[w]);
+    for (int w = 0; w < 4; ++w) store8<T>(&tiles[w][park_at], piece[w]);
     neg_mq = -mq_n;
     neg_dq = -dq_n;
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks) b1c[ks] = b1n[ks];
-    b1m = b1m_n;
     __syncthreads();
   }
-  if (q_ok && p.parts) {
-    float* dst = p.parts + (((int64_t)slice * H + h) * s + qi) * s;
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
-      const int kb = key0 + 16 * ks + 8 * g;
-      if (vec) {
-        if (kb < s) {
-#pragma unroll
-          for (int c = 0; c < 2; ++c)
-            *reinterpret_cast<f32x4*>(dst + kb + 4 * c) =
-                f32x4{acc[8 * ks + 4 * c], acc[8 * ks + 4 * c + 1], acc[8 * ks + 4 * c + 2], acc[8 * ks + 4 * c + 3]};
-        }
-      } else {
-#pragma unroll
-        for (int t = 0; t < 8; ++t)
-          if (kb + t < s) dst[kb + t] = acc[8 * ks + t];
-      }
-    }
-  } else if (q_ok) {
-    T* dst = (T*)p.db2 + ((int64_t)h * s + qi) * s;
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
-      const int kb = key0 + 16 * ks + 8 * g;
-      f32x8 v;
-#pragma unroll
-      for (int t = 0; t < 8; ++t) v[t] = acc[8 * ks + t];
-      if (vec) {
-        if (kb < s) store8<T>(dst + kb, from_f32<T>(v));
-      } else {
-#pragma unroll
-        for (int t = 0; t < 8; ++t)
-          if (kb + t < s) dst[kb + t] = from_f32<T>(v[t]);
-      }
-    }
-  }
+  if (q_ok) db2_store<T>(p, slice, h, qi, key0, g, acc);
 }
 
 // dBias2 = the slices' partial sums added in order, V values per thread (4 where the values of a slice are
@@ -993,6 +1081,30 @@ int triattn_bwd_slices(int n_rows, int s, int heads) {
   return want > 1 && want * heads * s * s * 4 <= (int64_t)128 << 20 ? (int)want : 1;
 }
 
+// dBias2's walk, 16-bit: waves of a workgroup and blocks of a wave.  A small one is a chain of rows, whose length counts: as long as
+// every SIMD can have a 32 x 32 block of its own, two waves of one block each.  Beyond, two blocks a wave, four waves or three; the work of a
+// compute unit is that of the workgroups it gets, in turn or at once, so the fullest one's waves count, and four do in the time of
+// three what loads a quarter less.  us at S rows of S positions, 4 heads, 64 x 64 tiles of four waves (before) / two waves of one block /
+// three of two / four of two: S = 64 7.4 / 5.6 / 8.7 / 9.0, 96 9.6 / 8.8 / 12.3 / 12.6, 160 15.2 / 13.6 / 16.4 / 17.6, 192 18.1 / 21.4 / 18.9 / 20.1, 256
+// 30.7 / 39 / 31 / 27.5, 288 50.8 / 54 / 45.2 / 48, 320 59.8 / 79 / 63 / 53, 352 87.8 / 96 / 74.4 / 77, 384 107 / 126 / 88 / 94, 416 139 / 172 / 138 / 132,
+// 512 222 / 324 / 250 / 215, 640 471 / 927 / 476 / 393, 768 781 / - / 763 / 659.
+template <typename T>
+static void db2_walk(const BwdParams& p, hipStream_t stream) {
+  const auto groups = [&](int queries, int keys) {
+    return (unsigned)((p.s + queries - 1) / queries) * (unsigned)((p.s + keys - 1) / keys) * (unsigned)p.heads * (unsigned)p.slices;
+  };
+  if constexpr (sizeof(T) == 2) {
+    const int64_t three = (int64_t)((groups(96, 64) + 255) / 256) * 3, four = (int64_t)((groups(128, 64) + 255) / 256) * 4;
+    if (groups(32, 32) <= 1024) attn_bwd_db2_kernel<2, 1><<<dim3(groups(64, 32)), dim3(128), 0, stream>>>(p);
+    else if (4 * four > 5 * three) attn_bwd_db2_kernel<3, 2><<<dim3(groups(96, 64)), dim3(192), 0, stream>>>(p);
+    else attn_bwd_db2_kernel<4, 2><<<dim3(groups(128, 64)), dim3(256), 0, stream>>>(p);
+  } else {
+    const dim3 grid(groups(64, 64));
+    if ((p.s & 7) == 0) attn_bwd_db2_fp32_kernel<true><<<grid, dim3(256), 0, stream>>>(p);
+    else attn_bwd_db2_fp32_kernel<false><<<grid, dim3(256), 0, stream>>>(p);
+  }
+}
+
 template <typename T>
 static void db2_sum(const BwdParams& p, int slices, hipStream_t stream) {
   const int64_t n = (int64_t)p.heads * p.s * p.s;
@@ -1009,8 +1121,7 @@ int triattn_bwd(const void* q, const void* k, const void* v, const void* b1, con
   if (n_rows == 0 || s == 0 || heads == 0) return 0;
   const int slices = parts && db2 ? triattn_bwd_slices(n_rows, s, heads) : 1;
   BwdParams p = {q, k, v, o, dout, b1, b2, lse, delta, dq, dk, dv, db2, n_rows, s, heads, slices > 1 ? parts : nullptr, slices};
-  const unsigned tiles = (unsigned)((s + 63) / 64);
-  const dim3 walk(((unsigned)((s + 127) / 128) * heads * n_rows + 7) / 8 * 8), pairs(tiles * tiles * heads * slices);
+  const dim3 walk(((unsigned)((s + 127) / 128) * heads * n_rows + 7) / 8 * 8);
   const bool joint = rows_at_once<T>(p);
   if constexpr (sizeof(T) == 2) if (joint) {
     const dim3 grid(((unsigned)heads * n_rows + 7) / 8 * 8);
@@ -1020,18 +1131,16 @@ int triattn_bwd(const void* q, const void* k, const void* v, const void* b1, con
     else if (s <= 512) attn_bwd_row_kernel<8, 2><<<grid, dim3(512), 0, stream>>>(p);
     else attn_bwd_row_kernel<8, 3><<<grid, dim3(512), 0, stream>>>(p);
   }
-  if (joint) {
-    if (db2 && (s & 7) == 0) attn_bwd_db2_kernel<T, true><<<pairs, dim3(256), 0, stream>>>(p);
-    else if (db2) attn_bwd_db2_kernel<T, false><<<pairs, dim3(256), 0, stream>>>(p);
-  } else if ((s & 7) == 0) {
-    attn_bwd_dq_kernel<T, true><<<walk, dim3(256), 0, stream>>>(p);   // (writes Delta: first)
-    attn_bwd_kv_kernel<T, true><<<walk, dim3(256), 0, stream>>>(p);
-    if (db2) attn_bwd_db2_kernel<T, true><<<pairs, dim3(256), 0, stream>>>(p);
-  } else {
-    attn_bwd_dq_kernel<T, false><<<walk, dim3(256), 0, stream>>>(p);
-    attn_bwd_kv_kernel<T, false><<<walk, dim3(256), 0, stream>>>(p);
-    if (db2) attn_bwd_db2_kernel<T, false><<<pairs, dim3(256), 0, stream>>>(p);
+  if (!joint) {
+    if ((s & 7) == 0) {
+      attn_bwd_dq_kernel<T, true><<<walk, dim3(256), 0, stream>>>(p);   // (writes Delta: first)
+      attn_bwd_kv_kernel<T, true><<<walk, dim3(256), 0, stream>>>(p);
+    } else {
+      attn_bwd_dq_kernel<T, false><<<walk, dim3(256), 0, stream>>>(p);
+      attn_bwd_kv_kernel<T, false><<<walk, dim3(256), 0, stream>>>(p);
+    }
   }
+  if (db2) db2_walk<T>(p, stream);
   if (slices > 1) db2_sum<T>(p, slices, stream);
   return 0;
 }

@@ -200,3 +200,16 @@ def test_bias2_of_minus_infinity_has_weight_zero(dtype, with_bias1, N, S, H):
     for name, g, w in zip(("dQ", "dK", "dV", "dBias2"), (qc.grad, kc.grad, vc.grad, b2c.grad), want[1:]):
         assert torch.isfinite(g).all() and rel_err(g, w) <= tol(dtype), name
     assert (b2c.grad[..., S - 2, 1] == 0).all() and (b2c.grad[..., 0, S // 2:] == 0).all()
+
+
+@pytest.mark.parametrize("N,S,H", [(17, 33, 1), (24, 97, 4), (40, 160, 4), (16, 191, 2),       # two waves of one block
+                                   (64, 192, 4), (70, 193, 5), (33, 257, 8), (64, 288, 4),      # three waves of two blocks
+                                   (64, 224, 4), (65, 289, 4), (64, 321, 5), (17, 800, 4)])     # four waves of two blocks
+def test_dbias2_in_workgroups_of_every_size(N, S, H):
+    """The three forms of dBias2's walk, at sizes that fill their tiles, just pass them and fall short of them, masked keys among
+    them.  Tolerance as for the other gradients: the reference's O and log-sum-exp are not rounded."""
+    q, k, v, b1, b2, do = (t.cuda() for t in _operands(1, N, S, H, torch.bfloat16, seed=N * S, n_masked=min(9, S // 3)))
+    want = _autograd_reference(q, k, v, b1, b2, do)[4]
+    got = _product(q, k, v, b1, b2, do)[4]
+    assert torch.isfinite(got).all()
+    assert rel_err(got, want) <= tol(torch.bfloat16)
