@@ -42,6 +42,8 @@ constexpr float kLog2e = 1.4426950408889634f;
 // optimistic path accepts
 enum { kOptimistic = 0, kClassic = 1, kMasked = 2, kOptimisticZero = 3 };
 constexpr float kOptimisticLimit = 1.0e12f;
+// fast_tile: this lane's sum of probabilities against the reference 0 that fp32 sums of P and of P V can be trusted with
+constexpr float kTrustedLow = 1.0e-25f, kTrustedHigh = 1.0e25f;
 constexpr float kLn2 = 0.6931471805599453f;
 // kClassic: a running maximum no larger than this (natural units, all lanes of the wave) is
 // replaced by the reference 0, which makes exp2() of the raw logit the probability
@@ -305,6 +307,8 @@ __global__ __launch_bounds__((NWQ * 64), (sizeof(T) == 2 ? (!std::is_void<TS>::v
   // Keys beyond n_keys hold garbage (or, below n, keys that are left out) in K, removed by the -inf mask bias, and
   // are zeroed in V^T (0 * garbage must stay 0).
   constexpr bool kDirect = sizeof(T) == 2;
+  constexpr bool kFast = sizeof(T) == 2 && !has_mask;
+  __shared__ int lds_vote[2][kFast ? NWQ : 1];
   constexpr int FPW = 8 * R / NWQ;   // fragments each wave moves per tile, of one operand and row
   static_assert(FPW >= 1 && FPW <= 4, "a wave's fragments are consecutive in memory");
   const int fid0 = wave * FPW, fr = fid0 >> 3, f0 = fid0 & 7;   // row, first fragment
@@ -357,11 +361,17 @@ __global__ __launch_bounds__((NWQ * 64), (sizeof(T) == 2 ? (!std::is_void<TS>::v
       pre_mv = m_base[__umul24(kc, m_stride)];   // both below 2^15
     }
   };
+  // all loads, in a form that the compiler counts by (it knows nothing of the direct-to-LDS loads)
+  auto landed = [] {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0)
+    asm volatile("" ::: "memory");
+  };
   auto stash = [&](int tile) {
     const int buf = tile & 1;
     const int key0 = tile * kKeyTile;
     const bool tail = MK != kMaskNone && key0 + kKeyTile > nk;   // uniform (kMaskNone: whole tiles only)
-    if constexpr (kDirect) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // (nothing younger than the tile's loads is under way)
+    if constexpr (kDirect) landed();
     if (!kDirect || tail) {
 #pragma unroll
       for (int j = 0; j < FPW; ++j) {
@@ -391,12 +401,14 @@ __global__ __launch_bounds__((NWQ * 64), (sizeof(T) == 2 ? (!std::is_void<TS>::v
   };
 
   // ---- per-wave bias tile: lane <-> query, [u][c] = keys key0 + 32g + 16u + 8c .. +7 ----
+  auto fetch_bias_half = [&](int tile, int u, V8 (&dst)[2]) {
+    const T* bp = b_tiles + (int64_t)min(tile, n_tiles - 1) * kAttnTileElems + u * 1024;
+#pragma unroll
+    for (int c = 0; c < 2; ++c) dst[c] = load8<T>(bp + c * 512);
+  };
   auto fetch_bias = [&](int tile, V8 (&dst)[2][2]) {
-    const T* bp = b_tiles + (int64_t)min(tile, n_tiles - 1) * kAttnTileElems;
 #pragma unroll
-    for (int u = 0; u < 2; ++u)
-#pragma unroll
-      for (int c = 0; c < 2; ++c) dst[u][c] = load8<T>(bp + (u * 2 + c) * 512);
+    for (int u = 0; u < 2; ++u) fetch_bias_half(tile, u, dst[u]);
   };
 
   // V^T fragment (u, c) of row r: keys 32g + 16u + 8c .. + 7 of channel lane % 32
@@ -407,15 +419,16 @@ __global__ __launch_bounds__((NWQ * 64), (sizeof(T) == 2 ? (!std::is_void<TS>::v
       return lds_kv[buf][r][4 + u * 2 + c][lane];
   };
   f32x16 acc_o[R];                // O^T per row
-  bool zero_reference = false;    // (uniform) every row's softmax reference is 0
   float m_run[R], l_run[R];       // running max (natural units) and denominator (this lane's keys)
+  auto reset = [&](float reference) {
 #pragma unroll
-  for (int r = 0; r < R; ++r) {
+    for (int r = 0; r < R; ++r) {
 #pragma unroll
-    for (int e = 0; e < 16; ++e) acc_o[r][e] = 0.0f;
-    m_run[r] = -INFINITY;
-    l_run[r] = 0.0f;
-  }
+      for (int e = 0; e < 16; ++e) acc_o[r][e] = 0.0f;
+      m_run[r] = reference;
+      l_run[r] = 0.0f;
+    }
+  };
 
   // One half of a key tile: logits, online softmax, P^T.  `tb` was fetched one tile ago.
   // Complete instantiations, so that the rarer paths share no code with - and cannot be
@@ -552,6 +565,10 @@ __global__ __launch_bounds__((NWQ * 64), (sizeof(T) == 2 ? (!std::is_void<TS>::v
     out.alpha = alpha;
     return true;
   };
+  auto bias_of = [](const V8 (&raw)[2]) {
+    const f32x8 b0 = to_f32(raw[0]), b1 = to_f32(raw[1]);
+    return __builtin_shufflevector(b0, b1, 0, 1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15);
+  };
   auto process_tile = [&](auto tail_tag, int tile, V8 (&tb)[2][2]) {
     constexpr bool LAST_PARTIAL = decltype(tail_tag)::value;   // the one tile with keys beyond n_keys
     const int buf = tile & 1;
@@ -575,54 +592,9 @@ __global__ __launch_bounds__((NWQ * 64), (sizeof(T) == 2 ? (!std::is_void<TS>::v
     for (int u = 0; u < 2; ++u) {
       const bool tail_tile = LAST_PARTIAL && tile_keys < 48 + 16 * u;
       if (LAST_PARTIAL && tile_keys <= 16 * u) continue;
-      auto bias_of = [](const V8 (&raw)[2]) {
-        const f32x8 b0 = to_f32(raw[0]), b1 = to_f32(raw[1]);
-        return __builtin_shufflevector(b0, b1, 0, 1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15);
-      };
-      // The common path of two rows: the reference is 0, no key is left out.  Both rows' logits are formed before the first
-      // row's exponentials, which run under the second row's products (the second takes the bias' registers), and the
-      // second's under the first's P.V (768 tokens 375 -> 363 us, 2048 6315 -> 6160).  What a row does is what half_row's
-      // kOptimisticZero does.  A probability sum out of range leaves this row, and the second one behind it, to the
-      // paths below (r_begin: rows that are done).
-      int r_begin = 0;
-      if constexpr (R == 2 && !has_mask) {
-        if (zero_reference && !tail_tile) {
-          const f32x16 tbf = bias_of(tb[u]);
-          V8 kf[2][2];
-          f32x16 s[2];
-#pragma unroll
-          for (int r = 0; r < 2; ++r)
-#pragma unroll
-            for (int kk = 0; kk < 2; ++kk) kf[r][kk] = lds_kv[buf][r][u * 2 + kk][lane];
-#pragma unroll
-          for (int r = 0; r < 2; ++r) {
-            s[r] = tbf;
-#pragma unroll
-            for (int kk = 0; kk < 2; ++kk) mma32(s[r], kf[r][kk], qf[r][kk]);
-          }
-#pragma unroll
-          for (int r = 0; r < 2; ++r) {
-            if (r_begin != r) break;
-            V8 vf[2], pf[2];
-#pragma unroll
-            for (int c = 0; c < 2; ++c) vf[c] = v_frag(buf, r, u, c);
-#pragma unroll
-            for (int e = 0; e < 16; ++e) s[r][e] = fast_exp2(s[r][e]);
-            const float psum = probabilities(s[r], pf);
-            if ((__builtin_amdgcn_ballot_w64(!(psum < kOptimisticLimit)) & q_ok_mask) != 0ull) break;
-            l_run[r] += psum;
-#pragma unroll
-            for (int c = 0; c < 2; ++c) mma32(acc_o[r], vf[c], pf[c]);
-            r_begin = r + 1;
-          }
-          if (r_begin == 2) continue;
-        }
-        asm volatile("" : "+v"(tb[u][0]), "+v"(tb[u][1]));   // (the bias is converted again: no registers for it on the common path)
-      }
       const f32x16 tbf = bias_of(tb[u]);
 #pragma unroll
       for (int r = 0; r < R; ++r) {
-        if (r < r_begin) continue;
         // the unmasked paths of one half: optimistic against the reference the earlier tiles
         // left, classic if there is none yet or the optimistic one had to give up
         auto unmasked_half = [&](auto ttag, HalfOut& out) -> bool {
@@ -656,17 +628,73 @@ __global__ __launch_bounds__((NWQ * 64), (sizeof(T) == 2 ? (!std::is_void<TS>::v
 #pragma unroll
         for (int c = 0; c < 2; ++c) mma32(acc_o[r], v_frag(buf, r, u, c), out.pf[c]);
       }
-      if constexpr (R == 2 && !has_mask)
-        zero_reference = ((__builtin_amdgcn_ballot_w64(m_run[0] != 0.0f) | __builtin_amdgcn_ballot_w64(m_run[1] != 0.0f)) & q_ok_mask) == 0ull;
     }
     }
   };
+  // The common path (16-bit, no mask): the reference is 0 in all lanes and stays it, and nothing looks at the sums on the way,
+  // so that a tile is one stretch of instructions without a branch.  All rows' logits of a half are formed before the first
+  // row's exponentials, which run under the second row's products, and the second's under the first's P.V.  The bias of the next tile is
+  // requested as soon as this one's is converted: half a step of work or more lies between every load and its wait.  What a
+  // row does is what half_row's kOptimisticZero does, bit for bit.
+  // us per launch, 4 heads, with a check and a branch per row and half / this: n = 128 6.1 / 5.8, 256 20.7 / 20.0, 320 37.5 / 36.5, 352
+  // 52.5 / 46.8, 384 52.5 / 49.2, 387 71.2 / 64.6, 512 113 / 105, 600 216 / 198, 768 369 / 347, 776 434 / 402, 1024 833 / 782, 2048
+  // 6292 / 5966.  What is left at 768 is 402 ns a tile and wave, where the tile's 8 MFMAs and 88 vector instructions alone take 265 ns
+  // at four waves per SIMD (two pipes that overlap by half).  Tried and no better: two chains of dot2; s_setprio
+  // around the logits' products; the next (half, row)'s logits ahead of this one's exponentials (14 spills: 768 353 -> 473).
+  auto fast_tile = [&](auto tail_tag, int tile, V8 (&tb)[2][2]) {
+    constexpr bool TAIL = decltype(tail_tag)::value;
+    const int buf = tile & 1;
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      if (TAIL && nk - tile * kKeyTile <= 16 * u) continue;   // (the half has no keys)
+      f32x16 tbf = bias_of(tb[u]);
+      asm volatile("" : "+v"(tbf) :: "memory");   // (converted before its registers are loaded again)
+      fetch_bias_half(tile + 1, u, tb[u]);
+      asm volatile("" ::: "memory");
+      V8 kf[R][2];
+      f32x16 s[R];
+#pragma unroll
+      for (int r = 0; r < R; ++r)
+#pragma unroll
+        for (int kk = 0; kk < 2; ++kk) kf[r][kk] = lds_kv[buf][r][u * 2 + kk][lane];
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        s[r] = tbf;
+#pragma unroll
+        for (int kk = 0; kk < 2; ++kk) mma32(s[r], kf[r][kk], qf[r][kk]);
+      }
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        V8 pf[2], vf[2];   // (V ahead of the exponentials)
+#pragma unroll
+        for (int c = 0; c < 2; ++c) vf[c] = v_frag(buf, r, u, c);
+        if constexpr (TAIL) {
+          const int kfirst = tile * kKeyTile + 32 * g + 16 * u;   // register e <-> key kfirst + e
+#pragma unroll
+          for (int e = 0; e < 16; ++e) s[r][e] = kfirst + e < nk ? s[r][e] : -INFINITY;
+        }
+#pragma unroll
+        for (int e = 0; e < 16; ++e) s[r][e] = fast_exp2(s[r][e]);
+        l_run[r] += probabilities(s[r], pf);
+#pragma unroll
+        for (int c = 0; c < 2; ++c) mma32(acc_o[r], vf[c], pf[c]);
+      }
+    }
+  };
   // Tile t+1 travels while tile t is processed; its bias tile is requested into the bias registers once tile t has
-  // consumed them, behind the wait for tile t+1.
+  // consumed them, behind the wait for tile t+1 (fast_tile: in mid-tile).
   V8 tbias[2][2];
   auto barrier = [] { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
+  auto start = [&](float reference) {
+    reset(reference);
+    fetch(0);
+    fetch_bias(0, tbias);
+    stash(0);
+    barrier();
+  };
   auto step = [&](auto tail_tag, int tile) {
     const bool more = tile + 1 < n_tiles;
+    if constexpr (kDirect) landed();   // (the bias: ahead of loads that the compiler does not count)
     if (more) fetch(tile + 1);
     process_tile(tail_tag, tile, tbias);
     if (more) {
@@ -675,17 +703,62 @@ __global__ __launch_bounds__((NWQ * 64), (sizeof(T) == 2 ? (!std::is_void<TS>::v
     }
     barrier();
   };
-
-  fetch(0);
-  fetch_bias(0, tbias);
-  stash(0);
-  barrier();
+  auto fast_step = [&](auto tail_tag, int tile) {
+    const bool more = tile + 1 < n_tiles;
+    if (more) fetch(tile + 1);
+    if (q_ok_mask != 0ull) fast_tile(tail_tag, tile, tbias);
+    if (more) stash(tile + 1);
+    landed();   // (the bias)
+  };
   // the tiles whose keys all take part, in a loop that knows nothing of a partial tile (with
   // its tests in the loop every tile was 7 % slower), then the partial one if there is one
   const int n_full = MK == kMaskNone ? n_tiles : nk / kKeyTile;
-  for (int tile = 0; tile < n_full; ++tile) step(std::false_type{}, tile);
+  // The workgroup walks by fast_tile first.  After tile 0 its waves compare: sums that are far from 0 but sound go on from
+  // there in the checked walk, others start again in it (4 % of the launch at 768 tokens, for logits with a deviation of 40);
+  // and sums that left the range that fp32 can be trusted with later on are found at the end (a logit some 57 above zero whose
+  // query had none above 27 in tile 0): that workgroup starts again as well.
+  int first = 0;   // tiles that are done
+  if constexpr (kFast) {
+    // the worst of what the workgroup's waves have to say; also the barrier of a step
+    auto vote = [&](int which, int v) {
+      if (lane == 0) lds_vote[which][wave] = v;
+      barrier();
+      int worst = 0;
+#pragma unroll
+      for (int w = 0; w < NWQ; ++w) worst = max(worst, lds_vote[which][w]);
+      return __builtin_amdgcn_readfirstlane(worst);
+    };
+    auto outside = [&](float lo, float hi) {   // (also a NaN)
+      uint64_t m = 0ull;
+#pragma unroll
+      for (int r = 0; r < R; ++r) m |= __builtin_amdgcn_ballot_w64(!(l_run[r] > lo && l_run[r] < hi));
+      return (m & q_ok_mask) != 0ull;
+    };
+    start(0.0f);
+    if (n_full > 0) {
+      fast_step(std::false_type{}, 0);
+      first = 1;
+      int verdict = vote(0, outside(kTrustedLow, kTrustedHigh) ? 2 : outside(kTrustedLow, kOptimisticLimit) ? 1 : 0);
+      if (verdict == 0) {
+        for (int tile = 1; tile < n_full; ++tile) {
+          fast_step(std::false_type{}, tile);
+          barrier();
+        }
+        if constexpr (MK != kMaskNone) {
+          if (n_full < n_tiles) fast_step(std::true_type{}, n_full);
+        }
+        first = n_tiles;
+        verdict = vote(1, outside(kTrustedLow, kTrustedHigh) ? 2 : 0);
+      }
+      if (verdict == 2) first = 0;
+    }
+    if (first == 0) start(-INFINITY);
+  } else {
+    start(-INFINITY);
+  }
+  for (int tile = first; tile < n_full; ++tile) step(std::false_type{}, tile);
   if constexpr (MK != kMaskNone) {
-    if (n_full < n_tiles) step(std::true_type{}, n_full);
+    if (first < n_tiles && n_full < n_tiles) step(std::true_type{}, n_full);
   }
 
   // ---- normalise, gate, store: lane <-> query, register e <-> d = acc_row(e, g) ----

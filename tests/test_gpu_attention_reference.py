@@ -1,0 +1,56 @@
+"""The triangle-attention core's common path takes every probability against the softmax reference 0 and looks at its sums after
+the first key tile and after the last: logits that its sums can take, that send the workgroup to the checked walk from the second
+tile on, and that make it start again; key ranges of less than a tile, one tile, and one key more."""
+
+import pytest
+import torch
+
+from protenix_amd import _lib
+from test_gpu_attention_rows import _core, _reference
+
+
+def _add(dev_bias, plain_bias, queries, keys, value):
+    """Bias of every one of the queries at every one of the keys, in the core's layout and in the plain one."""
+    qi, j = (t.reshape(-1) for t in torch.meshgrid(torch.as_tensor(queries), torch.as_tensor(keys), indexing="ij"))
+    plain_bias[:, qi, j] += value
+    dev_bias[:, qi // 32, j // 64, (j % 32) // 16, (j % 16) // 8, (j % 64) // 32, qi % 32, j % 8] = plain_bias[:, qi, j]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [65, 130, 353, 1057])
+@pytest.mark.parametrize("where", ["first", "last", "all"])
+# log2 units: sums up to 1e12 = 2^40 stay, up to 1e25 = 2^83 leave after the first tile, beyond (2^128: infinity) start again
+@pytest.mark.parametrize("value", [30.0, 60.0, 100.0, 200.0, -100.0])
+def test_logits_away_from_zero(n, where, value):
+    lib, heads = _lib.load(), 1
+    g = torch.Generator().manual_seed(n)
+    (q, kd, vd, bd), (pq, pk, pv, pb), pitch = _core(n, heads, 1.0, g)
+    keys = range(n) if where == "all" else [5 if where == "first" else n - 1]
+    _add(bd, pb, range(n) if n < 200 else [37, 38], keys, value)
+    dq, dk, dv, db = (t.cuda() for t in (q, kd, vd, bd))
+    st = torch.cuda.current_stream().cuda_stream
+    o = torch.full((heads, n, n, 32), 7.0, dtype=torch.bfloat16, device="cuda")
+    assert lib.ptx_triattn_fwd(dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), None, db.data_ptr(), None, o.data_ptr(), n, heads, 32,
+                               pitch, 0, 1e9, 1, st) == 0
+    o = o.cpu()
+    rows = [0, 1, n // 2, n - 2, n - 1]
+    # (probabilities and outputs are rounded to 8 significant bits: 2^-8 each of a weighted mean of |v| < 5)
+    err = (o[:, rows].float() - _reference(pq, pk, pv, pb, rows, n)).abs().max().item()
+    assert err <= 2 * 2.0 ** -8 * pv.abs().max().item(), (n, where, value, err)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [130, 353, 1057])
+@pytest.mark.parametrize("n_keys", [1, 16, 17, 63, 64, 65, 128, 129])
+def test_few_keys(n, n_keys):
+    lib, heads = _lib.load(), 1
+    g = torch.Generator().manual_seed(n_keys)
+    dev, plain, pitch = _core(n, heads, 1.0, g)
+    dq, dk, dv, db = (t.cuda() for t in dev)
+    st = torch.cuda.current_stream().cuda_stream
+    o = torch.full((heads, n, n, 32), 7.0, dtype=torch.bfloat16, device="cuda")
+    assert lib.ptx_triattn_fwd_rows(dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), None, db.data_ptr(), None, o.data_ptr(), n, heads, 32,
+                                    pitch, 0, 1e9, 0, n, n_keys, 1, st) == 0
+    rows = [0, 1, n // 2, n - 1]
+    err = (o.cpu()[:, rows].float() - _reference(*plain, rows, n_keys)).abs().max().item()
+    assert err <= 2 * 2.0 ** -8 * plain[2].abs().max().item(), (n, n_keys, err)
