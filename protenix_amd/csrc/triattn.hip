@@ -307,7 +307,8 @@ __global__ __launch_bounds__((NWQ * 64), (sizeof(T) == 2 ? (!std::is_void<TS>::v
   // Keys beyond n_keys hold garbage (or, below n, keys that are left out) in K, removed by the -inf mask bias, and
   // are zeroed in V^T (0 * garbage must stay 0).
   constexpr bool kDirect = sizeof(T) == 2;
-  constexpr bool kFast = sizeof(T) == 2 && !has_mask;
+  constexpr bool kFast = sizeof(T) == 2;
+  static_assert(!has_mask || R == 1, "a mask is looked at for one row per workgroup");
   __shared__ int lds_vote[2][kFast ? NWQ : 1];
   constexpr int FPW = 8 * R / NWQ;   // fragments each wave moves per tile, of one operand and row
   static_assert(FPW >= 1 && FPW <= 4, "a wave's fragments are consecutive in memory");
@@ -631,7 +632,7 @@ __global__ __launch_bounds__((NWQ * 64), (sizeof(T) == 2 ? (!std::is_void<TS>::v
     }
     }
   };
-  // The common path (16-bit, no mask): the reference is 0 in all lanes and stays it, and nothing looks at the sums on the way,
+  // The common path (16-bit; tiles without a masked key): the reference is 0 in all lanes and stays it, and nothing looks at the sums on the way,
   // so that a tile is one stretch of instructions without a branch.  All rows' logits of a half are formed before the first
   // row's exponentials, which run under the second row's products, and the second's under the first's P.V.  The bias of the next tile is
   // requested as soon as this one's is converted: half a step of work or more lies between every load and its wait.  What a
@@ -713,7 +714,7 @@ __global__ __launch_bounds__((NWQ * 64), (sizeof(T) == 2 ? (!std::is_void<TS>::v
   // the tiles whose keys all take part, in a loop that knows nothing of a partial tile (with
   // its tests in the loop every tile was 7 % slower), then the partial one if there is one
   const int n_full = MK == kMaskNone ? n_tiles : nk / kKeyTile;
-  // The workgroup walks by fast_tile first.  After tile 0 its waves compare: sums that are far from 0 but sound go on from
+  // The workgroup walks by fast_tile first, up to a masked key.  After tile 0 its waves compare: sums that are far from 0 but sound go on from
   // there in the checked walk, others start again in it (4 % of the launch at 768 tokens, for logits with a deviation of 40);
   // and sums that left the range that fp32 can be trusted with later on are found at the end (a logit some 57 above zero whose
   // query had none above 27 in tile 0): that workgroup starts again as well.
@@ -734,25 +735,37 @@ __global__ __launch_bounds__((NWQ * 64), (sizeof(T) == 2 ? (!std::is_void<TS>::v
       for (int r = 0; r < R; ++r) m |= __builtin_amdgcn_ballot_w64(!(l_run[r] > lo && l_run[r] < hi));
       return (m & q_ok_mask) != 0ull;
     };
+    // a key of the (staged) tile is masked: the same for all waves, whose row is the same
+    auto masked = [&](int tile) { return has_mask && __builtin_amdgcn_ballot_w64(lds_mb[tile & 1][0][lane] != 0.0f) != 0ull; };
     start(0.0f);
-    if (n_full > 0) {
+    int verdict = 0;
+    if (n_full > 0 && !masked(0)) {
       fast_step(std::false_type{}, 0);
       first = 1;
-      int verdict = vote(0, outside(kTrustedLow, kTrustedHigh) ? 2 : outside(kTrustedLow, kOptimisticLimit) ? 1 : 0);
+      verdict = vote(0, outside(kTrustedLow, kTrustedHigh) ? 2 : outside(kTrustedLow, kOptimisticLimit) ? 1 : 0);
       if (verdict == 0) {
-        for (int tile = 1; tile < n_full; ++tile) {
+        int tile = 1;
+        for (; tile < n_full; ++tile) {
+          if (masked(tile)) break;
           fast_step(std::false_type{}, tile);
           barrier();
         }
+        first = has_mask ? tile : n_tiles;
         if constexpr (MK != kMaskNone) {
-          if (n_full < n_tiles) fast_step(std::true_type{}, n_full);
+          if (n_full < n_tiles && (!has_mask || (tile == n_full && !masked(tile)))) {
+            fast_step(std::true_type{}, n_full);
+            first = n_tiles;
+          }
         }
-        first = n_tiles;
         verdict = vote(1, outside(kTrustedLow, kTrustedHigh) ? 2 : 0);
       }
       if (verdict == 2) first = 0;
     }
-    if (first == 0) start(-INFINITY);
+    if (has_mask && verdict == 0) {
+      if (first == 0) reset(-INFINITY);   // (tile 0 is staged)
+    } else if (first == 0) {
+      start(-INFINITY);
+    }
   } else {
     start(-INFINITY);
   }

@@ -54,3 +54,35 @@ def test_few_keys(n, n_keys):
     rows = [0, 1, n // 2, n - 1]
     err = (o.cpu()[:, rows].float() - _reference(*plain, rows, n_keys)).abs().max().item()
     assert err <= 2 * 2.0 ** -8 * plain[2].abs().max().item(), (n, n_keys, err)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [65, 200, 353])
+@pytest.mark.parametrize("key", [0, 63, 64, 130, 199, 352])
+@pytest.mark.parametrize("value", [0.0, 60.0, 100.0])
+def test_up_to_a_masked_key(n, key, value):
+    """A row leaves the common path where its first masked key is; logits as above, at a key before it and in the last tile."""
+    if key >= n:
+        pytest.skip("no such key")
+    lib, heads = _lib.load(), 1
+    g = torch.Generator().manual_seed(n)
+    (q, kd, vd, bd), (pq, pk, pv, pb), pitch = _core(n, heads, 1.0, g)
+    _add(bd, pb, [37, 38], [5], value)
+    _add(bd, pb, [40], [n - 1 if n - 1 != key else n - 2], value)
+    mask = torch.ones(n, n).bfloat16()
+    mask[:, key] = 0
+    mask[1] = 1                                   # a row without masked keys
+    mask[2, key:] = 0                             # (key = 0: all of them)
+    mask[2, 0] = 1
+    dq, dk, dv, db, dm = (t.cuda() for t in (q, kd, vd, bd, mask))
+    st = torch.cuda.current_stream().cuda_stream
+    o = torch.full((heads, n, n, 32), 7.0, dtype=torch.bfloat16, device="cuda")
+    assert lib.ptx_triattn_fwd(dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), None, db.data_ptr(), dm.data_ptr(), o.data_ptr(), n, heads, 32,
+                               pitch, 0, 1e9, 1, st) == 0
+    o = o.cpu()
+    for row in (0, 1, 2, n - 1):
+        keys = mask[row].bool()
+        ref = _reference(pq, pk[:, :, keys], pv[:, :, keys], pb[:, :, keys], [row], int(keys.sum()))
+        # (as above; the masked path adds ln 2 * (q.k) and the bias in fp32: 1e-6 of a logit of 100)
+        err = (o[:, [row]].float() - ref).abs().max().item()
+        assert err <= 2 * 2.0 ** -8 * pv.abs().max().item(), (n, key, value, row, err)
