@@ -39,7 +39,7 @@ constexpr int kD = 32;          // head dim
 constexpr int kKeyTile = 64;
 constexpr float kLog2e = 1.4426950408889634f;
 // half_row: code paths, and the largest per-lane probability sum of a half tile (16 values) the
-// optimistic path accepts
+// optimistic path accepts (16-bit against the reference 0: kTrustedHigh)
 enum { kOptimistic = 0, kClassic = 1, kMasked = 2, kOptimisticZero = 3 };
 constexpr float kOptimisticLimit = 1.0e12f;
 // fast_tile: this lane's sum of probabilities against the reference 0 that fp32 sums of P and of P V can be trusted with
@@ -420,6 +420,7 @@ __global__ __launch_bounds__((NWQ * 64), (sizeof(T) == 2 ? (!std::is_void<TS>::v
       return lds_kv[buf][r][4 + u * 2 + c][lane];
   };
   f32x16 acc_o[R];                // O^T per row
+  bool fresh = true;              // (uniform over the wave) tile 0 finds no reference
   float m_run[R], l_run[R];       // running max (natural units) and denominator (this lane's keys)
   auto reset = [&](float reference) {
 #pragma unroll
@@ -560,7 +561,8 @@ __global__ __launch_bounds__((NWQ * 64), (sizeof(T) == 2 ? (!std::is_void<TS>::v
     }
     const float psum = probabilities(s, out.pf);
     if constexpr (MODE == kOptimistic || MODE == kOptimisticZero) {
-      if ((__builtin_amdgcn_ballot_w64(!(psum < kOptimisticLimit)) & q_ok_mask) != 0ull) return false;
+      constexpr float limit = kFast && MODE == kOptimisticZero ? kTrustedHigh : kOptimisticLimit;
+      if ((__builtin_amdgcn_ballot_w64(!(psum < limit)) & q_ok_mask) != 0ull) return false;
     }
     out.psum = psum;
     out.alpha = alpha;
@@ -600,7 +602,7 @@ __global__ __launch_bounds__((NWQ * 64), (sizeof(T) == 2 ? (!std::is_void<TS>::v
         // left, classic if there is none yet or the optimistic one had to give up
         auto unmasked_half = [&](auto ttag, HalfOut& out) -> bool {
           bool done = false;
-          if (tile != 0 || u != 0) {
+          if (tile != 0 || u != 0 || !fresh) {
             if ((__builtin_amdgcn_ballot_w64(m_run[r] != 0.0f) & q_ok_mask) == 0ull)
               done = half_row(std::integral_constant<int, kOptimisticZero>{}, ttag, r, buf, u, key0, tb[u], tbf, out);
             else
@@ -714,36 +716,37 @@ __global__ __launch_bounds__((NWQ * 64), (sizeof(T) == 2 ? (!std::is_void<TS>::v
   // the tiles whose keys all take part, in a loop that knows nothing of a partial tile (with
   // its tests in the loop every tile was 7 % slower), then the partial one if there is one
   const int n_full = MK == kMaskNone ? n_tiles : nk / kKeyTile;
-  // The workgroup walks by fast_tile first, up to a masked key.  After tile 0 its waves compare: sums that are far from 0 but sound go on from
-  // there in the checked walk, others start again in it (4 % of the launch at 768 tokens, for logits with a deviation of 40);
-  // and sums that left the range that fp32 can be trusted with later on are found at the end (a logit some 57 above zero whose
-  // query had none above 27 in tile 0): that workgroup starts again as well.
+  // The workgroup walks by fast_tile first, up to a masked key.  After tile 0 and at the end its waves compare: if a sum of one
+  // left the range that fp32 can be trusted with (a logit some 57 above or below zero), the workgroup starts again in the checked
+  // walk (at 768 tokens 3 % of the launch if all find out after tile 0).  There the other waves keep the reference 0, as long as
+  // they can: what a wave computes does not depend on who shares its workgroup.
   int first = 0;   // tiles that are done
   if constexpr (kFast) {
-    // the worst of what the workgroup's waves have to say; also the barrier of a step
-    auto vote = [&](int which, int v) {
+    // whether it holds for one of the workgroup's waves; also the barrier of a step
+    auto vote = [&](int which, bool v) {
       if (lane == 0) lds_vote[which][wave] = v;
       barrier();
-      int worst = 0;
+      int any = 0;
 #pragma unroll
-      for (int w = 0; w < NWQ; ++w) worst = max(worst, lds_vote[which][w]);
-      return __builtin_amdgcn_readfirstlane(worst);
+      for (int w = 0; w < NWQ; ++w) any |= lds_vote[which][w];
+      return __builtin_amdgcn_readfirstlane(any) != 0;
     };
-    auto outside = [&](float lo, float hi) {   // (also a NaN)
+    auto outside = [&] {   // (also a NaN)
       uint64_t m = 0ull;
 #pragma unroll
-      for (int r = 0; r < R; ++r) m |= __builtin_amdgcn_ballot_w64(!(l_run[r] > lo && l_run[r] < hi));
+      for (int r = 0; r < R; ++r) m |= __builtin_amdgcn_ballot_w64(!(l_run[r] > kTrustedLow && l_run[r] < kTrustedHigh));
       return (m & q_ok_mask) != 0ull;
     };
     // a key of the (staged) tile is masked: the same for all waves, whose row is the same
     auto masked = [&](int tile) { return has_mask && __builtin_amdgcn_ballot_w64(lds_mb[tile & 1][0][lane] != 0.0f) != 0ull; };
     start(0.0f);
-    int verdict = 0;
+    bool again = false;
     if (n_full > 0 && !masked(0)) {
       fast_step(std::false_type{}, 0);
       first = 1;
-      verdict = vote(0, outside(kTrustedLow, kTrustedHigh) ? 2 : outside(kTrustedLow, kOptimisticLimit) ? 1 : 0);
-      if (verdict == 0) {
+      fresh = outside();
+      again = vote(0, fresh);
+      if (!again) {
         int tile = 1;
         for (; tile < n_full; ++tile) {
           if (masked(tile)) break;
@@ -752,19 +755,20 @@ __global__ __launch_bounds__((NWQ * 64), (sizeof(T) == 2 ? (!std::is_void<TS>::v
         }
         first = has_mask ? tile : n_tiles;
         if constexpr (MK != kMaskNone) {
-          if (n_full < n_tiles && (!has_mask || (tile == n_full && !masked(tile)))) {
+          if (n_full < n_tiles && (!has_mask || (tile == n_full && !masked(n_full)))) {
             fast_step(std::true_type{}, n_full);
             first = n_tiles;
           }
         }
-        verdict = vote(1, outside(kTrustedLow, kTrustedHigh) ? 2 : 0);
+        fresh = outside();
+        again = vote(1, fresh);
       }
-      if (verdict == 2) first = 0;
+      if (again) first = 0;
     }
-    if (has_mask && verdict == 0) {
+    if (has_mask && !again) {
       if (first == 0) reset(-INFINITY);   // (tile 0 is staged)
     } else if (first == 0) {
-      start(-INFINITY);
+      start(fresh ? -INFINITY : 0.0f);
     }
   } else {
     start(-INFINITY);
@@ -812,7 +816,7 @@ __global__ __launch_bounds__((NWQ * 64), (sizeof(T) == 2 ? (!std::is_void<TS>::v
   }
 }
 
-constexpr int kTwoRowsFrom = 352;   // (see triattn_fwd_ex)
+constexpr int kTwoRowsFrom = 272;   // (see triattn_fwd_ex)
 
 // Where the core reads standard layouts: with one row per wave (with two, the lanes' addresses take registers that it does not
 // have).
@@ -861,18 +865,16 @@ int triattn_fwd_ex(const T* q, const T* k, const T* vt, const T* g, const T* tri
   }
   // Two rows per wave (16-bit, no mask): the two rows share the query block and with it the bias tile - one load
   // and one conversion per logit for both, half the bias stream from the L2 - at 128 registers, so that four waves
-  // still share a SIMD (with a mask the kernel needs 160 and loses a wave).  Below 352 tokens the pairs of rows leave too few
-  // workgroups.  us per launch, 4 heads, one row (four waves) / two rows (four waves) / two rows (eight): n = 256 23.3 / 24.8 /
-  // 24.6, 320 39.9 / 40.0 / 47.8, 384 63 / 60 / 68, 387 86 / 78 / 83, 448 94 / 89 / 91, 480 128 / 118 / 120, 600 234 / 211 / 223, 768
-  // 395 / 363 / 366, 776 481 / 432 / 474, 1024 895 / 833 / 825, 1100 1215 / 1105 / 1105, 1536 3041 / 2707 / 2680, 2048 7157 / 6418 / 6150.
-  // (Before direct-to-LDS loads and two tiles in LDS instead of three, which made room for four workgroups of four waves per
-  // compute unit, and before two rows' products ran next to each other's exponentials: 384 67, 387 94, 600 233, 768 385, 776
-  // 494, 1024 856, 2048 6410.)
+  // still share a SIMD (with a mask the kernel needs 160 and loses a wave).  Below 272 tokens the pairs of rows leave too few
+  // workgroups.  us per launch, 4 heads, one row / two rows (four waves each): n = 200 17.2 / 17.5, 256 20.9 / 21.1, 288 34.1 / 33.2, 300 36.7 /
+  // 35.0, 320 35.8 / 34.1, 336 44.6 / 40.6, 350 50.7 / 46.4.
   const bool two_rows = sizeof(T) == 2 && !mask && n >= kTwoRowsFrom && row_count >= 2 && !standard;
-  // Eight waves share the staged K / V tiles of long rows: +2 % at n = 768 with one row per wave, even at 1024, -2.6 % at 1536; with
-  // two rows the figures above.  Where 256 queries do not divide n, the waves of a row's last workgroup that have no queries
-  // skip the arithmetic and only help to stage the tiles.
-  const bool wide = sizeof(T) == 2 && (two_rows ? n > 1056 : (n % 256 == 0 && n >= 1536) || n >= 2048);
+  // Eight waves share the staged K / V tiles of long rows.  Two rows: where that leaves no more waves without queries than four do (they
+  // skip the arithmetic and only help to stage the tiles) and the keys fill whole tiles (with a partial one its registers
+  // spill): four / eight 768 338 / 346, 1024 755 / 765, 1100 1001 / 1080, 1200 1346 / 1441, 1280 1475 / 1467, 1536 2509 / 2459, 2048
+  // 5909 / 5775.  One row: +2 % at n = 768, even at 1024, -2.6 % at 1536.
+  const bool wide = sizeof(T) == 2 && (two_rows ? n > 1056 && (n + 127) / 128 % 2 == 0 && n_keys % kKeyTile == 0
+                                                : (n % 256 == 0 && n >= 1536) || n >= 2048);
   const int mk = mask ? kMaskGiven : n_keys % kKeyTile ? kMaskTail : kMaskNone;
   const int n_qtiles = wide ? (n + 255) / 256 : (n + 127) / 128;
   const int R = two_rows ? 2 : 1;
@@ -920,7 +922,7 @@ int triattn_fwd_ex(const T* q, const T* k, const T* vt, const T* g, const T* tri
   } while (0)
   if (two_rows) {
     if constexpr (sizeof(T) == 2) {
-      if (mk == kMaskTail) PTX_ATTN_LAUNCH(2, kMaskTail);
+      if (mk == kMaskTail) PTX_ATTN_LAUNCH_R(2, 4, kMaskTail);
       else PTX_ATTN_LAUNCH(2, kMaskNone);
     }
   } else if (mk == kMaskGiven) {

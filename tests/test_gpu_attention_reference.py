@@ -17,7 +17,7 @@ def _add(dev_bias, plain_bias, queries, keys, value):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("n", [65, 130, 353, 1057])
+@pytest.mark.parametrize("n", [65, 130, 353, 1280])
 @pytest.mark.parametrize("where", ["first", "last", "all"])
 # log2 units: sums up to 1e12 = 2^40 stay, up to 1e25 = 2^83 leave after the first tile, beyond (2^128: infinity) start again
 @pytest.mark.parametrize("value", [30.0, 60.0, 100.0, 200.0, -100.0])
@@ -40,7 +40,7 @@ def test_logits_away_from_zero(n, where, value):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("n", [130, 353, 1057])
+@pytest.mark.parametrize("n", [130, 353, 1280])
 @pytest.mark.parametrize("n_keys", [1, 16, 17, 63, 64, 65, 128, 129])
 def test_few_keys(n, n_keys):
     lib, heads = _lib.load(), 1
