@@ -819,8 +819,10 @@ __global__ __launch_bounds__((NWQ * 64), (sizeof(T) == 2 ? (!std::is_void<TS>::v
 constexpr int kTwoRowsFrom = 272;   // (see triattn_fwd_ex)
 
 // Where the core reads standard layouts: with one row per wave (with two, the lanes' addresses take registers that it does not
-// have).
-bool triattn_fwd_standard(int n, bool masked) { return masked || n < kTwoRowsFrom; }
+// have).  Two rows per wave on repacked operands gain less than the repacking costs.  us, the operator's forward without Bias1, 4 heads,
+// S rows of S positions, repacked / as they are: 352 92 / 65, 384 101 / 73, 512 198 / 144, 640 334 / 298, 768 516 / 474, 1024 1089 / 1072, 1536
+// 3268 / 3273; 64 rows of 384 32 / 19, of 768 58 / 48.
+bool triattn_fwd_standard(int n, bool masked) { return masked || n < 1536; }
 
 // (one row and four waves at those sizes, and workgroups to spare)
 bool triattn_fwd_carries(int n, bool bits16) { return bits16 && n <= 256; }

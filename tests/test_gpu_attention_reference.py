@@ -6,7 +6,7 @@ import pytest
 import torch
 
 from protenix_amd import _lib
-from test_gpu_attention_rows import _core, _reference
+from test_gpu_attention_rows import _core, _reference, test_standard_layouts_equal_the_repacked_operands as _standard_layouts
 
 
 def _add(dev_bias, plain_bias, queries, keys, value):
@@ -86,3 +86,10 @@ def test_up_to_a_masked_key(n, key, value):
         # (as above; the masked path adds ln 2 * (q.k) and the bias in fp32: 1e-6 of a logit of 100)
         err = (o[:, [row]].float() - ref).abs().max().item()
         assert err <= 2 * 2.0 ** -8 * pv.abs().max().item(), (n, key, value, row, err)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,s", [(3, 353), (2, 640), (1, 1535), (2, 1536)])
+def test_operator_without_bias1(rows, s):
+    """Up to 1535 positions the operator's operands are read as they are, beyond they are repacked."""
+    _standard_layouts(rows, s, 2, False)
