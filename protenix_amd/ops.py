@@ -208,10 +208,10 @@ _mask_cache: list = []
 
 # Pair masks of padded batches are m (x) m with the padding at the end: the triangle attention
 # then runs its valid rows over the valid keys without a mask (see triangle_attention).  False
-# hands every mask to the kernels as it is (tests compare the two).  From 352 tokens on, where the unmasked
-# kernel takes two rows per wave; below, the second launch costs what the first one saves (us per update, two launches
-# against the masked kernel: 106 = 106 at N = 320 with 20 padded tokens, 118 against 126 at 352, 170 against 190 at 416 with 50,
-# 189 against 200 at 448; no gain at 352 with 1 padded token and at 384 with 32, whose keys fill whole tiles either way: 134 against 135).
+# hands every mask to the kernels as it is (tests compare the two).  From 352 tokens on; below, the second launch costs about what
+# the first one saves, and a new mask would have to be looked at (350 us; us per update of bf16 rows, two launches against the masked
+# kernel: 88 against 87 at N = 300 with 1 padded token, 86 against 89 with 20, 96 = 96 at 320 with 20, 105 against 111 at 340 with 10,
+# 109 against 118 at 351 with 30).
 # The two differ by the rounding of 16-bit probabilities (a relative 2e-3 of the update): the masked kernel moves the softmax reference to
 # the running maximum in a row's last tiles, the valid rows' does not.
 prefix_mask_enabled = True
