@@ -550,7 +550,8 @@ __global__ __launch_bounds__((NWQ * 64), (sizeof(T) == 2 ? (!std::is_void<TS>::v
 #pragma unroll
       for (int e = 0; e < 16; ++e) s[e] = fast_exp2(s[e]);
     } else if constexpr (!MASKED) {
-      const float nml = -m_run[r] * kLog2e;
+      // (as below: no key with a finite logit yet)
+      const float nml = -fmaxf(m_run[r], -2.0e38f) * kLog2e;
 #pragma unroll
       for (int e = 0; e < 16; ++e) s[e] = fast_exp2(s[e] + nml);
     } else {

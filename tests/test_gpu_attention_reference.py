@@ -5,7 +5,10 @@ tile on, and that make it start again; key ranges of less than a tile, one tile,
 import pytest
 import torch
 
+import protenix_amd as P
+from oracle import pairformer_oracle as O
 from protenix_amd import _lib
+from tests.util import rel_err, tol
 from test_gpu_attention_rows import _core, _reference, test_standard_layouts_equal_the_repacked_operands as _standard_layouts
 
 
@@ -93,3 +96,39 @@ def test_up_to_a_masked_key(n, key, value):
 def test_operator_without_bias1(rows, s):
     """Up to 1535 positions the operator's operands are read as they are, beyond they are repacked."""
     _standard_layouts(rows, s, 2, False)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [40, 65, 130, 353])
+@pytest.mark.parametrize("cut", [16, 32, 64, 128])
+def test_first_keys_at_minus_infinity(n, cut):
+    """A bias of -inf has weight zero also where a query has no other key in its first half tile, or first tiles."""
+    if cut >= n:
+        pytest.skip("no key left")
+    lib, heads = _lib.load(), 1
+    g = torch.Generator().manual_seed(n)
+    (q, kd, vd, bd), (pq, pk, pv, pb), pitch = _core(n, heads, 1.0, g)
+    _add(bd, pb, [0, 3, 37], range(cut), -float("inf"))
+    _add(bd, pb, [5], [j for j in range(n) if j % 32 < 16], -float("inf"))       # the first half of every tile
+    dq, dk, dv, db = (t.cuda() for t in (q, kd, vd, bd))
+    st = torch.cuda.current_stream().cuda_stream
+    o = torch.full((heads, n, n, 32), 7.0, dtype=torch.bfloat16, device="cuda")
+    assert lib.ptx_triattn_fwd(dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), None, db.data_ptr(), None, o.data_ptr(), n, heads, 32,
+                               pitch, 0, 1e9, 1, st) == 0
+    rows = [0, n // 2, n - 1]
+    # (as above; the reference's softmax gives such keys weight zero)
+    err = (o.cpu()[:, rows].float() - _reference(pq, pk, pv, pb, rows, n)).abs()
+    assert bool((err <= 2 * 2.0 ** -8 * pv.abs().max()).all()), (n, cut, err.max().item())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("s", [40, 200])
+def test_first_keys_at_minus_infinity_in_full_precision(s):
+    g = torch.Generator().manual_seed(s)
+    q, k, v = (torch.randn(1, 3, s, 2, 32, generator=g) for _ in range(3))
+    b1, b2 = torch.zeros(1, 3, 1, 1, s), torch.randn(1, 1, 2, s, s, generator=g)
+    q = q / 32 ** 0.5
+    b2[..., 3, torch.arange(s) % 32 < 16] = -float("inf")        # the first half of every tile
+    got = P.TriAttentionFunction.apply(*(t.cuda() for t in (q, k, v, b1, b2))).cpu()
+    want = O.softmax_attention(*(t.transpose(-2, -3) for t in (q, k, v)), [b1, b2]).transpose(-2, -3)
+    assert rel_err(got, want) <= tol(torch.float32)
