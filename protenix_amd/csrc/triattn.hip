@@ -39,13 +39,13 @@ constexpr int kD = 32;          // head dim
 constexpr int kKeyTile = 64;
 constexpr float kLog2e = 1.4426950408889634f;
 // half_row: code paths, and the largest per-lane probability sum of a half tile (16 values) the
-// optimistic path accepts (16-bit against the reference 0: kTrustedHigh)
+// optimistic paths accept
 enum { kOptimistic = 0, kClassic = 1, kMasked = 2, kOptimisticZero = 3 };
 constexpr float kOptimisticLimit = 1.0e12f;
-// fast_tile: this lane's sum of probabilities against the reference 0 that fp32 sums of P and of P V can be trusted with
-// (bf16 has fp32's exponents; error against 64 bits of logits with a deviation of 4.0: 1.888e-3, with the maximum as reference 1.879e-3)
-constexpr float kTrustedLow = 1.0e-25f, kTrustedHigh = 1.0e25f;
 constexpr float kLn2 = 0.6931471805599453f;
+// fast_tile: sums of a lane's first 16 probabilities against the reference 0 for which kClassic is sure to choose that reference
+// as well: the largest logit lies within 14 of 0 if the sum is below e^14 and above 16 e^-14, with a margin for rounding.
+constexpr float kNearZeroLow = 2.0e-5f, kNearZeroHigh = 1.0e6f;
 // kClassic: a running maximum no larger than this (natural units, all lanes of the wave) is
 // replaced by the reference 0, which makes exp2() of the raw logit the probability
 constexpr float kZeroReferenceLimit = 14.0f;
@@ -280,15 +280,15 @@ __global__ __launch_bounds__((NWQ * 64), (sizeof(T) == 2 ? (!std::is_void<TS>::v
   // wave takes (and with it the rounding of its valid queries) never depends on that content.
   const bool q_ok = q0 + ln < n;
   // (as a lane mask: wave-wide decisions are ballots of the condition alone, combined with this
-  // mask on the scalar unit)
-  const uint64_t q_ok_mask = __builtin_amdgcn_ballot_w64(q_ok);
+  // mask on the scalar unit; a wave with none only helps to stage)
+  uint64_t q_ok_mask = __builtin_amdgcn_ballot_w64(q_ok);
 
   // Q fragments (B operand): lane <-> query, slots <-> d = 16*kk + 8*g + t
   V8 qf[R][2];
   int64_t qrow[R];                       // head-major q / gate / o row of this lane's query
 #pragma unroll
   for (int r = 0; r < R; ++r) {
-    qrow[r] = h * ax.sh + min(i0 + r, n_rows - 1) * ax.si + qi * ax.sj;
+    qrow[r] = h * ax.sh + min(i0 + r, ax.row_end - 1) * ax.si + qi * ax.sj;
 #pragma unroll
     for (int kk = 0; kk < 2; ++kk) {
       qf[r][kk] = load8<T>(q + qrow[r] + 16 * kk + 8 * g);
@@ -315,8 +315,8 @@ __global__ __launch_bounds__((NWQ * 64), (sizeof(T) == 2 ? (!std::is_void<TS>::v
   static_assert(FPW >= 1 && FPW <= 4, "a wave's fragments are consecutive in memory");
   const int fid0 = wave * FPW, fr = fid0 >> 3, f0 = fid0 & 7;   // row, first fragment
   static_assert(!STD || kDirect, "standard layouts: 16-bit");
-  const T* const kv_base = STD ? (f0 < 4 ? k : vt) + h * ax.sh + min(i0 + fr, n_rows - 1) * ax.si
-                               : (f0 < 4 ? k : vt) + ((int64_t)h * n_rows + min(i0 + fr, n_rows - 1)) * key_tiles * kAttnTileElems + (f0 & 3) * 512;
+  const T* const kv_base = STD ? (f0 < 4 ? k : vt) + h * ax.sh + min(i0 + fr, ax.row_end - 1) * ax.si
+                               : (f0 < 4 ? k : vt) + ((int64_t)h * n_rows + min(i0 + fr, ax.row_end - 1)) * key_tiles * kAttnTileElems + (f0 & 3) * 512;
   // STD: this lane's key within the tile and its channels, of the wave's fragment j
   auto std_place = [&](int j, int& key, int& d) {
     const int f = (f0 + j) & 3;
@@ -332,7 +332,7 @@ __global__ __launch_bounds__((NWQ * 64), (sizeof(T) == 2 ? (!std::is_void<TS>::v
   V8 pre[kDirect ? 1 : FPW];
   T pre_mv;
   // mask value of key kc for this wave's row: m_base[kc * m_stride]
-  const int m_row = min(i0 + min(wave, R - 1), n_rows - 1);
+  const int m_row = min(i0 + min(wave, R - 1), ax.row_end - 1);
   const unsigned m_stride = mask_transposed ? n : 1;
   const T* m_base = has_mask ? mask + (mask_transposed ? (int64_t)m_row : (int64_t)m_row * n) : nullptr;
   auto fetch = [&](int tile) {
@@ -421,7 +421,6 @@ __global__ __launch_bounds__((NWQ * 64), (sizeof(T) == 2 ? (!std::is_void<TS>::v
       return lds_kv[buf][r][4 + u * 2 + c][lane];
   };
   f32x16 acc_o[R];                // O^T per row
-  bool fresh = true;              // (uniform over the wave) tile 0 finds no reference
   float m_run[R], l_run[R];       // running max (natural units) and denominator (this lane's keys)
   auto reset = [&](float reference) {
 #pragma unroll
@@ -563,8 +562,7 @@ __global__ __launch_bounds__((NWQ * 64), (sizeof(T) == 2 ? (!std::is_void<TS>::v
     }
     const float psum = probabilities(s, out.pf);
     if constexpr (MODE == kOptimistic || MODE == kOptimisticZero) {
-      constexpr float limit = kFast && MODE == kOptimisticZero ? kTrustedHigh : kOptimisticLimit;
-      if ((__builtin_amdgcn_ballot_w64(!(psum < limit)) & q_ok_mask) != 0ull) return false;
+      if ((__builtin_amdgcn_ballot_w64(!(psum < kOptimisticLimit)) & q_ok_mask) != 0ull) return false;
     }
     out.psum = psum;
     out.alpha = alpha;
@@ -604,7 +602,7 @@ __global__ __launch_bounds__((NWQ * 64), (sizeof(T) == 2 ? (!std::is_void<TS>::v
         // left, classic if there is none yet or the optimistic one had to give up
         auto unmasked_half = [&](auto ttag, HalfOut& out) -> bool {
           bool done = false;
-          if (tile != 0 || u != 0 || !fresh) {
+          if (tile != 0 || u != 0) {
             if ((__builtin_amdgcn_ballot_w64(m_run[r] != 0.0f) & q_ok_mask) == 0ull)
               done = half_row(std::integral_constant<int, kOptimisticZero>{}, ttag, r, buf, u, key0, tb[u], tbf, out);
             else
@@ -636,22 +634,32 @@ __global__ __launch_bounds__((NWQ * 64), (sizeof(T) == 2 ? (!std::is_void<TS>::v
     }
     }
   };
+  // whether the sums of all this wave's rows and queries lie in a range (a NaN does not)
+  auto all_between = [&](float low, float high) {
+    uint64_t out = 0ull;
+#pragma unroll
+    for (int r = 0; r < R; ++r) out |= __builtin_amdgcn_ballot_w64(!(l_run[r] > low && l_run[r] < high));
+    return (out & q_ok_mask) == 0ull;
+  };
   // The common path (16-bit; tiles without a masked key): the reference is 0 in all lanes and stays it, and nothing looks at the sums on the way,
   // so that a tile is one stretch of instructions without a branch.  All rows' logits of a half are formed before the first
   // row's exponentials, which run under the second row's products, and the second's under the first's P.V.  The bias of the next tile is
   // requested as soon as this one's is converted: half a step of work or more lies between every load and its wait.  What a
   // row does is what half_row's kOptimisticZero does, bit for bit.
-  // us per launch, 4 heads, with a check and a branch per row and half / this: n = 128 6.1 / 5.8, 256 20.7 / 20.0, 320 37.5 / 36.5, 352
-  // 52.5 / 46.8, 384 52.5 / 49.2, 387 71.2 / 64.6, 512 113 / 105, 600 216 / 198, 768 369 / 347, 776 434 / 402, 1024 833 / 782, 2048
-  // 6292 / 5966.  What is left at 768 is 402 ns a tile and wave, where the tile's 8 MFMAs and 88 vector instructions alone take 265 ns
+  // us per launch, 4 heads, with a check and a branch per row and half / this: n = 128 6.1 / 5.9, 256 22.4 / 22.1, 272 34.6 / 31.3, 384
+  // 55.6 / 51.8, 387 74.6 / 68.0, 600 224 / 203, 768 381 / 358, 1024 859 / 803, 1280 1642 / 1551, 2048
+  // 6558 / 6107.  What is left at 768 is 402 ns a tile and wave, where the tile's 8 MFMAs and 88 vector instructions alone take 265 ns
   // at four waves per SIMD (two pipes that overlap by half).  Tried and no better: two chains of dot2; s_setprio
   // around the logits' products; the next (half, row)'s logits ahead of this one's exponentials (14 spills: 768 353 -> 473).
-  auto fast_tile = [&](auto tail_tag, int tile, V8 (&tb)[2][2]) {
-    constexpr bool TAIL = decltype(tail_tag)::value;
+  // `first_tag`: tile 0.  Returns false, after its first half, where that leaves a row a reference other than 0.
+  auto fast_tile = [&](auto tail_tag, auto first_tag, int tile, V8 (&tb)[2][2]) -> bool {
+    constexpr bool TAIL = decltype(tail_tag)::value, FIRST = decltype(first_tag)::value;
     const int buf = tile & 1;
+    bool near_zero = true;
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
       if (TAIL && nk - tile * kKeyTile <= 16 * u) continue;   // (the half has no keys)
+      if (FIRST && !near_zero) continue;
       f32x16 tbf = bias_of(tb[u]);
       asm volatile("" : "+v"(tbf) :: "memory");   // (converted before its registers are loaded again)
       fetch_bias_half(tile + 1, u, tb[u]);
@@ -684,14 +692,17 @@ __global__ __launch_bounds__((NWQ * 64), (sizeof(T) == 2 ? (!std::is_void<TS>::v
 #pragma unroll
         for (int c = 0; c < 2; ++c) mma32(acc_o[r], vf[c], pf[c]);
       }
+      if constexpr (FIRST) {
+        if (u == 0) near_zero = all_between(kNearZeroLow, kNearZeroHigh);
+      }
     }
+    return near_zero;
   };
   // Tile t+1 travels while tile t is processed; its bias tile is requested into the bias registers once tile t has
   // consumed them, behind the wait for tile t+1 (fast_tile: in mid-tile).
   V8 tbias[2][2];
   auto barrier = [] { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
-  auto start = [&](float reference) {
-    reset(reference);
+  auto start = [&] {
     fetch(0);
     fetch_bias(0, tbias);
     stash(0);
@@ -708,74 +719,74 @@ __global__ __launch_bounds__((NWQ * 64), (sizeof(T) == 2 ? (!std::is_void<TS>::v
     }
     barrier();
   };
-  auto fast_step = [&](auto tail_tag, int tile) {
+  auto fast_step = [&](auto tail_tag, auto first_tag, int tile) -> bool {
     const bool more = tile + 1 < n_tiles;
     if (more) fetch(tile + 1);
-    if (q_ok_mask != 0ull) fast_tile(tail_tag, tile, tbias);
+    const bool near_zero = q_ok_mask == 0ull || fast_tile(tail_tag, first_tag, tile, tbias);
     if (more) stash(tile + 1);
     landed();   // (the bias)
+    return near_zero;
   };
   // the tiles whose keys all take part, in a loop that knows nothing of a partial tile (with
   // its tests in the loop every tile was 7 % slower), then the partial one if there is one
   const int n_full = MK == kMaskNone ? n_tiles : nk / kKeyTile;
-  // The workgroup walks by fast_tile first, up to a masked key.  After tile 0 and at the end its waves compare: if a sum of one
-  // left the range that fp32 can be trusted with (a logit some 57 above or below zero), the workgroup starts again in the checked
-  // walk (at 768 tokens 3 % of the launch if all find out after tile 0).  There the other waves keep the reference 0, as long as
-  // they can: what a wave computes does not depend on who shares its workgroup.
+  // What process_tile makes of a row is what counts: it depends on that row's 32 queries alone, and fast_tile does the same, bit for bit,
+  // as long as the row keeps the reference 0.  A workgroup whose rows all take it in their first half tile walks by
+  // fast_tile, up to a masked key, any other by process_tile from tile 0 on.  That no sum has reached the limit at which half_row
+  // would have left the reference 0 is looked at where the fast walk ends; waves with such a sum start again by process_tile.
+  // us per launch, 768 tokens, 4 heads, with the checks of process_tile throughout / so: logits with a deviation of 1.2 381 / 358; of 4
+  // 412 / 431, 8 425 / 445, 12 442 / 457, 40 561 / 575 (tile 0 twice); a logit of 41 (the limit is some 27) that first appears in the
+  // last tile, for every query 406 / 713 (everything twice), for one in each 128 397 / 543.  Tried: the checks in fast_tile, ahead of
+  // each half's P.V: such logits 380, all others 4 % longer; a look in every fourth tile: all 1 % longer.
   int first = 0;   // tiles that are done
+  reset(-INFINITY);
+  start();
   if constexpr (kFast) {
     // whether it holds for one of the workgroup's waves; also the barrier of a step
     auto vote = [&](int which, bool v) {
-      if (lane == 0) lds_vote[which][wave] = v;
+      lds_vote[which][wave] = v;   // (the same from all lanes)
       barrier();
       int any = 0;
 #pragma unroll
       for (int w = 0; w < NWQ; ++w) any |= lds_vote[which][w];
       return __builtin_amdgcn_readfirstlane(any) != 0;
     };
-    auto outside = [&] {   // (also a NaN)
-      uint64_t m = 0ull;
-#pragma unroll
-      for (int r = 0; r < R; ++r) m |= __builtin_amdgcn_ballot_w64(!(l_run[r] > kTrustedLow && l_run[r] < kTrustedHigh));
-      return (m & q_ok_mask) != 0ull;
-    };
     // a key of the (staged) tile is masked: the same for all waves, whose row is the same
     auto masked = [&](int tile) { return has_mask && __builtin_amdgcn_ballot_w64(lds_mb[tile & 1][0][lane] != 0.0f) != 0ull; };
-    start(0.0f);
+    const std::false_type no;
+    const std::true_type yes;
     bool again = false;
     if (n_full > 0 && !masked(0)) {
-      fast_step(std::false_type{}, 0);
+      again = vote(0, !fast_step(no, yes, 0));
       first = 1;
-      fresh = outside();
-      again = vote(0, fresh);
       if (!again) {
         int tile = 1;
         for (; tile < n_full; ++tile) {
           if (masked(tile)) break;
-          fast_step(std::false_type{}, tile);
+          fast_step(no, no, tile);
           barrier();
         }
         first = has_mask ? tile : n_tiles;
         if constexpr (MK != kMaskNone) {
           if (n_full < n_tiles && (!has_mask || (tile == n_full && !masked(n_full)))) {
-            fast_step(std::true_type{}, n_full);
+            fast_step(yes, no, n_full);
             first = n_tiles;
           }
         }
-        fresh = outside();
-        again = vote(1, fresh);
+        const bool out = !all_between(0.0f, kOptimisticLimit);
+        again = vote(1, out);
+        if (again && !out && first == n_tiles) q_ok_mask = 0ull;   // (done: in the second walk it only helps to stage)
       }
-      if (again) first = 0;
     }
-    if (MK != kMaskNone && R == 1 && !again) {
-      // tile 0 is staged (without a mask too, where less than a tile of keys leaves nothing to fast_tile: staged a second time
-      // 33, 48 and 63 tokens took 4.8, 4.7 and 4.9 us in place of 4.4, 4.5 and 4.6; with two rows per wave this form spills)
-      if (first == 0) reset(-INFINITY);
-    } else if (first == 0) {
-      start(fresh ? -INFINITY : 0.0f);
+    if (again) {
+      first = 0;
+      if (q_ok_mask != 0ull) reset(-INFINITY);
+      start();
     }
-  } else {
-    start(-INFINITY);
+    if (first > 0 || (again && q_ok_mask == 0ull)) {
+#pragma unroll
+      for (int r = 0; r < R; ++r) m_run[r] = 0.0f;
+    }
   }
   for (int tile = first; tile < n_full; ++tile) step(std::false_type{}, tile);
   if constexpr (MK != kMaskNone) {
@@ -789,7 +800,7 @@ __global__ __launch_bounds__((NWQ * 64), (sizeof(T) == 2 ? (!std::is_void<TS>::v
   int qi_again = qi;
   asm volatile("" : "+v"(qi_again));
 #pragma unroll
-  for (int r = 0; r < R; ++r) qrow[r] = h * ax.sh + min(i0 + r, n_rows - 1) * ax.si + qi_again * ax.sj;
+  for (int r = 0; r < R; ++r) qrow[r] = h * ax.sh + min(i0 + r, ax.row_end - 1) * ax.si + qi_again * ax.sj;
   f32x4 gv[R][4];
 #pragma unroll
   for (int r = 0; r < R; ++r)

@@ -132,3 +132,76 @@ def test_first_keys_at_minus_infinity_in_full_precision(s):
     got = P.TriAttentionFunction.apply(*(t.cuda() for t in (q, k, v, b1, b2))).cpu()
     want = O.softmax_attention(*(t.transpose(-2, -3) for t in (q, k, v)), [b1, b2]).transpose(-2, -3)
     assert rel_err(got, want) <= tol(torch.float32)
+
+
+def _rows(lib, dev, n, heads, pitch, row0, count, n_keys=None, o=None):
+    o = torch.full((heads, n, n, 32), 7.0, dtype=torch.bfloat16, device="cuda") if o is None else o
+    q, k, v, b = dev
+    assert lib.ptx_triattn_fwd_rows(q.data_ptr(), k.data_ptr(), v.data_ptr(), None, b.data_ptr(), None, o.data_ptr(), n, heads, 32, pitch,
+                                    0, 1e9, row0, count, n_keys or n, 1, torch.cuda.current_stream().cuda_stream) == 0
+    return o
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [130, 271, 272, 273, 353, 1152, 1280])
+@pytest.mark.parametrize("q_scale", [0.5, 1.0, 2.0, 4.0])
+def test_a_row_has_the_same_bits_in_any_company(n, q_scale):
+    """Rows by themselves and in a launch of all, whose workgroups take one or two of them, four or eight waves: logits that leave
+    the reference 0 in the first half tile of some rows, in later tiles of others, and rows that never do."""
+    lib, heads = _lib.load(), 1
+    g = torch.Generator().manual_seed(n)
+    (q, kd, vd, bd), (pq, pk, pv, pb), pitch = _core(n, heads, 1.0, g)
+    q = q.float()
+    q[:, ::3] *= q_scale
+    q[:, 1::5] *= 0.25
+    _add(bd, pb, [37], [n - 1], 45.0)                      # (log2 units) beyond the limit in the last tile
+    _add(bd, pb, [70], [64], 120.0)
+    dev = [t.cuda() for t in (q.bfloat16(), kd, vd, bd)]
+    whole = _rows(lib, dev, n, heads, pitch, 0, n)
+    assert bool(torch.isfinite(whole).all())
+    for row in sorted({0, 1, 2, 3, n // 2, n // 2 + 1, n - 2, n - 1}):
+        assert torch.equal(_rows(lib, dev, n, heads, pitch, row, 1)[:, row], whole[:, row]), (n, row)
+    pairs_the_other_way = _rows(lib, dev, n, heads, pitch, 1, n - 1)
+    assert torch.equal(pairs_the_other_way[:, 1:], whole[:, 1:])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [272, 353, 1280])
+def test_rows_behind_the_range_do_not_matter(n):
+    """An odd number of rows: the last one's partner in a workgroup of two lies behind the range, whatever is there."""
+    lib, heads = _lib.load(), 1
+    g = torch.Generator().manual_seed(n)
+    dev, _, pitch = _core(n, heads, 1.0, g)
+    dev = [t.cuda() for t in dev]
+    dev[0] = dev[0] * 4                                    # (logits whose sums depend on the reference they are taken against)
+    count = n - 30 + n % 2 - 1
+    assert count % 2 == 1
+    want = _rows(lib, dev, n, heads, pitch, 0, count)
+    for what in (float("nan"), 3.0e38, 50.0):
+        other = [t.clone() for t in dev]
+        other[0][:, count:] = what
+        got = _rows(lib, other, n, heads, pitch, 0, count)
+        assert torch.equal(got[:, :count], want[:, :count]) and bool((got[:, count:] == 7.0).all()), what
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [64, 130, 300, 1280])
+def test_the_largest_probability_is_exact_at_large_logits(n):
+    """From logits of 14 on the reference is the first half tile's maximum, whose probability is 1.  Two keys, at 2^24.125 and
+    2^22.5 (q = 0, so the logits are the bias): against the reference 0 the first would be rounded by 3.0e-3 of itself, the second by
+    1e-4; against the first, the second's 2^-1.625 is rounded by 1e-4.  What is left is the outputs' rounding, 2^-9 at most of
+    each and, over n 32 of them, some 1e-4 on average."""
+    lib, heads = _lib.load(), 1
+    g = torch.Generator().manual_seed(n)
+    (q, kd, vd, bd), (_, _, pv, pb), pitch = _core(n, heads, 0.0, g)
+    _add(bd, pb, range(n), range(n), -60.0)
+    for key, steps in ((5, (84.0, 0.125)), (9, (82.0, 0.5))):       # (each sum is a bf16 number)
+        for step in steps:
+            _add(bd, pb, range(n), [key], step)
+    vd[:, :, 0, 0, 0, 0, :, 5] = 0                         # V of key 5 is 0: half 0, key group 0, lane half 0
+    dev = [t.cuda() for t in (torch.zeros_like(q), kd, vd, bd)]
+    o = _rows(lib, dev, n, heads, pitch, 0, n).cpu().double()
+    v9 = pv[:, :, 9].double()                              # [head][row][channel]
+    ratio = (o / v9[:, :, None]).mean().item()
+    want = 1.0 / (1.0 + 2.0 ** 1.625)
+    assert abs(ratio / want - 1.0) <= 5e-4, ratio / want - 1.0
