@@ -1,5 +1,5 @@
-"""Rows of the attention core whose keys are all masked (the padded rows of a batch, as a range of rows): the mean of V where
-q.k and the bias drown in the mask, the masked path where they might not.  The reference is the same kernel over all rows
+"""Rows of the attention core whose keys are all masked (the padded rows of a batch, as the last rows of more than 256): the mean of V
+where q.k and the bias drown in the mask, the masked path where they might not.  The reference is the same kernel over all rows
 (ptx_triattn_fwd), which takes the masked path for every row (layers.py:286-291: (q.k + mask bias) + triangle bias in fp32)."""
 import pytest
 import torch
@@ -48,7 +48,8 @@ REL = 2.0 ** -8
 
 
 @pytest.mark.parametrize("transposed", [0, 1])
-@pytest.mark.parametrize("n,nv", [(2, 1), (31, 30), (33, 32), (64, 40), (65, 1), (97, 90), (129, 128), (200, 199), (257, 250), (385, 353),
+@pytest.mark.parametrize("n,nv", [(2, 1), (31, 30), (33, 32), (64, 40), (65, 1), (97, 90), (129, 128), (200, 199), (256, 250), (257, 250), (258, 257),
+                                  (289, 256), (385, 353),
                                   (1536, 1530), (2049, 2048)])
 def test_mean_of_v(n, nv, transposed):
     ops = _operands(n, n)
@@ -57,7 +58,7 @@ def test_mean_of_v(n, nv, transposed):
     assert (rows == rows[:, :, :1]).all()                       # every query alike
 
 
-@pytest.mark.parametrize("n,nv", [(64, 40), (97, 90), (300, 290)])
+@pytest.mark.parametrize("n,nv", [(64, 40), (97, 90), (257, 250), (300, 290)])
 def test_rows_that_are_not_uniform_take_the_masked_path(n, nv):
     """Bit for bit what the whole launch gives: logits or biases that the mask does not swallow, a key that is not masked."""
     q, k, vt, tb = _operands(n, n + 1)
@@ -67,11 +68,13 @@ def test_rows_that_are_not_uniform_take_the_masked_path(n, nv):
     whole, rows = _both(n, nv, big, k, vt, tb, mask)
     assert torch.equal(rows[1, 0], whole[1, 0])
     assert (rows - whole).abs().max() <= REL * whole.abs().max()
-    open_ = mask.clone()
-    open_[n - 1, 3] = 1                                          # the last row has a key
-    whole, rows = _both(n, nv, q, k, vt, tb, open_)
-    assert torch.equal(rows[:, -1], whole[:, -1])
-    assert (rows - whole).abs().max() <= REL * whole.abs().max()
+    for row in (n - 1, nv):                                      # the last row, or the first, has a key
+        for key in (0, 3):
+            open_ = mask.clone()
+            open_[row, key] = 1
+            whole, rows = _both(n, nv, q, k, vt, tb, open_)
+            assert torch.equal(rows[:, row - nv], whole[:, row - nv])
+            assert (rows - whole).abs().max() <= REL * whole.abs().max()
     for value in (1000.0, -float("inf"), float("nan")):          # a bias of head 0, block of queries 0, key 0
         odd = tb.clone()
         odd[0] = value
@@ -85,8 +88,8 @@ def test_rows_that_are_not_uniform_take_the_masked_path(n, nv):
         assert torch.equal(rows.isnan(), whole.isnan())
 
 
-def test_values_that_are_not_numbers_and_gates():
-    n, nv = 70, 60
+@pytest.mark.parametrize("n,nv", [(70, 60), (270, 260)])
+def test_values_that_are_not_numbers_and_gates(n, nv):
     q, k, vt, tb = _operands(n, 5)
     odd = vt.clone()
     odd[: odd.numel() // 2: 40001] = float("nan")
