@@ -849,7 +849,12 @@ __global__ __launch_bounds__(NWQ * 64, 3) void attn_bwd_db2_kernel(BwdParams p) 
   constexpr int kDo = kQ * 32, kK = 2 * kQ * 32, kV = kK + kKeys * 32;               // where they start
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, ln = lane & 31, g = lane >> 5;
   const int s = p.s, H = p.heads;
-  const int slice = blockIdx.x % p.slices, pair = blockIdx.x / p.slices, q_tiles = (s + kQ - 1) / kQ, k_tiles = (s + kKeys - 1) / kKeys;
+  const int q_tiles = (s + kQ - 1) / kQ, k_tiles = (s + kKeys - 1) / kKeys, slice = blockIdx.x % p.slices;
+  // One slice: workgroups in turn put the query tiles on the XCDs in turn, and where their number shares little with 8 every XCD
+  // fetches all of a row; neighbours then stay on one (figures: db2_walk).
+  const bool spans = p.slices == 1 && (q_tiles & 3) != 0;
+  const int pair = spans ? xcd_item((uint32_t)q_tiles * (uint32_t)k_tiles * (uint32_t)H) : blockIdx.x / p.slices;
+  if (pair >= q_tiles * k_tiles * H) return;
   const int row_begin = (int)((int64_t)p.n_rows * slice / p.slices), row_end = (int)((int64_t)p.n_rows * (slice + 1) / p.slices);
   const int qs0 = pair % q_tiles * kQ, ks0 = pair / q_tiles % k_tiles * kKeys, h = pair / q_tiles / k_tiles;
   const int q0 = qs0 + 32 * wave, qi = min(q0 + ln, s - 1);
@@ -1094,10 +1099,13 @@ static void db2_walk(const BwdParams& p, hipStream_t stream) {
     return (unsigned)((p.s + queries - 1) / queries) * (unsigned)((p.s + keys - 1) / keys) * (unsigned)p.heads * (unsigned)p.slices;
   };
   if constexpr (sizeof(T) == 2) {
+    // (with one slice spans of whole workgroups per XCD, see the kernel.  us, 64 rows, 4 heads, in turn / in spans: S = 1050 171 / 138, 1100 201 / 132,
+    // 1280 185 / 162, 1300 260 / 198; the query tiles a multiple of four, 1500 233 / 251, 2048 365 / 477; 3 rows of 600 7.5 / 6.6)
+    const auto grid = [&](int queries, int keys) { return dim3((groups(queries, keys) + 7) / 8 * 8); };
     const int64_t three = (int64_t)((groups(96, 64) + 255) / 256) * 3, four = (int64_t)((groups(128, 64) + 255) / 256) * 4;
-    if (groups(32, 32) <= 1024) attn_bwd_db2_kernel<2, 1><<<dim3(groups(64, 32)), dim3(128), 0, stream>>>(p);
-    else if (4 * four > 5 * three) attn_bwd_db2_kernel<3, 2><<<dim3(groups(96, 64)), dim3(192), 0, stream>>>(p);
-    else attn_bwd_db2_kernel<4, 2><<<dim3(groups(128, 64)), dim3(256), 0, stream>>>(p);
+    if (groups(32, 32) <= 1024) attn_bwd_db2_kernel<2, 1><<<grid(64, 32), dim3(128), 0, stream>>>(p);
+    else if (4 * four > 5 * three) attn_bwd_db2_kernel<3, 2><<<grid(96, 64), dim3(192), 0, stream>>>(p);
+    else attn_bwd_db2_kernel<4, 2><<<grid(128, 64), dim3(256), 0, stream>>>(p);
   } else {
     const dim3 grid(groups(64, 64));
     if ((p.s & 7) == 0) attn_bwd_db2_fp32_kernel<true><<<grid, dim3(256), 0, stream>>>(p);

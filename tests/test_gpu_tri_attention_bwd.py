@@ -204,7 +204,9 @@ def test_bias2_of_minus_infinity_has_weight_zero(dtype, with_bias1, N, S, H):
 
 @pytest.mark.parametrize("N,S,H", [(17, 33, 1), (24, 97, 4), (40, 160, 4), (16, 191, 2),       # two waves of one block
                                    (64, 192, 4), (70, 193, 5), (33, 257, 8), (64, 288, 4),      # three waves of two blocks
-                                   (64, 224, 4), (65, 289, 4), (64, 321, 5), (17, 800, 4)])     # four waves of two blocks
+                                   (64, 224, 4), (65, 289, 4), (64, 321, 5), (17, 800, 4),      # four waves of two blocks
+                                   # few rows, one slice: spans of tiles per XCD, each form, and tiles in turn (513)
+                                   (5, 97, 4), (3, 300, 2), (7, 520, 4), (5, 600, 4), (3, 1100, 4), (3, 513, 4), (2, 1030, 1)])
 def test_dbias2_in_workgroups_of_every_size(N, S, H):
     """The three forms of dBias2's walk, at sizes that fill their tiles, just pass them and fall short of them, masked keys among
     them.  Tolerance as for the other gradients: the reference's O and log-sum-exp are not rounded."""
