@@ -1,5 +1,6 @@
 // extern "C" boundary of libprotenix_amd.so: argument validation, dtype
 // dispatch, launch-error capture.  See include/protenix_amd.h for the contract.
+#include <algorithm>
 #include <stdarg.h>
 #include <stdio.h>
 
@@ -743,7 +744,7 @@ PTX_API int ptx_triattn_core_bwd(const void* q, const void* k, const void* v, co
 
 PTX_API int64_t ptx_triattn_core_bwd_partial_elems(int n_rows, int s, int heads) {
   if (n_rows <= 0 || s <= 0 || heads <= 0 || s > 8192 || heads > 64) return 0;
-  const int slices = ptx::triattn_bwd_slices(n_rows, s, heads);
+  const int slices = std::max(ptx::triattn_bwd_slices(n_rows, s, heads, true), ptx::triattn_bwd_slices(n_rows, s, heads, false));
   return slices > 1 ? (int64_t)slices * heads * s * s : 0;
 }
 

@@ -29,7 +29,6 @@ namespace ptx {
 namespace {
 
 constexpr float kBwdLog2e = 1.4426950408889634f;
-constexpr int64_t kDb2Workgroups = 1024;   // what the machine holds of dBias2's at once (triattn_bwd_slices)
 constexpr int kTP = 40;   // pitch of the LDS tiles (elements): 16-byte aligned rows, spread over banks
 
 struct BwdParams {
@@ -793,8 +792,8 @@ bool rows_at_once(const BwdParams& p) {
 // share.  Works on S^T like dQ.  Bias2 itself does not change along the walk and stays in registers; a row's Bias1 is added to it for the
 // initial value of the S^T accumulator, -Delta is that of dP^T.  Nothing in the walk looks at s: queries and keys beyond it repeat the last
 // one, and what accumulates for them is not stored.
-// The walk is cut into slices of rows: 384 tokens and 4 heads are 96 workgroups for 256 compute units that
-// hold four each, every one a serial chain over 384 rows.  Slices write fp32 partial sums that
+// The walk is cut into slices of rows: 384 tokens and 4 heads are 96 workgroups (of three waves; a compute unit holds twelve waves), every
+// one a serial chain over 384 rows.  Slices write fp32 partial sums that
 // attn_bwd_db2_sum_kernel adds in order (no atomics).  A slice's workgroups all go to one XCD
 // (workgroups are dealt to the XCDs in turn, and the slice is the fastest index), whose L2 then fetches the slice's rows
 // once; with a slice's workgroups on all eight the rows come through the memory-side cache eight times.  us at 384 rows,
@@ -1075,19 +1074,25 @@ __global__ __launch_bounds__(256) void attn_bwd_db2_sum_kernel(const float* __re
   }
 }
 
-// Slices of rows of dBias2's walk: eight, one per XCD, or as many more as give every compute unit its four
-// workgroups at once, of at least 8 rows, as long as the partial sums (4 S^2 H bytes per slice, written and
-// read once) stay within 128 MB.
-int triattn_bwd_slices(int n_rows, int s, int heads) {
-  const int64_t tiles = (s + 63) / 64, pairs = tiles * tiles * heads;
+// Slices of rows of dBias2's walk: eight, one per XCD, or as many more (multiples of eight) as 64 x 64 tiles make 1024 of, of at least
+// 8 rows, as long as the partial sums (4 S^2 H bytes per slice, written and read once) stay within 128 MB.  16-bit, up to 100 blocks of
+// 32 x 32: as many as make some 2300 blocks, one for 16 rows and eight more at most: there every block is a wave by itself (db2_walk),
+// of which a SIMD takes two in little more than the time of one, and what more slices save on the walk goes into their sums.  us, slices by
+// 64 x 64 tiles / by blocks, 4 heads: 256 rows of 64 19.5 / 18.6, 512 of 64 25.9 / 23.7, 512 of 96 31.0 / 25.7, 200 of 128 20.8 / 17.0, 512
+// of 128 33.3 / 26.7, 768 of 128 37.4 / 33.0, 160 of 160 21.0 / 18.0, 320 of 160 31.3 / 25.4; above 100: 512 of 128 with 8 heads 42.3 / 47.9, 448
+// of 224 46.3 / 50.5.
+int triattn_bwd_slices(int n_rows, int s, int heads, bool bits16) {
+  const int64_t tiles = (s + 63) / 64, pairs = tiles * tiles * heads, blocks = (int64_t)((s + 31) / 32) * ((s + 31) / 32) * heads;
   if (pairs <= 0 || n_rows <= 0) return 1;
-  int64_t want = std::min<int64_t>(std::max<int64_t>(8, kDb2Workgroups / pairs), n_rows / 8);
+  int64_t want = bits16 && blocks <= 100 ? std::min<int64_t>(2304 / blocks, n_rows / 16 + 8) : 1024 / pairs;
+  want = std::min<int64_t>(std::max<int64_t>(8, want), n_rows / 8);
   if (want > 8) want &= ~(int64_t)7;
   return want > 1 && want * heads * s * s * 4 <= (int64_t)128 << 20 ? (int)want : 1;
 }
 
-// dBias2's walk, 16-bit: waves of a workgroup and blocks of a wave.  A small one is a chain of rows, whose length counts: as long as
-// every SIMD can have a 32 x 32 block of its own, two waves of one block each.  Beyond, two blocks a wave, four waves or three; the work of a
+// dBias2's walk, 16-bit: waves of a workgroup and blocks of a wave.  A small one is a chain of rows, whose length counts: up to two
+// 32 x 32 blocks for every SIMD, two waves of one block each (a SIMD holds three; 2048 blocks: 256 rows of 256 in 8 slices 34.2 us,
+// four waves of two 38.1; 2304: 12 rows of 768 17.9 / 17.2).  Beyond, two blocks a wave, four waves or three; the work of a
 // compute unit is that of the workgroups it gets, in turn or at once, so the fullest one's waves count, and four do in the time of
 // three what loads a quarter less.  us at S rows of S positions, 4 heads, 64 x 64 tiles of four waves (before) / two waves of one block /
 // three of two / four of two: S = 64 7.4 / 5.6 / 8.7 / 9.0, 96 9.6 / 8.8 / 12.3 / 12.6, 160 15.2 / 13.6 / 16.4 / 17.6, 192 18.1 / 21.4 / 18.9 / 20.1, 256
@@ -1103,7 +1108,7 @@ static void db2_walk(const BwdParams& p, hipStream_t stream) {
     // 1280 185 / 162, 1300 260 / 198; the query tiles a multiple of four, 1500 233 / 251, 2048 365 / 477; 3 rows of 600 7.5 / 6.6)
     const auto grid = [&](int queries, int keys) { return dim3((groups(queries, keys) + 7) / 8 * 8); };
     const int64_t three = (int64_t)((groups(96, 64) + 255) / 256) * 3, four = (int64_t)((groups(128, 64) + 255) / 256) * 4;
-    if (groups(32, 32) <= 1024) attn_bwd_db2_kernel<2, 1><<<grid(64, 32), dim3(128), 0, stream>>>(p);
+    if (groups(32, 32) <= 2048) attn_bwd_db2_kernel<2, 1><<<grid(64, 32), dim3(128), 0, stream>>>(p);
     else if (4 * four > 5 * three) attn_bwd_db2_kernel<3, 2><<<grid(96, 64), dim3(192), 0, stream>>>(p);
     else attn_bwd_db2_kernel<4, 2><<<grid(128, 64), dim3(256), 0, stream>>>(p);
   } else {
@@ -1127,7 +1132,7 @@ int triattn_bwd(const void* q, const void* k, const void* v, const void* b1, con
                 const void* o, const float* lse, const void* dout, void* dq, void* dk, void* dv,
                 void* db2, float* delta, float* parts, int n_rows, int s, int heads, hipStream_t stream) {
   if (n_rows == 0 || s == 0 || heads == 0) return 0;
-  const int slices = parts && db2 ? triattn_bwd_slices(n_rows, s, heads) : 1;
+  const int slices = parts && db2 ? triattn_bwd_slices(n_rows, s, heads, sizeof(T) == 2) : 1;
   BwdParams p = {q, k, v, o, dout, b1, b2, lse, delta, dq, dk, dv, db2, n_rows, s, heads, slices > 1 ? parts : nullptr, slices};
   const dim3 walk(((unsigned)((s + 127) / 128) * heads * n_rows + 7) / 8 * 8);
   const bool joint = rows_at_once<T>(p);

@@ -225,7 +225,7 @@ int triattn_pack(const T* q, const T* k, const T* v, const T* bias2, T* qs, T* k
 // when db2 is given, dBias2 [heads][s][s], from Q (scaled), K, V, O, dO, the biases and the
 // forward's log2-sum-exp2; delta [n_rows][s][heads] is fp32 scratch; parts: fp32 scratch of
 // triattn_bwd_slices() * heads * s * s elements for the partial sums of dBias2, or null (one slice).
-int triattn_bwd_slices(int n_rows, int s, int heads);
+int triattn_bwd_slices(int n_rows, int s, int heads, bool bits16);
 template <typename T>
 int triattn_bwd(const void* q, const void* k, const void* v, const void* b1, const void* b2,
                 const void* o, const float* lse, const void* dout, void* dq, void* dk, void* dv,
