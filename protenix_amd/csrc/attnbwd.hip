@@ -535,7 +535,7 @@ __global__ __launch_bounds__(NW * 64, NBK == 1 ? 3 : 2) void attn_bwd_row_kernel
   typedef Vec8<T>::type V8;
   typedef Vec4<T>::type V4;
   constexpr int KB = NW * NBK, kExWave = 16 * kWave * 4;   // bytes of a wave's partial dQ
-  static_assert(1024 * (int)sizeof(T) <= kExWave, "a wave's dS tile fits its place for dQ");
+  static_assert(2 * 1024 * (int)sizeof(T) <= kExWave, "a wave's dS tile, and a block's dK and dV on their way out, fit its place for dQ");
   __shared__ __attribute__((aligned(32))) T kt[KB][1024];      // K, row-major, read by the wave that owns the block
   __shared__ __attribute__((aligned(32))) T rm[2][2][1024];      // Q, dO of the step
   __shared__ f32x8 stats[2][2][4];   // -log-sum-exp, -Delta of the step's queries

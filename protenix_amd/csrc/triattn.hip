@@ -892,7 +892,7 @@ int triattn_fwd_ex(const T* q, const T* k, const T* vt, const T* g, const T* tri
   }
   // Two rows per wave (16-bit, no mask): the two rows share the query block and with it the bias tile - one load
   // and one conversion per logit for both, half the bias stream from the L2 - at 128 registers, so that four waves
-  // still share a SIMD (with a mask the kernel needs 160 and loses a wave).  Below 272 tokens the pairs of rows leave too few
+  // still share a SIMD (a mask belongs to a row: one row per workgroup, 120 registers).  Below 272 tokens the pairs of rows leave too few
   // workgroups.  us per launch, 4 heads, one row / two rows (four waves each): n = 200 17.2 / 17.5, 256 20.9 / 21.1, 288 34.1 / 33.2, 300 36.7 /
   // 35.0, 320 35.8 / 34.1, 336 44.6 / 40.6, 350 50.7 / 46.4.
   const bool two_rows = sizeof(T) == 2 && !mask && n >= kTwoRowsFrom && row_count >= 2 && !standard;
@@ -930,15 +930,11 @@ int triattn_fwd_ex(const T* q, const T* k, const T* vt, const T* g, const T* tri
   }
   if constexpr (sizeof(T) == 2) {
     if (standard) {
-#define PTX_ATTN_LAUNCH_S(RR, MK)                                    \
-  do {                                                               \
-    if (wide) PTX_ATTN_LAUNCH_T(RR, 8, MK, void, true);              \
-    else PTX_ATTN_LAUNCH_T(RR, 4, MK, void, true);                   \
-  } while (0)
-      if (mk == kMaskGiven) PTX_ATTN_LAUNCH_S(1, kMaskGiven);
-      else if (mk == kMaskTail) PTX_ATTN_LAUNCH_S(1, kMaskTail);
-      else PTX_ATTN_LAUNCH_S(1, kMaskNone);
-#undef PTX_ATTN_LAUNCH_S
+      // (eight waves of one row: n >= 1536, where triattn_fwd_standard() asks for a mask)
+      if (mk == kMaskGiven && wide) PTX_ATTN_LAUNCH_T(1, 8, kMaskGiven, void, true);
+      else if (mk == kMaskGiven) PTX_ATTN_LAUNCH_T(1, 4, kMaskGiven, void, true);
+      else if (mk == kMaskTail) PTX_ATTN_LAUNCH_T(1, 4, kMaskTail, void, true);
+      else PTX_ATTN_LAUNCH_T(1, 4, kMaskNone, void, true);
       return 0;
     }
   }
