@@ -895,7 +895,10 @@ int triattn_fwd_ex(const T* q, const T* k, const T* vt, const T* g, const T* tri
   // still share a SIMD (a mask belongs to a row: one row per workgroup, 120 registers).  Below 272 tokens the pairs of rows leave too few
   // workgroups.  us per launch, 4 heads, one row / two rows (four waves each): n = 200 17.2 / 17.5, 256 20.9 / 21.1, 288 34.1 / 33.2, 300 36.7 /
   // 35.0, 320 35.8 / 34.1, 336 44.6 / 40.6, 350 50.7 / 46.4.
-  const bool two_rows = sizeof(T) == 2 && !mask && n >= kTwoRowsFrom && row_count >= 2 && !standard;
+  // Nor do they pay where one row per wave takes a single round of the machine, 1024 workgroups of four waves (a range of few rows): 272
+  // tokens, 64 rows (768 workgroups) 9.9 / 11.6, 85 (1020) 11.7 / 14.3, 100 15.2 / 14.7; 768, 2 rows 10.3 / 13.9, 32 18.4 / 21.2, 43 (1032)
+  // 32.2 / 28.5; 1024, 32 rows (1024) 29.7 / 29.0; 2048, 8 rows 31.9 / 46.3.
+  const bool two_rows = sizeof(T) == 2 && !mask && n >= kTwoRowsFrom && (int64_t)heads * row_count * ((n + 127) / 128) >= 1024 && !standard;
   // Eight waves share the staged K / V tiles of long rows.  Two rows: where that leaves no more waves without queries than four do (they
   // skip the arithmetic and only help to stage the tiles) and the keys fill whole tiles (with a partial one its registers
   // spill): four / eight 768 338 / 346, 1024 755 / 765, 1100 1001 / 1080, 1200 1346 / 1441, 1280 1475 / 1467, 1536 2509 / 2459, 2048

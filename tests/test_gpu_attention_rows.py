@@ -1,5 +1,5 @@
-"""The triangle-attention core where its workgroups change: two rows per wave from 352 tokens on, eight waves from 1057 on, odd
-numbers of rows and of query blocks, last key tiles of one key to a whole tile; and logits that leave the range of the
+"""The triangle-attention core where its workgroups change: two rows per wave from 272 tokens on, if there are enough of them, eight
+waves from 1057 on, if the queries fill them and the keys whole tiles; odd numbers of rows and of query blocks, last key tiles of one key to a whole tile; and logits that leave the range of the
 reference 0, which take rows off the common path in the middle of a wave's work."""
 import math
 
@@ -37,15 +37,15 @@ def _reference(q, k, v, b, rows, n_keys):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("n", [33, 351, 352, 353, 385, 417, 1057])
+@pytest.mark.parametrize("n", [33, 271, 272, 273, 351, 352, 353, 385, 417, 1057, 1152, 1280])
 @pytest.mark.parametrize("scale", [1.0, 40.0])
 def test_core(n, scale):
-    lib, heads = _lib.load(), 1
+    lib, heads = _lib.load(), 2 if 256 < n < 300 else 1        # (1024 workgroups of one row and 128 queries, for two rows per wave)
     g = torch.Generator().manual_seed(n)
     dev, plain, pitch = _core(n, heads, scale, g)
     dq, dk, dv, db = (t.cuda() for t in dev)
     st = torch.cuda.current_stream().cuda_stream
-    for row0, count, n_keys in ((0, n, n), (2, n - 3, n - 1)):
+    for row0, count, n_keys in ((0, n, n), (2, n - 3, n - 1), (1, n - 2, n)):
         o = torch.full((heads, n, n, 32), 7.0, dtype=torch.bfloat16, device="cuda")
         rc = lib.ptx_triattn_fwd_rows(dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), None, db.data_ptr(), None, o.data_ptr(), n, heads, 32,
                                       pitch, 0, 1e9, row0, count, n_keys, 1, st)
