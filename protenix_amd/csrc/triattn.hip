@@ -557,10 +557,10 @@ __global__ __launch_bounds__((NWQ * 64), (sizeof(T) == 2 ? (!std::is_void<TS>::v
 #pragma unroll
       for (int e = 0; e < 16; ++e) s[e] = fast_exp2(s[e]);
     } else if constexpr (!MASKED) {
-      // (as below: no key with a finite logit yet)
-      const float nml = -fmaxf(m_run[r], -2.0e38f) * kLog2e;
+      // (as below: no key with a finite logit yet; one rounding, in every instantiation)
+      const float mref = fmaxf(m_run[r], -2.0e38f);
 #pragma unroll
-      for (int e = 0; e < 16; ++e) s[e] = fast_exp2(s[e] + nml);
+      for (int e = 0; e < 16; ++e) s[e] = fast_exp2(__builtin_fmaf(mref, -kLog2e, s[e]));
     } else {
       // (no key with a finite logit yet: -inf minus a finite stand-in is -inf, weight 0, where
       // -inf minus -inf would not be a number)
@@ -667,7 +667,7 @@ __global__ __launch_bounds__((NWQ * 64), (sizeof(T) == 2 ? (!std::is_void<TS>::v
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
       if (TAIL && nk - tile * kKeyTile <= 16 * u) continue;   // (the half has no keys)
-      if (FIRST && !near_zero) continue;
+      if (FIRST && R == 2 && !near_zero) continue;   // (of one row, a small launch: a branch more than it saves)
       f32x16 tbf = bias_of(tb[u]);
       asm volatile("" : "+v"(tbf) :: "memory");   // (converted before its registers are loaded again)
       fetch_bias_half(tile + 1, u, tb[u]);
