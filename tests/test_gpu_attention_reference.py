@@ -1,6 +1,7 @@
-"""The triangle-attention core's common path takes every probability against the softmax reference 0 and looks at its sums after
-the first key tile and after the last: logits that its sums can take, that send the workgroup to the checked walk from the second
-tile on, and that make it start again; key ranges of less than a tile, one tile, and one key more."""
+"""The triangle-attention core's common path takes every probability against the softmax reference 0.  It is entered where that is
+the reference of every row's first half tile (the largest logit within 14 of 0, 2^20.2), looks at its sums at the end, and waves
+with one beyond 1e12 = 2^39.9 start again: logits on either side of both lines, early and late; key ranges of less than a tile, one
+tile, and one key more; rows whose bits are their own affair."""
 
 import pytest
 import torch
@@ -22,8 +23,8 @@ def _add(dev_bias, plain_bias, queries, keys, value):
 @pytest.mark.gpu
 @pytest.mark.parametrize("n", [65, 130, 353, 1280])
 @pytest.mark.parametrize("where", ["first", "last", "all"])
-# log2 units: sums up to 1e12 = 2^40 stay, up to 1e25 = 2^83 leave after the first tile, beyond (2^128: infinity) start again
-@pytest.mark.parametrize("value", [30.0, 60.0, 100.0, 200.0, -100.0])
+# log2 units: see above (2^128 and more: infinity)
+@pytest.mark.parametrize("value", [18.0, 22.0, 30.0, 38.0, 42.0, 60.0, 100.0, 200.0, -100.0])
 def test_logits_away_from_zero(n, where, value):
     lib, heads = _lib.load(), 1
     g = torch.Generator().manual_seed(n)
@@ -94,8 +95,20 @@ def test_up_to_a_masked_key(n, key, value):
 @pytest.mark.gpu
 @pytest.mark.parametrize("rows,s", [(3, 353), (2, 640), (1, 1535), (2, 1536)])
 def test_operator_without_bias1(rows, s):
-    """Up to 1535 positions the operator's operands are read as they are, beyond they are repacked."""
+    """Up to 1535 positions the operator's operands are read as they are, beyond they are repacked in both calls."""
     _standard_layouts(rows, s, 2, False)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,s", [(3, 353), (1, 1535), (2, 1536), (1, 1600)])
+def test_operator_without_bias1_against_full_precision(rows, s):
+    """On both sides of that line, against the operator on the same operands in fp32."""
+    g = torch.Generator().manual_seed(s)
+    q, k, v = (torch.randn(1, rows, s, 2, 32, generator=g).bfloat16() for _ in range(3))
+    q, b2 = (q.float() / 32 ** 0.5).bfloat16(), torch.randn(1, 1, 2, s, s, generator=g).bfloat16()
+    got = P.TriAttentionFunction.apply(*(t.cuda() for t in (q, k, v)), None, b2.cuda()).float().cpu()
+    want = O.softmax_attention(*(t.float().transpose(-2, -3) for t in (q, k, v)), [b2.float()]).transpose(-2, -3)
+    assert rel_err(got, want) <= tol(torch.bfloat16)
 
 
 @pytest.mark.gpu

@@ -1,6 +1,6 @@
 """The triangle-attention core where its workgroups change: two rows per wave from 272 tokens on, if there are enough of them, eight
-waves from 1057 on, if the queries fill them and the keys whole tiles; odd numbers of rows and of query blocks, last key tiles of one key to a whole tile; and logits that leave the range of the
-reference 0, which take rows off the common path in the middle of a wave's work."""
+waves from 1057 on, if the queries fill them and the keys whole tiles; odd numbers of rows and of query blocks, last key tiles of one
+key to a whole tile; and logits that leave the range of the reference 0, which take rows off the common path."""
 import math
 
 import pytest
