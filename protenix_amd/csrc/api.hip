@@ -719,7 +719,7 @@ PTX_API int ptx_triattn_core_fwd(const void* q, const void* k, const void* v, co
     float* lb = lse ? lse + (int64_t)b * n_rows * s * heads : nullptr;
     // 16-bit: q, K and V are read as they are, as long as the output does not overwrite them under way
     auto apart = [&](const char* t) { return ob + n_q * es <= t || t + n_q * es <= ob; };
-    const bool as_is = dtype == PTX_BF16 && ptx::triattn_fwd_standard(s, b1 != nullptr) && apart(qb) && apart(kb) && apart(vb);
+    const bool as_is = dtype == PTX_BF16 && ptx::triattn_fwd_standard(n_rows, s, heads, b1 != nullptr) && apart(qb) && apart(kb) && apart(vb);
     PTX_DISPATCH(dtype, {
       ptx::triattn_pack<T>(as_is ? nullptr : (const T*)qb, (const T*)kb, (const T*)vb, (const T*)b2, (T*)qs, (T*)kf,
                            (T*)vtf, (T*)bf, n_rows, s, heads, pitch, (hipStream_t)stream);

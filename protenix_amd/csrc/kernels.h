@@ -208,7 +208,7 @@ bool triattn_fwd_carries(int n, bool bits16);
 // The launch covers rows row_begin .. row_begin + row_count - 1 and lets keys 0 .. n_keys - 1
 // take part (keys beyond count as masked: weight exactly zero).  standard (16-bit): k and vt are K and V addressed by q's
 // strides, and q is not yet in log2 units; where triattn_fwd_standard().
-bool triattn_fwd_standard(int n, bool masked);
+bool triattn_fwd_standard(int n_rows, int n, int heads, bool masked);
 template <typename T>
 int triattn_fwd_ex(const T* q, const T* k, const T* vt, const T* g, const T* tri_bias,
                    const T* mask, T* o, int n_rows, int n, int heads, int key_pitch,

@@ -841,11 +841,18 @@ __global__ __launch_bounds__((NWQ * 64), (sizeof(T) == 2 ? (!std::is_void<TS>::v
 
 constexpr int kTwoRowsFrom = 272;   // (see triattn_fwd_ex)
 
+// workgroups of four waves that take one row each
+static int64_t one_row_groups(int n_rows, int n, int heads) { return (int64_t)heads * n_rows * ((n + 127) / 128); }
+
 // Where the core reads standard layouts: with one row per wave (with two, the lanes' addresses take registers that it does not
 // have).  Two rows per wave on repacked operands gain less than the repacking costs.  us, the operator's forward without Bias1, 4 heads,
 // S rows of S positions, repacked / as they are: 352 92 / 65, 384 101 / 73, 512 198 / 144, 640 334 / 298, 768 516 / 474, 1024 1089 / 1072, 1536
-// 3268 / 3273; 64 rows of 384 32 / 19, of 768 58 / 48.
-bool triattn_fwd_standard(int n, bool masked) { return masked || n < 1536; }
+// 3268 / 3273; 64 rows of 384 32 / 19, of 768 58 / 48.  Beyond,
+// where the rows are few one is taken per wave either way: 2 rows of 1536 68 / 42, 8 of 2048 (512 workgroups of four waves) 92 / 72, 4 of 4096
+// (512) 264 / 255, 7 of 4096 (896) 270 / 304: there repacked operands go to workgroups of eight.
+bool triattn_fwd_standard(int n_rows, int n, int heads, bool masked) {
+  return masked || n < 1536 || one_row_groups(n_rows, n, heads) <= 512;
+}
 
 // (one row and four waves at those sizes, and workgroups to spare)
 bool triattn_fwd_carries(int n, bool bits16) { return bits16 && n <= 256; }
@@ -898,12 +905,12 @@ int triattn_fwd_ex(const T* q, const T* k, const T* vt, const T* g, const T* tri
   // Nor do they pay where one row per wave takes a single round of the machine, 1024 workgroups of four waves (a range of few rows): 272
   // tokens, 64 rows (768 workgroups) 9.9 / 11.6, 85 (1020) 11.7 / 14.3, 100 15.2 / 14.7; 768, 2 rows 10.3 / 13.9, 32 18.4 / 21.2, 43 (1032)
   // 32.2 / 28.5; 1024, 32 rows (1024) 29.7 / 29.0; 2048, 8 rows 31.9 / 46.3.
-  const bool two_rows = sizeof(T) == 2 && !mask && n >= kTwoRowsFrom && (int64_t)heads * row_count * ((n + 127) / 128) >= 1024 && !standard;
+  const bool two_rows = sizeof(T) == 2 && !mask && n >= kTwoRowsFrom && one_row_groups(row_count, n, heads) >= 1024 && !standard;
   // Eight waves share the staged K / V tiles of long rows.  Two rows: where that leaves no more waves without queries than four do (they
   // skip the arithmetic and only help to stage the tiles) and the keys fill whole tiles (with a partial one its registers
   // spill): four / eight 768 338 / 346, 1024 755 / 765, 1100 1001 / 1080, 1200 1346 / 1441, 1280 1475 / 1467, 1536 2509 / 2459, 2048
   // 5909 / 5775.  One row: +2 % at n = 768, even at 1024, -2.6 % at 1536.
-  const bool wide = sizeof(T) == 2 && (two_rows ? n > 1056 && (n + 127) / 128 % 2 == 0 && n_keys % kKeyTile == 0
+  const bool wide = sizeof(T) == 2 && (mask || !standard) && (two_rows ? n > 1056 && (n + 127) / 128 % 2 == 0 && n_keys % kKeyTile == 0
                                                 : (n % 256 == 0 && n >= 1536) || n >= 2048);
   const int mk = mask ? kMaskGiven : n_keys % kKeyTile ? kMaskTail : kMaskNone;
   const int n_qtiles = wide ? (n + 255) / 256 : (n + 127) / 128;
@@ -933,7 +940,7 @@ int triattn_fwd_ex(const T* q, const T* k, const T* vt, const T* g, const T* tri
   }
   if constexpr (sizeof(T) == 2) {
     if (standard) {
-      // (eight waves of one row: n >= 1536, where triattn_fwd_standard() asks for a mask)
+      // (without a mask four waves: beyond 1535 positions triattn_fwd_standard() leaves few rows only)
       if (mk == kMaskGiven && wide) PTX_ATTN_LAUNCH_T(1, 8, kMaskGiven, void, true);
       else if (mk == kMaskGiven) PTX_ATTN_LAUNCH_T(1, 4, kMaskGiven, void, true);
       else if (mk == kMaskTail) PTX_ATTN_LAUNCH_T(1, 4, kMaskTail, void, true);

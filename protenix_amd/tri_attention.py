@@ -5,7 +5,7 @@ Mirrors protenix/model/tri_attention/op.py:37-77 (`TriAttentionFunction`: Q, K, 
 protenix/model/triangular/layers.py:539-583 (`_tri_attention`: q, k, v [*, H, Q, C] and a list of
 two biases), with the backward of op.py:79-163.  The N^3 logits are never materialised.  Runs the same
 attention core as `TriangleAttention`: 16-bit Q, K, V are read as they are (without a Bias1 up to 1535
-positions), Bias2 is repacked into the core's tile order; fp32 and longer rows cost one extra pass over Q, K, V.
+positions, beyond for few rows), Bias2 is repacked into the core's tile order; fp32 and longer rows cost one extra pass over Q, K, V.
 """
 from __future__ import annotations
 

@@ -93,16 +93,17 @@ def test_up_to_a_masked_key(n, key, value):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("rows,s", [(3, 353), (2, 640), (1, 1535), (2, 1536)])
+@pytest.mark.parametrize("rows,s", [(3, 353), (2, 640), (1, 1535), (1, 1536), (2, 1536), (21, 1600), (2, 2049)])
 def test_operator_without_bias1(rows, s):
-    """Up to 1535 positions the operator's operands are read as they are, beyond they are repacked in both calls."""
+    """Up to 1535 positions, and beyond where the rows are few (up to 512 workgroups of 128 queries; 21 of 1600 are more, and
+    repacked in both calls), the operator's operands are read as they are."""
     _standard_layouts(rows, s, 2, False)
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("rows,s", [(3, 353), (1, 1535), (2, 1536), (1, 1600)])
+@pytest.mark.parametrize("rows,s", [(3, 353), (1, 1535), (2, 1536), (21, 1600)])
 def test_operator_without_bias1_against_full_precision(rows, s):
-    """On both sides of that line, against the operator on the same operands in fp32."""
+    """On both sides of those lines, against the oracle on the same operands in fp32."""
     g = torch.Generator().manual_seed(s)
     q, k, v = (torch.randn(1, rows, s, 2, 32, generator=g).bfloat16() for _ in range(3))
     q, b2 = (q.float() / 32 ** 0.5).bfloat16(), torch.randn(1, 1, 2, s, s, generator=g).bfloat16()
