@@ -256,7 +256,7 @@ __global__ __launch_bounds__((NWQ * 64), (sizeof(T) == 2 ? (!std::is_void<TS>::v
   const int i0 = ax.row0 + (int)((item / n_qtiles) % n_rowgroups) * R;   // first of this workgroup's R rows
   const int h = (int)(item / ((int64_t)n_qtiles * n_rowgroups));
 
-  if constexpr (MK == kMaskGiven && !STD && R == 1 && sizeof(T) == 2) {
+  if constexpr (MK == kMaskGiven && !STD && !kCarries && R == 1 && sizeof(T) == 2) {
     if (ax.uniform_limit > 0.0f) {   // (what triattn_uniform_kernel left; nobody else's output lies here)
       const int first = qt * NWQ * 32, blocks = min(NWQ, (n - first + 31) >> 5);
       T* const rows = o + h * ax.sh + i0 * ax.si + (int64_t)first * kD;
